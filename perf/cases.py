@@ -91,7 +91,8 @@ def draw(rng):
         fp32 = rng.random() < 0.2
         forms = ["drop_in", "static_rows", "defer", "compact_defer"] + ([] if fp32 else ["folded"])
         form = rng.choice(forms if top_k == 1 else ["drop_in", "compact", "compact_defer"])
-        return _layer(None, _log_int(rng, 8, most), d, d_ff, rng.choice([4, 8, 12, 16, 32, 64, 128]), top_k, form,
+        experts = rng.choice([e for e in (4, 8, 12, 16, 32, 64, 128) if 2 * e * d * d_ff * (4 if fp32 else 2) <= 8.6e9])
+        return _layer(None, _log_int(rng, 8, most), d, d_ff, experts, top_k, form,
                       dtype="fp32" if fp32 else "bf16", capacity_factor=rng.choice([1.25, 2.0]),
                       skew=rng.choice([0.0, 0.0, 1.2]), bias=rng.random() < 0.25)
     if kind == "ffn":
