@@ -235,24 +235,13 @@ __global__ __launch_bounds__(WAVES * 64) void grouped_gemm_kernel(GemmArgs a) {
   // the epilogue.
   if (a.tags != nullptr) {
     for (int r = tid; r < rows; r += THREADS) {
-      int cell;
-      size_t gate_at;  // accumulate form: where the row's weight stands
-      if (a.tag_vector) {
-        const int entry = a.tags[static_cast<size_t>(row0) + r];
-        cell = a.tag_div > 1 ? (entry - 1) / a.tag_div : entry - 1;
-        cell = (entry >= 1 && cell < a.T) ? cell : -1;
-        gate_at = static_cast<size_t>(max(entry, 1)) - 1;
-      } else {
-        // the tag matrix has T rows; a load padded beyond T (capacity above the batch size) names
-        // slots that do not exist: they are empty, as in dispatch (route.cu:84-92 bounds the slot
-        // by the cell count)
-        const int slot = seat0 + r;
-        const int tag = slot < a.T ? a.tags[static_cast<size_t>(slot) * a.E + e] : 0;
-        cell = (tag >= 1 && tag <= a.T) ? tag - 1 : -1;
-        gate_at = static_cast<size_t>(max(cell, 0)) * a.E + e;
-      }
+      const int cell = routed_cell(a, e, row0 + r, seat0 + r);
       s_cell[r] = cell;
-      if (a.gates != nullptr) s_gate[r] = a.gates[cell >= 0 ? gate_at : 0];  // entry 0 for an empty slot: never used
+      if (a.gates != nullptr) {  // accumulate form: the weight of the row's entry, or of its cell on this path
+        const size_t at = a.tag_vector ? static_cast<size_t>(max(a.tags[row0 + r], 1)) - 1
+                                       : static_cast<size_t>(max(cell, 0)) * a.E + e;
+        s_gate[r] = a.gates[cell >= 0 ? at : 0];  // entry 0 for an empty slot: never used
+      }
       // side output for a combine that runs later: the cell of every row, written once per row block
       if (a.row_tags_out != nullptr && nt_first == 0) a.row_tags_out[static_cast<size_t>(row0) + r] = cell + 1;
     }
@@ -737,11 +726,6 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
     a.clocks = clocks;
     return launch_pingpong_gemm(a, act, as_stream(stream));
   }
-  if (out_is_f32) {
-    if (act == BRT_ACT_GELU) return launch_f32<BRT_ACT_GELU>(a, as_stream(stream));
-    if (act == BRT_ACT_RELU) return launch_f32<BRT_ACT_RELU>(a, as_stream(stream));
-    return launch_f32<BRT_ACT_NONE>(a, as_stream(stream));
-  }
   // Kernel choice.  Experts that average more than one row block take the ping-pong kernel
   // (grouped_gemm_pingpong.hip), whose 256 x 256 tile moves a third fewer operand bytes per flop,
   // when its tiles come in whole rounds over the CUs: at least two rounds, or one round that most
@@ -751,12 +735,19 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   // process against the 160-row kernel: 8 experts x 4096 rows 2048 -> 8192 -> 2048 1165 / 993 ->
   // 962 / 793 us, the ragged task-MoE shape 1585 / 1374 -> 1355 / 1211 us, the top-2 shape's
   // expanding GEMM (1232 tiles) 212 -> 166 us, 8 x 1824 rows 4096 -> 1024 (256 tiles) 146 -> 99 us;
-  // the top-2 shape's contracting GEMM (308 tiles on 256 CUs) 162 -> 173 us.
+  // the top-2 shape's contracting GEMM (308 tiles on 256 CUs) 162 -> 173 us.  The rule is the same
+  // for gathered, scattered and fp32-output rows: a gathering 1024 -> 4096 GEMM with GELU over 32768
+  // rows of 16 experts takes 437 us on the 160-row kernel and 336 us here.
   if (pingpong_gemm_applies(a) && static_cast<long>(P) > static_cast<long>(E) * 160) {
     const long tiles = (static_cast<long>(P + 255) / 256 + (E + 1) / 2) * ((N + 255) / 256);
     const long cus = device_cus();
     if (tiles >= 2 * cus || (4 * tiles >= 3 * cus && tiles <= cus))
       return launch_pingpong_gemm(a, act, as_stream(stream));
+  }
+  if (out_is_f32) {
+    if (act == BRT_ACT_GELU) return launch_f32<BRT_ACT_GELU>(a, as_stream(stream));
+    if (act == BRT_ACT_RELU) return launch_f32<BRT_ACT_RELU>(a, as_stream(stream));
+    return launch_f32<BRT_ACT_NONE>(a, as_stream(stream));
   }
   // Tile choice.  A wavefront owns 160 x 64 outputs (7 LDS fragment reads feed 10 MFMAs); a
   // workgroup is 2, 3 or 4 of them side by side.  The kernel is bound by how fast a CU can fill

@@ -38,6 +38,20 @@ struct GemmArgs {
 bool pingpong_gemm_applies(const GemmArgs& a);
 int launch_pingpong_gemm(GemmArgs& a, int act, hipStream_t st);
 
+// The routed forms: 0-based cell behind row `row` of the dispatched layout (seat `seat`, 0-based, of
+// expert e), -1 for an empty slot.  From the tag matrix a load padded beyond T (capacity above the
+// batch size) names slots that do not exist: they are empty, as in dispatch (route.cu:84-92 bounds
+// the slot by the cell count).
+__device__ __forceinline__ int routed_cell(const GemmArgs& a, int e, int row, int seat) {
+  if (a.tag_vector) {
+    const int entry = a.tags[row];
+    const int cell = a.tag_div > 1 ? (entry - 1) / a.tag_div : entry - 1;
+    return (entry >= 1 && cell < a.T) ? cell : -1;
+  }
+  const int tag = seat < a.T ? a.tags[static_cast<size_t>(seat) * a.E + e] : 0;
+  return (tag >= 1 && tag <= a.T) ? tag - 1 : -1;
+}
+
 // GELU(v) = v * Phi(v) = max(v, 0) - |v| * Phi(-|v|), branch free.  The tail probability is
 // exp2(Q(|v|)) with Q a degree-7 fit of log2 Phi(-x) on [0, 8] (|Q - log2 Phi| < 5e-5 there, so the
 // tail is good to 3.5e-5 relative; beyond 8 the product is below 5e-15 and Q keeps falling to -inf).

@@ -34,6 +34,10 @@
 //     this K-step has landed); the barrier that ends a phase publishes the data.
 //   - Workgroups are numbered in patch order (see grouped_gemm.hip): 4 row blocks x 8 column tiles
 //     of one expert on an XCD at a time, sharing both operands through that XCD's L2.
+//   - Routed rows cost the K loop nothing: a wavefront keeps the byte offsets of the eight row groups
+//     it loads in registers for any kind of row, so a gathered row (its cell's offset) and an
+//     activation or weight row (row times pitch) are the same load.  The cells pass through the
+//     first bytes of the stages once, before any operand lands there.
 //   - The epilogue sends the tile out 32 rows at a time through each wavefront's own corner of
 //     LDS (the stages are dead by then), full 128-byte rows per store.
 #include <algorithm>
@@ -66,9 +70,6 @@ constexpr int kSub = kBK / 16;                        // MFMA k-steps per stage
 constexpr int kHead = 4;                              // MFMAs of a C phase issued ahead of the barrier
 constexpr uint32_t kOutOfRange = 0x80000000u;         // buffer offset past any extent: reads as zero
 constexpr int kXcds = 8, kCusPerXcd = 32, kPatchRows = 4;
-constexpr int kImageRow = kNT * 32 * 2 + 16;          // padded row of a wavefront's 32-row output image
-constexpr int kImageB = 32 * kImageRow;
-static_assert(kWaves * kImageB <= kLdsBytes, "the output images must fit the stages");
 
 __device__ __forceinline__ i32x4 make_rsrc(const void* p, size_t bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(p);
@@ -109,11 +110,13 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-template <int ACT>
+template <int ACT, bool ROUTED, bool OUTF32>
 __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  // the tile's coordinates pass through the first bytes of the stages, before any load lands there
-  int* const s_tile = reinterpret_cast<int*>(smem);  // expert, first row, valid rows, column tile
+  // the tile's coordinates and, in the routed forms, the cells behind its rows pass through the
+  // first bytes of the stages, before any load lands there
+  int* const s_tile = reinterpret_cast<int*>(smem);  // expert, first row, valid rows, column tile, first seat
+  int* const s_cell = s_tile + 16;                   // 0-based cell of each row of the tile, -1 = empty slot
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -156,22 +159,45 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
           s_tile[1] = carry_m + incl_m - m + block * kBM;
           s_tile[2] = min(kBM, m - block * kBM);
           s_tile[3] = col;
+          s_tile[4] = block * kBM;
         }
       }
       carry_t += __shfl(incl_t, kWave - 1, kWave);
       carry_m += __shfl(incl_m, kWave - 1, kWave);
     }
-    if (!found && lane == 0) s_tile[0] = -1;
+    if (!found && lane == 0) {  // beyond the last entry of the list: how far, and where the rows end
+      s_tile[0] = -1;
+      s_tile[1] = carry_m;
+      s_tile[2] = t - carry_t;
+    }
   }
   __syncthreads();
   const int e = __builtin_amdgcn_readfirstlane(s_tile[0]);
-  if (e < 0) return;  // beyond the last entry of the list
+  if (e < 0) {
+    // Surplus workgroups clear the tags of the rows no path owns: the j-th takes rows
+    // [total + 256 j, total + 256 (j + 1)).  The grid holds P / 256 + E row blocks (rounded up) per
+    // column tile and the experts use at most (total + 255 E) / 256 of them, so enough are left.
+    if (ROUTED && a.row_tags_out != nullptr) {
+      const long r = static_cast<long>(s_tile[1]) + static_cast<long>(s_tile[2]) * kBM + tid;
+      if (tid < kBM && r < a.P) a.row_tags_out[r] = 0;
+    }
+    return;
+  }
   const int row0 = __builtin_amdgcn_readfirstlane(s_tile[1]);
   const int rows = min(__builtin_amdgcn_readfirstlane(s_tile[2]), a.P - row0);
   const int n0 = __builtin_amdgcn_readfirstlane(s_tile[3]) * kBN;
+  const int seat0 = __builtin_amdgcn_readfirstlane(s_tile[4]);
   const int K = a.K;
   const int k_tiles = K / kBK;
-  __syncthreads();  // everyone has read the coordinates; the loads may overwrite them
+  if constexpr (ROUTED) {  // one word per row, all of them in one round trip
+    if (tid < kBM) {
+      const int cell = tid < rows ? routed_cell(a, e, row0 + tid, seat0 + tid) : -1;
+      s_cell[tid] = cell;
+      // side output for a combine that runs later: written once per row block
+      if (a.row_tags_out != nullptr && n0 == 0 && tid < rows) a.row_tags_out[static_cast<size_t>(row0) + tid] = cell + 1;
+    }
+    __syncthreads();
+  }
 
   // ---- global -> LDS ---------------------------------------------------------------------------
   // A load fills one row group: 8 tile rows, a whole 128-byte line of each.  Group 0 loads the
@@ -182,25 +208,38 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // go into the scalar offset, so no per-load register stays live.  A row that does not exist
   // (past the expert's last row, past N) gets an offset past any extent: zeros, no memory request.
   const __bf16* const w_e = a.w[e];
-  const i32x4 res_a = make_rsrc(a.x + static_cast<size_t>(row0) * K, static_cast<size_t>(a.P - row0) * K * 2);
-  const i32x4 res_b = make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2);
+  // Every wavefront keeps the eight offsets of its rows in registers (the K-step alone goes into
+  // the scalar offset).  Gathered rows need that -- the cells of a row group are anywhere in x --
+  // and it takes the bounds check out of the loop for the others.
+  const bool gather = ROUTED && a.gather != 0;
+  const i32x4 res = wm == 0
+      ? (gather ? make_rsrc(a.x, static_cast<size_t>(a.T) * K * 2)
+                : make_rsrc(a.x + static_cast<size_t>(row0) * K, static_cast<size_t>(a.P - row0) * K * 2))
+      : make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2);
   const int cols = a.N - n0;  // weight rows that exist from n0 on
-  const uint32_t chunk_a = (lane & 7) ^ (((wn & 1) << 2) | (lane >> 4));
-  const int row_a = wn * 8 + (lane >> 3);
-  const uint32_t off_a = (static_cast<uint32_t>(row_a) * K + chunk_a * 8) * 2;
-  const uint32_t step_a = static_cast<uint32_t>(32) * K * 2;  // 4 row groups further
-  const uint32_t chunk_b = (lane & 7) ^ (lane >> 4);           // even row group; odd ones flip bit 2 (byte 64)
-  const int row_b = wn * 64 + (lane >> 3);
-  const uint32_t off_b = (static_cast<uint32_t>(row_b) * K + chunk_b * 8) * 2;
-  const uint32_t step_b = static_cast<uint32_t>(8) * K * 2;   // 1 row group further
+  uint32_t off[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int group = wm == 0 ? wn + 4 * i : wn * 8 + i;
+    const int row = group * 8 + (lane >> 3);
+    const uint32_t chunk = (lane & 7) ^ ((row >> 1) & 7);
+    int at = row;
+    bool there = row < (wm == 0 ? rows : cols);
+    if constexpr (ROUTED) {
+      if (gather && wm == 0) {
+        at = s_cell[row];
+        there = at >= 0;
+      }
+    }
+    off[i] = there ? (static_cast<uint32_t>(at) * K + chunk * 8) * 2 : kOutOfRange;
+  }
+  __syncthreads();  // everyone has read the coordinates and cells; the loads may overwrite them
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
   auto load_a = [&](int kt, uint32_t slot, int i) {
-    const uint32_t off = row_a + i * 32 < rows ? off_a : kOutOfRange;
-    load_to_lds(res_a, off, kt * kRowB + i * step_a, lds0 + slot + (wn + 4 * i) * 1024);
+    load_to_lds(res, off[i], kt * kRowB, lds0 + slot + (wn + 4 * i) * 1024);
   };
   auto load_b = [&](int kt, uint32_t slot, int i) {
-    const uint32_t off = row_b + i * 8 < cols ? off_b ^ ((i & 1) << 6) : kOutOfRange;
-    load_to_lds(res_b, off, kt * kRowB + i * step_b, lds0 + kBBase + slot + (wn * 8 + i) * 1024);
+    load_to_lds(res, off[i], kt * kRowB, lds0 + kBBase + slot + (wn * 8 + i) * 1024);
   };
 
   // ---- fragments -------------------------------------------------------------------------------
@@ -342,11 +381,17 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // wavefront's 32 j .. 32 j + 31) 8 * (r / 4) + 4 * (lane / 32) + r % 4, i.e. a lane holds 4
   // consecutive columns (8 bytes) of its row.
   const global_bf16 bias = a.bias != nullptr ? (global_bf16)(a.bias[e]) : (global_bf16)nullptr;
+  constexpr int kOutB = OUTF32 ? 4 : 2;                 // bytes of one output element
+  constexpr int kImageRow = kNT * 32 * kOutB + 16;      // padded row of this wavefront's 32-row image
+  constexpr int kImageB = 32 * kImageRow;
+  static_assert(kWaves * kImageB <= kLdsBytes, "the output images must fit the stages");
   char* const image = smem + wave * kImageB;
   const int mine = rows - wm * kMT * 32;  // rows of the tile this wavefront holds
   const int col_w = n0 + wn * kNT * 32;   // first column of this wavefront
-  __bf16* const out_w = a.out + (static_cast<size_t>(row0) + wm * kMT * 32) * a.N + col_w;
-  constexpr int kChunksPerRow = kNT * 32 / 8;  // 8 chunks of 16 bytes
+  const int row_w = row0 + wm * kMT * 32; // first row
+  constexpr int kChunk = 16 / kOutB;                    // elements of one 16-byte store
+  constexpr int kChunksPerRow = kNT * 32 / kChunk;
+  constexpr int kRowsPerPass = kWave / kChunksPerRow;
   // the bias of this lane's columns, all eight loads in one round trip
   bf16x4 bv[kNT][4];
 #pragma unroll
@@ -360,26 +405,57 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
 #pragma unroll
   for (int i = 0; i < kMT; ++i) {
     if (i * 32 >= mine) break;  // wave-uniform
+    // scattered rows: lane r of the pass holds the cell of row r (read again: LDS held operands)
+    int cell = -1;
+    if constexpr (ROUTED) {
+      if (a.scatter && lane < min(32, mine - i * 32)) {
+        const int r = row_w + i * 32 + lane;
+        cell = routed_cell(a, e, r, r - row0 + seat0);
+      }
+    }
 #pragma unroll
     for (int j = 0; j < kNT; ++j) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int col = j * 32 + 8 * g + 4 * frag_k;  // inside the wavefront's 64 columns
         const bf16x4 b4 = bv[j][g];
-        bf16x4 o;
+        float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          o[q] = static_cast<__bf16>(apply_act<ACT>(acc[i][j][4 * g + q] + static_cast<float>(b4[q])));
-        *reinterpret_cast<bf16x4*>(image + frag_row * kImageRow + col * 2) = o;
+        for (int q = 0; q < 4; ++q) v[q] = apply_act<ACT>(acc[i][j][4 * g + q] + static_cast<float>(b4[q]));
+        char* const to = image + frag_row * kImageRow + col * kOutB;
+        if constexpr (OUTF32) {
+          *reinterpret_cast<f32x4*>(to) = f32x4{v[0] + 0.0f, v[1] + 0.0f, v[2] + 0.0f, v[3] + 0.0f};  // -0 -> +0, as a combine would
+        } else {
+          *reinterpret_cast<bf16x4*>(to) = bf16x4{static_cast<__bf16>(v[0]), static_cast<__bf16>(v[1]),
+                                                  static_cast<__bf16>(v[2]), static_cast<__bf16>(v[3])};
+        }
       }
     }
     wave_fence();
     const int rows_i = min(32, mine - i * 32);
-    for (int q = lane; q < rows_i * kChunksPerRow; q += kWave) {
-      const int rl = q / kChunksPerRow, c = q - rl * kChunksPerRow;
-      if (col_w + c * 8 < a.N) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(image + rl * kImageRow + c * 16);
-        u32x4* to = reinterpret_cast<u32x4*>(out_w + static_cast<size_t>(i * 32 + rl) * a.N + c * 8);
+    const int c = lane % kChunksPerRow;
+    char* const out_b = OUTF32 ? reinterpret_cast<char*>(a.out_f32) : reinterpret_cast<char*>(a.out);
+#pragma unroll
+    for (int p = 0; p < 32 / kRowsPerPass; ++p) {
+      const int rl = p * kRowsPerPass + lane / kChunksPerRow;
+      long row = row_w + i * 32 + rl;
+      bool live = rl < rows_i && col_w + c * kChunk < a.N;
+      if constexpr (ROUTED) {
+        if (a.scatter) {
+          const int to = __shfl(cell, rl, kWave);
+          live = live && to >= 0;
+          row = to;
+        }
+      }
+      if (live) {
+        u32x4 v = *reinterpret_cast<const u32x4*>(image + rl * kImageRow + c * 16);
+        if constexpr (ROUTED && !OUTF32) {
+          if (a.scatter) {  // the combine this store stands for adds the row to zero: -0 becomes +0
+#pragma unroll
+            for (int w = 0; w < 4; ++w) v[w] = plus_zero<BRT_BF16>(v[w]);
+          }
+        }
+        u32x4* const to = reinterpret_cast<u32x4*>(out_b + (static_cast<size_t>(row) * a.N + col_w) * kOutB + c * 16);
         if (a.plain_out) *to = v;
         else stream_out(v, to);
       }
@@ -388,14 +464,14 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   }
 }
 
-template <int ACT>
+template <int ACT, bool ROUTED, bool OUTF32>
 int launch_pingpong(GemmArgs& a, hipStream_t st) {
   a.tiles_n = (a.N + kBN - 1) / kBN;
   // the sum over experts of ceil(M_e / 256) never exceeds P / 256 + E; whole rounds of XCD patches
   const long entries = (static_cast<long>(a.P + kBM - 1) / kBM + a.E) * a.tiles_n;
   const long round = kXcds * kCusPerXcd;
   const long grid = (entries + round - 1) / round * round;
-  auto* fn = &grouped_gemm_pingpong_kernel<ACT>;
+  auto* fn = &grouped_gemm_pingpong_kernel<ACT, ROUTED, OUTF32>;
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(fn), kLdsBytes); rc != BRT_OK) return rc;
   hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(grid)), dim3(kWaves * 64), kLdsBytes, st, a);
   return check_launch("grouped_gemm_pingpong_kernel");
@@ -403,16 +479,21 @@ int launch_pingpong(GemmArgs& a, hipStream_t st) {
 
 }  // namespace
 
-// Shapes the ping-pong tiles take: plain bf16 GEMMs (no gather / scatter, no fp32 output) with K
-// in whole K-steps of 64 and at least two of them.
-bool pingpong_gemm_applies(const GemmArgs& a) {
-  return a.tags == nullptr && a.out_f32 == nullptr && a.gates == nullptr && a.K % kBK == 0 && a.K >= 2 * kBK;
+// Shapes the ping-pong tiles take: K in whole K-steps of 64 and at least two of them; every form
+// but the weighted accumulate.
+bool pingpong_gemm_applies(const GemmArgs& a) { return a.gates == nullptr && a.K % kBK == 0 && a.K >= 2 * kBK; }
+
+template <int ACT>
+int launch_pingpong_form(GemmArgs& a, hipStream_t st) {
+  const bool f32 = a.out_f32 != nullptr;
+  if (a.tags != nullptr) return f32 ? launch_pingpong<ACT, true, true>(a, st) : launch_pingpong<ACT, true, false>(a, st);
+  return f32 ? launch_pingpong<ACT, false, true>(a, st) : launch_pingpong<ACT, false, false>(a, st);
 }
 
 int launch_pingpong_gemm(GemmArgs& a, int act, hipStream_t st) {
-  if (act == BRT_ACT_GELU) return launch_pingpong<BRT_ACT_GELU>(a, st);
-  if (act == BRT_ACT_RELU) return launch_pingpong<BRT_ACT_RELU>(a, st);
-  return launch_pingpong<BRT_ACT_NONE>(a, st);
+  if (act == BRT_ACT_GELU) return launch_pingpong_form<BRT_ACT_GELU>(a, st);
+  if (act == BRT_ACT_RELU) return launch_pingpong_form<BRT_ACT_RELU>(a, st);
+  return launch_pingpong_form<BRT_ACT_NONE>(a, st);
 }
 
 }  // namespace brt

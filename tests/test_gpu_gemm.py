@@ -529,6 +529,68 @@ def test_ping_pong_tiles(loads, K, N):
     run(loads, K, N, act="relu", bias=True, seed=2, slack=300)
 
 
+@pytest.mark.parametrize("T,E,K,N,k,cap,pad", [
+    (12000, 8, 128, 4096, 1, 1500, False),   # overflow dropped, the shortest K loop
+    (12000, 8, 192, 4104, 1, 1700, True),    # padded to the capacity: empty slots, odd K-steps, N tail
+    (13000, 5, 1024, 1000, 1, 4000, False),  # one round of tiles, N tail
+    (7000, 6, 256, 4096, 2, 2400, False),    # two entries per cell (gather only)
+])
+def test_ping_pong_tiles_with_routing_and_fp32_output(T, E, K, N, k, cap, pad):
+    """The routed and fp32-output forms on shapes the 256 x 256 ping-pong kernel takes: the same bits
+    as the plain form on dispatched rows, through the tag matrix and through the row entries, the row
+    tags of every row of a layout longer than the loads, and the fp32 accumulator (whose rounding to
+    bf16 the plain form stores)."""
+    from brainstorm_amd._C import router as c_router
+    from brainstorm_amd.jit import grouped_linear
+    from routing_cases import topk_mask
+
+    mask, _ = topk_mask(T, E, k, seed=T + E)
+    caps = torch.tensor([cap], dtype=torch.int32, device="cuda")
+    rows = E * cap if pad else T * k  # a bound, longer than what the clipped loads add up to
+    tiles = ((rows + 255) // 256 + (E + 1) // 2) * ((N + 255) // 256)
+    assert rows > E * 160 and (tiles >= 512 or 192 <= tiles <= 256), "not a ping-pong shape"
+    g = torch.Generator().manual_seed(E)
+    x = torch.randn(T, K, generator=g).to(torch.bfloat16).cuda()
+    ids, _ = c_router.gate_topk(torch.from_numpy(mask.astype(np.float32)).cuda(), k)
+    loads, _, _, row_entries = c_router.route_by_path(ids, E, caps, pad, rows=rows)
+    P = int(loads.sum())
+    y = c_router.dispatch_by_rows(x, row_entries, k)
+    ws, table = _expert_tables(E, K, N, 6)
+    want = torch.full((rows, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    grouped_linear(y, want, table, None, loads, K, N, "gelu")
+    assert torch.isfinite(want[:P].float()).all()
+
+    def check(got):
+        assert torch.equal(got[:P].view(torch.int16), want[:P].view(torch.int16))
+        assert torch.isnan(got[P:].float()).all()
+
+    got = torch.full_like(want, float("nan"))
+    grouped_linear(x, got, table, None, loads, K, N, "gelu", row_entries=row_entries, entries_per_cell=k, gather=True)
+    check(got)
+    wide = torch.full((rows, N), float("nan"), dtype=torch.float32, device="cuda")
+    grouped_linear(y, wide, table, None, loads, K, N, "gelu")
+    assert torch.equal(wide[:P].to(torch.bfloat16).float(), want[:P].float()) and torch.isnan(wide[P:]).all()
+    if k > 1:
+        return
+    tags, _ = c_router.generate_indices_and_loads(torch.from_numpy(mask).cuda(), caps, pad, False, True)
+    got = torch.full_like(want, float("nan"))
+    row_tags = torch.full((rows,), -7, dtype=torch.int32, device="cuda")
+    grouped_linear(x, got, table, None, loads, K, N, "gelu", tags=tags, gather=True, rows=rows, row_tags_out=row_tags)
+    check(got)
+    assert torch.equal(row_tags, row_entries)  # one entry per cell: the entries are the tags
+    live = row_entries[:P].long()
+    cells = torch.full((T, N), 3.0, device="cuda")
+    cells[live[live > 0] - 1] = want[:P].float()[live > 0]
+    for form in ({"tags": tags}, {"row_entries": row_entries}):
+        out = torch.full((T, N), 3.0, dtype=torch.bfloat16, device="cuda")
+        grouped_linear(y, out, table, None, loads, K, N, "gelu", scatter=True, rows=rows, **form)
+        assert torch.equal(out.float(), cells) and not (out.view(torch.int16) == -32768).any()
+    out = torch.full((T, N), 3.0, dtype=torch.float32, device="cuda")
+    grouped_linear(y, out, table, None, loads, K, N, "gelu", tags=tags, scatter=True, rows=rows)
+    assert torch.equal(out.to(torch.bfloat16).float(), cells)
+    del ws
+
+
 def test_grouped_gemm_random_shapes():
     """Seeded random expert counts, ragged loads (many empty), K and N that are any multiple of
     8, bias and activation at random, slack rows behind the loads."""
