@@ -744,6 +744,7 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
     if (tiles >= 2 * cus || (4 * tiles >= 3 * cus && tiles <= cus))
       return launch_pingpong_gemm(a, act, as_stream(stream));
   }
+  if (skinny_gemm_applies(a)) return launch_skinny_gemm(a, act, as_stream(stream));
   if (out_is_f32) {
     if (act == BRT_ACT_GELU) return launch_f32<BRT_ACT_GELU>(a, as_stream(stream));
     if (act == BRT_ACT_RELU) return launch_f32<BRT_ACT_RELU>(a, as_stream(stream));

@@ -38,18 +38,21 @@ struct GemmArgs {
 bool pingpong_gemm_applies(const GemmArgs& a);
 int launch_pingpong_gemm(GemmArgs& a, int act, hipStream_t st);
 
+// The split-K kernel for few rows per expert and few tiles (grouped_gemm_skinny.hip), every form.
+bool skinny_gemm_applies(const GemmArgs& a);
+int launch_skinny_gemm(GemmArgs& a, int act, hipStream_t st);
+
 // The routed forms: 0-based cell behind row `row` of the dispatched layout (seat `seat`, 0-based, of
 // expert e), -1 for an empty slot.  From the tag matrix a load padded beyond T (capacity above the
 // batch size) names slots that do not exist: they are empty, as in dispatch (route.cu:84-92 bounds
 // the slot by the cell count).
+__device__ __forceinline__ int cell_of_word(const GemmArgs& a, int word) {  // a tag or a row entry, 0 = empty
+  const int cell = a.tag_vector && a.tag_div > 1 ? (word - 1) / a.tag_div : word - 1;
+  return (word >= 1 && cell < a.T) ? cell : -1;
+}
 __device__ __forceinline__ int routed_cell(const GemmArgs& a, int e, int row, int seat) {
-  if (a.tag_vector) {
-    const int entry = a.tags[row];
-    const int cell = a.tag_div > 1 ? (entry - 1) / a.tag_div : entry - 1;
-    return (entry >= 1 && cell < a.T) ? cell : -1;
-  }
-  const int tag = seat < a.T ? a.tags[static_cast<size_t>(seat) * a.E + e] : 0;
-  return (tag >= 1 && tag <= a.T) ? tag - 1 : -1;
+  if (a.tag_vector) return cell_of_word(a, a.tags[row]);
+  return cell_of_word(a, seat < a.T ? a.tags[static_cast<size_t>(seat) * a.E + e] : 0);
 }
 
 // GELU(v) = v * Phi(v) = max(v, 0) - |v| * Phi(-|v|), branch free.  The tail probability is

@@ -591,6 +591,26 @@ def test_ping_pong_tiles_with_routing_and_fp32_output(T, E, K, N, k, cap, pad):
     del ws
 
 
+@pytest.mark.parametrize("K,N", [
+    (8, 8),        # one chunk of one K-step, one chunk of columns
+    (72, 56),      # K tail in the second K-step of the only wavefront that has a slice
+    (192, 72),     # two wavefronts share three K-steps; the second column tile holds 8 columns
+    (776, 1000),   # thirteen K-steps on four wavefronts, K and N tails
+    (1600, 96),    # a long K
+    (4096, 64),
+])
+@pytest.mark.parametrize("loads", [
+    [3, 1, 0, 6],                                # one row block each
+    [1, 31, 32, 33, 0, 63, 64, 65],              # around the row blocks of 32 and 64
+    [(e * 7) % 5 for e in range(130)],           # more than 64 experts, many of them empty
+    [150, 90, 130, 110],                         # blocks of 64 rows
+])
+def test_split_k_tiles(loads, K, N):
+    """Few rows or few tiles: the kernel whose wavefronts share K."""
+    run(loads, K, N)
+    run(loads, K, N, act="gelu", bias=True, seed=1, slack=40)
+
+
 def test_grouped_gemm_random_shapes():
     """Seeded random expert counts, ragged loads (many empty), K and N that are any multiple of
     8, bias and activation at random, slack rows behind the loads."""
