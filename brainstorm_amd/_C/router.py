@@ -3,7 +3,8 @@ pybind11 module of the reference (src/backend/torch/router.cc:479-513,
 python/brt/_C/router.pyi), implemented over the C ABI of ``libbrt_hip.so``.
 
 PyTorch is used for tensor allocation and stream handles only; every device
-computation of the seat-index path is a hand-written HIP kernel.  Work is
+computation of the seat-index path is a hand-written HIP kernel.  Argument checks,
+output allocation and launches live in ``csrc/native.cpp``.  Work is
 enqueued on the current PyTorch stream (the reference uses the default stream,
 router.cc:78; identical when no stream context is active).
 """
@@ -81,20 +82,6 @@ def _device_guard(device: torch.device):
     if device.index is None or device.index == torch._C._cuda_getDevice():
         return _NO_GUARD
     return torch.cuda.device(device)
-
-
-_workspaces = {}
-
-
-def _scan_workspace(device: torch.device, T: int, E: int) -> torch.Tensor:
-    """Scratch memory of the index scan, one per (device, stream), grown on demand."""
-    need = _lib.lib().brt_hip_scan_workspace_bytes(T, E)
-    key = (device.index, _stream())
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(max(need, 1 << 16), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
 
 
 class Route:
@@ -198,43 +185,14 @@ def topk_hot_mask(score: torch.Tensor, top_k: int) -> torch.Tensor:
     (protocol/topk.py:26-31: ``topk`` + ``zeros_like`` + ``scatter_``) in one kernel.  int32
     ``[cells, paths]`` with ones at the ``top_k`` largest scores of every row; NaN ranks
     highest, equal scores go to the lowest path."""
-    _check_on_device(score, "score")
-    if score.dim() != 2:
-        raise RuntimeError("score must be [cells, paths]")
-    if score.dtype not in _DT:
-        raise NotImplementedError("score data type is not supported")
-    T, E = score.shape
-    if not 0 <= top_k <= E:
-        raise RuntimeError("selected index k out of range")  # the message torch.topk gives
-    score = score.contiguous()
-    with _device_guard(score.device):
-        mask = torch.empty((T, E), dtype=torch.int32, device=score.device)
-        _lib.check(_lib.lib().brt_hip_topk_hot_mask(
-            _ptr(score), _ptr(mask), T, E, int(top_k), _DT[score.dtype], _stream()))
-    return mask
+    return _lib.native().topk_hot_mask(score, top_k)
 
 
 def throttle_hotmask(
     hot_mask: torch.Tensor, prefix: torch.Tensor, threshold: torch.Tensor
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """router.cc:15-31.  ``prefix`` is updated in place and returned."""
-    _check_on_device(hot_mask, "hot_mask")
-    _check_on_device(prefix, "prefix")
-    _check_on_device(threshold, "threshold")
-    for t, n in ((hot_mask, "hot_mask"), (prefix, "prefix"), (threshold, "threshold")):
-        _check_int32(t, n)
-    if hot_mask.size(1) != prefix.size(0) or hot_mask.size(1) != threshold.size(0):
-        raise RuntimeError("prefix/threshold must have one entry per path")
-    hot_mask = hot_mask.contiguous()
-    T, E = hot_mask.shape
-    with _device_guard(hot_mask.device):
-        throttled = torch.empty_like(hot_mask)
-        if T > 0:
-            ws = _scan_workspace(hot_mask.device, T, E)
-            _lib.check(_lib.lib().brt_hip_throttle_hotmask(
-                _ptr(hot_mask), _ptr(throttled), _ptr(prefix), _ptr(threshold.contiguous()),
-                T, E, _ptr(ws), ws.numel(), _stream()))
-    return throttled, prefix
+    return _lib.native().throttle_hotmask(hot_mask, prefix, threshold), prefix
 
 
 def generate_route(
@@ -249,32 +207,8 @@ def generate_route(
     caller's promise that no row of ``hot_mask`` has more than one nonzero; dispatch and combine
     calls that receive the route may then use the tag-driven combine (same results, one memory
     round trip less)."""
-    _check_on_device(hot_mask, "hot_mask")
-    _check_int32(hot_mask, "hot_mask")
-    T, E = hot_mask.size(0), hot_mask.size(1)
-    with _device_guard(hot_mask.device):
-        if hot_mask.numel() == 0:  # router.cc:59-62
-            indices = torch.zeros((0, E), dtype=hot_mask.dtype, device=hot_mask.device)
-            loads = torch.zeros((E,), dtype=hot_mask.dtype, device=hot_mask.device)
-            return Route(indices, loads, loads.clone(), is_tag_index, single_path)
-        caps = None
-        n_caps = 0
-        if supported_capacities is not None:
-            _check_on_device(supported_capacities, "supported_capacities")
-            _check_int32(supported_capacities, "supported_capacities")
-            caps = supported_capacities.contiguous()
-            n_caps = caps.size(0)
-        if capacity_padding and n_caps < 1:  # CHECK_GE, location.cu:350,365
-            raise RuntimeError("capacity_padding requires at least one supported capacity")
-        hot_mask = hot_mask.contiguous()
-        indices = torch.empty_like(hot_mask)  # the kernel writes every element in both formats
-        loads_and_counts = torch.empty((2, E), dtype=torch.int32, device=hot_mask.device)
-        loads, counts = loads_and_counts[0], loads_and_counts[1]
-        ws = _scan_workspace(hot_mask.device, T, E)
-        _lib.check(_lib.lib().brt_hip_generate_indices_and_loads(
-            _ptr(hot_mask), _ptr(indices), _ptr(loads), _ptr(counts), T, E, _ptr(caps), n_caps,
-            int(capacity_padding), int(path_wise_padding), int(is_tag_index),
-            _ptr(ws), ws.numel(), _stream()))
+    indices, loads, counts = _lib.native().generate(
+        hot_mask, supported_capacities, capacity_padding, path_wise_padding, is_tag_index)
     return Route(indices, loads, counts, is_tag_index, single_path)
 
 
@@ -356,96 +290,55 @@ def dispatch_with_indices_and_loads(
     _check_on_device(in_data, "in_data")
     _check_on_device(route_indices, "route_indices")
     _check_int32(route_indices, "route_indices")
-    device = in_data.device
-    T = in_data.size(0)
-    E = route_indices.size(1)
-    with _device_guard(device):
-        if T == 0:  # router.cc:150-168
-            shape = list(in_data.shape)
-            if is_1d_routing:
-                shape[0] = 0
-            else:
-                if len(shape) == 2:
-                    shape.append(1)
-                shape[1] = 0
-                shape = shape[1:]
-            out = torch.zeros(shape, dtype=in_data.dtype, device=device)
-            if tag_generating:
-                return [out, torch.zeros((0,), dtype=route_indices.dtype, device=device)]
-            return [out]
-        if in_data.dtype not in _DT:  # TORCH_CHECK_NOT_IMPLEMENTED, router.cc:266
-            raise NotImplementedError("data type is not supported")
-        dtype = _DT[in_data.dtype]
-        cell = in_data.numel() // T
-        if not is_1d_routing:
-            cell //= E
+    if in_data.size(0) == 0:
+        return _dispatch_of_no_cells(in_data, route_indices, tag_generating, is_1d_routing)
+    if in_data.dtype not in _DT:  # TORCH_CHECK_NOT_IMPLEMENTED, router.cc:266
+        raise NotImplementedError("data type is not supported")
+    counts = None
+    hidden_tags = False  # the rows of a single-path route carry their tags to the combine
+    if not is_tag_index:
+        route = _route_for(route, route_indices, loads, "dispatch_with_indices_and_loads")
+        if route is not None and not route.is_tag_index:
+            counts = route.counts
+            hidden_tags = route.single_path and is_1d_routing and not tag_generating
+    _check_int32(loads, "loads")
+    native = _lib.native()
+    dev_loads = loads if loads.is_cuda else loads.to(in_data.device, non_blocking=True)
+    # rows of the dispatched buffer (router.cc:189-202); data dependent, so one
+    # host read of the loads unless a fixed per-path stride was given
+    mpl = 0
+    if max_path_padding:
+        mpl = int(max_path_load) if max_path_load > 0 else max(native.int_list(loads))
+        total = mpl * route_indices.size(1)
+    elif rows is not None:
+        total = int(rows)
+    else:
+        total = sum(native.int_list(loads))
+    # with the true counts the kernel writes every row up to sum(loads) itself; rows past that
+    # (an upper bound was given) have no writer, and their tags start at zero
+    clear = counts is None or (rows is not None and not max_path_padding)
+    # tags None = arange(1, T+1) (router.cc:240-241), generated in the kernel
+    out, new_tags = native.dispatch(in_data, route_indices, dev_loads, counts, gates,
+                                    tags if tag_generating else None, tag_generating or hidden_tags,
+                                    total, mpl, is_1d_routing, is_tag_index, clear)
+    if hidden_tags:
+        route.row_tags, route.row_tags_stride = new_tags, mpl
+    return [out, new_tags] if tag_generating else [out]
 
-        pairing = None
-        if not is_tag_index:
-            pairing = _route_for(route, route_indices, loads, "dispatch_with_indices_and_loads")
-            if pairing is not None and pairing.is_tag_index:
-                pairing = None
-        counts = None if pairing is None else pairing.counts
-        _check_int32(loads, "loads")
-        dev_loads = loads if loads.is_cuda else loads.to(device, non_blocking=True)
 
-        # rows of the dispatched buffer (router.cc:189-202); data dependent, so one
-        # host read of the loads unless a fixed per-path stride was given
-        mpl = 0
-        if max_path_padding:
-            mpl = int(max_path_load) if max_path_load > 0 else int(loads.max().item())
-            total = mpl * E
-        elif rows is not None:
-            total = int(rows)
-        else:
-            total = int(loads.sum().item())
-
-        in_data = in_data.contiguous()
-        route_indices = route_indices.contiguous()
-        shape = list(in_data.shape)
-        if is_1d_routing:
-            shape[0] = total
-        else:
-            if len(shape) == 2:
-                shape.append(1)
-            shape[1] = total
-            shape = shape[1:]
-        # with the true counts the kernel writes every row up to sum(loads) itself; rows past that
-        # (an upper bound was given) have no writer
-        alloc = torch.empty if counts is not None and (rows is None or max_path_padding) else torch.zeros
-        out = alloc(shape, dtype=in_data.dtype, device=device)
-
-        dev_gates = None
-        if gates is not None:
-            if not is_1d_routing:
-                raise RuntimeError("gates are only supported with 1-d routing")  # route.cu:362
-            _check_on_device(gates, "gates")
-            if gates.dtype != in_data.dtype:  # CHECK_EQ, router.cc:226
-                raise RuntimeError("gates must have the dtype of in_data")
-            dev_gates = gates.contiguous()
-
-        old_tags = new_tags = None
-        if tag_generating:
-            if tags is not None:
-                _check_on_device(tags, "tags")
-                if tags.dtype != route_indices.dtype:
-                    raise RuntimeError("tags must have the dtype of route_indices")
-                old_tags = tags.contiguous()
-            # old_tags None = arange(1, T+1) (router.cc:240-241), generated in the kernel
-            new_tags = alloc((total,), dtype=route_indices.dtype, device=device)
-        hidden_tags = (pairing is not None and pairing.single_path and is_1d_routing
-                       and not tag_generating)
-        if hidden_tags and new_tags is None:  # rows past the loads have no writer: their tags start at zero
-            new_tags = alloc((total,), dtype=torch.int32, device=device)
-
-        _lib.check(_lib.lib().brt_hip_dispatch(
-            _ptr(in_data), _ptr(out), _ptr(dev_gates), _ptr(route_indices), _ptr(dev_loads),
-            _ptr(counts), _ptr(old_tags), _ptr(new_tags), T, cell, E, total, mpl,
-            int(is_1d_routing), int(is_tag_index), dtype, _stream()))
-        if hidden_tags:
-            pairing.row_tags, pairing.row_tags_stride = new_tags, mpl
+def _dispatch_of_no_cells(in_data, route_indices, tag_generating, is_1d_routing):
+    # router.cc:150-168
+    shape = list(in_data.shape)
+    if is_1d_routing:
+        shape[0] = 0
+    else:
+        if len(shape) == 2:
+            shape.append(1)
+        shape[1] = 0
+        shape = shape[1:]
+    out = torch.zeros(shape, dtype=in_data.dtype, device=in_data.device)
     if tag_generating:
-        return [out, new_tags]
+        return [out, torch.zeros((0,), dtype=route_indices.dtype, device=in_data.device)]
     return [out]
 
 
@@ -464,54 +357,19 @@ def route_and_dispatch(
     matrix is not read back).  Returns the route and the ``[rows, ...]`` path-major tensor, every
     row of it written (zeros where no cell owns the row); bit-identical to the two calls, which it
     makes itself for the shapes the fused kernel does not take."""
-    _check_on_device(in_data, "in_data")
-    _check_on_device(hot_mask, "hot_mask")
-    _check_int32(hot_mask, "hot_mask")
-    T, E = hot_mask.size(0), hot_mask.size(1)
-    if in_data.size(0) != T:
-        raise RuntimeError("in_data and hot_mask must have one row per cell")
     rows = int(rows)
-    n_caps = 0 if supported_capacities is None else supported_capacities.size(0)
-    cell_bytes = (in_data.numel() // T) * in_data.element_size() if T > 0 else 0
-    lib = _lib.lib()
-    # (a contiguous view whose storage offset breaks the 16-byte alignment takes the two calls)
-    fused = (T > 0 and in_data.dtype in _DT and in_data.data_ptr() % 16 == 0
-             and lib.brt_hip_route_and_dispatch_supported(
-        T, E, cell_bytes, n_caps, int(bool(path_wise_padding and capacity_padding))) == 1)
-    if not fused:
+    done = _lib.native().route_and_dispatch(in_data, hot_mask, rows, supported_capacities, capacity_padding,
+                                            path_wise_padding, single_path)
+    if done is None:  # a shape the fused kernel does not take
         route = generate_route(hot_mask, supported_capacities, capacity_padding, path_wise_padding,
                                False, single_path)
         out = dispatch_with_indices_and_loads(in_data, route.indices, route.loads, route=route,
                                               rows=rows)[0]
         return route, out
-    with _device_guard(in_data.device):
-        caps = None
-        if supported_capacities is not None:
-            _check_on_device(supported_capacities, "supported_capacities")
-            _check_int32(supported_capacities, "supported_capacities")
-            caps = supported_capacities.contiguous()
-        if capacity_padding and n_caps < 1:
-            raise RuntimeError("capacity_padding requires at least one supported capacity")
-        hot_mask = hot_mask.contiguous()
-        in_data = in_data.contiguous()
-        indices = torch.empty_like(hot_mask)
-        loads_and_counts = torch.empty((2, E), dtype=torch.int32, device=hot_mask.device)
-        loads, counts = loads_and_counts[0], loads_and_counts[1]
-        out = torch.empty([rows] + list(in_data.shape[1:]), dtype=in_data.dtype, device=in_data.device)
-        row_tags = torch.empty((rows,), dtype=torch.int32, device=in_data.device) if single_path else None
-        need = lib.brt_hip_route_and_dispatch_workspace_bytes(T, E, cell_bytes)
-        key = (in_data.device.index, _stream())
-        ws = _workspaces.get(key)
-        if ws is None or ws.numel() < need:
-            ws = torch.empty(max(need, 1 << 16), dtype=torch.uint8, device=in_data.device)
-            _workspaces[key] = ws
-        _lib.check(lib.brt_hip_route_and_dispatch(
-            _ptr(hot_mask), _ptr(in_data), _ptr(out), _ptr(indices), _ptr(loads), _ptr(counts),
-            _ptr(row_tags), T, E, rows, cell_bytes, _ptr(caps), n_caps, int(capacity_padding),
-            int(path_wise_padding), _ptr(ws), ws.numel(), _stream()))
-        route = Route(indices, loads, counts, False, single_path)
-        if single_path:
-            route.row_tags, route.row_tags_stride = row_tags, 0
+    indices, loads, counts, out, row_tags = done
+    route = Route(indices, loads, counts, False, single_path)
+    if single_path:
+        route.row_tags, route.row_tags_stride = row_tags, 0
     return route, out
 
 
@@ -542,29 +400,7 @@ def combine_by_row_tags(in_data: torch.Tensor, row_tags: torch.Tensor, cells: in
     route.cu:208-282): ``out[row_tags[p] - 1] = in_data[p]`` for every tagged row.  ``out_data``
     is updated in place (cells without a row keep their values); without it the result starts
     from zeros."""
-    _check_on_device(in_data, "in_data")
-    if in_data.dtype not in _DT:
-        raise NotImplementedError("data type is not supported")
-    P = in_data.size(0)
-    in_data = in_data.contiguous()
-    cell = in_data.numel() // P if P > 0 else 0
-    with _device_guard(in_data.device):
-        if out_data is not None:
-            if not out_data.is_contiguous():
-                raise RuntimeError("out_data must be contiguous (it is updated in place)")
-            result = out_data
-        else:
-            shape = list(in_data.shape)
-            shape[0] = cells
-            result = torch.zeros(shape, dtype=out_dtype or in_data.dtype, device=in_data.device)
-        if result.dtype not in _DT or result.numel() != cells * cell:
-            raise RuntimeError("out_data does not match [cell_num, *cell_shape]")
-        if row_tags.numel() < P:
-            raise RuntimeError("one tag per row is needed")
-        _lib.check(_lib.lib().brt_hip_combine_by_tags(
-            _ptr(in_data), _ptr(result), _ptr(row_tags), P, cell, cells, _DT[in_data.dtype],
-            _DT[result.dtype], _stream()))
-    return result
+    return _lib.native().combine_by_row_tags(in_data, row_tags, cells, out_data, out_dtype)
 
 
 def split_fused_cells_to_paths(
@@ -674,72 +510,30 @@ def combine_with_indices_and_loads(
     """
     _check_on_device(in_data, "in_data")
     _check_on_device(route_indices, "route_indices")
-    device = in_data.device
     T = route_indices.size(0)
-    with _device_guard(device):
+    if T <= 1:
         if T == 0:  # router.cc:386-397
             if not is_tag_index:
                 return [out_data if out_data is not None else torch.empty_like(in_data)]
             return [torch.empty_like(in_data), torch.empty_like(tags), torch.zeros_like(tags)]
-        if T == 1:  # router.cc:402-412
-            if not is_tag_index:
-                return [out_data + in_data if out_data is not None else in_data]
-            return [in_data, tags, torch.ones_like(tags)]
-
-        if is_tag_index:
+        if not is_tag_index:  # router.cc:402-412
+            return [out_data + in_data if out_data is not None else in_data]
+        return [in_data, tags, torch.ones_like(tags)]
+    if is_tag_index:
+        with _device_guard(in_data.device):
             return _combine_with_tags(in_data, route_indices, out_data, ever_padded, tags)
-
-        if loads is None:
-            raise RuntimeError("seat-index combine needs loads")
-        _check_int32(route_indices, "route_indices")
-        _check_int32(loads, "loads")
-        if in_data.dtype not in _DT:
-            raise NotImplementedError("data type is not supported")
-        E = route_indices.size(1)
-        dev_loads = loads.to(device, non_blocking=True).contiguous()
-        in_data = in_data.contiguous()
-        route_indices = route_indices.contiguous()
+    if loads is None:
+        raise RuntimeError("seat-index combine needs loads")
+    # single-path routes whose rows still carry the tags of the paired dispatch: scatter form
+    route = _route_for(route, route_indices, loads, "combine_with_indices_and_loads")
+    row_tags = None
+    if route is not None and route.single_path and route.row_tags is not None:
         P = in_data.size(0)
-        cell = in_data.numel() // P if P > 0 else 0
-        mpl = P // E if max_path_padding else 0  # router.cc:427-430
-        dev_gates = None
-        gate_dtype = _lib.F32
-        if gates is not None:
-            _check_on_device(gates, "gates")
-            if gates.dtype not in _DT:
-                raise NotImplementedError("gate data type is not supported")
-            dev_gates = gates.contiguous()
-            gate_dtype = _DT[gates.dtype]
-        if out_data is not None:
-            _check_on_device(out_data, "out_data")
-            if not out_data.is_contiguous():
-                raise RuntimeError("out_data must be contiguous (it is updated in place)")
-            result = out_data
-            residual = 1
-        else:
-            shape = list(in_data.shape)
-            shape[0] = T
-            result = torch.empty(shape, dtype=out_dtype or in_data.dtype, device=device)
-            residual = 0
-        if result.dtype not in _DT or result.numel() != T * cell:
-            raise RuntimeError("out_data does not match [cell_num, *cell_shape]")
-        # single-path routes whose rows still carry the tags of the paired dispatch:
-        # scatter form (identical rows; cells without a row keep the residual)
-        pairing = _route_for(route, route_indices, loads, "combine_with_indices_and_loads")
-        if (residual and dev_gates is None and pairing is not None and pairing.single_path
-                and pairing.row_tags is not None and pairing.row_tags.numel() == P
-                and pairing.row_tags_stride == mpl
-                and (cell * in_data.element_size()) % 16 == 0
-                and (result.dtype == in_data.dtype or result.dtype == torch.float32)):
-            _lib.check(_lib.lib().brt_hip_combine_by_tags(
-                _ptr(in_data), _ptr(result), _ptr(pairing.row_tags), P, cell, T,
-                _DT[in_data.dtype], _DT[result.dtype], _stream()))
-            return [result]
-        _lib.check(_lib.lib().brt_hip_combine(
-            _ptr(in_data), _ptr(result), _ptr(dev_gates), _ptr(route_indices), _ptr(dev_loads),
-            T, cell, E, P, mpl, residual, _DT[in_data.dtype], _DT[result.dtype], gate_dtype,
-            _stream()))
-        return [result]
+        mpl = P // route_indices.size(1) if max_path_padding else 0  # router.cc:427-430
+        if route.row_tags.size(0) == P and route.row_tags_stride == mpl:
+            row_tags = route.row_tags
+    return [_lib.native().combine(in_data, route_indices, loads, gates, out_data, out_dtype,
+                                  max_path_padding, row_tags)]
 
 
 def _combine_with_tags(in_data, route_indices, out_data, ever_padded, tags):
@@ -807,27 +601,7 @@ def gate_topk(score: torch.Tensor, top_k: int, softmax: bool = False,
     fp32, or with ``softmax`` their softmax over the row (the router probabilities of
     benchmark/switch_moe/switch_transformer.py:240-253).  One kernel for what the reference does
     with ``softmax`` + ``topk`` / ``argmax`` + ``zeros`` + ``scatter_`` (protocol/topk.py:26-31)."""
-    _check_on_device(score, "score")
-    if score.dim() != 2:
-        raise RuntimeError("score must be [cells, paths]")
-    if score.dtype not in _DT:
-        raise NotImplementedError("score data type is not supported")
-    T, E = score.shape
-    if not 0 <= top_k <= E:
-        raise RuntimeError("selected index k out of range")
-    score = score.contiguous()
-    with _device_guard(score.device):
-        ids = torch.empty((T, top_k), dtype=torch.int32, device=score.device)
-        weights = torch.empty((T, top_k), dtype=torch.float32, device=score.device)
-        mask = torch.empty((T, E), dtype=torch.int32, device=score.device) if hot_mask else None
-        if top_k > 0 or hot_mask:
-            _lib.check(_lib.lib().brt_hip_gate_topk(
-                _ptr(score), T, E, int(top_k), _DT[score.dtype], int(bool(softmax)), _ptr(ids),
-                _ptr(weights), _ptr(mask), _stream()))
-    return (ids, weights, mask) if hot_mask else (ids, weights)
-
-
-_route_workspaces = {}
+    return _lib.native().gate_topk(score, top_k, softmax, hot_mask)
 
 
 def route_by_path(
@@ -845,36 +619,8 @@ def route_by_path(
     ``path_num * max_path_load`` when padding every path to ``max_path_load``, else by default
     ``cells * k``, which always holds the ``sum(loads)`` rows of a route without capacity padding
     (no read-back of the loads is needed to size it; rows behind the last path are padding)."""
-    _check_on_device(path_ids, "path_ids")
-    _check_int32(path_ids, "path_ids")
-    if path_ids.dim() != 2:
-        raise RuntimeError("path_ids must be [cells, k]")
-    path_ids = path_ids.contiguous()
-    T, k = path_ids.shape
-    E = int(path_num)
-    caps = None
-    if supported_capacities is not None:
-        _check_int32(supported_capacities, "supported_capacities")
-        caps = supported_capacities.to(path_ids.device).contiguous()
-    if rows is None:
-        rows = E * int(max_path_load) if max_path_load else T * k
-    with _device_guard(path_ids.device):
-        dev = path_ids.device
-        loads_counts = torch.empty((2, E), dtype=torch.int32, device=dev)
-        seat_rows = torch.empty((T, k), dtype=torch.int32, device=dev)
-        row_entries = torch.empty((rows,), dtype=torch.int32, device=dev)
-        need = _lib.lib().brt_hip_route_by_path_workspace_bytes(T, k, E)
-        key = (dev.index, _stream())
-        ws = _route_workspaces.get(key)
-        if ws is None or ws.numel() < need:
-            ws = torch.empty(max(need, 1 << 16), dtype=torch.uint8, device=dev)
-            _route_workspaces[key] = ws
-        _lib.check(_lib.lib().brt_hip_route_by_path(
-            _ptr(path_ids), T, k, E, _ptr(caps), 0 if caps is None else caps.numel(),
-            int(capacity_padding), int(path_wise_padding), int(max_path_load),
-            _ptr(loads_counts[0]), _ptr(loads_counts[1]), _ptr(seat_rows), _ptr(row_entries),
-            int(rows), _ptr(ws), ws.numel(), _stream()))
-    return loads_counts[0], loads_counts[1], seat_rows, row_entries
+    return _lib.native().route_by_path(path_ids, path_num, supported_capacities, capacity_padding,
+                                       path_wise_padding, max_path_load, rows)
 
 
 def dispatch_by_rows(in_data: torch.Tensor, row_entries: torch.Tensor, k: int,
@@ -883,29 +629,7 @@ def dispatch_by_rows(in_data: torch.Tensor, row_entries: torch.Tensor, k: int,
     """``out[r] = in_data[(row_entries[r]-1) // k]`` (times ``weights.view(-1)[row_entries[r]-1]``,
     rounded once), zero rows where ``row_entries[r] == 0``: what ``dispatch_with_indices_and_loads``
     (router.cc:131-273) writes for the same route, every row written by the kernel."""
-    _check_on_device(in_data, "in_data")
-    _check_on_device(row_entries, "row_entries")
-    _check_int32(row_entries, "row_entries")
-    if in_data.dtype not in _DT:
-        raise NotImplementedError("in_data data type is not supported")
-    in_data = in_data.contiguous()
-    T = in_data.size(0)
-    cell = in_data.numel() // T if T > 0 else 0
-    P = row_entries.numel()
-    if weights is not None:
-        if weights.dtype != torch.float32 or weights.numel() != T * k:
-            raise RuntimeError("weights must be fp32 [cells, k]")
-        weights = weights.contiguous()
-    with _device_guard(in_data.device):
-        if out is None:
-            out = torch.empty((P,) + tuple(in_data.shape[1:]), dtype=in_data.dtype, device=in_data.device)
-        elif (out.dtype != in_data.dtype or not out.is_contiguous() or out.numel() != P * cell
-              or out.device != in_data.device):
-            raise RuntimeError("out must be a contiguous [rows, *cell_shape] tensor of the input's type")
-        _lib.check(_lib.lib().brt_hip_dispatch_by_rows(
-            _ptr(in_data), _ptr(out), _ptr(weights), _ptr(row_entries.contiguous()), P, T, int(k),
-            cell, _DT[in_data.dtype], _stream()))
-    return out
+    return _lib.native().dispatch_by_rows(in_data, row_entries, k, weights, out)
 
 
 def combine_by_rows(in_data: torch.Tensor, path_ids: torch.Tensor, seat_rows: torch.Tensor,
@@ -915,34 +639,4 @@ def combine_by_rows(in_data: torch.Tensor, path_ids: torch.Tensor, seat_rows: to
     in ascending path id, fp32 from zero: the result of ``combine_with_indices_and_loads``
     (router.cc:372-473) for the same route, bit for bit.  With ``out_data`` the result is
     written in place and cells without a row keep their value (the residual convention)."""
-    _check_on_device(in_data, "in_data")
-    for t, n in ((path_ids, "path_ids"), (seat_rows, "seat_rows")):
-        _check_on_device(t, n)
-        _check_int32(t, n)
-    if in_data.dtype not in _DT:
-        raise NotImplementedError("in_data data type is not supported")
-    if path_ids.shape != seat_rows.shape or path_ids.dim() != 2:
-        raise RuntimeError("path_ids and seat_rows must both be [cells, k]")
-    in_data = in_data.contiguous()
-    T, k = path_ids.shape
-    P = in_data.size(0)
-    cell = in_data.numel() // P if P > 0 else (out_data.numel() // T if out_data is not None and T > 0 else 0)
-    if weights is not None:
-        if weights.dtype != torch.float32 or weights.numel() != T * k:
-            raise RuntimeError("weights must be fp32 [cells, k]")
-        weights = weights.contiguous()
-    with _device_guard(in_data.device):
-        if out_data is not None:
-            if not out_data.is_contiguous() or out_data.numel() != T * cell:
-                raise RuntimeError("out_data must be a contiguous [cells, ...] tensor")
-            out = out_data
-        else:
-            out = torch.empty((T,) + tuple(in_data.shape[1:]), dtype=out_dtype or in_data.dtype,
-                              device=in_data.device)
-        if out.dtype not in _DT or (out.dtype != in_data.dtype and out.dtype != torch.float32):
-            raise NotImplementedError("output data type is not supported")
-        _lib.check(_lib.lib().brt_hip_combine_by_rows(
-            _ptr(in_data), _ptr(out), _ptr(weights), _ptr(path_ids.contiguous()),
-            _ptr(seat_rows.contiguous()), T, k, cell, P, int(out_data is not None),
-            _DT[in_data.dtype], _DT[out.dtype], _stream()))
-    return out
+    return _lib.native().combine_by_rows(in_data, path_ids, seat_rows, weights, out_data, out_dtype)

@@ -17,6 +17,7 @@ import torch  # noqa: F401
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libbrt_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "lib", "brt_native.so")
 CSRC_DIR = os.path.join(_HERE, "csrc")
 
 F32, F16, BF16 = 0, 1, 2
@@ -168,15 +169,36 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The host side of the ops (``csrc/native.cpp``): checks, output allocation and the call into
+    ``libbrt_hip.so`` for tensors.  The entry points take positional arguments only."""
+    global _native
+    if _native is None:
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `make -C {CSRC_DIR}`; "
+                               "there is no CPU fallback for the routing ops")
+        import importlib.machinery
+        import importlib.util
+
+        lib()
+        loader = importlib.machinery.ExtensionFileLoader("brt_native", NATIVE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("brt_native", loader))
+        loader.exec_module(module)
+        _native = module
+    return _native
+
+
 _calls = 0
 
 
 def call_count() -> int:
-    """Calls into the library that queued device work and were checked with :func:`check` since
-    the process started (every such call is one kernel launch, except index generation, the
+    """Calls into the library that queued device work since the process started (every such call is one kernel launch, except index generation, the
     compact route and the tag-index gather, which are two).  Tests use the difference around a
     layer to pin how many launches a route costs."""
-    return _calls
+    return _calls + (_native.calls() if _native is not None else 0)
 
 
 def check(code: int) -> None:

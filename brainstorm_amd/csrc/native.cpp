@@ -1,0 +1,584 @@
+// Host side of the routing ops and the grouped GEMM: argument checks, output allocation and the call
+// into libbrt_hip.so, for tensors handed over by Python (brainstorm_amd/_C/router.py and
+// brainstorm_amd/jit are thin wrappers around these functions and document them).
+//
+// Why native: a routed layer is 4 to 7 launches of 2.7 us of host time each, and the same work in
+// Python (a torch.empty is 1.7 us there and 0.4 us here, a foreign call with 17 converted arguments
+// 3 us, every check 0.1 us) took longer than most layers take on the device.  Positional arguments
+// only, no argument parser.
+//
+// Nothing is kept between calls: outputs and scratch memory come from torch's caching allocator, which
+// knows the stream.  Errors are raised as the exceptions the reference's binding raises
+// (src/backend/torch/torch.h:16-21, router.cc:266).
+#include <Python.h>
+
+#include <ATen/core/CachingHostAllocator.h>
+#include <ATen/core/Tensor.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/zeros.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <stdexcept>
+#include <string>
+
+#include "brt_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+unsigned long long g_calls = 0;  // calls into the library that queued device work (under the GIL)
+
+// An error with the Python type it is raised as.
+struct Raised : std::runtime_error {
+  PyObject* type;
+  Raised(PyObject* t, const std::string& what) : std::runtime_error(what), type(t) {}
+};
+[[noreturn]] void runtime_error(const std::string& what) { throw Raised(PyExc_RuntimeError, what); }
+[[noreturn]] void not_implemented(const std::string& what) { throw Raised(PyExc_NotImplementedError, what); }
+
+void check(int code) {
+  ++g_calls;
+  if (code == BRT_OK) return;
+  const std::string msg = brt_hip_last_error();
+  if (code == BRT_E_UNSUPPORTED) not_implemented(msg);
+  runtime_error("libbrt_hip error " + std::to_string(code) + ": " + msg);
+}
+
+// ---- arguments -----------------------------------------------------------------------------------
+struct Args {
+  PyObject* const* v;
+  Py_ssize_t n;
+
+  Tensor tensor(Py_ssize_t i) const {
+    PyObject* const o = v[i];
+    if (!THPVariable_CheckExact(o)) {
+      if (!THPVariable_Check(o)) throw Raised(PyExc_TypeError, "a tensor is expected");
+      // a subclass may stand for rows that are not there yet: asking for the address fills them
+      PyObject* const address = PyObject_CallMethod(o, "data_ptr", nullptr);
+      if (address == nullptr) throw Raised(nullptr, "");
+      Py_DECREF(address);
+    }
+    return THPVariable_Unpack(o);
+  }
+  bool none(Py_ssize_t i) const { return v[i] == Py_None; }
+  Tensor tensor_or_none(Py_ssize_t i) const { return none(i) ? Tensor() : tensor(i); }
+  long integer(Py_ssize_t i) const {
+    const long r = PyLong_AsLong(v[i]);
+    if (r == -1 && PyErr_Occurred()) throw Raised(nullptr, "");
+    return r;
+  }
+  bool flag(Py_ssize_t i) const {
+    const int r = PyObject_IsTrue(v[i]);
+    if (r < 0) throw Raised(nullptr, "");
+    return r != 0;
+  }
+  bool dtype(Py_ssize_t i, at::ScalarType* out) const {
+    if (none(i)) return false;
+    if (!THPDtype_Check(v[i])) throw Raised(PyExc_TypeError, "a dtype is expected");
+    *out = reinterpret_cast<THPDtype*>(v[i])->scalar_type;
+    return true;
+  }
+};
+
+PyObject* wrap(Tensor t) { return THPVariable_Wrap(std::move(t)); }
+PyObject* none() { Py_RETURN_NONE; }
+template <typename... T>
+PyObject* tuple(T... items) {
+  PyObject* const made[] = {items...};
+  PyObject* const t = PyTuple_New(sizeof...(items));
+  for (size_t i = 0; i < sizeof...(items); ++i) PyTuple_SET_ITEM(t, i, made[i]);
+  return t;
+}
+
+void on_device(const Tensor& t, const char* name) {
+  if (!t.is_cuda()) runtime_error(std::string(name) + " must be a CUDA tensor");
+}
+void int32(const Tensor& t, const char* name) {
+  if (t.scalar_type() != at::kInt)
+    runtime_error(std::string(name) + " must be an int32 tensor, got " + c10::toString(t.scalar_type()));
+}
+int code_of(at::ScalarType t) {  // BRT_F32 / BRT_F16 / BRT_BF16, -1 for anything else
+  return t == at::kFloat ? BRT_F32 : t == at::kHalf ? BRT_F16 : t == at::kBFloat16 ? BRT_BF16 : -1;
+}
+int data_type(const Tensor& t, const char* what) {
+  const int c = code_of(t.scalar_type());
+  if (c < 0) not_implemented(std::string(what) + " is not supported");
+  return c;
+}
+Tensor dense(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+int32_t* iptr(const Tensor& t) { return static_cast<int32_t*>(ptr(t)); }
+float* fptr(const Tensor& t) { return static_cast<float*>(ptr(t)); }
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+Tensor empty(at::IntArrayRef shape, at::ScalarType type, const Tensor& like) {
+  return Tensor(at::detail::empty_cuda(shape, type, like.device(), std::nullopt));
+}
+Tensor zeros(at::IntArrayRef shape, at::ScalarType type, const Tensor& like) {
+  return at::zeros(shape, at::TensorOptions().dtype(type).device(like.device()));
+}
+Tensor scratch(size_t bytes, const Tensor& like) {
+  return empty({static_cast<int64_t>(bytes < 16 ? 16 : bytes)}, at::kByte, like);
+}
+at::DimVector rows_of(const Tensor& t, int64_t rows) {  // the shape of t with another first dimension
+  at::DimVector s(t.sizes().begin(), t.sizes().end());
+  s[0] = rows;
+  return s;
+}
+
+// The menu of capacities of an index generation.
+struct Caps {
+  Tensor t;
+  int n = 0;
+  Caps(const Tensor& given, bool padding) {
+    if (given.defined()) {
+      on_device(given, "supported_capacities");
+      int32(given, "supported_capacities");
+      t = dense(given);
+      n = static_cast<int>(t.size(0));
+    }
+    if (padding && n < 1) runtime_error("capacity_padding requires at least one supported capacity");  // location.cu:350,365
+  }
+};
+
+// ---- gate ------------------------------------------------------------------------------------------
+Tensor scores(const Tensor& given, long top_k) {
+  on_device(given, "score");
+  if (given.dim() != 2) runtime_error("score must be [cells, paths]");
+  data_type(given, "score data type");
+  if (top_k < 0 || top_k > given.size(1)) runtime_error("selected index k out of range");  // the message torch.topk gives
+  return dense(given);
+}
+
+PyObject* topk_hot_mask(const Args& a) {
+  const long k = a.integer(1);
+  const Tensor score = scores(a.tensor(0), k);
+  const c10::DeviceGuard guard(score.device());
+  Tensor mask = empty(score.sizes(), at::kInt, score);
+  check(brt_hip_topk_hot_mask(ptr(score), iptr(mask), score.size(0), score.size(1), k, code_of(score.scalar_type()),
+                              stream_of(score)));
+  return wrap(mask);
+}
+
+PyObject* gate_topk(const Args& a) {  // score, k, softmax, hot_mask
+  const long k = a.integer(1);
+  const Tensor score = scores(a.tensor(0), k);
+  const c10::DeviceGuard guard(score.device());
+  const int64_t T = score.size(0);
+  Tensor ids = empty({T, k}, at::kInt, score), weights = empty({T, k}, at::kFloat, score), mask;
+  if (a.flag(3)) mask = empty(score.sizes(), at::kInt, score);
+  if (k > 0 || mask.defined())
+    check(brt_hip_gate_topk(ptr(score), T, score.size(1), k, code_of(score.scalar_type()), a.flag(2), iptr(ids),
+                            fptr(weights), iptr(mask), stream_of(score)));
+  return mask.defined() ? tuple(wrap(ids), wrap(weights), wrap(mask)) : tuple(wrap(ids), wrap(weights));
+}
+
+// ---- index generation --------------------------------------------------------------------------------
+PyObject* throttle_hotmask(const Args& a) {  // hot_mask, prefix (updated in place), threshold
+  const Tensor given = a.tensor(0), prefix = a.tensor(1), threshold = a.tensor(2);
+  on_device(given, "hot_mask"), on_device(prefix, "prefix"), on_device(threshold, "threshold");
+  int32(given, "hot_mask"), int32(prefix, "prefix"), int32(threshold, "threshold");
+  if (given.size(1) != prefix.size(0) || given.size(1) != threshold.size(0))
+    runtime_error("prefix/threshold must have one entry per path");
+  const Tensor mask = dense(given);
+  const c10::DeviceGuard guard(mask.device());
+  const int T = mask.size(0), E = mask.size(1);
+  Tensor out = empty(mask.sizes(), at::kInt, mask);
+  if (T > 0) {
+    const size_t bytes = brt_hip_scan_workspace_bytes(T, E);
+    const Tensor ws = scratch(bytes, mask), thr = dense(threshold);
+    check(brt_hip_throttle_hotmask(iptr(mask), iptr(out), iptr(prefix), iptr(thr), T, E, ptr(ws), ws.numel(),
+                                   stream_of(mask)));
+  }
+  return wrap(out);
+}
+
+PyObject* generate(const Args& a) {  // hot_mask, capacities, capacity_padding, path_wise_padding, is_tag_index
+  const Tensor given = a.tensor(0);
+  on_device(given, "hot_mask");
+  int32(given, "hot_mask");
+  const c10::DeviceGuard guard(given.device());
+  const int64_t T = given.size(0), E = given.size(1);
+  if (given.numel() == 0) {  // router.cc:59-62
+    Tensor both = zeros({2, E}, at::kInt, given);
+    return tuple(wrap(zeros({0, E}, at::kInt, given)), wrap(both.select(0, 0)), wrap(both.select(0, 1)));
+  }
+  const bool cap_pad = a.flag(2), path_pad = a.flag(3), tag = a.flag(4);
+  const Caps caps(a.tensor_or_none(1), cap_pad);
+  const Tensor mask = dense(given);
+  Tensor indices = empty(mask.sizes(), at::kInt, mask);  // the kernel writes every element in both formats
+  Tensor loads = empty({E}, at::kInt, mask), counts = empty({E}, at::kInt, mask);
+  const Tensor ws = scratch(brt_hip_scan_workspace_bytes(T, E), mask);
+  check(brt_hip_generate_indices_and_loads(iptr(mask), iptr(indices), iptr(loads), iptr(counts), T, E, iptr(caps.t),
+                                           caps.n, cap_pad, path_pad, tag, ptr(ws), ws.numel(), stream_of(mask)));
+  return tuple(wrap(indices), wrap(loads), wrap(counts));
+}
+
+// in_data, hot_mask, rows, capacities, capacity_padding, path_wise_padding, row_tags wanted
+// -> (indices, loads, counts, out, row_tags), or None where the fused kernel does not take the shape
+PyObject* route_and_dispatch(const Args& a) {
+  const Tensor cells = a.tensor(0), given = a.tensor(1);
+  on_device(cells, "in_data"), on_device(given, "hot_mask");
+  int32(given, "hot_mask");
+  const int64_t T = given.size(0), E = given.size(1), rows = a.integer(2);
+  if (cells.size(0) != T) runtime_error("in_data and hot_mask must have one row per cell");
+  const bool cap_pad = a.flag(4), path_pad = a.flag(5), want_tags = a.flag(6);
+  const Tensor menu = a.tensor_or_none(3);
+  const size_t cell_bytes = T > 0 ? cells.numel() / T * cells.element_size() : 0;
+  // (a contiguous view whose storage offset breaks the 16-byte alignment takes the two calls)
+  if (T == 0 || code_of(cells.scalar_type()) < 0 || reinterpret_cast<uintptr_t>(cells.data_ptr()) % 16 != 0 ||
+      brt_hip_route_and_dispatch_supported(T, E, cell_bytes, menu.defined() ? menu.size(0) : 0, path_pad && cap_pad) != 1)
+    return none();
+  const c10::DeviceGuard guard(cells.device());
+  const Caps caps(menu, cap_pad);
+  const Tensor mask = dense(given), in = dense(cells);
+  Tensor indices = empty(mask.sizes(), at::kInt, mask);
+  Tensor loads = empty({E}, at::kInt, mask), counts = empty({E}, at::kInt, mask);
+  Tensor out = empty(rows_of(in, rows), in.scalar_type(), in), tags;
+  if (want_tags) tags = empty({rows}, at::kInt, in);
+  const Tensor ws = scratch(brt_hip_route_and_dispatch_workspace_bytes(T, E, cell_bytes), in);
+  check(brt_hip_route_and_dispatch(iptr(mask), ptr(in), ptr(out), iptr(indices), iptr(loads), iptr(counts), iptr(tags), T,
+                                   E, rows, cell_bytes, iptr(caps.t), caps.n, cap_pad, path_pad, ptr(ws), ws.numel(),
+                                   stream_of(in)));
+  return tuple(wrap(indices), wrap(loads), wrap(counts), wrap(out), want_tags ? wrap(tags) : none());
+}
+
+PyObject* route_by_path(const Args& a) {  // path_ids, paths, capacities, cap_pad, path_pad, max_path_load, rows or None
+  const Tensor given = a.tensor(0);
+  on_device(given, "path_ids");
+  int32(given, "path_ids");
+  if (given.dim() != 2) runtime_error("path_ids must be [cells, k]");
+  const Tensor ids = dense(given);
+  const int64_t T = ids.size(0), k = ids.size(1), E = a.integer(1), mpl = a.integer(5);
+  const int64_t rows = !a.none(6) ? a.integer(6) : mpl ? E * mpl : T * k;
+  const c10::DeviceGuard guard(ids.device());
+  Tensor caps = a.tensor_or_none(2);
+  if (caps.defined()) {
+    int32(caps, "supported_capacities");
+    caps = dense(caps.device() == ids.device() ? caps : caps.to(ids.device()));
+  }
+  Tensor loads = empty({E}, at::kInt, ids), counts = empty({E}, at::kInt, ids);
+  Tensor seat_rows = empty({T, k}, at::kInt, ids), row_entries = empty({rows}, at::kInt, ids);
+  const Tensor ws = scratch(brt_hip_route_by_path_workspace_bytes(T, k, E), ids);
+  check(brt_hip_route_by_path(iptr(ids), T, k, E, iptr(caps), caps.defined() ? caps.numel() : 0, a.flag(3), a.flag(4), mpl,
+                              iptr(loads), iptr(counts), iptr(seat_rows), iptr(row_entries), rows, ptr(ws), ws.numel(),
+                              stream_of(ids)));
+  return tuple(wrap(loads), wrap(counts), wrap(seat_rows), wrap(row_entries));
+}
+
+// ---- rows --------------------------------------------------------------------------------------------
+// in_data, route_indices, loads (on the device), counts, gates, old_tags, tags wanted, rows of the output,
+// max_path_load, is_1d_routing, is_tag_index, outputs pre-zeroed -> (out, new_tags or None)
+PyObject* dispatch(const Args& a) {
+  const Tensor given = a.tensor(0), route = dense(a.tensor(1)), loads = a.tensor(2), counts = a.tensor_or_none(3);
+  Tensor gates = a.tensor_or_none(4), old_tags = a.tensor_or_none(5);
+  const bool want_tags = a.flag(6), one_d = a.flag(9), tag_index = a.flag(10), clear = a.flag(11);
+  const int64_t total = a.integer(7), mpl = a.integer(8);
+  const Tensor in = dense(given);
+  const c10::DeviceGuard guard(in.device());
+  const int64_t T = in.size(0), E = route.size(1);
+  int64_t cell = in.numel() / T;
+  at::DimVector shape(in.sizes().begin(), in.sizes().end());
+  if (one_d) {
+    shape[0] = total;
+  } else {
+    cell /= E;
+    if (shape.size() == 2) shape.push_back(1);
+    shape[1] = total;
+    shape.erase(shape.begin());
+  }
+  Tensor out = clear ? zeros(shape, in.scalar_type(), in) : empty(shape, in.scalar_type(), in);
+  if (gates.defined()) {
+    if (!one_d) runtime_error("gates are only supported with 1-d routing");  // route.cu:362
+    on_device(gates, "gates");
+    if (gates.scalar_type() != in.scalar_type()) runtime_error("gates must have the dtype of in_data");  // router.cc:226
+    gates = dense(gates);
+  }
+  if (old_tags.defined()) {
+    on_device(old_tags, "tags");
+    if (old_tags.scalar_type() != route.scalar_type()) runtime_error("tags must have the dtype of route_indices");
+    old_tags = dense(old_tags);
+  }
+  Tensor tags;
+  if (want_tags) tags = clear ? zeros({total}, at::kInt, in) : empty({total}, at::kInt, in);
+  check(brt_hip_dispatch(ptr(in), ptr(out), ptr(gates), iptr(route), iptr(loads), iptr(counts), iptr(old_tags), iptr(tags),
+                         T, cell, E, total, mpl, one_d, tag_index, code_of(in.scalar_type()), stream_of(in)));
+  return tuple(wrap(out), want_tags ? wrap(tags) : none());
+}
+
+// in_data, route_indices, loads, gates, out_data, out_dtype, max_path_padding, row_tags (a single-path route whose
+// rows carry the tags of the paired dispatch, laid out as in_data is) -> the combined cells
+PyObject* combine(const Args& a) {
+  const Tensor in = dense(a.tensor(0)), route = dense(a.tensor(1));
+  Tensor gates = a.tensor_or_none(3);
+  const Tensor residual = a.tensor_or_none(4), given_loads = a.tensor(2);
+  int32(route, "route_indices");
+  int32(given_loads, "loads");
+  const int in_type = data_type(in, "data type");
+  const c10::DeviceGuard guard(in.device());
+  const int64_t T = route.size(0), E = route.size(1), P = in.size(0), cell = P > 0 ? in.numel() / P : 0;
+  const int64_t mpl = a.flag(6) ? P / E : 0;  // router.cc:427-430
+  if (gates.defined()) {
+    on_device(gates, "gates");
+    data_type(gates, "gate data type");
+    gates = dense(gates);
+  }
+  Tensor out = residual;
+  if (residual.defined()) {
+    on_device(residual, "out_data");
+    if (!residual.is_contiguous()) runtime_error("out_data must be contiguous (it is updated in place)");
+  } else {
+    at::ScalarType type = in.scalar_type();
+    a.dtype(5, &type);
+    out = empty(rows_of(in, T), type, in);
+  }
+  const int out_type = code_of(out.scalar_type());
+  if (out_type < 0 || out.numel() != T * cell) runtime_error("out_data does not match [cell_num, *cell_shape]");
+  // scatter form (identical rows; cells without a row keep the residual)
+  if (residual.defined() && !gates.defined() && !a.none(7) && cell * in.element_size() % 16 == 0 &&
+      (out_type == in_type || out_type == BRT_F32)) {
+    const Tensor tags = a.tensor(7);
+    check(brt_hip_combine_by_tags(ptr(in), ptr(out), iptr(tags), P, cell, T, in_type, out_type, stream_of(in)));
+  } else {
+    const Tensor loads = dense(given_loads.device() == in.device() ? given_loads : given_loads.to(in.device()));
+    check(brt_hip_combine(ptr(in), ptr(out), ptr(gates), iptr(route), iptr(loads), T, cell, E, P, mpl, residual.defined(),
+                          in_type, out_type, gates.defined() ? code_of(gates.scalar_type()) : BRT_F32, stream_of(in)));
+  }
+  return wrap(out);
+}
+
+PyObject* combine_by_row_tags(const Args& a) {  // in_data, row_tags, cells, out_data, out_dtype
+  const Tensor given = a.tensor(0), tags = a.tensor(1), residual = a.tensor_or_none(3);
+  on_device(given, "in_data");
+  const int in_type = data_type(given, "data type");
+  const Tensor in = dense(given);
+  const c10::DeviceGuard guard(in.device());
+  const int64_t P = in.size(0), cells = a.integer(2), cell = P > 0 ? in.numel() / P : 0;
+  Tensor out = residual;
+  if (residual.defined()) {
+    if (!residual.is_contiguous()) runtime_error("out_data must be contiguous (it is updated in place)");
+  } else {
+    at::ScalarType type = in.scalar_type();
+    a.dtype(4, &type);
+    out = zeros(rows_of(in, cells), type, in);
+  }
+  if (code_of(out.scalar_type()) < 0 || out.numel() != cells * cell)
+    runtime_error("out_data does not match [cell_num, *cell_shape]");
+  if (tags.numel() < P) runtime_error("one tag per row is needed");
+  check(brt_hip_combine_by_tags(ptr(in), ptr(out), iptr(tags), P, cell, cells, in_type, code_of(out.scalar_type()),
+                                stream_of(in)));
+  return wrap(out);
+}
+
+Tensor entry_weights(const Tensor& given, int64_t entries) {
+  if (!given.defined()) return given;
+  if (given.scalar_type() != at::kFloat || given.numel() != entries) runtime_error("weights must be fp32 [cells, k]");
+  return dense(given);
+}
+
+PyObject* dispatch_by_rows(const Args& a) {  // in_data, row_entries, k, weights, out
+  const Tensor given = a.tensor(0), entries_given = a.tensor(1);
+  on_device(given, "in_data"), on_device(entries_given, "row_entries");
+  int32(entries_given, "row_entries");
+  const int type = data_type(given, "in_data data type");
+  const Tensor in = dense(given), entries = dense(entries_given);
+  const int64_t T = in.size(0), cell = T > 0 ? in.numel() / T : 0, P = entries.numel(), k = a.integer(2);
+  const Tensor weights = entry_weights(a.tensor_or_none(3), T * k);
+  const c10::DeviceGuard guard(in.device());
+  Tensor out = a.tensor_or_none(4);
+  if (!out.defined()) out = empty(rows_of(in, P), in.scalar_type(), in);
+  else if (out.scalar_type() != in.scalar_type() || !out.is_contiguous() || out.numel() != P * cell || out.device() != in.device())
+    runtime_error("out must be a contiguous [rows, *cell_shape] tensor of the input's type");
+  check(brt_hip_dispatch_by_rows(ptr(in), ptr(out), fptr(weights), iptr(entries), P, T, k, cell, type, stream_of(in)));
+  return wrap(out);
+}
+
+PyObject* combine_by_rows(const Args& a) {  // in_data, path_ids, seat_rows, weights, out_data, out_dtype
+  const Tensor given = a.tensor(0), ids_given = a.tensor(1), seats_given = a.tensor(2), residual = a.tensor_or_none(4);
+  on_device(given, "in_data"), on_device(ids_given, "path_ids");
+  int32(ids_given, "path_ids");
+  on_device(seats_given, "seat_rows");
+  int32(seats_given, "seat_rows");
+  const int in_type = data_type(given, "in_data data type");
+  if (ids_given.sizes() != seats_given.sizes() || ids_given.dim() != 2)
+    runtime_error("path_ids and seat_rows must both be [cells, k]");
+  const Tensor in = dense(given), ids = dense(ids_given), seats = dense(seats_given);
+  const int64_t T = ids.size(0), k = ids.size(1), P = in.size(0);
+  const int64_t cell = P > 0 ? in.numel() / P : residual.defined() && T > 0 ? residual.numel() / T : 0;
+  const Tensor weights = entry_weights(a.tensor_or_none(3), T * k);
+  const c10::DeviceGuard guard(in.device());
+  Tensor out = residual;
+  if (residual.defined()) {
+    if (!residual.is_contiguous() || residual.numel() != T * cell) runtime_error("out_data must be a contiguous [cells, ...] tensor");
+  } else {
+    at::ScalarType type = in.scalar_type();
+    a.dtype(5, &type);
+    out = empty(rows_of(in, T), type, in);
+  }
+  const int out_type = code_of(out.scalar_type());
+  if (out_type < 0 || (out_type != in_type && out_type != BRT_F32)) not_implemented("output data type is not supported");
+  check(brt_hip_combine_by_rows(ptr(in), ptr(out), fptr(weights), iptr(ids), iptr(seats), T, k, cell, P, residual.defined(),
+                                in_type, out_type, stream_of(in)));
+  return wrap(out);
+}
+
+// ---- grouped GEMM ------------------------------------------------------------------------------------
+// x, out, weight_table, bias_table, loads, in_features, out_features, activation code, tags, gather, scatter,
+// rows or None, row_entries, entries_per_cell, row_tags_out, gates
+PyObject* grouped_linear(const Args& a) {
+  const Tensor x = a.tensor(0), out = a.tensor(1), weights = a.tensor(2), biases = a.tensor_or_none(3), loads = a.tensor(4);
+  const int64_t K = a.integer(5), N = a.integer(6), act = a.integer(7);
+  const Tensor tags = a.tensor_or_none(8), entries = a.tensor_or_none(12), tags_out = a.tensor_or_none(14), gates = a.tensor_or_none(15);
+  const bool gather = a.flag(9), scatter = a.flag(10), routed = gather || scatter;
+  const int64_t k = a.integer(13);
+  if (x.scalar_type() != at::kBFloat16 || (out.scalar_type() != at::kBFloat16 && out.scalar_type() != at::kFloat))
+    not_implemented("the grouped GEMM computes in bf16 (fp32 accumulation); the output is bf16 or fp32");
+  const bool f32_out = out.scalar_type() == at::kFloat;
+  if (gates.defined()) {
+    if (!(scatter && f32_out)) runtime_error("gates fold the weighted combine into the store: scatter=True and an fp32 out");
+    if (!gates.is_cuda() || gates.scalar_type() != at::kFloat || !gates.is_contiguous())
+      runtime_error("gates must be a contiguous fp32 device tensor");
+  } else if (f32_out && entries.defined()) {
+    not_implemented("the row-entry form writes bf16");
+  }
+  if (!(x.is_cuda() && out.is_cuda() && loads.is_cuda())) runtime_error("grouped_linear needs device tensors");
+  if (loads.scalar_type() != at::kInt) runtime_error("capacities must be int32");
+  if (!(x.is_contiguous() && out.is_contiguous())) runtime_error("shared inputs must be contiguous");
+  if (x.numel() != x.size(0) * K || out.numel() != out.size(0) * N)
+    runtime_error("shared inputs do not match [rows, in_features] / [rows, out_features]");
+  int64_t cells = 0, rows = a.none(11) ? -1 : a.integer(11);
+  const bool by_rows = routed && entries.defined();
+  if (by_rows) {
+    if (!entries.is_cuda() || entries.scalar_type() != at::kInt || !entries.is_contiguous())
+      runtime_error("row_entries must be a contiguous int32 vector on the device");
+    if (gather && scatter && x.size(0) != out.size(0)) runtime_error("a gathered input / scattered output has one row per cell");
+    cells = gather ? x.size(0) : out.size(0);
+    if (rows < 0) rows = entries.numel();
+    else if (rows > entries.numel()) runtime_error("rows exceeds the row-entry vector");
+  } else if (routed) {
+    if (!tags.defined() || !tags.is_cuda() || tags.scalar_type() != at::kInt || !tags.is_contiguous())
+      runtime_error("gather/scatter need the contiguous int32 tag-index matrix on the device");
+    cells = tags.size(0);
+    if (tags.size(1) != loads.numel()) runtime_error("tags must have one column per branch");
+    if ((gather && x.size(0) != cells) || (scatter && out.size(0) != cells))
+      runtime_error("a gathered input / scattered output has one row per cell");
+  }
+  if (rows < 0) {
+    // neither side path-major: nothing bounds the rows but the caller (the slots of the tag matrix would
+    // launch a grid that is almost all empty row blocks)
+    if (gather && scatter) runtime_error("rows (an upper bound of sum(loads)) is needed when x is gathered and out scattered");
+    rows = scatter ? x.size(0) : out.size(0);
+  } else if ((!gather && rows > x.size(0)) || (!scatter && rows > out.size(0))) {
+    runtime_error("rows exceeds the path-major buffer");
+  }
+  if (!routed && x.size(0) != out.size(0)) runtime_error("shared inputs must have the same number of rows");
+  const c10::DeviceGuard guard(x.device());
+  void* const st = stream_of(x);
+  const void* const* const w = static_cast<const void* const*>(ptr(weights));
+  const void* const* const b = static_cast<const void* const*>(ptr(biases));
+  const int E = static_cast<int>(loads.numel());
+  if (gates.defined()) {
+    if (gates.numel() != cells * (by_rows ? k : E))
+      runtime_error("gates must hold one weight per cell and path (tags) or per entry (row_entries)");
+    check(brt_hip_grouped_gemm_accumulate(ptr(x), w, b, fptr(out), iptr(loads), iptr(by_rows ? entries : tags), by_rows ? k : 0,
+                                          fptr(gates), E, rows, cells, K, N, act, gather, st));
+  } else if (by_rows) {
+    check(brt_hip_grouped_gemm_by_rows(ptr(x), w, b, ptr(out), iptr(loads), iptr(entries), k, E, rows, cells, K, N, act, gather,
+                                       scatter, st));
+  } else if (routed) {
+    if (tags_out.defined() && (tags_out.scalar_type() != at::kInt || tags_out.numel() < rows || !tags_out.is_cuda()))
+      runtime_error("row_tags_out must be an int32 device vector with one entry per row");
+    if (f32_out)
+      check(brt_hip_grouped_gemm_routed_f32out(ptr(x), w, b, fptr(out), iptr(loads), iptr(tags), E, rows, cells, K, N, act, gather,
+                                               scatter, iptr(tags_out), st));
+    else
+      check(brt_hip_grouped_gemm_routed(ptr(x), w, b, ptr(out), iptr(loads), iptr(tags), E, rows, cells, K, N, act, gather,
+                                        scatter, iptr(tags_out), st));
+  } else if (f32_out) {
+    check(brt_hip_grouped_gemm_f32out(ptr(x), w, b, fptr(out), iptr(loads), E, rows, K, N, act, st));
+  } else {
+    check(brt_hip_grouped_gemm(ptr(x), w, b, ptr(out), iptr(loads), E, rows, K, N, act, st));
+  }
+  return none();
+}
+
+PyObject* cast_f32_to_bf16(const Args& a) {
+  const Tensor given = a.tensor(0);
+  if (given.scalar_type() != at::kFloat)
+    runtime_error(std::string("the cast kernel reads fp32, got ") + c10::toString(given.scalar_type()));
+  const Tensor in = dense(given);
+  const c10::DeviceGuard guard(in.device());
+  Tensor out = empty(in.sizes(), at::kBFloat16, in);
+  if (in.numel() > 0) check(brt_hip_cast_f32_to_bf16(fptr(in), ptr(out), in.numel(), stream_of(in)));
+  return wrap(out);
+}
+
+// ---- host reads --------------------------------------------------------------------------------------
+// The values of an int32 vector as a list: one copy to pinned memory on the current stream, which is then
+// waited for (other Python threads run meanwhile).
+PyObject* int_list(const Args& a) {
+  const Tensor given = a.tensor(0);
+  int32(given, "loads");
+  const Tensor t = dense(given);
+  const int64_t n = t.numel();
+  const int32_t* values = nullptr;
+  at::DataPtr host;
+  if (n > 0 && t.is_cuda()) {
+    const c10::DeviceGuard guard(t.device());
+    host = at::getHostAllocator(at::kCUDA)->allocate(n * 4);
+    const hipStream_t st = c10::hip::getCurrentHIPStream(t.get_device()).stream();
+    hipError_t rc = hipMemcpyAsync(host.get(), ptr(t), n * 4, hipMemcpyDeviceToHost, st);
+    if (rc == hipSuccess) {
+      Py_BEGIN_ALLOW_THREADS
+      rc = hipStreamSynchronize(st);
+      Py_END_ALLOW_THREADS
+    }
+    if (rc != hipSuccess) runtime_error(std::string("reading the loads: ") + hipGetErrorString(rc));
+    values = static_cast<const int32_t*>(host.get());
+  } else if (n > 0) {
+    values = iptr(t);
+  }
+  PyObject* const list = PyList_New(n);
+  for (int64_t i = 0; i < n; ++i) PyList_SET_ITEM(list, i, PyLong_FromLong(values[i]));
+  return list;
+}
+
+PyObject* calls(const Args&) { return PyLong_FromUnsignedLongLong(g_calls); }
+
+template <PyObject* (*FN)(const Args&), int N>
+PyObject* entry(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  if (n != N) {
+    PyErr_Format(PyExc_TypeError, "%d arguments are expected, got %zd", N, n);
+    return nullptr;
+  }
+  try {
+    return FN(Args{v, n});
+  } catch (const Raised& e) {
+    if (e.type != nullptr) PyErr_SetString(e.type, e.what());
+  } catch (...) {
+    torch::translate_exception_to_python(std::current_exception());
+  }
+  return nullptr;
+}
+
+#define BRT_ENTRY(name, n) \
+  { #name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&entry<name, n>)), METH_FASTCALL, nullptr }
+PyMethodDef methods[] = {
+    BRT_ENTRY(topk_hot_mask, 2),    BRT_ENTRY(gate_topk, 4),           BRT_ENTRY(throttle_hotmask, 3),
+    BRT_ENTRY(generate, 5),         BRT_ENTRY(route_and_dispatch, 7),  BRT_ENTRY(route_by_path, 7),
+    BRT_ENTRY(dispatch, 12),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
+    BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 6),     BRT_ENTRY(grouped_linear, 16),
+    BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(int_list, 1),
+    BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "brt_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_brt_native() { return PyModule_Create(&module); }

@@ -76,105 +76,15 @@ def grouped_linear(x: torch.Tensor, out: torch.Tensor, weight_table: torch.Tenso
     adds, so ``out`` must hold zeros (or what the sums are added to) before the call.  Equal to
     ``combine_with_indices_and_loads`` on the separate GEMM's output: bit for bit with at most two
     paths per cell, to the last bits of an fp32 sum taken in another order with more."""
-    if x.dtype != torch.bfloat16 or out.dtype not in (torch.bfloat16, torch.float32):
-        raise NotImplementedError("the grouped GEMM computes in bf16 (fp32 accumulation); "
-                                  "the output is bf16 or fp32")
-    pending = deferred.pending_of(x)
-    if pending is not None:
-        pending.materialize()  # an unfilled deferred buffer handed over as it is: the rows are dispatched first
-    f32_out = out.dtype == torch.float32
-    if gates is not None:
-        if not (scatter and f32_out):
-            raise RuntimeError("gates fold the weighted combine into the store: scatter=True and an fp32 out")
-        if not gates.is_cuda or gates.dtype != torch.float32 or not gates.is_contiguous():
-            raise RuntimeError("gates must be a contiguous fp32 device tensor")
-    elif f32_out and row_entries is not None:
-        raise NotImplementedError("the row-entry form writes bf16")
-    if not (x.is_cuda and out.is_cuda and loads.is_cuda):
-        raise RuntimeError("grouped_linear needs device tensors")
-    if loads.dtype != torch.int32:
-        raise RuntimeError("capacities must be int32")
-    if not (x.is_contiguous() and out.is_contiguous()):
-        raise RuntimeError("shared inputs must be contiguous")
-    if x.numel() != x.shape[0] * in_features or out.numel() != out.shape[0] * out_features:
-        raise RuntimeError("shared inputs do not match [rows, in_features] / [rows, out_features]")
-    routed = gather or scatter
-    cells = 0
-    if routed and row_entries is not None:
-        if not row_entries.is_cuda or row_entries.dtype != torch.int32 or not row_entries.is_contiguous():
-            raise RuntimeError("row_entries must be a contiguous int32 vector on the device")
-        if gather and scatter and x.shape[0] != out.shape[0]:
-            raise RuntimeError("a gathered input / scattered output has one row per cell")
-        cells = x.shape[0] if gather else out.shape[0]
-        if rows is None:
-            rows = row_entries.numel()
-        elif rows > row_entries.numel():
-            raise RuntimeError("rows exceeds the row-entry vector")
-    elif routed:
-        if tags is None or not tags.is_cuda or tags.dtype != torch.int32 or not tags.is_contiguous():
-            raise RuntimeError("gather/scatter need the contiguous int32 tag-index matrix on the device")
-        cells = tags.shape[0]
-        if tags.shape[1] != loads.numel():
-            raise RuntimeError("tags must have one column per branch")
-        if (gather and x.shape[0] != cells) or (scatter and out.shape[0] != cells):
-            raise RuntimeError("a gathered input / scattered output has one row per cell")
-    if rows is None:
-        if gather and scatter:
-            # neither side is path-major, so nothing bounds the rows but the caller: the slots of
-            # the tag matrix would launch a grid that is almost all empty row blocks
-            raise RuntimeError("rows (an upper bound of sum(loads)) is needed when x is gathered and out scattered")
-        rows = out.shape[0] if not scatter else x.shape[0]
-    elif (not gather and rows > x.shape[0]) or (not scatter and rows > out.shape[0]):
-        raise RuntimeError("rows exceeds the path-major buffer")
-    if not routed and x.shape[0] != out.shape[0]:
-        raise RuntimeError("shared inputs must have the same number of rows")
-    with torch.cuda.device(x.device):
-        lib = _lib.lib()
-        stream = torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
-        bias_ptr = None if bias_table is None else bias_table.data_ptr()
-        if gates is not None:
-            by_rows = row_entries is not None
-            k = int(entries_per_cell) if by_rows else 0
-            if gates.numel() != cells * (k if by_rows else loads.numel()):
-                raise RuntimeError("gates must hold one weight per cell and path (tags) or per entry (row_entries)")
-            _lib.check(lib.brt_hip_grouped_gemm_accumulate(
-                x.data_ptr(), weight_table.data_ptr(), bias_ptr, out.data_ptr(), loads.data_ptr(),
-                (row_entries if by_rows else tags).data_ptr(), k, gates.data_ptr(), loads.numel(), rows,
-                cells, in_features, out_features, _ACT[activation], int(gather), stream))
-        elif routed and row_entries is not None:
-            _lib.check(lib.brt_hip_grouped_gemm_by_rows(
-                x.data_ptr(), weight_table.data_ptr(), bias_ptr, out.data_ptr(), loads.data_ptr(),
-                row_entries.data_ptr(), int(entries_per_cell), loads.numel(), rows, cells,
-                in_features, out_features, _ACT[activation], int(gather), int(scatter), stream))
-        elif routed:
-            if row_tags_out is not None and (row_tags_out.dtype != torch.int32 or row_tags_out.numel() < rows
-                                             or not row_tags_out.is_cuda):
-                raise RuntimeError("row_tags_out must be an int32 device vector with one entry per row")
-            fn = lib.brt_hip_grouped_gemm_routed_f32out if f32_out else lib.brt_hip_grouped_gemm_routed
-            _lib.check(fn(
-                x.data_ptr(), weight_table.data_ptr(), bias_ptr, out.data_ptr(), loads.data_ptr(),
-                tags.data_ptr(), loads.numel(), rows, cells, in_features, out_features,
-                _ACT[activation], int(gather), int(scatter),
-                None if row_tags_out is None else row_tags_out.data_ptr(), stream))
-        else:
-            fn = lib.brt_hip_grouped_gemm_f32out if f32_out else lib.brt_hip_grouped_gemm
-            _lib.check(fn(
-                x.data_ptr(), weight_table.data_ptr(), bias_ptr, out.data_ptr(), loads.data_ptr(),
-                loads.numel(), rows, in_features, out_features, _ACT[activation], stream))
+    _lib.native().grouped_linear(
+        x, out, weight_table, bias_table, loads, in_features, out_features, _ACT[activation], tags, gather,
+        scatter, rows, row_entries, entries_per_cell, row_tags_out, gates)
     return out
 
 
 def _to_bf16(t: torch.Tensor) -> torch.Tensor:
     """fp32 -> bf16 (round to nearest even) with the library's cast kernel."""
-    if t.dtype != torch.float32:
-        raise RuntimeError(f"the cast kernel reads fp32, got {t.dtype}")
-    t = t.contiguous()
-    out = torch.empty(t.shape, dtype=torch.bfloat16, device=t.device)
-    if t.numel():
-        _lib.check(_lib.lib().brt_hip_cast_f32_to_bf16(
-            t.data_ptr(), out.data_ptr(), t.numel(),
-            torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())))
-    return out
+    return _lib.native().cast_f32_to_bf16(t)
 
 
 class _Bf16Weights:
