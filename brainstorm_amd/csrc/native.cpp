@@ -25,6 +25,7 @@
 
 #include <stdexcept>
 #include <string>
+#include <vector>
 
 #include "brt_hip.h"
 
@@ -508,6 +509,43 @@ PyObject* grouped_linear(const Args& a) {
   return none();
 }
 
+// operands (list or tuple), first, step, branches used, what -> (fp32, key): the tensors operands[first::step],
+// of which the used ones are all contiguous bf16 or all fp32, and what tells whether they are still the same
+// ones as at another call -- for bf16 the addresses of all of them; for fp32 also the object, the version
+// counter and the storage of each used one (`.data = ...` swaps the storage without touching the counter).
+PyObject* branch_key(const Args& a) {
+  PyObject* const seq = a.v[0];
+  if (!PyList_Check(seq) && !PyTuple_Check(seq)) throw Raised(PyExc_TypeError, "a list or tuple of branch operands is expected");
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq), first = a.integer(1), step = a.integer(2), used = a.integer(3);
+  PyObject* const* const items = PySequence_Fast_ITEMS(seq);
+  std::vector<uint64_t> key;
+  key.reserve(4 * n / step + 4);
+  bool fp32 = false;
+  Py_ssize_t b = 0;
+  for (Py_ssize_t i = first; i < n; i += step, ++b) {
+    if (fp32 && b >= used) break;  // branches past the capacities are never read, nor converted
+    if (!THPVariable_Check(items[i])) throw Raised(PyExc_TypeError, "branch operands are tensors");
+    const Tensor& t = THPVariable_Unpack(items[i]);
+    if (b < used) {
+      const bool f = t.scalar_type() == at::kFloat;
+      if (b == 0) fp32 = f, key.push_back(f);
+      if (f != fp32 || (!f && (t.scalar_type() != at::kBFloat16 || !t.is_contiguous()))) {
+        PyObject* const what = PyObject_Str(a.v[4]);
+        const std::string name = what != nullptr ? PyUnicode_AsUTF8(what) : "operands";
+        Py_XDECREF(what);
+        not_implemented("branch " + name + " must be contiguous bf16 or fp32 tensors of one dtype");
+      }
+    }
+    key.push_back(reinterpret_cast<uint64_t>(t.data_ptr()));
+    if (fp32) {
+      key.push_back(reinterpret_cast<uint64_t>(items[i]));
+      key.push_back(static_cast<uint64_t>(t._version()));
+      key.push_back(reinterpret_cast<uint64_t>(t.storage().data()));
+    }
+  }
+  return tuple(PyBool_FromLong(fp32), PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key.data()), key.size() * 8));
+}
+
 PyObject* cast_f32_to_bf16(const Args& a) {
   const Tensor given = a.tensor(0);
   if (given.scalar_type() != at::kFloat)
@@ -574,7 +612,7 @@ PyMethodDef methods[] = {
     BRT_ENTRY(generate, 5),         BRT_ENTRY(route_and_dispatch, 7),  BRT_ENTRY(route_by_path, 7),
     BRT_ENTRY(dispatch, 12),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
     BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 6),     BRT_ENTRY(grouped_linear, 16),
-    BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(int_list, 1),
+    BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5), BRT_ENTRY(int_list, 1),
     BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "brt_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

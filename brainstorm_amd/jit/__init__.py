@@ -28,21 +28,6 @@ __all__ = ["make_jit_kernel", "grouped_linear", "GroupedLinearKernel"]
 _ACT = {None: _lib.ACT_NONE, "none": _lib.ACT_NONE, "gelu": _lib.ACT_GELU, "relu": _lib.ACT_RELU}
 
 
-class _PointerTable:
-    """Device array of per-branch pointers, rebuilt only when the tensors change."""
-
-    def __init__(self):
-        self.key = None
-        self.table = None
-
-    def get(self, tensors: Sequence[torch.Tensor]) -> torch.Tensor:
-        key = tuple(t.data_ptr() for t in tensors)
-        if key != self.key:
-            self.table = torch.tensor(key, dtype=torch.int64, device=tensors[0].device)
-            self.key = key
-        return self.table
-
-
 def grouped_linear(x: torch.Tensor, out: torch.Tensor, weight_table: torch.Tensor,
                    bias_table: Optional[torch.Tensor], loads: torch.Tensor, in_features: int,
                    out_features: int, activation: Optional[str] = None, *,
@@ -87,23 +72,29 @@ def _to_bf16(t: torch.Tensor) -> torch.Tensor:
     return _lib.native().cast_f32_to_bf16(t)
 
 
-class _Bf16Weights:
-    """bf16 copies of fp32 branch parameters, converted again only when a parameter changed."""
+class _BranchOperands:
+    """Device array of the branches' pointers, rebuilt only when the tensors change; fp32 branches are
+    converted to bf16 copies then."""
 
-    def __init__(self):
-        self.keys = None
-        self.sources = None  # the converted tensors are held, so their addresses cannot be reused unnoticed
+    def __init__(self, what: str):
+        self.what = what
+        self.key = None
+        self.table = None
+        self.sources = None  # converted tensors are held, so their addresses cannot be reused unnoticed
         self.copies = None
 
-    def get(self, tensors: Sequence[torch.Tensor]) -> List[torch.Tensor]:
-        # `.data = ...` swaps the storage without touching the version counter: the storage's own
-        # address and the tensor's identity are part of the key
-        keys = tuple((id(t), t.data_ptr(), t._version, t.untyped_storage().data_ptr()) for t in tensors)
-        if keys != self.keys:
-            self.copies = [_to_bf16(t.detach()) for t in tensors]
-            self.sources = list(tensors)
-            self.keys = keys
-        return self.copies
+    def get(self, operands: Sequence[torch.Tensor], first: int, step: int, used: int) -> torch.Tensor:
+        fp32, key = _lib.native().branch_key(operands, first, step, used, self.what)
+        if key != self.key:
+            tensors = list(operands[first::step])
+            self.copies = self.sources = None
+            if fp32:
+                self.sources = tensors[:used]
+                self.copies = [_to_bf16(t.detach()) for t in self.sources]
+                tensors = self.copies
+            self.table = torch.tensor([t.data_ptr() for t in tensors], dtype=torch.int64, device=tensors[0].device)
+            self.key = key
+        return self.table
 
 
 class GroupedLinearKernel:
@@ -122,10 +113,8 @@ class GroupedLinearKernel:
         self.out_features = out_features
         self.has_bias = has_bias
         self.activation = activation
-        self._weights = _PointerTable()
-        self._biases = _PointerTable()
-        self._weights_bf16 = _Bf16Weights()
-        self._biases_bf16 = _Bf16Weights()
+        self._weights = _BranchOperands("weights")
+        self._biases = _BranchOperands("biases")
 
     def __call__(self, shared_inputs: List[torch.Tensor], standalone_inputs: Sequence[torch.Tensor],
                  capacities: Union[torch.Tensor, Sequence[int]] = (), *,
@@ -138,48 +127,43 @@ class GroupedLinearKernel:
         tensor of the routed GridTensor, as it came off the load stack) and must stem from a fused
         dispatch fabric built with ``compact_route=True``."""
         x, out = shared_inputs
-        standalone_inputs = list(standalone_inputs)
-        step = 2 if self.has_bias else 1
-        weights = standalone_inputs[0::step]
-        biases = standalone_inputs[1::step] if self.has_bias else None
+        if not isinstance(standalone_inputs, (list, tuple)):
+            standalone_inputs = list(standalone_inputs)
         if not torch.is_tensor(capacities):
             capacities = torch.tensor(list(capacities), dtype=torch.int32, device=out.device)
-        if capacities.numel() > len(weights):
+        step = 2 if self.has_bias else 1
+        used = capacities.numel()
+        if used > (len(standalone_inputs) + step - 1) // step:
             raise RuntimeError("more capacities than branches")
-        weights = self._branch_operands(weights, capacities.numel(), self._weights_bf16, "weights")
-        if biases:
-            biases = self._branch_operands(biases, capacities.numel(), self._biases_bf16, "biases")
-        route_loads = capacities
-        loads = capacities.to(device=out.device, dtype=torch.int32)
+        weights = self._weights.get(standalone_inputs, 0, step, used)
+        biases = self._biases.get(standalone_inputs, 1, step, used) if self.has_bias else None
+        loads = capacities
+        if loads.dtype != torch.int32 or loads.device != out.device:
+            loads = loads.to(device=out.device, dtype=torch.int32)
         if residual is not None:
-            return self._store_to_cells(x, weights, biases, loads, route_loads, residual)
+            return self._store_to_cells(x, weights, biases, loads, capacities, residual)
         state = deferred.pending_of(x)  # a DeferredRows, or the routed GridTensor itself
         if state is not None and not self._can_gather(state, out):
             state.materialize()
             state = None
         if state is not None:
-            # the rows of a deferred dispatch: read from the cells through the route's tag indices
+            # the rows of a deferred dispatch: read from the cells through the route
             route = state.route
             cells = state.cells if state.cells.dtype == torch.bfloat16 else _to_bf16(state.cells)
             if isinstance(route, c_router.CompactRoute):  # rows named by the row-entry vector
-                grouped_linear(cells, out, self._weights.get(weights),
-                               self._biases.get(biases) if biases else None, loads, self.in_features,
-                               self.out_features, self.activation, row_entries=route.row_entries,
+                grouped_linear(cells, out, weights, biases, loads, self.in_features, self.out_features,
+                               self.activation, row_entries=route.row_entries,
                                entries_per_cell=route.k, gather=True, rows=out.shape[0])
                 return
             row_tags = torch.empty((out.shape[0],), dtype=torch.int32, device=out.device)
-            grouped_linear(cells, out, self._weights.get(weights),
-                           self._biases.get(biases) if biases else None, loads, self.in_features,
-                           self.out_features, self.activation, tags=route.indices, gather=True,
+            grouped_linear(cells, out, weights, biases, loads, self.in_features, self.out_features,
+                           self.activation, tags=route.indices, gather=True,
                            rows=out.shape[0], row_tags_out=row_tags)
             route.row_tags, route.row_tags_stride = row_tags, 0
             return
         if x.dtype == torch.float32:
             x = _to_bf16(x)  # (a deferred buffer is filled by this read)
-        grouped_linear(
-            x, out, self._weights.get(weights),
-            self._biases.get(biases) if biases else None,
-            loads, self.in_features, self.out_features, self.activation)
+        grouped_linear(x, out, weights, biases, loads, self.in_features, self.out_features, self.activation)
 
     def _store_to_cells(self, x, weights, biases, loads, route_loads, residual):
         """The GEMM whose rows go straight to their cells in ``residual`` (combine folded in)."""
@@ -197,20 +181,10 @@ class GroupedLinearKernel:
             x = _to_bf16(x)
         if x.shape[0] != route.row_entries.numel():
             raise RuntimeError("the input does not have the rows of the dispatched layout")
-        grouped_linear(x, residual, self._weights.get(weights),
-                       self._biases.get(biases) if biases else None, loads, self.in_features,
+        grouped_linear(x, residual, weights, biases, loads, self.in_features,
                        self.out_features, self.activation, row_entries=route.row_entries,
                        entries_per_cell=1, scatter=True, rows=x.shape[0])
         route.combined_into = residual
-
-    def _branch_operands(self, tensors, used: int, cache: _Bf16Weights, what: str):
-        dtypes = {t.dtype for t in tensors[:used]}
-        if dtypes == {torch.float32}:
-            return cache.get(tensors[:used])  # branches past the capacities are never read, nor converted
-        for t in tensors[:used]:
-            if t.dtype != torch.bfloat16 or not t.is_contiguous():
-                raise NotImplementedError(f"branch {what} must be contiguous bf16 or fp32 tensors of one dtype")
-        return tensors
 
     def _can_gather(self, state, out: torch.Tensor) -> bool:
         cells = state.cells

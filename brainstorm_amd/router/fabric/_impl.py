@@ -227,12 +227,13 @@ class DispatchFabric(FabricBase):
                 score: torch.Tensor = None):
         caps = runtime_capacities if runtime_capacities is not None else self.supported_capacities
         in_flows = [in_flow] if self.flow_num == 1 else in_flow
-        self._route = c_router.generate_route(
+        route = c_router.generate_route(
             hot_mask, supported_capacities=caps, capacity_padding=self.capacity_padding,
             path_wise_padding=self.path_wise_padding,
             is_tag_index=self._defers(in_flows, runtime_capacities, hot_mask),
             single_path=getattr(hot_mask, "_brt_single_path", False))
-        route_indices, loads = self._route.indices, self._route.loads
+        self.__dict__["_route"] = route  # (not through nn.Module's attribute registration)
+        route_indices, loads = route.indices, route.loads
         self.capture_flow_stats(in_flows, route_indices, loads)
         all_out_flows, score = self.dispatch(in_flows, route_indices, loads, score)
         if self.flow_num == 1:
@@ -399,10 +400,11 @@ class FusedDispatchFabric(DispatchFabric):
             return False
         if any(logic != "1d" for logic in self.route_logics):
             return False
-        for flow in in_flows:
-            if (flow.dim() != 2 or flow.dtype not in (torch.bfloat16, torch.float32)
-                    or flow.shape[1] % 8 != 0 or flow.shape[0] == 0):
-                return False
+        with torch._C.DisableTorchFunctionSubclass():  # shapes of GridTensors, read as those of plain tensors
+            for flow in in_flows:
+                if (flow.dim() != 2 or flow.dtype not in (torch.bfloat16, torch.float32)
+                        or flow.shape[1] % 8 != 0 or flow.shape[0] == 0):
+                    return False
         return True
 
     def _static_rows(self, flow_data, route_indices) -> Optional[int]:
@@ -429,8 +431,9 @@ class FusedDispatchFabric(DispatchFabric):
         if len(in_flows) != 1 or runtime_capacities is not None or self.transforms[0]:
             return False
         flow = in_flows[0]
-        return (self.route_logics[0] == "1d" and flow.dim() >= 2 and flow.shape[0] > 0 and flow.is_cuda
-                and flow.dtype in (torch.float32, torch.float16, torch.bfloat16))
+        with torch._C.DisableTorchFunctionSubclass():
+            return (self.route_logics[0] == "1d" and flow.dim() >= 2 and flow.shape[0] > 0 and flow.is_cuda
+                    and flow.dtype in (torch.float32, torch.float16, torch.bfloat16))
 
     def _forward_compact(self, in_flows, decision, score):
         """The route from path ids: ``route_by_path`` lays it out (loads by the capacity rules of
@@ -456,16 +459,15 @@ class FusedDispatchFabric(DispatchFabric):
         route = c_router.CompactRoute(decision.path_ids, decision.scores, loads, counts, seat_rows,
                                       row_entries, paths, indices)
         c_router.remember_route(loads, route)
-        self._route = route
+        self.__dict__["_route"] = route
         self.capture_flow_stats(in_flows, indices, loads)  # (reads the dense matrix when capturing)
         level = len(tags) - 1
         extra = dict(extra or {})
         extra[_route_key(level)] = route
-        flat = data.view(cells, -1)
-        if (self.defer_dispatch and flat.shape[1] % 8 == 0
-                and data.dtype in (torch.bfloat16, torch.float32) and data.dim() == 2):
-            routed = torch.empty((rows, flat.shape[1]), dtype=data.dtype, device=data.device)
-            extra[_deferred_key(level)] = DeferredState(flat, route, routed, _deferred_key(level))
+        if (self.defer_dispatch and data.dim() == 2 and data.shape[1] % 8 == 0
+                and data.dtype in (torch.bfloat16, torch.float32)):
+            routed = torch.empty((rows, data.shape[1]), dtype=data.dtype, device=data.device)
+            extra[_deferred_key(level)] = DeferredState(data, route, routed, _deferred_key(level))
         else:
             routed = c_router.dispatch_by_rows(data, row_entries, k)
         out = init_grid_tensor(routed, tags[:-1] + [indices], load_stack[:-1] + [loads], extra)
@@ -482,14 +484,15 @@ class FusedDispatchFabric(DispatchFabric):
         # static rows, one flow, single-path route: index generation moves the rows itself
         data, tags, load_stack, extra = to_torch_tensor(in_flows[0], retrieve_attr=True)
         assert tags[-1] is None  # fused dispatch starts from freshly annotated cells
-        self._route, routed = c_router.route_and_dispatch(
+        route, routed = c_router.route_and_dispatch(
             data, hot_mask, self._row_bound(data.shape[0], hot_mask.shape[1]),
             supported_capacities=self.supported_capacities, capacity_padding=self.capacity_padding,
             path_wise_padding=self.path_wise_padding, single_path=True)
-        route_indices, loads = self._route.indices, self._route.loads
+        self.__dict__["_route"] = route
+        route_indices, loads = route.indices, route.loads
         self.capture_flow_stats(in_flows, route_indices, loads)
         extra = dict(extra or {})
-        extra[_route_key(len(tags) - 1)] = self._route
+        extra[_route_key(len(tags) - 1)] = route
         out = init_grid_tensor(routed, tags[:-1] + [route_indices], load_stack[:-1] + [loads], extra)
         return (out if self.flow_num == 1 else [out]), score
 
@@ -501,8 +504,9 @@ class FusedDispatchFabric(DispatchFabric):
         if len(in_flows) != 1 or runtime_capacities is not None or self.max_path_padding:
             return False
         flow = in_flows[0]
-        return (not self.transforms[0] and self.route_logics[0] == "1d" and flow.dim() >= 2
-                and flow.shape[0] > 0 and flow.is_cuda and hot_mask.dtype == torch.int32)
+        with torch._C.DisableTorchFunctionSubclass():
+            return (not self.transforms[0] and self.route_logics[0] == "1d" and flow.dim() >= 2
+                    and flow.shape[0] > 0 and flow.is_cuda and hot_mask.dtype == torch.int32)
 
     def dispatch(self, in_flows, route_indices, loads, score):
         all_out_flows = []

@@ -22,6 +22,9 @@ class Annotator(nn.Module):
         self.gridding = gridding
 
     def forward(self, t: torch.Tensor):
+        if type(t) is torch.Tensor and self.gridding and self.cell_shape is None and self.dims == [0] and t.is_contiguous() \
+                and t.dim() > 0:
+            return init_grid_tensor(t, [None], [None])  # the cells are the rows as they are
         assert self.dims[-1] < t.dim()
         rest = [d for d in range(t.dim()) if d not in self.dims]
         cell_shape = self.cell_shape if self.cell_shape is not None else [t.shape[d] for d in rest]

@@ -94,6 +94,12 @@ for _name in ("size", "dim", "numel", "nelement", "is_contiguous", "element_size
         _METADATA.add(_method)
 
 
+def shape_reads() -> frozenset:
+    """The metadata reads whose result is a plain value (not a tensor)."""
+    tensors = {getattr(torch.Tensor, name).__get__ for name in ("grad", "grad_fn")}
+    return frozenset(_METADATA - tensors)
+
+
 def is_metadata_read(func) -> bool:
     return func in _METADATA
 

@@ -55,6 +55,10 @@ def attach_cell_attr(ret, tag_stack, load_stack, extra_attrs_stack_dict=None):
     return ret
 
 
+# reads that return plain values: no result to attach the stacks to
+_SHAPE_READS = deferred.shape_reads()
+
+
 class GridTensor(torch.Tensor):
     # True: results of torch ops share the operand's stack objects (cheap, what
     # the routers expect); False: every hand-over makes a shallow copy.
@@ -183,6 +187,9 @@ class GridTensor(torch.Tensor):
     def __torch_function__(cls, func, types, args=(), kwargs=None):
         # Only plain attribute reads happen before the super() call, so no torch
         # function is re-entered here.
+        if func in _SHAPE_READS:  # nothing to carry over, nothing to fill
+            with torch._C.DisableTorchFunctionSubclass():
+                return func(*args, **(kwargs or {}))
         kwargs = kwargs or {}
         tags, loads, extra = collect_cell_attr(args)
         if tags is None and kwargs:  # operands passed by keyword only: torch.matmul(input=..., other=...)
@@ -211,7 +218,12 @@ def init_grid_tensor(tensor: torch.Tensor, tag_stack=None, load_stack=None,
                      extra_attr_dict=None) -> GridTensor:
     cell: GridTensor = tensor.as_subclass(GridTensor)
     if tag_stack and load_stack:
-        cell.deep_pack(tag_stack, load_stack, **(extra_attr_dict or {}))
+        assert isinstance(tag_stack, list) and isinstance(load_stack, list), (
+            "tag_stack and load_stack must be list")
+        attrs = cell.__dict__  # what deep_pack does
+        attrs[_TAGS] = GridTensor._transport(tag_stack)
+        attrs[_LOADS] = GridTensor._transport(load_stack)
+        attrs[_EXTRA] = dict(extra_attr_dict) if extra_attr_dict else {}
     else:
         cell.init_cell()
     return cell
@@ -227,7 +239,7 @@ def _as_plain(grid_t: torch.Tensor, extra) -> torch.Tensor:
     as a :class:`brainstorm_amd.runtime.deferred.DeferredRows`, which fills itself on first use."""
     with torch._C.DisableTorchFunctionSubclass():
         plain = grid_t.as_subclass(torch.Tensor)
-    return deferred.wrap_if_pending(plain, extra)
+    return deferred.wrap_if_pending(plain, extra) if extra else plain
 
 
 def deinit_grid_tensor(grid_t: GridTensor, retrieve_attr=True):
@@ -248,5 +260,9 @@ def to_torch_tensor(grid_t: GridTensor, retrieve_attr=False) -> Union[torch.Tens
     propagated needlessly); optionally also returns the stacks."""
     if not retrieve_attr:
         return _as_plain(grid_t, grid_t.__dict__.get(_EXTRA) if isinstance(grid_t, GridTensor) else None)
-    grid_t, tags, loads, extra = grid_t.copy_cell_attr()
+    attrs = grid_t.__dict__  # what copy_cell_attr does
+    assert _TAGS in attrs and _LOADS in attrs and _EXTRA in attrs
+    tags, loads, extra = attrs[_TAGS], attrs[_LOADS], attrs[_EXTRA]
+    if not GridTensor.SHALLOW_TRANSPORT:
+        tags, loads, extra = copy.copy(tags), copy.copy(loads), copy.copy(extra)
     return _as_plain(grid_t, extra), tags, loads, extra
