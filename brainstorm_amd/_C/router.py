@@ -634,9 +634,14 @@ def dispatch_by_rows(in_data: torch.Tensor, row_entries: torch.Tensor, k: int,
 
 def combine_by_rows(in_data: torch.Tensor, path_ids: torch.Tensor, seat_rows: torch.Tensor,
                     weights: Optional[torch.Tensor] = None, out_data: Optional[torch.Tensor] = None,
-                    out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+                    out_dtype: Optional[torch.dtype] = None, *,
+                    gates: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``out[t] = sum_j weights[t,j] * in_data[seat_rows[t,j]-1]`` over the entries that own a row,
     in ascending path id, fp32 from zero: the result of ``combine_with_indices_and_loads``
     (router.cc:372-473) for the same route, bit for bit.  With ``out_data`` the result is
-    written in place and cells without a row keep their value (the residual convention)."""
-    return _lib.native().combine_by_rows(in_data, path_ids, seat_rows, weights, out_data, out_dtype)
+    written in place and cells without a row keep their value (the residual convention).
+    ``gates`` (the ``[cells, paths]`` matrix, any data type) gives the weights instead:
+    ``gates[t, path_ids[t,j]]``."""
+    if gates is not None and weights is not None:
+        raise RuntimeError("weights or gates, not both")
+    return _lib.native().combine_by_rows(in_data, path_ids, seat_rows, weights, out_data, out_dtype, gates)

@@ -317,6 +317,8 @@ struct RowsArgs {
   const void* src;
   void* dst;
   const float* weights;   // [T, k] or null
+  const void* gates;      // combine: [T, E] of gate_dtype instead of weights, or null
+  int gate_dtype, E;
   const int* row_entries; // dispatch: [P]
   const int* ids;         // combine: [T, k]
   const int* seat_rows;   // combine: [T, k]
@@ -452,6 +454,13 @@ __global__ __launch_bounds__(kBlock) void combine_by_rows_kernel(RowsArgs a) {
     bool use[KMAX];
 #pragma unroll
     for (int j = 0; j < KMAX; ++j) use[j] = id[j] != kNone && (j == 0 || id[j] != id[j - 1]);
+    if (a.gates != nullptr) {
+      // weights straight from the gate matrix: requested with the rows, not ahead of them (the ids are
+      // known by now), so they cost no round trip of their own
+      const size_t gate0 = static_cast<size_t>(min(t0 + i, static_cast<long>(a.T) - 1)) * a.E;
+#pragma unroll
+      for (int j = 0; j < KMAX; ++j) g[j] = load_gate(a.gates, a.gate_dtype, gate0 + (use[j] ? min(max(id[j], 0), a.E - 1) : 0));
+    }
     const size_t to = static_cast<size_t>(t0 + i) * cpr;
     for (int off0 = 0; off0 < cpr; off0 += LPR * UPR) {
       float acc[UPR][NE];
@@ -642,10 +651,11 @@ extern "C" int brt_hip_dispatch_by_rows(const void* src, void* dst, const float*
   return check_launch("dispatch_by_rows_kernel");
 }
 
-extern "C" int brt_hip_combine_by_rows(const void* src, void* dst, const float* weights,
-                                       const int32_t* path_ids, const int32_t* seat_rows, int T,
-                                       int k, int cell, int P, int is_residual, int in_dtype,
-                                       int out_dtype, void* stream) {
+namespace {
+
+int combine_rows(const void* src, void* dst, const float* weights, const void* gates, int gate_dtype, int E,
+                 const int32_t* path_ids, const int32_t* seat_rows, int T, int k, int cell, int P, int is_residual,
+                 int in_dtype, int out_dtype, void* stream) {
   if (T < 0 || k <= 0 || cell < 0 || P < 0) return fail(BRT_E_INVALID, "bad shape T=%d k=%d cell=%d P=%d", T, k, cell, P);
   if (k > kMaxK) return fail(BRT_E_UNSUPPORTED, "more than %d paths per cell", kMaxK);
   if ((in_dtype != BRT_F32 && in_dtype != BRT_F16 && in_dtype != BRT_BF16) ||
@@ -659,6 +669,7 @@ extern "C" int brt_hip_combine_by_rows(const void* src, void* dst, const float* 
     return fail(BRT_E_UNSUPPORTED, "rows must be whole 16-byte units (row is %zu bytes)", row_bytes);
   RowsArgs a{};
   a.src = src; a.dst = dst; a.weights = weights; a.ids = path_ids; a.seat_rows = seat_rows;
+  a.gates = gates; a.gate_dtype = gate_dtype; a.E = E;
   a.T = T; a.P = P; a.k = k; a.is_residual = is_residual;
   a.cpr = static_cast<int>(row_bytes / 16);
   a.rows_pw = rows_per_wavefront(a.cpr, T);
@@ -683,4 +694,25 @@ extern "C" int brt_hip_combine_by_rows(const void* src, void* dst, const float* 
 #undef BRT_LAUNCH
 #undef BRT_LAUNCH_K
   return check_launch("combine_by_rows_kernel");
+}
+
+}  // namespace
+
+extern "C" int brt_hip_combine_by_rows(const void* src, void* dst, const float* weights,
+                                       const int32_t* path_ids, const int32_t* seat_rows, int T,
+                                       int k, int cell, int P, int is_residual, int in_dtype,
+                                       int out_dtype, void* stream) {
+  return combine_rows(src, dst, weights, nullptr, BRT_F32, 0, path_ids, seat_rows, T, k, cell, P, is_residual, in_dtype,
+                      out_dtype, stream);
+}
+
+extern "C" int brt_hip_combine_by_rows_gated(const void* src, void* dst, const void* gates, int gate_dtype, int E,
+                                             const int32_t* path_ids, const int32_t* seat_rows, int T, int k, int cell,
+                                             int P, int is_residual, int in_dtype, int out_dtype, void* stream) {
+  if (E <= 0 || static_cast<long>(T) * E >= (1l << 31)) return fail(BRT_E_UNSUPPORTED, "T*E >= 2^31, or no paths (E=%d)", E);
+  if (gate_dtype != BRT_F32 && gate_dtype != BRT_F16 && gate_dtype != BRT_BF16)
+    return fail(BRT_E_UNSUPPORTED, "gate dtype %d is not supported", gate_dtype);
+  if (T > 0 && !gates) return fail(BRT_E_INVALID, "null argument");
+  return combine_rows(src, dst, nullptr, gates, gate_dtype, E, path_ids, seat_rows, T, k, cell, P, is_residual, in_dtype,
+                      out_dtype, stream);
 }

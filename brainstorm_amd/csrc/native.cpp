@@ -400,7 +400,7 @@ PyObject* dispatch_by_rows(const Args& a) {  // in_data, row_entries, k, weights
   return wrap(out);
 }
 
-PyObject* combine_by_rows(const Args& a) {  // in_data, path_ids, seat_rows, weights, out_data, out_dtype
+PyObject* combine_by_rows(const Args& a) {  // in_data, path_ids, seat_rows, weights, out_data, out_dtype, gates
   const Tensor given = a.tensor(0), ids_given = a.tensor(1), seats_given = a.tensor(2), residual = a.tensor_or_none(4);
   on_device(given, "in_data"), on_device(ids_given, "path_ids");
   int32(ids_given, "path_ids");
@@ -424,6 +424,16 @@ PyObject* combine_by_rows(const Args& a) {  // in_data, path_ids, seat_rows, wei
   }
   const int out_type = code_of(out.scalar_type());
   if (out_type < 0 || (out_type != in_type && out_type != BRT_F32)) not_implemented("output data type is not supported");
+  Tensor gates = a.tensor_or_none(6);
+  if (gates.defined()) {
+    on_device(gates, "gates");
+    const int gate_type = data_type(gates, "gate data type");
+    if (gates.dim() != 2 || gates.size(0) != T) runtime_error("gates must be [cells, paths]");
+    gates = dense(gates);
+    check(brt_hip_combine_by_rows_gated(ptr(in), ptr(out), ptr(gates), gate_type, gates.size(1), iptr(ids), iptr(seats), T, k,
+                                        cell, P, residual.defined(), in_type, out_type, stream_of(in)));
+    return wrap(out);
+  }
   check(brt_hip_combine_by_rows(ptr(in), ptr(out), fptr(weights), iptr(ids), iptr(seats), T, k, cell, P, residual.defined(),
                                 in_type, out_type, stream_of(in)));
   return wrap(out);
@@ -611,7 +621,7 @@ PyMethodDef methods[] = {
     BRT_ENTRY(topk_hot_mask, 2),    BRT_ENTRY(gate_topk, 4),           BRT_ENTRY(throttle_hotmask, 3),
     BRT_ENTRY(generate, 5),         BRT_ENTRY(route_and_dispatch, 7),  BRT_ENTRY(route_by_path, 7),
     BRT_ENTRY(dispatch, 12),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
-    BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 6),     BRT_ENTRY(grouped_linear, 16),
+    BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 7),     BRT_ENTRY(grouped_linear, 16),
     BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5), BRT_ENTRY(int_list, 1),
     BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
 

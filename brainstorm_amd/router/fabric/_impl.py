@@ -577,10 +577,8 @@ class FusedCombineFabric(CombineFabric):
             if residual is not None:
                 return c_router.combine_by_row_tags(data, route.row_entries, route.cells, residual)
             return c_router.combine_by_row_tags(data, route.row_entries, route.cells)
-        weights = None
-        if gates is not None:  # the weight of every entry: the score of its cell on its path
-            weights = torch.gather(gates, 1, route.path_ids.long()).to(torch.float32)
-        return c_router.combine_by_rows(data, route.path_ids, route.seat_rows, weights, residual)
+        # weighted: every entry by the score of its cell on its path
+        return c_router.combine_by_rows(data, route.path_ids, route.seat_rows, None, residual, gates=gates)
 
     def _combine_deferred(self, data, route, state, gates, residual):
         """Combine of a route whose dispatch was deferred: tag-format indices; the row tags were

@@ -1023,3 +1023,27 @@ def test_decoder_greedy_search_protocol_on_the_gpu(brt_mod):
     with pytest.raises(NotImplementedError):
         make_protocol("decoder_beam_search", {"index_format": "seat_index", "pad_token_id": 0,
                                               "eos_token_id": eos}).cuda()(tokens)
+
+
+@pytest.mark.parametrize("T,E,d,k", [(1, 2, 8, 1), (777, 12, 96, 2), (300, 33, 1048, 5), (64, 8, 8, 8)])
+@pytest.mark.parametrize("gate_dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_combine_by_rows_takes_its_weights_from_the_gate_matrix(brt_mod, T, E, d, k, gate_dtype):
+    """gates=[cells, paths] gives the bits of weights = gates gathered at the path ids, for every lane-group
+    shape, one entry per cell, two and the most the kernel holds, dropped entries among them."""
+    c_router = brt_mod[1]
+    g = torch.Generator().manual_seed(T + k)
+    score = torch.randn(T, E, generator=g).cuda()
+    ids, _ = c_router.gate_topk(score, k)
+    caps = torch.tensor([max(1, T * k // E)], dtype=torch.int32, device="cuda")
+    _, _, seat_rows, row_entries = c_router.route_by_path(ids, E, caps)
+    gates = torch.softmax(score, dim=1).to(gate_dtype)
+    weights = torch.gather(gates, 1, ids.long()).float()
+    for dtype, out_dtype in ((torch.float32, None), (torch.bfloat16, None), (torch.float16, torch.float32)):
+        y = torch.randn(row_entries.numel(), d, generator=g).to(dtype).cuda()
+        want = c_router.combine_by_rows(y, ids, seat_rows, weights, out_dtype=out_dtype)
+        assert torch.equal(c_router.combine_by_rows(y, ids, seat_rows, out_dtype=out_dtype, gates=gates), want)
+        residual = torch.randn(T, d, generator=g).to(out_dtype or dtype).cuda()
+        want = c_router.combine_by_rows(y, ids, seat_rows, weights, residual.clone())
+        assert torch.equal(c_router.combine_by_rows(y, ids, seat_rows, None, residual, gates=gates), want)
+    with pytest.raises(RuntimeError):
+        c_router.combine_by_rows(y, ids, seat_rows, weights, gates=gates)
