@@ -29,7 +29,11 @@ constexpr int kWholeWaves = 8;    // a small route: one workgroup of 8 wavefront
 constexpr int kWholeChunks = 32;  // ... up to this many chunks of 64 entries
 constexpr int kSplitWaves = 4;    // larger routes: workgroups of 4 wavefronts, two launches
 constexpr int kSplitGroups = 32;  // ... in at most this many workgroups
-constexpr int kSoloEntries = 65536;  // routes up to this many entries: one launch, every workgroup counts the whole route
+// Routes up to this many entries: one launch, every workgroup counts the whole route.  Against two
+// launches: 32768 entries 8.2 / 8.9 us against 8.0 / 8.4 us on the device (16 paths / 32 skewed ones), but one
+// launch less for the host; 65536 entries 13.1 / 14.3 us against 10.1 / 10.7 us (8 / 64 paths).  With more than
+// 128 paths the two launches hand over more counters: 65536 entries, 256 paths 16.5 us against 21.0 us.
+constexpr int kSoloEntries = 32768, kSoloEntriesManyPaths = 65536, kManyPaths = 128;
 constexpr int kSplitWavesLarge = 16;  // ... of 16 wavefronts for routes beyond 32768 entries
 constexpr int kBatch = 4;        // chunks of 64 entries a wavefront keeps in flight
 constexpr int kMaxK = 8;         // paths per cell in combine_by_rows
@@ -155,6 +159,13 @@ __device__ __forceinline__ void sum_rows(Ptr cnt, int rows, int mine, int E, int
 // every workgroup takes them from a histogram of the whole id vector (at most 256 KB, read from
 // the L2) built with LDS atomics, one add per entry, instead of waiting for a counting kernel; only
 // its own range is ranked with the ballots.  No workgroup waits for another.
+//   Bound by the LDS: adds of a wavefront that meet in one word are serialised, and with one counter
+// per path a popular path collects dozens of them.  The histogram therefore keeps WAVES copies of every
+// counter, lane l adding to copy l % WAVES, in different banks; 8 wavefronts instead of 4 halve what
+// is left for routes beyond 8192 entries.  One counter and 4 wavefronts -> copies: 32768 entries on 32 paths skewed by
+// Zipf(1.2) 21.0 -> 8.9 us, on 16 even paths 12.2 -> 8.3 us, 8192 entries on 16 skewed paths 7.0 -> 5.1 us, on 64
+// even ones 5.3 -> 5.4 us.  (A byte per path in a column of every thread's own, four paths to a word, has
+// no conflicts at all, but clearing and summing the columns costs 3 us: 10.0 us for the skewed 32768.)
 enum RouteMode { kWhole = 0, kCount = 1, kEmit = 2, kSolo = 3 };
 
 template <int MODE, int WAVES>
@@ -167,8 +178,10 @@ __global__ __launch_bounds__(WAVES * kWave) void route_kernel(RouteArgs a) {
   int* s_load = s_seat + WAVES * E;                         // [E]
   int* s_start = s_load + E;                                // [E]
   int* s_kept = s_start + E;                                // [E] rows a path really fills
-  int* s_hist = s_kept + E;                                 // kSolo: [2][E] entries before this workgroup's range / from it on
-  int* s_caps = s_hist + (MODE == kSolo ? 2 * E : 0);       // [caps_in_lds]
+  constexpr int kCopies = WAVES;                            // of every counter of the histogram
+  const int hist_row = E | 1;                               // odd: the copies of a counter lie in different banks
+  int* s_hist = s_kept + E;                                 // kSolo: [2][kCopies][hist_row] entries before this workgroup's range / from it on
+  int* s_caps = s_hist + (MODE == kSolo ? 2 * kCopies * hist_row : 0);  // [caps_in_lds]
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x >> 6;
   const int unit = blockIdx.x * WAVES + w;
   constexpr int kStep = kWave * kBatch;
@@ -192,20 +205,20 @@ __global__ __launch_bounds__(WAVES * kWave) void route_kernel(RouteArgs a) {
   if (MODE != kEmit)
     for (int i = threadIdx.x; i < WAVES * E; i += WAVES * kWave) s_cnt[i] = 0;
   if (MODE == kSolo)
-    for (int i = threadIdx.x; i < 2 * E; i += WAVES * kWave) s_hist[i] = 0;
+    for (int i = threadIdx.x; i < 2 * kCopies * hist_row; i += WAVES * kWave) s_hist[i] = 0;
   __syncthreads();
   const int* caps = a.caps_in_lds != 0 ? s_caps : a.caps;
 
   if constexpr (MODE == kSolo) {
-    // histogram of every entry, split at the start of this workgroup's range: 16 ids per lane in
-    // flight, one LDS add each (the adds of a wavefront to one counter are serialised by the
-    // LDS, which for ids spread over the paths is a handful of passes)
+    // histogram of every entry, split at the start of this workgroup's range: 32 ids per lane in
+    // flight, one LDS add each
     const int own_lo = static_cast<int>(min(static_cast<long>(a.n), static_cast<long>(blockIdx.x) * WAVES * a.per_wave));
     constexpr int kFlight = 8, kThreads = WAVES * kWave;
     typedef int i32x4 __attribute__((ext_vector_type(4)));
     const bool quads = (reinterpret_cast<uintptr_t>(a.ids) & 15) == 0;  // 16-byte loads of 4 ids
     const int nq = quads ? a.n >> 2 : 0;
     const i32x4* ids4 = reinterpret_cast<const i32x4*>(a.ids);
+    int* const copy = s_hist + (threadIdx.x % kCopies) * hist_row;
 #pragma unroll 1
     for (int base = 0; base < nq; base += kFlight * kThreads) {
       i32x4 id[kFlight];
@@ -218,14 +231,14 @@ __global__ __launch_bounds__(WAVES * kWave) void route_kernel(RouteArgs a) {
         for (int c = 0; c < 4; ++c) {
           const int i = i4 * 4 + c, e = id[q][c];
           if (i4 < nq && e >= 0 && e < E)
-            __hip_atomic_fetch_add(&s_hist[(i < own_lo ? 0 : E) + e], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_fetch_add(&copy[(i < own_lo ? 0 : kCopies * hist_row) + e], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
       }
     }
     for (int i = nq * 4 + threadIdx.x; i < a.n; i += kThreads) {  // the tail, or everything behind a misaligned pointer
       const int e = a.ids[i];
       if (e >= 0 && e < E)
-        __hip_atomic_fetch_add(&s_hist[(i < own_lo ? 0 : E) + e], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add(&copy[(i < own_lo ? 0 : kCopies * hist_row) + e], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
   }
 
@@ -264,8 +277,15 @@ __global__ __launch_bounds__(WAVES * kWave) void route_kernel(RouteArgs a) {
     } else if constexpr (MODE == kSolo) {
       int own = 0;
       sum_rows<WAVES>(s_cnt, WAVES, w, E, e, &before, &own);
-      before += e < E ? s_hist[e] : 0;
-      total = e < E ? s_hist[e] + s_hist[E + e] : 0;
+      const int col = min(e, E - 1);
+      int ahead = 0, rest = 0;
+#pragma unroll
+      for (int c = 0; c < kCopies; ++c) {
+        ahead += s_hist[c * hist_row + col];
+        rest += s_hist[(kCopies + c) * hist_row + col];
+      }
+      before += ahead;
+      total = ahead + rest;
     } else if (e0 == 0) {
       before = before0;
       total = total0;
@@ -575,13 +595,19 @@ extern "C" int brt_hip_route_by_path(const int32_t* path_ids, int T, int k, int 
     hipLaunchKernelGGL((route_kernel<kWhole, kWholeWaves>), dim3(1), dim3(kWholeWaves * kWave), lds_bytes, st, a);
     return check_launch("route_kernel");
   }
-  if (n <= kSoloEntries) {
-    // one launch: workgroups of 4 wavefronts, each wavefront a whole number of chunks of its own
-    const int groups = std::min(kSplitGroups, (chunks + kSplitWaves - 1) / kSplitWaves);
-    a.per_wave = (chunks + groups * kSplitWaves - 1) / (groups * kSplitWaves) * kWave;
-    const size_t lds_bytes = (static_cast<size_t>(2 * kSplitWaves + 5) * E + a.caps_in_lds) * sizeof(int);
-    hipLaunchKernelGGL((route_kernel<kSolo, kSplitWaves>), dim3(groups), dim3(kSplitWaves * kWave), lds_bytes, st, a);
-    return check_launch("route_kernel");
+  if (n <= (E > kManyPaths ? kSoloEntriesManyPaths : kSoloEntries)) {
+    // one launch: each wavefront owns a whole number of chunks
+    auto solo = [&](auto waves) {
+      constexpr int kWaves = decltype(waves)::value;
+      const int groups = std::min(kSplitGroups, (chunks + kWaves - 1) / kWaves);
+      a.per_wave = (chunks + groups * kWaves - 1) / (groups * kWaves) * kWave;
+      const size_t words = static_cast<size_t>(2 * kWaves + 3) * E + 2 * kWaves * (E | 1) + a.caps_in_lds;
+      hipLaunchKernelGGL((route_kernel<kSolo, kWaves>), dim3(groups), dim3(kWaves * kWave), words * sizeof(int), st, a);
+      return check_launch("route_kernel");
+    };
+    // 8 wavefronts keep 35 words of LDS per path (64 KB: up to 430 paths), and pay off beyond 8192 entries
+    if (n > 8192 && E <= 256) return solo(std::integral_constant<int, 8>{});
+    return solo(std::integral_constant<int, 4>{});
   }
   int waves;
   split_geometry(n, &waves, &a.units, &a.per_wave);

@@ -708,6 +708,25 @@ def test_route_by_path_bit_exact(hip, T, E, k, hole, mode):
         assert np.array_equal(g, w), name
 
 
+@pytest.mark.parametrize("n,E", [
+    (2049, 1), (2050, 3), (8192, 64), (10810, 512),   # one launch, 4 wavefronts
+    (8193, 5), (32768, 128), (65536, 129), (30001, 256),  # one launch, 8 wavefronts
+    (65536, 257),                                     # many paths: 4 wavefronts whatever the entries
+    (32769, 128), (65537, 129),                       # two launches
+])
+@pytest.mark.parametrize("ids_of", ["one_path", "random"])
+def test_route_by_path_at_the_edges_of_its_forms(hip, n, E, ids_of):
+    """The one-launch and two-launch forms at the edges of their entries and paths, with every entry on
+    one path, ids outside the paths and a last workgroup that owns nothing."""
+    rng = np.random.default_rng(n + E)
+    ids = np.full((n, 1), E - 1) if ids_of == "one_path" else rng.integers(-1, E + 2, (n, 1))
+    ids = ids.astype(np.int32)
+    want = oracle.route_by_path(ids, E, [n // 2], False, False, 0, n)
+    got = hip.route_by_path(ids, E, [n // 2], False, False, 0, n)
+    for g, w, name in zip(got, want, ("loads", "counts", "seat_rows", "row_entries")):
+        assert np.array_equal(g, w), name
+
+
 def test_route_by_path_path_wise_padding_and_bad_arguments(hip):
     ids = _compact_route(500, 8, 2, seed=1)
     ids[ids == 3] = -1                                        # nobody takes path 3
