@@ -41,6 +41,7 @@ struct Raised : std::runtime_error {
   Raised(PyObject* t, const std::string& what) : std::runtime_error(what), type(t) {}
 };
 [[noreturn]] void runtime_error(const std::string& what) { throw Raised(PyExc_RuntimeError, what); }
+[[noreturn]] void index_error(const std::string& what) { throw Raised(PyExc_IndexError, what); }
 [[noreturn]] void not_implemented(const std::string& what) { throw Raised(PyExc_NotImplementedError, what); }
 
 void check(int code) {
@@ -103,6 +104,10 @@ void on_device(const Tensor& t, const char* name) {
 void int32(const Tensor& t, const char* name) {
   if (t.scalar_type() != at::kInt)
     runtime_error(std::string(name) + " must be an int32 tensor, got " + c10::toString(t.scalar_type()));
+}
+int64_t divided(int64_t a, int64_t b) {
+  if (b == 0) throw Raised(PyExc_ZeroDivisionError, "no cells or no paths to divide by");
+  return a / b;
 }
 int code_of(at::ScalarType t) {  // BRT_F32 / BRT_F16 / BRT_BF16, -1 for anything else
   return t == at::kFloat ? BRT_F32 : t == at::kHalf ? BRT_F16 : t == at::kBFloat16 ? BRT_BF16 : -1;
@@ -284,12 +289,13 @@ PyObject* dispatch(const Args& a) {
   const Tensor in = dense(given);
   const c10::DeviceGuard guard(in.device());
   const int64_t T = in.size(0), E = route.size(1);
-  int64_t cell = in.numel() / T;
+  int64_t cell = divided(in.numel(), T);
   at::DimVector shape(in.sizes().begin(), in.sizes().end());
   if (one_d) {
     shape[0] = total;
   } else {
-    cell /= E;
+    cell = divided(cell, E);
+    if (shape.size() < 2) index_error("2-d routing needs a [cells, paths, ...] input");
     if (shape.size() == 2) shape.push_back(1);
     shape[1] = total;
     shape.erase(shape.begin());
@@ -324,7 +330,7 @@ PyObject* combine(const Args& a) {
   const int in_type = data_type(in, "data type");
   const c10::DeviceGuard guard(in.device());
   const int64_t T = route.size(0), E = route.size(1), P = in.size(0), cell = P > 0 ? in.numel() / P : 0;
-  const int64_t mpl = a.flag(6) ? P / E : 0;  // router.cc:427-430
+  const int64_t mpl = a.flag(6) ? divided(P, E) : 0;  // router.cc:427-430
   if (gates.defined()) {
     on_device(gates, "gates");
     data_type(gates, "gate data type");

@@ -2,6 +2,9 @@
 import os
 import re
 
+import pytest
+import torch
+
 from brainstorm_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -107,3 +110,18 @@ def test_counts_of_two_to_the_31_and_more_are_refused():
     assert handle.brt_hip_route_by_path(None, 1 << 30, 2, E, None, 0, 0, 0, 0, None, None, None,
                                         None, 0, None, 0, None) == -4
     assert b"T*k" in handle.brt_hip_last_error()
+
+
+def test_native_ops_refuse_shapes_without_paths_or_columns_as_exceptions():
+    """Divisions by the paths and the second dimension of a 2-d route are checked in the native code (no
+    trap, no write past the shape), before anything is allocated or launched."""
+    native = _lib.native()
+    none = torch.zeros(0, dtype=torch.int32)
+    with pytest.raises(ZeroDivisionError):
+        native.dispatch(torch.zeros(4, 0), torch.zeros(4, 0, dtype=torch.int32), none, None, None, None, False, 0, 0,
+                        False, False, True)
+    with pytest.raises(IndexError):
+        native.dispatch(torch.zeros(4), torch.zeros(4, 2, dtype=torch.int32), none, None, None, None, False, 0, 0,
+                        False, False, True)
+    with pytest.raises(ZeroDivisionError):
+        native.combine(torch.zeros(4, 8), torch.zeros(4, 0, dtype=torch.int32), none, None, None, None, True, None)
