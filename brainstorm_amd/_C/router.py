@@ -644,4 +644,8 @@ def combine_by_rows(in_data: torch.Tensor, path_ids: torch.Tensor, seat_rows: to
     ``gates[t, path_ids[t,j]]``."""
     if gates is not None and weights is not None:
         raise RuntimeError("weights or gates, not both")
+    if gates is not None and not (gates.dtype in _DT and gates.dim() == 2 and gates.size(0) == path_ids.size(0)
+                                  and gates.numel() < 1 << 31):
+        # what the kernel does not read in place: other types (fp64 gates), more rows than cells
+        weights, gates = torch.gather(gates, 1, path_ids.long()).to(torch.float32), None
     return _lib.native().combine_by_rows(in_data, path_ids, seat_rows, weights, out_data, out_dtype, gates)

@@ -1026,7 +1026,7 @@ def test_decoder_greedy_search_protocol_on_the_gpu(brt_mod):
 
 
 @pytest.mark.parametrize("T,E,d,k", [(1, 2, 8, 1), (777, 12, 96, 2), (300, 33, 1048, 5), (64, 8, 8, 8)])
-@pytest.mark.parametrize("gate_dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("gate_dtype", [torch.float32, torch.float16, torch.bfloat16, torch.float64])
 def test_combine_by_rows_takes_its_weights_from_the_gate_matrix(brt_mod, T, E, d, k, gate_dtype):
     """gates=[cells, paths] gives the bits of weights = gates gathered at the path ids, for every lane-group
     shape, one entry per cell, two and the most the kernel holds, dropped entries among them."""
@@ -1042,6 +1042,8 @@ def test_combine_by_rows_takes_its_weights_from_the_gate_matrix(brt_mod, T, E, d
         y = torch.randn(row_entries.numel(), d, generator=g).to(dtype).cuda()
         want = c_router.combine_by_rows(y, ids, seat_rows, weights, out_dtype=out_dtype)
         assert torch.equal(c_router.combine_by_rows(y, ids, seat_rows, out_dtype=out_dtype, gates=gates), want)
+        longer = torch.cat([gates, gates[:1]])  # more rows than cells: the last ones belong to no cell
+        assert torch.equal(c_router.combine_by_rows(y, ids, seat_rows, out_dtype=out_dtype, gates=longer), want)
         residual = torch.randn(T, d, generator=g).to(out_dtype or dtype).cuda()
         want = c_router.combine_by_rows(y, ids, seat_rows, weights, residual.clone())
         assert torch.equal(c_router.combine_by_rows(y, ids, seat_rows, None, residual, gates=gates), want)
