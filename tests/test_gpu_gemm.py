@@ -517,6 +517,8 @@ def test_experts_with_many_row_blocks_in_patch_order(loads, K, N):
     ([70] * 70 + [6000, 3000, 5000], 128, 4096),               # more than 64 experts
     ([1824] * 8, 256, 1024),                                  # one round: 256 tiles for 256 CUs
     ([2000, 1700, 300, 1900, 1, 1800, 2047, 1500], 128, 1000),  # one round, ragged, N tail
+    # last row blocks of every number of 32-row tiles, shared by the two groups of wavefronts
+    ([768 + r for r in (1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 255)], 192, 2048),
 ])
 def test_ping_pong_tiles(loads, K, N):
     """Shapes the host sends to the 256 x 256 ping-pong kernel: experts that average more than 160
