@@ -138,21 +138,37 @@ __device__ __forceinline__ int sum_over_rows_in_wave(int v, int ep_shift) {
   return v;
 }
 
-// Second walk over one batch of row words held in registers: turns the mask words
-// into seats / throttled bits / tag slots.  Rows of one load are ordered by lane
-// group; all cross-lane traffic of the batch is issued first and does not depend
-// on the running sum (incl = sum over the groups up to and including this
-// lane's, tot = sum over all groups).
-template <int MODE>
-__device__ __forceinline__ void walk_batch(const int (&m)[kBatch], int i0, int n_ins, int& carry,
-                                           int thr, int total, long row_w, int rps, int ep, int sub,
-                                           int e, int lane, int col, bool col_ok, const ScanArgs& a) {
-  int incl[kBatch], tot[kBatch];
+// Sums over the rows that one load covers, for a batch of loads: incl = over the lane groups up to
+// and including this lane's, tot = over all groups, of the lanes that hold the same path.  A hot mask
+// holds zeros and ones, whose sums are bit counts of a ballot: six vector instructions per load, no
+// cross-lane move.  Words of any other value take a shuffle per doubling of the rows, whose latencies
+// add up: with 8 paths (8 rows per load, four shuffles) they were a third of the kernel.  Ballots here and
+// buffer loads below: 100352 x 8 throttled 10.2 -> 6.5 us, seat indices 8.5 -> 5.2 us; 16384 x 32 8.3 -> 6.2
+// and 6.7 -> 5.1 us.
+__device__ __forceinline__ void sums_of_loads(const int (&m)[kBatch], int n, int rps, int ep, int e, int lane,
+                                              int (&incl)[kBatch], int (&tot)[kBatch]) {
+  int other = 0;
 #pragma unroll
   for (int u = 0; u < kBatch; ++u) {
-    incl[u] = m[u];
-    tot[u] = m[u];
-    if (rps > 1 && i0 + u < n_ins) {  // wave-uniform
+    incl[u] = tot[u] = m[u];
+    other |= m[u] & ~1;
+  }
+  if (rps == 1) return;
+  if (__ballot(other != 0) == 0) {
+    unsigned long long path = 1ull << e;  // the lanes of this lane's path
+    for (int d = ep; d < kWave; d <<= 1) path |= path << d;
+    const unsigned long long upto = path & ((2ull << lane) - 1ull);  // ... up to this lane
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const unsigned long long ones = __ballot(m[u] != 0);  // zero behind the wavefront's last load
+      incl[u] = __popcll(ones & upto);
+      tot[u] = __popcll(ones & path);
+    }
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < kBatch; ++u) {
+    if (u < n) {  // wave-uniform
       int x = m[u];
       for (int d = ep; d < kWave; d <<= 1) {
         const int t = __shfl_up(x, d, kWave);
@@ -162,6 +178,17 @@ __device__ __forceinline__ void walk_batch(const int (&m)[kBatch], int i0, int n
       tot[u] = __shfl(x, (rps - 1) * ep + e, kWave);
     }
   }
+}
+
+// Second walk over one batch of row words held in registers: turns the mask words
+// into seats / throttled bits / tag slots.  The sums over the rows of every load come first and do
+// not depend on the running sum.
+template <int MODE>
+__device__ __forceinline__ void walk_batch(const int (&m)[kBatch], int i0, int n_ins, int& carry,
+                                           int thr, int total, long row_w, int rps, int ep, int sub,
+                                           int e, int lane, int col, bool col_ok, const ScanArgs& a) {
+  int incl[kBatch], tot[kBatch];
+  sums_of_loads(m, n_ins - i0, rps, ep, e, lane, incl, tot);
   // rows of this wavefront through one 64-bit base and 32-bit offsets: the address of every
   // store is one instruction instead of a 64-bit multiply-add chain
   int* __restrict__ out_w = a.out + row_w * a.E;
@@ -188,40 +215,63 @@ __device__ __forceinline__ void walk_batch(const int (&m)[kBatch], int i0, int n
   }
 }
 
-// Loads one batch of row words (zero beyond the band / the matrix).  One 64-bit base per
-// wavefront and 32-bit offsets; the loads are unconditional (a word outside the wavefront's rows
-// is read from its first row and dropped), so that they issue back to back.
-__device__ __forceinline__ void load_batch(int (&v)[kBatch], int i0, int n_ins, long row_w, int rps,
-                                           int sub, int col, bool col_ok, const ScanArgs& a) {
-  const int* __restrict__ mask_w = a.mask + min(row_w, a.T - 1l) * a.E;
-  const int rows_here = static_cast<int>(max(0l, min(static_cast<long>(a.rows_pw), a.T - row_w)));
-  bool ok[kBatch];
+// A buffer over `bytes` from base: a word outside reads as zero, so loads need no predicate, select or
+// 64-bit address of their own and issue back to back.
+constexpr unsigned kOutside = 0x80000000u;  // offset past any extent
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t words_at(const void* base, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0,
+                                           static_cast<int>(min(bytes, static_cast<size_t>(0x7fffffff))), 0x00020000);
+}
+
+// The rows of one wavefront as a buffer (empty for a wavefront past the matrix).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_of_wave(long row_w, const ScanArgs& a) {
+  const long rows_here = max(0l, min(static_cast<long>(a.rows_pw), a.T - row_w));
+  return words_at(a.mask + (rows_here > 0 ? row_w : 0) * a.E, static_cast<size_t>(rows_here) * a.E * 4);
+}
+
+// Loads one batch of row words (zero beyond the band / the matrix).
+__device__ __forceinline__ void load_batch(int (&v)[kBatch], __amdgpu_buffer_rsrc_t rows, int i0, int rps, int sub,
+                                           int col, bool col_ok, const ScanArgs& a) {
+  const unsigned first = col_ok ? (static_cast<unsigned>(i0 * rps + sub) * a.E + col) * 4u : kOutside;
+  const unsigned step = rps * a.E * 4u;
 #pragma unroll
-  for (int u = 0; u < kBatch; ++u) {
-    const int rl = (i0 + u) * rps + sub;
-    ok[u] = i0 + u < n_ins && col_ok && rl < rows_here;
-    v[u] = mask_w[ok[u] ? static_cast<unsigned>(rl) * a.E + col : 0u];
+  for (int u = 0; u < kBatch; ++u) v[u] = __builtin_amdgcn_raw_buffer_load_b32(rows, first + u * step, 0, 0);
+}
+
+// This lane's share of the column sums of bands [j0, end), every `step`-th of them.
+__device__ __forceinline__ int sum_of_bands(int j0, int end, int step, int col, bool col_ok, const ScanArgs& a) {
+  const __amdgpu_buffer_rsrc_t sums = words_at(a.partial, static_cast<size_t>(end) * a.E * 4);
+  int total = 0;
+  for (; j0 < end; j0 += step * kPartialBatch) {
+    int v[kPartialBatch];
+    const unsigned first = col_ok ? (static_cast<unsigned>(j0) * a.E + col) * 4u : kOutside;
+#pragma unroll
+    for (int u = 0; u < kPartialBatch; ++u)
+      v[u] = __builtin_amdgcn_raw_buffer_load_b32(sums, first + u * (step * a.E * 4u), 0, 0);
+#pragma unroll
+    for (int u = 0; u < kPartialBatch; ++u) total += v[u];
   }
-#pragma unroll
-  for (int u = 0; u < kBatch; ++u) v[u] = ok[u] ? v[u] : 0;
+  return total;
 }
 
 // pass 1: column sums of one band
 __global__ __launch_bounds__(kBlock) void band_count_kernel(ScanArgs a) {
   __shared__ int s_sum[kWavesPB][kWave];
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int E = a.E;
   const int ep = 1 << a.ep_shift, rps = kWave >> a.ep_shift;
   const int e = lane & (ep - 1), sub = lane >> a.ep_shift;
   const long row_w = (static_cast<long>(blockIdx.x) * kWavesPB + wave) * a.rows_pw;
   const int n_ins = a.n_ins;
+  const __amdgpu_buffer_rsrc_t rows = rows_of_wave(row_w, a);
   for (int c0 = 0; c0 < E; c0 += kWave) {
     const int col = c0 + e;
     const bool col_ok = col < E;
     int sum = 0;
     for (int i0 = 0; i0 < n_ins; i0 += kBatch) {
       int v[kBatch];
-      load_batch(v, i0, n_ins, row_w, rps, sub, col, col_ok, a);
+      load_batch(v, rows, i0, rps, sub, col, col_ok, a);
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) sum += v[u];
     }
@@ -246,56 +296,32 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
   __shared__ int s_above[kWavesPB][kWave];  // each wave's share of the sum over earlier bands
   __shared__ int s_own[kWavesPB][kWave];    // column sums of each wave's own rows
   __shared__ int s_below[kWavesPB][kWave];  // tag mode: share of the sum over later bands
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int E = a.E, band = blockIdx.x;
   const int ep = 1 << a.ep_shift, rps = kWave >> a.ep_shift;
   const int e = lane & (ep - 1), sub = lane >> a.ep_shift;
   const long row_w = (static_cast<long>(band) * kWavesPB + wave) * a.rows_pw;
   const int n_ins = a.n_ins;
+  const __amdgpu_buffer_rsrc_t rows = rows_of_wave(row_w, a);
 
   for (int c0 = 0; c0 < E; c0 += kWave) {
     const int col = c0 + e;
     const bool col_ok = col < E;
     // ---- own rows: the first batch stays in registers ---------------------------------
     int m0[kBatch];
-    load_batch(m0, 0, n_ins, row_w, rps, sub, col, col_ok, a);
+    load_batch(m0, rows, 0, rps, sub, col, col_ok, a);
     // ---- this wave's share of the offset: bands wave, wave+4, ... above this one ----
-    int above = 0, below = 0;
-    for (int j0 = wave + sub * kWavesPB; j0 < band; j0 += kWavesPB * rps * kPartialBatch) {
-      // unconditional loads through 32-bit offsets (an entry that does not count is read from
-      // the head of the table and dropped), so that they issue back to back
-      int v[kPartialBatch];
-      bool ok[kPartialBatch];
-#pragma unroll
-      for (int u = 0; u < kPartialBatch; ++u) {
-        const int j = j0 + u * kWavesPB * rps;
-        ok[u] = j < band && col_ok;
-        v[u] = a.partial[ok[u] ? static_cast<unsigned>(j) * E + col : 0u];
-      }
-#pragma unroll
-      for (int u = 0; u < kPartialBatch; ++u) above += ok[u] ? v[u] : 0;
-    }
-    if (MODE == kTag) {  // the tag list of a path ends at its total: the later bands count too
-      for (int j0 = band + 1 + wave + sub * kWavesPB; j0 < a.bands; j0 += kWavesPB * rps * kPartialBatch) {
-        int v[kPartialBatch];
-        bool ok[kPartialBatch];
-#pragma unroll
-        for (int u = 0; u < kPartialBatch; ++u) {
-          const int j = j0 + u * kWavesPB * rps;
-          ok[u] = j < a.bands && col_ok;
-          v[u] = a.partial[ok[u] ? static_cast<unsigned>(j) * E + col : 0u];
-        }
-#pragma unroll
-        for (int u = 0; u < kPartialBatch; ++u) below += ok[u] ? v[u] : 0;
-      }
-      below = sum_over_rows_in_wave(below, a.ep_shift);
-    }
+    int above = sum_of_bands(wave + sub * kWavesPB, band, kWavesPB * rps, col, col_ok, a), below = 0;
+    if (MODE == kTag)  // the tag list of a path ends at its total: the later bands count too
+      below = sum_over_rows_in_wave(sum_of_bands(band + 1 + wave + sub * kWavesPB, a.bands, kWavesPB * rps, col, col_ok, a),
+                                    a.ep_shift);
     int own = 0;
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) own += m0[u];
     for (int i0 = kBatch; i0 < n_ins; i0 += kBatch) {
       int v[kBatch];
-      load_batch(v, i0, n_ins, row_w, rps, sub, col, col_ok, a);
+      load_batch(v, rows, i0, rps, sub, col, col_ok, a);
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) own += v[u];
     }
@@ -334,7 +360,7 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
     walk_batch<MODE>(m0, 0, n_ins, carry, thr, total, row_w, rps, ep, sub, e, lane, col, col_ok, a);
     for (int i0 = kBatch; i0 < n_ins; i0 += kBatch) {
       int v[kBatch];
-      load_batch(v, i0, n_ins, row_w, rps, sub, col, col_ok, a);
+      load_batch(v, rows, i0, rps, sub, col, col_ok, a);
       walk_batch<MODE>(v, i0, n_ins, carry, thr, total, row_w, rps, ep, sub, e, lane, col, col_ok, a);
     }
 
@@ -398,18 +424,13 @@ __global__ __launch_bounds__(kBlock) void band_apply_dispatch_kernel(FusedArgs f
   // wavefront's rows, a band past the last, a lane past E) reads as zero -- no 64-bit address
   // arithmetic, no branch and no select stands between the loads, so all of them are in flight
   // before the first is used.
-  constexpr unsigned kOutside = 0x80000000u;
-  auto resource = [](const void* base, size_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0,
-                                             static_cast<int>(std::min<size_t>(bytes, 0x7fffffff)), 0x00020000);
-  };
   // Issue order = order of use (the memory counter retires loads in order): band sums, own mask
   // words, capacities, and last the wavefront's rows, which are stored at the very end.
   // ---- sums of the other bands (the host keeps the bands within kFusedPartials loads per lane) ----
   int part[kFusedPartials];
   const int j_first = wave + sub * kWavesPB, j_step = kWavesPB * rps;
   {
-    const __amdgpu_buffer_rsrc_t res_partial = resource(a.partial, static_cast<size_t>(a.bands) * E * 4);
+    const __amdgpu_buffer_rsrc_t res_partial = words_at(a.partial, static_cast<size_t>(a.bands) * E * 4);
     const unsigned partial_off = col_ok ? (j_first * E + e) * 4 : kOutside;
 #pragma unroll
     for (int u = 0; u < kFusedPartials; ++u)
@@ -419,20 +440,20 @@ __global__ __launch_bounds__(kBlock) void band_apply_dispatch_kernel(FusedArgs f
   int m0[kBatch];
   {
     const __amdgpu_buffer_rsrc_t res_mask =
-        resource(a.mask + (rows_here > 0 ? row_w : 0) * E, static_cast<size_t>(rows_here) * E * 4);
+        words_at(a.mask + (rows_here > 0 ? row_w : 0) * E, static_cast<size_t>(rows_here) * E * 4);
     const unsigned mask_off = col_ok ? (sub * E + e) * 4 : kOutside;
 #pragma unroll
     for (int u = 0; u < kBatch; ++u)
       m0[u] = __builtin_amdgcn_raw_buffer_load_b32(res_mask, mask_off + u * rps * E * 4, 0, 0);
   }
   // ---- capacity menu: lane i fetches entry i, lane e the path's own capacity (path-wise padding) ----
-  const __amdgpu_buffer_rsrc_t res_caps = resource(a.caps, static_cast<size_t>(a.C) * 4);
+  const __amdgpu_buffer_rsrc_t res_caps = words_at(a.caps, static_cast<size_t>(a.C) * 4);
   const int cap_lane = __builtin_amdgcn_raw_buffer_load_b32(res_caps, lane * 4, 0, 0);
   const int cap_own = __builtin_amdgcn_raw_buffer_load_b32(res_caps, col_ok ? e * 4 : kOutside, 0, 0);
   // ---- the wavefront's rows ------------------------------------------------------------------
   const int n_units = rows_here * cpr;
   const __amdgpu_buffer_rsrc_t res_rows =
-      resource(f.src + (rows_here > 0 ? row_w : 0) * cpr, static_cast<size_t>(n_units) * 16);
+      words_at(f.src + (rows_here > 0 ? row_w : 0) * cpr, static_cast<size_t>(n_units) * 16);
   u32x4 val[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i)
@@ -496,20 +517,7 @@ __global__ __launch_bounds__(kBlock) void band_apply_dispatch_kernel(FusedArgs f
   // ---- walk the rows: seats out, destination rows into the wavefront's table ----------------
   {
     int incl[kBatch], tot[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      incl[u] = m0[u];
-      tot[u] = m0[u];
-      if (rps > 1 && u < n_ins) {
-        int x = m0[u];
-        for (int d = ep; d < kWave; d <<= 1) {
-          const int t = __shfl_up(x, d, kWave);
-          if (lane >= d) x += t;
-        }
-        incl[u] = x;
-        tot[u] = __shfl(x, (rps - 1) * ep + e, kWave);
-      }
-    }
+    sums_of_loads(m0, n_ins, rps, ep, e, lane, incl, tot);
     int* __restrict__ out_w = a.out + row_w * E;
     const unsigned long long seg0 = ep == kWave ? ~0ull : ((1ull << ep) - 1ull);
 #pragma unroll

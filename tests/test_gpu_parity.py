@@ -66,6 +66,17 @@ def test_indices_general_mask_values_and_misaligned_buffers(hip):
     want = oracle.generate_indices_and_loads(mask)
     got = hip.generate_indices_and_loads(mask)
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    for T, E in ((3000, 1), (777, 3), (9000, 8), (2600, 31), (5000, 33), (300, 70)):  # 64 to 1 rows per load
+        mask = bernoulli_mask(T, E, 0.3, seed=T)
+        mask[T // 2 + 5:: 11] *= 3  # wavefronts of ones only, of ones and other values
+        mask[-1] = -2
+        want = oracle.generate_indices_and_loads(mask)
+        got = hip.generate_indices_and_loads(mask)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        prefix, threshold = np.full(E, 2, np.int32), np.full(E, T // 5, np.int32)
+        want = oracle.throttle_hotmask(mask, prefix, threshold)
+        got = hip.throttle_hotmask(mask, prefix, threshold)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     mask = bernoulli_mask(3001, 10, 0.2, seed=6)
     for tag in (False, True):
         want = oracle.generate_indices_and_loads(mask, is_tag_index=tag)
