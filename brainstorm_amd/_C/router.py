@@ -462,6 +462,9 @@ def fuse_split_cells_from_paths(
     return [out_data]
 
 
+_UNIQUE_WHOLE_MAX = 1 << 15  # BRT_UNIQUE_WHOLE_MAX
+
+
 def _unique_tags(tags: torch.Tensor):
     """``torch.unique(tags, sorted=True, return_inverse=True)`` (router.cc:362-366) without the
     sort: tags are cell numbers, so a presence table over ``[min, max]`` and one prefix sum give
@@ -472,7 +475,12 @@ def _unique_tags(tags: torch.Tensor):
         return torch.unique(tags, sorted=True, return_inverse=True)
     with _device_guard(tags.device):
         tags = tags.contiguous()
-        lo, hi = (int(v) for v in torch.stack(torch.aminmax(tags)).tolist())
+        if n <= _UNIQUE_WHOLE_MAX:  # one launch that finds the range itself, one read-back
+            unique, inverse, lo, hi = _lib.native().unique_tags(tags)
+            if unique is not None:
+                return unique, inverse
+        else:
+            lo, hi = (int(v) for v in torch.stack(torch.aminmax(tags)).tolist())
         span = hi - lo + 1
         ws_bytes = _lib.lib().brt_hip_unique_tags_workspace_bytes(lo, hi)
         if ws_bytes == 0 or span > 16 * n + (1 << 16):

@@ -574,8 +574,22 @@ PyObject* cast_f32_to_bf16(const Args& a) {
 }
 
 // ---- host reads --------------------------------------------------------------------------------------
-// The values of an int32 vector as a list: one copy to pinned memory on the current stream, which is then
-// waited for (other Python threads run meanwhile).
+// Copies from the device on the current stream into pinned memory and waits for the copy (other Python
+// threads run meanwhile).
+at::DataPtr read_back(const Tensor& t, size_t bytes, const char* what) {
+  at::DataPtr host = at::getHostAllocator(at::kCUDA)->allocate(bytes);
+  const hipStream_t st = c10::hip::getCurrentHIPStream(t.get_device()).stream();
+  hipError_t rc = hipMemcpyAsync(host.get(), ptr(t), bytes, hipMemcpyDeviceToHost, st);
+  if (rc == hipSuccess) {
+    Py_BEGIN_ALLOW_THREADS
+    rc = hipStreamSynchronize(st);
+    Py_END_ALLOW_THREADS
+  }
+  if (rc != hipSuccess) runtime_error(std::string(what) + ": " + hipGetErrorString(rc));
+  return host;
+}
+
+// The values of an int32 vector as a list.
 PyObject* int_list(const Args& a) {
   const Tensor given = a.tensor(0);
   int32(given, "loads");
@@ -585,15 +599,7 @@ PyObject* int_list(const Args& a) {
   at::DataPtr host;
   if (n > 0 && t.is_cuda()) {
     const c10::DeviceGuard guard(t.device());
-    host = at::getHostAllocator(at::kCUDA)->allocate(n * 4);
-    const hipStream_t st = c10::hip::getCurrentHIPStream(t.get_device()).stream();
-    hipError_t rc = hipMemcpyAsync(host.get(), ptr(t), n * 4, hipMemcpyDeviceToHost, st);
-    if (rc == hipSuccess) {
-      Py_BEGIN_ALLOW_THREADS
-      rc = hipStreamSynchronize(st);
-      Py_END_ALLOW_THREADS
-    }
-    if (rc != hipSuccess) runtime_error(std::string("reading the loads: ") + hipGetErrorString(rc));
+    host = read_back(t, n * 4, "reading the loads");
     values = static_cast<const int32_t*>(host.get());
   } else if (n > 0) {
     values = iptr(t);
@@ -601,6 +607,25 @@ PyObject* int_list(const Args& a) {
   PyObject* const list = PyList_New(n);
   for (int64_t i = 0; i < n; ++i) PyList_SET_ITEM(list, i, PyLong_FromLong(values[i]));
   return list;
+}
+
+// tags (a vector of 1 to BRT_UNIQUE_WHOLE_MAX int32 or int64 on the device) -> (unique, inverse, lo, hi), the first
+// two None where the range is more than one workgroup's table holds
+PyObject* unique_tags(const Args& a) {
+  const Tensor tags = dense(a.tensor(0));
+  on_device(tags, "tags");
+  const bool narrow = tags.scalar_type() == at::kInt;
+  if (!narrow && tags.scalar_type() != at::kLong) runtime_error("tags must be int32 or int64");
+  const c10::DeviceGuard guard(tags.device());
+  const int64_t n = tags.numel();
+  Tensor unique = empty({n}, tags.scalar_type(), tags), inverse = empty({n}, at::kLong, tags), found = empty({3}, at::kLong, tags);
+  check(brt_hip_unique_tags_whole(ptr(tags), narrow ? 32 : 64, n, ptr(unique), static_cast<int64_t*>(ptr(inverse)),
+                                  static_cast<int64_t*>(ptr(found)), stream_of(tags)));
+  const at::DataPtr host = read_back(found, 24, "reading the number of tags");
+  const int64_t* const v = static_cast<const int64_t*>(host.get());
+  PyObject *const lo = PyLong_FromLongLong(v[1]), *const hi = PyLong_FromLongLong(v[2]);
+  if (v[0] < 0) return tuple(none(), none(), lo, hi);
+  return tuple(wrap(unique.narrow(0, 0, v[0])), wrap(inverse), lo, hi);
 }
 
 PyObject* calls(const Args&) { return PyLong_FromUnsignedLongLong(g_calls); }
@@ -628,8 +653,8 @@ PyMethodDef methods[] = {
     BRT_ENTRY(generate, 5),         BRT_ENTRY(route_and_dispatch, 7),  BRT_ENTRY(route_by_path, 7),
     BRT_ENTRY(dispatch, 12),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
     BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 7),     BRT_ENTRY(grouped_linear, 16),
-    BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5), BRT_ENTRY(int_list, 1),
-    BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
+    BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5),        BRT_ENTRY(int_list, 1),
+    BRT_ENTRY(unique_tags, 1),      BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "brt_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -113,29 +113,27 @@ __global__ void inverse_kernel(const K* __restrict__ keys, long n, long lo, long
 // The whole unique in one workgroup, the table in LDS: for ranges of up to kSmallRange tags and
 // inputs short enough for 1024 threads to walk twice.
 constexpr int kSmallRange = 32768;
-constexpr long kSmallCount = 1l << 15;
+constexpr long kSmallCount = BRT_UNIQUE_WHOLE_MAX;
 
 constexpr int kKeysInFlight = 8;
 
+// A batch of keys per thread.  The loads are unconditional (an index past the end reads the last key
+// again and is dropped), all in flight together; one at a time, every key would be a memory round
+// trip of its own for this one workgroup.
 template <typename K>
-__global__ __launch_bounds__(kScanThreads) void unique_small_kernel(const K* __restrict__ keys, int n,
-                                                                    long lo, int range,
-                                                                    K* __restrict__ unique,
-                                                                    int64_t* __restrict__ inverse,
-                                                                    int* __restrict__ n_unique) {
-  extern __shared__ int s_table[];
+__device__ __forceinline__ void key_batch(const K* __restrict__ keys, int n, int base, K (&v)[kKeysInFlight]) {
+#pragma unroll
+  for (int j = 0; j < kKeysInFlight; ++j)
+    v[j] = keys[min(base + j * kScanThreads + static_cast<int>(threadIdx.x), n - 1)];  // n >= 1
+}
+
+// The first batch, `held`, stays in registers for the inverse at the end.  The number of unique keys is
+// returned to the last thread.
+template <typename K>
+__device__ __forceinline__ int unique_in_lds(const K* __restrict__ keys, int n, long lo, int range, const K (&held)[kKeysInFlight],
+                                             K* __restrict__ unique, int64_t* __restrict__ inverse, int* s_table) {
   __shared__ int s_wave[kScanThreads / kWave];
   const int tid = threadIdx.x, wave = tid >> 6;
-  // The keys are fetched in batches of kKeysInFlight loads per thread (unconditional: an index
-  // past the end reads the last key again and is dropped), all in flight together; one at a
-  // time, every key would be a memory round trip of its own for this one workgroup.  The first
-  // batch stays in registers for the inverse at the end.
-  auto key_batch = [&](int base, K (&v)[kKeysInFlight]) {
-#pragma unroll
-    for (int j = 0; j < kKeysInFlight; ++j) v[j] = keys[min(base + j * kScanThreads + tid, n - 1)];  // n >= 1
-  };
-  K held[kKeysInFlight];
-  key_batch(0, held);
   for (int i = tid; i < range; i += kScanThreads) s_table[i] = 0;
   __syncthreads();
   for (int base = 0; base < n; base += kKeysInFlight * kScanThreads) {
@@ -144,7 +142,7 @@ __global__ __launch_bounds__(kScanThreads) void unique_small_kernel(const K* __r
 #pragma unroll
       for (int j = 0; j < kKeysInFlight; ++j) v[j] = held[j];
     } else {
-      key_batch(base, v);
+      key_batch(keys, n, base, v);
     }
 #pragma unroll
     for (int j = 0; j < kKeysInFlight; ++j) {
@@ -170,7 +168,6 @@ __global__ __launch_bounds__(kScanThreads) void unique_small_kernel(const K* __r
     if (flag) unique[rank] = static_cast<K>(lo + i);
     rank += flag;
   }
-  if (tid == kScanThreads - 1) *n_unique = rank;
   __syncthreads();
   for (int base = 0; base < n; base += kKeysInFlight * kScanThreads) {
     K v[kKeysInFlight];
@@ -178,7 +175,7 @@ __global__ __launch_bounds__(kScanThreads) void unique_small_kernel(const K* __r
 #pragma unroll
       for (int j = 0; j < kKeysInFlight; ++j) v[j] = held[j];
     } else {
-      key_batch(base, v);
+      key_batch(keys, n, base, v);
     }
 #pragma unroll
     for (int j = 0; j < kKeysInFlight; ++j) {
@@ -187,6 +184,56 @@ __global__ __launch_bounds__(kScanThreads) void unique_small_kernel(const K* __r
       if (i < n) inverse[i] = (k >= 0 && k < range) ? s_table[k] : -1;
     }
   }
+  return rank;
+}
+
+template <typename K>
+__global__ __launch_bounds__(kScanThreads) void unique_small_kernel(const K* __restrict__ keys, int n, long lo, int range,
+                                                                    K* __restrict__ unique, int64_t* __restrict__ inverse,
+                                                                    int* __restrict__ n_unique) {
+  extern __shared__ int s_table[];
+  K held[kKeysInFlight];
+  key_batch(keys, n, 0, held);
+  const int count = unique_in_lds(keys, n, lo, range, held, unique, inverse, s_table);
+  if (threadIdx.x == kScanThreads - 1) *n_unique = count;
+}
+
+// The same when the range is not known: the keys are read once for their smallest and largest, which go
+// into found[1] and found[2]; found[0] is the number of unique keys, or -1 (nothing else written)
+// where the range is more than the table holds.  Bound by latency, as is all around it: finding the range with
+// library calls took three launches and a wait of the host before this one (gathering 2048 cells of 4 flows by
+// their tags 243 -> 166 us).
+template <typename K>
+__global__ __launch_bounds__(kScanThreads) void unique_whole_kernel(const K* __restrict__ keys, int n, K* __restrict__ unique,
+                                                                    int64_t* __restrict__ inverse, int64_t* __restrict__ found) {
+  extern __shared__ int s_table[];
+  __shared__ K s_lo[kScanThreads / kWave], s_hi[kScanThreads / kWave];
+  K held[kKeysInFlight];
+  key_batch(keys, n, 0, held);
+  K lo = held[0], hi = held[0];
+  auto take = [&](const K (&v)[kKeysInFlight]) {
+#pragma unroll
+    for (int j = 0; j < kKeysInFlight; ++j) lo = min(lo, v[j]), hi = max(hi, v[j]);
+  };
+  take(held);
+  for (int base = kKeysInFlight * kScanThreads; base < n; base += kKeysInFlight * kScanThreads) {
+    K v[kKeysInFlight];
+    key_batch(keys, n, base, v);
+    take(v);
+  }
+  for (int d = 1; d < kWave; d <<= 1) lo = min(lo, __shfl_xor(lo, d, kWave)), hi = max(hi, __shfl_xor(hi, d, kWave));
+  if (lane_id() == 0) s_lo[threadIdx.x >> 6] = lo, s_hi[threadIdx.x >> 6] = hi;
+  __syncthreads();
+  for (int w = 0; w < kScanThreads / kWave; ++w) lo = min(lo, s_lo[w]), hi = max(hi, s_hi[w]);
+  const uint64_t span = static_cast<uint64_t>(hi) - static_cast<uint64_t>(lo);  // range - 1, whatever the signs
+  const bool last = threadIdx.x == kScanThreads - 1;
+  if (last) found[1] = lo, found[2] = hi;
+  if (span >= kSmallRange) {
+    if (last) found[0] = -1;
+    return;
+  }
+  const int count = unique_in_lds(keys, n, static_cast<long>(lo), static_cast<int>(span) + 1, held, unique, inverse, s_table);
+  if (last) found[0] = count;
 }
 
 // Pushes row p on the list of output row index[p]: head[r] is 1 + the row pushed last (0: empty),
@@ -349,19 +396,9 @@ extern "C" int brt_hip_unique_tags(const void* tags, int tag_bits, long n, long 
     return fail(BRT_E_INVALID, "workspace of %zu bytes, need %zu", workspace_bytes, need);
   if (range <= kSmallRange && n >= 1 && n <= kSmallCount) {  // (no keys: the general path below)
     const size_t lds = static_cast<size_t>(range) * sizeof(int);
-    // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
-    static bool configured[2][64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 63;
-    const int which = tag_bits == 32 ? 0 : 1;
-    if (!configured[which][dev] || dev == 63) {
-      const void* fn = which == 0 ? reinterpret_cast<const void*>(&unique_small_kernel<int32_t>)
-                                  : reinterpret_cast<const void*>(&unique_small_kernel<int64_t>);
-      if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              kSmallRange * static_cast<int>(sizeof(int))) != hipSuccess)
-        return fail(BRT_E_LAUNCH, "cannot reserve %d bytes of LDS", kSmallRange * 4);
-      configured[which][dev] = true;
-    }
+    const void* fn = tag_bits == 32 ? reinterpret_cast<const void*>(&unique_small_kernel<int32_t>)
+                                    : reinterpret_cast<const void*>(&unique_small_kernel<int64_t>);
+    if (const int rc = allow_dynamic_lds(fn, kSmallRange * static_cast<int>(sizeof(int))); rc != BRT_OK) return rc;
     if (tag_bits == 32)
       hipLaunchKernelGGL(unique_small_kernel<int32_t>, dim3(1), dim3(kScanThreads), lds, st,
                          static_cast<const int32_t*>(tags), static_cast<int>(n), lo, static_cast<int>(range),
@@ -405,6 +442,26 @@ extern "C" int brt_hip_unique_tags(const void* tags, int tag_bits, long n, long 
                          lo, range, table, inverse);
   }
   return check_launch("unique_tags");
+}
+
+extern "C" int brt_hip_unique_tags_whole(const void* tags, int tag_bits, long n, void* unique_tags, int64_t* inverse,
+                                         int64_t* found, void* stream) {
+  if (tag_bits != 32 && tag_bits != 64) return fail(BRT_E_INVALID, "tag_bits must be 32 or 64, got %d", tag_bits);
+  if (n < 1) return fail(BRT_E_INVALID, "bad arguments n=%ld", n);
+  if (n > kSmallCount) return fail(BRT_E_UNSUPPORTED, "more than %ld tags", kSmallCount);
+  if (!tags || !unique_tags || !inverse || !found) return fail(BRT_E_INVALID, "null argument");
+  const int lds = kSmallRange * static_cast<int>(sizeof(int));
+  const bool narrow = tag_bits == 32;
+  const void* fn = narrow ? reinterpret_cast<const void*>(&unique_whole_kernel<int32_t>)
+                          : reinterpret_cast<const void*>(&unique_whole_kernel<int64_t>);
+  if (const int rc = allow_dynamic_lds(fn, lds); rc != BRT_OK) return rc;
+  if (narrow)
+    hipLaunchKernelGGL(unique_whole_kernel<int32_t>, dim3(1), dim3(kScanThreads), lds, as_stream(stream),
+                       static_cast<const int32_t*>(tags), static_cast<int>(n), static_cast<int32_t*>(unique_tags), inverse, found);
+  else
+    hipLaunchKernelGGL(unique_whole_kernel<int64_t>, dim3(1), dim3(kScanThreads), lds, as_stream(stream),
+                       static_cast<const int64_t*>(tags), static_cast<int>(n), static_cast<int64_t*>(unique_tags), inverse, found);
+  return check_launch("unique_whole_kernel");
 }
 
 extern "C" size_t brt_hip_combine_by_index_workspace_bytes(int P, int n_out) {

@@ -360,6 +360,10 @@ int brt_hip_grouped_gemm_accumulate(const void* x, const void* const* weights,
  *   unique_tags), `n_unique` [1] int32 on the device.  No sort: a presence table over the range
  *   and one prefix sum.  hi-lo+1 may be at most 2^25 (BRT_E_UNSUPPORTED beyond; the workspace
  *   size query returns 0 then).
+ *   brt_hip_unique_tags_whole is the form for 1 to BRT_UNIQUE_WHOLE_MAX tags of unknown range: one launch,
+ *   no workspace, room for n unique tags, and `found` [3] int64 on the device: the number of unique tags,
+ *   the smallest and the largest tag.  A number of -1 says that hi-lo+1 exceeds 32768; nothing else is
+ *   written then, and the range form is to be called.
  *
  * brt_hip_combine_by_index replaces the tag-mode branch of combine_with_indices_and_loads
  *   (router.cc:449-472: `repeat` of the index to one int64 per element + `scatter_reduce`
@@ -377,6 +381,9 @@ size_t brt_hip_unique_tags_workspace_bytes(long lo, long hi);
 int brt_hip_unique_tags(const void* tags, int tag_bits, long n, long lo, long hi, void* workspace,
                         size_t workspace_bytes, void* unique_tags, int64_t* inverse,
                         int32_t* n_unique, void* stream);
+#define BRT_UNIQUE_WHOLE_MAX 32768
+int brt_hip_unique_tags_whole(const void* tags, int tag_bits, long n, void* unique_tags,
+                              int64_t* inverse, int64_t* found, void* stream);
 size_t brt_hip_combine_by_index_workspace_bytes(int P, int n_out);
 int brt_hip_combine_by_index(const void* in_data, void* out_data, const void* index, int index_bits,
                              int P, int cell, int n_out, void* workspace, size_t workspace_bytes,

@@ -519,6 +519,11 @@ def test_experts_with_many_row_blocks_in_patch_order(loads, K, N):
     ([2000, 1700, 300, 1900, 1, 1800, 2047, 1500], 128, 1000),  # one round, ragged, N tail
     # last row blocks of every number of 32-row tiles, shared by the two groups of wavefronts
     ([768 + r for r in (1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 255)], 192, 2048),
+    # the last round's whole tiles cut in four (528 tiles and 16 light ones), in two (592 and 16, parts past the
+    # expert's rows among them), with more than 128 experts
+    ([5000, 3328, 100], 128, 4096),
+    ([100, 5000, 4300], 128, 4096),
+    ([0] * 100 + [5000, 100] + [0] * 64 + [130, 26000, 0], 128, 1024),
 ])
 def test_ping_pong_tiles(loads, K, N):
     """Shapes the host sends to the 256 x 256 ping-pong kernel: experts that average more than 160
@@ -536,6 +541,7 @@ def test_ping_pong_tiles(loads, K, N):
     (12000, 8, 192, 4104, 1, 1700, True),    # padded to the capacity: empty slots, odd K-steps, N tail
     (13000, 5, 1024, 1000, 1, 4000, False),  # one round of tiles, N tail
     (7000, 6, 256, 4096, 2, 2400, False),    # two entries per cell (gather only)
+    (8800, 2, 128, 4096, 1, 8000, False),    # tiles cut in four, light tiles last
 ])
 def test_ping_pong_tiles_with_routing_and_fp32_output(T, E, K, N, k, cap, pad):
     """The routed and fp32-output forms on shapes the 256 x 256 ping-pong kernel takes: the same bits

@@ -504,15 +504,29 @@ def _route(hip, mask, caps=None, pad=False):
     (20000, 0, 8191, np.int64),          # one scan block, every tag many times
     (30000, -5000, 60000, np.int32),     # 8 scan blocks, negative tags
     (100000, 100, 1500000, np.int64),    # 184 scan blocks, most tags absent
+    (32768, 5, 32772, np.int32),         # the most keys and the widest range of one workgroup
+    (8193, -20000, 12767, np.int64), (8192, -20000, 12768, np.int64),  # ... one key past a batch, one tag too wide
+    (700, -2 ** 63, 2 ** 63 - 2, np.int64), (3, -2 ** 31, 2 ** 31 - 2, np.int32),
 ])
 def test_unique_tags_bit_exact(hip, n, lo, hi, kind):
     rng = np.random.default_rng(n + hi)
     tags = rng.integers(lo, hi + 1, size=n).astype(kind)
     tags[0], tags[-1] = lo, hi
-    unique, inverse = hip.unique_tags(tags)
-    want_u, want_i = oracle.unique_tags(tags)
-    assert unique.dtype == kind and np.array_equal(unique, want_u)
-    assert np.array_equal(inverse, want_i)
+    want_u, want_i = np.unique(tags, return_inverse=True)
+    if hi - lo < 1 << 25:
+        unique, inverse = hip.unique_tags(tags)
+        oracle_u, oracle_i = oracle.unique_tags(tags)
+        assert np.array_equal(oracle_u, want_u) and np.array_equal(oracle_i, want_i)
+        assert unique.dtype == kind and np.array_equal(unique, want_u)
+        assert np.array_equal(inverse, want_i)
+    # the op finds the range itself, in the kernel for up to 32768 tags
+    import torch
+
+    from brainstorm_amd._C.router import _unique_tags
+
+    unique, inverse = _unique_tags(torch.from_numpy(tags).cuda())
+    assert unique.cpu().numpy().dtype == kind and np.array_equal(unique.cpu().numpy(), want_u)
+    assert np.array_equal(inverse.cpu().numpy(), want_i)
 
 
 def test_unique_tags_with_a_wider_range_than_the_data(hip):
