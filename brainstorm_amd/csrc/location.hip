@@ -229,9 +229,22 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_of_wave(long row_w, const
   return words_at(a.mask + (rows_here > 0 ? row_w : 0) * a.E, static_cast<size_t>(rows_here) * a.E * 4);
 }
 
+// The byte offsets into such a buffer are 32 bits wide and loads reach up to 124 rows of E words past its
+// end: from this many paths on they could wrap round, and the kernels take 64-bit addresses (WIDE).
+constexpr int kWidePaths = 1 << 20;
+
 // Loads one batch of row words (zero beyond the band / the matrix).
-__device__ __forceinline__ void load_batch(int (&v)[kBatch], __amdgpu_buffer_rsrc_t rows, int i0, int rps, int sub,
-                                           int col, bool col_ok, const ScanArgs& a) {
+template <bool WIDE>
+__device__ __forceinline__ void load_batch(int (&v)[kBatch], __amdgpu_buffer_rsrc_t rows, long row_w, int i0, int rps,
+                                           int sub, int col, bool col_ok, const ScanArgs& a) {
+  if constexpr (WIDE) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int rl = (i0 + u) * rps + sub;
+      v[u] = col_ok && rl < a.rows_pw && row_w + rl < a.T ? a.mask[static_cast<size_t>(row_w + rl) * a.E + col] : 0;
+    }
+    return;
+  }
   const unsigned first = col_ok ? (static_cast<unsigned>(i0 * rps + sub) * a.E + col) * 4u : kOutside;
   const unsigned step = rps * a.E * 4u;
 #pragma unroll
@@ -239,9 +252,14 @@ __device__ __forceinline__ void load_batch(int (&v)[kBatch], __amdgpu_buffer_rsr
 }
 
 // This lane's share of the column sums of bands [j0, end), every `step`-th of them.
+template <bool WIDE>
 __device__ __forceinline__ int sum_of_bands(int j0, int end, int step, int col, bool col_ok, const ScanArgs& a) {
-  const __amdgpu_buffer_rsrc_t sums = words_at(a.partial, static_cast<size_t>(end) * a.E * 4);
   int total = 0;
+  if constexpr (WIDE) {
+    for (; j0 < end; j0 += step) total += col_ok ? a.partial[static_cast<size_t>(j0) * a.E + col] : 0;
+    return total;
+  }
+  const __amdgpu_buffer_rsrc_t sums = words_at(a.partial, static_cast<size_t>(end) * a.E * 4);
   for (; j0 < end; j0 += step * kPartialBatch) {
     int v[kPartialBatch];
     const unsigned first = col_ok ? (static_cast<unsigned>(j0) * a.E + col) * 4u : kOutside;
@@ -255,6 +273,7 @@ __device__ __forceinline__ int sum_of_bands(int j0, int end, int step, int col, 
 }
 
 // pass 1: column sums of one band
+template <bool WIDE>
 __global__ __launch_bounds__(kBlock) void band_count_kernel(ScanArgs a) {
   __shared__ int s_sum[kWavesPB][kWave];
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -271,7 +290,7 @@ __global__ __launch_bounds__(kBlock) void band_count_kernel(ScanArgs a) {
     int sum = 0;
     for (int i0 = 0; i0 < n_ins; i0 += kBatch) {
       int v[kBatch];
-      load_batch(v, rows, i0, rps, sub, col, col_ok, a);
+      load_batch<WIDE>(v, rows, row_w, i0, rps, sub, col, col_ok, a);
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) sum += v[u];
     }
@@ -291,7 +310,7 @@ __global__ __launch_bounds__(kBlock) void band_count_kernel(ScanArgs a) {
 }
 
 // pass 2: offsets from the bands above, running sums in registers, results out
-template <int MODE, int kWavesPB>
+template <int MODE, int kWavesPB, bool WIDE>
 __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a) {
   __shared__ int s_above[kWavesPB][kWave];  // each wave's share of the sum over earlier bands
   __shared__ int s_own[kWavesPB][kWave];    // column sums of each wave's own rows
@@ -310,18 +329,18 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
     const bool col_ok = col < E;
     // ---- own rows: the first batch stays in registers ---------------------------------
     int m0[kBatch];
-    load_batch(m0, rows, 0, rps, sub, col, col_ok, a);
+    load_batch<WIDE>(m0, rows, row_w, 0, rps, sub, col, col_ok, a);
     // ---- this wave's share of the offset: bands wave, wave+4, ... above this one ----
-    int above = sum_of_bands(wave + sub * kWavesPB, band, kWavesPB * rps, col, col_ok, a), below = 0;
+    int above = sum_of_bands<WIDE>(wave + sub * kWavesPB, band, kWavesPB * rps, col, col_ok, a), below = 0;
     if (MODE == kTag)  // the tag list of a path ends at its total: the later bands count too
-      below = sum_over_rows_in_wave(sum_of_bands(band + 1 + wave + sub * kWavesPB, a.bands, kWavesPB * rps, col, col_ok, a),
+      below = sum_over_rows_in_wave(sum_of_bands<WIDE>(band + 1 + wave + sub * kWavesPB, a.bands, kWavesPB * rps, col, col_ok, a),
                                     a.ep_shift);
     int own = 0;
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) own += m0[u];
     for (int i0 = kBatch; i0 < n_ins; i0 += kBatch) {
       int v[kBatch];
-      load_batch(v, rows, i0, rps, sub, col, col_ok, a);
+      load_batch<WIDE>(v, rows, row_w, i0, rps, sub, col, col_ok, a);
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) own += v[u];
     }
@@ -360,7 +379,7 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
     walk_batch<MODE>(m0, 0, n_ins, carry, thr, total, row_w, rps, ep, sub, e, lane, col, col_ok, a);
     for (int i0 = kBatch; i0 < n_ins; i0 += kBatch) {
       int v[kBatch];
-      load_batch(v, rows, i0, rps, sub, col, col_ok, a);
+      load_batch<WIDE>(v, rows, row_w, i0, rps, sub, col, col_ok, a);
       walk_batch<MODE>(v, i0, n_ins, carry, thr, total, row_w, rps, ep, sub, e, lane, col, col_ok, a);
     }
 
@@ -688,21 +707,28 @@ int launch_scan(int mode, ScanArgs& a, void* workspace, size_t workspace_bytes, 
   if (g.waves_pb == kWavesSingle) {
     const dim3 block(kWavesSingle * kWave);
     if (mode == kSeat)
-      hipLaunchKernelGGL((band_apply_kernel<kSeat, kWavesSingle>), grid, block, 0, st, a);
+      hipLaunchKernelGGL((band_apply_kernel<kSeat, kWavesSingle, false>), grid, block, 0, st, a);
     else if (mode == kTag)
-      hipLaunchKernelGGL((band_apply_kernel<kTag, kWavesSingle>), grid, block, 0, st, a);
+      hipLaunchKernelGGL((band_apply_kernel<kTag, kWavesSingle, false>), grid, block, 0, st, a);
     else
-      hipLaunchKernelGGL((band_apply_kernel<kThrottle, kWavesSingle>), grid, block, 0, st, a);
+      hipLaunchKernelGGL((band_apply_kernel<kThrottle, kWavesSingle, false>), grid, block, 0, st, a);
     return check_launch("band_apply_kernel");
   }
-  if (g.bands > 1)  // a single band has nothing above it
-    hipLaunchKernelGGL(band_count_kernel, grid, dim3(kBlock), 0, st, a);
-  if (mode == kSeat)
-    hipLaunchKernelGGL((band_apply_kernel<kSeat, kWavesPB>), grid, dim3(kBlock), 0, st, a);
-  else if (mode == kTag)
-    hipLaunchKernelGGL((band_apply_kernel<kTag, kWavesPB>), grid, dim3(kBlock), 0, st, a);
+  auto launch = [&](auto wide) {
+    constexpr bool kWide = decltype(wide)::value;
+    if (g.bands > 1)  // a single band has nothing above it
+      hipLaunchKernelGGL(band_count_kernel<kWide>, grid, dim3(kBlock), 0, st, a);
+    if (mode == kSeat)
+      hipLaunchKernelGGL((band_apply_kernel<kSeat, kWavesPB, kWide>), grid, dim3(kBlock), 0, st, a);
+    else if (mode == kTag)
+      hipLaunchKernelGGL((band_apply_kernel<kTag, kWavesPB, kWide>), grid, dim3(kBlock), 0, st, a);
+    else
+      hipLaunchKernelGGL((band_apply_kernel<kThrottle, kWavesPB, kWide>), grid, dim3(kBlock), 0, st, a);
+  };
+  if (a.E < kWidePaths)
+    launch(std::false_type{});
   else
-    hipLaunchKernelGGL((band_apply_kernel<kThrottle, kWavesPB>), grid, dim3(kBlock), 0, st, a);
+    launch(std::true_type{});
   return check_launch("band_apply_kernel");
 }
 
@@ -896,7 +922,7 @@ extern "C" int brt_hip_route_and_dispatch(const int32_t* mask, const void* cells
   f.cpr = static_cast<int>(cell_bytes / 16);
   hipStream_t st = as_stream(stream);
   const dim3 grid(g.bands);
-  if (g.bands > 1) hipLaunchKernelGGL(band_count_kernel, grid, dim3(kBlock), 0, st, a);
+  if (g.bands > 1) hipLaunchKernelGGL(band_count_kernel<false>, grid, dim3(kBlock), 0, st, a);
   // rows of more than 128 bytes leave as streaming stores, shorter ones merge in the L2 (as in dispatch)
   const int units = (g.rows_pw * f.cpr + kWave - 1) / kWave;  // per lane
   auto go = [&](auto stream_t, auto nv_t) {

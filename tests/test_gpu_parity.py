@@ -84,6 +84,20 @@ def test_indices_general_mask_values_and_misaligned_buffers(hip):
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
 
 
+# on both sides of the widest matrix that is read through 32-bit byte offsets, and where those would wrap round
+@pytest.mark.parametrize("T,E", [(9, (1 << 20) - 1), (9, 1 << 20), (6, (1 << 24) + 8)])
+def test_index_generation_of_very_many_paths(hip, T, E):
+    mask = np.random.default_rng(E).integers(0, 2, (T, E), dtype=np.int8).astype(np.int32)
+    for tag in (False, True):
+        want = oracle.generate_indices_and_loads(mask, is_tag_index=tag)
+        got = hip.generate_indices_and_loads(mask, is_tag_index=tag)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    prefix, threshold = np.ones(E, np.int32), np.full(E, 3, np.int32)
+    want = oracle.throttle_hotmask(mask, prefix, threshold)
+    got = hip.throttle_hotmask(mask, prefix, threshold)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("tag", [False, True])
 def test_capacity_rules_bit_exact(hip, tag):
     caps = [1, 2, 4, 8, 16, 32, 64, 128, 256, 512]
