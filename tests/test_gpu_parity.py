@@ -304,6 +304,28 @@ def test_dispatch_odd_row_sizes_use_narrower_accesses(hip):
                 assert same_bits(got, want), (dtype, cell)
 
 
+# few paths: a step covers 64 to 4 cells, of which a wavefront takes 1, a part or all by the number of cells
+@pytest.mark.parametrize("T,E,k,cell,dtype", [
+    (1, 4, 1, 512, "f32"), (2049, 4, 2, 512, "f32"), (4095, 1, 1, 256, "bf16"), (8191, 3, 2, 260, "f32"), (8193, 4, 2, 512, "bf16"),
+    (20001, 8, 2, 96, "f16"), (517, 2, 2, 16, "bf16"), (3001, 4, 3, 33, "f32"), (1025, 16, 2, 2056, "bf16"), (40001, 4, 1, 256, "f16"),
+])
+def test_routes_with_few_paths_bit_exact(hip, T, E, k, cell, dtype):
+    mask, logits = topk_mask(T, E, k, seed=T + E)
+    x = as_dtype_bits(np.random.default_rng(T).standard_normal((T, cell)), dtype)
+    gates = as_dtype_bits(softmax(logits), dtype)
+    cap = max(1, int(0.9 * T * k / E))
+    for caps, pad in ((None, False), ([cap, 2 * cap, 64 * cap], True)):
+        idx, loads = oracle.generate_indices_and_loads(mask, caps, pad)
+        for g in (None, gates):
+            rows, _ = oracle.dispatch(x, idx, loads, gates=g, dtype=dtype)
+            for counts in (None, mask.sum(0).astype(np.int32)):
+                assert same_bits(hip.dispatch(x, idx, loads, g, counts, dtype=dtype)[0], rows)
+            for r in (None, x):
+                want = oracle.combine(rows, idx, loads, gates=g, out_data=r, in_dtype=dtype, out_dtype=dtype, gate_dtype=dtype)
+                got = hip.combine(rows, idx, loads, g, r, in_dtype=dtype, out_dtype=dtype, gate_dtype=dtype)
+                assert same_bits(got, want), (g is None, r is None)
+
+
 # --------------------------------------------------------------------- combine
 @pytest.mark.parametrize("T,E,k,cell", DISPATCH_SHAPES)
 @pytest.mark.parametrize("in_dtype,out_dtype,gate_dtype", [
