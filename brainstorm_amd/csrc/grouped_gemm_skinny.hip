@@ -344,23 +344,30 @@ int launch_act(GemmArgs& a, int act, hipStream_t st) {
 
 // Where this kernel is taken, against the 160-row kernel.  Both were timed on 2 to 200 rows per expert,
 // 4 to 128 experts, 512 <-> 2048, 768 <-> 3072, 1024 <-> 4096, 2048 <-> 8192 and 320 <-> 640; the
-// rule is within 1.4 % of the faster one on average (the 160-row kernel alone: 44 % off).
-//   - Up to 40 rows per expert: always (8 experts x 3 rows 3072 -> 768: 43.9 -> 9.7 us, 32 x 8 rows
-//     4096 -> 1024 68.3 -> 46.3 us, 64 x 8 rows 768 -> 3072 55.2 -> 48.3 us), except when the weights
-//     are so many that the wide tiles fill the chip for many rounds and stream them at the memory's
-//     rate anyway (32 x 8 rows 8192 -> 2048, 1.07 GB: 171 us there, 200 us here).
+// rule gives up small gains rather than lose where the 160-row kernel is the faster one.
+//   - Up to 28 rows per expert (one row block): while the weights are less than 0.3 GB (8 experts x 3 rows
+//     3072 -> 768: 43.9 -> 9.7 us, 32 x 8 rows 4096 -> 1024 68.3 -> 46.3 us).  Beyond, the wide tiles stream
+//     them at the memory's rate (32 x 19 rows 6656 -> 1664, 709 MB: 113 us there, 129 us here; 32 x 16 rows
+//     1920 -> 3840, 472 MB: 75.5 and 84.0 us), except where they cannot: half of the CUs without a
+//     tile (16 x 12 rows 6656 -> 1664 89.6 -> 66.7 us), a K whose rows lie multiples of 4 KB apart (64 x 16
+//     rows 4096 -> 1024 119 -> 91 us) or experts of which many get no row at all (128 experts, 183 rows
+//     896 -> 3584 124 -> 96 us); up to 1 GB (32 x 8 rows 8192 -> 2048, 1.07 GB: 171 us there, 200 us here).
 //   - More rows: every block of 32 or 64 rows streams the weights again (from the L2), which pays
 //     while the 160-row kernel has too few 160 x 256 tiles for the CUs: up to 72 of them, however many
 //     rows that are (8 x 120 rows 3072 -> 768 46.9 -> 22.4 us, 4 x 1300 rows 1024 -> 256 24.5 -> 12.3 us,
 //     32 x 120 rows 2048 -> 512 36.6 -> 36.2 us; not 64 x 120 rows, 128 tiles: 44.9 -> 59.9 us), and up to
-//     160 for few experts of up to 128 rows (4 x 120 rows 2048 -> 8192 77.2 -> 43.0 us).
+//     160 for few experts of up to 128 rows and 0.15 GB (4 x 120 rows 2048 -> 8192 77.2 -> 43.0 us; not 16 x 40
+//     rows 3840 -> 1920, 236 MB: 55.9 -> 72.5 us).
 bool skinny_gemm_applies(const GemmArgs& a) {
   const long used = std::min(a.E, a.P);
   const long tiles = std::max<long>((a.P + 159) / 160, used) * ((a.N + 255) / 256);
   const double weight_bytes = 2.0 * used * a.N * a.K;
   if (tiles <= 72) return true;
-  if (a.P <= 40 * used) return weight_bytes < 1e9;
-  return a.P <= 128 * used && tiles <= 160 && a.E <= 16 && weight_bytes < 3e8;
+  if (a.P <= 28 * used) {
+    if (weight_bytes < 3e8) return true;
+    return weight_bytes < 1e9 && (tiles <= 128 || a.K % 2048 == 0 || 2l * a.P <= 3 * used);
+  }
+  return a.P <= 128 * used && tiles <= 160 && a.E <= 16 && weight_bytes < 1.5e8;
 }
 
 // Shape of the tile.  Few workgroups: the narrowest one, so that every CU gets one (at most 264 of 32 x
