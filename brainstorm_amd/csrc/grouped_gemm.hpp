@@ -38,7 +38,7 @@ struct GemmArgs {
 bool pingpong_gemm_applies(const GemmArgs& a);
 int launch_pingpong_gemm(GemmArgs& a, int act, hipStream_t st);
 
-// The split-K kernel for few rows per expert and few tiles (grouped_gemm_skinny.hip), every form.
+// The kernel for few rows per expert and few tiles (grouped_gemm_skinny.hip), every form.
 bool skinny_gemm_applies(const GemmArgs& a);
 int launch_skinny_gemm(GemmArgs& a, int act, hipStream_t st);
 

@@ -2,23 +2,28 @@
 // where the weights have to be streamed by as many CUs as there are and nothing else costs anything.
 //
 // Same contract as grouped_gemm.hip (out[rows of e] = act(x[rows of e] @ W_e^T + b_e), one launch,
-// loads read on the device; reference: src/jit/compiler.cu:151-246).  What differs:
+// loads read on the device; reference: src/jit/compiler.cu:151-246), and the same bits: the products of an
+// output element are summed in order of K by the same instruction in all three kernels, so that a
+// row does not depend on which of them the number of rows selects.  What differs:
 //
 //   - A workgroup owns XR rows x 32 * NT columns, a tile so small that even a contracting GEMM of a
-//     few experts has a workgroup per CU, and its S wavefronts split K between them: each multiplies its
-//     own slice of K for the whole tile, and the partial sums meet in LDS at the end, added in
-//     wavefront order (the result does not depend on timing).
-//     Every tile shape splits K the same way, so a row's bits do not depend on the shape.
-//   - A wavefront's K loop is its own: operands go from global memory straight into its corner of
-//     LDS (a ring of D K-steps of 64, whole 128-byte lines per row, swizzled on the global side as
-//     in grouped_gemm_pingpong.hip), waits count its own loads, and there is no barrier.
-//     A deep ring matters less than many wavefronts with requests in flight: two or three workgroups
-//     share a CU.
+//     few experts has a workgroup per CU.  One wavefront per 32 x 32 block multiplies it over all of K;
+//     all four load.
+//   - Operands go from global memory straight into LDS (a ring of D K-steps of 64, whole 128-byte lines
+//     per row, swizzled on the global side as in grouped_gemm_pingpong.hip).  Every wavefront loads a quarter
+//     of each K-step, waits for its own part of the next one and meets the others at one
+//     barrier per K-step, behind which that K-step can be read and the stage of the one being
+//     multiplied be filled again.
+//   - Bound by the chain of K-steps where tiles are few: four dependent MFMAs and the fragment reads of the
+//     next K-step, which run behind them; about 170 ns per K-step (8 experts x 3 rows 3072 -> 768:
+//     11.2 us; the four wavefronts summing a quarter of K each, which gives other bits, 10.7 us; one
+//     wavefront that loads by itself 18.7 us).  K-steps of 128 with half the barriers change nothing.
 //   - Rows past the expert's load and past N address past the buffer extent: zeros, no request.
 //   - Every wavefront finds the tile by itself (DPP scan + ballot over the loads, the weight
 //     pointers fetched in the same round trip), so the first weight request leaves two round trips
 //     after the start.  Gathered rows add one, which the weight requests do not wait for.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "grouped_gemm.hpp"
@@ -63,36 +68,41 @@ __device__ __forceinline__ void load_word_to_lds(const i32x4& rsrc, uint32_t vof
 
 template <int N>
 __device__ __forceinline__ void wait_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
-// waits until at most `left` of this wavefront's loads are outstanding (rounded down to an even number)
+// waits until at most `left` of this wavefront's loads are outstanding
 __device__ __forceinline__ void wait_loads(int left) {
-  switch (left >> 1) {
-#define BRT_WAIT(n) case n: wait_loads_but<2 * n>(); break;
+  switch (left) {
+#define BRT_WAIT(n) case n: wait_loads_but<n>(); break;
     BRT_WAIT(1) BRT_WAIT(2) BRT_WAIT(3) BRT_WAIT(4) BRT_WAIT(5) BRT_WAIT(6) BRT_WAIT(7) BRT_WAIT(8)
-    BRT_WAIT(9) BRT_WAIT(10) BRT_WAIT(11) BRT_WAIT(12) BRT_WAIT(13) BRT_WAIT(14) BRT_WAIT(15) BRT_WAIT(16)
-    BRT_WAIT(17) BRT_WAIT(18) BRT_WAIT(19) BRT_WAIT(20) BRT_WAIT(21) BRT_WAIT(22) BRT_WAIT(23) BRT_WAIT(24)
+    BRT_WAIT(9) BRT_WAIT(10) BRT_WAIT(11) BRT_WAIT(12)
 #undef BRT_WAIT
     default: wait_loads_but<0>();
   }
 }
-__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory"); }
+// lgkmcnt(0) alone, known to the compiler (which counts on behind it)
+__device__ __forceinline__ void wait_lds() {
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  asm volatile("" : : : "memory");
+}
 
-template <int XR, int NT, int S, int D>
+constexpr int kWaves = 4;
+
+template <int XR, int NT, int D>
 struct Shape {
   static constexpr int kXi = XR / 8, kWi = NT * 4;             // load instructions of one K-step: rows of x, weight rows
+  static constexpr int kXw = kXi / kWaves, kWw = kWi / kWaves;  // ... of one wavefront
   static constexpr int kStage = (kXi + kWi) * 1024;
   static constexpr int kBN = NT * 32;
-  static constexpr int kSumRow = kBN * 4 + 16;                 // padded row of a partial sum
-  static constexpr int kRing = D * kStage > XR * kSumRow ? D * kStage : XR * kSumRow;
-  static constexpr int kLds = S * kRing;
-  static_assert(XR % 32 == 0, "whole MFMA row tiles");
-  static_assert(D * (kXi + kWi) <= 48, "the waits count up to 48 loads");
+  static constexpr int kSumRow = kBN * 4 + 16;                 // padded row of the sums on their way out
+  static constexpr int kLds = D * kStage > XR * kSumRow ? D * kStage : XR * kSumRow;
+  static_assert(XR % 32 == 0 && XR / 32 * NT <= kWaves, "at most one 32 x 32 block per wavefront");
+  static_assert(D >= 2 && (D - 1) * (kXw + kWw) <= 12 && D * kWw <= 12, "the waits count up to 12 loads");
 };
 
-template <int XR, int NT, int S, int D, int ACT, bool ROUTED, bool OUTF32>
-__global__ __launch_bounds__(S * 64) void grouped_gemm_skinny_kernel(GemmArgs a) {
-  using H = Shape<XR, NT, S, D>;
-  constexpr int MT = XR / 32;
-  constexpr int kXi = H::kXi, kWi = H::kWi, kL = kXi + kWi;
+template <int XR, int NT, int D, int ACT, bool ROUTED, bool OUTF32>
+__global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(GemmArgs a) {
+  using H = Shape<XR, NT, D>;
+  constexpr int kWi = H::kWi, kXw = H::kXw, kWw = H::kWw, kL = kXw + kWw;
+  constexpr int kBlocks = XR / 32 * NT;  // 32 x 32 blocks of the tile, one wavefront each
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -134,137 +144,164 @@ __global__ __launch_bounds__(S * 64) void grouped_gemm_skinny_kernel(GemmArgs a)
     return;
   }
 
-  // ---- this wavefront's slice of K: at least two K-steps ------------------------------------------
   const int k_tiles = (K + kBK - 1) / kBK;
-  const int per = max(2, (k_tiles + S - 1) / S);
-  const int parts = (k_tiles + per - 1) / per;  // wavefronts that have one
-  const int kt0 = wave * per, n = __builtin_amdgcn_readfirstlane(min(per, k_tiles - kt0));
-  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem))) + wave * H::kRing;
-  char* const ring = smem + wave * H::kRing;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
 
-  f32x16 acc[MT][NT];
+  // ---- this wavefront's loads: row groups of 8 rows, kWw of the weights and kXw of x ----------------
+  // Lane l lands at slot l & 7 of row l >> 3 of the 8 rows a load fills and fetches chunk
+  // slot ^ ((row >> 1) & 7) of that row; a chunk past K (the last K-step only) reads as zero.
+  const bool gather = ROUTED && a.gather != 0;
+  const i32x4 res_w = make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2);
+  const i32x4 res_x = gather ? make_rsrc(a.x, static_cast<size_t>(a.T) * K * 2)
+                             : make_rsrc(a.x + static_cast<size_t>(row0) * K, static_cast<size_t>(a.P - row0) * K * 2);
+  const int r8 = lane >> 3;
+  const int first_w = wave * kWw, first_x = wave * kXw;  // row groups
+  auto chunk = [&](int group) { return (lane & 7) ^ (r8 >> 1) ^ ((group & 1) << 2); };
+  uint32_t off_w[kWw], off_x[kXw];
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int i = 0; i < kWw; ++i) {
+    const int row = (first_w + i) * 8 + r8;
+    off_w[i] = n0 + row < a.N ? (static_cast<uint32_t>(row) * K + chunk(first_w + i) * 8) * 2 : kOutOfRange;
+  }
+  const int tail_chunks = K % kBK != 0 ? (K % kBK) / 8 : 8;  // chunks of the last K-step that exist
+  auto fetch = [&](const i32x4& res, uint32_t off, int group, int kt, uint32_t to) {
+    if (kt == k_tiles - 1 && chunk(group) >= tail_chunks) off = kOutOfRange;
+    load_to_lds(res, off, kt * kRowB, to);
+  };
+  auto load_w = [&](int s, uint32_t stage, int i) { fetch(res_w, off_w[i], first_w + i, s, lds0 + stage + (first_w + i) * 1024); };
+  auto load_x = [&](int s, uint32_t stage, int i) { fetch(res_x, off_x[i], first_x + i, s, lds0 + stage + (kWi + first_x + i) * 1024); };
+  const int primed = min(D, k_tiles);
+  if (gather) {
+    // The words that name this wavefront's rows land in the last stage's room for them (a direct load, so
+    // that waiting for it does not wait for the weight requests behind it).
+    const uint32_t words = (D - 1) * H::kStage + (kWi + first_x) * 1024;
+    const int row = first_x * 8 + lane;
+    const bool slot_ok = lane < kXw * 8 && row < rows && (a.tag_vector || seat0 + row < a.T);
+    const size_t first = a.tag_vector ? static_cast<size_t>(row0) : static_cast<size_t>(seat0) * a.E + e;
+    const i32x4 res_t = make_rsrc(a.tags + first, static_cast<size_t>(XR) * (a.tag_vector ? 1 : a.E) * 4);
+    load_word_to_lds(res_t, slot_ok ? static_cast<uint32_t>(row) * (a.tag_vector ? 1 : a.E) * 4 : kOutOfRange, lds0 + words);
+    for (int s = 0; s < primed; ++s)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = f32x16{};
-
-  if (n > 0) {
-    // Lane l lands at slot l & 7 of row l >> 3 of the 8 rows a load fills and fetches chunk
-    // slot ^ ((row >> 1) & 7) of that row; a chunk past K (the last K-step only) reads as zero.
-    const bool gather = ROUTED && a.gather != 0;
-    const i32x4 res_w = make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2);
-    const i32x4 res_x = gather ? make_rsrc(a.x, static_cast<size_t>(a.T) * K * 2)
-                               : make_rsrc(a.x + static_cast<size_t>(row0) * K, static_cast<size_t>(a.P - row0) * K * 2);
-    const int r8 = lane >> 3;
-    const int chunk0 = (lane & 7) ^ (r8 >> 1);  // even groups of 8 rows; odd ones flip bit 2
-    uint32_t off_w[kWi], off_x[kXi];
+      for (int i = 0; i < kWw; ++i) load_w(s, s * H::kStage, i);
+    wait_loads(primed * kWw);
 #pragma unroll
-    for (int i = 0; i < kWi; ++i) {
-      const int row = i * 8 + r8;
-      off_w[i] = n0 + row < a.N ? (static_cast<uint32_t>(row) * K + (chunk0 ^ ((i & 1) << 2)) * 8) * 2 : kOutOfRange;
+    for (int i = 0; i < kXw; ++i) {
+      const int word = *reinterpret_cast<const volatile int*>(smem + words + (i * 8 + r8) * 4);
+      const int cell = cell_of_word(a, word);
+      off_x[i] = cell >= 0 ? (static_cast<uint32_t>(cell) * K + chunk(first_x + i) * 8) * 2 : kOutOfRange;
     }
-    const int tail_chunks = K % kBK != 0 ? (K % kBK) / 8 : 8;  // chunks of the last K-step that exist
-    auto fetch = [&](const i32x4& res, uint32_t off, int i, int kt, uint32_t to) {
-      if (kt == k_tiles - 1 && (chunk0 ^ ((i & 1) << 2)) >= tail_chunks) off = kOutOfRange;
-      load_to_lds(res, off, kt * kRowB, to);
-    };
-    auto load_w = [&](int s) {
-      const uint32_t to = lds0 + (s % D) * H::kStage;
+    wait_lds();
+    for (int s = 0; s < primed; ++s)
 #pragma unroll
-      for (int i = 0; i < kWi; ++i) fetch(res_w, off_w[i], i, kt0 + s, to + i * 1024);
-    };
-    auto load_x = [&](int s) {
-      const uint32_t to = lds0 + (s % D) * H::kStage + kWi * 1024;
+      for (int i = 0; i < kXw; ++i) load_x(s, s * H::kStage, i);
+  } else {
 #pragma unroll
-      for (int i = 0; i < kXi; ++i) fetch(res_x, off_x[i], i, kt0 + s, to + i * 1024);
-    };
-    const int primed = min(D, n);
-    if (gather) {
-      // The words that name the rows land in the last stage's room for x (a direct load, so that
-      // waiting for it does not wait for the weight requests behind it).
-      const int last = D - 1;
-      const uint32_t words = lds0 + last * H::kStage + kWi * 1024;
-      const bool slot_ok = lane < rows && (a.tag_vector || seat0 + lane < a.T);
-      const size_t first = a.tag_vector ? static_cast<size_t>(row0) : static_cast<size_t>(seat0) * a.E + e;
-      const i32x4 res_t = make_rsrc(a.tags + first, static_cast<size_t>(XR) * (a.tag_vector ? 1 : a.E) * 4);
-      load_word_to_lds(res_t, slot_ok ? static_cast<uint32_t>(lane) * (a.tag_vector ? 1 : a.E) * 4 : kOutOfRange, words);
-      for (int s = 0; s < primed; ++s) load_w(s);
-      wait_loads(primed * kWi);
+    for (int i = 0; i < kXw; ++i) {
+      const int row = (first_x + i) * 8 + r8;
+      off_x[i] = row < rows ? (static_cast<uint32_t>(row) * K + chunk(first_x + i) * 8) * 2 : kOutOfRange;
+    }
+    for (int s = 0; s < primed; ++s) {
 #pragma unroll
-      for (int i = 0; i < kXi; ++i) {
-        const int word = *reinterpret_cast<const volatile int*>(ring + last * H::kStage + kWi * 1024 + (i * 8 + r8) * 4);
-        const int cell = cell_of_word(a, word);
-        off_x[i] = cell >= 0 ? (static_cast<uint32_t>(cell) * K + (chunk0 ^ ((i & 1) << 2)) * 8) * 2 : kOutOfRange;
+      for (int i = 0; i < kWw; ++i) load_w(s, s * H::kStage, i);
+#pragma unroll
+      for (int i = 0; i < kXw; ++i) load_x(s, s * H::kStage, i);
+    }
+  }
+
+  // ---- K loop ----------------------------------------------------------------------------------------
+  // MFMA operand: this lane feeds row (lane % 32), k-half (lane / 32) of a 32 x 16 block
+  const bool multiplies = wave < kBlocks;
+  const int block_x = wave / NT, block_w = wave % NT;
+  const int frag_row = lane & 31, frag_k = lane >> 5;
+  const int swz = (frag_row >> 1) & 7;
+  const char* const from_w = smem + (block_w * 32 + frag_row) * kRowB;
+  const char* const from_x = smem + kWi * 1024 + (block_x * 32 + frag_row) * kRowB;
+  struct Frags {
+    bf16x8 w[kSub], x[kSub];
+  };
+  auto read_frags = [&](Frags& f, uint32_t stage, int ks) {
+    const uint32_t at = stage + (((ks * 2 + frag_k) ^ swz) << 4);
+    f.w[ks] = *reinterpret_cast<const bf16x8*>(from_w + at);
+    f.x[ks] = *reinterpret_cast<const bf16x8*>(from_x + at);
+  };
+  // this wavefront's loads issued after the last one of K-step s, once K-steps up to `issued` have been requested
+  auto younger = [&](int s, int issued) {
+    return gather && s < primed ? (primed - 1 - s) * kXw + max(issued + 1 - primed, 0) * kL : (issued - s) * kL;
+  };
+  f32x16 acc = {};
+  // K-step s, whose stage every wavefront has read: the loads of s + D go there.  A multiplying wavefront has
+  // its fragments in `cur`; those of s + 1 come out of the next stage meanwhile (no branch around the reads:
+  // the compiler would wait for all of them in front of every MFMA; behind the last K-step they
+  // read words that nothing uses).
+  using Yes = std::integral_constant<bool, true>;
+  using No = std::integral_constant<bool, false>;
+  uint32_t stage = 0;
+  auto step = [&](const Frags& cur, Frags& next, int s, auto multiply, auto fills) {
+    constexpr bool kMultiply = decltype(multiply)::value, kFills = decltype(fills)::value;
+    const uint32_t ahead = stage + H::kStage == D * H::kStage ? 0 : stage + H::kStage;
+    if (kFills && !(gather && s < primed)) wait_loads_but<(D - 2) * kL>();
+    else if (s + 1 < k_tiles) wait_loads(younger(s + 1, min(s + D, k_tiles) - 1));
+    __builtin_amdgcn_s_barrier();
+    if (!kFills && s + D < k_tiles) {
+#pragma unroll
+      for (int i = 0; i < kL; ++i) i < kWw ? load_w(s + D, stage, i) : load_x(s + D, stage, i - kWw);
+    }
+#pragma unroll
+    for (int ks = 0; ks < kSub; ++ks) {
+      if constexpr (kMultiply) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.w[ks], cur.x[ks], acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        read_frags(next, ahead, ks);
       }
+      if constexpr (kFills) {
+#pragma unroll
+        for (int i = ks * kL / kSub; i < (ks + 1) * kL / kSub; ++i) i < kWw ? load_w(s + D, stage, i) : load_x(s + D, stage, i - kWw);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (kMultiply) wait_lds();  // behind the next barrier the stage of s + 1 may be filled again
+    stage = ahead;
+  };
+  auto k_loop = [&](auto multiply) {
+    Frags f0, f1;
+    wait_loads(younger(0, primed - 1));
+    __builtin_amdgcn_s_barrier();
+    if constexpr (decltype(multiply)::value) {
+#pragma unroll
+      for (int ks = 0; ks < kSub; ++ks) read_frags(f0, 0, ks);
       wait_lds();
-      for (int s = 0; s < primed; ++s) load_x(s);
-    } else {
-#pragma unroll
-      for (int i = 0; i < kXi; ++i) {
-        const int row = i * 8 + r8;
-        off_x[i] = row < rows ? (static_cast<uint32_t>(row) * K + (chunk0 ^ ((i & 1) << 2)) * 8) * 2 : kOutOfRange;
-      }
-      for (int s = 0; s < primed; ++s) load_w(s), load_x(s);
     }
+    int s = 0;
+    for (; s + 1 + D < k_tiles; s += 2) {
+      step(f0, f1, s, multiply, Yes{});
+      step(f1, f0, s + 1, multiply, Yes{});
+    }
+    for (; s < k_tiles; s += 2) {
+      step(f0, f1, s, multiply, No{});
+      if (s + 1 < k_tiles) step(f1, f0, s + 1, multiply, No{});
+    }
+  };
+  if (multiplies) k_loop(Yes{});
+  else k_loop(No{});
 
-    // MFMA operand: this lane feeds row (lane % 32), k-half (lane / 32) of a 32 x 16 block
-    const int frag_row = lane & 31, frag_k = lane >> 5;
-    const int swz = (frag_row >> 1) & 7;
-    const int frag_w = frag_row * kRowB;
-    const int frag_x = kWi * 1024 + frag_row * kRowB;
-    for (int s = 0; s < n; ++s) {
-      // loads issued after the last one of K-step s
-      int younger = min(D - 1, n - 1 - s) * kL;
-      if (gather && s < primed) younger = (primed - 1 - s) * kXi + min(s, max(n - D, 0)) * kL;
-      wait_loads(younger);
-      const char* const at = ring + (s % D) * H::kStage;
-      bf16x8 fw[kSub][NT], fx[kSub][MT];
+  // The sums into LDS (behind the last barrier nothing reads or fills the stages): element r of a block is
+  // its row lane % 32, column 8 * (r / 4) + 4 * (lane / 32) + r % 4
+  if (multiplies) {
 #pragma unroll
-      for (int ks = 0; ks < kSub; ++ks) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-          fw[ks][j] = *reinterpret_cast<const bf16x8*>(at + frag_w + j * 32 * kRowB + (((ks * 2 + frag_k) ^ swz) << 4));
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-          fx[ks][i] = *reinterpret_cast<const bf16x8*>(at + frag_x + i * 32 * kRowB + (((ks * 2 + frag_k) ^ swz) << 4));
-      }
-      wait_lds();  // the fragments are in registers: the slot may be filled again
-      if (s + D < n) load_w(s + D), load_x(s + D);
-#pragma unroll
-      for (int ks = 0; ks < kSub; ++ks)
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int j = 0; j < NT; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[ks][j], fx[ks][i], acc[i][j], 0, 0, 0);
-    }
-
-    // partial sums into this wavefront's ring (every load has landed): element r of tile (i, j) is
-    // row 32 i + lane % 32, column 32 j + 8 * (r / 4) + 4 * (lane / 32) + r % 4
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<f32x4*>(ring + (i * 32 + frag_row) * H::kSumRow + (j * 32 + 8 * g + 4 * frag_k) * 4) =
-              f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-    }
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(smem + (block_x * 32 + frag_row) * H::kSumRow + (block_w * 32 + 8 * g + 4 * frag_k) * 4) =
+          f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
   }
   __syncthreads();
 
-  // ---- sum over the wavefronts, bias, activation ---------------------------------------------------
+  // ---- bias, activation ---------------------------------------------------
   auto column_sum = [&](int r, int c) {  // one output element (accumulate form)
-    float v = 0.0f;
-    for (int s = 0; s < parts; ++s) {
-      const float p = reinterpret_cast<const float*>(smem + s * H::kRing + r * H::kSumRow)[c];
-      v = s == 0 ? p : v + p;
-    }
+    const float v = reinterpret_cast<const float*>(smem + r * H::kSumRow)[c];
     return apply_act<ACT>(v + (a.bias != nullptr ? static_cast<float>(a.bias[e][n0 + c]) : 0.0f));
   };
   if constexpr (ROUTED && !OUTF32) {
     if (a.gates != nullptr) {  // acc_out[cell] += gate * bf16(row), as in grouped_gemm.hip
-      for (int q = tid; q < rows * H::kBN; q += S * 64) {
+      for (int q = tid; q < rows * H::kBN; q += kWaves * kWave) {
         const int r = q / H::kBN, c = q - r * H::kBN;
         const int cell = routed_cell(a, e, row0 + r, seat0 + r);
         if (cell < 0 || n0 + c >= a.N) continue;
@@ -277,7 +314,7 @@ __global__ __launch_bounds__(S * 64) void grouped_gemm_skinny_kernel(GemmArgs a)
   }
   // 8 columns of one row per thread and step: 16-byte stores (two of them for fp32)
   constexpr int kChunks = H::kBN / 8;
-  for (int q = tid; q < rows * kChunks; q += S * 64) {
+  for (int q = tid; q < rows * kChunks; q += kWaves * kWave) {
     const int r = q / kChunks, c = q - r * kChunks;
     if (n0 + c * 8 >= a.N) continue;
     long to = row0 + r;
@@ -289,11 +326,9 @@ __global__ __launch_bounds__(S * 64) void grouped_gemm_skinny_kernel(GemmArgs a)
     }
     if (to < 0) continue;
     float v[8];
-    for (int s = 0; s < parts; ++s) {
-      const float* const from = reinterpret_cast<const float*>(smem + s * H::kRing + r * H::kSumRow) + c * 8;
+    const float* const from = reinterpret_cast<const float*>(smem + r * H::kSumRow) + c * 8;
 #pragma unroll
-      for (int w = 0; w < 8; ++w) v[w] = s == 0 ? from[w] : v[w] + from[w];
-    }
+    for (int w = 0; w < 8; ++w) v[w] = from[w];
     const __bf16* const bias = a.bias != nullptr ? a.bias[e] + n0 + c * 8 : nullptr;
 #pragma unroll
     for (int w = 0; w < 8; ++w) v[w] = apply_act<ACT>(v[w] + (bias != nullptr ? static_cast<float>(bias[w]) : 0.0f));
@@ -314,73 +349,88 @@ __global__ __launch_bounds__(S * 64) void grouped_gemm_skinny_kernel(GemmArgs a)
   }
 }
 
-template <int XR, int NT, int S, int D, int ACT, bool ROUTED, bool OUTF32>
+template <int XR, int NT, int D, int ACT, bool ROUTED, bool OUTF32>
 int launch(GemmArgs& a, hipStream_t st) {
-  using H = Shape<XR, NT, S, D>;
+  using H = Shape<XR, NT, D>;
   a.tiles_n = (a.N + H::kBN - 1) / H::kBN;
   // the sum over experts of ceil(M_e / XR) never exceeds P / XR + min(E, P)
   const long blocks = (static_cast<long>(a.P) + XR - 1) / XR + std::min(a.E, a.P);
-  auto* fn = &grouped_gemm_skinny_kernel<XR, NT, S, D, ACT, ROUTED, OUTF32>;
+  auto* fn = &grouped_gemm_skinny_kernel<XR, NT, D, ACT, ROUTED, OUTF32>;
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(fn), H::kLds); rc != BRT_OK) return rc;
-  hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks * a.tiles_n)), dim3(S * 64), H::kLds, st, a);
+  hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks * a.tiles_n)), dim3(kWaves * kWave), H::kLds, st, a);
   return check_launch("grouped_gemm_skinny_kernel");
 }
 
-template <int XR, int NT, int S, int D, int ACT>
+template <int XR, int NT, int D, int ACT>
 int launch_form(GemmArgs& a, hipStream_t st) {
   const bool f32 = a.out_f32 != nullptr;
-  if (a.tags != nullptr) return f32 ? launch<XR, NT, S, D, ACT, true, true>(a, st) : launch<XR, NT, S, D, ACT, true, false>(a, st);
-  return f32 ? launch<XR, NT, S, D, ACT, false, true>(a, st) : launch<XR, NT, S, D, ACT, false, false>(a, st);
+  if (a.tags != nullptr) return f32 ? launch<XR, NT, D, ACT, true, true>(a, st) : launch<XR, NT, D, ACT, true, false>(a, st);
+  return f32 ? launch<XR, NT, D, ACT, false, true>(a, st) : launch<XR, NT, D, ACT, false, false>(a, st);
 }
 
-template <int XR, int NT, int S, int D>
+template <int XR, int NT, int D>
 int launch_act(GemmArgs& a, int act, hipStream_t st) {
-  if (act == BRT_ACT_GELU) return launch_form<XR, NT, S, D, BRT_ACT_GELU>(a, st);
-  if (act == BRT_ACT_RELU) return launch_form<XR, NT, S, D, BRT_ACT_RELU>(a, st);
-  return launch_form<XR, NT, S, D, BRT_ACT_NONE>(a, st);
+  if (act == BRT_ACT_GELU) return launch_form<XR, NT, D, BRT_ACT_GELU>(a, st);
+  if (act == BRT_ACT_RELU) return launch_form<XR, NT, D, BRT_ACT_RELU>(a, st);
+  return launch_form<XR, NT, D, BRT_ACT_NONE>(a, st);
 }
 
 }  // namespace
 
-// Where this kernel is taken, against the 160-row kernel.  Both were timed on 2 to 200 rows per expert,
-// 4 to 128 experts, 512 <-> 2048, 768 <-> 3072, 1024 <-> 4096, 2048 <-> 8192 and 320 <-> 640; the
-// rule gives up small gains rather than lose where the 160-row kernel is the faster one.
+// Where this kernel is taken, against the 160-row kernel.  Both were timed on 1 to 2000 rows per expert,
+// 2 to 128 experts and 2 MB to 1 GB of weights (us, 160-row kernel -> this one); the rule gives up small gains
+// rather than lose where the 160-row kernel is the faster one.
 //   - Up to 28 rows per expert (one row block): while the weights are less than 0.3 GB (8 experts x 3 rows
-//     3072 -> 768: 43.9 -> 9.7 us, 32 x 8 rows 4096 -> 1024 68.3 -> 46.3 us).  Beyond, the wide tiles stream
-//     them at the memory's rate (32 x 19 rows 6656 -> 1664, 709 MB: 113 us there, 129 us here; 32 x 16 rows
-//     1920 -> 3840, 472 MB: 75.5 and 84.0 us), except where they cannot: half of the CUs without a
-//     tile (16 x 12 rows 6656 -> 1664 89.6 -> 66.7 us), a K whose rows lie multiples of 4 KB apart (64 x 16
-//     rows 4096 -> 1024 119 -> 91 us) or experts of which many get no row at all (128 experts, 183 rows
-//     896 -> 3584 124 -> 96 us); up to 1 GB (32 x 8 rows 8192 -> 2048, 1.07 GB: 171 us there, 200 us here).
-//   - More rows: every block of 32 or 64 rows streams the weights again (from the L2), which pays
-//     while the 160-row kernel has too few 160 x 256 tiles for the CUs: up to 72 of them, however many
-//     rows that are (8 x 120 rows 3072 -> 768 46.9 -> 22.4 us, 4 x 1300 rows 1024 -> 256 24.5 -> 12.3 us,
-//     32 x 120 rows 2048 -> 512 36.6 -> 36.2 us; not 64 x 120 rows, 128 tiles: 44.9 -> 59.9 us), and up to
-//     160 for few experts of up to 128 rows and 0.15 GB (4 x 120 rows 2048 -> 8192 77.2 -> 43.0 us; not 16 x 40
-//     rows 3840 -> 1920, 236 MB: 55.9 -> 72.5 us).
+//     3072 -> 768 43.7 -> 11.2, 32 x 6 rows 4096 -> 1024 62.9 -> 55.2, 1024 -> 4096 47.6 -> 46.5).  Beyond, the wide
+//     tiles stream them at the memory's rate (32 x 24 rows 2560 -> 1920, 314 MB: 56.0 there, 60.3 here; 64 x 6 rows
+//     1024 -> 4096, 536 MB: 86.8 and 90.7), except where they cannot: half of the CUs without a tile
+//     (16 x 12 rows 6656 -> 1664 89.6 -> 64.5), a K whose rows lie multiples of 4 KB apart (64 x 16 rows
+//     4096 -> 1024 120.8 -> 108.3, 32 x 20 rows 2048 -> 2560 80.9 -> 65.8) or experts of which many get no
+//     row at all; up to 1 GB (32 x 8 rows 8192 -> 2048, 1.07 GB: 163 there, 226 here).
+//   - Up to 64 rows: every block of rows streams the weights again (from the L2), which pays while the
+//     160-row kernel has too few 160 x 256 tiles for the CUs: up to 72 of them, and up to 160 with less than
+//     0.15 GB (16 x 64 rows 512 -> 2048 14.4 -> 10.1, 32 x 40 rows 768 -> 1024 17.2 -> 13.8, 16 x 60 rows
+//     1024 -> 2560, 160 tiles, 21.5 -> 20.9; not 16 x 40 rows 3840 -> 1920, 236 MB).
+//   - More: up to 96 tiles (8 x 120 rows 768 -> 3072 19.0 -> 15.6, 3072 -> 768 46.4 -> 21.0, 16 x 100 rows
+//     768 -> 1536 18.6 -> 15.1; 112 tiles, 14 x 120 rows 1024 -> 2048: 22.3 there, 23.3 here; 144 tiles, 16 x 120
+//     rows 1024 -> 2304: 22.7 and 30.5) of up to 32 experts (32 x 120 rows 2048 -> 512 35.1 -> 29.5; with more of
+//     them every XCD reads most of x and of the weights: 64 x 120 rows 2048 -> 256 35.7 there, 43.1 here),
+//     and up to 160 with fewer experts than XCDs, some of which the 160-row kernel leaves idle (4 x 120 rows
+//     2048 -> 8192 69.3 -> 41.9).
 bool skinny_gemm_applies(const GemmArgs& a) {
   const long used = std::min(a.E, a.P);
   const long tiles = std::max<long>((a.P + 159) / 160, used) * ((a.N + 255) / 256);
   const double weight_bytes = 2.0 * used * a.N * a.K;
+  if (a.P > 64 * used) {
+    if (tiles <= 96) return used <= 32;
+    return a.P <= 128 * used && tiles <= 160 && used < 8 && weight_bytes < 1.5e8;
+  }
   if (tiles <= 72) return true;
   if (a.P <= 28 * used) {
     if (weight_bytes < 3e8) return true;
     return weight_bytes < 1e9 && (tiles <= 128 || a.K % 2048 == 0 || 2l * a.P <= 3 * used);
   }
-  return a.P <= 128 * used && tiles <= 160 && a.E <= 16 && weight_bytes < 1.5e8;
+  return tiles <= 160 && weight_bytes < 1.5e8;
 }
 
-// Shape of the tile.  Few workgroups: the narrowest one, so that every CU gets one (at most 264 of 32 x
-// 64).  Else 64 columns, which read the activation rows half as often; 64 rows where experts have
-// more than 64 (the weights are streamed half as often).  A long K with few rows (K = 3072, 24 rows,
-// 8 experts: 11.1 us against 15.4 us) stays on the narrow tile, whose two stages keep loads in flight.
+// Shape of the tile; the estimates take an expert's last row block as half full.
+//   - 64 x 64 where experts have more than 32 rows and that makes a tile for most CUs (8 x 120 rows
+//     768 -> 3072 15.7 us, 19.3 with 32 x 64): with a short K three stages and three workgroups on a CU
+//     (16 x 64 rows 512 -> 2048 10.2 us, four stages 11.5), else four (8 x 120 rows 3072 -> 768 20.9, three 22.7).
+//   - 32 x 32 where even 32 x 64 would leave half of the CUs without a tile (8 x 3 rows 3072 -> 768 11.2 us, 13.4),
+//     and for a short K with so few rows that reading them twice as often costs nothing (32 x 6 rows
+//     1024 -> 4096 46.2 us, 50.0).
+//   - 32 x 64 otherwise (8 x 28 rows 4096 -> 1024 19.8 us, 32 x 32 22.4; 32 x 6 rows 4096 -> 1024 55.1 and 62.2).
 int launch_skinny_gemm(GemmArgs& a, int act, hipStream_t st) {
   const long used = std::min(a.E, a.P);
   const double rows = static_cast<double>(a.P) / used;
-  const bool narrow = used * std::max(1.0, rows / 32 + 0.5) * a.N / 64 <= 264 || (rows <= 40 && a.K > 1536);
-  if (narrow) return launch_act<32, 1, 4, 2>(a, act, st);
-  if (rows <= 40 || (rows <= 64 && a.K <= 1024)) return launch_act<32, 2, 4, 1>(a, act, st);
-  return launch_act<64, 2, 4, 1>(a, act, st);
+  auto tiles = [&](int block) { return used * (rows > block ? rows / block + 0.5 : 1.0) * ((a.N + 63) / 64); };
+  if (rows > 32 && tiles(64) >= 192) {
+    if (a.K <= 1024) return launch_act<64, 2, 3>(a, act, st);
+    return launch_act<64, 2, 4>(a, act, st);
+  }
+  if (tiles(32) <= 112 || (tiles(32) <= 160 && a.K <= 2048) || (rows <= 16 && a.K <= 1536)) return launch_act<32, 1, 6>(a, act, st);
+  return launch_act<32, 2, 5>(a, act, st);
 }
 
 }  // namespace brt

@@ -601,9 +601,9 @@ def test_ping_pong_tiles_with_routing_and_fp32_output(T, E, K, N, k, cap, pad):
 
 @pytest.mark.parametrize("K,N", [
     (8, 8),        # one chunk of one K-step, one chunk of columns
-    (72, 56),      # K tail in the second K-step of the only wavefront that has a slice
-    (192, 72),     # two wavefronts share three K-steps; the second column tile holds 8 columns
-    (776, 1000),   # thirteen K-steps on four wavefronts, K and N tails
+    (72, 56),      # two K-steps, the second one cut
+    (192, 72),     # three K-steps; the second column tile holds 8 columns
+    (776, 1000),   # thirteen K-steps, K and N tails
     (1600, 96),    # a long K
     (4096, 64),
 ])
@@ -614,9 +614,76 @@ def test_ping_pong_tiles_with_routing_and_fp32_output(T, E, K, N, k, cap, pad):
     [150, 90, 130, 110],                         # blocks of 64 rows
 ])
 def test_split_k_tiles(loads, K, N):
-    """Few rows or few tiles: the kernel whose wavefronts share K."""
+    """Few rows or few tiles: the kernel with tiles of 32 or 64 rows."""
     run(loads, K, N)
     run(loads, K, N, act="gelu", bias=True, seed=1, slack=40)
+
+
+def _kernel_for(P, E, K, N):
+    """Which kernel the host takes for these sizes (all but the weighted accumulate form), on 256 CUs."""
+    used = min(E, P)
+    big = ((P + 255) // 256 + (E + 1) // 2) * -(-N // 256)
+    if K % 64 == 0 and K >= 128 and P > E * 160 and (big >= 512 or 192 <= big <= 256):
+        return "ping-pong"
+    tiles = max((P + 159) // 160, used) * -(-N // 256)
+    weight = 2.0 * used * N * K
+    if P > 64 * used:
+        few = used <= 32 if tiles <= 96 else P <= 128 * used and tiles <= 160 and used < 8 and weight < 1.5e8
+    elif tiles <= 72:
+        few = True
+    elif P <= 28 * used:
+        few = weight < 3e8 or (weight < 1e9 and (tiles <= 128 or K % 2048 == 0 or 2 * P <= 3 * used))
+    else:
+        few = tiles <= 160 and weight < 1.5e8
+    return "few rows" if few else "160 rows"
+
+
+@pytest.mark.parametrize("loads,K,N,bounds", [
+    ([9, 0, 3, 1, 20, 31, 2, 8, 17, 1, 7, 4], 1088, 4104, {"few rows": 103, "160 rows": 2400, "ping-pong": 8000}),
+    ([3, 70, 0, 33, 150], 1096, 136, {"few rows": 256, "160 rows": 16000}),  # K and N tails
+    ([30] * 32, 4096, 1024, {"few rows": 960 - 64, "160 rows": 1024}),       # what a layer keeps and what it may keep
+])
+def test_bits_of_a_row_do_not_depend_on_the_rows_of_the_launch(loads, K, N, bounds):
+    """The number of rows of the path-major buffers (the rows that exist, or a bound of them) selects the
+    kernel; the products of an output element are summed in order of K by all of them, so the rows
+    are the same bit for bit: plain, fp32-output, gathering and scattering forms."""
+    from brainstorm_amd.jit import grouped_linear
+
+    E, live = len(loads), bounds["few rows"]
+    if sum(loads) > live:  # the first experts lose rows until they fit
+        loads = [m - (sum(loads) - live) // E for m in loads]
+    assert sum(loads) == live
+    g = torch.Generator(device="cuda").manual_seed(K)
+    w = (torch.randn(E, N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    bias = torch.randn(E, N, generator=g, device="cuda").to(torch.bfloat16)
+    table, bias_table = (torch.tensor([t[e].data_ptr() for e in range(E)], dtype=torch.int64, device="cuda") for t in (w, bias))
+    d_loads = torch.tensor(loads, dtype=torch.int32, device="cuda")
+    cells = torch.randn(live + 9, K, generator=g, device="cuda").to(torch.bfloat16)
+    order = torch.randperm(live + 9, generator=g, device="cuda")[:live]
+    results = {}
+    for kernel, P in bounds.items():
+        assert _kernel_for(P, E, K, N) == kernel
+        x = torch.zeros(P, K, dtype=torch.bfloat16, device="cuda")
+        x[:live] = cells[order]
+        entries = torch.zeros(P, dtype=torch.int32, device="cuda")
+        entries[:live] = order.int() + 1
+        got = []
+        for dtype in (torch.bfloat16, torch.float32):
+            out = torch.full((P, N), float("nan"), dtype=dtype, device="cuda")
+            grouped_linear(x, out, table, bias_table, d_loads, K, N, "gelu")
+            got.append(out[:live])
+        out = torch.full((P, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        grouped_linear(cells, out, table, bias_table, d_loads, K, N, "gelu", row_entries=entries, gather=True)
+        got.append(out[:live])
+        out = torch.full((live + 9, N), 3.0, dtype=torch.bfloat16, device="cuda")
+        grouped_linear(x, out, table, bias_table, d_loads, K, N, "gelu", row_entries=entries, scatter=True)
+        got.append(out)
+        results[kernel] = got
+    first = results.pop("few rows")
+    assert torch.isfinite(first[1]).all()
+    for kernel, got in results.items():
+        for form, a, b in zip(("bf16", "fp32", "gathered", "scattered"), first, got):
+            assert torch.equal(a, b), (kernel, form)
 
 
 def test_grouped_gemm_random_shapes():
