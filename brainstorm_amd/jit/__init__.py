@@ -87,13 +87,13 @@ class _BranchOperands:
         fp32, key = _lib.native().branch_key(operands, first, step, used, self.what)
         if key != self.key:
             tensors = list(operands[first::step])
-            self.copies = self.sources = None
+            sources = copies = None
             if fp32:
-                self.sources = tensors[:used]
-                self.copies = [_to_bf16(t.detach()) for t in self.sources]
-                tensors = self.copies
-            self.table = torch.tensor([t.data_ptr() for t in tensors], dtype=torch.int64, device=tensors[0].device)
-            self.key = key
+                sources = tensors[:used]
+                tensors = copies = [_to_bf16(t.detach()) for t in sources]
+            table = torch.tensor([t.data_ptr() for t in tensors], dtype=torch.int64, device=tensors[0].device)
+            # all of it or nothing: a conversion that fails leaves the copies behind the old key and table alive
+            self.sources, self.copies, self.table, self.key = sources, copies, table, key
         return self.table
 
 
