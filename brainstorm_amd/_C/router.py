@@ -649,7 +649,7 @@ def combine_by_rows(in_data: torch.Tensor, path_ids: torch.Tensor, seat_rows: to
     (router.cc:372-473) for the same route, bit for bit.  With ``out_data`` the result is
     written in place and cells without a row keep their value (the residual convention).
     ``gates`` (the ``[cells, paths]`` matrix, any data type) gives the weights instead:
-    ``gates[t, path_ids[t,j]]``."""
+    ``gates[t, path_ids[t,j]]``; it has a column for every path id (the ids are not read back to check it)."""
     if gates is not None and weights is not None:
         raise RuntimeError("weights or gates, not both")
     if gates is not None and not (gates.dtype in _DT and gates.dim() == 2 and gates.size(0) == path_ids.size(0)

@@ -578,6 +578,8 @@ class FusedCombineFabric(CombineFabric):
                 return c_router.combine_by_row_tags(data, route.row_entries, route.cells, residual)
             return c_router.combine_by_row_tags(data, route.row_entries, route.cells)
         # weighted: every entry by the score of its cell on its path
+        if gates is not None and gates.dim() == 2 and gates.size(1) < route.paths:
+            raise RuntimeError(f"the score has {gates.size(1)} columns for {route.paths} paths")
         return c_router.combine_by_rows(data, route.path_ids, route.seat_rows, None, residual, gates=gates)
 
     def _combine_deferred(self, data, route, state, gates, residual):

@@ -446,7 +446,8 @@ int brt_hip_combine_by_rows(const void* src, void* dst, const float* weights,
                             int cell, int P, int is_residual, int in_dtype, int out_dtype,
                             void* stream);
 /* The same with the weights taken from the [T,E] gate matrix (gate_dtype): the weight of entry (t, j)
- * is gates[t, path_ids[t, j]], widened to fp32. */
+ * is gates[t, path_ids[t, j]], widened to fp32.  Every path id has to be below E: one that is not would be
+ * weighted by the nearest column (nothing outside the matrix is read). */
 int brt_hip_combine_by_rows_gated(const void* src, void* dst, const void* gates, int gate_dtype, int E,
                                   const int32_t* path_ids, const int32_t* seat_rows, int T, int k, int cell,
                                   int P, int is_residual, int in_dtype, int out_dtype, void* stream);
