@@ -190,6 +190,7 @@ PyObject* throttle_hotmask(const Args& a) {  // hot_mask, prefix (updated in pla
   const Tensor given = a.tensor(0), prefix = a.tensor(1), threshold = a.tensor(2);
   on_device(given, "hot_mask"), on_device(prefix, "prefix"), on_device(threshold, "threshold");
   int32(given, "hot_mask"), int32(prefix, "prefix"), int32(threshold, "threshold");
+  if (given.dim() != 2) throw Raised(PyExc_ValueError, "hot_mask must be [cells, paths]");
   if (given.size(1) != prefix.size(0) || given.size(1) != threshold.size(0))
     runtime_error("prefix/threshold must have one entry per path");
   const Tensor mask = dense(given);

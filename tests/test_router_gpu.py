@@ -1049,3 +1049,13 @@ def test_combine_by_rows_takes_its_weights_from_the_gate_matrix(brt_mod, T, E, d
         assert torch.equal(c_router.combine_by_rows(y, ids, seat_rows, None, residual, gates=gates), want)
     with pytest.raises(RuntimeError):
         c_router.combine_by_rows(y, ids, seat_rows, weights, gates=gates)
+
+
+@pytest.mark.parametrize("shape", [(6,), (6, 4, 2), (2, 3, 4, 1)])
+def test_throttle_refuses_masks_that_are_not_cells_by_paths(brt_mod, shape):
+    c_router = brt_mod[1]
+    mask = torch.ones(shape, dtype=torch.int32, device="cuda")
+    paths = shape[1] if len(shape) > 1 else 1
+    with pytest.raises((ValueError, IndexError)):
+        c_router.throttle_hotmask(mask, torch.zeros(paths, dtype=torch.int32, device="cuda"),
+                                  torch.full((paths,), 2, dtype=torch.int32, device="cuda"))
