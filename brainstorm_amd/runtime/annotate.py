@@ -23,7 +23,7 @@ class Annotator(nn.Module):
 
     def forward(self, t: torch.Tensor):
         if type(t) is torch.Tensor and self.gridding and self.cell_shape is None and self.dims == [0] and t.is_contiguous() \
-                and t.dim() > 0:
+                and t.dim() > 0 and t.numel() > 0:
             return init_grid_tensor(t, [None], [None])  # the cells are the rows as they are
         assert self.dims[-1] < t.dim()
         rest = [d for d in range(t.dim()) if d not in self.dims]

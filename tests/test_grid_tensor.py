@@ -212,3 +212,15 @@ def test_deferred_buffer_fills_itself_before_any_read_and_not_for_metadata():
     other = torch.ones(6, 3)
     assert deferred.pending_state(grid.extra_attr_dict, other) is None  # another tensor is not the buffer
     assert deferred.wrap_if_pending(other, grid.extra_attr_dict) is other and state.fills == 0
+
+
+@pytest.mark.parametrize("shape", [(5, 0), (0, 0), (3, 0, 2)])
+def test_annotator_refuses_cells_of_no_elements(shape):
+    """Their number cannot be told from the number of elements."""
+    with pytest.raises(RuntimeError, match="ambiguous"):
+        brt.Annotator([0])(torch.zeros(shape))
+
+
+def test_annotator_takes_no_cells():
+    cells = brt.Annotator([0])(torch.zeros(0, 7))
+    assert tuple(cells.shape) == (0, 7) and cells.tag_stack == [None]
