@@ -586,7 +586,10 @@ at::DataPtr read_back(const Tensor& t, size_t bytes, const char* what) {
     rc = hipStreamSynchronize(st);
     Py_END_ALLOW_THREADS
   }
-  if (rc != hipSuccess) runtime_error(std::string(what) + ": " + hipGetErrorString(rc));
+  if (rc != hipSuccess) {
+    (void)hipGetLastError();  // reported here, not by the next launch that looks for an error
+    runtime_error(std::string(what) + ": " + hipGetErrorString(rc));
+  }
   return host;
 }
 

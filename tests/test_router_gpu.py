@@ -1059,3 +1059,31 @@ def test_throttle_refuses_masks_that_are_not_cells_by_paths(brt_mod, shape):
     with pytest.raises((ValueError, IndexError)):
         c_router.throttle_hotmask(mask, torch.zeros(paths, dtype=torch.int32, device="cuda"),
                                   torch.full((paths,), 2, dtype=torch.int32, device="cuda"))
+
+
+def test_a_read_back_that_is_refused_leaves_no_error_behind():
+    """Waiting for the loads is not possible while the stream is captured.  The error is raised where it happens;
+    the next call that asks the runtime for an error must not find it again."""
+    import ctypes
+
+    from brainstorm_amd import _lib
+
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    loads = torch.tensor([3, 1, 2], dtype=torch.int32, device="cuda")
+    assert _lib.native().int_list(loads) == [3, 1, 2]  # the pinned buffer is there before the capture
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        relaxed = 2  # hipStreamCaptureModeRelaxed
+        assert hip.hipStreamBeginCapture(ctypes.c_void_p(side.cuda_stream), relaxed) == 0
+        with pytest.raises(RuntimeError, match="reading the loads"):
+            _lib.native().int_list(loads)
+        left = hip.hipPeekAtLastError()
+        graph = ctypes.c_void_p()
+        hip.hipStreamEndCapture(ctypes.c_void_p(side.cuda_stream), ctypes.byref(graph))
+        hip.hipGetLastError()  # the capture is invalid and says so
+        if graph.value:
+            hip.hipGraphDestroy(graph)
+    assert left == 0
+    assert _lib.native().int_list(loads) == [3, 1, 2]
