@@ -354,7 +354,8 @@ PyObject* combine(const Args& a) {
     const Tensor tags = a.tensor(7);
     check(brt_hip_combine_by_tags(ptr(in), ptr(out), iptr(tags), P, cell, T, in_type, out_type, stream_of(in)));
   } else {
-    const Tensor loads = dense(given_loads.device() == in.device() ? given_loads : given_loads.to(in.device()));
+    const Tensor loads =
+        dense(given_loads.device() == in.device() ? given_loads : given_loads.to(in.options().dtype(at::kInt), /*non_blocking=*/true));
     check(brt_hip_combine(ptr(in), ptr(out), ptr(gates), iptr(route), iptr(loads), T, cell, E, P, mpl, residual.defined(),
                           in_type, out_type, gates.defined() ? code_of(gates.scalar_type()) : BRT_F32, stream_of(in)));
   }

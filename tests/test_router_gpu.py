@@ -1087,3 +1087,20 @@ def test_a_read_back_that_is_refused_leaves_no_error_behind():
             hip.hipGraphDestroy(graph)
     assert left == 0
     assert _lib.native().int_list(loads) == [3, 1, 2]
+
+
+def test_combine_does_not_wait_for_the_device_to_bring_host_loads_over(brt_mod):
+    c_router = brt_mod[1]
+    mask = torch.eye(8, 4, dtype=torch.int32).cuda()
+    mask[4:, 1] = 1
+    x = torch.randn(8, 16).cuda()
+    indices, loads = c_router.generate_indices_and_loads(mask)
+    (y,) = c_router.dispatch_with_indices_and_loads(x, indices, loads)
+    (want,) = c_router.combine_with_indices_and_loads(y, indices, loads)
+    host_loads = loads.cpu()
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        (got,) = c_router.combine_with_indices_and_loads(y, indices, host_loads)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    assert torch.equal(got, want)
