@@ -185,7 +185,7 @@ def topk_hot_mask(score: torch.Tensor, top_k: int) -> torch.Tensor:
     (protocol/topk.py:26-31: ``topk`` + ``zeros_like`` + ``scatter_``) in one kernel.  int32
     ``[cells, paths]`` with ones at the ``top_k`` largest scores of every row; NaN ranks
     highest, equal scores go to the lowest path."""
-    return _lib.native().topk_hot_mask(score, top_k)
+    return _lib.native().topk_hot_mask(score, int(top_k))
 
 
 def throttle_hotmask(
@@ -627,8 +627,8 @@ def route_by_path(
     ``path_num * max_path_load`` when padding every path to ``max_path_load``, else by default
     ``cells * k``, which always holds the ``sum(loads)`` rows of a route without capacity padding
     (no read-back of the loads is needed to size it; rows behind the last path are padding)."""
-    return _lib.native().route_by_path(path_ids, path_num, supported_capacities, capacity_padding,
-                                       path_wise_padding, max_path_load, rows)
+    return _lib.native().route_by_path(path_ids, int(path_num), supported_capacities, capacity_padding,
+                                       path_wise_padding, int(max_path_load), rows)
 
 
 def dispatch_by_rows(in_data: torch.Tensor, row_entries: torch.Tensor, k: int,
@@ -637,7 +637,7 @@ def dispatch_by_rows(in_data: torch.Tensor, row_entries: torch.Tensor, k: int,
     """``out[r] = in_data[(row_entries[r]-1) // k]`` (times ``weights.view(-1)[row_entries[r]-1]``,
     rounded once), zero rows where ``row_entries[r] == 0``: what ``dispatch_with_indices_and_loads``
     (router.cc:131-273) writes for the same route, every row written by the kernel."""
-    return _lib.native().dispatch_by_rows(in_data, row_entries, k, weights, out)
+    return _lib.native().dispatch_by_rows(in_data, row_entries, int(k), weights, out)
 
 
 def combine_by_rows(in_data: torch.Tensor, path_ids: torch.Tensor, seat_rows: torch.Tensor,

@@ -63,7 +63,7 @@ def grouped_linear(x: torch.Tensor, out: torch.Tensor, weight_table: torch.Tenso
     paths per cell, to the last bits of an fp32 sum taken in another order with more."""
     _lib.native().grouped_linear(
         x, out, weight_table, bias_table, loads, in_features, out_features, _ACT[activation], tags, gather,
-        scatter, rows, row_entries, entries_per_cell, row_tags_out, gates)
+        scatter, rows, row_entries, int(entries_per_cell), row_tags_out, gates)
     return out
 
 

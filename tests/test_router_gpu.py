@@ -1104,3 +1104,16 @@ def test_combine_does_not_wait_for_the_device_to_bring_host_loads_over(brt_mod):
     finally:
         torch.cuda.set_sync_debug_mode("default")
     assert torch.equal(got, want)
+
+
+def test_counts_given_as_whole_floats_are_taken(brt_mod):
+    """Numbers that come out of a division of sizes: what int() makes of them."""
+    c_router = brt_mod[1]
+    score = torch.randn(40, 4, generator=torch.Generator().manual_seed(3)).cuda()
+    assert torch.equal(c_router.topk_hot_mask(score, 2.0), c_router.topk_hot_mask(score, 2))
+    ids, _ = c_router.gate_topk(score, 2)
+    want = c_router.route_by_path(ids, 4, max_path_load=32)
+    got = c_router.route_by_path(ids, 4.0, max_path_load=32.0)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    x = torch.randn(40, 16).cuda()
+    assert torch.equal(c_router.dispatch_by_rows(x, want[3], 2.0), c_router.dispatch_by_rows(x, want[3], 2))
