@@ -519,8 +519,7 @@ def test_experts_with_many_row_blocks_in_patch_order(loads, K, N):
     ([2000, 1700, 300, 1900, 1, 1800, 2047, 1500], 128, 1000),  # one round, ragged, N tail
     # last row blocks of every number of 32-row tiles, shared by the two groups of wavefronts
     ([768 + r for r in (1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 255)], 192, 2048),
-    # the last round's whole tiles cut in four (528 tiles and 16 light ones), in two (592 and 16, parts past the
-    # expert's rows among them), with more than 128 experts
+    # 528 whole tiles and 16 light ones, 592 and 16, more than 128 experts
     ([5000, 3328, 100], 128, 4096),
     ([100, 5000, 4300], 128, 4096),
     ([0] * 100 + [5000, 100] + [0] * 64 + [130, 26000, 0], 128, 1024),
@@ -541,7 +540,7 @@ def test_ping_pong_tiles(loads, K, N):
     (12000, 8, 192, 4104, 1, 1700, True),    # padded to the capacity: empty slots, odd K-steps, N tail
     (13000, 5, 1024, 1000, 1, 4000, False),  # one round of tiles, N tail
     (7000, 6, 256, 4096, 2, 2400, False),    # two entries per cell (gather only)
-    (8800, 2, 128, 4096, 1, 8000, False),    # tiles cut in four, light tiles last
+    (8800, 2, 128, 4096, 1, 8000, False),    # two experts, one round of tiles and 32 over
 ])
 def test_ping_pong_tiles_with_routing_and_fp32_output(T, E, K, N, k, cap, pad):
     """The routed and fp32-output forms on shapes the 256 x 256 ping-pong kernel takes: the same bits
@@ -684,6 +683,110 @@ def test_bits_of_a_row_do_not_depend_on_the_rows_of_the_launch(loads, K, N, boun
     for kernel, got in results.items():
         for form, a, b in zip(("bf16", "fp32", "gathered", "scattered"), first, got):
             assert torch.equal(a, b), (kernel, form)
+
+
+def _few_rows_tile(P, E, K, N):
+    """Tile of the few-rows kernel for these sizes: rows x columns, stages."""
+    used = min(E, P)
+    rows = P / used
+
+    def tiles(block):
+        return used * (rows / block + 0.5 if rows > block else 1.0) * -(-N // 64)
+
+    if rows > 32 and tiles(64) >= 192:
+        return (64, 64, 3) if K <= 1024 else (64, 64, 4)
+    if tiles(32) <= 112 or (tiles(32) <= 160 and K <= 2048) or (rows <= 16 and K <= 1536):
+        return (32, 32, 6)
+    return (32, 64, 5)
+
+
+@pytest.mark.parametrize("T,E,K,N,cap,pad,kernel", [
+    (9000, 40, 136, 264, 230, False, "160 rows"),          # several row blocks per expert, K and N tails, overflow dropped
+    (2000, 64, 72, 776, 40, False, "160 rows"),            # part of one row block per expert
+    (100, 34, 136, 264, 256, True, "160 rows"),            # loads name slots past the tag matrix, most rows are padding
+    (4000, 80, 192, 520, 50, True, "160 rows"),            # whole K-steps, padded to the capacity
+    (100, 8, 136, 72, 14, False, (32, 32, 6)),
+    (150, 130, 840, 136, 2, False, (32, 32, 6)),           # more than 64 experts, fourteen K-steps on six stages
+    (600, 20, 200, 776, 33, False, (32, 64, 5)),
+    (600, 20, 456, 776, 32, True, (32, 64, 5)),            # eight K-steps on five stages
+    (1000, 20, 136, 776, 55, False, (64, 64, 3)),          # blocks of 64 rows and their remainders
+    (1000, 20, 328, 776, 70, True, (64, 64, 3)),
+    (1000, 20, 1096, 776, 60, True, (64, 64, 4)),
+    (50, 20, 1224, 1032, 60, True, (64, 64, 4)),           # loads name slots past the tag matrix
+])
+def test_every_form_of_the_row_streaming_kernels(T, E, K, N, cap, pad, kernel):
+    """The 160-row kernel and every tile of the few-rows kernel: the plain form against torch, and the bits of its
+    rows from the fp32-output, gathering (tag matrix, row entries, with the row tags as a side output), scattering
+    and accumulating forms, in a layout longer than the loads."""
+    from brainstorm_amd._C import router as c_router
+    from brainstorm_amd.jit import grouped_linear
+    from routing_cases import topk_mask
+
+    rows = E * cap if pad else T  # a bound
+    want_kernel = kernel if isinstance(kernel, str) else "few rows"
+    assert _kernel_for(rows, E, K, N) == want_kernel
+    if want_kernel == "few rows":
+        assert _few_rows_tile(rows, E, K, N) == kernel
+    mask, _ = topk_mask(T, E, 1, seed=T + K)
+    caps = torch.tensor([cap], dtype=torch.int32, device="cuda")
+    d_mask = torch.from_numpy(mask).cuda()
+    ids = torch.from_numpy(mask.argmax(1).astype(np.int32)).cuda().view(T, 1)
+    loads, _, _, entries = c_router.route_by_path(ids, E, caps, pad, rows=rows)
+    tags, loads_t = c_router.generate_indices_and_loads(d_mask, caps, pad, False, True)
+    assert torch.equal(loads, loads_t)
+    P = int(loads.sum())
+    assert int((entries > 0).sum()) < rows, "nothing dropped and nothing padded"
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn(T, K, generator=g).to(torch.bfloat16).cuda()
+    ws, table = _expert_tables(E, K, N, 6)
+    bias = torch.randn(E, N, generator=g).to(torch.bfloat16).cuda()
+    bias_table = torch.tensor([b.data_ptr() for b in bias], dtype=torch.int64, device="cuda")
+    y = c_router.dispatch_by_rows(x, entries, 1)
+    live = entries[:P].long()
+    kept = live > 0
+
+    def launch(src, out, **kwargs):
+        grouped_linear(src, out, table, bias_table, loads, K, N, "gelu", rows=rows, **kwargs)
+        return out
+
+    def empty(n, dtype=torch.bfloat16, fill=float("nan")):
+        return torch.full((n, N), fill, dtype=dtype, device="cuda")
+
+    plain = empty(rows)
+    launch(y, plain)
+    want = reference(y[:P], ws, list(bias), loads.cpu().tolist(), "gelu")
+    assert (plain[:P].float() - want).abs().max() < 1e-2 * want.abs().max()
+    assert torch.isnan(plain[P:].float()).all()
+    wide = launch(y, empty(rows, torch.float32))
+    assert torch.equal(wide[:P].to(torch.bfloat16).float(), plain[:P].float()) and torch.isnan(wide[P:]).all()
+
+    def same_rows(got, rows_of):
+        assert torch.equal(got[:P], rows_of[:P]) and torch.isnan(got[P:].float()).all()
+
+    for dtype, rows_of in ((torch.bfloat16, plain), (torch.float32, wide)):
+        row_tags = torch.full((rows,), -7, dtype=torch.int32, device="cuda")
+        same_rows(launch(x, empty(rows, dtype), tags=tags, gather=True, row_tags_out=row_tags), rows_of)
+        assert torch.equal(row_tags, entries)  # one entry per cell: the entries are the tags
+        cells = empty(T, dtype, 3.0)
+        cells[live[kept] - 1] = rows_of[:P][kept] + 0.0
+        row_tags.fill_(-7)
+        assert torch.equal(launch(y, empty(T, dtype, 3.0), tags=tags, scatter=True, row_tags_out=row_tags), cells)
+        assert torch.equal(row_tags, entries)
+        if dtype == torch.bfloat16:  # the row entries (bf16 only)
+            same_rows(launch(x, empty(rows), row_entries=entries, gather=True), rows_of)
+            assert torch.equal(launch(y, empty(T, dtype, 3.0), row_entries=entries, scatter=True), cells)
+            assert torch.equal(launch(x, empty(T, dtype, 3.0), row_entries=entries, gather=True, scatter=True), cells)
+    # accumulating form: one addend per cell, its product rounded once
+    for by_rows in (False, True):
+        gates = torch.rand(T, 1 if by_rows else E, generator=g).cuda()
+        weight = gates.view(-1) if by_rows else gates.gather(1, ids.long()).view(-1)
+        sums = torch.zeros(T, N, device="cuda")
+        sums[live[kept] - 1] = plain[:P][kept].float() * weight[live[kept] - 1, None]
+        where = {"row_entries": entries} if by_rows else {"tags": tags}
+        got = launch(y, torch.zeros(T, N, device="cuda"), scatter=True, gates=gates.view(-1) if by_rows else gates, **where)
+        assert torch.equal(got, sums)
+        got = launch(x, torch.zeros(T, N, device="cuda"), gather=True, scatter=True, gates=gates.view(-1) if by_rows else gates, **where)
+        assert torch.equal(got, sums)
 
 
 def test_grouped_gemm_random_shapes():
