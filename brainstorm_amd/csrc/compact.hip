@@ -595,8 +595,11 @@ extern "C" int brt_hip_route_by_path(const int32_t* path_ids, int T, int k, int 
     hipLaunchKernelGGL((route_kernel<kWhole, kWholeWaves>), dim3(1), dim3(kWholeWaves * kWave), lds_bytes, st, a);
     return check_launch("route_kernel");
   }
-  if (n <= (E > kManyPaths ? kSoloEntriesManyPaths : kSoloEntries)) {
-    // one launch: each wavefront owns a whole number of chunks
+  const size_t need = brt_hip_route_by_path_workspace_bytes(T, k, E);
+  const bool room = workspace != nullptr && workspace_bytes >= need && aligned(workspace, 4);
+  if (n <= (E > kManyPaths || !room ? kSoloEntriesManyPaths : kSoloEntries)) {
+    // one launch: each wavefront owns a whole number of chunks.  (Routes of up to 65536 entries were always
+    // taken without a workspace, and still are.)
     auto solo = [&](auto waves) {
       constexpr int kWaves = decltype(waves)::value;
       const int groups = std::min(kSplitGroups, (chunks + kWaves - 1) / kWaves);
@@ -611,8 +614,7 @@ extern "C" int brt_hip_route_by_path(const int32_t* path_ids, int T, int k, int 
   }
   int waves;
   split_geometry(n, &waves, &a.units, &a.per_wave);
-  const size_t need = static_cast<size_t>(a.units / waves + a.units) * E * sizeof(int);
-  if (workspace == nullptr || workspace_bytes < need || !aligned(workspace, 4))
+  if (!room)
     return fail(BRT_E_WORKSPACE, "route_by_path needs %zu bytes of workspace, got %zu", need, workspace_bytes);
   a.ws = static_cast<int*>(workspace);
   const dim3 grid(a.units / waves), block(waves * kWave);

@@ -414,10 +414,11 @@ int brt_hip_combine_by_index(const void* in_data, void* out_data, const void* in
  *   order; entry (t,j) of path e with seat s <= loads[e] owns row start[e] + s, start[e] = sum
  *   of the loads before e, or e * max_path_load when max_path_load != 0 (seats beyond
  *   max_path_load are dropped then).  Rows beyond P are dropped; row_entries is written whole
- *   ([0,P)), it needs no zero fill.  E <= 512.  Routes of up to 2048 entries take one launch of
- *   one workgroup; larger ones two launches that pass per-wavefront counters through the
+ *   ([0,P)), it needs no zero fill.  E <= 512.  Routes of up to 32768 entries (65536 with more than 128
+ *   paths) take one launch; larger ones two launches that pass per-wavefront counters through the
  *   workspace (size from brt_hip_route_by_path_workspace_bytes, 4-byte aligned, uninitialised,
- *   not shared between calls that run at the same time).
+ *   not shared between calls that run at the same time).  Without a workspace of that size one launch
+ *   takes up to 65536 entries; more are refused.
  *
  * brt_hip_dispatch_by_rows: dst[r] = src[(row_entries[r]-1) / k] (times weights[row_entries[r]-1]
  *   when weights != NULL: an fp32 product, then rounded to the data type), zero rows where

@@ -281,7 +281,7 @@ def gate_topk(score_bits, k, dtype="f32", softmax=False, want_mask=False):
 
 
 def route_by_path(path_ids, E, caps=None, capacity_padding=False, path_wise_padding=False,
-                  max_path_load=0, P=None):
+                  max_path_load=0, P=None, workspace=True):
     """-> (loads, counts, seat_rows, row_entries)."""
     ids = np.ascontiguousarray(path_ids, dtype=np.int32)
     T, k = ids.shape
@@ -298,7 +298,7 @@ def route_by_path(path_ids, E, caps=None, capacity_padding=False, path_wise_padd
     _lib.check(_lib.lib().brt_hip_route_by_path(
         ptr(d_ids), T, k, E, ptr(d_caps), 0 if caps is None else len(caps), int(capacity_padding),
         int(path_wise_padding), int(max_path_load), ptr(d_loads), ptr(d_counts), ptr(d_rows),
-        ptr(d_entries), P, ptr(ws), need, stream()))
+        ptr(d_entries), P, ptr(ws) if workspace else None, need if workspace else 0, stream()))
     torch.cuda.synchronize()
     return host(d_loads), host(d_counts), host(d_rows), host(d_entries)
 

@@ -788,6 +788,21 @@ def test_route_by_path_at_the_edges_of_its_forms(hip, n, E, ids_of):
         assert np.array_equal(g, w), name
 
 
+@pytest.mark.parametrize("n,E", [(2048, 16), (32768, 16), (32769, 16), (40001, 128), (65536, 64), (65536, 300)])
+def test_route_by_path_without_a_workspace(hip, n, E):
+    """Up to 65536 entries are routed in one launch where the caller brings no workspace."""
+    ids = np.random.default_rng(n + E).integers(0, E, (n, 1)).astype(np.int32)
+    want = oracle.route_by_path(ids, E, [n // 2], False, False, 0, n)
+    got = hip.route_by_path(ids, E, [n // 2], False, False, 0, n, workspace=False)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+
+
+def test_route_by_path_refuses_more_entries_without_a_workspace(hip):
+    with pytest.raises(RuntimeError, match="bytes of workspace"):
+        hip.route_by_path(np.zeros((65537, 1), dtype=np.int32), 16, [4], False, False, 0, 65537, workspace=False)
+
+
 def test_route_by_path_path_wise_padding_and_bad_arguments(hip):
     ids = _compact_route(500, 8, 2, seed=1)
     ids[ids == 3] = -1                                        # nobody takes path 3
