@@ -27,14 +27,13 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWholeWaves = 8;    // a small route: one workgroup of 8 wavefronts, one launch
 constexpr int kWholeChunks = 32;  // ... up to this many chunks of 64 entries
-constexpr int kSplitWaves = 4;    // larger routes: workgroups of 4 wavefronts, two launches
-constexpr int kSplitGroups = 32;  // ... in at most this many workgroups
+constexpr int kSplitGroups = 32;  // larger routes: at most this many workgroups, in one launch or two
 // Routes up to this many entries: one launch, every workgroup counts the whole route.  Against two
 // launches: 32768 entries 8.2 / 8.9 us against 8.0 / 8.4 us on the device (16 paths / 32 skewed ones), but one
 // launch less for the host; 65536 entries 13.1 / 14.3 us against 10.1 / 10.7 us (8 / 64 paths).  With more than
 // 128 paths the two launches hand over more counters: 65536 entries, 256 paths 16.5 us against 21.0 us.
 constexpr int kSoloEntries = 32768, kSoloEntriesManyPaths = 65536, kManyPaths = 128;
-constexpr int kSplitWavesLarge = 16;  // ... of 16 wavefronts for routes beyond 32768 entries
+constexpr int kSplitWaves = 16;   // two launches: workgroups of 16 wavefronts
 constexpr int kBatch = 4;        // chunks of 64 entries a wavefront keeps in flight
 constexpr int kMaxK = 8;         // paths per cell in combine_by_rows
 constexpr int kMaxRoutePaths = 512;  // (2 * kWholeWaves + 3) * E words of LDS
@@ -148,7 +147,7 @@ __device__ __forceinline__ void sum_rows(Ptr cnt, int rows, int mine, int E, int
   }
 }
 
-// kWhole: one workgroup computes the route (small routes: one launch).  kCount + kEmit: the
+// kWhole: one workgroup computes the route (small routes: one launch).  kCount + kEmit (the largest): the
 // same work spread over up to kSplitGroups workgroups in two launches; a unit is a wavefront and
 // its contiguous range of entries.  The counters travel through `ws`: [groups][E] sums per
 // workgroup, then [units][E] per unit, so that a unit finds its first seats with one round of
@@ -537,16 +536,13 @@ using namespace brt;
 
 namespace {
 
-// Wavefronts per workgroup, units and entries per unit of the two-launch form: at most
-// kSplitGroups workgroups, of 4 wavefronts while that keeps a unit within one batch of chunks, of
-// 16 beyond.
-void split_geometry(int n, int* waves, int* units, int* per_wave) {
+// Units and entries per unit of the two-launch form: at most kSplitGroups workgroups.
+void split_geometry(int n, int* units, int* per_wave) {
   const int chunks = (n + kWave - 1) / kWave;
-  *waves = chunks <= kSplitGroups * kSplitWaves * kBatch ? kSplitWaves : kSplitWavesLarge;
-  const int most = kSplitGroups * *waves;
+  const int most = kSplitGroups * kSplitWaves;
   const int chunks_pw = std::max(1, (chunks + most - 1) / most);
   const int used = (chunks + chunks_pw - 1) / chunks_pw;
-  *units = (used + *waves - 1) / *waves * *waves;
+  *units = (used + kSplitWaves - 1) / kSplitWaves * kSplitWaves;
   *per_wave = chunks_pw * kWave;
 }
 
@@ -554,9 +550,9 @@ void split_geometry(int n, int* waves, int* units, int* per_wave) {
 
 extern "C" size_t brt_hip_route_by_path_workspace_bytes(int T, int k, int E) {
   if (T <= 0 || k <= 0 || E <= 0 || static_cast<long>(T) * k >= (1l << 31)) return 0;
-  int waves, units, per_wave;
-  split_geometry(T * k, &waves, &units, &per_wave);
-  return static_cast<size_t>(units / waves + units) * E * sizeof(int);
+  int units, per_wave;
+  split_geometry(T * k, &units, &per_wave);
+  return static_cast<size_t>(units / kSplitWaves + units) * E * sizeof(int);
 }
 
 extern "C" int brt_hip_route_by_path(const int32_t* path_ids, int T, int k, int E, const int32_t* caps,
@@ -612,20 +608,14 @@ extern "C" int brt_hip_route_by_path(const int32_t* path_ids, int T, int k, int 
     if (n > 8192 && E <= 256) return solo(std::integral_constant<int, 8>{});
     return solo(std::integral_constant<int, 4>{});
   }
-  int waves;
-  split_geometry(n, &waves, &a.units, &a.per_wave);
+  split_geometry(n, &a.units, &a.per_wave);
   if (!room)
     return fail(BRT_E_WORKSPACE, "route_by_path needs %zu bytes of workspace, got %zu", need, workspace_bytes);
   a.ws = static_cast<int*>(workspace);
-  const dim3 grid(a.units / waves), block(waves * kWave);
-  const size_t lds_bytes = (static_cast<size_t>(waves + 3) * E + a.caps_in_lds) * sizeof(int);
-  if (waves == kSplitWaves) {
-    hipLaunchKernelGGL((route_kernel<kCount, kSplitWaves>), grid, block, lds_bytes, st, a);
-    hipLaunchKernelGGL((route_kernel<kEmit, kSplitWaves>), grid, block, lds_bytes, st, a);
-  } else {
-    hipLaunchKernelGGL((route_kernel<kCount, kSplitWavesLarge>), grid, block, lds_bytes, st, a);
-    hipLaunchKernelGGL((route_kernel<kEmit, kSplitWavesLarge>), grid, block, lds_bytes, st, a);
-  }
+  const dim3 grid(a.units / kSplitWaves), block(kSplitWaves * kWave);
+  const size_t lds_bytes = (static_cast<size_t>(kSplitWaves + 3) * E + a.caps_in_lds) * sizeof(int);
+  hipLaunchKernelGGL((route_kernel<kCount, kSplitWaves>), grid, block, lds_bytes, st, a);
+  hipLaunchKernelGGL((route_kernel<kEmit, kSplitWaves>), grid, block, lds_bytes, st, a);
   return check_launch("route_kernel");
 }
 

@@ -203,10 +203,9 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // A load fills one row group: 8 tile rows, a whole 128-byte line of each.  Group 0 loads the
   // activation rows, wavefront wn taking row groups wn + 4 i (i = 0..7); group 1 the weight rows,
   // wavefront wn taking the 64 rows of its own columns, row groups 8 wn + i.  Lane l lands at slot
-  // l & 7 of row l >> 3 of the group and fetches chunk (l & 7) ^ ((row >> 1) & 7) of that row.  The
-  // lane's row inside the group and its chunk are the vector offset; the row group and the K-step
-  // go into the scalar offset, so no per-load register stays live.  A row that does not exist
-  // (past the expert's last row, past N) gets an offset past any extent: zeros, no memory request.
+  // l & 7 of row l >> 3 of the group and fetches chunk (l & 7) ^ ((row >> 1) & 7) of that row.  A row
+  // that does not exist (past the expert's last row, past N) gets an offset past any extent: zeros,
+  // no memory request.
   const __bf16* const w_e = a.w[e];
   // Every wavefront keeps the eight offsets of its rows in registers (the K-step alone goes into
   // the scalar offset).  Gathered rows need that -- the cells of a row group are anywhere in x --
@@ -250,7 +249,8 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // The row tiles that hold rows are shared evenly by the two groups, group 0 taking the first `half`
   // rows: with 128 rows or fewer in one group the phases of a K-step would run one after the other.
   // (Halves fixed at 128 rows: the ragged FFN of 128 experts, 108 of its 201 row blocks part-filled,
-  // 2556 -> 2532 us; top-2 over 16384 cells of 32 skewed experts 390 -> 387 us.)
+  // 2556 -> 2532 us; top-2 over 16384 cells of 32 skewed experts 390 -> 387 us; two runs of one side
+  // differ by half of that.)
   const int half = __builtin_amdgcn_readfirstlane(((rows + 63) >> 6) << 5);
   const int first_row = wm * half;  // of this wavefront, inside the tile
   const int frag_x = (first_row + frag_row) * kRowB;

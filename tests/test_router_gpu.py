@@ -941,6 +941,45 @@ def test_task_hash_and_label_protocols_route_on_the_gpu(brt_mod):
     assert np.array_equal(brt.to_torch_tensor(out).cpu().numpy(), x.cpu().numpy() * 2)
 
 
+def test_forms_of_a_layer_are_bit_identical_where_they_take_different_kernels(brt_mod):
+    """64 experts, 2000 cells of which 1700 find room: the expanding GEMM of the drop-in form is sized by the kept
+    rows (at most 28 per expert: the few-rows kernel), that of the other forms by a bound of them (the 160-row kernel)."""
+    brt, _, ScatterRouter, GatherRouter = brt_mod
+    from brt.jit import make_jit_kernel
+
+    T, E, d, dff, cap = 2000, 64, 328, 520, 29
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    x = torch.randn(T, d, device="cuda", generator=gen).to(torch.bfloat16)
+    score = torch.randn(T, E, device="cuda", generator=gen)
+    torch.manual_seed(12)
+    wi = nn.ModuleList(nn.Linear(d, dff) for _ in range(E)).cuda().to(torch.bfloat16)
+    wo = nn.ModuleList(nn.Linear(dff, d, bias=False) for _ in range(E)).cuda().to(torch.bfloat16)
+    fused_wi = make_jit_kernel(wi, None, opt_level="homo_fuse", activation="gelu")
+    fused_wo = make_jit_kernel(wo, None, opt_level="homo_fuse")
+    wi_operands = [p for m in wi for p in (m.weight, m.bias)]
+
+    def layer(kwargs):
+        scatter = ScatterRouter(protocol_type="topk", fabric_type="fused_dispatch",
+                                fabric_kwargs={"supported_capacities": [cap], **kwargs}).cuda()
+        gather = GatherRouter(fabric_type="fused_combine").cuda()
+        states, tags, loads, extra = brt.to_torch_tensor(scatter(brt.Annotator([0])(x), score), retrieve_attr=True)
+        rows = states.shape[0]
+        h = torch.empty((rows, dff), device="cuda", dtype=torch.bfloat16)
+        fused_wi(shared_inputs=[states, h], standalone_inputs=wi_operands, capacities=loads[-1])
+        y = torch.empty((rows, d), device="cuda", dtype=torch.bfloat16)
+        fused_wo(shared_inputs=[h, y], standalone_inputs=[m.weight for m in wo], capacities=loads[-1])
+        kept = int(loads[-1].sum())
+        return rows, h[:kept], brt.to_torch_tensor(gather(brt.to_grid_tensor(y, tags, loads, extra), x.clone()))
+
+    rows, h, out = layer({})
+    assert rows == h.shape[0] <= 28 * E
+    for kwargs in ({"static_rows": True}, {"defer_dispatch": True}, {"compact_route": True},
+                   {"compact_route": True, "defer_dispatch": True}):
+        bound, got_h, got = layer(kwargs)
+        assert bound > 28 * E, kwargs
+        assert torch.equal(got_h, h) and torch.equal(got, out), kwargs
+
+
 @pytest.mark.parametrize("fabric_kwargs", [{"defer_dispatch": True}, {"static_rows": True}])
 def test_deferred_and_static_rows_layers_replay_from_a_hip_graph(brt_mod, fabric_kwargs):
     """Neither form reads the loads back, so the layer (router objects and jit kernels, written as
