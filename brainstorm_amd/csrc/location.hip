@@ -32,6 +32,14 @@
 // (from cache).  The indices are written exactly once.  Masks small enough for one workgroup of
 // eight wavefronts to hold in registers skip pass 1: that workgroup is the only band, and its
 // wavefronts' column sums meet in LDS (one launch).
+//
+// Index generation from masks of up to 256 KB is one launch too: every workgroup adds up all the rows
+// above its own by itself.  That reads the mask several times, from the caches, in the round trip in
+// which two launches read the bands' sums, and takes no kernel boundary: bound by its three dependent
+// round trips (rows, result, launch), not by bytes.  Seats, back to back in a graph: 1024 x 16 6.1 -> 4.1 us,
+// 1024 x 64 5.8 -> 4.6, 4096 x 16 6.2 -> 5.0, 8192 x 8 6.5 -> 5.1, 16384 x 4 6.6 -> 5.3; tags 1024 x 16
+// 6.9 -> 5.7, 8192 x 8 7.3 -> 6.9.  (Throttling stays at two launches: its last workgroup overwrites the prefix that
+// the others read.)
 #include <algorithm>
 #include <cstdlib>
 #include <mutex>
@@ -62,12 +70,20 @@ struct ScanGeometry {
   int ep_shift;  // log2 of the lanes one row occupies (E <= 64), 6 otherwise
   int rows_pw;   // rows per wavefront (multiple of the rows one load covers)
   int bands;     // workgroups
-  int waves_pb;  // wavefronts per workgroup: kWavesPB, or kWavesSingle for the one-workgroup form
+  int waves_pb;  // wavefronts per workgroup: kWavesPB, kWavesSingle for the one-workgroup form, kWavesWhole
+                 // where every workgroup adds up all rows above its own
 };
 
 constexpr int kWavesSingle = 8;  // 512 threads: the kernel keeps its 256 registers per lane
+constexpr int kWavesWhole = 16;
+constexpr int kWholeLoads = 1024;  // most loads of 64 words that cover a mask of this form: 256 KB
+constexpr int kWholeRows = 2;      // loads that cover a wavefront's rows
 
-ScanGeometry scan_geometry(int T, int E, bool tag_mode) {
+// Rows that are whole 16-byte units, or that fill a load without gaps.  With others the lanes past E tear the loads
+// of the rows above apart (4096 x 9: 10.2 us in one launch, 7.6 in two; 4000 x 12: 5.0 and 6.4).
+bool whole_rows(int E) { return E % 4 == 0 || E <= 2; }
+
+ScanGeometry scan_geometry(int T, int E, bool tag_mode, bool whole_ok) {
   ScanGeometry g;
   int shift = 0;
   while ((1 << shift) < std::min(E, kWave)) ++shift;
@@ -96,6 +112,15 @@ ScanGeometry scan_geometry(int T, int E, bool tag_mode) {
     g.rows_pw = static_cast<int>(rows_pw);
     g.bands = 1;
     g.waves_pb = kWavesSingle;
+    return g;
+  }
+  // One launch in which every workgroup adds up all rows above its own itself (figures at the head of the file).  The
+  // gain shrinks with the rows to add up: at 64 loads per lane (kWholeLoads) it is 1.2 us for seats, 0.4 us for tags.
+  const long loads = (static_cast<long>(T) + rps - 1) / rps;
+  if (forced_bands <= 0 && whole_ok && whole_rows(E) && E <= kWave && loads <= kWholeLoads) {
+    g.rows_pw = kWholeRows * rps;
+    g.bands = static_cast<int>((loads + kWholeRows * kWavesWhole - 1) / (kWholeRows * kWavesWhole));
+    g.waves_pb = kWavesWhole;
     return g;
   }
   // Enough bands that a wavefront's rows fit one batch of loads, at least 128 (so
@@ -145,11 +170,12 @@ __device__ __forceinline__ int sum_over_rows_in_wave(int v, int ep_shift) {
 // add up: with 8 paths (8 rows per load, four shuffles) they were a third of the kernel.  Ballots here and
 // buffer loads below: 100352 x 8 throttled 10.2 -> 6.5 us, seat indices 8.5 -> 5.2 us; 16384 x 32 8.3 -> 6.2
 // and 6.7 -> 5.1 us.
-__device__ __forceinline__ void sums_of_loads(const int (&m)[kBatch], int n, int rps, int ep, int e, int lane,
-                                              int (&incl)[kBatch], int (&tot)[kBatch]) {
+template <int N>
+__device__ __forceinline__ void sums_of_loads(const int (&m)[N], int n, int rps, int ep, int e, int lane,
+                                              int (&incl)[N], int (&tot)[N]) {
   int other = 0;
 #pragma unroll
-  for (int u = 0; u < kBatch; ++u) {
+  for (int u = 0; u < N; ++u) {
     incl[u] = tot[u] = m[u];
     other |= m[u] & ~1;
   }
@@ -159,7 +185,7 @@ __device__ __forceinline__ void sums_of_loads(const int (&m)[kBatch], int n, int
     for (int d = ep; d < kWave; d <<= 1) path |= path << d;
     const unsigned long long upto = path & ((2ull << lane) - 1ull);  // ... up to this lane
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
+    for (int u = 0; u < N; ++u) {
       const unsigned long long ones = __ballot(m[u] != 0);  // zero behind the wavefront's last load
       incl[u] = __popcll(ones & upto);
       tot[u] = __popcll(ones & path);
@@ -167,7 +193,7 @@ __device__ __forceinline__ void sums_of_loads(const int (&m)[kBatch], int n, int
     return;
   }
 #pragma unroll
-  for (int u = 0; u < kBatch; ++u) {
+  for (int u = 0; u < N; ++u) {
     if (u < n) {  // wave-uniform
       int x = m[u];
       for (int d = ep; d < kWave; d <<= 1) {
@@ -183,18 +209,18 @@ __device__ __forceinline__ void sums_of_loads(const int (&m)[kBatch], int n, int
 // Second walk over one batch of row words held in registers: turns the mask words
 // into seats / throttled bits / tag slots.  The sums over the rows of every load come first and do
 // not depend on the running sum.
-template <int MODE>
-__device__ __forceinline__ void walk_batch(const int (&m)[kBatch], int i0, int n_ins, int& carry,
+template <int MODE, int N>
+__device__ __forceinline__ void walk_batch(const int (&m)[N], int i0, int n_ins, int& carry,
                                            int thr, int total, long row_w, int rps, int ep, int sub,
                                            int e, int lane, int col, bool col_ok, const ScanArgs& a) {
-  int incl[kBatch], tot[kBatch];
+  int incl[N], tot[N];
   sums_of_loads(m, n_ins - i0, rps, ep, e, lane, incl, tot);
   // rows of this wavefront through one 64-bit base and 32-bit offsets: the address of every
   // store is one instruction instead of a 64-bit multiply-add chain
   int* __restrict__ out_w = a.out + row_w * a.E;
   const int rows_here = static_cast<int>(max(0l, min(static_cast<long>(a.rows_pw), a.T - row_w)));
 #pragma unroll
-  for (int u = 0; u < kBatch; ++u) {
+  for (int u = 0; u < N; ++u) {
     const int run = carry + incl[u];
     carry += tot[u];
     const int rl = (i0 + u) * rps + sub;  // row within the wavefront's rows
@@ -234,12 +260,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_of_wave(long row_w, const
 constexpr int kWidePaths = 1 << 20;
 
 // Loads one batch of row words (zero beyond the band / the matrix).
-template <bool WIDE>
-__device__ __forceinline__ void load_batch(int (&v)[kBatch], __amdgpu_buffer_rsrc_t rows, long row_w, int i0, int rps,
+template <bool WIDE, int N>
+__device__ __forceinline__ void load_batch(int (&v)[N], __amdgpu_buffer_rsrc_t rows, long row_w, int i0, int rps,
                                            int sub, int col, bool col_ok, const ScanArgs& a) {
   if constexpr (WIDE) {
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
+    for (int u = 0; u < N; ++u) {
       const int rl = (i0 + u) * rps + sub;
       v[u] = col_ok && rl < a.rows_pw && row_w + rl < a.T ? a.mask[static_cast<size_t>(row_w + rl) * a.E + col] : 0;
     }
@@ -248,7 +274,7 @@ __device__ __forceinline__ void load_batch(int (&v)[kBatch], __amdgpu_buffer_rsr
   const unsigned first = col_ok ? (static_cast<unsigned>(i0 * rps + sub) * a.E + col) * 4u : kOutside;
   const unsigned step = rps * a.E * 4u;
 #pragma unroll
-  for (int u = 0; u < kBatch; ++u) v[u] = __builtin_amdgcn_raw_buffer_load_b32(rows, first + u * step, 0, 0);
+  for (int u = 0; u < N; ++u) v[u] = __builtin_amdgcn_raw_buffer_load_b32(rows, first + u * step, 0, 0);
 }
 
 // This lane's share of the column sums of bands [j0, end), every `step`-th of them.
@@ -309,14 +335,16 @@ __global__ __launch_bounds__(kBlock) void band_count_kernel(ScanArgs a) {
   }
 }
 
-// pass 2: offsets from the bands above, running sums in registers, results out
-template <int MODE, int kWavesPB, bool WIDE>
+// pass 2: offsets from the bands above, running sums in registers, results out.  WHOLE: there was no pass 1,
+// the offsets are the column sums of all rows above (a row is a band of its own).
+template <int MODE, int kWavesPB, bool WIDE, bool WHOLE = false>
 __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a) {
   __shared__ int s_above[kWavesPB][kWave];  // each wave's share of the sum over earlier bands
   __shared__ int s_own[kWavesPB][kWave];    // column sums of each wave's own rows
   __shared__ int s_below[kWavesPB][kWave];  // tag mode: share of the sum over later bands
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int kOwn = WHOLE ? kWholeRows : kBatch;  // loads of this wavefront's rows that stay in registers
   const int E = a.E, band = blockIdx.x;
   const int ep = 1 << a.ep_shift, rps = kWave >> a.ep_shift;
   const int e = lane & (ep - 1), sub = lane >> a.ep_shift;
@@ -328,21 +356,24 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
     const int col = c0 + e;
     const bool col_ok = col < E;
     // ---- own rows: the first batch stays in registers ---------------------------------
-    int m0[kBatch];
+    int m0[kOwn];
     load_batch<WIDE>(m0, rows, row_w, 0, rps, sub, col, col_ok, a);
     // ---- this wave's share of the offset: bands wave, wave+4, ... above this one ----
-    int above = sum_of_bands<WIDE>(wave + sub * kWavesPB, band, kWavesPB * rps, col, col_ok, a), below = 0;
+    // (consecutive rows in one load where the rows of the mask are the bands: they are next to each other)
+    const int rows_pb = WHOLE ? kWavesPB * a.rows_pw : 1, all = WHOLE ? a.T : a.bands;
+    const int share = WHOLE ? wave * rps + sub : wave + sub * kWavesPB;
+    int above = sum_of_bands<WIDE>(share, min(band * rows_pb, all), kWavesPB * rps, col, col_ok, a), below = 0;
     if (MODE == kTag)  // the tag list of a path ends at its total: the later bands count too
-      below = sum_over_rows_in_wave(sum_of_bands<WIDE>(band + 1 + wave + sub * kWavesPB, a.bands, kWavesPB * rps, col, col_ok, a),
-                                    a.ep_shift);
+      below = sum_over_rows_in_wave(
+          sum_of_bands<WIDE>((band + 1) * rows_pb + share, all, kWavesPB * rps, col, col_ok, a), a.ep_shift);
     int own = 0;
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) own += m0[u];
-    for (int i0 = kBatch; i0 < n_ins; i0 += kBatch) {
-      int v[kBatch];
+    for (int u = 0; u < kOwn; ++u) own += m0[u];
+    for (int i0 = kOwn; i0 < n_ins; i0 += kOwn) {
+      int v[kOwn];
       load_batch<WIDE>(v, rows, row_w, i0, rps, sub, col, col_ok, a);
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) own += v[u];
+      for (int u = 0; u < kOwn; ++u) own += v[u];
     }
     above = sum_over_rows_in_wave(above, a.ep_shift);
     own = sum_over_rows_in_wave(own, a.ep_shift);
@@ -377,8 +408,8 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
     // ---- walk the rows again: running sum per path, one result per element ----------
     const int total = band_total + later;  // tag mode: entries of this path's list
     walk_batch<MODE>(m0, 0, n_ins, carry, thr, total, row_w, rps, ep, sub, e, lane, col, col_ok, a);
-    for (int i0 = kBatch; i0 < n_ins; i0 += kBatch) {
-      int v[kBatch];
+    for (int i0 = kOwn; i0 < n_ins; i0 += kOwn) {
+      int v[kOwn];
       load_batch<WIDE>(v, rows, row_w, i0, rps, sub, col, col_ok, a);
       walk_batch<MODE>(v, i0, n_ins, carry, thr, total, row_w, rps, ep, sub, e, lane, col, col_ok, a);
     }
@@ -447,9 +478,13 @@ __global__ __launch_bounds__(kBlock) void band_apply_dispatch_kernel(FusedArgs f
   // words, capacities, and last the wavefront's rows, which are stored at the very end.
   // ---- sums of the other bands (the host keeps the bands within kFusedPartials loads per lane) ----
   int part[kFusedPartials];
-  const int j_first = wave + sub * kWavesPB, j_step = kWavesPB * rps;
+  // (without a pass 1 every row of the mask is a band of its own here, as in band_apply_kernel)
+  const bool whole = a.partial == a.mask;
+  const int rows_pb = whole ? kWavesPB * a.rows_pw : 1;
+  const int j_first = whole ? wave * rps + sub : wave + sub * kWavesPB, j_step = kWavesPB * rps;
+  const int j_own = band * rows_pb, j_later = j_own + rows_pb;
   {
-    const __amdgpu_buffer_rsrc_t res_partial = words_at(a.partial, static_cast<size_t>(a.bands) * E * 4);
+    const __amdgpu_buffer_rsrc_t res_partial = words_at(a.partial, static_cast<size_t>(whole ? a.T : a.bands) * E * 4);
     const unsigned partial_off = col_ok ? (j_first * E + e) * 4 : kOutside;
 #pragma unroll
     for (int u = 0; u < kFusedPartials; ++u)
@@ -483,8 +518,8 @@ __global__ __launch_bounds__(kBlock) void band_apply_dispatch_kernel(FusedArgs f
 #pragma unroll
   for (int u = 0; u < kFusedPartials; ++u) {
     const int j = j_first + u * j_step;
-    above += j < band ? part[u] : 0;
-    below += j > band ? part[u] : 0;
+    above += j < j_own ? part[u] : 0;
+    below += j >= j_later ? part[u] : 0;
   }
   int capv[kFusedCaps];
 #pragma unroll
@@ -689,8 +724,14 @@ __global__ __launch_bounds__(256) void tag_to_seat_kernel(const int* __restrict_
   }
 }
 
+// Whether the matrices share words: with one launch a workgroup may write rows that another has yet to add up.
+bool same_words(const int* mask, const int* out, int T, int E) {
+  const uintptr_t m = reinterpret_cast<uintptr_t>(mask), o = reinterpret_cast<uintptr_t>(out), bytes = static_cast<uintptr_t>(T) * E * 4;
+  return m < o + bytes && o < m + bytes;
+}
+
 int launch_scan(int mode, ScanArgs& a, void* workspace, size_t workspace_bytes, void* stream) {
-  const ScanGeometry g = scan_geometry(a.T, a.E, mode == kTag);
+  const ScanGeometry g = scan_geometry(a.T, a.E, mode == kTag, mode != kThrottle && !same_words(a.mask, a.out, a.T, a.E));
   const size_t need = brt_hip_scan_workspace_bytes(a.T, a.E);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(BRT_E_WORKSPACE, "scan workspace too small: %zu < %zu bytes", workspace_bytes,
@@ -712,6 +753,13 @@ int launch_scan(int mode, ScanArgs& a, void* workspace, size_t workspace_bytes, 
       hipLaunchKernelGGL((band_apply_kernel<kTag, kWavesSingle, false>), grid, block, 0, st, a);
     else
       hipLaunchKernelGGL((band_apply_kernel<kThrottle, kWavesSingle, false>), grid, block, 0, st, a);
+    return check_launch("band_apply_kernel");
+  }
+  if (g.waves_pb == kWavesWhole) {
+    a.partial = const_cast<int*>(a.mask);
+    const dim3 block(kWavesWhole * kWave);
+    if (mode == kSeat) hipLaunchKernelGGL((band_apply_kernel<kSeat, kWavesWhole, false, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((band_apply_kernel<kTag, kWavesWhole, false, true>), grid, block, 0, st, a);
     return check_launch("band_apply_kernel");
   }
   auto launch = [&](auto wide) {
@@ -787,7 +835,7 @@ using namespace brt;
 extern "C" size_t brt_hip_scan_workspace_bytes(int T, int E) {
   if (T <= 0 || E <= 0) return 0;
   // enough for either index format (tag indices leave the one-workgroup form earlier)
-  const int bands = std::max(scan_geometry(T, E, false).bands, scan_geometry(T, E, true).bands);
+  const int bands = std::max(scan_geometry(T, E, false, false).bands, scan_geometry(T, E, true, false).bands);
   return (static_cast<size_t>(bands) + 1) * E * sizeof(int);
 }
 
@@ -922,7 +970,13 @@ extern "C" int brt_hip_route_and_dispatch(const int32_t* mask, const void* cells
   f.cpr = static_cast<int>(cell_bytes / 16);
   hipStream_t st = as_stream(stream);
   const dim3 grid(g.bands);
-  if (g.bands > 1) hipLaunchKernelGGL(band_count_kernel<false>, grid, dim3(kBlock), 0, st, a);
+  const int rps = kWave >> g.ep_shift;
+  // one launch while a lane's batch of loads covers the whole mask, up to 64 KB: 1024 x 16 cells of 1 KB 8.4 -> 6.2 us,
+  // 256 x 64 cells of 2 KB 7.7 -> 5.4, 100 x 8 8.8 -> 6.6, 16384 x 1 cells of 128 bytes 10.9 -> 7.1
+  if (g.bands > 1 && whole_rows(E) && T <= kFusedPartials * kWavesPB * rps && !same_words(mask, indices, T, E))
+    a.partial = const_cast<int*>(mask);
+  else if (g.bands > 1)
+    hipLaunchKernelGGL(band_count_kernel<false>, grid, dim3(kBlock), 0, st, a);
   // rows of more than 128 bytes leave as streaming stores, shorter ones merge in the L2 (as in dispatch)
   const int units = (g.rows_pw * f.cpr + kWave - 1) / kWave;  // per lane
   auto go = [&](auto stream_t, auto nv_t) {

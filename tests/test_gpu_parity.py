@@ -85,6 +85,35 @@ def test_indices_general_mask_values_and_misaligned_buffers(hip):
 
 
 # on both sides of the widest matrix that is read through 32-bit byte offsets, and where those would wrap round
+@pytest.mark.parametrize("T,E", [
+    (513, 16), (4096, 16), (4097, 16),        # behind the one-workgroup form; the last of one launch, the first of two
+    (129, 64), (1024, 64), (1025, 64), (700, 40), (4000, 12), (8189, 8), (16384, 4),
+    (32768, 2), (65536, 1), (65537, 1), (4096, 9), (3000, 6),  # few paths; rows that are no 16-byte units
+])
+def test_indices_of_masks_one_launch_takes(hip, T, E):
+    """Around the sizes where every workgroup adds up the rows above its own: seats and tags, zeros and
+    ones and (seats) other words, and index generation in place."""
+    rng = np.random.default_rng(T + E)
+    mask = (rng.random((T, E)) < 0.3).astype(np.int32)
+    caps = [max(1, T // 5)]
+    for tag in (False, True):
+        idx, loads, counts = hip.generate_indices_and_loads(mask, caps, is_tag_index=tag, want_counts=True)
+        o_idx, o_loads = oracle.generate_indices_and_loads(mask, caps, is_tag_index=tag)
+        assert np.array_equal(idx, o_idx) and np.array_equal(loads, o_loads)
+        assert np.array_equal(counts, mask.sum(axis=0))
+    words = mask.copy()
+    words[:: 7] *= -3
+    idx, loads = hip.generate_indices_and_loads(words)
+    o_idx, o_loads = oracle.generate_indices_and_loads(words)
+    assert np.array_equal(idx, o_idx) and np.array_equal(loads, o_loads)
+    # in place: the words above a workgroup's rows must not be the results of another one
+    lib, ws = hip._lib.lib(), hip.workspace(T, E)
+    both, loads = hip.dev(words), hip.dev(np.zeros(E, dtype=np.int32))
+    hip._lib.check(lib.brt_hip_generate_indices_and_loads(hip.ptr(both), hip.ptr(both), hip.ptr(loads), None, T, E, None, 0, 0, 0, 0,
+                                                          hip.ptr(ws), ws.numel(), hip.stream()))
+    assert np.array_equal(hip.host(both), o_idx) and np.array_equal(hip.host(loads), o_loads)
+
+
 @pytest.mark.parametrize("T,E", [(9, (1 << 20) - 1), (9, 1 << 20), (6, (1 << 24) + 8)])
 def test_index_generation_of_very_many_paths(hip, T, E):
     mask = np.random.default_rng(E).integers(0, 2, (T, E), dtype=np.int8).astype(np.int32)
@@ -228,6 +257,15 @@ def test_route_and_dispatch_bit_exact(hip, T, E, k, cell, dtype):
             n = min(P, total)
             assert same_bits(rows[:n], want[:n]) and np.array_equal(tags[:n], want_tags[:n])
             assert not rows[n:].any() and not tags[n:].any()  # rows past the last path are zero
+
+
+@pytest.mark.parametrize("T,E,k,cell,dtype", [
+    (1024, 16, 1, 512, "bf16"), (1025, 16, 2, 64, "bf16"), (256, 64, 2, 128, "f16"), (257, 64, 1, 64, "bf16"), (64, 64, 1, 8, "f32"),
+    (1000, 12, 1, 64, "bf16"), (8192, 2, 1, 32, "f16"), (16384, 1, 1, 8, "f16"), (16385, 1, 1, 8, "f16"), (900, 9, 1, 16, "f32"),
+])
+def test_route_and_dispatch_of_masks_one_launch_takes(hip, T, E, k, cell, dtype):
+    """Around the 64 KB of mask up to which every workgroup adds up the other rows itself."""
+    test_route_and_dispatch_bit_exact(hip, T, E, k, cell, dtype)
 
 
 def test_route_and_dispatch_with_int32_arrays_that_are_only_4_byte_aligned(hip):
