@@ -23,6 +23,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <chrono>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -576,13 +577,47 @@ PyObject* cast_f32_to_bf16(const Args& a) {
 }
 
 // ---- host reads --------------------------------------------------------------------------------------
+// Whether the word that a kernel sets behind its data is set, within the time that a program's next few launches
+// would take; behind more work than that the caller waits for the stream, which does not keep a core busy.
+bool seen_within(const int32_t* word, std::chrono::microseconds limit) {
+  const auto end = std::chrono::steady_clock::now() + limit;
+  do {
+    for (int i = 0; i < 64; ++i) {
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != 0) return true;
+      __builtin_ia32_pause();
+    }
+  } while (std::chrono::steady_clock::now() < end);
+  return false;
+}
+
 // Copies from the device on the current stream into pinned memory and waits for the copy (other Python
-// threads run meanwhile).
+// threads run meanwhile).  Few words are stored there by a kernel and watched for; more, or a stream that is being
+// captured (where reading back is an error), take the runtime's copy and wait.
 at::DataPtr read_back(const Tensor& t, size_t bytes, const char* what) {
-  at::DataPtr host = at::getHostAllocator(at::kCUDA)->allocate(bytes);
+  constexpr size_t kFewBytes = 4096;
+  at::DataPtr host = at::getHostAllocator(at::kCUDA)->allocate(bytes + 4);
   const hipStream_t st = c10::hip::getCurrentHIPStream(t.get_device()).stream();
-  hipError_t rc = hipMemcpyAsync(host.get(), ptr(t), bytes, hipMemcpyDeviceToHost, st);
-  if (rc == hipSuccess) {
+  void* seen_from_device = nullptr;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  bool watch = bytes <= kFewBytes && bytes % 4 == 0;
+  if (watch && (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
+                hipHostGetDevicePointer(&seen_from_device, host.get(), 0) != hipSuccess)) {
+    (void)hipGetLastError();  // what asking left behind, if anything
+    watch = false;
+  }
+  hipError_t rc = hipSuccess;
+  if (watch) {
+    int32_t* const word = static_cast<int32_t*>(host.get()) + bytes / 4;
+    __atomic_store_n(word, 0, __ATOMIC_RELEASE);
+    if (brt_hip_copy_to_host(iptr(t), static_cast<int32_t*>(seen_from_device), static_cast<int>(bytes / 4), st) != BRT_OK)
+      runtime_error(std::string(what) + ": " + brt_hip_last_error());
+    Py_BEGIN_ALLOW_THREADS
+    watch = seen_within(word, std::chrono::microseconds(500));
+    Py_END_ALLOW_THREADS
+  } else {
+    rc = hipMemcpyAsync(host.get(), ptr(t), bytes, hipMemcpyDeviceToHost, st);
+  }
+  if (rc == hipSuccess && !watch) {
     Py_BEGIN_ALLOW_THREADS
     rc = hipStreamSynchronize(st);
     Py_END_ALLOW_THREADS

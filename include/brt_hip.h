@@ -454,6 +454,14 @@ int brt_hip_combine_by_rows_gated(const void* src, void* dst, const void* gates,
                                   int P, int is_residual, int in_dtype, int out_dtype, void* stream);
 
 /*
+ * src[0 .. words-1] to host[0 .. words-1], then host[words] = 1: host memory of words + 1 words that the device can
+ * write (hipHostMalloc).  A host that cleared host[words] before the call may watch it (acquire loads) instead of waiting
+ * for the stream; nothing is written behind it.  Takes the place of the copy and the wait with which the reference reads
+ * the loads (src/backend/torch/router.cc:197-201).  Not for a captured stream: a replay would write to the same memory.
+ */
+int brt_hip_copy_to_host(const int32_t* src, int32_t* host, int words, void* stream);
+
+/*
  * Measurement aid (no counterpart in the reference; bench.py reports what it reads beside the
  * compute-bound shapes): brt_hip_grouped_gemm through the 256 x 256 ping-pong kernel, whatever the
  * shape (BRT_E_UNSUPPORTED when that kernel does not take it: K must be a multiple of 64 and at

@@ -1156,3 +1156,20 @@ def test_counts_given_as_whole_floats_are_taken(brt_mod):
     assert all(torch.equal(a, b) for a, b in zip(got, want))
     x = torch.randn(40, 16).cuda()
     assert torch.equal(c_router.dispatch_by_rows(x, want[3], 2.0), c_router.dispatch_by_rows(x, want[3], 2))
+
+
+@pytest.mark.parametrize("n", [1, 16, 64, 65, 256, 257, 1024, 1025, 5000])
+def test_words_read_back_by_the_host(n):
+    """Around the widths of the kernel that stores them into host memory and the size up to which it is taken, behind
+    little work and behind more than the host watches for."""
+    from brainstorm_amd import _lib
+
+    words = torch.randint(-2**31, 2**31 - 1, (3 * n + 1,), dtype=torch.int64).to(torch.int32)
+    for wait in (0, 4_000_000):
+        for view in (words[:n], words[1:n + 1], words[::3][:n]):
+            on_device = view.cuda() if view.is_contiguous() else words.cuda()[::3][:n]
+            if wait:
+                torch.cuda._sleep(wait)
+            shifted = on_device + 0  # queued behind the work
+            assert _lib.native().int_list(shifted) == view.tolist()
+            assert _lib.native().int_list(on_device) == view.tolist()
