@@ -21,6 +21,7 @@ _DT = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF
 __all__ = [
     "topk_hot_mask",
     "throttle_hotmask",
+    "top1_to_capacity",
     "Route",
     "CompactRoute",
     "remember_route",
@@ -193,6 +194,13 @@ def throttle_hotmask(
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """router.cc:15-31.  ``prefix`` is updated in place and returned."""
     return _lib.native().throttle_hotmask(hot_mask, prefix, threshold), prefix
+
+
+def top1_to_capacity(score: torch.Tensor, capacity: int):
+    """Not in the reference's extension: ``topk_hot_mask(score, 1)`` throttled from a zero prefix to ``capacity``
+    cells of every path, and the capacity of every path as an int32 vector (swin_moe.py:101-126), in two launches; None
+    where the fused kernels do not take the shape."""
+    return _lib.native().top1_to_capacity(score, int(capacity))
 
 
 def generate_route(

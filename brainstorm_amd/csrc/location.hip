@@ -46,6 +46,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "gate.hpp"
 #include "rows.hpp"
 
 // Scratch of brt_hip_generate_indices_and_loads_static: the per-band column sums that the first
@@ -140,14 +141,28 @@ ScanGeometry scan_geometry(int T, int E, bool tag_mode, bool whole_ok) {
   return g;
 }
 
+// Bands of a throttled top-1 route: always the two-launch form (its first launch reads the scores anyway).
+ScanGeometry top1_geometry(int T, int E) {
+  ScanGeometry g = scan_geometry(T, E, true, false);
+  if (g.waves_pb != kWavesPB) {  // a mask that one workgroup of eight wavefronts would hold
+    const int rps = kWave >> g.ep_shift;
+    g.rows_pw = (T + kWavesPB * rps - 1) / (kWavesPB * rps) * rps;
+    g.waves_pb = kWavesPB;
+    g.bands = 1;
+  }
+  return g;
+}
+
 struct ScanArgs {
   const int* mask;
   int* out;
   int* loads;
   int* counts;
   const int* caps;
-  int* prefix;           // throttle only, updated in place
-  const int* threshold;  // throttle only
+  int* prefix;           // throttle only, updated in place; null: no cell was taken before
+  const int* threshold;  // throttle only; null: `capacity` cells of every path
+  int capacity;
+  int* capacities;       // throttle only: `capacity` of every path, written where non-null
   int* partial;          // [bands][E] per-band column sums
   int* prefix_in;        // throttle only: copy of prefix taken by pass 1 ([E])
   int T, E, C;
@@ -335,6 +350,48 @@ __global__ __launch_bounds__(kBlock) void band_count_kernel(ScanArgs a) {
   }
 }
 
+// pass 1 of a throttled top-1 route: the hot mask of the largest score of every row (order of torch.topk as in
+// gate.hip) and the column sums of the band, from one read of the scores; up to 64 paths.  Bound by the round trip of
+// a batch of loads; the mask and its sums by themselves take a launch each (100352 x 8 fp32 scores: 4.1 + 3.4 us).
+template <int DT>
+__global__ __launch_bounds__(kBlock) void band_top1_kernel(const void* scores, ScanArgs a, int* mask) {
+  __shared__ int s_sum[kWavesPB][kWave];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int E = a.E, ep = 1 << a.ep_shift, rps = kWave >> a.ep_shift;
+  const int e = lane & (ep - 1), sub = lane >> a.ep_shift;
+  const unsigned long long row_lanes = (ep == kWave ? ~0ull : ((1ull << ep) - 1ull)) << (sub * ep);
+  const long row_w = (static_cast<long>(blockIdx.x) * kWavesPB + wave) * a.rows_pw;
+  const int rows_here = static_cast<int>(max(0l, min(static_cast<long>(a.rows_pw), a.T - row_w)));
+  int sum = 0;
+  for (int i0 = 0; i0 < a.n_ins; i0 += kBatch) {
+    uint32_t key[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int rl = (i0 + u) * rps + sub;
+      key[u] = rl < rows_here && e < E ? score_key(load_score<DT>(scores, static_cast<size_t>(row_w + rl) * E + e)) : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (i0 + u >= a.n_ins) break;  // wave-uniform
+      const uint32_t best = segment_max(key[u], ep);
+      const unsigned long long tied = __ballot(key[u] == best && key[u] != 0) & row_lanes;
+      const int taken = tied != 0 && lane == __builtin_ctzll(tied) ? 1 : 0;
+      sum += taken;
+      if (key[u] != 0) mask[static_cast<size_t>(row_w + (i0 + u) * rps + sub) * E + e] = taken;
+    }
+  }
+  sum = sum_over_rows_in_wave(sum, a.ep_shift);
+  if (sub == 0) s_sum[wave][e] = sum;
+  __syncthreads();
+  if (tid < E) {
+    int total = 0;
+#pragma unroll
+    for (int k = 0; k < kWavesPB; ++k) total += s_sum[k][tid];
+    a.partial[static_cast<size_t>(blockIdx.x) * E + tid] = total;
+  }
+}
+
 // pass 2: offsets from the bands above, running sums in registers, results out.  WHOLE: there was no pass 1,
 // the offsets are the column sums of all rows above (a row is a band of its own).
 template <int MODE, int kWavesPB, bool WIDE, bool WHOLE = false>
@@ -381,8 +438,8 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
     // the end of its walk, which no wavefront may overtake
     int thr = 0, pre_in = 0;
     if (MODE == kThrottle && col_ok) {
-      pre_in = (a.bands > 1 ? a.prefix_in : a.prefix)[col];
-      thr = a.threshold[col];
+      if (a.prefix != nullptr) pre_in = (a.bands > 1 ? a.prefix_in : a.prefix)[col];
+      thr = a.threshold != nullptr ? a.threshold[col] : a.capacity;
     }
     if (c0 > 0) __syncthreads();
     if (sub == 0) {
@@ -417,7 +474,8 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
     // ---- totals: loads / counts / throttle prefix (last band only) ---------------------
     if (band == a.bands - 1 && wave == 0 && sub == 0 && col_ok) {
       if (MODE == kThrottle) {
-        a.prefix[col] = min(band_total + pre_in, thr);
+        if (a.prefix != nullptr) a.prefix[col] = min(band_total + pre_in, thr);
+        if (a.capacities != nullptr) a.capacities[col] = a.capacity;
       } else {
         a.loads[col] =
             finalize_load(band_total, a.caps, a.C, a.capacity_padding, a.path_wise_padding, col);
@@ -1008,6 +1066,46 @@ extern "C" int brt_hip_throttle_hotmask(const int32_t* mask, int32_t* out, int32
   a.T = T;
   a.E = E;
   return launch_scan(kThrottle, a, workspace, workspace_bytes, stream);
+}
+
+extern "C" int brt_hip_top1_to_capacity(const void* scores, int dtype, int32_t* mask, int32_t* out, int32_t* capacities,
+                                        int capacity, int T, int E, void* workspace, size_t workspace_bytes, void* stream) {
+  if (T < 0 || E <= 0) return fail(BRT_E_INVALID, "bad shape T=%d E=%d", T, E);
+  if (dtype != BRT_F32 && dtype != BRT_F16 && dtype != BRT_BF16) return fail(BRT_E_UNSUPPORTED, "dtype %d is not supported", dtype);
+  if (E > kWave) return fail(BRT_E_UNSUPPORTED, "top1_to_capacity takes up to %d paths, got %d", kWave, E);
+  if (static_cast<long>(T) * E >= (1l << 31)) return fail(BRT_E_UNSUPPORTED, "T*E >= 2^31");
+  if (!capacities) return fail(BRT_E_INVALID, "null argument");
+  if (T == 0) {
+    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, as_stream(stream), capacities, E, capacity);
+    return check_launch("fill_int_kernel");
+  }
+  if (!scores || !mask || !out) return fail(BRT_E_INVALID, "null argument");
+  if (same_words(mask, out, T, E)) return fail(BRT_E_INVALID, "mask and out must not overlap");
+  const ScanGeometry g = top1_geometry(T, E);
+  const size_t need = (static_cast<size_t>(g.bands) + 1) * E * sizeof(int);
+  if (workspace == nullptr || workspace_bytes < need)
+    return fail(BRT_E_WORKSPACE, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
+  if (!aligned(workspace, 4)) return fail(BRT_E_INVALID, "workspace must be 4-byte aligned");
+  ScanArgs a{};
+  a.mask = mask;
+  a.out = out;
+  a.capacity = capacity;
+  a.capacities = capacities;
+  a.partial = static_cast<int*>(workspace);
+  a.T = T;
+  a.E = E;
+  a.ep_shift = g.ep_shift;
+  a.rows_pw = g.rows_pw;
+  a.n_ins = g.rows_pw >> (6 - g.ep_shift);
+  a.bands = g.bands;
+  const dim3 grid(g.bands), block(kBlock);
+  hipStream_t st = as_stream(stream);
+  if (dtype == BRT_F32) hipLaunchKernelGGL(band_top1_kernel<BRT_F32>, grid, block, 0, st, scores, a, mask);
+  else if (dtype == BRT_F16) hipLaunchKernelGGL(band_top1_kernel<BRT_F16>, grid, block, 0, st, scores, a, mask);
+  else hipLaunchKernelGGL(band_top1_kernel<BRT_BF16>, grid, block, 0, st, scores, a, mask);
+  if (const int rc = check_launch("band_top1_kernel"); rc != BRT_OK) return rc;
+  hipLaunchKernelGGL((band_apply_kernel<kThrottle, kWavesPB, false>), grid, block, 0, st, a);
+  return check_launch("band_apply_kernel");
 }
 
 extern "C" int brt_hip_convert_index_format(const int32_t* src, int32_t* dst,

@@ -99,12 +99,16 @@ def _one_hot_int32(indices: torch.Tensor, like: torch.Tensor) -> torch.Tensor:
     return torch.zeros(like.shape, dtype=torch.int32, device=like.device).scatter_(1, indices, 1)
 
 
+def _kernel_takes(score) -> bool:
+    return (score.is_cuda and score.dim() == 2 and score.shape[1] <= 1024
+            and score.dtype in (torch.float32, torch.float16, torch.bfloat16))
+
+
 def _topk_hot_mask(score, top_k):
     """int32 mask with ones at the ``top_k`` largest scores of every row (``torch.topk`` +
     ``zeros_like`` + ``scatter_``, protocol/topk.py:26-31): one kernel where the score is a 2-d
     device tensor of up to 1024 paths, the three torch launches otherwise."""
-    if (score.is_cuda and score.dim() == 2 and score.shape[1] <= 1024
-            and score.dtype in (torch.float32, torch.float16, torch.bfloat16)):
+    if _kernel_takes(score):
         return c_router.topk_hot_mask(score, top_k)
     return _one_hot_int32(torch.topk(score, top_k, dim=1).indices, score)
 
@@ -316,9 +320,13 @@ class SwinMoEProtocol(ProtocolBase):
 
     def make_route_decision(self, score, logits_wo_noise, logits):
         paths = score.size(1)
-        mask = _topk_hot_mask(score, 1)  # the first of the top-k choices (swin_moe.py:101-107)
         loss = self.generate_auxiliary(score, logits_wo_noise, logits, None)
         cap = self.runtime_capacity(score.size(0), paths)
+        if not self.batch_prioritized_routing and _kernel_takes(score):
+            both = c_router.top1_to_capacity(score, cap)
+            if both is not None:
+                return both[0], both[1], score, loss
+        mask = _topk_hot_mask(score, 1)  # the first of the top-k choices (swin_moe.py:101-107)
         runtime_capacities = torch.full((paths,), cap, dtype=torch.int32, device=score.device)
         prefix = torch.zeros((paths,), dtype=torch.int32, device=score.device)
         hot_mask, _ = throttle_to_capacity(

@@ -454,6 +454,16 @@ int brt_hip_combine_by_rows_gated(const void* src, void* dst, const void* gates,
                                   int P, int is_residual, int in_dtype, int out_dtype, void* stream);
 
 /*
+ * brt_hip_topk_hot_mask with k = 1 and brt_hip_throttle_hotmask from a zero prefix with one capacity for all paths, in two
+ * launches and one read of the scores: mask [T,E] the hot mask, out [T,E] what the capacity leaves of it, capacities [E] the
+ * capacity of every path (what python/brt/router/protocol/swin_moe.py:101-126 makes of them).  mask and out must not
+ * overlap.  E <= 64.  Workspace of brt_hip_scan_workspace_bytes(T, E) bytes, 4-byte aligned, uninitialised.
+ */
+int brt_hip_top1_to_capacity(const void* scores, int dtype, int32_t* mask, int32_t* out, int32_t* capacities,
+                             int capacity, int T, int E, void* workspace, size_t workspace_bytes,
+                             void* stream);
+
+/*
  * src[0 .. words-1] to host[0 .. words-1], then host[words] = 1: host memory of words + 1 words that the device can
  * write (hipHostMalloc).  A host that cleared host[words] before the call may watch it (acquire loads) instead of waiting
  * for the stream; nothing is written behind it.  Takes the place of the copy and the wait with which the reference reads

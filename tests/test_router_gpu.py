@@ -1173,3 +1173,28 @@ def test_words_read_back_by_the_host(n):
             shifted = on_device + 0  # queued behind the work
             assert _lib.native().int_list(shifted) == view.tolist()
             assert _lib.native().int_list(on_device) == view.tolist()
+
+
+@pytest.mark.parametrize("T,E,dtype", [
+    (1, 1, torch.float32), (5, 8, torch.float16), (128, 64, torch.bfloat16), (129, 64, torch.float32), (100, 3, torch.bfloat16),
+    (777, 5, torch.float32), (8192, 8, torch.float16), (40000, 33, torch.bfloat16), (100352, 8, torch.float16), (131075, 2, torch.float32),
+])
+def test_top1_to_capacity_is_the_mask_throttled(brt_mod, T, E, dtype):
+    """One read of the scores gives what the hot mask and the throttle give one after the other: ties, NaN and
+    infinities among the scores, capacities of nothing, of some and of all cells."""
+    c_router = brt_mod[1]
+    gen = torch.Generator().manual_seed(T + E)
+    score = torch.randint(-3, 4, (T, E), generator=gen).float()  # many ties
+    score[::5] = torch.randn(score[::5].shape, generator=gen)
+    for at, v in ((0, float("nan")), (T // 2, float("inf")), (T - 1, -float("inf"))):
+        score[at, (at * 7) % E] = v
+    score[T // 3] = -float("inf")
+    score = score.to(dtype).cuda()
+    for capacity in (0, 1, max(1, T // E), T, 2**31 - 1):
+        mask = c_router.topk_hot_mask(score, 1)
+        limit = torch.full((E,), capacity, dtype=torch.int32, device="cuda")
+        want, _ = c_router.throttle_hotmask(mask, torch.zeros(E, dtype=torch.int32, device="cuda"), limit)
+        got, capacities = c_router.top1_to_capacity(score, capacity)
+        assert torch.equal(got, want) and torch.equal(capacities, limit)
+    assert c_router.top1_to_capacity(torch.zeros(4, 65, device="cuda"), 2) is None
+    assert c_router.top1_to_capacity(torch.zeros(0, 4, device="cuda"), 2) is None
