@@ -141,6 +141,12 @@ SIGNATURES = {
         [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int,
          _c_int, _c_int, _c_ptr],
     ),
+    "brt_hip_grouped_gemm_f32in_supported": (_c_int, [_c_int] * 6),
+    "brt_hip_grouped_gemm_f32in": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int,
+         _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
+    ),
     "brt_hip_top1_to_capacity": (
         _c_int,
         [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_size, _c_ptr],
@@ -210,7 +216,8 @@ _calls = 0
 
 def call_count() -> int:
     """Calls into the library that queued device work since the process started (every such call is one kernel launch, except index generation, the
-    compact route and the tag-index gather, which are two).  Tests use the difference around a
+    compact route and the tag-index gather, which are two; a GEMM that rounds fp32 rows itself counts
+    as the cast and the GEMM whose work it does).  Tests use the difference around a
     layer to pin how many launches a route costs."""
     return _calls + (_native.calls() if _native is not None else 0)
 

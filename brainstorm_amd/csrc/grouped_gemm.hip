@@ -678,11 +678,26 @@ using namespace brt;
 
 namespace {
 
+// The rule for the ping-pong kernel (its reasons where the kernel is chosen).
+bool wide_tiles_come_in_rounds(const GemmArgs& a) {
+  if (!pingpong_gemm_applies(a) || static_cast<long>(a.P) <= static_cast<long>(a.E) * 160) return false;
+  const long tiles = (static_cast<long>(a.P + 255) / 256 + (a.E + 1) / 2) * ((a.N + 255) / 256);
+  const long cus = device_cus();
+  return tiles >= 2 * cus || (4 * tiles >= 3 * cus && tiles <= cus);
+}
+
+// fp32 rows are rounded by the kernel itself where bf16 rows of that shape would take the few-rows kernel.
+bool takes_f32_rows(int E, int P, int K, int N) {
+  GemmArgs a{};
+  a.E = E; a.P = P; a.K = K; a.N = N;
+  return E > 0 && P > 0 && K > 0 && N > 0 && K % 8 == 0 && N % 8 == 0 && !wide_tiles_come_in_rounds(a) && skinny_gemm_applies(a);
+}
+
 int grouped_gemm_impl(const void* x, const void* const* weights, const void* const* biases, void* out,
                       const int32_t* loads, const int32_t* tags, int entries_per_cell, int E, int P,
                       int T, int K, int N, int act, int gather_in, int scatter_out, void* stream,
                       bool out_is_f32 = false, int32_t* row_tags_out = nullptr,
-                      const float* gates = nullptr, long long* clocks = nullptr) {
+                      const float* gates = nullptr, long long* clocks = nullptr, bool x_is_f32 = false) {
   if (E <= 0 || P < 0 || K <= 0 || N <= 0 || T < 0)
     return fail(BRT_E_INVALID, "bad shape E=%d P=%d T=%d K=%d N=%d", E, P, T, K, N);
   if (K % 8 != 0 || N % 8 != 0)
@@ -693,7 +708,7 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   if ((gather_in || scatter_out) && T == 0) return BRT_OK;
   if (!x || !weights || !out || !loads) return fail(BRT_E_INVALID, "null argument");
   if ((gather_in || scatter_out) && !tags) return fail(BRT_E_INVALID, "gather/scatter need the tag matrix");
-  if (gather_in && static_cast<size_t>(T) * K * 2 > 0x7fffffffull)
+  if (gather_in && static_cast<size_t>(T) * K * (x_is_f32 ? 4 : 2) > 0x7fffffffull)
     return fail(BRT_E_UNSUPPORTED, "gathered input of %d x %d exceeds 2 GiB", T, K);
   if (!aligned(x, 16) || !aligned(out, 16)) return fail(BRT_E_INVALID, "x/out must be 16-byte aligned");
   if (gates != nullptr && (!scatter_out || out_is_f32 || !aligned(gates, 4)))
@@ -726,6 +741,12 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
     a.clocks = clocks;
     return launch_pingpong_gemm(a, act, as_stream(stream));
   }
+  a.x_f32 = x_is_f32;
+  if (x_is_f32) {
+    if (!takes_f32_rows(E, P, K, N))
+      return fail(BRT_E_UNSUPPORTED, "fp32 rows are taken by the few-rows kernel only, not with E=%d P=%d K=%d N=%d", E, P, K, N);
+    return launch_skinny_gemm(a, act, as_stream(stream));
+  }
   // Kernel choice.  Experts that average more than one row block take the ping-pong kernel
   // (grouped_gemm_pingpong.hip), whose 256 x 256 tile moves a third fewer operand bytes per flop,
   // when its tiles come in whole rounds over the CUs: at least two rounds, or one round that most
@@ -738,12 +759,7 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   // the top-2 shape's contracting GEMM (308 tiles on 256 CUs) 162 -> 173 us.  The rule is the same
   // for gathered, scattered and fp32-output rows: a gathering 1024 -> 4096 GEMM with GELU over 32768
   // rows of 16 experts takes 437 us on the 160-row kernel and 336 us here.
-  if (pingpong_gemm_applies(a) && static_cast<long>(P) > static_cast<long>(E) * 160) {
-    const long tiles = (static_cast<long>(P + 255) / 256 + (E + 1) / 2) * ((N + 255) / 256);
-    const long cus = device_cus();
-    if (tiles >= 2 * cus || (4 * tiles >= 3 * cus && tiles <= cus))
-      return launch_pingpong_gemm(a, act, as_stream(stream));
-  }
+  if (wide_tiles_come_in_rounds(a)) return launch_pingpong_gemm(a, act, as_stream(stream));
   if (skinny_gemm_applies(a)) return launch_skinny_gemm(a, act, as_stream(stream));
   if (out_is_f32) {
     if (act == BRT_ACT_GELU) return launch_f32<BRT_ACT_GELU>(a, as_stream(stream));
@@ -831,6 +847,20 @@ __global__ __launch_bounds__(256) void cast_f32_to_bf16_kernel(const float* __re
   }
 }
 }  // namespace
+
+extern "C" int brt_hip_grouped_gemm_f32in_supported(int E, int P, int T, int K, int N, int gather_in) {
+  if (gather_in && static_cast<size_t>(T) * K * 4 > 0x7fffffffull) return 0;
+  return takes_f32_rows(E, P, K, N) ? 1 : 0;
+}
+
+extern "C" int brt_hip_grouped_gemm_f32in(const float* x, const void* const* weights, const void* const* biases, void* out,
+                                          int out_is_f32, const int32_t* loads, const int32_t* tags, int entries_per_cell, int E,
+                                          int P, int T, int K, int N, int act, int gather_in, int32_t* row_tags_out, void* stream) {
+  if (entries_per_cell < 0) return fail(BRT_E_INVALID, "entries per cell must not be negative, got %d", entries_per_cell);
+  if (entries_per_cell > 0 && row_tags_out != nullptr) return fail(BRT_E_INVALID, "row tags come from the tag matrix only");
+  return grouped_gemm_impl(x, weights, biases, out, loads, gather_in ? tags : nullptr, entries_per_cell, E, P, T, K, N, act, gather_in, 0,
+                           stream, out_is_f32 != 0, row_tags_out, nullptr, nullptr, true);
+}
 
 extern "C" int brt_hip_cast_f32_to_bf16(const float* src, void* dst, size_t n, void* stream) {
   if (n == 0) return BRT_OK;

@@ -6,7 +6,7 @@
 namespace brt {
 
 struct GemmArgs {
-  const __bf16* x;
+  const __bf16* x;     // (fp32 where x_f32 is set: few-rows kernel only)
   const __bf16* const* w;
   const __bf16* const* bias;
   __bf16* out;
@@ -19,6 +19,7 @@ struct GemmArgs {
   int tag_div;      // entries per cell (k) of the row-entry vector
   int E, P, K, N, T;
   int plain_out;  // ordinary output stores instead of streaming ones (a small output that is read at once)
+  int x_f32;
   int gather, scatter;  // rows of x / of out are addressed through the tags
   // accumulate form (scatter only): non-null gates turn the store of a row into
   // acc_out[cell] += gate * (the row rounded to bf16), fp32 atomic adds; gate of the row's cell on

@@ -19,6 +19,8 @@
 //     11.2 us; the four wavefronts summing a quarter of K each, which gives other bits, 10.7 us; one
 //     wavefront that loads by itself 18.7 us).  K-steps of 128 with half the barriers change nothing.
 //   - Rows past the expert's load and past N address past the buffer extent: zeros, no request.
+//   - fp32 rows of x (X32) are loaded as they are and rounded to bf16 on their way from LDS to the matrix unit: the cast
+//     kernel and its pass over the rows go (16 experts x 60 rows 512 -> 2048 -> 512 in fp32: a launch each of 3.3 us).
 //   - Every wavefront finds the tile by itself (DPP scan + ballot over the loads, the weight
 //     pointers fetched in the same round trip), so the first weight request leaves two round trips
 //     after the start.  Gathered rows add one, which the weight requests do not wait for.
@@ -33,6 +35,7 @@ namespace brt {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
@@ -73,7 +76,7 @@ __device__ __forceinline__ void wait_loads(int left) {
   switch (left) {
 #define BRT_WAIT(n) case n: wait_loads_but<n>(); break;
     BRT_WAIT(1) BRT_WAIT(2) BRT_WAIT(3) BRT_WAIT(4) BRT_WAIT(5) BRT_WAIT(6) BRT_WAIT(7) BRT_WAIT(8)
-    BRT_WAIT(9) BRT_WAIT(10) BRT_WAIT(11) BRT_WAIT(12)
+    BRT_WAIT(9) BRT_WAIT(10) BRT_WAIT(11) BRT_WAIT(12) BRT_WAIT(13) BRT_WAIT(14) BRT_WAIT(15) BRT_WAIT(16)
 #undef BRT_WAIT
     default: wait_loads_but<0>();
   }
@@ -86,21 +89,24 @@ __device__ __forceinline__ void wait_lds() {
 
 constexpr int kWaves = 4;
 
-template <int XR, int NT, int D>
+template <int XR, int NT, int D, bool X32>
 struct Shape {
-  static constexpr int kXi = XR / 8, kWi = NT * 4;             // load instructions of one K-step: rows of x, weight rows
+  static constexpr int kXRowB = X32 ? 2 * kRowB : kRowB;       // bytes of one row of x in one stage
+  static constexpr int kXRows = 1024 / kXRowB;                 // rows of x that one load instruction fills
+  static constexpr int kXi = XR / kXRows, kWi = NT * 4;        // load instructions of one K-step: rows of x, weight rows
   static constexpr int kXw = kXi / kWaves, kWw = kWi / kWaves;  // ... of one wavefront
   static constexpr int kStage = (kXi + kWi) * 1024;
   static constexpr int kBN = NT * 32;
   static constexpr int kSumRow = kBN * 4 + 16;                 // padded row of the sums on their way out
   static constexpr int kLds = D * kStage > XR * kSumRow ? D * kStage : XR * kSumRow;
   static_assert(XR % 32 == 0 && XR / 32 * NT <= kWaves, "at most one 32 x 32 block per wavefront");
-  static_assert(D >= 2 && (D - 1) * (kXw + kWw) <= 12 && D * kWw <= 12, "the waits count up to 12 loads");
+  static_assert(D >= 2 && (D - 1) * (kXw + kWw) <= 16 && D * kWw <= 16, "the waits count up to 16 loads");
 };
 
-template <int XR, int NT, int D, int ACT, bool ROUTED, bool OUTF32>
+template <int XR, int NT, int D, int ACT, bool ROUTED, bool OUTF32, bool X32>
 __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(GemmArgs a) {
-  using H = Shape<XR, NT, D>;
+  using H = Shape<XR, NT, D, X32>;
+  constexpr int kXB = X32 ? 4 : 2;  // bytes of one element of x
   constexpr int kWi = H::kWi, kXw = H::kXw, kWw = H::kWw, kL = kXw + kWw;
   constexpr int kBlocks = XR / 32 * NT;  // 32 x 32 blocks of the tile, one wavefront each
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -152,11 +158,15 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
   // slot ^ ((row >> 1) & 7) of that row; a chunk past K (the last K-step only) reads as zero.
   const bool gather = ROUTED && a.gather != 0;
   const i32x4 res_w = make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2);
-  const i32x4 res_x = gather ? make_rsrc(a.x, static_cast<size_t>(a.T) * K * 2)
-                             : make_rsrc(a.x + static_cast<size_t>(row0) * K, static_cast<size_t>(a.P - row0) * K * 2);
+  const char* const x_b = reinterpret_cast<const char*>(a.x);
+  const i32x4 res_x = gather ? make_rsrc(x_b, static_cast<size_t>(a.T) * K * kXB)
+                             : make_rsrc(x_b + static_cast<size_t>(row0) * K * kXB, static_cast<size_t>(a.P - row0) * K * kXB);
   const int r8 = lane >> 3;
   const int first_w = wave * kWw, first_x = wave * kXw;  // row groups
   auto chunk = [&](int group) { return (lane & 7) ^ (r8 >> 1) ^ ((group & 1) << 2); };
+  // fp32 rows of x are 16 chunks of 4 elements: lane l lands at slot l & 15 of row l >> 4 and fetches chunk slot ^ (row & 15)
+  const int rx = X32 ? lane >> 4 : r8;
+  auto chunk_x = [&](int group) { return X32 ? (lane & 15) ^ ((group * 4 + rx) & 15) : chunk(group); };
   uint32_t off_w[kWw], off_x[kXw];
 #pragma unroll
   for (int i = 0; i < kWw; ++i) {
@@ -164,19 +174,21 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
     off_w[i] = n0 + row < a.N ? (static_cast<uint32_t>(row) * K + chunk(first_w + i) * 8) * 2 : kOutOfRange;
   }
   const int tail_chunks = K % kBK != 0 ? (K % kBK) / 8 : 8;  // chunks of the last K-step that exist
-  auto fetch = [&](const i32x4& res, uint32_t off, int group, int kt, uint32_t to) {
-    if (kt == k_tiles - 1 && chunk(group) >= tail_chunks) off = kOutOfRange;
-    load_to_lds(res, off, kt * kRowB, to);
+  auto load_w = [&](int s, uint32_t stage, int i) {
+    const bool there = s < k_tiles - 1 || chunk(first_w + i) < tail_chunks;
+    load_to_lds(res_w, there ? off_w[i] : kOutOfRange, s * kRowB, lds0 + stage + (first_w + i) * 1024);
   };
-  auto load_w = [&](int s, uint32_t stage, int i) { fetch(res_w, off_w[i], first_w + i, s, lds0 + stage + (first_w + i) * 1024); };
-  auto load_x = [&](int s, uint32_t stage, int i) { fetch(res_x, off_x[i], first_x + i, s, lds0 + stage + (kWi + first_x + i) * 1024); };
+  auto load_x = [&](int s, uint32_t stage, int i) {
+    const bool there = s < k_tiles - 1 || chunk_x(first_x + i) < (X32 ? 2 : 1) * tail_chunks;
+    load_to_lds(res_x, there ? off_x[i] : kOutOfRange, s * H::kXRowB, lds0 + stage + (kWi + first_x + i) * 1024);
+  };
   const int primed = min(D, k_tiles);
   if (gather) {
     // The words that name this wavefront's rows land in the last stage's room for them (a direct load, so
     // that waiting for it does not wait for the weight requests behind it).
     const uint32_t words = (D - 1) * H::kStage + (kWi + first_x) * 1024;
-    const int row = first_x * 8 + lane;
-    const bool slot_ok = lane < kXw * 8 && row < rows && (a.tag_vector || seat0 + row < a.T);
+    const int row = first_x * H::kXRows + lane;
+    const bool slot_ok = lane < kXw * H::kXRows && row < rows && (a.tag_vector || seat0 + row < a.T);
     const size_t first = a.tag_vector ? static_cast<size_t>(row0) : static_cast<size_t>(seat0) * a.E + e;
     const i32x4 res_t = make_rsrc(a.tags + first, static_cast<size_t>(XR) * (a.tag_vector ? 1 : a.E) * 4);
     load_word_to_lds(res_t, slot_ok ? static_cast<uint32_t>(row) * (a.tag_vector ? 1 : a.E) * 4 : kOutOfRange, lds0 + words);
@@ -186,9 +198,9 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
     wait_loads(primed * kWw);
 #pragma unroll
     for (int i = 0; i < kXw; ++i) {
-      const int word = *reinterpret_cast<const volatile int*>(smem + words + (i * 8 + r8) * 4);
+      const int word = *reinterpret_cast<const volatile int*>(smem + words + (i * H::kXRows + rx) * 4);
       const int cell = cell_of_word(a, word);
-      off_x[i] = cell >= 0 ? (static_cast<uint32_t>(cell) * K + chunk(first_x + i) * 8) * 2 : kOutOfRange;
+      off_x[i] = cell >= 0 ? static_cast<uint32_t>(cell) * K * kXB + chunk_x(first_x + i) * 16 : kOutOfRange;
     }
     wait_lds();
     for (int s = 0; s < primed; ++s)
@@ -197,8 +209,8 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
   } else {
 #pragma unroll
     for (int i = 0; i < kXw; ++i) {
-      const int row = (first_x + i) * 8 + r8;
-      off_x[i] = row < rows ? (static_cast<uint32_t>(row) * K + chunk(first_x + i) * 8) * 2 : kOutOfRange;
+      const int row = (first_x + i) * H::kXRows + rx;
+      off_x[i] = row < rows ? static_cast<uint32_t>(row) * K * kXB + chunk_x(first_x + i) * 16 : kOutOfRange;
     }
     for (int s = 0; s < primed; ++s) {
 #pragma unroll
@@ -215,14 +227,27 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
   const int frag_row = lane & 31, frag_k = lane >> 5;
   const int swz = (frag_row >> 1) & 7;
   const char* const from_w = smem + (block_w * 32 + frag_row) * kRowB;
-  const char* const from_x = smem + kWi * 1024 + (block_x * 32 + frag_row) * kRowB;
+  const char* const from_x = smem + kWi * 1024 + (block_x * 32 + frag_row) * H::kXRowB;
   struct Frags {
-    bf16x8 w[kSub], x[kSub];
+    bf16x8 w[kSub];
+    std::conditional_t<X32, f32x8, bf16x8> x[kSub];
+  };
+  // fp32 rows are rounded to bf16 on their way from LDS (to nearest even, as the cast kernel does)
+  auto x_of = [](const Frags& f, int ks) {
+    if constexpr (X32) return __builtin_convertvector(f.x[ks], bf16x8);
+    else return f.x[ks];
   };
   auto read_frags = [&](Frags& f, uint32_t stage, int ks) {
     const uint32_t at = stage + (((ks * 2 + frag_k) ^ swz) << 4);
     f.w[ks] = *reinterpret_cast<const bf16x8*>(from_w + at);
-    f.x[ks] = *reinterpret_cast<const bf16x8*>(from_x + at);
+    if constexpr (X32) {
+      const int c = (ks * 2 + frag_k) * 2, swz_x = frag_row & 15;
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(from_x + stage + ((c ^ swz_x) << 4));
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(from_x + stage + (((c + 1) ^ swz_x) << 4));
+      f.x[ks] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    } else {
+      f.x[ks] = *reinterpret_cast<const bf16x8*>(from_x + at);
+    }
   };
   // this wavefront's loads issued after the last one of K-step s, once K-steps up to `issued` have been requested
   auto younger = [&](int s, int issued) {
@@ -249,7 +274,7 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
 #pragma unroll
     for (int ks = 0; ks < kSub; ++ks) {
       if constexpr (kMultiply) {
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.w[ks], cur.x[ks], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.w[ks], x_of(cur, ks), acc, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         read_frags(next, ahead, ks);
       }
@@ -349,23 +374,29 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
   }
 }
 
-template <int XR, int NT, int D, int ACT, bool ROUTED, bool OUTF32>
+template <int XR, int NT, int D, int ACT, bool ROUTED, bool OUTF32, bool X32>
 int launch(GemmArgs& a, hipStream_t st) {
-  using H = Shape<XR, NT, D>;
+  using H = Shape<XR, NT, D, X32>;
   a.tiles_n = (a.N + H::kBN - 1) / H::kBN;
   // the sum over experts of ceil(M_e / XR) never exceeds P / XR + min(E, P)
   const long blocks = (static_cast<long>(a.P) + XR - 1) / XR + std::min(a.E, a.P);
-  auto* fn = &grouped_gemm_skinny_kernel<XR, NT, D, ACT, ROUTED, OUTF32>;
+  auto* fn = &grouped_gemm_skinny_kernel<XR, NT, D, ACT, ROUTED, OUTF32, X32>;
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(fn), H::kLds); rc != BRT_OK) return rc;
   hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks * a.tiles_n)), dim3(kWaves * kWave), H::kLds, st, a);
   return check_launch("grouped_gemm_skinny_kernel");
 }
 
+template <int XR, int NT, int D, int ACT, bool X32>
+int launch_of(GemmArgs& a, hipStream_t st) {
+  const bool f32 = a.out_f32 != nullptr;
+  if (a.tags != nullptr) return f32 ? launch<XR, NT, D, ACT, true, true, X32>(a, st) : launch<XR, NT, D, ACT, true, false, X32>(a, st);
+  return f32 ? launch<XR, NT, D, ACT, false, true, X32>(a, st) : launch<XR, NT, D, ACT, false, false, X32>(a, st);
+}
+
 template <int XR, int NT, int D, int ACT>
 int launch_form(GemmArgs& a, hipStream_t st) {
-  const bool f32 = a.out_f32 != nullptr;
-  if (a.tags != nullptr) return f32 ? launch<XR, NT, D, ACT, true, true>(a, st) : launch<XR, NT, D, ACT, true, false>(a, st);
-  return f32 ? launch<XR, NT, D, ACT, false, true>(a, st) : launch<XR, NT, D, ACT, false, false>(a, st);
+  // (fp32 rows take twice the room: three stages of 64 x 64 still leave room for two workgroups on a CU)
+  return a.x_f32 ? launch_of<XR, NT, XR == 64 ? 3 : D, ACT, true>(a, st) : launch_of<XR, NT, D, ACT, false>(a, st);
 }
 
 template <int XR, int NT, int D>

@@ -466,13 +466,25 @@ PyObject* combine_by_rows(const Args& a) {  // in_data, path_ids, seat_rows, wei
 // ---- grouped GEMM ------------------------------------------------------------------------------------
 // x, out, weight_table, bias_table, loads, in_features, out_features, activation code, tags, gather, scatter,
 // rows or None, row_entries, entries_per_cell, row_tags_out, gates
-PyObject* grouped_linear(const Args& a) {
-  const Tensor x = a.tensor(0), out = a.tensor(1), weights = a.tensor(2), biases = a.tensor_or_none(3), loads = a.tensor(4);
+Tensor rounded_to_bf16(const Tensor& given) {
+  const Tensor in = dense(given);
+  const c10::DeviceGuard guard(in.device());
+  Tensor out = empty(in.sizes(), at::kBFloat16, in);
+  if (in.numel() > 0) check(brt_hip_cast_f32_to_bf16(fptr(in), ptr(out), in.numel(), stream_of(in)));
+  return out;
+}
+
+// takes_f32: fp32 rows of x are taken too, rounded to bf16 by the GEMM itself where its kernel does that
+PyObject* grouped_linear_of(const Args& a, bool takes_f32) {
+  Tensor x = a.tensor(0);
+  const bool f32_rows = takes_f32 && x.scalar_type() == at::kFloat && x.is_cuda();
+  if (f32_rows) x = dense(x);
+  const Tensor out = a.tensor(1), weights = a.tensor(2), biases = a.tensor_or_none(3), loads = a.tensor(4);
   const int64_t K = a.integer(5), N = a.integer(6), act = a.integer(7);
   const Tensor tags = a.tensor_or_none(8), entries = a.tensor_or_none(12), tags_out = a.tensor_or_none(14), gates = a.tensor_or_none(15);
   const bool gather = a.flag(9), scatter = a.flag(10), routed = gather || scatter;
   const int64_t k = a.integer(13);
-  if (x.scalar_type() != at::kBFloat16 || (out.scalar_type() != at::kBFloat16 && out.scalar_type() != at::kFloat))
+  if ((x.scalar_type() != at::kBFloat16 && !f32_rows) || (out.scalar_type() != at::kBFloat16 && out.scalar_type() != at::kFloat))
     not_implemented("the grouped GEMM computes in bf16 (fp32 accumulation); the output is bf16 or fp32");
   const bool f32_out = out.scalar_type() == at::kFloat;
   if (gates.defined()) {
@@ -518,6 +530,17 @@ PyObject* grouped_linear(const Args& a) {
   const void* const* const w = static_cast<const void* const*>(ptr(weights));
   const void* const* const b = static_cast<const void* const*>(ptr(biases));
   const int E = static_cast<int>(loads.numel());
+  if (f32_rows) {
+    if (!scatter && !gates.defined() && brt_hip_grouped_gemm_f32in_supported(E, rows, cells, K, N, gather) == 1) {
+      if (gather && !by_rows && tags_out.defined() && (tags_out.scalar_type() != at::kInt || tags_out.numel() < rows || !tags_out.is_cuda()))
+        runtime_error("row_tags_out must be an int32 device vector with one entry per row");
+      ++g_calls;  // the rounding, whoever does it: a layer counts the same ops for any number of rows
+      check(brt_hip_grouped_gemm_f32in(fptr(x), w, b, ptr(out), f32_out, iptr(loads), gather ? iptr(by_rows ? entries : tags) : nullptr,
+                                       by_rows ? k : 0, E, rows, cells, K, N, act, gather, by_rows ? nullptr : iptr(tags_out), st));
+      return none();
+    }
+    x = rounded_to_bf16(x);
+  }
   if (gates.defined()) {
     if (gates.numel() != cells * (by_rows ? k : E))
       runtime_error("gates must hold one weight per cell and path (tags) or per entry (row_entries)");
@@ -542,6 +565,9 @@ PyObject* grouped_linear(const Args& a) {
   }
   return none();
 }
+
+PyObject* grouped_linear(const Args& a) { return grouped_linear_of(a, false); }
+PyObject* grouped_linear_f32(const Args& a) { return grouped_linear_of(a, true); }
 
 // operands (list or tuple), first, step, branches used, what -> (fp32, key): the tensors operands[first::step],
 // of which the used ones are all contiguous bf16 or all fp32, and what tells whether they are still the same
@@ -584,11 +610,7 @@ PyObject* cast_f32_to_bf16(const Args& a) {
   const Tensor given = a.tensor(0);
   if (given.scalar_type() != at::kFloat)
     runtime_error(std::string("the cast kernel reads fp32, got ") + c10::toString(given.scalar_type()));
-  const Tensor in = dense(given);
-  const c10::DeviceGuard guard(in.device());
-  Tensor out = empty(in.sizes(), at::kBFloat16, in);
-  if (in.numel() > 0) check(brt_hip_cast_f32_to_bf16(fptr(in), ptr(out), in.numel(), stream_of(in)));
-  return wrap(out);
+  return wrap(rounded_to_bf16(given));
 }
 
 // ---- host reads --------------------------------------------------------------------------------------
@@ -708,7 +730,7 @@ PyMethodDef methods[] = {
     BRT_ENTRY(generate, 5),         BRT_ENTRY(route_and_dispatch, 7),  BRT_ENTRY(route_by_path, 7),
     BRT_ENTRY(dispatch, 12),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
     BRT_ENTRY(top1_to_capacity, 2), BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 7),     BRT_ENTRY(grouped_linear, 16),
-    BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5),        BRT_ENTRY(int_list, 1),
+    BRT_ENTRY(grouped_linear_f32, 16), BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5),        BRT_ENTRY(int_list, 1),
     BRT_ENTRY(unique_tags, 1),      BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "brt_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -61,10 +61,22 @@ def grouped_linear(x: torch.Tensor, out: torch.Tensor, weight_table: torch.Tenso
     adds, so ``out`` must hold zeros (or what the sums are added to) before the call.  Equal to
     ``combine_with_indices_and_loads`` on the separate GEMM's output: bit for bit with at most two
     paths per cell, to the last bits of an fp32 sum taken in another order with more."""
-    _lib.native().grouped_linear(
-        x, out, weight_table, bias_table, loads, in_features, out_features, _ACT[activation], tags, gather,
-        scatter, rows, row_entries, int(entries_per_cell), row_tags_out, gates)
+    return _launch(_lib.native().grouped_linear, x, out, weight_table, bias_table, loads, in_features, out_features, activation,
+                   tags=tags, gather=gather, scatter=scatter, rows=rows, row_entries=row_entries,
+                   entries_per_cell=entries_per_cell, row_tags_out=row_tags_out, gates=gates)
+
+
+def _launch(op, x, out, weight_table, bias_table, loads, in_features, out_features, activation, *, tags=None, gather=False,
+            scatter=False, rows=None, row_entries=None, entries_per_cell=1, row_tags_out=None, gates=None) -> torch.Tensor:
+    op(x, out, weight_table, bias_table, loads, in_features, out_features, _ACT[activation], tags, gather,
+       scatter, rows, row_entries, int(entries_per_cell), row_tags_out, gates)
     return out
+
+
+def _linear(x, out, *args, **kwargs) -> torch.Tensor:
+    """:func:`grouped_linear` that takes fp32 rows of ``x`` too: they are rounded to bf16 first, by the kernel for few
+    rows itself and by the cast kernel for the others."""
+    return _launch(_lib.native().grouped_linear_f32, x, out, *args, **kwargs)
 
 
 def _to_bf16(t: torch.Tensor) -> torch.Tensor:
@@ -149,21 +161,20 @@ class GroupedLinearKernel:
         if state is not None:
             # the rows of a deferred dispatch: read from the cells through the route
             route = state.route
-            cells = state.cells if state.cells.dtype == torch.bfloat16 else _to_bf16(state.cells)
+            cells = state.cells
             if isinstance(route, c_router.CompactRoute):  # rows named by the row-entry vector
-                grouped_linear(cells, out, weights, biases, loads, self.in_features, self.out_features,
-                               self.activation, row_entries=route.row_entries,
-                               entries_per_cell=route.k, gather=True, rows=out.shape[0])
+                _linear(cells, out, weights, biases, loads, self.in_features, self.out_features,
+                        self.activation, row_entries=route.row_entries,
+                        entries_per_cell=route.k, gather=True, rows=out.shape[0])
                 return
             row_tags = torch.empty((out.shape[0],), dtype=torch.int32, device=out.device)
-            grouped_linear(cells, out, weights, biases, loads, self.in_features, self.out_features,
-                           self.activation, tags=route.indices, gather=True,
-                           rows=out.shape[0], row_tags_out=row_tags)
+            _linear(cells, out, weights, biases, loads, self.in_features, self.out_features,
+                    self.activation, tags=route.indices, gather=True,
+                    rows=out.shape[0], row_tags_out=row_tags)
             route.row_tags, route.row_tags_stride = row_tags, 0
             return
-        if x.dtype == torch.float32:
-            x = _to_bf16(x)  # (a deferred buffer is filled by this read)
-        grouped_linear(x, out, weights, biases, loads, self.in_features, self.out_features, self.activation)
+        # (a deferred buffer is filled by this read)
+        _linear(x, out, weights, biases, loads, self.in_features, self.out_features, self.activation)
 
     def _store_to_cells(self, x, weights, biases, loads, route_loads, residual):
         """The GEMM whose rows go straight to their cells in ``residual`` (combine folded in)."""

@@ -454,6 +454,19 @@ int brt_hip_combine_by_rows_gated(const void* src, void* dst, const void* gates,
                                   int P, int is_residual, int in_dtype, int out_dtype, void* stream);
 
 /*
+ * brt_hip_grouped_gemm / _f32out / _routed / _routed_f32out / _by_rows on fp32 rows of x (16-byte aligned), which the
+ * kernel rounds to bf16 itself: the bits of brt_hip_cast_f32_to_bf16 followed by the bf16 form, without that pass.
+ * gather_in as in the routed forms, from the tag matrix (entries_per_cell = 0; row_tags_out as there) or the row
+ * entries (entries_per_cell = k); else tags is ignored.  Only for shapes that the kernel for few rows takes:
+ * brt_hip_grouped_gemm_f32in_supported says which (1), others are refused (BRT_E_UNSUPPORTED).
+ */
+int brt_hip_grouped_gemm_f32in_supported(int E, int P, int T, int K, int N, int gather_in);
+int brt_hip_grouped_gemm_f32in(const float* x, const void* const* weights, const void* const* biases,
+                               void* out, int out_is_f32, const int32_t* loads, const int32_t* tags,
+                               int entries_per_cell, int E, int P, int T, int K, int N, int act,
+                               int gather_in, int32_t* row_tags_out, void* stream);
+
+/*
  * brt_hip_topk_hot_mask with k = 1 and brt_hip_throttle_hotmask from a zero prefix with one capacity for all paths, in two
  * launches and one read of the scores: mask [T,E] the hot mask, out [T,E] what the capacity leaves of it, capacities [E] the
  * capacity of every path (what python/brt/router/protocol/swin_moe.py:101-126 makes of them).  mask and out must not

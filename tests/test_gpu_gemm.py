@@ -1044,3 +1044,55 @@ def test_timed_grouped_gemm_gives_the_same_rows_and_plausible_clocks():
                                         d_loads.data_ptr(), E, P, 72, N, ACT["none"], clocks.data_ptr(), st) == -4
     assert L.brt_hip_grouped_gemm_timed(x.data_ptr(), wt.data_ptr(), bt.data_ptr(), timed.data_ptr(),
                                         d_loads.data_ptr(), E, P, K, N, ACT["none"], None, st) == -1
+
+
+@pytest.mark.parametrize("E,rows,K,N,act,bias", [
+    (8, 3, 768, 3072, "gelu", False), (8, 3, 3072, 768, None, True), (4, 30, 72, 320, "relu", True),  # 32-row tiles, K tails
+    (16, 60, 512, 2048, "gelu", True), (16, 60, 2048, 512, None, False), (8, 120, 136, 776, "gelu", False),  # 64 rows, N tails
+    (32, 6, 8, 64, None, True), (1, 1, 64, 8, None, False), (5, 33, 1288, 264, "gelu", True),
+    (6, 1000, 512, 1024, "gelu", True), (2, 4000, 256, 4096, None, False),  # shapes that are cast first
+])
+def test_fp32_rows_are_rounded_by_the_kernel(E, rows, K, N, act, bias):
+    """fp32 rows give the bits of the cast kernel and the bf16 form: plain, gathered by row entries and by the tag
+    matrix, into bf16 and fp32; ragged loads with empty experts; values whose rounding ties, overflows or is lost."""
+    from brainstorm_amd import _lib, jit
+    from brainstorm_amd._C import router as c_router
+    from routing_cases import topk_mask
+
+    T = E * rows
+    mask, _ = topk_mask(T, E, 1, seed=T + K)
+    g = torch.Generator().manual_seed(K + N)
+    x = torch.randn(T, K, generator=g)
+    x[0, : min(K, 8)] = torch.tensor([0.0, -0.0, 1.00390625, 1.01171875, 3.4e38, -3.4e38, 1e-40, -1e-41])[: min(K, 8)]
+    if rows > 2:
+        x[T // 2, 0], x[T // 2 + 1, K - 1] = float("inf"), float("nan")
+    x = x.cuda()
+    ws, table = _expert_tables(E, K, N, 3)
+    biases = [torch.randn(N, generator=g).to(torch.bfloat16).cuda() for _ in range(E)] if bias else None
+    bias_table = torch.tensor([b.data_ptr() for b in biases], dtype=torch.int64, device="cuda") if bias else None
+    d_mask = torch.from_numpy(mask).cuda()
+    ids, _ = c_router.gate_topk(d_mask.float(), 1)
+    loads, _, _, row_entries = c_router.route_by_path(ids, E, None, False, rows=T)
+    tags, tag_loads = c_router.generate_indices_and_loads(d_mask, None, False, False, True)
+    assert torch.equal(loads, tag_loads)
+
+    def bits(t):
+        return t.view(torch.int16 if t.dtype == torch.bfloat16 else torch.int32)
+
+    half = _lib.native().cast_f32_to_bf16(x)
+    y, y_half = c_router.dispatch_by_rows(x, row_entries, 1), c_router.dispatch_by_rows(half, row_entries, 1)
+    for dtype in (torch.bfloat16, torch.float32):
+        for form in ({}, {"tags": tags, "gather": True}, {"row_entries": row_entries, "gather": True}):
+            if dtype == torch.float32 and "row_entries" in form:
+                continue
+            got, want = (torch.full((T, N), 7.0, dtype=dtype, device="cuda") for _ in range(2))
+            tags_of = [torch.full((T,), -7, dtype=torch.int32, device="cuda") for _ in range(2)]
+            extra = [dict(form, rows=T) if form else {} for _ in range(2)]
+            if "tags" in form:
+                extra[0]["row_tags_out"], extra[1]["row_tags_out"] = tags_of
+            jit._linear(x if form else y, got, table, bias_table, loads, K, N, act, **extra[0])
+            jit.grouped_linear(half if form else y_half, want, table, bias_table, loads, K, N, act, **extra[1])
+            assert torch.equal(bits(got), bits(want)) and torch.equal(*tags_of)
+    with pytest.raises(NotImplementedError):
+        jit.grouped_linear(y, got, table, bias_table, loads, K, N, act)
+    del ws
