@@ -10,6 +10,7 @@ router.cc:78; identical when no stream context is active).
 """
 from __future__ import annotations
 
+import itertools
 from typing import List, Optional, Tuple
 
 import torch
@@ -286,6 +287,7 @@ def dispatch_with_indices_and_loads(
     *,
     route: Optional[Route] = None,
     rows: Optional[int] = None,
+    host_loads: Optional[List[int]] = None,
 ) -> List[torch.Tensor]:
     """router.cc:131-273.  Returns ``[out]`` or ``[out, new_tags]``.  ``route`` (keyword only,
     not in the reference): the :class:`Route` the indices came from; the kernel then zero-fills
@@ -294,7 +296,7 @@ def dispatch_with_indices_and_loads(
     bound of ``sum(loads)`` known to the caller; the output then has that many rows (those past
     the loads are zero) and the loads are not read back to the host (router.cc:197-201 sizes
     the output from ``loads.sum().item()``, which stalls the stream; that is what happens without
-    ``rows``)."""
+    ``rows``).  ``host_loads`` (likewise): the values of ``loads``, where the caller has just read them."""
     _check_on_device(in_data, "in_data")
     _check_on_device(route_indices, "route_indices")
     _check_int32(route_indices, "route_indices")
@@ -321,7 +323,7 @@ def dispatch_with_indices_and_loads(
     elif rows is not None:
         total = int(rows)
     else:
-        total = sum(native.int_list(loads))
+        total = sum(native.int_list(loads) if host_loads is None else host_loads)
     # with the true counts the kernel writes every row up to sum(loads) itself; rows past that
     # (an upper bound was given) have no writer, and their tags start at zero
     clear = counts is None or (rows is not None and not max_path_padding)
@@ -332,6 +334,11 @@ def dispatch_with_indices_and_loads(
     if hidden_tags:
         route.row_tags, route.row_tags_stride = new_tags, mpl
     return [out, new_tags] if tag_generating else [out]
+
+
+def loads_on_host(loads: torch.Tensor) -> List[int]:
+    """The values of an int32 loads vector (one wait for the stream's work so far)."""
+    return _lib.native().int_list(loads)
 
 
 def _dispatch_of_no_cells(in_data, route_indices, tag_generating, is_1d_routing):
@@ -418,29 +425,30 @@ def split_fused_cells_to_paths(
     is_load_split: bool = False,
     is_tag_split: bool = False,
     tags: Optional[torch.Tensor] = None,
+    *,
+    host_loads: Optional[List[int]] = None,
 ) -> List[List[torch.Tensor]]:
-    """router.cc:285-335: per-path views (``narrow``) of the fused buffer."""
+    """router.cc:285-335: per-path views (``narrow``) of the fused buffer.  ``host_loads`` (keyword only,
+    not in the reference): the values of ``loads``, where the caller has just read them."""
     path_num = loads.numel()
     if is_tag_split:
         is_load_split = True
         if tags is None:
             raise RuntimeError("is_tag_split needs tags")
-    datas, load_list, tag_list = [], [], []
     if max_path_padding:
-        stride = in_data.size(0) // path_num
-        bounds = [(i * stride, stride) for i in range(path_num)]
+        rows = [in_data.size(0) // path_num] * path_num
+    elif host_loads is not None:
+        rows = host_loads
     else:
-        host_loads = loads.cpu().tolist()
-        bounds, start = [], 0
-        for load in host_loads:
-            bounds.append((start, load))
-            start += load
-    for i, (start, length) in enumerate(bounds):
-        datas.append(in_data.narrow(0, start, length))
-        if is_load_split:
-            load_list.append(loads.narrow(0, i, 1))
-        if is_tag_split:
-            tag_list.append(tags.narrow(0, start, length))
+        rows = _lib.native().int_list(loads) if loads.dtype == torch.int32 and loads.dim() == 1 else loads.cpu().tolist()
+    if type(in_data) is torch.Tensor and type(loads) is torch.Tensor and (tags is None or type(tags) is torch.Tensor):
+        datas, load_list, tag_list = _lib.native().split_rows(
+            in_data, rows, loads if is_load_split else None, tags if is_tag_split else None)
+    else:
+        starts = [0, *itertools.accumulate(rows)]
+        datas = [in_data.narrow(0, s, n) for s, n in zip(starts, rows)]
+        load_list = [loads.narrow(0, i, 1) for i in range(len(rows))] if is_load_split else []
+        tag_list = [tags.narrow(0, s, n) for s, n in zip(starts, rows)] if is_tag_split else []
     if is_tag_split:
         return [datas, load_list, tag_list]
     if is_load_split:
@@ -574,8 +582,7 @@ def _combine_with_tags(in_data, route_indices, out_data, ever_padded, tags):
         if ever_padded and int(tags_value[0].item()) == 0:
             result = result.narrow(0, 1, n - 1)
             tags_value = tags_value.narrow(0, 1, n - 1)
-    out_loads = torch.tensor([tags_value.numel()], dtype=torch.int32, device=in_data.device)
-    return [result, tags_value, out_loads]
+    return [result, tags_value, _lib.native().one_value(tags_value.numel(), in_data)]
 
 
 def _sum_rows_by_index(in_data, index, n, shape):
@@ -589,16 +596,7 @@ def _sum_rows_by_index(in_data, index, n, shape):
         expanded = index.view(-1, 1).repeat(1, cell).view_as(in_data)
         zeros = torch.zeros(shape, dtype=in_data.dtype, device=in_data.device)
         return torch.scatter_reduce(zeros, 0, expanded, in_data, "sum")
-    in_data = in_data.contiguous()
-    index = index.contiguous()
-    cell = in_data.numel() // P
-    result = torch.empty(shape, dtype=in_data.dtype, device=in_data.device)
-    ws_bytes = _lib.lib().brt_hip_combine_by_index_workspace_bytes(P, n)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=in_data.device)
-    _lib.check(_lib.lib().brt_hip_combine_by_index(
-        _ptr(in_data), _ptr(result), _ptr(index), 32 if index.dtype == torch.int32 else 64, P, cell,
-        n, _ptr(ws), ws_bytes, _DT[in_data.dtype], _DT[in_data.dtype], _stream()))
-    return result
+    return _lib.native().sum_rows_by_index(in_data, index, n)
 
 
 # legacy name (sample/cpp/router.ipynb:258-266) of the seat-index combine

@@ -15,6 +15,7 @@
 #include <ATen/core/CachingHostAllocator.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/full.h>
 #include <ATen/ops/zeros.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -705,6 +706,103 @@ PyObject* unique_tags(const Args& a) {
   return tuple(wrap(unique.narrow(0, 0, v[0])), wrap(inverse), lo, hi);
 }
 
+// ---- tensors that carry a route ----------------------------------------------------------------------
+// (neither reads the rows: a buffer that is not filled yet stays so)
+const Tensor& as_it_is(PyObject* o) {
+  if (!THPVariable_Check(o)) throw Raised(PyExc_TypeError, "a tensor is expected");
+  return THPVariable_Unpack(o);
+}
+
+// t.as_subclass(torch.Tensor) without a turn through __torch_function__
+PyObject* plain(const Args& a) { return wrap(as_it_is(a.v[0]).alias()); }
+
+// t.as_subclass(class), likewise
+PyObject* of_class(const Args& a) {
+  if (!PyType_Check(a.v[1])) throw Raised(PyExc_TypeError, "a class is expected");
+  return THPVariable_Wrap(as_it_is(a.v[0]).alias(), reinterpret_cast<PyTypeObject*>(a.v[1]));
+}
+
+// rows, columns, dtype, like -> an uninitialised [rows, columns] matrix on like's device
+PyObject* matrix(const Args& a) {
+  const Tensor& like = as_it_is(a.v[3]);
+  at::ScalarType type = like.scalar_type();
+  a.dtype(2, &type);
+  if (!like.is_cuda()) runtime_error("a device tensor is expected");
+  return wrap(empty({a.integer(0), a.integer(1)}, type, like));
+}
+
+// tensor, class, tag stack, load stack, extra attributes (a dict or None): tensor.as_subclass(class) with the three in
+// its dictionary, the last as a copy
+PyObject* grid(const Args& a) {
+  static PyObject* const keys[3] = {PyUnicode_InternFromString("cell_tag_stack"), PyUnicode_InternFromString("cell_load_stack"),
+                                    PyUnicode_InternFromString("cell_extra_attr_dict")};
+  if (!PyType_Check(a.v[1])) throw Raised(PyExc_TypeError, "a class is expected");
+  PyObject* const made = THPVariable_Wrap(as_it_is(a.v[0]).alias(), reinterpret_cast<PyTypeObject*>(a.v[1]));
+  PyObject* const attrs = made != nullptr ? PyObject_GenericGetDict(made, nullptr) : nullptr;
+  PyObject* const extra = attrs == nullptr ? nullptr : PyDict_Check(a.v[4]) ? PyDict_Copy(a.v[4]) : PyDict_New();
+  const bool done = extra != nullptr && PyDict_SetItem(attrs, keys[0], a.v[2]) == 0 && PyDict_SetItem(attrs, keys[1], a.v[3]) == 0 &&
+                    PyDict_SetItem(attrs, keys[2], extra) == 0;
+  Py_XDECREF(extra);
+  Py_XDECREF(attrs);
+  if (!done) {
+    Py_XDECREF(made);
+    throw Raised(nullptr, "");
+  }
+  return made;
+}
+
+// data, rows of every path (a list), loads or None, tags or None -> the three as lists of views by path (an empty
+// list for None)
+PyObject* split_rows(const Args& a) {
+  const Tensor data = a.tensor(0), loads = a.tensor_or_none(2), tags = a.tensor_or_none(3);
+  if (!PyList_Check(a.v[1])) throw Raised(PyExc_TypeError, "a list of rows is expected");
+  const Py_ssize_t paths = PyList_GET_SIZE(a.v[1]);
+  std::vector<int64_t> rows(paths);
+  for (Py_ssize_t i = 0; i < paths; ++i) {
+    rows[i] = PyLong_AsLong(PyList_GET_ITEM(a.v[1], i));
+    if (rows[i] == -1 && PyErr_Occurred()) throw Raised(nullptr, "");
+  }
+  std::vector<Tensor> views[3];
+  int64_t start = 0;
+  for (Py_ssize_t i = 0; i < paths; ++i) {
+    views[0].push_back(data.narrow(0, start, rows[i]));
+    if (loads.defined()) views[1].push_back(loads.narrow(0, i, 1));
+    if (tags.defined()) views[2].push_back(tags.narrow(0, start, rows[i]));
+    start += rows[i];
+  }
+  PyObject* lists[3];
+  for (int k = 0; k < 3; ++k) {
+    lists[k] = PyList_New(views[k].size());
+    for (size_t i = 0; i < views[k].size(); ++i) PyList_SET_ITEM(lists[k], i, wrap(std::move(views[k][i])));
+  }
+  return tuple(lists[0], lists[1], lists[2]);
+}
+
+// in_data, index, rows of the result: zeros(rows, ...) with in_data's rows added at their index, in ascending row order
+PyObject* sum_rows_by_index(const Args& a) {
+  const Tensor given = a.tensor(0), index_given = a.tensor(1);
+  const Tensor in = dense(given), index = dense(index_given);
+  on_device(in, "in_data"), on_device(index, "route_indices");
+  const int type = data_type(in, "data type");
+  if (index.scalar_type() != at::kInt && index.scalar_type() != at::kLong) runtime_error("route_indices must be int32 or int64");
+  const int64_t P = in.size(0), n = a.integer(2);
+  if (index.numel() != P) runtime_error("one index per row is needed");
+  const c10::DeviceGuard guard(in.device());
+  Tensor out = empty(rows_of(in, n), in.scalar_type(), in);
+  const size_t bytes = brt_hip_combine_by_index_workspace_bytes(P, n);
+  const Tensor ws = scratch(bytes, in);
+  check(brt_hip_combine_by_index(ptr(in), ptr(out), ptr(index), index.scalar_type() == at::kInt ? 32 : 64, P, divided(in.numel(), P), n,
+                                 ptr(ws), ws.numel(), type, type, stream_of(in)));
+  return wrap(out);
+}
+
+// value, like -> [value] as an int32 vector on like's device, without a wait
+PyObject* one_value(const Args& a) {
+  const Tensor& like = as_it_is(a.v[1]);
+  const c10::DeviceGuard guard(like.device());
+  return wrap(at::full({1}, static_cast<int64_t>(a.integer(0)), at::TensorOptions().dtype(at::kInt).device(like.device())));
+}
+
 PyObject* calls(const Args&) { return PyLong_FromUnsignedLongLong(g_calls); }
 
 template <PyObject* (*FN)(const Args&), int N>
@@ -731,7 +829,9 @@ PyMethodDef methods[] = {
     BRT_ENTRY(dispatch, 12),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
     BRT_ENTRY(top1_to_capacity, 2), BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 7),     BRT_ENTRY(grouped_linear, 16),
     BRT_ENTRY(grouped_linear_f32, 16), BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5),        BRT_ENTRY(int_list, 1),
-    BRT_ENTRY(unique_tags, 1),      BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
+    BRT_ENTRY(plain, 1),            BRT_ENTRY(of_class, 2),            BRT_ENTRY(matrix, 4),
+    BRT_ENTRY(grid, 5),                BRT_ENTRY(split_rows, 4),
+    BRT_ENTRY(sum_rows_by_index, 3), BRT_ENTRY(one_value, 2),         BRT_ENTRY(unique_tags, 1),      BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "brt_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -61,22 +61,19 @@ def grouped_linear(x: torch.Tensor, out: torch.Tensor, weight_table: torch.Tenso
     adds, so ``out`` must hold zeros (or what the sums are added to) before the call.  Equal to
     ``combine_with_indices_and_loads`` on the separate GEMM's output: bit for bit with at most two
     paths per cell, to the last bits of an fp32 sum taken in another order with more."""
-    return _launch(_lib.native().grouped_linear, x, out, weight_table, bias_table, loads, in_features, out_features, activation,
-                   tags=tags, gather=gather, scatter=scatter, rows=rows, row_entries=row_entries,
-                   entries_per_cell=entries_per_cell, row_tags_out=row_tags_out, gates=gates)
-
-
-def _launch(op, x, out, weight_table, bias_table, loads, in_features, out_features, activation, *, tags=None, gather=False,
-            scatter=False, rows=None, row_entries=None, entries_per_cell=1, row_tags_out=None, gates=None) -> torch.Tensor:
-    op(x, out, weight_table, bias_table, loads, in_features, out_features, _ACT[activation], tags, gather,
-       scatter, rows, row_entries, int(entries_per_cell), row_tags_out, gates)
+    _lib.native().grouped_linear(
+        x, out, weight_table, bias_table, loads, in_features, out_features, _ACT[activation], tags, gather,
+        scatter, rows, row_entries, int(entries_per_cell), row_tags_out, gates)
     return out
 
 
-def _linear(x, out, *args, **kwargs) -> torch.Tensor:
+def _linear(x, out, weight_table, bias_table, loads, in_features, out_features, activation, *, tags=None, gather=False,
+            rows=None, row_entries=None, entries_per_cell=1, row_tags_out=None) -> None:
     """:func:`grouped_linear` that takes fp32 rows of ``x`` too: they are rounded to bf16 first, by the kernel for few
     rows itself and by the cast kernel for the others."""
-    return _launch(_lib.native().grouped_linear_f32, x, out, *args, **kwargs)
+    _lib.native().grouped_linear_f32(
+        x, out, weight_table, bias_table, loads, in_features, out_features, _ACT[activation], tags, gather,
+        False, rows, row_entries, entries_per_cell, row_tags_out, None)
 
 
 def _to_bf16(t: torch.Tensor) -> torch.Tensor:

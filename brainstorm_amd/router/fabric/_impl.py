@@ -12,6 +12,7 @@ import numpy as np
 import torch
 import torch.nn as nn
 
+from brainstorm_amd import _lib
 from brainstorm_amd._C import router as c_router
 from brainstorm_amd.router.protocol._impl import CompactHotMask
 from brainstorm_amd.runtime.deferred import lazy_tensor
@@ -243,14 +244,14 @@ class DispatchFabric(FabricBase):
     def _defers(self, in_flows, runtime_capacities, hot_mask) -> bool:
         return False  # only the fused fabric can leave the dispatch to the expert kernel
 
-    def _dispatch_flow(self, flow_idx, flow_data, flow_tag, route_indices, loads, score):
+    def _dispatch_flow(self, flow_idx, flow_data, flow_tag, route_indices, loads, score, host_loads=None):
         # positional layout of the reference call (generic.py:127-137): the 5th
         # argument is tag_generating, seat indices are always what is dispatched with
         return c_router.dispatch_with_indices_and_loads(
             flow_data, route_indices, loads, score if self.transforms[flow_idx] else None,
             self.is_tag_index, flow_tag, self.max_path_padding, self.max_path_load,
             self.route_logics[flow_idx] == "1d", route=self._route,
-            rows=self._static_rows(flow_data, route_indices))
+            rows=self._static_rows(flow_data, route_indices), host_loads=host_loads)
 
     def _static_rows(self, flow_data, route_indices) -> Optional[int]:
         return None  # size the output from the loads, as the reference does
@@ -258,22 +259,27 @@ class DispatchFabric(FabricBase):
     def dispatch(self, in_flows, route_indices, loads, score):
         all_out_flows = []
         path_num = route_indices.size(1)
+        # the rows are sized and split by the same loads: one read-back for both, and for all flows
+        host_loads = None
+        if not self.max_path_padding and loads.dtype == torch.int32 and loads.dim() == 1:
+            host_loads = c_router.loads_on_host(loads)
         for flow_idx in range(self.flow_num):
             data, tags, load_stack, extra = to_torch_tensor(in_flows[flow_idx], retrieve_attr=True)
             flow_tag = tags[-1]
             tags, load_stack = tags[:-1], load_stack[:-1]
-            routed = self._dispatch_flow(flow_idx, data, flow_tag, route_indices, loads, score)
+            routed = self._dispatch_flow(flow_idx, data, flow_tag, route_indices, loads, score, host_loads)
             if self.is_tag_index:
                 routed_data, routed_tags = routed
                 datas, path_loads, path_tags = c_router.split_fused_cells_to_paths(
                     routed_data, loads, self.max_path_padding, is_load_split=True,
-                    is_tag_split=True, tags=routed_tags)
+                    is_tag_split=True, tags=routed_tags, host_loads=host_loads)
                 all_out_flows.append([
                     init_grid_tensor(datas[i], tags + [path_tags[i]], load_stack + [path_loads[i]], extra)
                     for i in range(path_num)])
             else:
                 (datas,) = c_router.split_fused_cells_to_paths(
-                    routed[0], loads, self.max_path_padding, is_load_split=False, is_tag_split=False)
+                    routed[0], loads, self.max_path_padding, is_load_split=False, is_tag_split=False,
+                    host_loads=host_loads)
                 all_out_flows.append([
                     init_grid_tensor(datas[i], tags + [route_indices], load_stack + [loads], extra)
                     for i in range(path_num)])
@@ -455,7 +461,7 @@ class FusedDispatchFabric(DispatchFabric):
                 decision.dense(), caps, self.capacity_padding, self.path_wise_padding, False)
             buffer.copy_(indices)
 
-        indices = lazy_tensor(torch.empty((cells, paths), dtype=torch.int32, device=data.device), fill_dense)
+        indices = lazy_tensor(_lib.native().matrix(cells, paths, torch.int32, data), fill_dense)
         route = c_router.CompactRoute(decision.path_ids, decision.scores, loads, counts, seat_rows,
                                       row_entries, paths, indices)
         c_router.remember_route(loads, route)
@@ -466,7 +472,7 @@ class FusedDispatchFabric(DispatchFabric):
         extra[_route_key(level)] = route
         if (self.defer_dispatch and data.dim() == 2 and data.shape[1] % 8 == 0
                 and data.dtype in (torch.bfloat16, torch.float32)):
-            routed = torch.empty((rows, data.shape[1]), dtype=data.dtype, device=data.device)
+            routed = _lib.native().matrix(rows, data.shape[1], None, data)
             extra[_deferred_key(level)] = DeferredState(data, route, routed, _deferred_key(level))
         else:
             routed = c_router.dispatch_by_rows(data, row_entries, k)

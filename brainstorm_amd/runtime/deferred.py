@@ -17,6 +17,8 @@ from typing import Any, Optional
 
 import torch
 
+from brainstorm_amd import _lib
+
 __all__ = ["DeferredState", "DeferredRows", "LazyFill", "lazy_tensor", "pending_state", "pending_of",
            "wrap_if_pending", "settle"]
 
@@ -74,8 +76,7 @@ class LazyFill:
 def lazy_tensor(buffer: torch.Tensor, fill) -> torch.Tensor:
     """``buffer`` as a tensor that runs ``fill(buffer)`` before its first read; shape, dtype and
     device can be read without filling it."""
-    with torch._C.DisableTorchFunctionSubclass():
-        wrapped = buffer.as_subclass(DeferredRows)
+    wrapped = _lib.native().of_class(buffer, DeferredRows)
     wrapped.__dict__["_brt_state"] = LazyFill(buffer, fill)
     return wrapped
 
@@ -176,8 +177,7 @@ def wrap_if_pending(t: torch.Tensor, extra: Optional[dict]) -> torch.Tensor:
     state = pending_state(extra, t)
     if state is None:
         return t
-    with torch._C.DisableTorchFunctionSubclass():
-        wrapped = t.as_subclass(DeferredRows)
+    wrapped = _lib.native().of_class(t, DeferredRows)
     wrapped.__dict__["_brt_state"] = state
     return wrapped
 
