@@ -92,6 +92,13 @@ __device__ __forceinline__ void load_to_lds(const i32x4& rsrc, uint32_t voffset,
                : "memory");
 }
 
+// what is the same in all lanes, in scalar registers (the compiler cannot always tell)
+__device__ __forceinline__ i32x4 in_scalars(i32x4 r) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_readfirstlane(r[i]);
+  return r;
+}
+
 __device__ __forceinline__ void stream_out(const u32x4& v, u32x4* p) {
   asm volatile("global_store_dwordx4 %0, %1, off sc1 nt" : : "v"(p), "v"(v) : "memory");
 }
@@ -113,10 +120,9 @@ __device__ __forceinline__ void wave_fence() {
 template <int ACT, bool ROUTED, bool OUTF32>
 __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  // the tile's coordinates and, in the routed forms, the cells behind its rows pass through the
-  // first bytes of the stages, before any load lands there
-  int* const s_tile = reinterpret_cast<int*>(smem);  // expert, first row, valid rows, column tile, first seat
-  int* const s_cell = s_tile + 16;                   // 0-based cell of each row of the tile, -1 = empty slot
+  // in the routed forms the cells behind the tile's rows pass through the first bytes of the stages, before any
+  // load lands there
+  int* const s_cell = reinterpret_cast<int*>(smem);  // 0-based cell of each row of the tile, -1 = empty slot
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -127,66 +133,51 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // ---- which tile: patch order (grouped_gemm.hip) ----------------------------------------------
   const int xcd = blockIdx.x % kXcds, idx = blockIdx.x / kXcds;
   const int t = ((idx / kCusPerXcd) * kXcds + xcd) * kCusPerXcd + idx % kCusPerXcd;
-  if (tid < kWave) {
-    int carry_t = 0, carry_m = 0;
-    bool found = false;
-    for (int base = 0; base < a.E && !found; base += kWave) {
-      const int e = base + lane;
-      const int m = e < a.E ? a.loads[e] : 0;
-      const int blocks = (m + kBM - 1) / kBM;
-      const int tiles = blocks * a.tiles_n;
-      const int incl_t = wave_inclusive_scan(tiles), incl_m = wave_inclusive_scan(m);
-      const int first = carry_t + incl_t - tiles;
-      const bool hit = t >= first && t < first + tiles;
-      if (__ballot(hit) != 0) {
-        found = true;
-        if (hit) {
-          const int local = t - first, per_group = kPatchRows * a.tiles_n;
-          const int full = blocks / kPatchRows;
-          const int g = local / per_group;
-          int col, block;
-          if (g < full) {
-            const int r = local - g * per_group;
-            col = r / kPatchRows;
-            block = g * kPatchRows + r % kPatchRows;
-          } else {
-            const int last = blocks - full * kPatchRows;
-            const int r = local - full * per_group;
-            col = r / last;
-            block = full * kPatchRows + r % last;
-          }
-          s_tile[0] = e;
-          s_tile[1] = carry_m + incl_m - m + block * kBM;
-          s_tile[2] = min(kBM, m - block * kBM);
-          s_tile[3] = col;
-          s_tile[4] = block * kBM;
-        }
-      }
-      carry_t += __shfl(incl_t, kWave - 1, kWave);
-      carry_m += __shfl(incl_m, kWave - 1, kWave);
+  // Every wavefront finds the tile by itself, the weight pointers fetched in the same round trip as the loads: no
+  // exchange through LDS and no second trip stand before the first requests, and the K loop starts when the first K-step
+  // has landed.  Against one wavefront that looks, LDS, a load of the pointer and a wait for two K-steps:
+  // 16 x 2048 rows 1024 -> 4096 + GELU 278.8 -> 274.3 us (0.6 us a tile), 64 x 400 rows 768 -> 3072 174.1 -> 169.7, 8 x 4096 rows
+  // 2048 -> 8192 907.9 -> 899.0; contracting GEMMs, whose tiles take four times as long, within 0.5 %.
+  // (The 160-row kernel, which starts once per CU, lost 0.5 to 1 % by the same change.)
+  int e = -1, carry_t = 0, carry_m = 0, row0 = 0, rows = 0, seat0 = 0, n0 = 0;
+  const __bf16* w_e = nullptr;
+  for (int base = 0; base < a.E; base += kWave) {
+    const int el = min(base + lane, a.E - 1);
+    const int given = a.loads[el], m = base + lane < a.E ? given : 0;
+    const uint64_t wp = reinterpret_cast<uint64_t>(a.w[el]);
+    const int tiles = (m + kBM - 1) / kBM * a.tiles_n;
+    const int incl_t = wave_inclusive_scan(tiles), incl_m = wave_inclusive_scan(m);
+    const int first = carry_t + incl_t - tiles;
+    const unsigned long long hit = __ballot(t >= first && t < first + tiles);
+    if (hit != 0) {
+      const int src = __builtin_ctzll(hit);
+      const int mine = read_lane(m, src), blocks = (mine + kBM - 1) / kBM;
+      const int local = t - read_lane(first, src), per_group = kPatchRows * a.tiles_n;
+      const int full = blocks / kPatchRows, g = min(local / per_group, full);
+      const int r = local - g * per_group, wide = g < full ? kPatchRows : blocks - full * kPatchRows;
+      const int col = r / wide, block = g * kPatchRows + r - col * wide;
+      e = base + src;
+      seat0 = block * kBM;
+      row0 = carry_m + read_lane(incl_m - m, src) + seat0;
+      rows = min(min(kBM, mine - seat0), a.P - row0);
+      n0 = col * kBN;
+      w_e = reinterpret_cast<const __bf16*>(static_cast<uint64_t>(static_cast<uint32_t>(read_lane(static_cast<int>(wp), src))) |
+                                            static_cast<uint64_t>(static_cast<uint32_t>(read_lane(static_cast<int>(wp >> 32), src))) << 32);
+      break;
     }
-    if (!found && lane == 0) {  // beyond the last entry of the list: how far, and where the rows end
-      s_tile[0] = -1;
-      s_tile[1] = carry_m;
-      s_tile[2] = t - carry_t;
-    }
+    carry_t += read_lane(incl_t, kWave - 1);
+    carry_m += read_lane(incl_m, kWave - 1);
   }
-  __syncthreads();
-  const int e = __builtin_amdgcn_readfirstlane(s_tile[0]);
   if (e < 0) {
     // Surplus workgroups clear the tags of the rows no path owns: the j-th takes rows
     // [total + 256 j, total + 256 (j + 1)).  The grid holds P / 256 + E row blocks (rounded up) per
     // column tile and the experts use at most (total + 255 E) / 256 of them, so enough are left.
     if (ROUTED && a.row_tags_out != nullptr) {
-      const long r = static_cast<long>(s_tile[1]) + static_cast<long>(s_tile[2]) * kBM + tid;
+      const long r = static_cast<long>(carry_m) + static_cast<long>(t - carry_t) * kBM + tid;
       if (tid < kBM && r < a.P) a.row_tags_out[r] = 0;
     }
     return;
   }
-  const int row0 = __builtin_amdgcn_readfirstlane(s_tile[1]);
-  const int rows = min(__builtin_amdgcn_readfirstlane(s_tile[2]), a.P - row0);
-  const int n0 = __builtin_amdgcn_readfirstlane(s_tile[3]) * kBN;
-  const int seat0 = __builtin_amdgcn_readfirstlane(s_tile[4]);
   const int K = a.K;
   const int k_tiles = K / kBK;
   if constexpr (ROUTED) {  // one word per row, all of them in one round trip
@@ -206,15 +197,14 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // l & 7 of row l >> 3 of the group and fetches chunk (l & 7) ^ ((row >> 1) & 7) of that row.  A row
   // that does not exist (past the expert's last row, past N) gets an offset past any extent: zeros,
   // no memory request.
-  const __bf16* const w_e = a.w[e];
   // Every wavefront keeps the eight offsets of its rows in registers (the K-step alone goes into
   // the scalar offset).  Gathered rows need that -- the cells of a row group are anywhere in x --
   // and it takes the bounds check out of the loop for the others.
   const bool gather = ROUTED && a.gather != 0;
-  const i32x4 res = wm == 0
+  const i32x4 res = in_scalars(wm == 0
       ? (gather ? make_rsrc(a.x, static_cast<size_t>(a.T) * K * 2)
                 : make_rsrc(a.x + static_cast<size_t>(row0) * K, static_cast<size_t>(a.P - row0) * K * 2))
-      : make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2);
+      : make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2));
   const int cols = a.N - n0;  // weight rows that exist from n0 on
   uint32_t off[8];
 #pragma unroll
@@ -232,7 +222,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     }
     off[i] = there ? (static_cast<uint32_t>(at) * K + chunk * 8) * 2 : kOutOfRange;
   }
-  __syncthreads();  // everyone has read the coordinates and cells; the loads may overwrite them
+  if constexpr (ROUTED) __syncthreads();  // everyone has read the cells; the loads may overwrite them
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
   auto load_a = [&](int kt, uint32_t slot, int i) {
     load_to_lds(res, off[i], kt * kRowB, lds0 + slot + (wn + 4 * i) * 1024);
@@ -279,7 +269,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
 #pragma unroll
     for (int i = 0; i < 8; ++i) load_b(1, kTileB, i);
   }
-  wait_loads_all();
+  wait_loads_but_8();  // K-step 0
   block_barrier();
   // Group 1 starts one phase late.  From here on a barrier ends group 0's M phase and group 1's C
   // phase, the next one group 0's C phase and group 1's M phase, and so on.
