@@ -364,21 +364,29 @@ __global__ __launch_bounds__(kBlock) void band_top1_kernel(const void* scores, S
   const long row_w = (static_cast<long>(blockIdx.x) * kWavesPB + wave) * a.rows_pw;
   const int rows_here = static_cast<int>(max(0l, min(static_cast<long>(a.rows_pw), a.T - row_w)));
   int sum = 0;
+  // (buffer loads and stores: a guard around each would be a branch with a wait of its own)
+  constexpr int kScoreB = DT == BRT_F32 ? 4 : 2;
+  const size_t before = static_cast<size_t>(rows_here > 0 ? row_w : 0) * E, words = static_cast<size_t>(rows_here) * E;
+  const __amdgpu_buffer_rsrc_t from = words_at(static_cast<const char*>(scores) + before * kScoreB, words * kScoreB);
+  const __amdgpu_buffer_rsrc_t to = words_at(mask + before, words * 4);
   for (int i0 = 0; i0 < a.n_ins; i0 += kBatch) {
-    uint32_t key[kBatch];
+    const unsigned first = e < E ? static_cast<unsigned>(i0 * rps + sub) * E + e : kOutside / 4, step = rps * E;
+    uint32_t bits[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const int rl = (i0 + u) * rps + sub;
-      key[u] = rl < rows_here && e < E ? score_key(load_score<DT>(scores, static_cast<size_t>(row_w + rl) * E + e)) : 0u;
+      if constexpr (DT == BRT_F32) bits[u] = __builtin_amdgcn_raw_buffer_load_b32(from, (first + u * step) * 4u, 0, 0);
+      else bits[u] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(from, (first + u * step) * 2u, 0, 0));
     }
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       if (i0 + u >= a.n_ins) break;  // wave-uniform
-      const uint32_t best = segment_max(key[u], ep);
-      const unsigned long long tied = __ballot(key[u] == best && key[u] != 0) & row_lanes;
+      const bool live = e < E && (i0 + u) * rps + sub < rows_here;
+      const uint32_t key = live ? score_key(DT == BRT_F32 ? __uint_as_float(bits[u]) : half_bits_to_float<DT>(bits[u])) : 0u;
+      const uint32_t best = segment_max(key, ep);
+      const unsigned long long tied = __ballot(key == best && key != 0) & row_lanes;
       const int taken = tied != 0 && lane == __builtin_ctzll(tied) ? 1 : 0;
       sum += taken;
-      if (key[u] != 0) mask[static_cast<size_t>(row_w + (i0 + u) * rps + sub) * E + e] = taken;
+      __builtin_amdgcn_raw_buffer_store_b32(taken, to, live ? (first + u * step) * 4u : kOutside, 0, 0);
     }
   }
   sum = sum_over_rows_in_wave(sum, a.ep_shift);
