@@ -20,7 +20,7 @@
 //     wavefront that loads by itself 18.7 us).  K-steps of 128 with half the barriers change nothing.
 //   - Rows past the expert's load and past N address past the buffer extent: zeros, no request.
 //   - fp32 rows of x (X32) are loaded as they are and rounded to bf16 on their way from LDS to the matrix unit: the cast
-//     kernel and its pass over the rows go (16 experts x 60 rows 512 -> 2048 -> 512 in fp32: a launch each of 3.3 us).
+//     kernel and its pass over the rows go (figures at the choice of the tile).
 //   - Every wavefront finds the tile by itself (DPP scan + ballot over the loads, the weight
 //     pointers fetched in the same round trip), so the first weight request leaves two round trips
 //     after the start.  Gathered rows add one, which the weight requests do not wait for.
@@ -393,17 +393,11 @@ int launch_of(GemmArgs& a, hipStream_t st) {
   return f32 ? launch<XR, NT, D, ACT, false, true, X32>(a, st) : launch<XR, NT, D, ACT, false, false, X32>(a, st);
 }
 
-template <int XR, int NT, int D, int ACT>
-int launch_form(GemmArgs& a, hipStream_t st) {
-  // (fp32 rows take twice the room: three stages of 64 x 64 still leave room for two workgroups on a CU)
-  return a.x_f32 ? launch_of<XR, NT, XR == 64 ? 3 : D, ACT, true>(a, st) : launch_of<XR, NT, D, ACT, false>(a, st);
-}
-
-template <int XR, int NT, int D>
+template <int XR, int NT, int D, bool X32 = false>
 int launch_act(GemmArgs& a, int act, hipStream_t st) {
-  if (act == BRT_ACT_GELU) return launch_form<XR, NT, D, BRT_ACT_GELU>(a, st);
-  if (act == BRT_ACT_RELU) return launch_form<XR, NT, D, BRT_ACT_RELU>(a, st);
-  return launch_form<XR, NT, D, BRT_ACT_NONE>(a, st);
+  if (act == BRT_ACT_GELU) return launch_of<XR, NT, D, BRT_ACT_GELU, X32>(a, st);
+  if (act == BRT_ACT_RELU) return launch_of<XR, NT, D, BRT_ACT_RELU, X32>(a, st);
+  return launch_of<XR, NT, D, BRT_ACT_NONE, X32>(a, st);
 }
 
 }  // namespace
@@ -456,6 +450,17 @@ int launch_skinny_gemm(GemmArgs& a, int act, hipStream_t st) {
   const long used = std::min(a.E, a.P);
   const double rows = static_cast<double>(a.P) / used;
   auto tiles = [&](int block) { return used * (rows > block ? rows / block + 0.5 : 1.0) * ((a.N + 63) / 64); };
+  if (a.x_f32) {
+    // fp32 rows take twice the room, so two stages of 64 x 64 are as many as leave three workgroups on a CU (16 x 60 rows
+    // 512 -> 2048 12.4 us, three stages 12.6, cast and bf16 14.1; a long K wants three: 2048 -> 512 18.4, two 22.7),
+    // four of 32 x 64 otherwise (64 x 8 rows 512 -> 1024 16.7, 32 x 32 24.7, cast and bf16 20.6; 8 x 3 rows 768 -> 3072
+    // 9.8, 12.9 and 11.7), and 32 x 32 only where those leave half of the CUs without a tile (8 x 28 rows 4096 -> 1024
+    // 21.9, 23.8 and 25.9; 8 x 3 rows 3072 -> 768 13.2, 13.5 and 12.2).
+    if (rows > 32 && tiles(64) >= 192)
+      return a.K <= 1024 ? launch_act<64, 2, 2, true>(a, act, st) : launch_act<64, 2, 3, true>(a, act, st);
+    if (tiles(32) <= 128) return launch_act<32, 1, 4, true>(a, act, st);
+    return launch_act<32, 2, 4, true>(a, act, st);
+  }
   if (rows > 32 && tiles(64) >= 192) {
     if (a.K <= 1024) return launch_act<64, 2, 3>(a, act, st);
     return launch_act<64, 2, 4>(a, act, st);
