@@ -352,7 +352,8 @@ __global__ __launch_bounds__(kBlock) void band_count_kernel(ScanArgs a) {
 
 // pass 1 of a throttled top-1 route: the hot mask of the largest score of every row (order of torch.topk as in
 // gate.hip) and the column sums of the band, from one read of the scores; up to 64 paths.  Bound by the round trip of
-// a batch of loads; the mask and its sums by themselves take a launch each (100352 x 8 fp32 scores: 4.1 + 3.4 us).
+// a batch of loads; the mask and its sums by themselves take a launch each (100352 x 8 fp32 scores: 4.1 + 3.4 us in a
+// trace, 7.1 here and a boundary less; with the throttle behind it 10.4 us back to back, 11.7 in three launches).
 template <int DT>
 __global__ __launch_bounds__(kBlock) void band_top1_kernel(const void* scores, ScanArgs a, int* mask) {
   __shared__ int s_sum[kWavesPB][kWave];
