@@ -435,14 +435,16 @@ def split_fused_cells_to_paths(
         is_load_split = True
         if tags is None:
             raise RuntimeError("is_tag_split needs tags")
+    native = _lib.native_or_none()
     if max_path_padding:
         rows = [in_data.size(0) // path_num] * path_num
     elif host_loads is not None:
         rows = host_loads
     else:
-        rows = _lib.native().int_list(loads) if loads.dtype == torch.int32 and loads.dim() == 1 else loads.cpu().tolist()
-    if type(in_data) is torch.Tensor and type(loads) is torch.Tensor and (tags is None or type(tags) is torch.Tensor):
-        datas, load_list, tag_list = _lib.native().split_rows(
+        listed = native is not None and loads.dtype == torch.int32 and loads.dim() == 1
+        rows = native.int_list(loads) if listed else loads.cpu().tolist()
+    if native is not None and type(in_data) is torch.Tensor and type(loads) is torch.Tensor and (tags is None or type(tags) is torch.Tensor):
+        datas, load_list, tag_list = native.split_rows(
             in_data, rows, loads if is_load_split else None, tags if is_tag_split else None)
     else:
         starts = [0, *itertools.accumulate(rows)]

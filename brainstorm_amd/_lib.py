@@ -211,6 +211,11 @@ def native():
     return _native
 
 
+def native_or_none():
+    """:func:`native`, or None where it has not been built (flows can be annotated without it)."""
+    return native() if _native is not None or os.path.exists(NATIVE_PATH) else None
+
+
 _calls = 0
 
 

@@ -73,10 +73,18 @@ class LazyFill:
             self.done = True
 
 
+def _as_deferred(t: torch.Tensor) -> torch.Tensor:
+    native = _lib.native_or_none()
+    if native is not None:
+        return native.of_class(t, DeferredRows)
+    with torch._C.DisableTorchFunctionSubclass():
+        return t.as_subclass(DeferredRows)
+
+
 def lazy_tensor(buffer: torch.Tensor, fill) -> torch.Tensor:
     """``buffer`` as a tensor that runs ``fill(buffer)`` before its first read; shape, dtype and
     device can be read without filling it."""
-    wrapped = _lib.native().of_class(buffer, DeferredRows)
+    wrapped = _as_deferred(buffer)
     wrapped.__dict__["_brt_state"] = LazyFill(buffer, fill)
     return wrapped
 
@@ -177,7 +185,7 @@ def wrap_if_pending(t: torch.Tensor, extra: Optional[dict]) -> torch.Tensor:
     state = pending_state(extra, t)
     if state is None:
         return t
-    wrapped = _lib.native().of_class(t, DeferredRows)
+    wrapped = _as_deferred(t)
     wrapped.__dict__["_brt_state"] = state
     return wrapped
 

@@ -219,7 +219,9 @@ def init_grid_tensor(tensor: torch.Tensor, tag_stack=None, load_stack=None,
                      extra_attr_dict=None) -> GridTensor:
     if type(tensor) is torch.Tensor and type(tag_stack) is list and type(load_stack) is list and tag_stack and load_stack \
             and GridTensor.SHALLOW_TRANSPORT and (extra_attr_dict is None or type(extra_attr_dict) is dict):
-        return _lib.native().grid(tensor, GridTensor, tag_stack, load_stack, extra_attr_dict)  # as below
+        native = _lib.native_or_none()
+        if native is not None:
+            return native.grid(tensor, GridTensor, tag_stack, load_stack, extra_attr_dict)  # as below
     cell: GridTensor = tensor.as_subclass(GridTensor)
     if tag_stack and load_stack:
         assert isinstance(tag_stack, list) and isinstance(load_stack, list), (
@@ -241,7 +243,12 @@ def init_grid_tensor_from(tensor: torch.Tensor, from_gird_tensor: GridTensor) ->
 def _as_plain(grid_t: torch.Tensor, extra) -> torch.Tensor:
     """The tensor without the GridTensor subclass; an unfilled deferred dispatch buffer comes out
     as a :class:`brainstorm_amd.runtime.deferred.DeferredRows`, which fills itself on first use."""
-    plain = _lib.native().plain(grid_t)
+    native = _lib.native_or_none()
+    if native is not None:
+        plain = native.plain(grid_t)
+    else:
+        with torch._C.DisableTorchFunctionSubclass():
+            plain = grid_t.as_subclass(torch.Tensor)
     return deferred.wrap_if_pending(plain, extra) if extra else plain
 
 

@@ -224,3 +224,28 @@ def test_annotator_refuses_cells_of_no_elements(shape):
 def test_annotator_takes_no_cells():
     cells = brt.Annotator([0])(torch.zeros(0, 7))
     assert tuple(cells.shape) == (0, 7) and cells.tag_stack == [None]
+
+
+@pytest.mark.parametrize("built", [True, False])
+def test_flows_are_wrapped_the_same_with_and_without_the_native_module(monkeypatch, built):
+    """Wrapping shares storage and stacks, copies the extra attributes, keeps autograd's link, and leaves a buffer that
+    is not filled yet alone -- in native code and, where that has not been built, in Python."""
+    from brainstorm_amd import _lib
+    from brainstorm_amd.runtime import deferred
+
+    if not built:
+        monkeypatch.setattr(_lib, "native_or_none", lambda: None)
+    base = torch.randn(4, 3, requires_grad=True)
+    tags, loads, extra = [None], [torch.tensor([4])], {"key": 1}
+    grid = init_grid_tensor(base, tags, loads, extra)
+    assert type(grid).__name__ == "GridTensor" and grid.data_ptr() == base.data_ptr()
+    assert grid.tag_stack is tags and grid.load_stack is loads
+    assert grid.extra_attr_dict == extra and grid.extra_attr_dict is not extra
+    plain, got_tags, got_loads, _ = brt.to_torch_tensor(grid, retrieve_attr=True)
+    assert type(plain) is torch.Tensor and got_tags is tags and got_loads is loads
+    plain.sum().backward()
+    assert torch.equal(base.grad, torch.ones_like(base))
+    filled = []
+    lazy = deferred.lazy_tensor(torch.zeros(3), lambda b: filled.append(b.fill_(2.0)))
+    assert not filled and lazy.shape == (3,)
+    assert float(lazy.sum()) == 6.0 and len(filled) == 1
