@@ -441,7 +441,7 @@ def split_fused_cells_to_paths(
     elif host_loads is not None:
         rows = host_loads
     else:
-        listed = native is not None and loads.dtype == torch.int32 and loads.dim() == 1
+        listed = native is not None and type(loads) is torch.Tensor and loads.dtype == torch.int32 and loads.dim() == 1
         rows = native.int_list(loads) if listed else loads.cpu().tolist()
     if native is not None and type(in_data) is torch.Tensor and type(loads) is torch.Tensor and (tags is None or type(tags) is torch.Tensor):
         datas, load_list, tag_list = native.split_rows(

@@ -675,6 +675,8 @@ PyObject* int_list(const Args& a) {
   const int64_t n = t.numel();
   const int32_t* values = nullptr;
   at::DataPtr host;
+  // a tensor that only stands for others (of the meta device, or under a fake-tensor mode) has no values
+  if (n > 0 && ptr(t) == nullptr) not_implemented("Cannot copy out of a tensor without data");
   if (n > 0 && t.is_cuda()) {
     const c10::DeviceGuard guard(t.device());
     host = read_back(t, n * 4, "reading the loads");

@@ -1,10 +1,13 @@
 """GridTensor / Annotator / Registry behaviour (scenarios of the reference's
 test/python/grid_tensor_test.py:13-71), CPU only."""
+import os
+
 import pytest
 import torch
 import torch.nn as nn
 
 import brt
+from brainstorm_amd import _lib
 from brt.runtime.grid_tensor import GridTensor, init_grid_tensor, deinit_grid_tensor
 from brt.runtime import Registry
 
@@ -249,3 +252,19 @@ def test_flows_are_wrapped_the_same_with_and_without_the_native_module(monkeypat
     lazy = deferred.lazy_tensor(torch.zeros(3), lambda b: filled.append(b.fill_(2.0)))
     assert not filled and lazy.shape == (3,)
     assert float(lazy.sum()) == 6.0 and len(filled) == 1
+
+
+def test_loads_without_data_are_refused():
+    """Fake and meta tensors have no words that a split could go by."""
+    import brt._C.router as c_router
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    loads, rows = torch.tensor([2, 0, 3], dtype=torch.int32), torch.zeros(5, 2)
+    with pytest.raises(NotImplementedError):
+        c_router.split_fused_cells_to_paths(rows, loads.to("meta"))
+    with pytest.raises(Exception, match="_local_scalar_dense"):  # what reading a fake tensor raises
+        c_router.split_fused_cells_to_paths(rows, FakeTensorMode().from_tensor(loads))
+    if os.path.exists(_lib.NATIVE_PATH):
+        for nothing in (loads.to("meta"), FakeTensorMode().from_tensor(loads)):
+            with pytest.raises(NotImplementedError):
+                _lib.native().int_list(nothing)
