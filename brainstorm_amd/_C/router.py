@@ -435,15 +435,18 @@ def split_fused_cells_to_paths(
         is_load_split = True
         if tags is None:
             raise RuntimeError("is_tag_split needs tags")
-    native = _lib.native_or_none()
+    # (where a compiler, tracer or mode looks on, the views are made by torch's own calls)
+    native = None if torch.compiler.is_compiling() else _lib.native_or_none()
+    if native is not None and not native.ordinary(in_data, loads, tags):
+        native = None
     if max_path_padding:
         rows = [in_data.size(0) // path_num] * path_num
     elif host_loads is not None:
         rows = host_loads
     else:
-        listed = native is not None and type(loads) is torch.Tensor and loads.dtype == torch.int32 and loads.dim() == 1
+        listed = native is not None and loads.dtype == torch.int32 and loads.dim() == 1
         rows = native.int_list(loads) if listed else loads.cpu().tolist()
-    if native is not None and type(in_data) is torch.Tensor and type(loads) is torch.Tensor and (tags is None or type(tags) is torch.Tensor):
+    if native is not None:
         datas, load_list, tag_list = native.split_rows(
             in_data, rows, loads if is_load_split else None, tags if is_tag_split else None)
     else:

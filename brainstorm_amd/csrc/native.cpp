@@ -12,12 +12,14 @@
 // (src/backend/torch/torch.h:16-21, router.cc:266).
 #include <Python.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/CachingHostAllocator.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/full.h>
 #include <ATen/ops/zeros.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/Dtype.h>
@@ -715,13 +717,31 @@ const Tensor& as_it_is(PyObject* o) {
   return THPVariable_Unpack(o);
 }
 
+// Whether a view made here is what the same call from Python makes: no mode or tracer looks on at torch's calls, and
+// the tensor does not answer them in Python.  Where not, the entries below leave the work to Python (None).
+bool unobserved(const Tensor& t) {
+  return !at::impl::torch_function_mode_enabled() && !c10::impl::dispatch_mode_enabled() && !t.key_set().has(c10::DispatchKey::Python);
+}
+
+// tensors (or None) -> whether all of them are ordinary ones, and unobserved
+PyObject* ordinary(const Args& a) {
+  bool all = true;
+  for (Py_ssize_t i = 0; i < a.n && all; ++i)
+    all = a.none(i) || (THPVariable_CheckExact(a.v[i]) && unobserved(THPVariable_Unpack(a.v[i])));
+  return PyBool_FromLong(all);
+}
+
 // t.as_subclass(torch.Tensor) without a turn through __torch_function__
-PyObject* plain(const Args& a) { return wrap(as_it_is(a.v[0]).alias()); }
+PyObject* plain(const Args& a) {
+  const Tensor& t = as_it_is(a.v[0]);
+  return unobserved(t) ? wrap(t.alias()) : none();
+}
 
 // t.as_subclass(class), likewise
 PyObject* of_class(const Args& a) {
   if (!PyType_Check(a.v[1])) throw Raised(PyExc_TypeError, "a class is expected");
-  return THPVariable_Wrap(as_it_is(a.v[0]).alias(), reinterpret_cast<PyTypeObject*>(a.v[1]));
+  const Tensor& t = as_it_is(a.v[0]);
+  return unobserved(t) ? THPVariable_Wrap(t.alias(), reinterpret_cast<PyTypeObject*>(a.v[1])) : none();
 }
 
 // rows, columns, dtype, like -> an uninitialised [rows, columns] matrix on like's device
@@ -739,7 +759,9 @@ PyObject* grid(const Args& a) {
   static PyObject* const keys[3] = {PyUnicode_InternFromString("cell_tag_stack"), PyUnicode_InternFromString("cell_load_stack"),
                                     PyUnicode_InternFromString("cell_extra_attr_dict")};
   if (!PyType_Check(a.v[1])) throw Raised(PyExc_TypeError, "a class is expected");
-  PyObject* const made = THPVariable_Wrap(as_it_is(a.v[0]).alias(), reinterpret_cast<PyTypeObject*>(a.v[1]));
+  const Tensor& t = as_it_is(a.v[0]);
+  if (!unobserved(t)) return none();
+  PyObject* const made = THPVariable_Wrap(t.alias(), reinterpret_cast<PyTypeObject*>(a.v[1]));
   PyObject* const attrs = made != nullptr ? PyObject_GenericGetDict(made, nullptr) : nullptr;
   PyObject* const extra = attrs == nullptr ? nullptr : PyDict_Check(a.v[4]) ? PyDict_Copy(a.v[4]) : PyDict_New();
   const bool done = extra != nullptr && PyDict_SetItem(attrs, keys[0], a.v[2]) == 0 && PyDict_SetItem(attrs, keys[1], a.v[3]) == 0 &&
@@ -831,7 +853,7 @@ PyMethodDef methods[] = {
     BRT_ENTRY(dispatch, 12),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
     BRT_ENTRY(top1_to_capacity, 2), BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 7),     BRT_ENTRY(grouped_linear, 16),
     BRT_ENTRY(grouped_linear_f32, 16), BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5),        BRT_ENTRY(int_list, 1),
-    BRT_ENTRY(plain, 1),            BRT_ENTRY(of_class, 2),            BRT_ENTRY(matrix, 4),
+    BRT_ENTRY(ordinary, 3),         BRT_ENTRY(plain, 1),            BRT_ENTRY(of_class, 2),            BRT_ENTRY(matrix, 4),
     BRT_ENTRY(grid, 5),                BRT_ENTRY(split_rows, 4),
     BRT_ENTRY(sum_rows_by_index, 3), BRT_ENTRY(one_value, 2),         BRT_ENTRY(unique_tags, 1),      BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
 

@@ -75,8 +75,9 @@ class LazyFill:
 
 def _as_deferred(t: torch.Tensor) -> torch.Tensor:
     native = _lib.native_or_none()
-    if native is not None:
-        return native.of_class(t, DeferredRows)
+    wrapped = native.of_class(t, DeferredRows) if native is not None else None
+    if wrapped is not None:
+        return wrapped
     with torch._C.DisableTorchFunctionSubclass():
         return t.as_subclass(DeferredRows)
 

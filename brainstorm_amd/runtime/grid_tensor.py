@@ -220,8 +220,9 @@ def init_grid_tensor(tensor: torch.Tensor, tag_stack=None, load_stack=None,
     if type(tensor) is torch.Tensor and type(tag_stack) is list and type(load_stack) is list and tag_stack and load_stack \
             and GridTensor.SHALLOW_TRANSPORT and (extra_attr_dict is None or type(extra_attr_dict) is dict):
         native = _lib.native_or_none()
-        if native is not None:
-            return native.grid(tensor, GridTensor, tag_stack, load_stack, extra_attr_dict)  # as below
+        grid = native.grid(tensor, GridTensor, tag_stack, load_stack, extra_attr_dict) if native is not None else None
+        if grid is not None:
+            return grid  # as below
     cell: GridTensor = tensor.as_subclass(GridTensor)
     if tag_stack and load_stack:
         assert isinstance(tag_stack, list) and isinstance(load_stack, list), (
@@ -244,9 +245,8 @@ def _as_plain(grid_t: torch.Tensor, extra) -> torch.Tensor:
     """The tensor without the GridTensor subclass; an unfilled deferred dispatch buffer comes out
     as a :class:`brainstorm_amd.runtime.deferred.DeferredRows`, which fills itself on first use."""
     native = _lib.native_or_none()
-    if native is not None:
-        plain = native.plain(grid_t)
-    else:
+    plain = native.plain(grid_t) if native is not None else None
+    if plain is None:
         with torch._C.DisableTorchFunctionSubclass():
             plain = grid_t.as_subclass(torch.Tensor)
     return deferred.wrap_if_pending(plain, extra) if extra else plain

@@ -268,3 +268,55 @@ def test_loads_without_data_are_refused():
         for nothing in (loads.to("meta"), FakeTensorMode().from_tensor(loads)):
             with pytest.raises(NotImplementedError):
                 _lib.native().int_list(nothing)
+
+
+def _observed_passes():
+    import brt._C.router as c_router
+    from brainstorm_amd.runtime import deferred
+
+    loads = torch.tensor([2, 0, 3], dtype=torch.int32)
+    return {
+        "annotate": lambda x: brt.to_torch_tensor(brt.Annotator([0])(x)) * 2,
+        "wrap": lambda x: brt.to_torch_tensor(init_grid_tensor(x, [None], [loads], {}), retrieve_attr=True)[0] * 2,
+        "lazy": lambda x: deferred.lazy_tensor(x, lambda rows: None) * 2,
+        "split": lambda x: torch.cat([r * 2 for r in c_router.split_fused_cells_to_paths(x, loads)[0]]),
+        "split with loads": lambda x: torch.cat(c_router.split_fused_cells_to_paths(x, loads, is_load_split=True)[0]) * 2,
+    }
+
+
+@pytest.mark.parametrize("name", list(_observed_passes()))
+def test_flows_under_modes_and_tracers(name):
+    """Wrapping and splitting work where a dispatch mode, a function mode or a tracer looks on, which see of them
+    what they see without the native module."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Dispatched(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Called(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+
+    run, x = _observed_passes()[name], torch.arange(10.0).view(5, 2)
+    for mode in (Dispatched, Called):
+        logs = []
+        for native in (_lib.native_or_none, lambda: None):
+            seen = []
+            with pytest.MonkeyPatch.context() as patch, mode():
+                patch.setattr(_lib, "native_or_none", native)
+                out = run(x)
+            assert torch.equal(out, 2 * x)
+            logs.append(seen)
+        assert logs[0] == logs[1]
+    assert torch.equal(make_fx(run)(x)(x), 2 * x)
+
+
+def test_split_compiles_as_one_graph():
+    run = _observed_passes()["split"]
+    x = torch.arange(10.0).view(5, 2)
+    assert torch.equal(torch.compile(run, backend="eager", fullgraph=True)(x), 2 * x)
