@@ -141,14 +141,18 @@ ScanGeometry scan_geometry(int T, int E, bool tag_mode, bool whole_ok) {
   return g;
 }
 
-// Bands of a throttled top-1 route: always the two-launch form (its first launch reads the scores anyway).
+// Bands of a throttled top-1 route: always the two-launch form (its first launch reads the scores anyway).  A mask that one
+// workgroup of eight wavefronts would hold is spread over workgroups of four with at most eight loads each: a load costs
+// the selection of its rows' best score, one after the other (128 x 64 in one workgroup 15.5 us, 7.6 so, 10.1 as
+// mask and throttle; 64 x 33 9.5, 7.7 and 9.2).
 ScanGeometry top1_geometry(int T, int E) {
+  constexpr int kMostLoads = 8;
   ScanGeometry g = scan_geometry(T, E, true, false);
-  if (g.waves_pb != kWavesPB) {  // a mask that one workgroup of eight wavefronts would hold
-    const int rps = kWave >> g.ep_shift;
-    g.rows_pw = (T + kWavesPB * rps - 1) / (kWavesPB * rps) * rps;
+  if (g.waves_pb != kWavesPB) {
+    const int rps = kWave >> g.ep_shift, loads_pw = std::min((T + kWavesPB * rps - 1) / (kWavesPB * rps), kMostLoads);
+    g.rows_pw = loads_pw * rps;
     g.waves_pb = kWavesPB;
-    g.bands = 1;
+    g.bands = (T + kWavesPB * g.rows_pw - 1) / (kWavesPB * g.rows_pw);
   }
   return g;
 }
@@ -797,9 +801,15 @@ bool same_words(const int* mask, const int* out, int T, int E) {
   return m < o + bytes && o < m + bytes;
 }
 
+size_t scan_workspace_bytes(int T, int E) {
+  // enough for either index format (tag indices leave the one-workgroup form earlier)
+  const int bands = std::max(scan_geometry(T, E, false, false).bands, scan_geometry(T, E, true, false).bands);
+  return (static_cast<size_t>(bands) + 1) * E * sizeof(int);
+}
+
 int launch_scan(int mode, ScanArgs& a, void* workspace, size_t workspace_bytes, void* stream) {
   const ScanGeometry g = scan_geometry(a.T, a.E, mode == kTag, mode != kThrottle && !same_words(a.mask, a.out, a.T, a.E));
-  const size_t need = brt_hip_scan_workspace_bytes(a.T, a.E);
+  const size_t need = scan_workspace_bytes(a.T, a.E);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(BRT_E_WORKSPACE, "scan workspace too small: %zu < %zu bytes", workspace_bytes,
                 need);
@@ -901,9 +911,8 @@ using namespace brt;
 
 extern "C" size_t brt_hip_scan_workspace_bytes(int T, int E) {
   if (T <= 0 || E <= 0) return 0;
-  // enough for either index format (tag indices leave the one-workgroup form earlier)
-  const int bands = std::max(scan_geometry(T, E, false, false).bands, scan_geometry(T, E, true, false).bands);
-  return (static_cast<size_t>(bands) + 1) * E * sizeof(int);
+  const size_t top1 = E <= kWave ? (static_cast<size_t>(top1_geometry(T, E).bands) + 1) * E * sizeof(int) : 0;
+  return std::max(scan_workspace_bytes(T, E), top1);
 }
 
 extern "C" int brt_hip_generate_indices_and_loads(const int32_t* mask, int32_t* indices,
@@ -954,7 +963,7 @@ extern "C" int brt_hip_generate_indices_and_loads_static(const int32_t* mask, in
                                                          void* stream) {
   if (T < 0 || E <= 0) return fail(BRT_E_INVALID, "bad shape T=%d E=%d", T, E);
   if (static_cast<long>(T) * E >= (1l << 31)) return fail(BRT_E_UNSUPPORTED, "T*E >= 2^31");
-  const size_t need = brt_hip_scan_workspace_bytes(T, E);
+  const size_t need = scan_workspace_bytes(T, E);
   if (need > kStaticScratchInts * sizeof(int))
     return fail(BRT_E_WORKSPACE,
                 "a [%d,%d] mask needs %zu bytes of scratch, the built-in buffer holds %zu: use "

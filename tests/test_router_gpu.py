@@ -1177,7 +1177,8 @@ def test_words_read_back_by_the_host(n):
 
 @pytest.mark.parametrize("T,E,dtype", [
     (1, 1, torch.float32), (5, 8, torch.float16), (128, 64, torch.bfloat16), (129, 64, torch.float32), (100, 3, torch.bfloat16),
-    (777, 5, torch.float32), (8192, 8, torch.float16), (40000, 33, torch.bfloat16), (100352, 8, torch.float16), (131075, 2, torch.float32),
+    (777, 5, torch.float32), (33, 33, torch.float32), (127, 40, torch.float16), (65, 17, torch.float32),  # several bands of few rows
+    (8192, 8, torch.float16), (40000, 33, torch.bfloat16), (100352, 8, torch.float16), (131075, 2, torch.float32),
 ])
 def test_top1_to_capacity_is_the_mask_throttled(brt_mod, T, E, dtype):
     """One read of the scores gives what the hot mask and the throttle give one after the other: ties, NaN and
