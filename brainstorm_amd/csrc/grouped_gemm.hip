@@ -686,13 +686,9 @@ bool wide_tiles_come_in_rounds(const GemmArgs& a) {
   return tiles >= 2 * cus || (4 * tiles >= 3 * cus && tiles <= cus);
 }
 
-// fp32 rows are rounded by the kernel itself where bf16 rows of that shape would take the few-rows kernel, with up to 64
-// rows per expert: with more every column tile reads twice the bytes of many rows again (32 x 120 rows 2048 -> 512
-// 48.9 us, cast and bf16 39.5; 8 x 120 rows 3072 -> 768 28.5 and 27.1).
-bool takes_f32_rows(int E, int P, int K, int N) {
-  GemmArgs a{};
-  a.E = E; a.P = P; a.K = K; a.N = N;
-  return E > 0 && P > 0 && K > 0 && N > 0 && K % 8 == 0 && N % 8 == 0 && P <= 64l * std::min(E, P) && !wide_tiles_come_in_rounds(a) && skinny_gemm_applies(a);
+// Shapes whose fp32 rows the few-rows kernel rounds itself when asked to; where that is the faster way, skinny_gemm_takes_f32 says.
+bool runs_on_f32_rows(const GemmArgs& a) {
+  return a.P <= 64l * std::min(a.E, a.P) && !wide_tiles_come_in_rounds(a) && skinny_gemm_applies(a);
 }
 
 int grouped_gemm_impl(const void* x, const void* const* weights, const void* const* biases, void* out,
@@ -745,7 +741,7 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   }
   a.x_f32 = x_is_f32;
   if (x_is_f32) {
-    if (!takes_f32_rows(E, P, K, N))
+    if (!runs_on_f32_rows(a))
       return fail(BRT_E_UNSUPPORTED, "fp32 rows are taken by the few-rows kernel only, not with E=%d P=%d K=%d N=%d", E, P, K, N);
     return launch_skinny_gemm(a, act, as_stream(stream));
   }
@@ -852,7 +848,10 @@ __global__ __launch_bounds__(256) void cast_f32_to_bf16_kernel(const float* __re
 
 extern "C" int brt_hip_grouped_gemm_f32in_supported(int E, int P, int T, int K, int N, int gather_in) {
   if (gather_in && static_cast<size_t>(T) * K * 4 > 0x7fffffffull) return 0;
-  return takes_f32_rows(E, P, K, N) ? 1 : 0;
+  if (E <= 0 || P <= 0 || K <= 0 || N <= 0 || K % 8 != 0 || N % 8 != 0) return 0;
+  GemmArgs a{};
+  a.E = E; a.P = P; a.K = K; a.N = N;
+  return runs_on_f32_rows(a) && skinny_gemm_takes_f32(a, gather_in ? T : 0) ? 1 : 0;
 }
 
 extern "C" int brt_hip_grouped_gemm_f32in(const float* x, const void* const* weights, const void* const* biases, void* out,

@@ -41,6 +41,7 @@ int launch_pingpong_gemm(GemmArgs& a, int act, hipStream_t st);
 
 // The kernel for few rows per expert and few tiles (grouped_gemm_skinny.hip), every form.
 bool skinny_gemm_applies(const GemmArgs& a);
+bool skinny_gemm_takes_f32(const GemmArgs& a, int cells);
 int launch_skinny_gemm(GemmArgs& a, int act, hipStream_t st);
 
 // The routed forms: 0-based cell behind row `row` of the dispatched layout (seat `seat`, 0-based, of

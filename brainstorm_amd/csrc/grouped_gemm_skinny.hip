@@ -438,7 +438,47 @@ bool skinny_gemm_applies(const GemmArgs& a) {
   return tiles <= 160 && weight_bytes < 1.5e8;
 }
 
-// Shape of the tile; the estimates take an expert's last row block as half full.
+namespace {
+// Estimated tiles of `block` x 64 of the result; an expert's last row block is taken as half full.
+double narrow_tiles(const GemmArgs& a, int block) {
+  const long used = std::min(a.E, a.P);
+  const double rows = static_cast<double>(a.P) / used;
+  return used * (rows > block ? rows / block + 0.5 : 1.0) * ((a.N + 63) / 64);
+}
+bool takes_64_rows(const GemmArgs& a) { return a.P > 32l * std::min(a.E, a.P) && narrow_tiles(a, 64) >= 192; }
+}  // namespace
+
+// Where fp32 rows are rounded by this kernel, of the shapes of up to 64 rows per expert whose bf16 rows it takes
+// (skinny_gemm_applies): where it is faster than the cast kernel and the bf16 form behind each other.  It saves a
+// launch and a pass over the rows, but every column tile reads twice the bytes of the rows again, and fewer stages
+// fit the LDS.  The line was drawn on 3757 shapes (1 to 64 rows per expert, 4 to 128 experts, K 256 to 8192, N 512
+// to 8192, rows in order or gathered for one or two paths; both sides back to back in a graph; more rows lose: 32
+// x 120 rows 2048 -> 512 39.5 us cast and GEMM, 48.9 here): 28 of the 2899 it takes are more than 2 % slower than
+// cast and GEMM, the worst 6 % (128 x 28 rows 520 -> 1032 gathered 45.0 us cast, 47.7 here), and the mean is 11 %
+// faster.  Of 900 other shapes drawn from those ranges, half of them with ragged loads, it takes 772: 16 are over
+// 2 % slower (the worst 4 x 32 ragged rows 1792 -> 7168, 29.0 and 33.6), the mean is 13 % faster.  Not taken (us,
+// cast and GEMM, this kernel):
+//   - 64-row tiles with 10 MB of rows or more (64 x 64 rows 2048 -> 512 50.0 and 59.0), a K beyond 2048, 0.12 GB of
+//     weights (4 x 64 rows 2048 -> 8192 36.0 and 37.4), or rows gathered for several paths, which the cast reads only
+//     once, unless K is short (12 x 64 rows 768 -> 3072 for two paths 21.9 and 23.8);
+//   - 32 x 32 tiles with a K beyond 2048, whose chain four stages do not cover (4 x 8 rows 4096 -> 1024 16.5 and 18.6),
+//     except where the tiles reach most CUs (8 x 16 rows 4096 -> 1024 24.5 and 21.4, 12 x 8 rows 2560 -> 640 17.1 and 14.5);
+//   - 32 x 64 tiles with more than 32 rows and a K beyond 2048 (12 x 64 rows 3072 -> 768 36.2 and 38.5), with 16 MB of
+//     rows (128 x 28 rows 1536 -> 512 52.2 and 55.3), and a K from 2048 on whose few rows cost no time to cast beside 0.12 GB
+//     of weights (64 x 3 rows 2048 -> 1024 55.7 and 57.1).
+// cells: rows of x where they are gathered, 0 where they are not.
+bool skinny_gemm_takes_f32(const GemmArgs& a, int cells) {
+  const long used = std::min(a.E, a.P);
+  const double row_bytes = 4.0 * a.P * a.K, weight_bytes = 2.0 * used * a.N * a.K;
+  if (takes_64_rows(a))
+    return a.K <= 2048 && row_bytes <= 1e7 && weight_bytes <= 1.2e8 && (cells == 0 || cells >= a.P || a.K <= 512);
+  if (narrow_tiles(a, 32) <= 128)
+    return a.K <= 2048 || (a.K <= 4096 && used * ((a.N + 63) / 64) >= 96 && (a.K <= 2560 || a.P >= 16 * used));
+  if (a.P > 32 * used) return a.K <= 2048;
+  return row_bytes <= 1.6e7 && (a.K < 2048 || a.P >= 16 * used || weight_bytes <= 1.2e8);
+}
+
+// Shape of the tile.
 //   - 64 x 64 where experts have more than 32 rows and that makes a tile for most CUs (8 x 120 rows
 //     768 -> 3072 15.7 us, 19.3 with 32 x 64): with a short K three stages and three workgroups on a CU
 //     (16 x 64 rows 512 -> 2048 10.2 us, four stages 11.5), else four (8 x 120 rows 3072 -> 768 20.9, three 22.7).
@@ -447,25 +487,26 @@ bool skinny_gemm_applies(const GemmArgs& a) {
 //     1024 -> 4096 46.2 us, 50.0).
 //   - 32 x 64 otherwise (8 x 28 rows 4096 -> 1024 19.8 us, 32 x 32 22.4; 32 x 6 rows 4096 -> 1024 55.1 and 62.2).
 int launch_skinny_gemm(GemmArgs& a, int act, hipStream_t st) {
-  const long used = std::min(a.E, a.P);
-  const double rows = static_cast<double>(a.P) / used;
-  auto tiles = [&](int block) { return used * (rows > block ? rows / block + 0.5 : 1.0) * ((a.N + 63) / 64); };
+  const double rows = static_cast<double>(a.P) / std::min(a.E, a.P), tiles32 = narrow_tiles(a, 32);
+  const bool tall = takes_64_rows(a);
   if (a.x_f32) {
-    // fp32 rows take twice the room, so two stages of 64 x 64 are as many as leave three workgroups on a CU (16 x 60 rows
-    // 512 -> 2048 12.4 us, three stages 12.6, cast and bf16 14.1; a long K wants three: 2048 -> 512 18.4, two 22.7),
-    // four of 32 x 64 otherwise (64 x 8 rows 512 -> 1024 16.7, 32 x 32 24.7, cast and bf16 20.6; 8 x 3 rows 768 -> 3072
-    // 9.8, 12.9 and 11.7), and 32 x 32 only where those leave half of the CUs without a tile (8 x 28 rows 4096 -> 1024
-    // 21.9, 23.8 and 25.9; 8 x 3 rows 3072 -> 768 13.2, 13.5 and 12.2).
-    if (rows > 32 && tiles(64) >= 192)
-      return a.K <= 1024 ? launch_act<64, 2, 2, true>(a, act, st) : launch_act<64, 2, 3, true>(a, act, st);
-    if (tiles(32) <= 128) return launch_act<32, 1, 4, true>(a, act, st);
+    // fp32 rows take twice the room, so 64 x 64 tiles have three stages, two workgroups on a CU (4 x 33 rows 1024 -> 4096
+    // 11.8 us, two stages 16.5, cast and bf16 13.2; 8 x 40 rows 1024 -> 2048 12.0, 16.7 and 13.7), and two stages and three
+    // workgroups where there are two tiles per CU and K is short (16 x 64 rows 640 -> 2560 22.7, three stages 23.3) or K is
+    // hardly longer than the stages (384); 32 x 64 tiles have four (64 x 8 rows 512 -> 1024 16.7, 32 x 32 24.7, cast and bf16
+    // 20.6; 8 x 3 rows 768 -> 3072 9.8, 12.9 and 11.7), and 32 x 32 are taken only where those leave half of the CUs without a
+    // tile (8 x 28 rows 4096 -> 1024 22.1, 23.9 and 26.3).
+    if (tall)
+      return a.K <= 384 || (a.K <= 768 && narrow_tiles(a, 64) >= 512) ? launch_act<64, 2, 2, true>(a, act, st)
+                                                                    : launch_act<64, 2, 3, true>(a, act, st);
+    if (tiles32 <= 128) return launch_act<32, 1, 4, true>(a, act, st);
     return launch_act<32, 2, 4, true>(a, act, st);
   }
-  if (rows > 32 && tiles(64) >= 192) {
+  if (tall) {
     if (a.K <= 1024) return launch_act<64, 2, 3>(a, act, st);
     return launch_act<64, 2, 4>(a, act, st);
   }
-  if (tiles(32) <= 112 || (tiles(32) <= 160 && a.K <= 2048) || (rows <= 16 && a.K <= 1536)) return launch_act<32, 1, 6>(a, act, st);
+  if (tiles32 <= 112 || (tiles32 <= 160 && a.K <= 2048) || (rows <= 16 && a.K <= 1536)) return launch_act<32, 1, 6>(a, act, st);
   return launch_act<32, 2, 5>(a, act, st);
 }
 

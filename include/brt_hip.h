@@ -457,8 +457,8 @@ int brt_hip_combine_by_rows_gated(const void* src, void* dst, const void* gates,
  * brt_hip_grouped_gemm / _f32out / _routed / _routed_f32out / _by_rows on fp32 rows of x (16-byte aligned), which the
  * kernel rounds to bf16 itself: the bits of brt_hip_cast_f32_to_bf16 followed by the bf16 form, without that pass.
  * gather_in as in the routed forms, from the tag matrix (entries_per_cell = 0; row_tags_out as there) or the row
- * entries (entries_per_cell = k); else tags is ignored.  Only for shapes that the kernel for few rows takes:
- * brt_hip_grouped_gemm_f32in_supported says which (1), others are refused (BRT_E_UNSUPPORTED).
+ * entries (entries_per_cell = k); else tags is ignored.  Only for shapes that the kernel for few rows takes, others
+ * are refused (BRT_E_UNSUPPORTED); brt_hip_grouped_gemm_f32in_supported says where it is the faster way too (1).
  */
 int brt_hip_grouped_gemm_f32in_supported(int E, int P, int T, int K, int N, int gather_in);
 int brt_hip_grouped_gemm_f32in(const float* x, const void* const* weights, const void* const* biases,

@@ -1046,20 +1046,27 @@ def test_timed_grouped_gemm_gives_the_same_rows_and_plausible_clocks():
                                         d_loads.data_ptr(), E, P, K, N, ACT["none"], None, st) == -1
 
 
-@pytest.mark.parametrize("E,rows,K,N,act,bias", [
-    (8, 3, 768, 3072, "gelu", False), (8, 3, 3072, 768, None, True), (4, 30, 72, 320, "relu", True),  # 32-row tiles, K tails
-    (16, 60, 512, 2048, "gelu", True), (16, 60, 2048, 512, None, False), (8, 120, 136, 776, "gelu", False),  # 64 rows, N tails
-    (32, 6, 8, 64, None, True), (1, 1, 64, 8, None, False), (5, 33, 1288, 264, "gelu", True),
-    (6, 1000, 512, 1024, "gelu", True), (2, 4000, 256, 4096, None, False),  # shapes that are cast first
+@pytest.mark.parametrize("by_kernel,E,rows,K,N,act,bias", [
+    (1, 8, 3, 768, 3072, "gelu", False), (1, 24, 10, 72, 392, None, True),  # 32 x 64 tiles, K and N tails
+    (1, 16, 60, 2048, 512, None, False), (1, 16, 40, 200, 328, "relu", True),  # ... of more than 32 rows
+    (1, 32, 6, 8, 64, None, True), (1, 4, 30, 72, 320, "relu", True), (1, 1, 1, 64, 8, None, False),  # 32 x 32 tiles
+    (1, 5, 33, 1288, 264, "gelu", True), (1, 12, 17, 2568, 520, None, True),  # ... the last of a K beyond 2048
+    (1, 16, 50, 264, 1000, None, True), (1, 16, 60, 512, 2048, "gelu", True), (1, 16, 60, 520, 2040, "relu", False),  # 64 x 64, two stages
+    (1, 16, 60, 1096, 1032, "gelu", True), (1, 16, 60, 2048, 1024, None, False), (1, 4, 33, 1024, 4096, "relu", True),  # ... three
+    (0, 8, 3, 3072, 768, None, True), (0, 4, 8, 4096, 1024, "gelu", False), (0, 8, 120, 136, 776, "gelu", False),  # shapes that are cast first
+    (0, 6, 1000, 512, 1024, "gelu", True), (0, 2, 4000, 256, 4096, None, False),
 ])
-def test_fp32_rows_are_rounded_by_the_kernel(E, rows, K, N, act, bias):
+def test_fp32_rows_are_rounded_by_the_kernel(by_kernel, E, rows, K, N, act, bias):
     """fp32 rows give the bits of the cast kernel and the bf16 form: plain, gathered by row entries and by the tag
-    matrix, into bf16 and fp32; ragged loads with empty experts; values whose rounding ties, overflows or is lost."""
+    matrix, into bf16 and fp32; ragged loads with empty experts; values whose rounding ties, overflows or is lost.  The
+    shapes meant for the kernel are its own, and without the odd values it is what an fp32 product of the rounded
+    operands gives, to the error of K fp32 sums of both sides."""
     from brainstorm_amd import _lib, jit
     from brainstorm_amd._C import router as c_router
     from routing_cases import topk_mask
 
     T = E * rows
+    assert [_lib.lib().brt_hip_grouped_gemm_f32in_supported(E, T, T, K, N, g) for g in (0, 1)] == [by_kernel] * 2
     mask, _ = topk_mask(T, E, 1, seed=T + K)
     g = torch.Generator().manual_seed(K + N)
     x = torch.randn(T, K, generator=g)
@@ -1095,4 +1102,15 @@ def test_fp32_rows_are_rounded_by_the_kernel(E, rows, K, N, act, bias):
             assert torch.equal(bits(got), bits(want)) and torch.equal(*tags_of)
     with pytest.raises(NotImplementedError):
         jit.grouped_linear(y, got, table, bias_table, loads, K, N, act)
+    if by_kernel and act != "gelu":
+        y = torch.randn(T, K, generator=g).cuda()
+        jit._linear(y, got, table, bias_table, loads, K, N, act)
+        start, rounded = 0, y.bfloat16().double()
+        for e, load in enumerate(loads.tolist()):
+            r, w = rounded[start:start + load], ws[e].double()
+            want = r @ w.t() + (biases[e].double() if bias else 0.0)
+            # products of bf16 are exact in fp32: what errs are K additions (and the bias), each by at most 2^-23 of the sum of magnitudes
+            bound = (K + 1) * 2.0 ** -23 * (r.abs() @ w.abs().t() + (biases[e].double().abs() if bias else 0.0))
+            assert ((got[start:start + load].double() - (want.relu() if act else want)).abs() <= bound).all()
+            start += load
     del ws
