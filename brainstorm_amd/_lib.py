@@ -220,10 +220,10 @@ _calls = 0
 
 
 def call_count() -> int:
-    """Calls into the library that queued device work since the process started (every such call is one kernel launch, except index generation, the
-    compact route and the tag-index gather, which are two; a GEMM that rounds fp32 rows itself counts
-    as the cast and the GEMM whose work it does).  Tests use the difference around a
-    layer to pin how many launches a route costs."""
+    """Calls into the library that queued device work since the process started, read-backs of a few words
+    among them.  Every such call is one kernel launch, except the compact route, the tag-index gather and the throttled
+    top-1 route, which are two, and index generation and throttling, which are one or two by the size of the mask.
+    Tests use the difference around a layer to pin how many launches a route costs."""
     return _calls + (_native.calls() if _native is not None else 0)
 
 

@@ -537,7 +537,6 @@ PyObject* grouped_linear_of(const Args& a, bool takes_f32) {
     if (!scatter && !gates.defined() && brt_hip_grouped_gemm_f32in_supported(E, rows, cells, K, N, gather) == 1) {
       if (gather && !by_rows && tags_out.defined() && (tags_out.scalar_type() != at::kInt || tags_out.numel() < rows || !tags_out.is_cuda()))
         runtime_error("row_tags_out must be an int32 device vector with one entry per row");
-      ++g_calls;  // the rounding, whoever does it: a layer counts the same ops for any number of rows
       check(brt_hip_grouped_gemm_f32in(fptr(x), w, b, ptr(out), f32_out, iptr(loads), gather ? iptr(by_rows ? entries : tags) : nullptr,
                                        by_rows ? k : 0, E, rows, cells, K, N, act, gather, by_rows ? nullptr : iptr(tags_out), st));
       return none();
@@ -649,6 +648,7 @@ at::DataPtr read_back(const Tensor& t, size_t bytes, const char* what) {
   if (watch) {
     int32_t* const word = static_cast<int32_t*>(host.get()) + bytes / 4;
     __atomic_store_n(word, 0, __ATOMIC_RELEASE);
+    ++g_calls;
     if (brt_hip_copy_to_host(iptr(t), static_cast<int32_t*>(seen_from_device), static_cast<int>(bytes / 4), st) != BRT_OK)
       runtime_error(std::string(what) + ": " + brt_hip_last_error());
     Py_BEGIN_ALLOW_THREADS

@@ -524,8 +524,8 @@ def _switch_layer(brt_mod, defer, E, d, dff, cap, pad, dtype, seed, static=False
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_deferred_fused_dispatch_is_the_same_layer_in_four_launches(brt_mod, pad, dtype):
     """defer_dispatch=True: the expert's first kernel gathers its rows from the cells, no dispatch
-    kernel runs.  Same caller code, bit-identical result, and the layer is four calls into the
-    library (index generation, two grouped GEMMs, the tag-driven combine) against five."""
+    kernel runs and no loads are read back.  Same caller code, bit-identical result, and the layer is five calls into the
+    library (hot mask, index generation, two grouped GEMMs, the tag-driven combine) against seven."""
     from brainstorm_amd import _lib
 
     T, E, d, dff, cap = 2048, 16, 256, 512, 160
@@ -541,9 +541,10 @@ def test_deferred_fused_dispatch_is_the_same_layer_in_four_launches(brt_mod, pad
         results.append(layer(residual, score))
         calls.append(_lib.call_count() - before)
         assert results[-1].data_ptr() == residual.data_ptr()  # combined in place, as the reference does
-    # topk mask, index generation, [dispatch,] (casts of fp32 operands,) GEMM, GEMM, combine
+    # topk mask, index generation, [read-back of the loads, dispatch,] (casts of fp32 rows, too many for the GEMM to round
+    # them itself,) GEMM, GEMM, combine
     casts = 2 if dtype == torch.float32 else 0
-    assert calls[0] == 6 + casts and calls[1] == 5 + casts, calls
+    assert calls[0] == 7 + casts and calls[1] == 5 + casts, calls
     assert torch.equal(results[0], results[1])
     assert not torch.equal(results[0], hidden)
     # static_rows=True: index generation moves the rows itself (one call for the two), nothing is
@@ -554,6 +555,20 @@ def test_deferred_fused_dispatch_is_the_same_layer_in_four_launches(brt_mod, pad
     out = layer(hidden.clone(), score)
     assert _lib.call_count() - before == 5 + casts
     assert torch.equal(out, results[0])
+
+
+@pytest.mark.parametrize("T,casts", [(512, 0), (2048, 2)])
+def test_fp32_layer_casts_only_rows_that_are_many(brt_mod, T, casts):
+    """mask, route with rows, GEMM, GEMM, combine: fp32 rows are cast before a GEMM only where it does not round them."""
+    from brainstorm_amd import _lib
+
+    g = torch.Generator().manual_seed(T)
+    hidden, score = torch.randn(T, 256, generator=g).cuda(), torch.randn(T, 16, generator=g).cuda()
+    layer = _switch_layer(brt_mod, False, 16, 256, 512, T, False, torch.float32, seed=33, static=True)
+    layer(hidden.clone(), score)
+    before = _lib.call_count()
+    layer(hidden.clone(), score)
+    assert _lib.call_count() - before == 5 + casts
 
 
 def test_deferred_rows_fill_themselves_when_anything_else_reads_them(brt_mod):
@@ -626,7 +641,7 @@ def test_compact_route_through_the_router_objects_top1(brt_mod, caps):
     """compact_route=True: the topk protocol hands the fabric path ids, route_by_path lays the route
     out, the first GEMM gathers its rows by the row-entry vector, the tag-driven combine (or, given
     the residual, the last GEMM itself) puts them back.  Same caller code as the dense layer, the
-    same bits, five calls into the library (four with the folded combine) against six."""
+    same bits, five calls into the library (four with the folded combine) against seven."""
     from brainstorm_amd import _lib
 
     T, E, d, dff = 2048, 16, 256, 512
@@ -635,7 +650,7 @@ def test_compact_route_through_the_router_objects_top1(brt_mod, caps):
     score = torch.randn(T, E, generator=g).cuda()
     caps = caps or {}
     variants = [
-        (dict(caps), False, 6),                                                   # mask, indexgen, dispatch, 2 GEMMs, combine
+        (dict(caps), False, 7),                                                   # mask, indexgen, read-back, dispatch, 2 GEMMs, combine
         (dict(caps, compact_route=True), False, 6),                               # gate, route, dispatch_by_rows, 2 GEMMs, combine
         (dict(caps, compact_route=True, defer_dispatch=True), False, 5),          # gate, route, gathering GEMM, GEMM, combine
         (dict(caps, compact_route=True, defer_dispatch=True), True, 4),           # gate, route, gathering GEMM, scattering GEMM
@@ -668,7 +683,7 @@ def test_compact_route_through_the_router_objects_top2(brt_mod, weighted):
     score = torch.softmax(torch.randn(T, E, generator=g), dim=1).cuda()
     caps = {"supported_capacities": [450]}  # some cells lose a path, a few both
     results = []
-    for fabric_kwargs, want_calls in ((dict(caps), 6), (dict(caps, compact_route=True), 6),
+    for fabric_kwargs, want_calls in ((dict(caps), 7), (dict(caps, compact_route=True), 6),  # (the first reads the loads back)
                                       (dict(caps, compact_route=True, defer_dispatch=True), 5)):
         layer = _moe_layer(brt_mod, E, d, dff, 2, torch.bfloat16, 54, fabric_kwargs, weighted=weighted)
         layer(hidden.clone(), score)
