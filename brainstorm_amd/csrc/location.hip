@@ -91,7 +91,6 @@ ScanGeometry scan_geometry(int T, int E, bool tag_mode, bool whole_ok) {
   g.ep_shift = shift;
   g.waves_pb = kWavesPB;
   const int rps = kWave >> shift;  // rows per load instruction
-  constexpr int forced_bands = 0;  // a fixed number of workgroups, for experiments
   // Small masks (decode-sized batches) take one launch of one workgroup, the column sums of its
   // wavefronts meeting in LDS.  Up to four loads per lane of a 4-wavefront workgroup that is
   // the ordinary kernel with a single band (16 x 8: 4.1 us, 128 x 8: 4.7 us); up to one batch of
@@ -100,13 +99,13 @@ ScanGeometry scan_geometry(int T, int E, bool tag_mode, bool whole_ok) {
   // over the whole matrix, which one CU does slowly: beyond 128 rows they take the two launches
   // (512 x 16: 8.9 us against 10.6 us).  Larger masks are faster spread over many CUs, launch
   // cost and all.
-  if (forced_bands <= 0 && E <= kWave && static_cast<long>(T) <= 4l * kWavesPB * rps) {
+  if (E <= kWave && static_cast<long>(T) <= 4l * kWavesPB * rps) {
     long rows_pw = (static_cast<long>(T) + kWavesPB - 1) / kWavesPB;
     g.rows_pw = static_cast<int>(std::max<long>((rows_pw + rps - 1) / rps * rps, rps));
     g.bands = 1;
     return g;
   }
-  if (forced_bands <= 0 && E <= kWave && (!tag_mode || T <= 128) &&
+  if (E <= kWave && (!tag_mode || T <= 128) &&
       static_cast<long>(T) <= static_cast<long>(kWavesSingle) * kBatch * rps) {
     long rows_pw = (static_cast<long>(T) + kWavesSingle - 1) / kWavesSingle;
     rows_pw = std::max<long>((rows_pw + rps - 1) / rps * rps, rps);
@@ -118,7 +117,7 @@ ScanGeometry scan_geometry(int T, int E, bool tag_mode, bool whole_ok) {
   // One launch in which every workgroup adds up all rows above its own itself (figures at the head of the file).  The
   // gain shrinks with the rows to add up: at 64 loads per lane (kWholeLoads) it is 1.2 us for seats, 0.4 us for tags.
   const long loads = (static_cast<long>(T) + rps - 1) / rps;
-  if (forced_bands <= 0 && whole_ok && whole_rows(E) && E <= kWave && loads <= kWholeLoads) {
+  if (whole_ok && whole_rows(E) && E <= kWave && loads <= kWholeLoads) {
     g.rows_pw = kWholeRows * rps;
     g.bands = static_cast<int>((loads + kWholeRows * kWavesWhole - 1) / (kWholeRows * kWavesWhole));
     g.waves_pb = kWavesWhole;
@@ -129,7 +128,7 @@ ScanGeometry scan_geometry(int T, int E, bool tag_mode, bool whole_ok) {
   // over earlier bands every band has to form.
   const long one_batch = static_cast<long>(kWavesPB) * kBatch * rps;
   const int fit = static_cast<int>(std::min<long>(kMaxBands, (T + one_batch - 1) / one_batch));
-  const int want = forced_bands > 0 ? forced_bands : std::max(128, fit);
+  const int want = std::max(128, fit);
   long rows_pb = (static_cast<long>(T) + want - 1) / want;
   rows_pb = std::max<long>(rows_pb, (static_cast<long>(T) + kMaxBands - 1) / kMaxBands);
   long rows_pw = (rows_pb + kWavesPB - 1) / kWavesPB;
