@@ -467,8 +467,6 @@ PyObject* combine_by_rows(const Args& a) {  // in_data, path_ids, seat_rows, wei
 }
 
 // ---- grouped GEMM ------------------------------------------------------------------------------------
-// x, out, weight_table, bias_table, loads, in_features, out_features, activation code, tags, gather, scatter,
-// rows or None, row_entries, entries_per_cell, row_tags_out, gates
 Tensor rounded_to_bf16(const Tensor& given) {
   const Tensor in = dense(given);
   const c10::DeviceGuard guard(in.device());
@@ -477,6 +475,8 @@ Tensor rounded_to_bf16(const Tensor& given) {
   return out;
 }
 
+// x, out, weight_table, bias_table, loads, in_features, out_features, activation code, tags, gather, scatter,
+// rows or None, row_entries, entries_per_cell, row_tags_out, gates
 // takes_f32: fp32 rows of x are taken too, rounded to bf16 by the GEMM itself where its kernel does that
 PyObject* grouped_linear_of(const Args& a, bool takes_f32) {
   Tensor x = a.tensor(0);

@@ -84,7 +84,6 @@ def test_indices_general_mask_values_and_misaligned_buffers(hip):
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
 
 
-# on both sides of the widest matrix that is read through 32-bit byte offsets, and where those would wrap round
 @pytest.mark.parametrize("T,E", [
     (513, 16), (4096, 16), (4097, 16),        # behind the one-workgroup form; the last of one launch, the first of two
     (129, 64), (1024, 64), (1025, 64), (700, 40), (4000, 12), (8189, 8), (16384, 4),
@@ -114,6 +113,7 @@ def test_indices_of_masks_one_launch_takes(hip, T, E):
     assert np.array_equal(hip.host(both), o_idx) and np.array_equal(hip.host(loads), o_loads)
 
 
+# on both sides of the widest matrix that is read through 32-bit byte offsets, and where those would wrap round
 @pytest.mark.parametrize("T,E", [(9, (1 << 20) - 1), (9, 1 << 20), (6, (1 << 24) + 8)])
 def test_index_generation_of_very_many_paths(hip, T, E):
     mask = np.random.default_rng(E).integers(0, 2, (T, E), dtype=np.int8).astype(np.int32)

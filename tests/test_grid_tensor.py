@@ -233,11 +233,12 @@ def test_annotator_takes_no_cells():
 def test_flows_are_wrapped_the_same_with_and_without_the_native_module(monkeypatch, built):
     """Wrapping shares storage and stacks, copies the extra attributes, keeps autograd's link, and leaves a buffer that
     is not filled yet alone -- in native code and, where that has not been built, in Python."""
-    from brainstorm_amd import _lib
     from brainstorm_amd.runtime import deferred
 
     if not built:
         monkeypatch.setattr(_lib, "native_or_none", lambda: None)
+    elif _lib.native_or_none() is None:
+        pytest.skip("the native module has not been built")
     base = torch.randn(4, 3, requires_grad=True)
     tags, loads, extra = [None], [torch.tensor([4])], {"key": 1}
     grid = init_grid_tensor(base, tags, loads, extra)
@@ -252,6 +253,28 @@ def test_flows_are_wrapped_the_same_with_and_without_the_native_module(monkeypat
     lazy = deferred.lazy_tensor(torch.zeros(3), lambda b: filled.append(b.fill_(2.0)))
     assert not filled and lazy.shape == (3,)
     assert float(lazy.sum()) == 6.0 and len(filled) == 1
+
+
+@pytest.mark.parametrize("sizes", [[2, 0, 3], [0, 0], [5], [1] * 7])
+def test_fused_cells_are_split_the_same_with_and_without_the_native_module(monkeypatch, sizes):
+    """Rows, loads and tags of every path as views: loads read or handed over, on a fixed stride, of a tensor whose gradient is
+    asked for and of one that is not contiguous."""
+    import brt._C.router as c_router
+
+    if _lib.native_or_none() is None:
+        pytest.skip("the native module has not been built")
+    n, loads = sum(sizes), torch.tensor(sizes, dtype=torch.int32)
+    tags = torch.arange(1, n + 1, dtype=torch.int32)
+    for rows in (torch.randn(n, 3), torch.randn(n, 3, requires_grad=True), torch.randn(3, n).t(), torch.randn(n)):
+        for kwargs in ({}, {"is_load_split": True}, {"is_tag_split": True, "tags": tags}, {"host_loads": sizes}, {"max_path_padding": True}):
+            native = c_router.split_fused_cells_to_paths(rows, loads, **kwargs)
+            with monkeypatch.context() as patch:
+                patch.setattr(_lib, "native_or_none", lambda: None)
+                plain = c_router.split_fused_cells_to_paths(rows, loads, **kwargs)
+            assert [len(part) for part in native] == [len(part) for part in plain]
+            for got, want in zip(sum(native, []), sum(plain, [])):
+                assert torch.equal(got, want) and got.data_ptr() == want.data_ptr() and got.stride() == want.stride()
+                assert got.requires_grad == want.requires_grad and type(got) is torch.Tensor
 
 
 def test_loads_without_data_are_refused():

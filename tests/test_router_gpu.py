@@ -1190,6 +1190,37 @@ def test_words_read_back_by_the_host(n):
             assert _lib.native().int_list(on_device) == view.tolist()
 
 
+def test_words_read_back_by_threads_on_streams_of_their_own():
+    """Each thread gets its own words, read over and over through blocks that the threads hand on to each other, behind
+    little work and, now and then, behind more than the host watches for."""
+    import threading
+
+    from brainstorm_amd import _lib
+
+    wrong = []
+
+    def read(thread):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                words = torch.arange(64, dtype=torch.int32, device="cuda")
+                for i in range(150):
+                    if i % 50 == thread:
+                        torch.cuda._sleep(4_000_000)
+                    n = 1 + (7 * i + thread) % 64
+                    want = [thread * 1_000_000 + i * 100 + w for w in range(n)]
+                    if _lib.native().int_list(words[:n] + (thread * 1_000_000 + i * 100)) != want:
+                        wrong.append((thread, i))
+        except Exception as error:  # (a thread's exception ends the thread only)
+            wrong.append((thread, error))
+
+    threads = [threading.Thread(target=read, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
 @pytest.mark.parametrize("T,E,dtype", [
     (1, 1, torch.float32), (5, 8, torch.float16), (128, 64, torch.bfloat16), (129, 64, torch.float32), (100, 3, torch.bfloat16),
     (777, 5, torch.float32), (33, 33, torch.float32), (127, 40, torch.float16), (65, 17, torch.float32),  # several bands of few rows
