@@ -143,7 +143,7 @@ ScanGeometry scan_geometry(int T, int E, bool tag_mode, bool whole_ok) {
 // Bands of a throttled top-1 route: always the two-launch form (its first launch reads the scores anyway).  A mask that one
 // workgroup of eight wavefronts would hold is spread over workgroups of four with at most eight loads each: a load costs
 // the selection of its rows' best score, one after the other (128 x 64 in one workgroup 15.5 us, 7.6 so, 10.1 as
-// mask and throttle; 64 x 33 9.5, 7.7 and 9.2).
+// mask, two fills and throttle; 64 x 33 9.5, 7.7 and 9.2).
 ScanGeometry top1_geometry(int T, int E) {
   constexpr int kMostLoads = 8;
   ScanGeometry g = scan_geometry(T, E, true, false);
