@@ -678,12 +678,38 @@ using namespace brt;
 
 namespace {
 
+// Tile of the 160-row kernel.  A wavefront owns 160 x 64 outputs (7 LDS fragment reads feed 10 MFMAs); a
+// workgroup is 2, 3 or 4 of them side by side.  The kernel is bound by how fast a CU can fill
+// its L1 (about 29 KB/us, L2 hits included), so the width is the one that gives the busiest CU
+// the fewest operand bytes: wide tiles re-read the activation rows less often, narrow ones
+// keep all CUs busy when there are few tiles (only the 2-wavefront tile fits twice on a CU).
+struct Width {
+  int waves;
+  double cost;  // operand rows the busiest CU streams per K
+};
+Width width_of_160_row_tiles(int P, int E, int N) {
+  const int cus = device_cus();
+  const long row_blocks = estimated_row_blocks(P, E);
+  Width best{0, 0};
+  for (int waves = 4; waves >= 2; --waves) {
+    const long tiles = row_blocks * ((N + 64 * waves - 1) / (64 * waves));
+    const long slots = static_cast<long>(cus) * (waves == 2 ? 2 : 1);
+    const double rounds = static_cast<double>((tiles + slots - 1) / slots) * (waves == 2 ? 2 : 1);
+    const double cost = rounds * (160 + 64 * waves);
+    if (best.waves == 0 || cost < best.cost) best = {waves, cost};
+  }
+  return best;
+}
+
 // The rule for the ping-pong kernel (its reasons where the kernel is chosen).
 bool wide_tiles_come_in_rounds(const GemmArgs& a) {
   if (!pingpong_gemm_applies(a) || static_cast<long>(a.P) <= static_cast<long>(a.E) * 160) return false;
   const long tiles = (static_cast<long>(a.P + 255) / 256 + (a.E + 1) / 2) * ((a.N + 255) / 256);
   const long cus = device_cus();
-  return tiles >= 2 * cus || (4 * tiles >= 3 * cus && tiles <= cus);
+  if (4 * tiles < 3 * cus) return false;
+  if (4 * tiles <= 5 * cus || 5 * tiles >= 8 * cus) return true;
+  const Width other = width_of_160_row_tiles(a.P, a.E, a.N);
+  return other.waves != 2 && (2 * tiles >= 3 * cus || other.cost > 2 * (160 + 64 * 4));
 }
 
 // Shapes whose fp32 rows the few-rows kernel rounds itself when asked to; where that is the faster way, skinny_gemm_takes_f32 says.
@@ -747,15 +773,19 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   }
   // Kernel choice.  Experts that average more than one row block take the ping-pong kernel
   // (grouped_gemm_pingpong.hip), whose 256 x 256 tile moves a third fewer operand bytes per flop,
-  // when its tiles come in whole rounds over the CUs: at least two rounds, or one round that most
-  // CUs take part in.  In between (one to two tiles per CU) a CU with two tiles sets the time and
-  // the smaller tiles of the 160-row kernel spread better.  The tile count is an estimate: the
+  // when its tiles fill a round over the CUs to three quarters or more.  The tile count is an estimate: the
   // loads are on the device; an expert's last row block is taken as half full.  Measured in one
   // process against the 160-row kernel: 8 experts x 4096 rows 2048 -> 8192 -> 2048 1165 / 993 ->
   // 962 / 793 us, the ragged task-MoE shape 1585 / 1374 -> 1355 / 1211 us, the top-2 shape's
-  // expanding GEMM (1232 tiles) 212 -> 166 us, 8 x 1824 rows 4096 -> 1024 (256 tiles) 146 -> 99 us;
-  // the top-2 shape's contracting GEMM (308 tiles on 256 CUs) 162 -> 173 us.  The rule is the same
-  // for gathered, scattered and fp32-output rows: a gathering 1024 -> 4096 GEMM with GELU over 32768
+  // expanding GEMM (1232 tiles) 212 -> 166 us, 8 x 1824 rows 4096 -> 1024 (256 tiles) 146 -> 99 us; with one to two rounds, whose
+  // end is cut into units, 8 x 1000 rows 4096 -> 2048 148 -> 115 us, 64 x 400 rows 3072 -> 768 172 -> 145, 4 x 8000 rows 256 -> 1024 58 -> 34
+  // (60 shapes of 1.0 to 2.0 rounds: 1.29 times as fast in the mean).  Between 1.25 and 1.5 rounds the end is too long to be
+  // cut and too short to fill the second round, and where the 160-row kernel is through in two rounds of its own
+  // the two are level on average (60 x 270 rows 4096 -> 1024 170 us there, 188 here; 12 x 1092 rows
+  // 5888 -> 1472 216 and 257; 64 x 337 rows 2816 -> 704 156 and 128): those stay there, and those of up to 1.6 rounds for which two
+  // narrow workgroups of it fit a CU (4 x 8070 rows 1280 -> 640 62 and 68).  Below three quarters of a round the 160-row
+  // tiles spread better (4 x 4060 rows 1792 -> 448, half a round, 37.9 us there, 46.9 here).
+  // The rule is the same for gathered, scattered and fp32-output rows: a gathering 1024 -> 4096 GEMM with GELU over 32768
   // rows of 16 experts takes 437 us on the 160-row kernel and 336 us here.
   if (wide_tiles_come_in_rounds(a)) return launch_pingpong_gemm(a, act, as_stream(stream));
   if (skinny_gemm_applies(a)) return launch_skinny_gemm(a, act, as_stream(stream));
@@ -764,29 +794,10 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
     if (act == BRT_ACT_RELU) return launch_f32<BRT_ACT_RELU>(a, as_stream(stream));
     return launch_f32<BRT_ACT_NONE>(a, as_stream(stream));
   }
-  // Tile choice.  A wavefront owns 160 x 64 outputs (7 LDS fragment reads feed 10 MFMAs); a
-  // workgroup is 2, 3 or 4 of them side by side.  The kernel is bound by how fast a CU can fill
-  // its L1 (about 29 KB/us, L2 hits included), so the shape is the one that gives the busiest CU
-  // the fewest operand bytes: wide tiles re-read the activation rows less often, narrow ones
-  // keep all CUs busy when there are few tiles (only the 2-wavefront tile fits twice on a CU).
-  constexpr int forced = 0;  // a fixed tile shape (21..24), for experiments
-  int shape = forced;
-  if (shape == 0) {
-    const int cus = device_cus();
-    const long row_blocks = estimated_row_blocks(P, E);
-    double best = 0;
-    for (int waves = 4; waves >= 2; --waves) {
-      const long tiles = row_blocks * ((N + 64 * waves - 1) / (64 * waves));
-      const long slots = static_cast<long>(cus) * (waves == 2 ? 2 : 1);
-      const double rounds = static_cast<double>((tiles + slots - 1) / slots) * (waves == 2 ? 2 : 1);
-      const double cost = rounds * (160 + 64 * waves);  // operand rows the busiest CU streams per K
-      if (shape == 0 || cost < best) { best = cost; shape = 20 + waves; }
-    }
-  }
-  if (shape == 24) return launch<5, 2, 4>(a, act, as_stream(stream));
-  if (shape == 23) return launch<5, 2, 3>(a, act, as_stream(stream));
-  if (shape == 22) return launch<5, 2, 2>(a, act, as_stream(stream));
-  return launch<5, 1, 4>(a, act, as_stream(stream));
+  const int waves = width_of_160_row_tiles(P, E, N).waves;
+  if (waves == 4) return launch<5, 2, 4>(a, act, as_stream(stream));
+  if (waves == 3) return launch<5, 2, 3>(a, act, as_stream(stream));
+  return launch<5, 2, 2>(a, act, as_stream(stream));
 }
 
 }  // namespace

@@ -38,6 +38,12 @@
 //     it loads in registers for any kind of row, so a gathered row (its cell's offset) and an
 //     activation or weight row (row times pitch) are the same load.  The cells pass through the
 //     first bytes of the stages once, before any operand lands there.
+//   - What the list of tiles holds beyond whole rounds over the CUs would keep a few of them busy for as long as a whole round, and the
+//     experts' last row blocks, which hold few rows, for more than half as long (the weights of 256 columns come into one CU at
+//     40 GB/s).  Where that is at most half a round it is cut into units of 256 rows x 64 columns: each wavefront loads its share of a
+//     K-step and multiplies 32 rows (or 32 x 32 blocks of fewer rows) of a ring of four to eight K-steps, one barrier per K-step, the loads
+//     between the MFMAs (in front of them a K-step took 0.65 us instead of 0.53).  Bound by the fills of LDS, 40 KB a
+//     K-step at 64 bytes a clock.  32768 rows of 16 experts 4096 -> 1024 268 -> 229 us, 32 x 1000 rows 512 -> 1024 61 -> 50.
 //   - The epilogue sends the tile out 32 rows at a time through each wavefront's own corner of
 //     LDS (the stages are dead by then), full 128-byte rows per store.
 #include <algorithm>
@@ -70,6 +76,13 @@ constexpr int kSub = kBK / 16;                        // MFMA k-steps per stage
 constexpr int kHead = 4;                              // MFMAs of a C phase issued ahead of the barrier
 constexpr uint32_t kOutOfRange = 0x80000000u;         // buffer offset past any extent: reads as zero
 constexpr int kXcds = 8, kCusPerXcd = 32, kPatchRows = 4;
+constexpr int kRound = kXcds * kCusPerXcd;  // tiles of a whole round
+// The end of the list that is cut into units (see the kernel).  A unit of 256 rows takes 0.4 to 0.5 of a tile's time (4 x 1024 rows
+// 4096 -> 1024, 256 units: 40 us against 102 us for the 64 tiles they are made of), one of up to 128 rows a third (38 us and 73), so two
+// rounds of them, 128 tiles, are what a round of whole tiles costs: 16 x 256 rows 4096 -> 2048 105 us against 108.  In a list of more
+// than ten rounds the CUs are no longer in step, and nothing is left to gain (98 blocks 2048 -> 8192, 12.25 rounds: 763 us cut, 756 not).
+constexpr int kFewRows = 128, kMostCut = 128, kMostRounds = 10;
+constexpr int kUnitCols = 64;
 
 __device__ __forceinline__ i32x4 make_rsrc(const void* p, size_t bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(p);
@@ -106,6 +119,8 @@ __device__ __forceinline__ void stream_out(const u32x4& v, u32x4* p) {
 __device__ __forceinline__ void wait_loads_all() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
 // everything but the 8 loads this wavefront issued in the current K-step has landed
 __device__ __forceinline__ void wait_loads_but_8() { asm volatile("s_waitcnt vmcnt(8)" : : : "memory"); }
+template <int N>
+__device__ __forceinline__ void wait_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory"); }
 __device__ __forceinline__ void block_barrier() {
   asm volatile("" ::: "memory");
@@ -130,53 +145,127 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // also its ping-pong group; wn is its 64 columns.
   const int wm = wave >> 2, wn = wave & 3;
 
-  // ---- which tile: patch order (grouped_gemm.hip) ----------------------------------------------
-  const int xcd = blockIdx.x % kXcds, idx = blockIdx.x / kXcds;
-  const int t = ((idx / kCusPerXcd) * kXcds + xcd) * kCusPerXcd + idx % kCusPerXcd;
-  // Every wavefront finds the tile by itself, the weight pointers fetched in the same round trip as the loads: no
+  // ---- which tile ------------------------------------------------------------------------------
+  // The list holds the tiles of the row blocks in patch order (grouped_gemm.hip).  What it holds beyond whole rounds over
+  // the CUs is cut into units of 256 rows x 64 columns, four for a tile, if it is little: first the experts' last row blocks
+  // of few rows, as far as needed (`moved` blocks, taken out of the list and put behind it), then the end of the list.
+  // Every wavefront finds its tile by itself, the weight pointers fetched in the same round trip as the loads: no
   // exchange through LDS and no second trip stand before the first requests, and the K loop starts when the first K-step
   // has landed.  Against one wavefront that looks, LDS, a load of the pointer and a wait for two K-steps:
   // 16 x 2048 rows 1024 -> 4096 + GELU 278.8 -> 274.3 us (0.6 us a tile), 64 x 400 rows 768 -> 3072 174.1 -> 169.7, 8 x 4096 rows
   // 2048 -> 8192 907.9 -> 899.0; contracting GEMMs, whose tiles take four times as long, within 0.5 %.
   // (The 160-row kernel, which starts once per CU, lost 0.5 to 1 % by the same change.)
-  int e = -1, carry_t = 0, carry_m = 0, row0 = 0, rows = 0, seat0 = 0, n0 = 0;
+  // A lane looks at two experts: up to 128 of them take one round trip and one scan.
+  const int xcd = blockIdx.x % kXcds, idx = blockIdx.x / kXcds;
+  const int t = ((idx / kCusPerXcd) * kXcds + xcd) * kCusPerXcd + idx % kCusPerXcd;
+  const int tn = a.tiles_n;
+  struct Two {
+    int m[2], many[2], few[2];  // rows; row blocks of more than kFewRows rows, and of fewer (one at most)
+    int incl_m, incl_b;         // rows and blocks up to this lane's experts and with them (blocks of few rows in the low byte)
+    uint64_t w[2];
+  };
+  auto read_two = [&](int base) {
+    Two v;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int el = base + 2 * lane + i, at = min(el, a.E - 1);
+      const int given = a.loads[at];
+      v.w[i] = reinterpret_cast<uint64_t>(a.w[at]);
+      v.m[i] = el < a.E ? given : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int over = v.m[i] & (kBM - 1);
+      v.many[i] = (v.m[i] >> 8) + (over > kFewRows ? 1 : 0);
+      v.few[i] = over > 0 && over <= kFewRows ? 1 : 0;
+    }
+    v.incl_b = wave_inclusive_scan((v.many[0] + v.many[1]) << 8 | (v.few[0] + v.few[1]));
+    v.incl_m = wave_inclusive_scan(v.m[0] + v.m[1]);
+    return v;
+  };
+  auto over_tn = [&](int n) {  // n / tn
+    const int q = static_cast<int>(__umulhi(static_cast<uint32_t>(n), a.tiles_n_inverse));
+    return n - q * tn >= tn ? q + 1 : q;
+  };
+  Two two = read_two(0);
+  const int sums = read_lane(two.incl_b, kWave - 1);
+  int many = sums >> 8, few = sums & 255;
+  for (int base = 2 * kWave; base < a.E; base += 2 * kWave) {
+    const int more = read_lane(read_two(base).incl_b, kWave - 1);
+    many += more >> 8, few += more & 255;
+  }
+  const int tiles = (many + few) * tn, rest = tiles & (kRound - 1);
+  int moved = min(few, over_tn(rest + tn - 1));
+  int cut = max(moved * tn, rest);  // tiles
+  if (cut > kMostCut || tiles > kMostRounds * kRound || tiles + 3 * cut > a.grid - (a.row_tags_out != nullptr ? 1 : 0)) cut = 0;
+  if (cut == 0) moved = 0;
+  const int listed = tiles - moved * tn, whole = tiles - cut, used = tiles + 3 * cut;
+  if (t >= used) {
+    // Surplus workgroups clear the tags of the rows no path owns, 256 of them a step.  The grid holds P / 256 + E row blocks
+    // (rounded up) per column tile, the experts use at most (total + 255 E) / 256, and the cut leaves at least one.
+    if (ROUTED && a.row_tags_out != nullptr && tid < kBM) {
+      long total = 0;
+      for (int base = 0; base < a.E; base += 2 * kWave) total += read_lane(read_two(base).incl_m, kWave - 1);
+      for (long r = total + static_cast<long>(t - used) * kBM + tid; r < a.P; r += static_cast<long>(a.grid - used) * kBM) a.row_tags_out[r] = 0;
+    }
+    return;
+  }
+  const bool narrow = t >= whole;
+  const int tile = narrow ? whole + ((t - whole) >> 2) : t;
+  const bool apart = tile >= listed;  // of a moved block
+  const int place = apart ? tile - listed : tile;
+  int e = 0, row0 = 0, rows = 0, seat0 = 0, n0 = 0;
   const __bf16* w_e = nullptr;
-  for (int base = 0; base < a.E; base += kWave) {
-    const int el = min(base + lane, a.E - 1);
-    const int given = a.loads[el], m = base + lane < a.E ? given : 0;
-    const uint64_t wp = reinterpret_cast<uint64_t>(a.w[el]);
-    const int tiles = (m + kBM - 1) / kBM * a.tiles_n;
-    const int incl_t = wave_inclusive_scan(tiles), incl_m = wave_inclusive_scan(m);
-    const int first = carry_t + incl_t - tiles;
-    const unsigned long long hit = __ballot(t >= first && t < first + tiles);
+  for (int base = 0, carry_many = 0, carry_few = 0, carry_m = 0;;) {
+    const int few_own = two.few[0] + two.few[1], many_own = two.many[0] + two.many[1];
+    const int few_with = carry_few + (two.incl_b & 255), few_before = few_with - few_own;
+    const int many_with = carry_many + (two.incl_b >> 8);
+    const int first = apart ? min(few_before, moved) : many_with - many_own + max(few_before - moved, 0);
+    const int last = apart ? min(few_with, moved) : many_with + max(few_with - moved, 0);
+    const unsigned long long hit = __ballot(place >= first * tn && place < last * tn);
     if (hit != 0) {
       const int src = __builtin_ctzll(hit);
-      const int mine = read_lane(m, src), blocks = (mine + kBM - 1) / kBM;
-      const int local = t - read_lane(first, src), per_group = kPatchRows * a.tiles_n;
-      const int full = blocks / kPatchRows, g = min(local / per_group, full);
-      const int r = local - g * per_group, wide = g < full ? kPatchRows : blocks - full * kPatchRows;
-      const int col = r / wide, block = g * kPatchRows + r - col * wide;
-      e = base + src;
+      int local = place - read_lane(first, src) * tn;  // among the tiles of the lane's two experts
+      const int before = read_lane(few_before, src), few0 = read_lane(two.few[0], src), few1 = read_lane(two.few[1], src);
+      const int many0 = read_lane(two.many[0], src), many1 = read_lane(two.many[1], src);
+      const int m0 = read_lane(two.m[0], src), m1 = read_lane(two.m[1], src);
+      // blocks of the first of them that are looked for
+      const int moved0 = few0 != 0 && before < moved ? 1 : 0, moved1 = few1 != 0 && before + few0 < moved ? 1 : 0;
+      const int blocks0 = apart ? moved0 : many0 + few0 - moved0;
+      const bool second = local >= blocks0 * tn;
+      if (second) local -= blocks0 * tn;
+      const int m = second ? m1 : m0;
+      int block, col;
+      if (apart) {
+        block = second ? many1 : many0;
+        col = local;
+      } else {
+        const int blocks = second ? many1 + few1 - moved1 : blocks0;
+        const int g = min(over_tn(local) / kPatchRows, blocks / kPatchRows);
+        const int r = local - g * kPatchRows * tn, wide = min(blocks - g * kPatchRows, kPatchRows);
+        col = wide == 4 ? r >> 2 : wide == 3 ? static_cast<int>(__umulhi(static_cast<uint32_t>(r), 0x55555556u)) : wide == 2 ? r >> 1 : r;
+        block = g * kPatchRows + r - col * wide;
+      }
+      const uint64_t wp = second ? two.w[1] : two.w[0];
+      e = base + 2 * src + (second ? 1 : 0);
       seat0 = block * kBM;
-      row0 = carry_m + read_lane(incl_m - m, src) + seat0;
-      rows = min(min(kBM, mine - seat0), a.P - row0);
+      row0 = carry_m + read_lane(two.incl_m, src) - m1 - (second ? 0 : m0) + seat0;
+      rows = min(min(kBM, m - seat0), a.P - row0);
       n0 = col * kBN;
       w_e = reinterpret_cast<const __bf16*>(static_cast<uint64_t>(static_cast<uint32_t>(read_lane(static_cast<int>(wp), src))) |
                                             static_cast<uint64_t>(static_cast<uint32_t>(read_lane(static_cast<int>(wp >> 32), src))) << 32);
       break;
     }
-    carry_t += read_lane(incl_t, kWave - 1);
-    carry_m += read_lane(incl_m, kWave - 1);
+    carry_many += read_lane(two.incl_b, kWave - 1) >> 8;
+    carry_few += read_lane(two.incl_b, kWave - 1) & 255;
+    carry_m += read_lane(two.incl_m, kWave - 1);
+    base += 2 * kWave;
+    if (base >= a.E) return;  // (no tile of the list is here)
+    two = read_two(base);
   }
-  if (e < 0) {
-    // Surplus workgroups clear the tags of the rows no path owns: the j-th takes rows
-    // [total + 256 j, total + 256 (j + 1)).  The grid holds P / 256 + E row blocks (rounded up) per
-    // column tile and the experts use at most (total + 255 E) / 256 of them, so enough are left.
-    if (ROUTED && a.row_tags_out != nullptr) {
-      const long r = static_cast<long>(carry_m) + static_cast<long>(t - carry_t) * kBM + tid;
-      if (tid < kBM && r < a.P) a.row_tags_out[r] = 0;
-    }
-    return;
+  if (narrow) {
+    n0 += ((t - whole) & 3) * kUnitCols;
+    if (n0 >= a.N) return;
   }
   const int K = a.K;
   const int k_tiles = K / kBK;
@@ -190,6 +279,221 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     __syncthreads();
   }
 
+  const int frag_row = lane & 31, frag_k = lane >> 5;
+  const int swz = (frag_row >> 1) & 7;
+  auto frag_off = [&](int ks) { return ((ks * 2 + frag_k) ^ swz) << 4; };
+  const bool gather = ROUTED && a.gather != 0;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
+
+  // ---- epilogue: bias + activation, bf16, 32 rows at a time through this wavefront's image -----
+  // transposed accumulator: element r of tile (i, j) is output row 32 i + lane % 32, column (of the
+  // wavefront's 32 j .. 32 j + 31) 8 * (r / 4) + 4 * (lane / 32) + r % 4, i.e. a lane holds 4
+  // consecutive columns (8 bytes) of its row.
+  auto epilogue = [&](auto& acc, int first_row, int mine, int col_w) {
+    constexpr int MT = sizeof(acc) / sizeof(acc[0]), NT = sizeof(acc[0]) / sizeof(acc[0][0]);
+    const int row_w = row0 + first_row;
+    const global_bf16 bias = a.bias != nullptr ? (global_bf16)(a.bias[e]) : (global_bf16)nullptr;
+    constexpr int kOutB = OUTF32 ? 4 : 2;                 // bytes of one output element
+    constexpr int kImageRow = NT * 32 * kOutB + 16;      // padded row of this wavefront's 32-row image
+    constexpr int kImageB = 32 * kImageRow;
+    static_assert(kWaves * kImageB <= kLdsBytes, "the output images must fit the stages");
+    char* const image = smem + wave * kImageB;
+    constexpr int kChunk = 16 / kOutB;                    // elements of one 16-byte store
+    constexpr int kChunksPerRow = NT * 32 / kChunk;
+    constexpr int kRowsPerPass = kWave / kChunksPerRow;
+    // the bias of this lane's columns, all eight loads in one round trip
+    bf16x4 bv[NT][4];
+  #pragma unroll
+    for (int j = 0; j < NT; ++j)
+  #pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int col = col_w + j * 32 + 8 * g + 4 * frag_k;
+        bv[j][g] = bf16x4{};
+        if (bias != nullptr && col < a.N) bv[j][g] = *(global_bf16x4)(bias + col);
+      }
+  #pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      if (i * 32 >= mine) break;  // wave-uniform
+      // scattered rows: lane r of the pass holds the cell of row r (read again: LDS held operands)
+      int cell = -1;
+      if constexpr (ROUTED) {
+        if (a.scatter && lane < min(32, mine - i * 32)) {
+          const int r = row_w + i * 32 + lane;
+          cell = routed_cell(a, e, r, r - row0 + seat0);
+        }
+      }
+  #pragma unroll
+      for (int j = 0; j < NT; ++j) {
+  #pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int col = j * 32 + 8 * g + 4 * frag_k;  // inside the wavefront's 64 columns
+          const bf16x4 b4 = bv[j][g];
+          float v[4];
+  #pragma unroll
+          for (int q = 0; q < 4; ++q) v[q] = apply_act<ACT>(acc[i][j][4 * g + q] + static_cast<float>(b4[q]));
+          char* const to = image + frag_row * kImageRow + col * kOutB;
+          if constexpr (OUTF32) {
+            *reinterpret_cast<f32x4*>(to) = f32x4{v[0] + 0.0f, v[1] + 0.0f, v[2] + 0.0f, v[3] + 0.0f};  // -0 -> +0, as a combine would
+          } else {
+            *reinterpret_cast<bf16x4*>(to) = bf16x4{static_cast<__bf16>(v[0]), static_cast<__bf16>(v[1]),
+                                                    static_cast<__bf16>(v[2]), static_cast<__bf16>(v[3])};
+          }
+        }
+      }
+      wave_fence();
+      const int rows_i = min(32, mine - i * 32);
+      const int c = lane % kChunksPerRow;
+      char* const out_b = OUTF32 ? reinterpret_cast<char*>(a.out_f32) : reinterpret_cast<char*>(a.out);
+  #pragma unroll
+      for (int p = 0; p < 32 / kRowsPerPass; ++p) {
+        const int rl = p * kRowsPerPass + lane / kChunksPerRow;
+        long row = row_w + i * 32 + rl;
+        bool live = rl < rows_i && col_w + c * kChunk < a.N;
+        if constexpr (ROUTED) {
+          if (a.scatter) {
+            const int to = __shfl(cell, rl, kWave);
+            live = live && to >= 0;
+            row = to;
+          }
+        }
+        if (live) {
+          u32x4 v = *reinterpret_cast<const u32x4*>(image + rl * kImageRow + c * 16);
+          if constexpr (ROUTED && !OUTF32) {
+            if (a.scatter) {  // the combine this store stands for adds the row to zero: -0 becomes +0
+  #pragma unroll
+              for (int w = 0; w < 4; ++w) v[w] = plus_zero<BRT_BF16>(v[w]);
+            }
+          }
+          u32x4* const to = reinterpret_cast<u32x4*>(out_b + (static_cast<size_t>(row) * a.N + col_w) * kOutB + c * 16);
+          if (a.plain_out) *to = v;
+          else stream_out(v, to);
+        }
+      }
+      wave_fence();
+    }
+  };
+
+  // ---- a unit of the end of the list: `rows` rows, 64 columns from n0 on ---------------------------
+  if (narrow) {
+    const i32x4 res_x = in_scalars(gather ? make_rsrc(a.x, static_cast<size_t>(a.T) * K * 2)
+                                          : make_rsrc(a.x + static_cast<size_t>(row0) * K, static_cast<size_t>(a.P - row0) * K * 2));
+    const i32x4 res_u = in_scalars(make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2));
+    auto unit = [&](auto rows_tag) {
+      constexpr int UR = decltype(rows_tag)::value;         // rows of the unit
+      constexpr int kXw = UR / 64, kL = kXw + 1;            // row groups of x a wavefront loads, loads of a K-step
+      constexpr int UNT = UR == 256 ? 2 : 1;                // 32 x 32 blocks of a wavefront, side by side
+      constexpr int kStage = (UR + kUnitCols) * kRowB;
+      constexpr int D = UR == 256 ? 4 : UR == 128 ? 6 : 8;  // K-steps in flight and in LDS
+      static_assert(D * kStage <= kLdsBytes, "the ring must fit");
+      uint32_t off[kL];
+#pragma unroll
+      for (int i = 0; i < kL; ++i) {
+        const int row = (i == 0 ? wave : wave * kXw + i - 1) * 8 + (lane >> 3);
+        const uint32_t chunk = (lane & 7) ^ ((row >> 1) & 7);
+        int at = row;
+        bool there = row < (i == 0 ? a.N - n0 : rows);
+        if constexpr (ROUTED) {
+          if (gather && i > 0) {
+            at = s_cell[row];
+            there = at >= 0;
+          }
+        }
+        off[i] = there ? (static_cast<uint32_t>(at) * K + chunk * 8) * 2 : kOutOfRange;
+      }
+      if constexpr (ROUTED) __syncthreads();  // everyone has read the cells
+      auto fetch = [&](int s, uint32_t stage, int i) {
+        load_to_lds(i == 0 ? res_u : res_x, off[i], s * kRowB, lds0 + stage + (i == 0 ? UR / 8 + wave : wave * kXw + i - 1) * 1024);
+      };
+      const int tile_x = UNT == 2 ? wave : wave >> 1, tile_w = UNT == 2 ? 0 : wave & 1;
+      const int first_row = tile_x * 32, mine = __builtin_amdgcn_readfirstlane(max(min(rows - first_row, 32), 0));
+      f32x16 acc[1][UNT];
+#pragma unroll
+      for (int j = 0; j < UNT; ++j) acc[0][j] = f32x16{};
+      struct Frags {
+        bf16x8 w[kSub][UNT], x[kSub];
+      };
+      const char* const from_x = smem + (first_row + frag_row) * kRowB;
+      const char* const from_w = smem + (UR + tile_w * 32 + frag_row) * kRowB;
+      auto read_frags = [&](Frags& f, uint32_t stage, int ks) {
+        f.x[ks] = *reinterpret_cast<const bf16x8*>(from_x + stage + frag_off(ks));
+#pragma unroll
+        for (int j = 0; j < UNT; ++j) f.w[ks][j] = *reinterpret_cast<const bf16x8*>(from_w + stage + frag_off(ks) + j * 32 * kRowB);
+      };
+      const int primed = min(D, k_tiles);
+      for (int s = 0; s < primed; ++s)
+#pragma unroll
+        for (int i = 0; i < kL; ++i) fetch(s, s * kStage, i);
+      // all but the last `younger` K-steps requested have landed
+      auto landed = [&](int younger) {
+        if (younger >= D - 1) wait_loads_but<(D - 1) * kL>();
+        else if (younger == D - 2) wait_loads_but<(D - 2) * kL>();
+        else if (D > 4 && younger == D - 3) wait_loads_but<(D > 4 ? D - 3 : 1) * kL>();
+        else if (D > 5 && younger == D - 4) wait_loads_but<(D > 5 ? D - 4 : 1) * kL>();
+        else if (D > 6 && younger == D - 5) wait_loads_but<(D > 6 ? D - 5 : 1) * kL>();
+        else if (D > 7 && younger == D - 6) wait_loads_but<(D > 7 ? D - 6 : 1) * kL>();
+        else if (younger == 1) wait_loads_but<kL>();
+        else wait_loads_all();
+      };
+      landed(primed - 1);
+      block_barrier();
+      uint32_t stage = 0;
+      auto step = [&](const Frags& cur, Frags& next, int s, auto multiply, auto fills) {
+        constexpr bool kMultiply = decltype(multiply)::value, kFills = decltype(fills)::value;
+        const uint32_t ahead = stage == (D - 1) * kStage ? 0 : stage + kStage;
+        if constexpr (kFills) wait_loads_but<(D - 2) * kL>();
+        else landed(min(s + D - 1, k_tiles - 1) - (s + 1));
+        block_barrier();
+        if (!kFills && s + D < k_tiles) {
+#pragma unroll
+          for (int i = 0; i < kL; ++i) fetch(s + D, stage, i);
+        }
+#pragma unroll
+        for (int ks = 0; ks < kSub; ++ks) {
+          if constexpr (kMultiply) {
+#pragma unroll
+            for (int j = 0; j < UNT; ++j) acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.w[ks][j], cur.x[ks], acc[0][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            read_frags(next, ahead, ks);
+          }
+          if constexpr (kFills) {
+#pragma unroll
+            for (int i = ks * kL / kSub; i < (ks + 1) * kL / kSub; ++i) fetch(s + D, stage, i);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (kMultiply) wait_lds();
+        stage = ahead;
+      };
+      auto loop = [&](auto multiply) {
+        Frags f0, f1;
+        if constexpr (decltype(multiply)::value) {
+#pragma unroll
+          for (int ks = 0; ks < kSub; ++ks) read_frags(f0, 0, ks);
+          wait_lds();
+        }
+        int s = 0;
+        for (; s + 1 + D < k_tiles; s += 2) {
+          step(f0, f1, s, multiply, std::true_type{});
+          step(f1, f0, s + 1, multiply, std::true_type{});
+        }
+        for (; s < k_tiles; s += 2) {
+          step(f0, f1, s, multiply, std::false_type{});
+          if (s + 1 < k_tiles) step(f1, f0, s + 1, multiply, std::false_type{});
+        }
+      };
+      if (mine > 0) {
+        loop(std::true_type{});
+        epilogue(acc, first_row, mine, n0 + tile_w * 32);
+      } else {
+        loop(std::false_type{});
+      }
+    };
+    if (rows <= 64) unit(std::integral_constant<int, 64>{});
+    else if (rows <= 128) unit(std::integral_constant<int, 128>{});
+    else unit(std::integral_constant<int, 256>{});
+    return;
+  }
+
   // ---- global -> LDS ---------------------------------------------------------------------------
   // A load fills one row group: 8 tile rows, a whole 128-byte line of each.  Group 0 loads the
   // activation rows, wavefront wn taking row groups wn + 4 i (i = 0..7); group 1 the weight rows,
@@ -200,7 +504,6 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // Every wavefront keeps the eight offsets of its rows in registers (the K-step alone goes into
   // the scalar offset).  Gathered rows need that -- the cells of a row group are anywhere in x --
   // and it takes the bounds check out of the loop for the others.
-  const bool gather = ROUTED && a.gather != 0;
   const i32x4 res = in_scalars(wm == 0
       ? (gather ? make_rsrc(a.x, static_cast<size_t>(a.T) * K * 2)
                 : make_rsrc(a.x + static_cast<size_t>(row0) * K, static_cast<size_t>(a.P - row0) * K * 2))
@@ -223,7 +526,6 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     off[i] = there ? (static_cast<uint32_t>(at) * K + chunk * 8) * 2 : kOutOfRange;
   }
   if constexpr (ROUTED) __syncthreads();  // everyone has read the cells; the loads may overwrite them
-  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
   auto load_a = [&](int kt, uint32_t slot, int i) {
     load_to_lds(res, off[i], kt * kRowB, lds0 + slot + (wn + 4 * i) * 1024);
   };
@@ -234,8 +536,6 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // ---- fragments -------------------------------------------------------------------------------
   // MFMA operand: this lane feeds row (lane % 32), k-half (lane / 32) of a 32 x 16 block; chunk
   // ks * 2 + lane / 32 of the row sits in slot chunk ^ ((row >> 1) & 7)
-  const int frag_row = lane & 31, frag_k = lane >> 5;
-  const int swz = (frag_row >> 1) & 7;
   // The row tiles that hold rows are shared evenly by the two groups, group 0 taking the first `half`
   // rows: with 128 rows or fewer in one group the phases of a K-step would run one after the other.
   // (Halves fixed at 128 rows: the ragged FFN of 128 experts, 108 of its 201 row blocks part-filled,
@@ -245,7 +545,6 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   const int first_row = wm * half;  // of this wavefront, inside the tile
   const int frag_x = (first_row + frag_row) * kRowB;
   const int frag_w = kBBase + (wn * kNT * 32 + frag_row) * kRowB;
-  auto frag_off = [&](int ks) { return ((ks * 2 + frag_k) ^ swz) << 4; };
 
   f32x16 acc[kMT][kNT];
 #pragma unroll
@@ -375,91 +674,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   if (wm == 0) block_barrier();  // group 1's last C phase
   block_barrier();               // no wavefront reads a stage any more: the epilogue may write over them
 
-  // ---- epilogue: bias + activation, bf16, 32 rows at a time through this wavefront's image -----
-  // transposed accumulator: element r of tile (i, j) is output row 32 i + lane % 32, column (of the
-  // wavefront's 32 j .. 32 j + 31) 8 * (r / 4) + 4 * (lane / 32) + r % 4, i.e. a lane holds 4
-  // consecutive columns (8 bytes) of its row.
-  const global_bf16 bias = a.bias != nullptr ? (global_bf16)(a.bias[e]) : (global_bf16)nullptr;
-  constexpr int kOutB = OUTF32 ? 4 : 2;                 // bytes of one output element
-  constexpr int kImageRow = kNT * 32 * kOutB + 16;      // padded row of this wavefront's 32-row image
-  constexpr int kImageB = 32 * kImageRow;
-  static_assert(kWaves * kImageB <= kLdsBytes, "the output images must fit the stages");
-  char* const image = smem + wave * kImageB;
-  const int col_w = n0 + wn * kNT * 32;   // first column of this wavefront
-  const int row_w = row0 + first_row;     // first row
-  constexpr int kChunk = 16 / kOutB;                    // elements of one 16-byte store
-  constexpr int kChunksPerRow = kNT * 32 / kChunk;
-  constexpr int kRowsPerPass = kWave / kChunksPerRow;
-  // the bias of this lane's columns, all eight loads in one round trip
-  bf16x4 bv[kNT][4];
-#pragma unroll
-  for (int j = 0; j < kNT; ++j)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int col = col_w + j * 32 + 8 * g + 4 * frag_k;
-      bv[j][g] = bf16x4{};
-      if (bias != nullptr && col < a.N) bv[j][g] = *(global_bf16x4)(bias + col);
-    }
-#pragma unroll
-  for (int i = 0; i < kMT; ++i) {
-    if (i * 32 >= mine) break;  // wave-uniform
-    // scattered rows: lane r of the pass holds the cell of row r (read again: LDS held operands)
-    int cell = -1;
-    if constexpr (ROUTED) {
-      if (a.scatter && lane < min(32, mine - i * 32)) {
-        const int r = row_w + i * 32 + lane;
-        cell = routed_cell(a, e, r, r - row0 + seat0);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kNT; ++j) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int col = j * 32 + 8 * g + 4 * frag_k;  // inside the wavefront's 64 columns
-        const bf16x4 b4 = bv[j][g];
-        float v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = apply_act<ACT>(acc[i][j][4 * g + q] + static_cast<float>(b4[q]));
-        char* const to = image + frag_row * kImageRow + col * kOutB;
-        if constexpr (OUTF32) {
-          *reinterpret_cast<f32x4*>(to) = f32x4{v[0] + 0.0f, v[1] + 0.0f, v[2] + 0.0f, v[3] + 0.0f};  // -0 -> +0, as a combine would
-        } else {
-          *reinterpret_cast<bf16x4*>(to) = bf16x4{static_cast<__bf16>(v[0]), static_cast<__bf16>(v[1]),
-                                                  static_cast<__bf16>(v[2]), static_cast<__bf16>(v[3])};
-        }
-      }
-    }
-    wave_fence();
-    const int rows_i = min(32, mine - i * 32);
-    const int c = lane % kChunksPerRow;
-    char* const out_b = OUTF32 ? reinterpret_cast<char*>(a.out_f32) : reinterpret_cast<char*>(a.out);
-#pragma unroll
-    for (int p = 0; p < 32 / kRowsPerPass; ++p) {
-      const int rl = p * kRowsPerPass + lane / kChunksPerRow;
-      long row = row_w + i * 32 + rl;
-      bool live = rl < rows_i && col_w + c * kChunk < a.N;
-      if constexpr (ROUTED) {
-        if (a.scatter) {
-          const int to = __shfl(cell, rl, kWave);
-          live = live && to >= 0;
-          row = to;
-        }
-      }
-      if (live) {
-        u32x4 v = *reinterpret_cast<const u32x4*>(image + rl * kImageRow + c * 16);
-        if constexpr (ROUTED && !OUTF32) {
-          if (a.scatter) {  // the combine this store stands for adds the row to zero: -0 becomes +0
-#pragma unroll
-            for (int w = 0; w < 4; ++w) v[w] = plus_zero<BRT_BF16>(v[w]);
-          }
-        }
-        u32x4* const to = reinterpret_cast<u32x4*>(out_b + (static_cast<size_t>(row) * a.N + col_w) * kOutB + c * 16);
-        if (a.plain_out) *to = v;
-        else stream_out(v, to);
-      }
-    }
-    wave_fence();
-  }
+  epilogue(acc, first_row, mine, n0 + wn * kNT * 32);
 }
 
 template <int ACT, bool ROUTED, bool OUTF32>
@@ -469,6 +684,8 @@ int launch_pingpong(GemmArgs& a, hipStream_t st) {
   const long entries = (static_cast<long>(a.P + kBM - 1) / kBM + a.E) * a.tiles_n;
   const long round = kXcds * kCusPerXcd;
   const long grid = (entries + round - 1) / round * round;
+  a.grid = static_cast<int>(grid);
+  a.tiles_n_inverse = 0xffffffffu / static_cast<uint32_t>(a.tiles_n);
   auto* fn = &grouped_gemm_pingpong_kernel<ACT, ROUTED, OUTF32>;
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(fn), kLdsBytes); rc != BRT_OK) return rc;
   hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(grid)), dim3(kWaves * 64), kLdsBytes, st, a);

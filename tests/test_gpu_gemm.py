@@ -535,6 +535,36 @@ def test_ping_pong_tiles(loads, K, N):
     run(loads, K, N, act="relu", bias=True, seed=2, slack=300)
 
 
+def _tiles_cut(loads, P, N, tags_out=False):
+    """Tiles of the end of the ping-pong kernel's list that are cut into units of 256 rows x 64 columns."""
+    tn = -(-N // 256)
+    few = sum(1 for m in loads if 0 < m % 256 <= 128)
+    tiles = sum(-(-m // 256) for m in loads) * tn
+    rest = tiles % 256
+    cut = max(min(few, -(-rest // tn)) * tn, rest)
+    grid = -(-(-(-P // 256) + len(loads)) * tn // 256) * 256
+    return 0 if cut > 128 or tiles > 2560 or tiles + 3 * cut > grid - int(tags_out) else cut
+
+
+@pytest.mark.parametrize("loads,K,N,cut", [
+    ([2049] + [2048] * 7, 128, 4096, 16),                 # one row over whole rounds, the shortest K loop (two K-steps)
+    ([2048 + 64, 2048 + 65], 192, 4104, 50),              # blocks of 64 and 65 rows, last tiles of 8 columns: units without columns
+    ([2048 + 128, 31, 33, 65, 0, 2048 + 129, 127, 97], 320, 3328, 52),  # blocks of few rows cut, others in the list; five K-steps
+    ([1024] * 17, 256, 1024, 16),                          # nothing but whole blocks at the end
+    ([256 * 9] * 16, 320, 1000, 64),                       # a quarter of a round: every workgroup of the grid has its unit
+    ([700, 1500, 100, 2300, 1], 512, 3640, 44),            # as many K-steps as the deepest ring holds
+    ([1800, 900, 0, 2200, 260], 576, 3328, 43),            # and one more
+    ([5000, 3328 + 40, 0, 300], 1088, 2048, 32),           # seventeen K-steps: every ring goes round
+    ([0] * 130 + [3] * 100 + [8000, 9000, 24000, 1], 128, 512, 14),  # more than 128 experts
+])
+def test_end_of_the_list_of_ping_pong_tiles_in_units(loads, K, N, cut):
+    P, E = sum(loads), len(loads)
+    assert _kernel_for(P, E, K, N) == "ping-pong" and _tiles_cut(loads, P, N) == cut
+    run(loads, K, N)
+    run(loads, K, N, act="gelu", bias=True, seed=1)
+    run(loads, K, N, act="relu", bias=True, seed=2, slack=300)
+
+
 @pytest.mark.parametrize("T,E,K,N,k,cap,pad", [
     (12000, 8, 128, 4096, 1, 1500, False),   # overflow dropped, the shortest K loop
     (12000, 8, 192, 4104, 1, 1700, True),    # padded to the capacity: empty slots, odd K-steps, N tail
@@ -598,6 +628,24 @@ def test_ping_pong_tiles_with_routing_and_fp32_output(T, E, K, N, k, cap, pad):
     del ws
 
 
+@pytest.mark.parametrize("T,E,K,N,k,cap,pad", [
+    (16500, 4, 128, 2048, 1, 4140, False),   # overflow dropped, every expert with few rows over whole blocks
+    (4500, 4, 320, 6912, 1, 1026, True),     # padded to the capacity: last blocks of two rows
+    (17000, 4, 576, 2048, 2, 8209, False),   # two entries per cell (gather only)
+    (132000, 2, 192, 256, 1, 65560, False),  # one column tile
+])
+def test_units_with_routing_and_fp32_output(T, E, K, N, k, cap, pad):
+    from brainstorm_amd._C import router as c_router
+    from routing_cases import topk_mask
+
+    mask, _ = topk_mask(T, E, k, seed=T + E)
+    ids, _ = c_router.gate_topk(torch.from_numpy(mask.astype(np.float32)).cuda(), k)
+    rows = E * cap if pad else T * k
+    loads = c_router.route_by_path(ids, E, torch.tensor([cap], dtype=torch.int32, device="cuda"), pad, rows=rows)[0].tolist()
+    assert _tiles_cut(loads, rows, N, tags_out=True) > 0
+    test_ping_pong_tiles_with_routing_and_fp32_output(T, E, K, N, k, cap, pad)
+
+
 @pytest.mark.parametrize("K,N", [
     (8, 8),        # one chunk of one K-step, one chunk of columns
     (72, 56),      # two K-steps, the second one cut
@@ -622,8 +670,14 @@ def _kernel_for(P, E, K, N):
     """Which kernel the host takes for these sizes (all but the weighted accumulate form), on 256 CUs."""
     used = min(E, P)
     big = ((P + 255) // 256 + (E + 1) // 2) * -(-N // 256)
-    if K % 64 == 0 and K >= 128 and P > E * 160 and (big >= 512 or 192 <= big <= 256):
-        return "ping-pong"
+    if K % 64 == 0 and K >= 128 and P > E * 160 and big >= 192:
+        def rounds(waves):  # of the 160-row kernel's tiles; two workgroups of two wavefronts fit a CU
+            n = max((P + 159) // 160, used) * -(-N // (64 * waves))
+            return -(-n // 512) * 2 if waves == 2 else -(-n // 256)
+
+        cost, waves = min((rounds(w) * (160 + 64 * w), -w) for w in (2, 3, 4))
+        if big <= 320 or 5 * big >= 8 * 256 or (waves != -2 and (big >= 384 or cost > 832)):
+            return "ping-pong"
     tiles = max((P + 159) // 160, used) * -(-N // 256)
     weight = 2.0 * used * N * K
     if P > 64 * used:
@@ -638,7 +692,7 @@ def _kernel_for(P, E, K, N):
 
 
 @pytest.mark.parametrize("loads,K,N,bounds", [
-    ([9, 0, 3, 1, 20, 31, 2, 8, 17, 1, 7, 4], 1088, 4104, {"few rows": 103, "160 rows": 2400, "ping-pong": 8000}),
+    ([9, 0, 3, 1, 20, 31, 2, 8, 17, 1, 7, 4], 1088, 4104, {"few rows": 103, "160 rows": 1900, "ping-pong": 8000}),
     ([3, 70, 0, 33, 150], 1096, 136, {"few rows": 256, "160 rows": 16000}),  # K and N tails
     ([30] * 32, 4096, 1024, {"few rows": 960 - 64, "160 rows": 1024}),       # what a layer keeps and what it may keep
 ])
