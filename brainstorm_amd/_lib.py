@@ -151,6 +151,11 @@ SIGNATURES = {
         _c_int,
         [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_size, _c_ptr],
     ),
+    "brt_hip_top1_route_to_capacity": (
+        _c_int,
+        [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr,
+         _c_size, _c_ptr],
+    ),
     "brt_hip_copy_to_host": (_c_int, [_c_ptr, _c_ptr, _c_int, _c_ptr]),
     "brt_hip_probe_mfma_rate": (_c_int, [_c_int, _c_int, _c_ptr, _c_ptr]),
     "brt_hip_grouped_gemm_timed": (

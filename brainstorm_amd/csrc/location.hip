@@ -65,7 +65,7 @@ constexpr int kBatch = 16;         // row loads in flight per lane
 constexpr int kPartialBatch = 32;  // loads of earlier bands' sums in flight per lane
 constexpr int kMaxBands = 512;
 
-enum { kSeat = 0, kTag = 1, kThrottle = 2 };
+enum { kSeat = 0, kTag = 1, kThrottle = 2, kThrottleSeat = 3 };  // (the last: throttled bits, and the seats of what is left)
 
 struct ScanGeometry {
   int ep_shift;  // log2 of the lanes one row occupies (E <= 64), 6 otherwise
@@ -166,6 +166,7 @@ struct ScanArgs {
   const int* threshold;  // throttle only; null: `capacity` cells of every path
   int capacity;
   int* capacities;       // throttle only: `capacity` of every path, written where non-null
+  int* seats;            // throttle with seats only: their matrix; loads and counts are those of what is left
   int* partial;          // [bands][E] per-band column sums
   int* prefix_in;        // throttle only: copy of prefix taken by pass 1 ([E])
   int T, E, C;
@@ -236,6 +237,7 @@ __device__ __forceinline__ void walk_batch(const int (&m)[N], int i0, int n_ins,
   // rows of this wavefront through one 64-bit base and 32-bit offsets: the address of every
   // store is one instruction instead of a 64-bit multiply-add chain
   int* __restrict__ out_w = a.out + row_w * a.E;
+  int* __restrict__ seats_w = MODE == kThrottleSeat ? a.seats + row_w * a.E : nullptr;
   const int rows_here = static_cast<int>(max(0l, min(static_cast<long>(a.rows_pw), a.T - row_w)));
 #pragma unroll
   for (int u = 0; u < N; ++u) {
@@ -248,6 +250,10 @@ __device__ __forceinline__ void walk_batch(const int (&m)[N], int i0, int n_ins,
         out_w[at] = run * m[u];  // location * mask, location.cu:177-178
       } else if (MODE == kThrottle) {
         out_w[at] = (m[u] == 1 && run <= thr) ? 1 : 0;
+      } else if (MODE == kThrottleSeat) {  // words of 0 and 1 from a zero prefix: whoever is left has seen no one turned away
+        const int left = (m[u] == 1 && run <= thr) ? 1 : 0;
+        out_w[at] = left;
+        seats_w[at] = run * left;
       } else {
         const int index = run * m[u];
         if (index >= 1 && index <= a.T)
@@ -449,7 +455,7 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
     // read before the barrier: with a single band the first wavefront overwrites prefix[] at
     // the end of its walk, which no wavefront may overtake
     int thr = 0, pre_in = 0;
-    if (MODE == kThrottle && col_ok) {
+    if ((MODE == kThrottle || MODE == kThrottleSeat) && col_ok) {
       if (a.prefix != nullptr) pre_in = (a.bands > 1 ? a.prefix_in : a.prefix)[col];
       thr = a.threshold != nullptr ? a.threshold[col] : a.capacity;
     }
@@ -488,6 +494,11 @@ __global__ __launch_bounds__(kWavesPB * kWave) void band_apply_kernel(ScanArgs a
       if (MODE == kThrottle) {
         if (a.prefix != nullptr) a.prefix[col] = min(band_total + pre_in, thr);
         if (a.capacities != nullptr) a.capacities[col] = a.capacity;
+      } else if (MODE == kThrottleSeat) {  // finalize_load with `capacity` for every entry of the menu
+        const int left = min(band_total, a.capacity);
+        a.loads[col] = a.path_wise_padding ? a.capacity : left == 0 ? 0 : a.capacity_padding ? a.capacity : left;
+        a.counts[col] = left;
+        a.capacities[col] = a.capacity;
       } else {
         a.loads[col] =
             finalize_load(band_total, a.caps, a.C, a.capacity_padding, a.path_wise_padding, col);
@@ -1085,8 +1096,12 @@ extern "C" int brt_hip_throttle_hotmask(const int32_t* mask, int32_t* out, int32
   return launch_scan(kThrottle, a, workspace, workspace_bytes, stream);
 }
 
-extern "C" int brt_hip_top1_to_capacity(const void* scores, int dtype, int32_t* mask, int32_t* out, int32_t* capacities,
-                                        int capacity, int T, int E, void* workspace, size_t workspace_bytes, void* stream) {
+namespace {
+
+// The throttled top-1 mask, and with `seats` the route of what the throttle leaves (a.seats, loads, counts and padding set).
+int top1_to_capacity(const void* scores, int dtype, int32_t* mask, ScanArgs a, void* workspace, size_t workspace_bytes, void* stream) {
+  const int T = a.T, E = a.E, capacity = a.capacity;
+  int32_t *const out = a.out, *const capacities = a.capacities;
   if (T < 0 || E <= 0) return fail(BRT_E_INVALID, "bad shape T=%d E=%d", T, E);
   if (dtype != BRT_F32 && dtype != BRT_F16 && dtype != BRT_BF16) return fail(BRT_E_UNSUPPORTED, "dtype %d is not supported", dtype);
   if (E > kWave) return fail(BRT_E_UNSUPPORTED, "top1_to_capacity takes up to %d paths, got %d", kWave, E);
@@ -1103,14 +1118,8 @@ extern "C" int brt_hip_top1_to_capacity(const void* scores, int dtype, int32_t* 
   if (workspace == nullptr || workspace_bytes < need)
     return fail(BRT_E_WORKSPACE, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
   if (!aligned(workspace, 4)) return fail(BRT_E_INVALID, "workspace must be 4-byte aligned");
-  ScanArgs a{};
   a.mask = mask;
-  a.out = out;
-  a.capacity = capacity;
-  a.capacities = capacities;
   a.partial = static_cast<int*>(workspace);
-  a.T = T;
-  a.E = E;
   a.ep_shift = g.ep_shift;
   a.rows_pw = g.rows_pw;
   a.n_ins = g.rows_pw >> (6 - g.ep_shift);
@@ -1121,8 +1130,46 @@ extern "C" int brt_hip_top1_to_capacity(const void* scores, int dtype, int32_t* 
   else if (dtype == BRT_F16) hipLaunchKernelGGL(band_top1_kernel<BRT_F16>, grid, block, 0, st, scores, a, mask);
   else hipLaunchKernelGGL(band_top1_kernel<BRT_BF16>, grid, block, 0, st, scores, a, mask);
   if (const int rc = check_launch("band_top1_kernel"); rc != BRT_OK) return rc;
-  hipLaunchKernelGGL((band_apply_kernel<kThrottle, kWavesPB, false>), grid, block, 0, st, a);
+  if (a.seats != nullptr) hipLaunchKernelGGL((band_apply_kernel<kThrottleSeat, kWavesPB, false>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((band_apply_kernel<kThrottle, kWavesPB, false>), grid, block, 0, st, a);
   return check_launch("band_apply_kernel");
+}
+
+}  // namespace
+
+extern "C" int brt_hip_top1_to_capacity(const void* scores, int dtype, int32_t* mask, int32_t* out, int32_t* capacities,
+                                        int capacity, int T, int E, void* workspace, size_t workspace_bytes, void* stream) {
+  ScanArgs a{};
+  a.out = out;
+  a.capacity = capacity;
+  a.capacities = capacities;
+  a.T = T;
+  a.E = E;
+  return top1_to_capacity(scores, dtype, mask, a, workspace, workspace_bytes, stream);
+}
+
+// The second launch knows the running number of every cell and whether it is turned away, which is all that index
+// generation would find out by reading the throttled mask twice more: 100352 x 8 fp32 scores 12.7 us for this, 11.0
+// for brt_hip_top1_to_capacity alone and 19.5 with index generation behind it, 4096 x 8 7.1, 7.0 and 11.7 (back to back
+// in a graph).  Bound by the same round trips; the seats are one more store a word.
+extern "C" int brt_hip_top1_route_to_capacity(const void* scores, int dtype, int32_t* mask, int32_t* out, int32_t* seats,
+                                              int32_t* loads, int32_t* counts, int32_t* capacities, int capacity,
+                                              int capacity_padding, int path_wise_padding, int T, int E, void* workspace,
+                                              size_t workspace_bytes, void* stream) {
+  if (T <= 0 || capacity < 0) return fail(BRT_E_INVALID, "bad shape T=%d or capacity %d", T, capacity);
+  if (!seats || !loads || !counts) return fail(BRT_E_INVALID, "null argument");
+  ScanArgs a{};
+  a.out = out;
+  a.seats = seats;
+  a.loads = loads;
+  a.counts = counts;
+  a.capacity = capacity;
+  a.capacities = capacities;
+  a.capacity_padding = capacity_padding;
+  a.path_wise_padding = capacity_padding && path_wise_padding;
+  a.T = T;
+  a.E = E;
+  return top1_to_capacity(scores, dtype, mask, a, workspace, workspace_bytes, stream);
 }
 
 extern "C" int brt_hip_convert_index_format(const int32_t* src, int32_t* dst,

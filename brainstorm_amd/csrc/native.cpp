@@ -225,6 +225,23 @@ PyObject* top1_to_capacity(const Args& a) {
   return tuple(wrap(out), wrap(caps));
 }
 
+// ... and the route of the throttled mask: score, capacity, capacity_padding, path_wise_padding -> (mask, capacities, seats,
+// loads, counts), or None likewise
+PyObject* top1_route_to_capacity(const Args& a) {
+  const Tensor score = scores(a.tensor(0), 1);
+  const long capacity = a.integer(1);
+  const int64_t T = score.size(0), E = score.size(1);
+  if (T == 0 || E > 64 || capacity < 0 || capacity > INT32_MAX) return none();
+  const c10::DeviceGuard guard(score.device());
+  Tensor mask = empty(score.sizes(), at::kInt, score), out = empty(score.sizes(), at::kInt, score), caps = empty({E}, at::kInt, score);
+  Tensor seats = empty(score.sizes(), at::kInt, score), loads = empty({E}, at::kInt, score), counts = empty({E}, at::kInt, score);
+  const Tensor ws = scratch(brt_hip_scan_workspace_bytes(T, E), score);
+  check(brt_hip_top1_route_to_capacity(ptr(score), code_of(score.scalar_type()), iptr(mask), iptr(out), iptr(seats), iptr(loads),
+                                       iptr(counts), iptr(caps), static_cast<int>(capacity), a.flag(2), a.flag(3), T, E, ptr(ws),
+                                       ws.numel(), stream_of(score)));
+  return tuple(wrap(out), wrap(caps), wrap(seats), wrap(loads), wrap(counts));
+}
+
 PyObject* generate(const Args& a) {  // hot_mask, capacities, capacity_padding, path_wise_padding, is_tag_index
   const Tensor given = a.tensor(0);
   on_device(given, "hot_mask");
@@ -851,7 +868,7 @@ PyMethodDef methods[] = {
     BRT_ENTRY(topk_hot_mask, 2),    BRT_ENTRY(gate_topk, 4),           BRT_ENTRY(throttle_hotmask, 3),
     BRT_ENTRY(generate, 5),         BRT_ENTRY(route_and_dispatch, 7),  BRT_ENTRY(route_by_path, 7),
     BRT_ENTRY(dispatch, 12),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
-    BRT_ENTRY(top1_to_capacity, 2), BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 7),     BRT_ENTRY(grouped_linear, 16),
+    BRT_ENTRY(top1_to_capacity, 2), BRT_ENTRY(top1_route_to_capacity, 4), BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 7),     BRT_ENTRY(grouped_linear, 16),
     BRT_ENTRY(grouped_linear_f32, 16), BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5),        BRT_ENTRY(int_list, 1),
     BRT_ENTRY(ordinary, 3),         BRT_ENTRY(plain, 1),            BRT_ENTRY(of_class, 2),            BRT_ENTRY(matrix, 4),
     BRT_ENTRY(grid, 5),                BRT_ENTRY(split_rows, 4),

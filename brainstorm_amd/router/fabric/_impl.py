@@ -228,11 +228,15 @@ class DispatchFabric(FabricBase):
                 score: torch.Tensor = None):
         caps = runtime_capacities if runtime_capacities is not None else self.supported_capacities
         in_flows = [in_flow] if self.flow_num == 1 else in_flow
-        route = c_router.generate_route(
-            hot_mask, supported_capacities=caps, capacity_padding=self.capacity_padding,
-            path_wise_padding=self.path_wise_padding,
-            is_tag_index=self._defers(in_flows, runtime_capacities, hot_mask),
-            single_path=getattr(hot_mask, "_brt_single_path", False))
+        as_tags = self._defers(in_flows, runtime_capacities, hot_mask)
+        route = None
+        if not as_tags and hasattr(hot_mask, "_brt_generated"):  # the protocol's kernel has laid the route out too
+            route = c_router.take_generated_route(hot_mask, caps, self.capacity_padding, self.path_wise_padding)
+        if route is None:
+            route = c_router.generate_route(
+                hot_mask, supported_capacities=caps, capacity_padding=self.capacity_padding,
+                path_wise_padding=self.path_wise_padding, is_tag_index=as_tags,
+                single_path=getattr(hot_mask, "_brt_single_path", False))
         self.__dict__["_route"] = route  # (not through nn.Module's attribute registration)
         route_indices, loads = route.indices, route.loads
         self.capture_flow_stats(in_flows, route_indices, loads)

@@ -311,6 +311,9 @@ class SwinMoEProtocol(ProtocolBase):
         self.group = group
         self.is_gshard_loss = is_gshard_loss
         self.alignment = alignment
+        #: set by a SwinMoEScatterRouter: (capacity_padding, path_wise_padding) of the fabric that takes the decision, whose
+        #: route the throttling kernel then lays out along with the mask
+        self.padding = None
 
     def runtime_capacity(self, cells: int, paths: int) -> int:
         if self.capacity_factor <= 0:
@@ -323,7 +326,8 @@ class SwinMoEProtocol(ProtocolBase):
         loss = self.generate_auxiliary(score, logits_wo_noise, logits, None)
         cap = self.runtime_capacity(score.size(0), paths)
         if not self.batch_prioritized_routing and _kernel_takes(score):
-            both = c_router.top1_to_capacity(score, cap)
+            both = (c_router.top1_to_capacity(score, cap) if self.padding is None
+                    else c_router.top1_route_to_capacity(score, cap, *self.padding))
             if both is not None:
                 return both[0], both[1], score, loss
         mask = _topk_hot_mask(score, 1)  # the first of the top-k choices (swin_moe.py:101-107)

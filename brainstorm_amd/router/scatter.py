@@ -95,6 +95,8 @@ class SwinMoEScatterRouter(RouterBase):
         self.fabric_kwargs = _merged(
             {"flow_num": 1, "route_logic": ["1d"], "transform": [False]}, fabric_kwargs)
         self.fabric = make_fabric(fabric_type, self.fabric_kwargs)
+        if hasattr(self.fabric, "capacity_padding"):  # a fabric that generates indices from the mask
+            self.protocol.padding = (self.fabric.capacity_padding, self.fabric.path_wise_padding)
 
     def forward(self, in_flows, score, logits_wo_noise, logits):
         hot_mask, runtime_capacities, new_score, _loss = self.protocol(score, logits_wo_noise, logits)

@@ -477,6 +477,16 @@ int brt_hip_top1_to_capacity(const void* scores, int dtype, int32_t* mask, int32
                              void* stream);
 
 /*
+ * The same two launches, which also write what brt_hip_generate_indices_and_loads makes of `out` with a menu of `capacity`
+ * for every path: seats [T,E], loads [E] and counts [E] (capacity_padding and path_wise_padding as there).  T > 0,
+ * capacity >= 0; seats must not overlap mask or out.
+ */
+int brt_hip_top1_route_to_capacity(const void* scores, int dtype, int32_t* mask, int32_t* out, int32_t* seats,
+                                   int32_t* loads, int32_t* counts, int32_t* capacities, int capacity,
+                                   int capacity_padding, int path_wise_padding, int T, int E,
+                                   void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * src[0 .. words-1] to host[0 .. words-1], then host[words] = 1: host memory of words + 1 words that the device can
  * write (hipHostMalloc).  A host that cleared host[words] before the call may watch it (acquire loads) instead of waiting
  * for the stream; nothing is written behind it.  Takes the place of the copy and the wait with which the reference reads

@@ -1245,3 +1245,65 @@ def test_top1_to_capacity_is_the_mask_throttled(brt_mod, T, E, dtype):
         assert torch.equal(got, want) and torch.equal(capacities, limit)
     assert c_router.top1_to_capacity(torch.zeros(4, 65, device="cuda"), 2) is None
     assert c_router.top1_to_capacity(torch.zeros(0, 4, device="cuda"), 2) is None
+
+
+@pytest.mark.parametrize("T,E,dtype", [
+    (1, 1, torch.float32), (5, 8, torch.float16), (129, 64, torch.float32), (777, 5, torch.float32), (127, 40, torch.float16),
+    (8192, 8, torch.bfloat16), (40000, 33, torch.bfloat16), (100352, 8, torch.float16), (131075, 2, torch.float32),
+])
+def test_route_generated_along_with_the_throttled_mask(brt_mod, T, E, dtype):
+    """What the throttling kernel lays out is what index generation makes of the throttled mask, for every padding."""
+    c_router = brt_mod[1]
+    score = torch.randint(-3, 4, (T, E), generator=torch.Generator().manual_seed(T + E)).to(dtype).cuda()
+    score[T // 2] = float("nan")
+    for capacity in (0, 1, max(1, T // E), T, 2**31 - 1):
+        mask, limit = c_router.top1_to_capacity(score, capacity)
+        for padding in ((False, False), (True, False), (True, True), (False, True)):
+            want = c_router.generate_route(mask, limit, *padding)
+            got_mask, got_limit = c_router.top1_route_to_capacity(score, capacity, *padding)
+            assert torch.equal(got_mask, mask) and torch.equal(got_limit, limit)
+            route = c_router.take_generated_route(got_mask, got_limit, *padding)
+            for name in ("indices", "loads", "counts"):
+                assert torch.equal(getattr(route, name), getattr(want, name)), (capacity, padding, name)
+            assert c_router.take_generated_route(got_mask, got_limit, *padding) is None  # handed out once
+
+
+def test_changed_decisions_of_a_swin_router_are_routed_as_they_are(brt_mod):
+    """The route that comes with the mask is used for that mask, those capacities and that padding only."""
+    brt, c_router = brt_mod[:2]
+    from brt.router import SwinMoEScatterRouter
+
+    x = torch.randn(512, 16, generator=torch.Generator().manual_seed(1)).cuda()
+    score = torch.randn(512, 4, generator=torch.Generator().manual_seed(2)).cuda()
+
+    def rows_of(hook=None, padding=True):
+        router = SwinMoEScatterRouter(protocol_kwargs={"capacity_factor": 1.0}, fabric_type="fused_dispatch", fabric_kwargs={
+            "capacity_padding": True, "max_path_padding": True, "max_path_load": 160}).cuda()
+        router.fabric.capacity_padding = padding
+        if hook is not None:
+            router.protocol.register_forward_hook(hook)
+        out, _ = router(brt.Annotator([0])(x), score, None, None)
+        return brt.to_torch_tensor(out), out.tag, out.load
+
+    def check(hook, change, padding=True):
+        mask, limit = c_router.top1_to_capacity(score, 128)
+        mask, limit = change(mask, limit)
+        route = c_router.generate_route(mask, limit, padding)
+        (want,) = c_router.dispatch_with_indices_and_loads(x, route.indices, route.loads, max_path_padding=True, max_path_load=160)
+        rows, indices, loads = rows_of(hook, padding)
+        assert torch.equal(rows, want) and torch.equal(indices, route.indices) and torch.equal(loads, route.loads)
+
+    def without_some(module, args, out):
+        out[0][::3] = 0
+
+    def smaller(module, args, out):
+        out[1].fill_(100)
+
+    def another(module, args, out):
+        return (out[0].clone(), *out[1:])
+
+    check(None, lambda m, c: (m, c))
+    check(without_some, lambda m, c: (torch.where(torch.arange(512, device="cuda")[:, None] % 3 == 0, 0, m), c))
+    check(smaller, lambda m, c: (m, torch.full_like(c, 100)))
+    check(another, lambda m, c: (m, c))
+    check(None, lambda m, c: (m, c), padding=False)
