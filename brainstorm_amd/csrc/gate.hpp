@@ -30,8 +30,18 @@ __device__ __forceinline__ uint32_t segment_max(uint32_t v, int width) {
     return static_cast<int>(max(static_cast<uint32_t>(x), static_cast<uint32_t>(y)));
   }));
 }
-__device__ __forceinline__ int segment_min(int v, int width) {
-  return segment_all_reduce(v, width, [](int x, int y) { return min(x, y); });
+// Maximum over the 64 lanes, in every lane as one scalar: lanes that a DPP step leaves out take 0, the least key.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+#define BRT_MAX_STEP(CTRL, ROWS)                                                                           \
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, ROWS, 0xf, false)))
+  BRT_MAX_STEP(0x111, 0xf);  // row_shr:1
+  BRT_MAX_STEP(0x112, 0xf);  // row_shr:2
+  BRT_MAX_STEP(0x114, 0xf);  // row_shr:4
+  BRT_MAX_STEP(0x118, 0xf);  // row_shr:8
+  BRT_MAX_STEP(0x142, 0xa);  // row_bcast:15 -> rows 1,3
+  BRT_MAX_STEP(0x143, 0xc);  // row_bcast:31 -> rows 2,3
+#undef BRT_MAX_STEP
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), kWave - 1));
 }
 
 }  // namespace brt

@@ -502,6 +502,29 @@ def test_topk_hot_mask_bit_exact(hip, T, E, k, dtype):
     assert (got.sum(1) == k).all()
 
 
+# rows of 33 columns and more, on both sides of every number of columns per lane, several rows a step with a part-filled last
+# step, and one row a step (8192 rows and fewer); NaN, infinities, both zeros and ties among them
+@pytest.mark.parametrize("T,E,k,dtype", [
+    (20001, 33, 2, "f32"), (40003, 64, 4, "bf16"), (8192, 64, 3, "f32"), (8193, 65, 1, "f16"), (66001, 128, 2, "f32"),
+    (16387, 129, 3, "f32"), (9001, 256, 2, "bf16"), (8197, 257, 2, "f32"), (3, 128, 128, "f32"),
+])
+def test_topk_of_many_columns_bit_exact(hip, T, E, k, dtype):
+    rng = np.random.default_rng(T + E)
+    score = rng.standard_normal((T, E)).astype(np.float32)
+    special = np.array([np.nan, np.inf, -np.inf, 0.0, -0.0, 1.0], dtype=np.float32)
+    score[:: 7] = special[rng.integers(0, 6, (len(score[:: 7]), E))]
+    bits = as_dtype_bits(score, dtype)
+    score = bits_to_f32(bits, dtype)
+    mask = oracle.topk_hot_mask(score, k)
+    assert np.array_equal(hip.topk_hot_mask(bits, k, dtype), mask)
+    ids, w, got = hip.gate_topk(bits, k, dtype, want_mask=True)
+    want_ids, want_w = oracle.gate_topk(score, k)
+    assert np.array_equal(ids, want_ids) and np.array_equal(w, want_w, equal_nan=True) and np.array_equal(got, mask)
+    finite = np.isfinite(score).all(1)
+    p, want_p = hip.gate_topk(bits, k, dtype, softmax=True)[1][finite], oracle.gate_topk(score, k, softmax=True)[1][finite]
+    assert np.allclose(p, want_p, rtol=2e-6, atol=1e-30)  # exp and a sum of E terms in fp32
+
+
 def test_topk_hot_mask_special_values(hip):
     score = np.array([[1.0, 1.0, 1.0, 1.0], [0.0, -0.0, 0.0, -1.0],
                       [np.nan, 5.0, np.inf, -np.inf], [-np.inf, -np.inf, np.nan, np.nan]], dtype=np.float32)
