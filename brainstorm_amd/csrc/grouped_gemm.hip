@@ -760,7 +760,7 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   // stores in the expanding GEMM that GEMM takes 102 us instead of 87 us).
   a.plain_out = N < K && static_cast<size_t>(P) * N * 2 <= (size_t{32} << 20);
   if (clocks != nullptr) {  // the timed form: the ping-pong kernel or nothing
-    if (!pingpong_gemm_applies(a) || out_is_f32)
+    if (!pingpong_gemm_applies(a) || K % kBK != 0 || out_is_f32)
       return fail(BRT_E_UNSUPPORTED, "the timed form runs the ping-pong kernel only (bf16 output, no tags, K a multiple of 64 and >= 128)");
     a.clocks = clocks;
     return launch_pingpong_gemm(a, act, as_stream(stream));
@@ -785,6 +785,9 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   // 5888 -> 1472 216 and 257; 64 x 337 rows 2816 -> 704 156 and 128): those stay there, and those of up to 1.6 rounds for which two
   // narrow workgroups of it fit a CU (4 x 8070 rows 1280 -> 640 62 and 68).  Below three quarters of a round the 160-row
   // tiles spread better (4 x 4060 rows 1792 -> 448, half a round, 37.9 us there, 46.9 here).
+  // Widths that are no multiple of a K-step of 64 are under the same rule: 8 x 1024 rows 1592 -> 6368 278 us there, 187 here,
+  // 6368 -> 1592 218 and 176, 4 x 3000 rows 4384 -> 1096 155 and 120, 64 x 400 rows 360 -> 1440 105 and 63, 12 x 700 rows 7200 -> 1800
+  // 279 and 276, 4 x 4000 rows 264 -> 528 (three column tiles for 528 columns) 22.5 and 22.8.
   // The rule is the same for gathered, scattered and fp32-output rows: a gathering 1024 -> 4096 GEMM with GELU over 32768
   // rows of 16 experts takes 437 us on the 160-row kernel and 336 us here.
   if (wide_tiles_come_in_rounds(a)) return launch_pingpong_gemm(a, act, as_stream(stream));

@@ -565,6 +565,44 @@ def test_end_of_the_list_of_ping_pong_tiles_in_units(loads, K, N, cut):
     run(loads, K, N, act="relu", bias=True, seed=2, slack=300)
 
 
+# K = 64 n + 8, 56 and others: the part-filled K-step is the third and later ones, in the list and in units of 64, 128 and 256 rows whose
+# rings of four to eight K-steps it ends inside, at the end of and behind
+@pytest.mark.parametrize("loads,K,N", [
+    ([1024] * 8, 136, 4096),
+    ([3000, 0, 1, 2900, 257, 255, 1500, 700], 248, 4096),
+    ([5000, 31, 4000, 129], 1096, 4104),
+    ([2048 + 64, 2048 + 65], 200, 4104),
+    ([2048 + 128, 31, 33, 65, 0, 2048 + 129, 127, 97], 312, 3328),
+    ([700, 1500, 100, 2300, 1], 504, 3640),
+    ([1800, 900, 0, 2200, 260], 520, 3328),
+    ([5000, 3328 + 40, 0, 300], 1144, 2048),
+])
+def test_ping_pong_tiles_of_part_filled_k_steps(loads, K, N):
+    """The bits of the same rows with K filled up with zeros, and nothing of the neighbouring rows in them."""
+    from brainstorm_amd.jit import grouped_linear
+
+    P, E, whole = sum(loads), len(loads), -(-K // 64) * 64
+    assert _kernel_for(P, E, K, N) == _kernel_for(P, E, whole, N) == "ping-pong"
+    run(loads, K, N, act="gelu", bias=True)
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn(P, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(E, N, K, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    x[7::97, 0], w[:, 11::89, 0] = float("nan"), float("inf")  # what follows the rows 6, 103, ... and 10, 99, ...
+    d_loads = torch.tensor(loads, dtype=torch.int32, device="cuda")
+
+    def product(x, w):
+        out = torch.empty(P, N, dtype=torch.bfloat16, device="cuda")
+        table = torch.tensor([w[e].data_ptr() for e in range(E)], dtype=torch.int64, device="cuda")
+        grouped_linear(x, out, table, None, d_loads, x.shape[1], N)
+        torch.cuda.synchronize()
+        return out
+
+    got, want = product(x, w), product(torch.nn.functional.pad(x, (0, whole - K)), torch.nn.functional.pad(w, (0, whole - K)))
+    clean = torch.isfinite(want)
+    assert clean.sum() == (P - len(x[7::97])) * (N - len(range(11, N, 89)))
+    assert torch.equal(torch.isfinite(got), clean) and torch.equal(got[clean].view(torch.int16), want[clean].view(torch.int16))
+
+
 @pytest.mark.parametrize("T,E,K,N,k,cap,pad", [
     (12000, 8, 128, 4096, 1, 1500, False),   # overflow dropped, the shortest K loop
     (12000, 8, 192, 4104, 1, 1700, True),    # padded to the capacity: empty slots, odd K-steps, N tail
@@ -670,7 +708,7 @@ def _kernel_for(P, E, K, N):
     """Which kernel the host takes for these sizes (all but the weighted accumulate form), on 256 CUs."""
     used = min(E, P)
     big = ((P + 255) // 256 + (E + 1) // 2) * -(-N // 256)
-    if K % 64 == 0 and K >= 128 and P > E * 160 and big >= 192:
+    if K >= 128 and P > E * 160 and big >= 192:
         def rounds(waves):  # of the 160-row kernel's tiles; two workgroups of two wavefronts fit a CU
             n = max((P + 159) // 160, used) * -(-N // (64 * waves))
             return -(-n // 512) * 2 if waves == 2 else -(-n // 256)
