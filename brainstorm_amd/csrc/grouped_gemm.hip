@@ -620,7 +620,11 @@ int launch_act(GemmArgs& a, hipStream_t st) {
   // experts of at most one row block on average.  Experts with many row blocks read their
   // weights once per row block, and those re-reads are served by the caches only if the first
   // read left the lines there.
-  const bool stream_weights = static_cast<long>(a.P) <= static_cast<long>(a.E) * BM;
+  const bool read_once = static_cast<long>(a.P) <= static_cast<long>(a.E) * BM;
+  // ... and rows are whole 128-byte lines: of others a K-step of 64 reads parts of two lines, and a line that is not kept comes from
+  // memory again for the next K-step (us, streamed and not: 32 x 100 rows 888 -> 3552 68 and 48, 8 x 150 rows 1592 -> 6368 55 and 36,
+  // 64 x 100 rows 2016 -> 504 45 and 35, 12 x 140 rows 1800 -> 7200 152 and 139).
+  const bool stream_weights = read_once && a.K % kBK == 0;
   // only the 4-wavefront tiles have the registers to walk column tiles
   constexpr bool kCanWalk = WAVES == 4;
   if (!kCanWalk) a.walk = 1, a.groups_n = a.tiles_n;
@@ -630,7 +634,7 @@ int launch_act(GemmArgs& a, hipStream_t st) {
   // 1652 -> 1596 us and 1443 -> 1379 us, 8 experts x 4096 rows 1106 -> 1053 us and 1019 -> 999 us,
   // the top-2 shape with three row blocks per expert the same within 2 %; 2, 8 or 16 row blocks per
   // patch instead of 4 change these by less than 1 %.
-  a.patch = (a.tags == nullptr && !stream_weights) ? 1 : 0;
+  a.patch = (a.tags == nullptr && !read_once) ? 1 : 0;
   long grid_wgs = static_cast<long>(a.tiles_m_max) * a.groups_n;
   if (a.patch) grid_wgs = (grid_wgs + 255) / 256 * 256;  // whole rounds of 32 workgroups per XCD
   const dim3 blocks(static_cast<unsigned>(grid_wgs)), threads(WAVES * 64);
