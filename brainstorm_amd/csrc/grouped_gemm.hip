@@ -718,7 +718,7 @@ bool wide_tiles_come_in_rounds(const GemmArgs& a) {
 
 // Shapes whose fp32 rows the few-rows kernel rounds itself when asked to; where that is the faster way, skinny_gemm_takes_f32 says.
 bool runs_on_f32_rows(const GemmArgs& a) {
-  return a.P <= 64l * std::min(a.E, a.P) && !wide_tiles_come_in_rounds(a) && skinny_gemm_applies(a);
+  return a.P <= 64l * std::min(a.E, a.P) && !wide_tiles_come_in_rounds(a) && few_rows_by_weight(a);
 }
 
 int grouped_gemm_impl(const void* x, const void* const* weights, const void* const* biases, void* out,

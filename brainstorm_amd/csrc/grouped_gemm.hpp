@@ -43,6 +43,7 @@ int launch_pingpong_gemm(GemmArgs& a, int act, hipStream_t st);
 
 // The kernel for few rows per expert and few tiles (grouped_gemm_skinny.hip), every form.
 bool skinny_gemm_applies(const GemmArgs& a);
+bool few_rows_by_weight(const GemmArgs& a);  // ... and fp32 rows may be handed to it
 bool skinny_gemm_takes_f32(const GemmArgs& a, int cells);
 int launch_skinny_gemm(GemmArgs& a, int act, hipStream_t st);
 

@@ -427,7 +427,7 @@ int launch_act(GemmArgs& a, int act, hipStream_t st) {
 //     them every XCD reads most of x and of the weights: 64 x 120 rows 2048 -> 256 35.7 there, 43.1 here),
 //     and up to 160 with fewer experts than XCDs, some of which the 160-row kernel leaves idle (4 x 120 rows
 //     2048 -> 8192 69.3 -> 41.9).
-bool skinny_gemm_applies(const GemmArgs& a) {
+bool few_rows_by_weight(const GemmArgs& a) {
   const long used = std::min(a.E, a.P);
   const long tiles = std::max<long>((a.P + 159) / 160, used) * ((a.N + 255) / 256);
   const double weight_bytes = 2.0 * used * a.N * a.K;
@@ -443,6 +443,15 @@ bool skinny_gemm_applies(const GemmArgs& a) {
   return tiles <= 160 && weight_bytes < 1.5e8;
 }
 
+// Besides, with any weight, few rows whose weight rows are no whole 128-byte lines: this kernel keeps the memory's rate there
+// (64 x 4 rows 1432 -> 4680 146 us), the wide tiles, which walk the lines of 256 columns at a time, do not (181).  68 drawn shapes of
+// 0.3 to 4.2 GB, 1 to 20 rows per expert: 0.85 of the wide tiles' time in the mean; with more rows, or more than 12 and a long K, the
+// two are level or those win (64 x 15 rows 4848 -> 2032 241 us here, 234 there; 64 x 31 rows 5152 -> 680 100 and 93).
+bool skinny_gemm_applies(const GemmArgs& a) {
+  const long used = std::min(a.E, a.P);
+  return few_rows_by_weight(a) || (a.K % kBK != 0 && a.P <= (a.K < 4096 ? 20 : 12) * used);
+}
+
 namespace {
 // Estimated tiles of `block` x 64 of the result; an expert's last row block is taken as half full.
 double narrow_tiles(const GemmArgs& a, int block) {
@@ -454,7 +463,7 @@ bool takes_64_rows(const GemmArgs& a) { return a.P > 32l * std::min(a.E, a.P) &&
 }  // namespace
 
 // Where fp32 rows are rounded by this kernel, of the shapes of up to 64 rows per expert whose bf16 rows it takes
-// (skinny_gemm_applies): where it is faster than the cast kernel and the bf16 form behind each other.  It saves a
+// (few_rows_by_weight): where it is faster than the cast kernel and the bf16 form behind each other.  It saves a
 // launch and a pass over the rows, but every column tile reads twice the bytes of the rows again, and fewer stages
 // fit the LDS.  The line was drawn on 3757 shapes (1 to 64 rows per expert, 4 to 128 experts, K 256 to 8192, N 512
 // to 8192, rows in order or gathered for one or two paths; both sides back to back in a graph; more rows lose: 32

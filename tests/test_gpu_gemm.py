@@ -565,6 +565,18 @@ def test_end_of_the_list_of_ping_pong_tiles_in_units(loads, K, N, cut):
     run(loads, K, N, act="relu", bias=True, seed=2, slack=300)
 
 
+# 0.3 GB of weights and more in rows that are no whole 128-byte lines: few rows, and a row too many for them
+@pytest.mark.parametrize("loads,K,N,kernel", [
+    ([20] * 59 + [0, 40], 1592, 1608, "few rows"),
+    ([20] * 59 + [0, 41], 1592, 1608, "160 rows"),
+    ([12] * 16, 4104, 2304, "few rows"),
+    ([12] * 15 + [13], 4104, 2304, "160 rows"),
+])
+def test_few_rows_of_large_weights_in_part_filled_lines(loads, K, N, kernel):
+    assert _kernel_for(sum(loads), len(loads), K, N) == kernel
+    run(loads, K, N, act="gelu", bias=True)
+
+
 # K = 64 n + 8, 56 and others: the part-filled K-step is the third and later ones, in the list and in units of 64, 128 and 256 rows whose
 # rings of four to eight K-steps it ends inside, at the end of and behind
 @pytest.mark.parametrize("loads,K,N", [
@@ -724,6 +736,7 @@ def _kernel_for(P, E, K, N):
         few = True
     elif P <= 28 * used:
         few = weight < 3e8 or (weight < 1e9 and (tiles <= 128 or K % 2048 == 0 or 2 * P <= 3 * used))
+        few = few or (K % 64 != 0 and P <= (20 if K < 4096 else 12) * used)
     else:
         few = tiles <= 160 and weight < 1.5e8
     return "few rows" if few else "160 rows"
