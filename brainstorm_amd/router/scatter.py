@@ -58,10 +58,11 @@ class ScatterRouter(RouterBase):
             self.protocol.compact = True
 
     def _route(self, in_flows, score: torch.Tensor):
-        hot_mask = self.protocol(score)
+        modules = self._modules  # (an attribute of a Module that is a Module is looked up by Python code)
+        hot_mask = modules["protocol"](score)
         if self.dispatch_score:
             in_flows = in_flows + [score] if isinstance(in_flows, list) else [in_flows, score]
-        return self.fabric(in_flows, hot_mask, None, score)
+        return modules["fabric"](in_flows, hot_mask, None, score)
 
     def forward(self, in_flows, score: torch.Tensor):
         out_flows, _ = self._route(in_flows, score)
@@ -99,7 +100,8 @@ class SwinMoEScatterRouter(RouterBase):
             self.protocol.padding = (self.fabric.capacity_padding, self.fabric.path_wise_padding)
 
     def forward(self, in_flows, score, logits_wo_noise, logits):
+        fabric = self.fabric
         hot_mask, runtime_capacities, new_score, _loss = self.protocol(score, logits_wo_noise, logits)
-        if self.fabric.max_path_load == 0:  # fixed stride = the runtime capacity (one host read)
-            self.fabric.max_path_load = runtime_capacities[0].item()
-        return self.fabric(in_flows, hot_mask, runtime_capacities, new_score)
+        if fabric.max_path_load == 0:  # fixed stride = the runtime capacity (one host read)
+            fabric.max_path_load = runtime_capacities[0].item()
+        return fabric(in_flows, hot_mask, runtime_capacities, new_score)

@@ -117,6 +117,23 @@ def is_metadata_read(func) -> bool:
 class DeferredRows(torch.Tensor):
     """Plain-tensor view of a deferred buffer (what ``brt.to_torch_tensor`` returns for it)."""
 
+    # What an expert reads of its rows to allocate its outputs, as the buffer has it: 0.3 us each instead of 0.9 through
+    # ``__torch_function__``.  Nothing changes them in place: an operator is given a filled plain alias (`_settled`).
+    @property
+    def shape(self):
+        state = self.__dict__.get("_brt_state")
+        return state.buffer.shape if state is not None else _plain(self).shape
+
+    @property
+    def dtype(self):
+        state = self.__dict__.get("_brt_state")
+        return state.buffer.dtype if state is not None else _plain(self).dtype
+
+    @property
+    def device(self):
+        state = self.__dict__.get("_brt_state")
+        return state.buffer.device if state is not None else _plain(self).device
+
     @classmethod
     def __torch_function__(cls, func, types, args=(), kwargs=None):
         kwargs = kwargs or {}

@@ -343,3 +343,20 @@ def test_split_compiles_as_one_graph():
     run = _observed_passes()["split"]
     x = torch.arange(10.0).view(5, 2)
     assert torch.equal(torch.compile(run, backend="eager", fullgraph=True)(x), 2 * x)
+
+
+def test_metadata_of_unfilled_rows_is_read_without_filling_them():
+    import copy
+
+    from brainstorm_amd.runtime.deferred import DeferredRows, lazy_tensor
+
+    fills = []
+    buffer = torch.empty(3, 5, dtype=torch.bfloat16)
+    rows = lazy_tensor(buffer, lambda b: fills.append(b.fill_(2)))
+    assert (rows.shape, rows.dtype, rows.device) == (torch.Size([3, 5]), torch.bfloat16, buffer.device)
+    assert rows.shape[0] == rows.size(0) == len(rows) and not fills
+    assert torch.equal(rows + 1, torch.full((3, 5), 3, dtype=torch.bfloat16)) and len(fills) == 1
+    assert rows.shape == buffer.shape and len(fills) == 1
+    stateless = buffer.as_subclass(DeferredRows)  # what a copy that drops the attributes is
+    assert (stateless.shape, stateless.dtype, stateless.device) == (buffer.shape, buffer.dtype, buffer.device)
+    assert copy.copy(rows).shape == buffer.shape
