@@ -716,6 +716,23 @@ bool wide_tiles_come_in_rounds(const GemmArgs& a) {
   return other.waves != 2 && (2 * tiles >= 3 * cus || other.cost > 2 * (160 + 64 * 4));
 }
 
+// 29 to 64 rows per expert, beyond what skinny_gemm_applies takes: where the 160-row tiles leave a large part of their last round over
+// the CUs empty (or are fewer than the CUs), 64 x 64 tiles are faster though every block of rows reads the weights again.  Both sides by
+// the operand rows that the busiest, respectively the average, CU streams.  The line was drawn on 285 shapes of uniform loads that the
+// 160-row kernel had before, and tried on 130 others, two thirds of them with ragged and skewed loads: 0.71 of its time in the mean, the worst 2 % over it.  us, 160-row and few-rows:
+// 64 x 43 rows 256 -> 5312 72 and 39, 12 x 39 rows 1344 -> 7168 73 and 39, 60 x 46 rows 384 -> 3136 59 and 30, 4 x 53 rows 3008 -> 6464
+// 89 and 28.  Not taken: contracting shapes (64 x 60 rows 2240 -> 768 42 and 54, 64 x 33 rows 2880 -> 832 53 and 66), large weights
+// of skewed experts (8 x 58 rows 2496 -> 9984 87 and 95), more rows (32 x 65 rows 1376 -> 5504 112 and 157); a K below 256 was not timed.
+bool short_rounds_suit_few_rows(const GemmArgs& a) {
+  const long used = std::min(a.E, a.P);
+  if (a.P <= 28 * used || a.P > 64 * used || a.N < a.K || a.K < 256) return false;
+  const double weight_bytes = 2.0 * used * a.N * a.K;
+  const double few = 128.0 * used * ((a.N + 63) / 64) / device_cus(), wide = width_of_160_row_tiles(a.P, a.E, a.N).cost;
+  if (a.N < 2l * a.K) return few < 0.9 * wide && weight_bytes < 4e8;
+  if (weight_bytes < 2.5e8) return few < (used > 8 ? 1.1 : 1.0) * wide;
+  return few < 0.95 * wide && weight_bytes < 1.2e9 && a.P <= 48 * used;
+}
+
 // Shapes whose fp32 rows the few-rows kernel rounds itself when asked to; where that is the faster way, skinny_gemm_takes_f32 says.
 bool runs_on_f32_rows(const GemmArgs& a) {
   return a.P <= 64l * std::min(a.E, a.P) && !wide_tiles_come_in_rounds(a) && few_rows_by_weight(a);
@@ -795,7 +812,7 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   // The rule is the same for gathered, scattered and fp32-output rows: a gathering 1024 -> 4096 GEMM with GELU over 32768
   // rows of 16 experts takes 437 us on the 160-row kernel and 336 us here.
   if (wide_tiles_come_in_rounds(a)) return launch_pingpong_gemm(a, act, as_stream(stream));
-  if (skinny_gemm_applies(a)) return launch_skinny_gemm(a, act, as_stream(stream));
+  if (skinny_gemm_applies(a) || short_rounds_suit_few_rows(a)) return launch_skinny_gemm(a, act, as_stream(stream));
   if (out_is_f32) {
     if (act == BRT_ACT_GELU) return launch_f32<BRT_ACT_GELU>(a, as_stream(stream));
     if (act == BRT_ACT_RELU) return launch_f32<BRT_ACT_RELU>(a, as_stream(stream));

@@ -577,6 +577,19 @@ def test_few_rows_of_large_weights_in_part_filled_lines(loads, K, N, kernel):
     run(loads, K, N, act="gelu", bias=True)
 
 
+# 29 to 64 rows per expert where the 160-row tiles come in part-filled rounds, and where they do not
+@pytest.mark.parametrize("loads,K,N,kernel", [
+    ([43] * 60 + [0, 1, 160, 11], 256, 5312, "few rows"),
+    ([64] * 12, 1344, 7168, "few rows"),
+    ([64] * 11 + [65], 1344, 7168, "160 rows"),
+    ([45] * 12, 2048, 3136, "few rows"),
+    ([60] * 64, 896, 3584, "160 rows"),
+])
+def test_few_rows_where_wide_tiles_fill_part_of_a_round(loads, K, N, kernel):
+    assert _kernel_for(sum(loads), len(loads), K, N) == kernel
+    run(loads, K, N, act="gelu", bias=True)
+
+
 # K = 64 n + 8, 56 and others: the part-filled K-step is the third and later ones, in the list and in units of 64, 128 and 256 rows whose
 # rings of four to eight K-steps it ends inside, at the end of and behind
 @pytest.mark.parametrize("loads,K,N", [
@@ -739,6 +752,11 @@ def _kernel_for(P, E, K, N):
         few = few or (K % 64 != 0 and P <= (20 if K < 4096 else 12) * used)
     else:
         few = tiles <= 160 and weight < 1.5e8
+        if N >= K >= 256:  # part-filled rounds of the 160-row tiles
+            share = 128 * used * -(-N // 64) / 256 / min(-(-used * -(-N // (64 * w)) // (512 if w == 2 else 256)) * (2 if w == 2 else 1)
+                                                         * (160 + 64 * w) for w in (2, 3, 4))
+            few = few or ((share < (1.1 if used > 8 else 1.0) if weight < 2.5e8 else share < 0.95 and weight < 1.2e9 and P <= 48 * used)
+                          if N >= 2 * K else weight < 4e8 and share < 0.9)
     return "few rows" if few else "160 rows"
 
 
