@@ -24,7 +24,6 @@ __all__ = [
     "throttle_hotmask",
     "top1_to_capacity",
     "top1_route_to_capacity",
-    "take_generated_route",
     "Route",
     "CompactRoute",
     "remember_route",
@@ -206,36 +205,14 @@ def top1_to_capacity(score: torch.Tensor, capacity: int):
     return _lib.native().top1_to_capacity(score, int(capacity))
 
 
-class _GeneratedRoute:
-    """The route of a hot mask, generated along with the mask, and what it was generated from."""
-
-    __slots__ = ("route", "capacities", "options", "versions")
-
-    def __init__(self, route, mask, capacities, options):
-        self.route, self.capacities, self.options = route, capacities, options
-        self.versions = (mask._version, capacities._version)
-
-
 def top1_route_to_capacity(score: torch.Tensor, capacity: int, capacity_padding: bool, path_wise_padding: bool):
-    """:func:`top1_to_capacity` whose second launch also lays out the seats of the throttled mask (not in the reference).
-    Returns the same pair; :func:`take_generated_route` hands the route over to whoever asks for it next."""
-    options = (bool(capacity_padding), bool(path_wise_padding))
-    made = _lib.native().top1_route_to_capacity(score, int(capacity), *options)
+    """:func:`top1_to_capacity` whose second launch also lays out the seats of the throttled mask (not in the reference):
+    the same pair, and the :class:`Route` that ``generate_route`` would make of it."""
+    made = _lib.native().top1_route_to_capacity(score, int(capacity), bool(capacity_padding), bool(path_wise_padding))
     if made is None:
         return None
     mask, capacities, seats, loads, counts = made
-    mask._brt_generated = _GeneratedRoute(Route(seats, loads, counts, False, True), mask, capacities, options)
-    return mask, capacities
-
-
-def take_generated_route(hot_mask: torch.Tensor, supported_capacities, capacity_padding: bool, path_wise_padding: bool):
-    """What ``generate_route`` would return for these arguments (seat indices) if it was generated along with the mask and
-    nothing has changed since, else None.  Handed out once: its tensors belong to one caller."""
-    made = hot_mask.__dict__.pop("_brt_generated", None)
-    if (made is None or supported_capacities is not made.capacities or (bool(capacity_padding), bool(path_wise_padding)) != made.options
-            or (hot_mask._version, supported_capacities._version) != made.versions):
-        return None
-    return made.route
+    return mask, capacities, Route(seats, loads, counts, False, True)
 
 
 def generate_route(

@@ -225,14 +225,12 @@ class DispatchFabric(FabricBase):
         self._route = None  # the route of the forward call in progress
 
     def forward(self, in_flow, hot_mask: torch.Tensor, runtime_capacities: torch.Tensor = None,
-                score: torch.Tensor = None):
+                score: torch.Tensor = None, route: Optional[c_router.Route] = None):
+        """``route`` (not in the reference): the seat route of this mask and these capacities, from a caller that has it."""
         caps = runtime_capacities if runtime_capacities is not None else self.supported_capacities
         in_flows = [in_flow] if self.flow_num == 1 else in_flow
         as_tags = self._defers(in_flows, runtime_capacities, hot_mask)
-        route = None
-        if not as_tags and hasattr(hot_mask, "_brt_generated"):  # the protocol's kernel has laid the route out too
-            route = c_router.take_generated_route(hot_mask, caps, self.capacity_padding, self.path_wise_padding)
-        if route is None:
+        if route is None or as_tags:
             route = c_router.generate_route(
                 hot_mask, supported_capacities=caps, capacity_padding=self.capacity_padding,
                 path_wise_padding=self.path_wise_padding, is_tag_index=as_tags,
@@ -483,14 +481,14 @@ class FusedDispatchFabric(DispatchFabric):
         out = init_grid_tensor(routed, tags[:-1] + [indices], load_stack[:-1] + [loads], extra)
         return (out if self.flow_num == 1 else [out]), score
 
-    def forward(self, in_flow, hot_mask, runtime_capacities=None, score=None):
+    def forward(self, in_flow, hot_mask, runtime_capacities=None, score=None, route=None):
         in_flows = [in_flow] if self.flow_num == 1 else in_flow
         if isinstance(hot_mask, CompactHotMask):
             if self._takes_compact(in_flows, runtime_capacities):
                 return self._forward_compact(in_flows, hot_mask, score)
             hot_mask = hot_mask.dense()  # a shape this path does not take: the mask, as the reference
         if not self._in_one_step(in_flows, runtime_capacities, hot_mask):
-            return super().forward(in_flow, hot_mask, runtime_capacities, score)
+            return super().forward(in_flow, hot_mask, runtime_capacities, score, route)
         # static rows, one flow, single-path route: index generation moves the rows itself
         data, tags, load_stack, extra = to_torch_tensor(in_flows[0], retrieve_attr=True)
         assert tags[-1] is None  # fused dispatch starts from freshly annotated cells

@@ -311,9 +311,6 @@ class SwinMoEProtocol(ProtocolBase):
         self.group = group
         self.is_gshard_loss = is_gshard_loss
         self.alignment = alignment
-        #: set by a SwinMoEScatterRouter: (capacity_padding, path_wise_padding) of the fabric that takes the decision, whose
-        #: route the throttling kernel then lays out along with the mask
-        self.padding = None
 
     def runtime_capacity(self, cells: int, paths: int) -> int:
         if self.capacity_factor <= 0:
@@ -321,21 +318,25 @@ class SwinMoEProtocol(ProtocolBase):
         per_path = (int(cells) + paths - 1) // paths
         return self.top_k * int(self.capacity_factor * per_path)  # swin_moe.py:112-119
 
-    def make_route_decision(self, score, logits_wo_noise, logits):
+    def make_route_decision(self, score, logits_wo_noise, logits, padding=None):
+        """Hot mask, runtime capacities, score, loss.  With ``padding`` (not in the reference), the (capacity_padding,
+        path_wise_padding) of the fabric that is handed this decision: a fifth value, the route that the throttling kernel
+        laid out for it along with the mask, or None."""
         paths = score.size(1)
         loss = self.generate_auxiliary(score, logits_wo_noise, logits, None)
         cap = self.runtime_capacity(score.size(0), paths)
         if not self.batch_prioritized_routing and _kernel_takes(score):
-            both = (c_router.top1_to_capacity(score, cap) if self.padding is None
-                    else c_router.top1_route_to_capacity(score, cap, *self.padding))
-            if both is not None:
-                return both[0], both[1], score, loss
+            made = (c_router.top1_to_capacity(score, cap) if padding is None
+                    else c_router.top1_route_to_capacity(score, cap, *padding))
+            if made is not None:
+                return (*made[:2], score, loss, *made[2:])
         mask = _topk_hot_mask(score, 1)  # the first of the top-k choices (swin_moe.py:101-107)
         runtime_capacities = torch.full((paths,), cap, dtype=torch.int32, device=score.device)
         prefix = torch.zeros((paths,), dtype=torch.int32, device=score.device)
         hot_mask, _ = throttle_to_capacity(
             mask, prefix, runtime_capacities, self.batch_prioritized_routing, score)
-        return hot_mask, runtime_capacities, score, loss
+        decision = (hot_mask, runtime_capacities, score, loss)
+        return decision if padding is None else (*decision, None)
 
     def generate_auxiliary(self, score, logits_wo_noise, logits, topk_ids):
         return None  # the reference's auxiliary loss is commented out (swin_moe.py:241-252)

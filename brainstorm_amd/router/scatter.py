@@ -7,10 +7,11 @@ and ``SwinMoEScatterRouter`` return ``(flows, score)`` (:254-255, :162-165).
 from typing import Any, Dict
 
 import torch
+from torch.nn.modules.module import _has_any_global_hook
 
 from brainstorm_amd.router.base import RouterBase, register_router
-from brainstorm_amd.router.fabric import make_fabric
-from brainstorm_amd.router.protocol import make_protocol
+from brainstorm_amd.router.fabric import DispatchFabric, FusedDispatchFabric, make_fabric
+from brainstorm_amd.router.protocol import ProtocolBase, SwinMoEProtocol, make_protocol
 
 __all__ = ["ScatterRouter", "SwinMoEScatterRouter", "TaskScatterRouter"]
 
@@ -77,6 +78,24 @@ class TaskScatterRouter(ScatterRouter):
         return self._route(in_flows, score)
 
 
+_OWN_FORWARD, _OWN_DECISION = ProtocolBase.forward, SwinMoEProtocol.make_route_decision
+_OWN_DISPATCH = (DispatchFabric.forward, FusedDispatchFabric.forward)
+
+
+def _padding_of_a_route_made_with_the_mask(protocol, fabric):
+    """(capacity_padding, path_wise_padding) where the decision goes from the protocol's kernel straight into the fabric's
+    index generation, which the kernel may then do along with it; None where a hook, a subclass, a replaced method or the
+    protocol's check can see the mask in between: they may change it, and index generation reads what they leave."""
+    if (not isinstance(protocol, SwinMoEProtocol) or not isinstance(fabric, DispatchFabric)
+            or protocol._forward_hooks or protocol._forward_pre_hooks or fabric._forward_hooks
+            or fabric._forward_pre_hooks or _has_any_global_hook() or protocol.debug
+            or getattr(protocol.forward, "__func__", None) is not _OWN_FORWARD
+            or getattr(protocol.make_route_decision, "__func__", None) is not _OWN_DECISION
+            or getattr(fabric.forward, "__func__", None) not in _OWN_DISPATCH):
+        return None
+    return fabric.capacity_padding, fabric.path_wise_padding
+
+
 @register_router("swin_moe_scatter")
 class SwinMoEScatterRouter(RouterBase):
     ALLOWED_PROTOCOL_TYPES = ["swin_moe"]
@@ -96,12 +115,17 @@ class SwinMoEScatterRouter(RouterBase):
         self.fabric_kwargs = _merged(
             {"flow_num": 1, "route_logic": ["1d"], "transform": [False]}, fabric_kwargs)
         self.fabric = make_fabric(fabric_type, self.fabric_kwargs)
-        if hasattr(self.fabric, "capacity_padding"):  # a fabric that generates indices from the mask
-            self.protocol.padding = (self.fabric.capacity_padding, self.fabric.path_wise_padding)
 
     def forward(self, in_flows, score, logits_wo_noise, logits):
-        fabric = self.fabric
-        hot_mask, runtime_capacities, new_score, _loss = self.protocol(score, logits_wo_noise, logits)
+        protocol, fabric = self.protocol, self.fabric
+        padding = _padding_of_a_route_made_with_the_mask(protocol, fabric)
+        if padding is None:
+            hot_mask, runtime_capacities, new_score, _loss = protocol(score, logits_wo_noise, logits)
+            fabric, route = self.fabric, None
+        else:
+            hot_mask, runtime_capacities, new_score, _loss, route = protocol(score, logits_wo_noise, logits, padding=padding)
         if fabric.max_path_load == 0:  # fixed stride = the runtime capacity (one host read)
             fabric.max_path_load = runtime_capacities[0].item()
-        return fabric(in_flows, hot_mask, runtime_capacities, new_score)
+        if route is None:
+            return fabric(in_flows, hot_mask, runtime_capacities, new_score)
+        return fabric(in_flows, hot_mask, runtime_capacities, new_score, route)
