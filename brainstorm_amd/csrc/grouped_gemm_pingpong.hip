@@ -197,7 +197,9 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   const int tiles = (many + few) * tn, rest = tiles & (kRound - 1);
   int moved = min(few, over_tn(rest + tn - 1));
   int cut = max(moved * tn, rest);  // tiles
-  if (cut > kMostCut || tiles > kMostRounds * kRound || tiles + 3 * cut > a.grid - (a.row_tags_out != nullptr ? 1 : 0)) cut = 0;
+  // (the timed form wants the clocks of a whole tile, also of a list that would be cut to the last)
+  if (a.clocks != nullptr || cut > kMostCut || tiles > kMostRounds * kRound ||
+      tiles + 3 * cut > a.grid - (a.row_tags_out != nullptr ? 1 : 0)) cut = 0;
   if (cut == 0) moved = 0;
   const int listed = tiles - moved * tn, whole = tiles - cut, used = tiles + 3 * cut;
   if (t >= used) {

@@ -1169,6 +1169,36 @@ def test_timed_grouped_gemm_gives_the_same_rows_and_plausible_clocks():
                                         d_loads.data_ptr(), E, P, K, N, ACT["none"], None, st) == -1
 
 
+@pytest.mark.parametrize("loads,K,N", [
+    ([1024] * 4, 512, 1024),              # 64 tiles: a list that the plain form cuts into units to the last
+    ([1024] * 8, 512, 512),
+    ([100, 0, 30, 129], 192, 256),        # blocks of few rows and nothing else
+    ([2049] + [2048] * 7, 128, 4096),     # the end of the list
+])
+def test_timed_grouped_gemm_writes_its_clocks_whatever_the_list(loads, K, N):
+    from brainstorm_amd import _lib
+
+    L = _lib.lib()
+    E, P = len(loads), sum(loads)
+    ws, wt = _expert_tables(E, K, N, 3)
+    x = torch.randn(P, K, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).cuda()
+    d_loads = torch.tensor(loads, dtype=torch.int32, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    plain, timed = torch.full((2, P, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    clocks = torch.zeros(3, dtype=torch.int64, device="cuda")
+    _lib.check(L.brt_hip_grouped_gemm(x.data_ptr(), wt.data_ptr(), None, plain.data_ptr(), d_loads.data_ptr(), E, P, K, N,
+                                      ACT["none"], st))
+    _lib.check(L.brt_hip_grouped_gemm_timed(x.data_ptr(), wt.data_ptr(), None, timed.data_ptr(), d_loads.data_ptr(), E, P, K, N,
+                                            ACT["none"], clocks.data_ptr(), st))
+    torch.cuda.synchronize()
+    assert torch.equal(plain.view(torch.int16), timed.view(torch.int16))
+    shader, ticks, k_steps = (int(v) for v in clocks)
+    assert k_steps == K // 64 and shader > 0 and ticks > 0
+    if loads[0] >= 256:  # a full tile
+        assert shader >= 2048 * k_steps
+    del ws
+
+
 @pytest.mark.parametrize("by_kernel,E,rows,K,N,act,bias", [
     (1, 8, 3, 768, 3072, "gelu", False), (1, 24, 10, 72, 392, None, True),  # 32 x 64 tiles, K and N tails
     (1, 16, 60, 2048, 512, None, False), (1, 16, 40, 200, 328, "relu", True),  # ... of more than 32 rows
