@@ -28,7 +28,7 @@ struct GemmArgs {
   float* acc_out;
   int tiles_n, tiles_m_max;
   int walk, groups_n;  // column tiles one workgroup walks, ceil(tiles_n / walk)
-  int grid;                  // workgroups (ping-pong kernel)
+  int grid;                  // workgroups, 0 where no tile may be cut into units (ping-pong kernel)
   uint32_t tiles_n_inverse;  // (2^32 - 1) / tiles_n (ping-pong kernel)
   int patch;           // workgroups in patch order (experts with several row blocks), see the kernel
   // measurement aid (ping-pong kernel only): non-null, the workgroup of the first tile writes the

@@ -197,9 +197,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   const int tiles = (many + few) * tn, rest = tiles & (kRound - 1);
   int moved = min(few, over_tn(rest + tn - 1));
   int cut = max(moved * tn, rest);  // tiles
-  // (the timed form wants the clocks of a whole tile, also of a list that would be cut to the last)
-  if (a.clocks != nullptr || cut > kMostCut || tiles > kMostRounds * kRound ||
-      tiles + 3 * cut > a.grid - (a.row_tags_out != nullptr ? 1 : 0)) cut = 0;
+  if (cut > kMostCut || tiles > kMostRounds * kRound || tiles + 3 * cut > a.grid - (a.row_tags_out != nullptr ? 1 : 0)) cut = 0;
   if (cut == 0) moved = 0;
   const int listed = tiles - moved * tn, whole = tiles - cut, used = tiles + 3 * cut;
   if (t >= used) {
@@ -707,7 +705,9 @@ int launch_pingpong(GemmArgs& a, hipStream_t st) {
   const long entries = (static_cast<long>(a.P + kBM - 1) / kBM + a.E) * a.tiles_n;
   const long round = kXcds * kCusPerXcd;
   const long grid = (entries + round - 1) / round * round;
-  a.grid = static_cast<int>(grid);
+  // The timed form wants the clocks of a whole tile, also of a list that would be cut to the last: it is told of no workgroups for units.
+  // (A test of a.clocks in the kernel itself cost 32768 rows of 16 experts 1024 -> 4096 -> 1024 7 us of 577.)
+  a.grid = a.clocks != nullptr ? 0 : static_cast<int>(grid);
   a.tiles_n_inverse = 0xffffffffu / static_cast<uint32_t>(a.tiles_n);
   auto* fn = &grouped_gemm_pingpong_kernel<ACT, ROUTED, OUTF32>;
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(fn), kLdsBytes); rc != BRT_OK) return rc;
