@@ -360,3 +360,59 @@ def test_metadata_of_unfilled_rows_is_read_without_filling_them():
     stateless = buffer.as_subclass(DeferredRows)  # what a copy that drops the attributes is
     assert (stateless.shape, stateless.dtype, stateless.device) == (buffer.shape, buffer.dtype, buffer.device)
     assert copy.copy(rows).shape == buffer.shape
+
+
+_METADATA_READS = {
+    "shape": lambda rows: torch.ones(3) * rows.shape[0],
+    "dtype": lambda rows: torch.ones(3, dtype=rows.dtype),
+    "device": lambda rows: torch.ones(3, device=rows.device),
+}
+
+
+@pytest.mark.parametrize("built", [True, False])
+@pytest.mark.parametrize("name", list(_METADATA_READS))
+def test_metadata_reads_of_unfilled_rows_compile_as_one_graph(monkeypatch, name, built):
+    """... of rows of several sizes, of an alias without its state, and inside a function mode.  (Compiling fills the rows that it is
+    handed; what is asked here is that it takes them.)"""
+    from brainstorm_amd.runtime.deferred import DeferredRows, DeferredState, lazy_tensor, wrap_if_pending
+    from torch.overrides import TorchFunctionMode
+
+    class Passing(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    if not built:
+        monkeypatch.setattr(_lib, "native_or_none", lambda: None)
+    run = _METADATA_READS[name]
+    monkeypatch.setattr(DeferredState, "materialize", lambda self: None)
+    kinds = {
+        "lazy": lambda buffer: lazy_tensor(buffer, lambda b: None),
+        "deferred": lambda buffer: wrap_if_pending(buffer.view(buffer.shape), {"key": DeferredState(None, None, buffer, "key")}),
+        "alias": lambda buffer: buffer.as_subclass(DeferredRows),
+    }
+    for kind, make in kinds.items():
+        torch._dynamo.reset()
+        compiled = torch.compile(run, backend="eager", fullgraph=True)
+        for size in (4, 6, 1, 9):
+            rows = make(torch.empty(size, 2, dtype=torch.bfloat16))
+            assert isinstance(rows, DeferredRows)
+            want = run(torch.empty(size, 2, dtype=torch.bfloat16))
+            assert torch.equal(compiled(rows), want) and compiled(rows).dtype == want.dtype, (kind, size)
+        with Passing():
+            assert torch.equal(compiled(rows), want), kind
+
+
+def test_function_modes_see_metadata_reads_of_unfilled_rows():
+    from brainstorm_amd.runtime.deferred import DeferredRows, lazy_tensor
+    from torch.overrides import TorchFunctionMode
+
+    class Called(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append((func, type(args[0])))
+            return func(*args, **(kwargs or {}))
+
+    rows = lazy_tensor(torch.empty(3, 5), lambda b: seen.append("filled"))
+    seen = []
+    with Called():
+        assert (rows.shape, rows.dtype, rows.device) == ((3, 5), torch.float32, torch.device("cpu"))
+    assert seen == [(getattr(torch.Tensor, name).__get__, DeferredRows) for name in ("shape", "dtype", "device")]
