@@ -414,5 +414,6 @@ def test_function_modes_see_metadata_reads_of_unfilled_rows():
     rows = lazy_tensor(torch.empty(3, 5), lambda b: seen.append("filled"))
     seen = []
     with Called():
-        assert (rows.shape, rows.dtype, rows.device) == ((3, 5), torch.float32, torch.device("cpu"))
+        read = (rows.shape, rows.dtype, rows.device)
+    assert read == ((3, 5), torch.float32, torch.device("cpu"))
     assert seen == [(getattr(torch.Tensor, name).__get__, DeferredRows) for name in ("shape", "dtype", "device")]
