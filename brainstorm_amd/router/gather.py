@@ -28,4 +28,4 @@ class GatherRouter(RouterBase):
         self.fabric = make_fabric(fabric_type, self.fabric_kwargs)
 
     def forward(self, in_flows, residual_flows=None, score=None):
-        return self._modules["fabric"](in_flows, residual_flows, score)
+        return self.fabric(in_flows, residual_flows, score)

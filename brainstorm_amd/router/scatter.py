@@ -59,11 +59,10 @@ class ScatterRouter(RouterBase):
             self.protocol.compact = True
 
     def _route(self, in_flows, score: torch.Tensor):
-        modules = self._modules  # (an attribute of a Module that is a Module is looked up by Python code)
-        hot_mask = modules["protocol"](score)
+        hot_mask = self.protocol(score)
         if self.dispatch_score:
             in_flows = in_flows + [score] if isinstance(in_flows, list) else [in_flows, score]
-        return modules["fabric"](in_flows, hot_mask, None, score)
+        return self.fabric(in_flows, hot_mask, None, score)
 
     def forward(self, in_flows, score: torch.Tensor):
         out_flows, _ = self._route(in_flows, score)
