@@ -119,12 +119,12 @@ def _metadata(name: str) -> property:
     ``__torch_function__``, which is left for function modes, that see the read there.  Nothing changes the value in place: an
     operator is given a filled plain alias (`_settled`).  A compiler follows the plain attributes; torch's own accessor would
     lead it back here."""
-    of_tensor = getattr(torch.Tensor, name).__get__
+    of_tensor, modes = getattr(torch.Tensor, name).__get__, torch._C._len_torch_function_stack
 
     def read(self):
         state = self._brt_state
-        if state is not None and not torch._C._len_torch_function_stack():
-            return getattr(state.buffer, name)
+        if state is not None and not modes():
+            return of_tensor(state.buffer)
         if torch.compiler.is_compiling():
             with torch._C.DisableTorchFunctionSubclass():
                 return getattr(self.detach(), name)
