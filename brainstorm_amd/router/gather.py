@@ -1,7 +1,7 @@
 """Gather router: per-path flows -> one flow (python/brt/router/gather.py:19-54)."""
 from typing import Any, Dict
 
-from brainstorm_amd.router.base import RouterBase, register_router
+from brainstorm_amd.router.base import Child, RouterBase, register_router
 from brainstorm_amd.router.fabric import make_fabric
 
 __all__ = ["GatherRouter"]
@@ -16,6 +16,8 @@ class GatherRouter(RouterBase):
     combine fabric.  With ``residual_flows`` the cells no path returned keep the
     residual value and the result is written into the residual tensor.
     """
+
+    fabric = Child()
 
     def __init__(self, fabric_type: str = "combine", fabric_kwargs: Dict[str, Any] = None):
         super().__init__()

@@ -9,7 +9,7 @@ from typing import Any, Dict
 import torch
 from torch.nn.modules.module import _has_any_global_hook
 
-from brainstorm_amd.router.base import RouterBase, register_router
+from brainstorm_amd.router.base import Child, RouterBase, register_router
 from brainstorm_amd.router.fabric import DispatchFabric, FusedDispatchFabric, make_fabric
 from brainstorm_amd.router.protocol import ProtocolBase, SwinMoEProtocol, make_protocol
 
@@ -36,6 +36,8 @@ class ScatterRouter(RouterBase):
     With ``dispatch_score=True`` the score tensor is routed as a second flow
     (2-d routing: path e receives ``score[:, e]`` of its cells).
     """
+
+    protocol, fabric = Child(), Child()
 
     def __init__(self, dispatch_score=False, protocol_type: str = "topk",
                  fabric_type: str = "dispatch", protocol_kwargs: Dict[str, Any] = None,
@@ -98,6 +100,7 @@ def _padding_of_a_route_made_with_the_mask(protocol, fabric):
 @register_router("swin_moe_scatter")
 class SwinMoEScatterRouter(RouterBase):
     ALLOWED_PROTOCOL_TYPES = ["swin_moe"]
+    protocol, fabric = Child(), Child()
 
     def __init__(self, protocol_type: str = "swin_moe", fabric_type: str = "dispatch",
                  protocol_kwargs: Dict[str, Any] = None, fabric_kwargs: Dict[str, Any] = None):

@@ -1,5 +1,8 @@
 """Routers call the protocol and the fabric that their attributes name at the call (no GPU needed)."""
+import copy
+
 import pytest
+import torch.nn as nn
 
 from brainstorm_amd.router import GatherRouter, ScatterRouter
 
@@ -34,3 +37,22 @@ def test_routers_call_children_that_a_subclass_names(swapped):
     else:
         assert scatter("flow", "score")[0] == "property"
     assert Gather()("flows")[0] == ("property", "flows", None, None)
+
+
+def test_children_of_routers_are_ordinary_modules():
+    gather = GatherRouter()
+    assert [name for name, _ in gather.named_children()] == ["fabric"] and list(gather.state_dict()) == []
+    other = copy.deepcopy(gather)
+    assert type(other.fabric) is type(gather.fabric) and other.fabric is not gather.fabric
+    gather.fabric = other.fabric
+    assert gather.fabric is other.fabric and gather._modules["fabric"] is other.fabric
+    gather._modules["fabric"] = nn.Identity()  # as passes that replace modules do
+    assert isinstance(gather.fabric, nn.Identity)
+    gather.fabric = None
+    assert gather.fabric is None
+    del gather.fabric
+    assert not hasattr(gather, "fabric")
+    with pytest.raises(AttributeError, match="'GatherRouter' object has no attribute 'fabric'"):
+        gather.fabric
+    gather.add_module("fabric", other.fabric)
+    assert gather.fabric is other.fabric
