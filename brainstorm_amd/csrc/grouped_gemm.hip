@@ -733,6 +733,13 @@ bool short_rounds_suit_few_rows(const GemmArgs& a) {
   return few < 0.95 * wide && weight_bytes < 1.2e9 && a.P <= 48 * used;
 }
 
+// The kernel of a shape and form (the reasons where it is launched).
+int kernel_of(const GemmArgs& a) {
+  if (wide_tiles_come_in_rounds(a)) return BRT_GEMM_PING_PONG;
+  if (skinny_gemm_applies(a) || short_rounds_suit_few_rows(a)) return BRT_GEMM_FEW_ROWS;
+  return BRT_GEMM_160_ROWS;
+}
+
 // Shapes whose fp32 rows the few-rows kernel rounds itself when asked to; where that is the faster way, skinny_gemm_takes_f32 says.
 bool runs_on_f32_rows(const GemmArgs& a) {
   return a.P <= 64l * std::min(a.E, a.P) && !wide_tiles_come_in_rounds(a) && few_rows_by_weight(a);
@@ -811,8 +818,9 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   // 279 and 276, 4 x 4000 rows 264 -> 528 (three column tiles for 528 columns) 22.5 and 22.8.
   // The rule is the same for gathered, scattered and fp32-output rows: a gathering 1024 -> 4096 GEMM with GELU over 32768
   // rows of 16 experts takes 437 us on the 160-row kernel and 336 us here.
-  if (wide_tiles_come_in_rounds(a)) return launch_pingpong_gemm(a, act, as_stream(stream));
-  if (skinny_gemm_applies(a) || short_rounds_suit_few_rows(a)) return launch_skinny_gemm(a, act, as_stream(stream));
+  const int kernel = kernel_of(a);
+  if (kernel == BRT_GEMM_PING_PONG) return launch_pingpong_gemm(a, act, as_stream(stream));
+  if (kernel == BRT_GEMM_FEW_ROWS) return launch_skinny_gemm(a, act, as_stream(stream));
   if (out_is_f32) {
     if (act == BRT_ACT_GELU) return launch_f32<BRT_ACT_GELU>(a, as_stream(stream));
     if (act == BRT_ACT_RELU) return launch_f32<BRT_ACT_RELU>(a, as_stream(stream));
@@ -830,6 +838,16 @@ extern "C" int brt_hip_grouped_gemm(const void* x, const void* const* weights,
                                     const void* const* biases, void* out, const int32_t* loads,
                                     int E, int P, int K, int N, int act, void* stream) {
   return grouped_gemm_impl(x, weights, biases, out, loads, nullptr, 0, E, P, 0, K, N, act, 0, 0, stream);
+}
+
+extern "C" int brt_hip_grouped_gemm_kernel(int E, int P, int K, int N, int accumulates) {
+  if (E <= 0 || P <= 0 || K <= 0 || N <= 0 || K % 8 != 0 || N % 8 != 0)
+    return fail(BRT_E_INVALID, "no kernel for E=%d P=%d K=%d N=%d", E, P, K, N);
+  GemmArgs a{};
+  const float gate = 0.0f;
+  a.E = E; a.P = P; a.K = K; a.N = N;
+  a.gates = accumulates ? &gate : nullptr;
+  return kernel_of(a);
 }
 
 extern "C" int brt_hip_grouped_gemm_timed(const void* x, const void* const* weights, const void* const* biases,

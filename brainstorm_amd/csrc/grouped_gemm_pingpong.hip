@@ -83,6 +83,18 @@ constexpr int kRound = kXcds * kCusPerXcd;  // tiles of a whole round
 // than ten rounds the CUs are no longer in step, and nothing is left to gain (98 blocks 2048 -> 8192, 12.25 rounds: 763 us cut, 756 not).
 constexpr int kFewRows = 128, kMostCut = 128, kMostRounds = 10;
 constexpr int kUnitCols = 64;
+struct ListEnd {
+  int moved, cut;  // row blocks of few rows put behind the list, tiles cut in all
+};
+template <typename OverTn>
+__host__ __device__ __forceinline__ ListEnd end_of_list(const GemmArgs& a, int tiles, int few, OverTn over_tn) {
+  const int tn = a.tiles_n, rest = tiles & (kRound - 1);
+  int moved = min(few, over_tn(rest + tn - 1));
+  int cut = max(moved * tn, rest);
+  if (cut > kMostCut || tiles > kMostRounds * kRound || tiles + 3 * cut > a.grid - (a.row_tags_out != nullptr ? 1 : 0)) cut = 0;
+  if (cut == 0) moved = 0;
+  return {moved, cut};
+}
 
 __device__ __forceinline__ i32x4 make_rsrc(const void* p, size_t bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(p);
@@ -194,11 +206,8 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     const int more = read_lane(read_two(base).incl_b, kWave - 1);
     many += more >> 8, few += more & 255;
   }
-  const int tiles = (many + few) * tn, rest = tiles & (kRound - 1);
-  int moved = min(few, over_tn(rest + tn - 1));
-  int cut = max(moved * tn, rest);  // tiles
-  if (cut > kMostCut || tiles > kMostRounds * kRound || tiles + 3 * cut > a.grid - (a.row_tags_out != nullptr ? 1 : 0)) cut = 0;
-  if (cut == 0) moved = 0;
+  const int tiles = (many + few) * tn;
+  const auto [moved, cut] = end_of_list(a, tiles, few, over_tn);
   const int listed = tiles - moved * tn, whole = tiles - cut, used = tiles + 3 * cut;
   if (t >= used) {
     // Surplus workgroups clear the tags of the rows no path owns, 256 of them a step.  The grid holds P / 256 + E row blocks
@@ -698,13 +707,16 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   epilogue(acc, first_row, mine, n0 + wn * kNT * 32);
 }
 
+// The sum over experts of ceil(M_e / 256) never exceeds P / 256 + E; whole rounds of XCD patches.
+long workgroups_of_list(int P, int E, int tiles_n) {
+  const long entries = (static_cast<long>(P + kBM - 1) / kBM + E) * tiles_n;
+  return (entries + kRound - 1) / kRound * kRound;
+}
+
 template <int ACT, bool ROUTED, bool OUTF32>
 int launch_pingpong(GemmArgs& a, hipStream_t st) {
   a.tiles_n = (a.N + kBN - 1) / kBN;
-  // the sum over experts of ceil(M_e / 256) never exceeds P / 256 + E; whole rounds of XCD patches
-  const long entries = (static_cast<long>(a.P + kBM - 1) / kBM + a.E) * a.tiles_n;
-  const long round = kXcds * kCusPerXcd;
-  const long grid = (entries + round - 1) / round * round;
+  const long grid = workgroups_of_list(a.P, a.E, a.tiles_n);
   // The timed form wants the clocks of a whole tile, also of a list that would be cut to the last: it is told of no workgroups for units.
   // (A test of a.clocks in the kernel itself cost 32768 rows of 16 experts 1024 -> 4096 -> 1024 7 us of 577.)
   a.grid = a.clocks != nullptr ? 0 : static_cast<int>(grid);
@@ -739,3 +751,23 @@ int launch_pingpong_gemm(GemmArgs& a, int act, hipStream_t st) {
 }
 
 }  // namespace brt
+
+extern "C" int brt_hip_grouped_gemm_tiles_cut(const int32_t* loads, int E, int P, int N, int row_tags) {
+  using namespace brt;
+  if (!loads || E <= 0 || P < 0 || N <= 0) return fail(BRT_E_INVALID, "bad arguments E=%d P=%d N=%d", E, P, N);
+  GemmArgs a{};
+  int some_tag = 0;
+  a.tiles_n = (N + kBN - 1) / kBN;
+  a.grid = static_cast<int>(workgroups_of_list(P, E, a.tiles_n));
+  a.row_tags_out = row_tags ? &some_tag : nullptr;
+  long blocks = 0;
+  int few = 0;
+  for (int e = 0; e < E; ++e) {
+    if (loads[e] < 0) return fail(BRT_E_INVALID, "expert %d has %d rows", e, loads[e]);
+    const int over = loads[e] % kBM;
+    blocks += (loads[e] + kBM - 1) / kBM;
+    few += over > 0 && over <= kFewRows;
+  }
+  if (blocks * a.tiles_n > 0x7fffffffll) return fail(BRT_E_INVALID, "%ld row blocks of %d tiles", blocks, a.tiles_n);
+  return end_of_list(a, static_cast<int>(blocks * a.tiles_n), few, [&](int n) { return n / a.tiles_n; }).cut;
+}

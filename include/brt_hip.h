@@ -495,6 +495,19 @@ int brt_hip_top1_route_to_capacity(const void* scores, int dtype, int32_t* mask,
 int brt_hip_copy_to_host(const int32_t* src, int32_t* host, int words, void* stream);
 
 /*
+ * Which kernel the grouped GEMM of these sizes runs on (no counterpart in the reference; for tests and measurements):
+ * one of the three below, or BRT_E_INVALID.  accumulates: the weighted accumulate form.
+ */
+enum { BRT_GEMM_PING_PONG = 1, BRT_GEMM_FEW_ROWS = 2, BRT_GEMM_160_ROWS = 3 };
+int brt_hip_grouped_gemm_kernel(int E, int P, int K, int N, int accumulates);
+
+/*
+ * ... and how many tiles of 256 x 256 at the end of its list the ping-pong kernel cuts into units of 64 columns, for loads
+ * [E] in host memory; row_tags: a routed form that writes row tags.
+ */
+int brt_hip_grouped_gemm_tiles_cut(const int32_t* loads, int E, int P, int N, int row_tags);
+
+/*
  * Measurement aid (no counterpart in the reference; bench.py reports what it reads beside the
  * compute-bound shapes): brt_hip_grouped_gemm through the 256 x 256 ping-pong kernel, whatever the
  * shape (BRT_E_UNSUPPORTED when that kernel does not take it: K must be a multiple of 64 and at

@@ -536,14 +536,11 @@ def test_ping_pong_tiles(loads, K, N):
 
 
 def _tiles_cut(loads, P, N, tags_out=False):
-    """Tiles of the end of the ping-pong kernel's list that are cut into units of 256 rows x 64 columns."""
-    tn = -(-N // 256)
-    few = sum(1 for m in loads if 0 < m % 256 <= 128)
-    tiles = sum(-(-m // 256) for m in loads) * tn
-    rest = tiles % 256
-    cut = max(min(few, -(-rest // tn)) * tn, rest)
-    grid = -(-(-(-P // 256) + len(loads)) * tn // 256) * 256
-    return 0 if cut > 128 or tiles > 2560 or tiles + 3 * cut > grid - int(tags_out) else cut
+    """Tiles of the end of the ping-pong kernel's list that are cut into units of 256 rows x 64 columns, as the kernel's own rule has it."""
+    from brainstorm_amd import _lib
+
+    host_loads = torch.tensor(loads, dtype=torch.int32)
+    return _lib.lib().brt_hip_grouped_gemm_tiles_cut(host_loads.data_ptr(), len(loads), P, N, int(tags_out))
 
 
 @pytest.mark.parametrize("loads,K,N,cut", [
@@ -730,34 +727,24 @@ def test_split_k_tiles(loads, K, N):
 
 
 def _kernel_for(P, E, K, N):
-    """Which kernel the host takes for these sizes (all but the weighted accumulate form), on 256 CUs."""
-    used = min(E, P)
-    big = ((P + 255) // 256 + (E + 1) // 2) * -(-N // 256)
-    if K >= 128 and P > E * 160 and big >= 192:
-        def rounds(waves):  # of the 160-row kernel's tiles; two workgroups of two wavefronts fit a CU
-            n = max((P + 159) // 160, used) * -(-N // (64 * waves))
-            return -(-n // 512) * 2 if waves == 2 else -(-n // 256)
+    """The kernel that the library takes for these sizes (all but the weighted accumulate form)."""
+    from brainstorm_amd import _lib
 
-        cost, waves = min((rounds(w) * (160 + 64 * w), -w) for w in (2, 3, 4))
-        if big <= 320 or 5 * big >= 8 * 256 or (waves != -2 and (big >= 384 or cost > 832)):
-            return "ping-pong"
-    tiles = max((P + 159) // 160, used) * -(-N // 256)
-    weight = 2.0 * used * N * K
-    if P > 64 * used:
-        few = used <= 32 if tiles <= 96 else P <= 128 * used and tiles <= 160 and used < 8 and weight < 1.5e8
-    elif tiles <= 72:
-        few = True
-    elif P <= 28 * used:
-        few = weight < 3e8 or (weight < 1e9 and (tiles <= 128 or K % 2048 == 0 or 2 * P <= 3 * used))
-        few = few or (K % 64 != 0 and P <= (20 if K < 4096 else 12) * used)
-    else:
-        few = tiles <= 160 and weight < 1.5e8
-        if N >= K >= 256:  # part-filled rounds of the 160-row tiles
-            share = 128 * used * -(-N // 64) / 256 / min(-(-used * -(-N // (64 * w)) // (512 if w == 2 else 256)) * (2 if w == 2 else 1)
-                                                         * (160 + 64 * w) for w in (2, 3, 4))
-            few = few or ((share < (1.1 if used > 8 else 1.0) if weight < 2.5e8 else share < 0.95 and weight < 1.2e9 and P <= 48 * used)
-                          if N >= 2 * K else weight < 4e8 and share < 0.9)
-    return "few rows" if few else "160 rows"
+    return {1: "ping-pong", 2: "few rows", 3: "160 rows"}[_lib.lib().brt_hip_grouped_gemm_kernel(E, P, K, N, 0)]
+
+
+def test_kernel_of_the_accumulate_form_and_of_bad_sizes():
+    from brainstorm_amd import _lib
+
+    L = _lib.lib()
+    assert L.brt_hip_grouped_gemm_kernel(8, 8192, 512, 2048, 0) == 1 and L.brt_hip_grouped_gemm_kernel(8, 8192, 512, 2048, 1) == 3
+    assert L.brt_hip_grouped_gemm_kernel(8, 24, 768, 3072, 1) == 2
+    for sizes in ((0, 1, 8, 8), (1, 0, 8, 8), (1, 1, 12, 8), (1, 1, 8, 4)):
+        assert L.brt_hip_grouped_gemm_kernel(*sizes, 0) == -1  # BRT_E_INVALID
+    assert L.brt_hip_grouped_gemm_tiles_cut(None, 1, 1, 8, 0) == -1
+    loads = torch.tensor([1024] * 4, dtype=torch.int32)
+    assert L.brt_hip_grouped_gemm_tiles_cut(loads.data_ptr(), 4, 4096, 1024, 0) == 64  # 256 workgroups, all of them units
+    assert L.brt_hip_grouped_gemm_tiles_cut(loads.data_ptr(), 4, 4096, 1024, 1) == 0   # one is needed to clear row tags
 
 
 @pytest.mark.parametrize("loads,K,N,bounds", [
