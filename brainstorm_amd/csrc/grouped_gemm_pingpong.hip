@@ -77,11 +77,15 @@ constexpr int kHead = 4;                              // MFMAs of a C phase issu
 constexpr uint32_t kOutOfRange = 0x80000000u;         // buffer offset past any extent: reads as zero
 constexpr int kXcds = 8, kCusPerXcd = 32, kPatchRows = 4;
 constexpr int kRound = kXcds * kCusPerXcd;  // tiles of a whole round
-// The end of the list that is cut into units (see the kernel).  A unit of 256 rows takes 0.4 to 0.5 of a tile's time (4 x 1024 rows
-// 4096 -> 1024, 256 units: 40 us against 102 us for the 64 tiles they are made of), one of up to 128 rows a third (38 us and 73), so two
-// rounds of them, 128 tiles, are what a round of whole tiles costs: 16 x 256 rows 4096 -> 2048 105 us against 108.  In a list of more
-// than ten rounds the CUs are no longer in step, and nothing is left to gain (98 blocks 2048 -> 8192, 12.25 rounds: 763 us cut, 756 not).
-constexpr int kFewRows = 128, kMostCut = 128, kMostRounds = 10;
+// The end of the list that is cut into units (see the kernel).  It takes the CUs one round of units up to 64 tiles and two up to 128,
+// against a round in which the tiles leave most CUs idle.  A unit of 256 rows takes 0.4 to 0.5 of a tile's time (4 x 1024 rows
+// 4096 -> 1024, 256 units: 40 us against 102 us for the 64 tiles they are made of), one of up to 128 rows half of what its block
+// takes as a tile (38 us and 73).  Of lists of one to two rounds (us, not cut and cut): 65 tiles 0.79 to 0.96 of the time, 80 tiles 0.93
+// to 0.95 (4 x 1704 rows 1504 -> 3008 80 and 75), 92 to 104 tiles 0.96 to 1.02, 108 and more 1.00 to 1.08 (8 x 785 skewed rows
+// 3592 -> 3272 191 and 205, 64 x 393 rows 2288 -> 736 127 and 135); where all of them are blocks of few rows 105 tiles 0.83 to 0.92
+// (60 x 265 rows 4152 -> 592) and 116 to 126 0.89 to 0.93.  In a list of more than ten rounds the CUs are no longer in step, and nothing
+// is left to gain (98 blocks 2048 -> 8192, 12.25 rounds: 763 us cut, 756 not).
+constexpr int kFewRows = 128, kMostCut = 104, kMostCutOfFewRows = 128, kMostRounds = 10;
 constexpr int kUnitCols = 64;
 struct ListEnd {
   int moved, cut;  // row blocks of few rows put behind the list, tiles cut in all
@@ -91,7 +95,8 @@ __host__ __device__ __forceinline__ ListEnd end_of_list(const GemmArgs& a, int t
   const int tn = a.tiles_n, rest = tiles & (kRound - 1);
   int moved = min(few, over_tn(rest + tn - 1));
   int cut = max(moved * tn, rest);
-  if (cut > kMostCut || tiles > kMostRounds * kRound || tiles + 3 * cut > a.grid - (a.row_tags_out != nullptr ? 1 : 0)) cut = 0;
+  const int most = moved * tn >= rest ? kMostCutOfFewRows : kMostCut;
+  if (cut > most || tiles > kMostRounds * kRound || tiles + 3 * cut > a.grid - (a.row_tags_out != nullptr ? 1 : 0)) cut = 0;
   if (cut == 0) moved = 0;
   return {moved, cut};
 }

@@ -562,6 +562,21 @@ def test_end_of_the_list_of_ping_pong_tiles_in_units(loads, K, N, cut):
     run(loads, K, N, act="relu", bias=True, seed=2, slack=300)
 
 
+# row blocks of a round (64 of four tiles) and over, whole ones and ones of few rows; experts without rows give the grid its room
+@pytest.mark.parametrize("whole,few,cut", [
+    (64 + 26, 0, 104),
+    (64 + 27, 0, 0),
+    (64 + 18, 8, 104),       # whole blocks behind those of few rows
+    (64 + 19, 8, 0),
+    (62, 32, 120),           # blocks of few rows alone: up to 128
+    (64, 32, 128),
+    (65, 32, 0),
+])
+def test_most_of_the_end_of_the_list_that_is_cut(whole, few, cut):
+    loads = [whole * 256 - 3 * 256] + [100] * few + [512, 256] + [0] * 80
+    assert _tiles_cut(loads, sum(loads), 776) == cut
+
+
 # 0.3 GB of weights and more in rows that are no whole 128-byte lines: few rows, and a row too many for them
 @pytest.mark.parametrize("loads,K,N,kernel", [
     ([20] * 59 + [0, 40], 1592, 1608, "few rows"),
