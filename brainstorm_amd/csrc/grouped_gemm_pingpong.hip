@@ -83,9 +83,9 @@ constexpr int kRound = kXcds * kCusPerXcd;  // tiles of a whole round
 // takes as a tile (38 us and 73).  Of lists of one to two rounds (us, not cut and cut): 65 tiles 0.79 to 0.96 of the time, 80 tiles 0.93
 // to 0.95 (4 x 1704 rows 1504 -> 3008 80 and 75), 92 to 104 tiles 0.96 to 1.02, 108 and more 1.00 to 1.08 (8 x 785 skewed rows
 // 3592 -> 3272 191 and 205, 64 x 393 rows 2288 -> 736 127 and 135); where all of them are blocks of few rows 105 tiles 0.83 to 0.92
-// (60 x 265 rows 4152 -> 592) and 116 to 126 0.89 to 0.93.  In a list of more than ten rounds the CUs are no longer in step, and nothing
+// (60 x 265 rows 4152 -> 592) and 116 0.89, 128 of 128 rows 1.07 (32 x 640 rows 6024 -> 928 311 and 333).  In a list of more than ten rounds the CUs are no longer in step, and nothing
 // is left to gain (98 blocks 2048 -> 8192, 12.25 rounds: 763 us cut, 756 not).
-constexpr int kFewRows = 128, kMostCut = 104, kMostCutOfFewRows = 128, kMostRounds = 10;
+constexpr int kFewRows = 128, kMostCut = 104, kMostCutOfFewRows = 116, kMostRounds = 10;
 constexpr int kUnitCols = 64;
 struct ListEnd {
   int moved, cut;  // row blocks of few rows put behind the list, tiles cut in all
@@ -712,9 +712,21 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   epilogue(acc, first_row, mine, n0 + wn * kNT * 32);
 }
 
-// The sum over experts of ceil(M_e / 256) never exceeds P / 256 + E; whole rounds of XCD patches.
+// The sum over experts of ceil(M_e / 256) never exceeds P / 256 + E; whole rounds of XCD patches.  What the loads leave of it is room for
+// units, and of experts with a little over whole blocks each nothing is left, so there are as many workgroups as the end of a list of
+// even loads needs (us, without them and with them: 60 x 274 rows 7608 -> 608 378 and 328, 16 x 296 rows 4032 -> 2312 151 and 134, 32 x 294
+// rows 7448 -> 1096 347 and 279).  Room for the longest end of any list costs others more than it gives: 64 x 400 rows 768 -> 3072
+// 141 -> 147 us, 16 x 2048 rows 4096 -> 1024 213 -> 218.
 long workgroups_of_list(int P, int E, int tiles_n) {
-  const long entries = (static_cast<long>(P + kBM - 1) / kBM + E) * tiles_n;
+  const int used = std::min(E, P), rows = used > 0 ? (P + used - 1) / used : 0, over = rows % kBM;
+  const long even = static_cast<long>((rows + kBM - 1) / kBM) * used * tiles_n;
+  GemmArgs any{};
+  any.tiles_n = tiles_n;
+  any.grid = 0x7fffffff;
+  long entries = (static_cast<long>(P + kBM - 1) / kBM + E) * tiles_n;
+  if (even <= kMostRounds * kRound)
+    entries = std::max(entries, even + 3 * end_of_list(any, static_cast<int>(even), over > 0 && over <= kFewRows ? used : 0,
+                                                       [=](int n) { return n / tiles_n; }).cut);
   return (entries + kRound - 1) / kRound * kRound;
 }
 

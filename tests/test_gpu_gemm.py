@@ -553,6 +553,9 @@ def _tiles_cut(loads, P, N, tags_out=False):
     ([1800, 900, 0, 2200, 260], 576, 3328, 43),            # and one more
     ([5000, 3328 + 40, 0, 300], 1088, 2048, 32),           # seventeen K-steps: every ring goes round
     ([0] * 130 + [3] * 100 + [8000, 9000, 24000, 1], 128, 512, 14),  # more than 128 experts
+    ([274] * 60, 192, 608, 105),                           # even loads a little over a block: units of 18 rows
+    ([302] * 8, 320, 4904, 80),                            # ... of 46
+    ([350] * 16, 136, 2312, 70),                           # ... of 94
 ])
 def test_end_of_the_list_of_ping_pong_tiles_in_units(loads, K, N, cut):
     P, E = sum(loads), len(loads)
@@ -568,9 +571,8 @@ def test_end_of_the_list_of_ping_pong_tiles_in_units(loads, K, N, cut):
     (64 + 27, 0, 0),
     (64 + 18, 8, 104),       # whole blocks behind those of few rows
     (64 + 19, 8, 0),
-    (62, 32, 120),           # blocks of few rows alone: up to 128
-    (64, 32, 128),
-    (65, 32, 0),
+    (61, 32, 116),           # blocks of few rows alone: up to 116
+    (62, 32, 0),
 ])
 def test_most_of_the_end_of_the_list_that_is_cut(whole, few, cut):
     loads = [whole * 256 - 3 * 256] + [100] * few + [512, 256] + [0] * 80
