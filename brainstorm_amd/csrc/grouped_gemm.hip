@@ -816,8 +816,14 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   // Widths that are no multiple of a K-step of 64 are under the same rule: 8 x 1024 rows 1592 -> 6368 278 us there, 187 here,
   // 6368 -> 1592 218 and 176, 4 x 3000 rows 4384 -> 1096 155 and 120, 64 x 400 rows 360 -> 1440 105 and 63, 12 x 700 rows 7200 -> 1800
   // 279 and 276, 4 x 4000 rows 264 -> 528 (three column tiles for 528 columns) 22.5 and 22.8.
+  // Even loads a little over one 256-row block are the weak spot: with 257 to 320 rows the two are level in the mean, as long as the
+  // end of the list is cut (16 x 296 rows 4032 -> 2312 138 us there, 134 here), and those win by up to a quarter where the last blocks fill
+  // half a round or a whole one (16 x 266 rows 3416 -> 2976 151 and 186); of the same averages ragged loads are 0.9 and skewed ones 0.77 of
+  // their time here, and the host does not know which it has.
   // The rule is the same for gathered, scattered and fp32-output rows: a gathering 1024 -> 4096 GEMM with GELU over 32768
-  // rows of 16 experts takes 437 us on the 160-row kernel and 336 us here.
+  // rows of 16 experts takes 437 us on the 160-row kernel and 336 us here; fp32 output, 420 drawn shapes of one to two rounds, 0.81 of that
+  // kernel's time in the mean, 18 more than 3 % over it (64 x 270 rows 7504 -> 696 1.22).  That kernel's fp32 tiles are always four
+  // wavefronts wide; of 240 drawn shapes of 1.25 to 1.6 rounds their own cost selects the same 90 as the width for bf16 output.
   const int kernel = kernel_of(a);
   if (kernel == BRT_GEMM_PING_PONG) return launch_pingpong_gemm(a, act, as_stream(stream));
   if (kernel == BRT_GEMM_FEW_ROWS) return launch_skinny_gemm(a, act, as_stream(stream));

@@ -757,11 +757,12 @@ int launch_pingpong_form(GemmArgs& a, hipStream_t st) {
 }
 
 int launch_pingpong_gemm(GemmArgs& a, int act, hipStream_t st) {
-  // bf16 rows that are no whole 64-byte pieces are written with ordinary stores whatever their size: the pieces of neighbouring
+  // Rows that are no whole 64-byte pieces are written with ordinary stores whatever their size: the pieces of neighbouring
   // wavefronts that lie in one of them meet in the L2 (us, streamed and not: 16 x 500 rows 936 -> 1872 43.0 and 38.2, 16 x 2000 rows
   // 1000 -> 2000 163 and 149, 32 x 1000 rows 520 -> 1040 81 and 74, 16 x 2048 rows 1024 -> 4104 319 and 313; whole pieces, 4 x 8000
-  // rows 1992 -> 7968, 941 and 1020).  On the 160-row kernel it is level or loses (12 x 140 rows 1800 -> 7208 140 and 143).
-  if (a.out_f32 == nullptr && a.N % 32 != 0) a.plain_out = 1;
+  // rows 1992 -> 7968, 941 and 1020; fp32 rows 16 x 1732 rows 640 -> 984 74 and 53, 32 x 298 rows 272 -> 2088 63 and 43, 32 x 1000 rows
+  // 1024 -> 4104 367 and 320).  On the 160-row kernel it is level or loses (12 x 140 rows 1800 -> 7208 140 and 143).
+  if (a.N % (a.out_f32 != nullptr ? 16 : 32) != 0) a.plain_out = 1;
   if (act == BRT_ACT_GELU) return launch_pingpong_form<BRT_ACT_GELU>(a, st);
   if (act == BRT_ACT_RELU) return launch_pingpong_form<BRT_ACT_RELU>(a, st);
   return launch_pingpong_form<BRT_ACT_NONE>(a, st);
