@@ -719,9 +719,15 @@ bool wide_tiles_come_in_rounds(const GemmArgs& a) {
 // 29 to 64 rows per expert, beyond what skinny_gemm_applies takes: where the 160-row tiles leave a large part of their last round over
 // the CUs empty (or are fewer than the CUs), 64 x 64 tiles are faster though every block of rows reads the weights again.  Both sides by
 // the operand rows that the busiest, respectively the average, CU streams.  The line was drawn on 285 shapes of uniform loads that the
-// 160-row kernel had before, and tried on 130 others, two thirds of them with ragged and skewed loads: 0.71 of its time in the mean, the worst 2 % over it.  us, 160-row and few-rows:
-// 64 x 43 rows 256 -> 5312 72 and 39, 12 x 39 rows 1344 -> 7168 73 and 39, 60 x 46 rows 384 -> 3136 59 and 30, 4 x 53 rows 3008 -> 6464
-// 89 and 28.  Not taken: contracting shapes (64 x 60 rows 2240 -> 768 42 and 54, 64 x 33 rows 2880 -> 832 53 and 66), large weights
+// 160-row kernel had before.  us, 160-row and few-rows: 64 x 43 rows 256 -> 5312 72 and 39, 12 x 39 rows 1344 -> 7168 73 and 39,
+// 60 x 46 rows 384 -> 3136 59 and 30, 4 x 53 rows 3008 -> 6464 89 and 28.  Of 300 other shapes that it takes, 170 of them with skewed loads,
+// the mean is 0.79 of the 160-row kernel's time, 27 are more than 3 % over it: even loads of 8 to 32 experts where that kernel is through in
+// one round (8 x 62 rows 2560 -> 4480 42 and 50, 16 x 59 rows 1792 -> 3584 1.19), whose skewed loads win (0.70 and 0.83 for these two).
+// The bounds on the weights come from the 256 MB last-level cache: up to 0.25 GB the second block of an expert's rows finds them there,
+// beyond it reads them from memory again, so 48 rows are the limit, and with 1.2 GB the wide tiles stream them as fast as memory
+// gives (30 drawn shapes with N >= 2 K behind these lines: even loads 0.85 to 1.18 of the 160-row kernel's time up to 1.2 GB, 1.02 to 1.28
+// above, skewed ones 0.78 in the mean).  With N < 2 K there are fewer column tiles for the same weights, and the line lies lower.
+// Not taken: contracting shapes (64 x 60 rows 2240 -> 768 42 and 54, 64 x 33 rows 2880 -> 832 53 and 66), large weights
 // of skewed experts (8 x 58 rows 2496 -> 9984 87 and 95), more rows (32 x 65 rows 1376 -> 5504 112 and 157); a K below 256 was not timed.
 bool short_rounds_suit_few_rows(const GemmArgs& a) {
   const long used = std::min(a.E, a.P);

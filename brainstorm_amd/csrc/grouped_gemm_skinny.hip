@@ -446,7 +446,11 @@ bool few_rows_by_weight(const GemmArgs& a) {
 // Besides, with any weight, few rows whose weight rows are no whole 128-byte lines: this kernel keeps the memory's rate there
 // (64 x 4 rows 1432 -> 4680 146 us), the wide tiles, which walk the lines of 256 columns at a time, do not (181).  68 drawn shapes of
 // 0.3 to 4.2 GB, 1 to 20 rows per expert: 0.85 of the wide tiles' time in the mean; with more rows, or more than 12 and a long K, the
-// two are level or those win (64 x 15 rows 4848 -> 2032 241 us here, 234 there; 64 x 31 rows 5152 -> 680 100 and 93).
+// two are level or those win (64 x 15 rows 4848 -> 2032 241 us here, 234 there; 64 x 31 rows 5152 -> 680 100 and 93).  An expert with many of the
+// rows reads its weights again for every 32 of them, and still skewed loads gain more than even ones, as the wide tiles then wait for
+// that expert's: of 69 skewed loads of 33 drawn shapes, 1 to 20 rows on average and up to 1194 with one expert, 0.69 of their time in the mean and 0.94
+// at worst (64 x 19 rows 2400 -> 1248 85 us and 94 with 368 of them on one expert, 32 x 16 rows 2040 -> 4992 156 and 182 with 492), of 171 even ones
+// 0.91, the worst 1.07 (32 x 19 rows 3976 -> 6136 329 and 308).
 bool skinny_gemm_applies(const GemmArgs& a) {
   const long used = std::min(a.E, a.P);
   return few_rows_by_weight(a) || (a.K % kBK != 0 && a.P <= (a.K < 4096 ? 20 : 12) * used);
