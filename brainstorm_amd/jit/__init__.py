@@ -199,7 +199,8 @@ class GroupedLinearKernel:
         return (cells.dim() == 2 and cells.shape[1] == self.in_features and out.dim() == 2
                 and out.shape[0] == state.buffer.shape[0] and out.is_contiguous()
                 and cells.dtype in (torch.bfloat16, torch.float32)
-                and out.dtype in (torch.bfloat16, torch.float32))
+                # rows that the row-entry vector names are written in bf16 only
+                and (out.dtype == torch.bfloat16 or (out.dtype == torch.float32 and not isinstance(state.route, c_router.CompactRoute))))
 
 
 def make_jit_kernel(modules, sample_inputs=None, method: str = "forward", opt_level=None,

@@ -694,6 +694,23 @@ def test_compact_route_through_the_router_objects_top2(brt_mod, weighted):
         assert torch.equal(results[0], other)
 
 
+@pytest.mark.parametrize("T,top_k", [(24, 1), (2048, 1), (1536, 2)])  # few rows per expert, which are rounded by the GEMM, and more
+def test_deferred_compact_route_of_fp32_cells(brt_mod, T, top_k):
+    """fp32 cells and outputs: the rows are dispatched after all, to the bits of the other forms."""
+    E, d, dff = 8, 128, 256
+    g = torch.Generator().manual_seed(55)
+    hidden = torch.randn(T, d, generator=g).cuda()
+    score = torch.softmax(torch.randn(T, E, generator=g), dim=1).cuda()
+    caps = {"supported_capacities": [T // 4]}
+    results = []
+    for form in ({}, {"compact_route": True}, {"compact_route": True, "defer_dispatch": True}):
+        layer = _moe_layer(brt_mod, E, d, dff, top_k, torch.float32, 56, dict(caps, **form), weighted=top_k > 1)
+        results.append(layer(hidden.clone(), score))
+    assert not torch.equal(results[0], hidden)
+    for other in results[1:]:
+        assert torch.equal(results[0], other)
+
+
 def test_compact_route_keeps_the_reference_format_for_whoever_reads_it(brt_mod):
     """The tag stack of a compact route carries the dense seat matrix of the reference, generated
     only when something reads it; the loads are the reference's; a fabric that does not take the
