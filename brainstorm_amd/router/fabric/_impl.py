@@ -440,8 +440,11 @@ class FusedDispatchFabric(DispatchFabric):
             return False
         flow = in_flows[0]
         with torch._C.DisableTorchFunctionSubclass():
-            return (self.route_logics[0] == "1d" and flow.dim() >= 2 and flow.shape[0] > 0 and flow.is_cuda
-                    and flow.dtype in (torch.float32, torch.float16, torch.bfloat16))
+            shape = flow.shape
+            return (self.route_logics[0] == "1d" and len(shape) >= 2 and shape[0] > 0 and flow.is_cuda
+                    and flow.dtype in (torch.float32, torch.float16, torch.bfloat16)
+                    # rows are moved in whole 16-byte units
+                    and flow.nbytes % (16 * shape[0]) == 0 and (flow.data_ptr() % 16 == 0 or not flow.is_contiguous()))
 
     def _forward_compact(self, in_flows, decision, score):
         """The route from path ids: ``route_by_path`` lays it out (loads by the capacity rules of

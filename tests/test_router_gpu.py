@@ -711,6 +711,28 @@ def test_deferred_compact_route_of_fp32_cells(brt_mod, T, top_k):
         assert torch.equal(results[0], other)
 
 
+@pytest.mark.parametrize("kwargs", [{"compact_route": True}, {"compact_route": True, "defer_dispatch": True}])
+@pytest.mark.parametrize("d,dtype,offset,top_k", [(19, torch.bfloat16, 0, 1), (21, torch.float32, 0, 2), (12, torch.float16, 0, 2),
+                                                  (16, torch.bfloat16, 1, 1), (8, torch.bfloat16, 0, 2)])
+def test_compact_route_of_rows_that_are_no_16_byte_units(brt_mod, d, dtype, offset, top_k, kwargs):
+    """Rows of other lengths and unaligned ones take the mask, to the same rows and result; the last is a width that the compact form moves."""
+    brt, _, ScatterRouter, GatherRouter = brt_mod
+    T, E = 56, 8
+    g = torch.Generator().manual_seed(57)
+    x = torch.randn(T * d + offset, generator=g).to(dtype).cuda()[offset:].view(T, d)
+    score = torch.softmax(torch.randn(T, E, generator=g), dim=1).cuda()
+    results = []
+    for form in ({}, kwargs):
+        scatter = ScatterRouter(protocol_type="topk", protocol_kwargs={"top_k": top_k}, fabric_type="fused_dispatch",
+                                fabric_kwargs=form).cuda()
+        gather = GatherRouter(fabric_type="fused_combine", fabric_kwargs={"transform": top_k > 1}).cuda()
+        routed = scatter(brt.Annotator([0])(x), score)
+        kept = int(routed.load.sum())
+        results.append((brt.to_torch_tensor(routed)[:kept].clone(), brt.to_torch_tensor(gather(routed, None, score))))
+    for want, got in zip(*results):
+        assert want.shape == got.shape and torch.equal(want, got)
+
+
 def test_compact_route_keeps_the_reference_format_for_whoever_reads_it(brt_mod):
     """The tag stack of a compact route carries the dense seat matrix of the reference, generated
     only when something reads it; the loads are the reference's; a fabric that does not take the
