@@ -718,14 +718,14 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
 // rows 7448 -> 1096 347 and 279).  Room for the longest end of any list costs others more than it gives: 64 x 400 rows 768 -> 3072
 // 141 -> 147 us, 16 x 2048 rows 4096 -> 1024 213 -> 218.
 long workgroups_of_list(int P, int E, int tiles_n) {
-  const int used = std::min(E, P), rows = used > 0 ? (P + used - 1) / used : 0, over = rows % kBM;
-  const long even = static_cast<long>((rows + kBM - 1) / kBM) * used * tiles_n;
+  const long used = std::min(E, P), rows = used > 0 ? (P + used - 1) / used : 0, over = rows % kBM;
+  const long even = (rows + kBM - 1) / kBM * used * tiles_n;
   GemmArgs any{};
   any.tiles_n = tiles_n;
   any.grid = 0x7fffffff;
   long entries = (static_cast<long>(P + kBM - 1) / kBM + E) * tiles_n;
   if (even <= kMostRounds * kRound)
-    entries = std::max(entries, even + 3 * end_of_list(any, static_cast<int>(even), over > 0 && over <= kFewRows ? used : 0,
+    entries = std::max(entries, even + 3 * end_of_list(any, static_cast<int>(even), over > 0 && over <= kFewRows ? static_cast<int>(used) : 0,
                                                        [=](int n) { return n / tiles_n; }).cut);
   return (entries + kRound - 1) / kRound * kRound;
 }
