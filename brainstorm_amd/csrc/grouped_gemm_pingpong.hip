@@ -6,10 +6,10 @@
 // Same contract as grouped_gemm.hip (out[rows of e] = act(x[rows of e] @ W_e^T + b_e), one launch,
 // loads read on the device; reference: src/jit/compiler.cu:151-246).  What differs:
 //
-//   - A workgroup is 8 wavefronts, two per SIMD, each owning 128 x 64 outputs (8 accumulator tiles
-//     of v_mfma_f32_32x32x16_bf16 = 128 registers, and the 24 fragments of a whole K-step of 64 in
+//   - A workgroup is 8 wavefronts, two per SIMD, each owning 128 x 64 outputs (32 accumulator tiles
+//     of v_mfma_f32_16x16x32_bf16 = 128 registers, and the 24 fragments of a whole K-step of 64 in
 //     96 more).  The wavefronts of a SIMD belong to two groups that run half a K-step apart: while
-//     one group issues its 32 MFMAs (C phase), the other reads its fragments from LDS and requests
+//     one group issues its 64 MFMAs (C phase), the other reads its fragments from LDS and requests
 //     operands from memory (M phase); a workgroup barrier separates the phases.  The matrix pipe
 //     of a SIMD therefore always has a wavefront that does nothing but multiply, and the memory
 //     instructions of the other one never stand between two MFMAs.
@@ -24,9 +24,14 @@
 //     rows one phase earlier), once its own weight fragments are in registers.  Every request has
 //     three to four phases to land, and each wavefront issues its 8 loads of a K-step in its M
 //     phase, between fragment reads.  A K-step is 2 x 1024 clocks of MFMA per SIMD and measures
-//     about 2100 (s_memtime at the phase boundaries: M phase 820-865, C phase's MFMAs back to back),
-//     at a shader clock of 1.3-1.6 GHz under this load (boxes differ): time, not clocks, is what is left to win,
-//     i.e. less energy per K-step.  Its 64 KB of loads alone take 0.62 us per CU when the rows are up to 8 KB apart and 1.08 us when they
+//     about 2150, at the 1.5 to 1.7 GHz that the part sustains with them: it is the package's power that sets the time of a K-step
+//     (1.35 to 1.45 us; with fewer clocks the clock rate falls), so what counts is its energy.  That of the 16 x 16 x 32 instruction is
+//     lower than that of v_mfma_f32_32x32x16_bf16, which reads and writes every accumulator twice as often; both sum the products of
+//     an output element to the same bits.  us, 32 x 32 x 16 and this: 8 x 4096 rows 2048 -> 8192 + GELU 906 and 876, 8192 -> 2048 776 and
+//     752, 16 x 2048 rows 1024 -> 4096 + GELU 271 and 262, 4096 -> 1024 210 and 204, 64 x 400 rows 768 -> 3072 + GELU 161 and 155.
+//     Four wavefronts of 128 x 128 outputs, the accumulators in the AGPRs (128 KB of fragment reads a K-step instead of 192, 2400 clocks at 1.75
+//     GHz), need as much without an activation and 4 to 15 % more with GELU: nothing runs beside a wavefront's epilogue there.
+//     The 64 KB of loads of a K-step alone take 0.62 us per CU when the rows are up to 8 KB apart and 1.08 us when they
 //     are 16 KB apart (K = 8192: the 512 rows of a tile pair then lie in 128 regions of 64 KB,
 //     more than a CU's address translation holds), so the load stream has to be fed in every
 //     phase and must not wait for anything.
@@ -41,7 +46,7 @@
 //   - What the list of tiles holds beyond whole rounds over the CUs would keep a few of them busy for as long as a whole round, and the
 //     experts' last row blocks, which hold few rows, for more than half as long (the weights of 256 columns come into one CU at
 //     40 GB/s).  Where that is at most half a round it is cut into units of 256 rows x 64 columns: each wavefront loads its share of a
-//     K-step and multiplies 32 rows (or 32 x 32 blocks of fewer rows) of a ring of four to eight K-steps, one barrier per K-step, the loads
+//     K-step and multiplies 32 rows (or 32 x 32 outputs of fewer rows) of a ring of four to eight K-steps, one barrier per K-step, the loads
 //     between the MFMAs (in front of them a K-step took 0.65 us instead of 0.53).  Bound by the fills of LDS, 40 KB a
 //     K-step at 64 bytes a clock.  32768 rows of 16 experts 4096 -> 1024 268 -> 229 us, 32 x 1000 rows 512 -> 1024 61 -> 50.
 //   - The epilogue sends the tile out 32 rows at a time through each wavefront's own corner of
@@ -59,21 +64,20 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef const bf16x4 __attribute__((address_space(1)))* global_bf16x4;
 typedef const __bf16 __attribute__((address_space(1)))* global_bf16;
 
 constexpr int kWaves = 8;
-constexpr int kMT = 4, kNT = 2;                       // 32 x 32 tiles per wavefront: 128 x 64
+constexpr int kMT = 8, kNT = 4;                       // 16 x 16 tiles per wavefront: 128 x 64
 constexpr int kBM = 256, kBN = 256, kBK = 64;
 constexpr int kRowB = kBK * 2;                        // bytes of one tile row in one stage: one cache line
 constexpr int kTileB = kBM * kRowB;                   // one operand of one K-step: 32 KB
 constexpr int kAStages = 3, kBStages = 2;
 constexpr int kBBase = kAStages * kTileB;             // the weight ring follows the activation ring
 constexpr int kLdsBytes = (kAStages + kBStages) * kTileB;  // 163840: all of a CU's LDS
-constexpr int kSub = kBK / 16;                        // MFMA k-steps per stage
-constexpr int kHead = 4;                              // MFMAs of a C phase issued ahead of the barrier
+constexpr int kSub = kBK / 32;                        // MFMA k-steps per stage
+constexpr int kHead = 8;                              // MFMAs of a C phase issued ahead of the barrier
 constexpr uint32_t kOutOfRange = 0x80000000u;         // buffer offset past any extent: reads as zero
 constexpr int kXcds = 8, kCusPerXcd = 32, kPatchRows = 4;
 constexpr int kRound = kXcds * kCusPerXcd;  // tiles of a whole round
@@ -122,6 +126,17 @@ __device__ __forceinline__ void load_to_lds(const i32x4& rsrc, uint32_t voffset,
                : "memory");
 }
 
+// acc += w x, 16 x 16 x 32.  In place: as a builtin the instruction gets other registers for its result, and accumulators are moved.
+// The compiler does not know its wait states then: mfma_wait_states() stands before anything else reads an accumulator.
+__device__ __forceinline__ void multiply_add(f32x4& acc, const bf16x8& w, const bf16x8& x) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(w), "v"(x));
+}
+__device__ __forceinline__ void mfma_wait_states() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 15" : : : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // what is the same in all lanes, in scalar registers (the compiler cannot always tell)
 __device__ __forceinline__ i32x4 in_scalars(i32x4 r) {
 #pragma unroll
@@ -130,7 +145,8 @@ __device__ __forceinline__ i32x4 in_scalars(i32x4 r) {
 }
 
 __device__ __forceinline__ void stream_out(const u32x4& v, u32x4* p) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1 nt" : : "v"(p), "v"(v) : "memory");
+  // (a store of more than 64 bits wants one wait state before its data registers are written again)
+  asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 0" : : "v"(p), "v"(v) : "memory");
 }
 
 __device__ __forceinline__ void wait_loads_all() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
@@ -302,40 +318,39 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     __syncthreads();
   }
 
-  const int frag_row = lane & 31, frag_k = lane >> 5;
+  // MFMA operand: this lane feeds row lane % 16, chunk lane / 16 (of 8 elements) of a 16 x 32 block; chunk
+  // ks * 4 + lane / 16 of a stage's row sits in slot chunk ^ ((row >> 1) & 7)
+  const int frag_row = lane & 15, frag_k = lane >> 4;
   const int swz = (frag_row >> 1) & 7;
-  auto frag_off = [&](int ks) { return ((ks * 2 + frag_k) ^ swz) << 4; };
+  auto frag_off = [&](int ks) { return ((ks * 4 + frag_k) ^ swz) << 4; };
   const bool gather = ROUTED && a.gather != 0;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
 
   // ---- epilogue: bias + activation, bf16, 32 rows at a time through this wavefront's image -----
-  // transposed accumulator: element r of tile (i, j) is output row 32 i + lane % 32, column (of the
-  // wavefront's 32 j .. 32 j + 31) 8 * (r / 4) + 4 * (lane / 32) + r % 4, i.e. a lane holds 4
-  // consecutive columns (8 bytes) of its row.
+  // transposed accumulator: element r of tile (i, j) is output row 16 i + lane % 16, column (of the
+  // wavefront's) 16 j + 4 * (lane / 16) + r, i.e. a lane holds 4 consecutive columns (8 bytes) of its row.
   auto epilogue = [&](auto& acc, int first_row, int mine, int col_w) {
     constexpr int MT = sizeof(acc) / sizeof(acc[0]), NT = sizeof(acc[0]) / sizeof(acc[0][0]);
     const int row_w = row0 + first_row;
     const global_bf16 bias = a.bias != nullptr ? (global_bf16)(a.bias[e]) : (global_bf16)nullptr;
     constexpr int kOutB = OUTF32 ? 4 : 2;                 // bytes of one output element
-    constexpr int kImageRow = NT * 32 * kOutB + 16;      // padded row of this wavefront's 32-row image
+    constexpr int kImageRow = NT * 16 * kOutB + 16;      // padded row of this wavefront's 32-row image
     constexpr int kImageB = 32 * kImageRow;
     static_assert(kWaves * kImageB <= kLdsBytes, "the output images must fit the stages");
     char* const image = smem + wave * kImageB;
     constexpr int kChunk = 16 / kOutB;                    // elements of one 16-byte store
-    constexpr int kChunksPerRow = NT * 32 / kChunk;
+    constexpr int kChunksPerRow = NT * 16 / kChunk;
     constexpr int kRowsPerPass = kWave / kChunksPerRow;
-    // the bias of this lane's columns, all eight loads in one round trip
-    bf16x4 bv[NT][4];
+    // the bias of this lane's columns, all loads in one round trip
+    bf16x4 bv[NT];
   #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int j = 0; j < NT; ++j) {
+      const int col = col_w + j * 16 + 4 * frag_k;
+      bv[j] = bf16x4{};
+      if (bias != nullptr && col < a.N) bv[j] = *(global_bf16x4)(bias + col);
+    }
   #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int col = col_w + j * 32 + 8 * g + 4 * frag_k;
-        bv[j][g] = bf16x4{};
-        if (bias != nullptr && col < a.N) bv[j][g] = *(global_bf16x4)(bias + col);
-      }
-  #pragma unroll
-    for (int i = 0; i < MT; ++i) {
+    for (int i = 0; i < MT / 2; ++i) {
       if (i * 32 >= mine) break;  // wave-uniform
       // scattered rows: lane r of the pass holds the cell of row r (read again: LDS held operands)
       int cell = -1;
@@ -346,15 +361,14 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
         }
       }
   #pragma unroll
-      for (int j = 0; j < NT; ++j) {
+      for (int ii = 0; ii < 2; ++ii) {
   #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int col = j * 32 + 8 * g + 4 * frag_k;  // inside the wavefront's 64 columns
-          const bf16x4 b4 = bv[j][g];
+        for (int j = 0; j < NT; ++j) {
+          const bf16x4 b4 = bv[j];
           float v[4];
   #pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] = apply_act<ACT>(acc[i][j][4 * g + q] + static_cast<float>(b4[q]));
-          char* const to = image + frag_row * kImageRow + col * kOutB;
+          for (int q = 0; q < 4; ++q) v[q] = apply_act<ACT>(acc[2 * i + ii][j][q] + static_cast<float>(b4[q]));
+          char* const to = image + (ii * 16 + frag_row) * kImageRow + (16 * j + 4 * frag_k) * kOutB;
           if constexpr (OUTF32) {
             *reinterpret_cast<f32x4*>(to) = f32x4{v[0] + 0.0f, v[1] + 0.0f, v[2] + 0.0f, v[3] + 0.0f};  // -0 -> +0, as a combine would
           } else {
@@ -404,7 +418,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     auto unit = [&](auto rows_tag) {
       constexpr int UR = decltype(rows_tag)::value;         // rows of the unit
       constexpr int kXw = UR / 64, kL = kXw + 1;            // row groups of x a wavefront loads, loads of a K-step
-      constexpr int UNT = UR == 256 ? 2 : 1;                // 32 x 32 blocks of a wavefront, side by side
+      constexpr int UMT = 2, UNT = UR == 256 ? 4 : 2;       // 16 x 16 tiles of a wavefront: 32 rows, all columns or half of them
       constexpr int kStage = (UR + kUnitCols) * kRowB;
       constexpr int D = UR == 256 ? 4 : UR == 128 ? 6 : 8;  // K-steps in flight and in LDS
       static_assert(D * kStage <= kLdsBytes, "the ring must fit");
@@ -427,20 +441,23 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
       auto fetch = [&](int s, uint32_t stage, int i) {
         load_to_lds(i == 0 ? res_u : res_x, off[i], s * kRowB, lds0 + stage + (i == 0 ? UR / 8 + wave : wave * kXw + i - 1) * 1024);
       };
-      const int tile_x = UNT == 2 ? wave : wave >> 1, tile_w = UNT == 2 ? 0 : wave & 1;
+      const int tile_x = UNT == 4 ? wave : wave >> 1, tile_w = UNT == 4 ? 0 : wave & 1;
       const int first_row = tile_x * 32, mine = __builtin_amdgcn_readfirstlane(max(min(rows - first_row, 32), 0));
-      f32x16 acc[1][UNT];
+      f32x4 acc[UMT][UNT];
 #pragma unroll
-      for (int j = 0; j < UNT; ++j) acc[0][j] = f32x16{};
+      for (int i = 0; i < UMT; ++i)
+#pragma unroll
+        for (int j = 0; j < UNT; ++j) acc[i][j] = f32x4{};
       struct Frags {
-        bf16x8 w[kSub][UNT], x[kSub];
+        bf16x8 w[kSub][UNT], x[kSub][UMT];
       };
       const char* const from_x = smem + (first_row + frag_row) * kRowB;
       const char* const from_w = smem + (UR + tile_w * 32 + frag_row) * kRowB;
-      auto read_frags = [&](Frags& f, uint32_t stage, int ks) {
-        f.x[ks] = *reinterpret_cast<const bf16x8*>(from_x + stage + frag_off(ks));
-#pragma unroll
-        for (int j = 0; j < UNT; ++j) f.w[ks][j] = *reinterpret_cast<const bf16x8*>(from_w + stage + frag_off(ks) + j * 32 * kRowB);
+      constexpr int kReads = UMT + UNT;  // of a k-step
+      auto read_frag = [&](Frags& f, uint32_t stage, int q) {
+        const int ks = q / kReads, of = q % kReads;
+        if (of < UNT) f.w[ks][of] = *reinterpret_cast<const bf16x8*>(from_w + stage + frag_off(ks) + of * 16 * kRowB);
+        else f.x[ks][of - UNT] = *reinterpret_cast<const bf16x8*>(from_x + stage + frag_off(ks) + (of - UNT) * 16 * kRowB);
       };
       auto cut_off = [&] {
 #pragma unroll
@@ -477,17 +494,20 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
 #pragma unroll
           for (int i = 0; i < kL; ++i) fetch(s + D, stage, i);
         }
+        // the MFMAs of the K-step, and evenly behind them the reads for the next one and the requests
+        constexpr int kMfmas = kSub * UMT * UNT;
 #pragma unroll
-        for (int ks = 0; ks < kSub; ++ks) {
+        for (int n = 0; n < kMfmas; ++n) {
           if constexpr (kMultiply) {
-#pragma unroll
-            for (int j = 0; j < UNT; ++j) acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.w[ks][j], cur.x[ks], acc[0][j], 0, 0, 0);
+            const int ks = n / (UMT * UNT), i = n / UNT % UMT, j = n % UNT;
+            multiply_add(acc[i][j], cur.w[ks][j], cur.x[ks][i]);
             __builtin_amdgcn_sched_barrier(0);
-            read_frags(next, ahead, ks);
+#pragma unroll
+            for (int q = n * kSub * kReads / kMfmas; q < (n + 1) * kSub * kReads / kMfmas; ++q) read_frag(next, ahead, q);
           }
           if constexpr (kFills) {
 #pragma unroll
-            for (int i = ks * kL / kSub; i < (ks + 1) * kL / kSub; ++i) fetch(s + D, stage, i);
+            for (int i = n * kL / kMfmas; i < (n + 1) * kL / kMfmas; ++i) fetch(s + D, stage, i);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -498,7 +518,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
         Frags f0, f1;
         if constexpr (decltype(multiply)::value) {
 #pragma unroll
-          for (int ks = 0; ks < kSub; ++ks) read_frags(f0, 0, ks);
+          for (int q = 0; q < kSub * kReads; ++q) read_frag(f0, 0, q);
           wait_lds();
         }
         int s = 0;
@@ -513,6 +533,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
       };
       if (mine > 0) {
         loop(std::true_type{});
+        mfma_wait_states();
         epilogue(acc, first_row, mine, n0 + tile_w * 32);
       } else {
         loop(std::false_type{});
@@ -564,8 +585,6 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   };
 
   // ---- fragments -------------------------------------------------------------------------------
-  // MFMA operand: this lane feeds row (lane % 32), k-half (lane / 32) of a 32 x 16 block; chunk
-  // ks * 2 + lane / 32 of the row sits in slot chunk ^ ((row >> 1) & 7)
   // The row tiles that hold rows are shared evenly by the two groups, group 0 taking the first `half`
   // rows: with 128 rows or fewer in one group the phases of a K-step would run one after the other.
   // (Halves fixed at 128 rows: the ragged FFN of 128 experts, 108 of its 201 row blocks part-filled,
@@ -574,17 +593,17 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   const int half = __builtin_amdgcn_readfirstlane(((rows + 63) >> 6) << 5);
   const int first_row = wm * half;  // of this wavefront, inside the tile
   const int frag_x = (first_row + frag_row) * kRowB;
-  const int frag_w = kBBase + (wn * kNT * 32 + frag_row) * kRowB;
+  const int frag_w = kBBase + (wn * kNT * 16 + frag_row) * kRowB;
 
-  f32x16 acc[kMT][kNT];
+  f32x4 acc[kMT][kNT];
 #pragma unroll
   for (int i = 0; i < kMT; ++i)
 #pragma unroll
-    for (int j = 0; j < kNT; ++j) acc[i][j] = f32x16{};
+    for (int j = 0; j < kNT; ++j) acc[i][j] = f32x4{};
   bf16x8 fw[kSub][kNT], fx[kSub][kMT];
-  // row tiles of this wavefront that hold rows (wave-uniform)
   const int mine = min(rows - first_row, half);  // rows of this wavefront
-  const int n_i = __builtin_amdgcn_readfirstlane(max((mine + 31) >> 5, 0));
+  // pairs of its row tiles that hold rows (wave-uniform)
+  const int pairs = __builtin_amdgcn_readfirstlane(max((mine + 31) >> 5, 0));
 
   auto cut_off = [&] {
 #pragma unroll
@@ -625,7 +644,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
 #pragma unroll
         for (int ks = 0; ks < kSub; ++ks)
 #pragma unroll
-          for (int j = 0; j < kNT; ++j) fw[ks][j] = *reinterpret_cast<const bf16x8*>(pb + frag_off(ks) + j * 32 * kRowB);
+          for (int j = 0; j < kNT; ++j) fw[ks][j] = *reinterpret_cast<const bf16x8*>(pb + frag_off(ks) + j * 16 * kRowB);
       }
       if (wm == 0) {
         // the activation rows go into the slot that held K-step kt - 1: both groups have read it
@@ -634,9 +653,9 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
 #pragma unroll
           for (int i = 0; i < kMT; ++i) {
             if constexpr (NI > 0) {
-              if (i < NI) fx[ks][i] = *reinterpret_cast<const bf16x8*>(pa + frag_off(ks) + i * 32 * kRowB);
+              if (i < NI) fx[ks][i] = *reinterpret_cast<const bf16x8*>(pa + frag_off(ks) + i * 16 * kRowB);
             }
-            if ((i & 1) && more) load_a(kt + 2, a_load, ks * 2 + (i >> 1));
+            if ((i & 1) && more) load_a(kt + 2, a_load, ks * 4 + (i >> 1));
           }
         }
         wait_lds();
@@ -649,9 +668,9 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
 #pragma unroll
           for (int i = 0; i < kMT; ++i) {
             if constexpr (NI > 0) {
-              if (i < NI) fx[ks][i] = *reinterpret_cast<const bf16x8*>(pa + frag_off(ks) + i * 32 * kRowB);
+              if (i < NI) fx[ks][i] = *reinterpret_cast<const bf16x8*>(pa + frag_off(ks) + i * 16 * kRowB);
             }
-            if ((i & 1) && more) load_b(kt + 2, b_cur, ks * 2 + (i >> 1));
+            if ((i & 1) && more) load_b(kt + 2, b_cur, ks * 4 + (i >> 1));
           }
         }
         wait_lds();
@@ -670,13 +689,13 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
             for (int j = 0; j < kNT; ++j) {
               const int n = (ks * NI + i) * kNT + j;
               if (n >= kFirst && n < kLast)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[ks][j], fx[ks][i], acc[i][j], 0, 0, 0);
+                multiply_add(acc[i][j], fw[ks][j], fx[ks][i]);
             }
       };
       // ---- C phase: nothing but the MFMAs of the K-step.  The first kHead of them are issued
       // before the barrier: they queue up behind the other group's last MFMAs and keep the matrix
-      // pipe fed while the barrier lets both groups through (2.5 % on every shape measured; with 8
-      // instead of 4 the group reaches the barrier too late for the other one's M phase).
+      // pipe fed while the barrier lets both groups through (2.5 % on every shape measured; with twice
+      // as many the group reaches the barrier too late for the other one's M phase).
       __builtin_amdgcn_sched_barrier(0);
       multiply(std::integral_constant<int, 0>{}, std::integral_constant<int, kHead>{});
       __builtin_amdgcn_sched_barrier(0);
@@ -696,11 +715,12 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     }
   };
   const long long clock0 = __builtin_amdgcn_s_memtime(), tick0 = __builtin_amdgcn_s_memrealtime();
-  if (n_i == 4) k_loop(std::integral_constant<int, 4>{});
-  else if (n_i == 3) k_loop(std::integral_constant<int, 3>{});
-  else if (n_i == 2) k_loop(std::integral_constant<int, 2>{});
-  else if (n_i == 1) k_loop(std::integral_constant<int, 1>{});
+  if (pairs == 4) k_loop(std::integral_constant<int, 8>{});
+  else if (pairs == 3) k_loop(std::integral_constant<int, 6>{});
+  else if (pairs == 2) k_loop(std::integral_constant<int, 4>{});
+  else if (pairs == 1) k_loop(std::integral_constant<int, 2>{});
   else k_loop(std::integral_constant<int, 0>{});
+  mfma_wait_states();
   if (a.clocks != nullptr && t == 0 && tid == 0) {  // measurement aid: this wavefront's K loop
     a.clocks[0] = __builtin_amdgcn_s_memtime() - clock0;
     a.clocks[1] = __builtin_amdgcn_s_memrealtime() - tick0;
@@ -709,7 +729,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   if (wm == 0) block_barrier();  // group 1's last C phase
   block_barrier();               // no wavefront reads a stage any more: the epilogue may write over them
 
-  epilogue(acc, first_row, mine, n0 + wn * kNT * 32);
+  epilogue(acc, first_row, mine, n0 + wn * kNT * 16);
 }
 
 // The sum over experts of ceil(M_e / 256) never exceeds P / 256 + E; whole rounds of XCD patches.  What the loads leave of it is room for
