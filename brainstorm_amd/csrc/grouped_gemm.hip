@@ -70,7 +70,8 @@ constexpr int kStreamingLoad = 2;
 // gives), 152 us with `sc1` or `sc0 sc1`, 160 us with ordinary stores; each GEMM on its own takes
 // the same time with `nt` and `sc1 nt`.  There is no builtin for the pair of bits.
 __device__ __forceinline__ void stream_out(const u32x4& v, u32x4* p) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1 nt" : : "v"(p), "v"(v) : "memory");
+  // (a store of more than 64 bits wants one wait state before its data registers are written again)
+  asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 0" : : "v"(p), "v"(v) : "memory");
 }
 
 template <int N>
