@@ -29,7 +29,7 @@ struct GemmArgs {
   int tiles_n, tiles_m_max;
   int walk, groups_n;  // column tiles one workgroup walks, ceil(tiles_n / walk)
   int grid;                  // workgroups, 0 where no tile may be cut into units (ping-pong kernel)
-  uint32_t tiles_n_inverse;  // (2^32 - 1) / tiles_n (ping-pong kernel)
+  uint32_t tiles_n_inverse, walk_inverse;  // (2^32 - 1) / tiles_n, / walk (ping-pong kernel)
   int patch;           // workgroups in patch order (experts with several row blocks), see the kernel
   // measurement aid (ping-pong kernel only): non-null, the workgroup of the first tile writes the
   // shader clocks (s_memtime) and the ticks of the constant 100 MHz counter (s_memrealtime) its

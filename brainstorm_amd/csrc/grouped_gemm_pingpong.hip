@@ -43,6 +43,8 @@
 //     it loads in registers for any kind of row, so a gathered row (its cell's offset) and an
 //     activation or weight row (row times pitch) are the same load.  The cells pass through the
 //     first bytes of the stages once, before any operand lands there.
+//   - A workgroup of the whole rounds walks two column tiles (or three or five) of its row block: the requests of the last K-steps
+//     of a tile are the first ones of the next, and the images of the finished rows go through the one slot of the rings that is free.
 //   - What the list of tiles holds beyond whole rounds over the CUs would keep a few of them busy for as long as a whole round, and the
 //     experts' last row blocks, which hold few rows, for more than half as long (the weights of 256 columns come into one CU at
 //     40 GB/s).  Where that is at most half a round it is cut into units of 256 rows x 64 columns: each wavefront loads its share of a
@@ -52,8 +54,8 @@
 //   - The epilogue sends the tile out 32 rows at a time through each wavefront's own corner of
 //     LDS (the stages are dead by then), full 128-byte rows per store.
 #include <algorithm>
-#include <cstdlib>
 #include <type_traits>
+#include <utility>
 
 #include "common.hpp"
 #include "grouped_gemm.hpp"
@@ -78,9 +80,10 @@ constexpr int kBBase = kAStages * kTileB;             // the weight ring follows
 constexpr int kLdsBytes = (kAStages + kBStages) * kTileB;  // 163840: all of a CU's LDS
 constexpr int kSub = kBK / 32;                        // MFMA k-steps per stage
 constexpr int kHead = 8;                              // MFMAs of a C phase issued ahead of the barrier
-constexpr uint32_t kOutOfRange = 0x80000000u;         // buffer offset past any extent: reads as zero
+constexpr uint32_t kOutOfRange = 0xf0000000u;         // buffer offset past any extent, also with what a load adds: reads as zero
 constexpr int kXcds = 8, kCusPerXcd = 32, kPatchRows = 4;
-constexpr int kRound = kXcds * kCusPerXcd;  // tiles of a whole round
+constexpr int kRoundBits = 8, kRound = kXcds * kCusPerXcd;  // tiles of a whole round
+static_assert(kRound == 1 << kRoundBits);
 // The end of the list that is cut into units (see the kernel).  It takes the CUs one round of units up to 64 tiles and two up to 128,
 // against a round in which the tiles leave most CUs idle.  A unit of 256 rows takes 0.4 to 0.5 of a tile's time (4 x 1024 rows
 // 4096 -> 1024, 256 units: 40 us against 102 us for the 64 tiles they are made of), one of up to 128 rows half of what its block
@@ -115,16 +118,25 @@ __device__ __forceinline__ i32x4 make_rsrc(const void* p, size_t bytes) {
   return r;
 }
 
-// 16 bytes per lane from the buffer straight into LDS at lds_base + 16 * lane (wave-uniform
-// lds_base in M0).  Counts on vmcnt like any load; the compiler does not know it touches LDS,
-// so every wait for such a load is written out below.
+// 16 bytes per lane from the buffer straight into LDS at lds_base + kAt + 16 * lane (wave-uniform lds_base in M0, one wait
+// state between its write and the load); the instruction's offset kAt is added to the place in the buffer too.  Counts on vmcnt
+// like any load; the compiler does not know it touches LDS, so every wait for such a load is written out below.
+template <int kAt = 0>
 __device__ __forceinline__ void load_to_lds(const i32x4& rsrc, uint32_t voffset, uint32_t soffset,
                                             uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "s"(lds_base), "v"(voffset), "s"(rsrc), "s"(soffset)
-               : "memory");
+  if constexpr (kAt == 0)
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "{m0}"(lds_base), "v"(voffset), "s"(rsrc), "s"(soffset)
+                 : "memory");
+  else  // M0 is what it was for the load before
+    asm volatile("buffer_load_dwordx4 %1, %2, %3 offen offset:%4 lds"
+                 :
+                 : "{m0}"(lds_base), "v"(voffset), "s"(rsrc), "s"(soffset), "n"(kAt)
+                 : "memory");
 }
+template <typename Fn, int... I>
+__device__ __forceinline__ void for_each(Fn&& fn, std::integer_sequence<int, I...>) { (fn(std::integral_constant<int, I>{}), ...); }
 
 // acc += w x, 16 x 16 x 32.  In place: as a builtin the instruction gets other registers for its result, and accumulators are moved.
 // The compiler does not know its wait states then: mfma_wait_states() stands before anything else reads an accumulator.
@@ -216,10 +228,12 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     v.incl_m = wave_inclusive_scan(v.m[0] + v.m[1]);
     return v;
   };
-  auto over_tn = [&](int n) {  // n / tn
-    const int q = static_cast<int>(__umulhi(static_cast<uint32_t>(n), a.tiles_n_inverse));
-    return n - q * tn >= tn ? q + 1 : q;
+  auto over = [](int n, int d, uint32_t inverse) {  // n / d
+    const int q = static_cast<int>(__umulhi(static_cast<uint32_t>(n), inverse));
+    return n - q * d >= d ? q + 1 : q;
   };
+  auto over_tn = [&](int n) { return over(n, tn, a.tiles_n_inverse); };
+  auto over_walk = [&](int n) { return over(n, a.walk, a.walk_inverse); };
   Two two = read_two(0);
   const int sums = read_lane(two.incl_b, kWave - 1);
   int many = sums >> 8, few = sums & 255;
@@ -229,19 +243,24 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   }
   const int tiles = (many + few) * tn;
   const auto [moved, cut] = end_of_list(a, tiles, few, over_tn);
-  const int listed = tiles - moved * tn, whole = tiles - cut, used = tiles + 3 * cut;
+  const int listed = tiles - moved * tn, whole = tiles - cut;
+  // Whole rounds over the CUs of `walk` tiles each come first, one workgroup for the column tiles of a row block.
+  const int walkers = a.walk > 1 ? over_walk(whole >> kRoundBits) << kRoundBits : 0, walked = walkers * a.walk;
+  const int used = walkers + (whole - walked) + 4 * cut;
   if (t >= used) {
     // Surplus workgroups clear the tags of the rows no path owns, 256 of them a step.  The grid holds P / 256 + E row blocks
     // (rounded up) per column tile, the experts use at most (total + 255 E) / 256, and the cut leaves at least one.
     if (ROUTED && a.row_tags_out != nullptr && tid < kBM) {
       long total = 0;
       for (int base = 0; base < a.E; base += 2 * kWave) total += read_lane(read_two(base).incl_m, kWave - 1);
-      for (long r = total + static_cast<long>(t - used) * kBM + tid; r < a.P; r += static_cast<long>(a.grid - used) * kBM) a.row_tags_out[r] = 0;
+      for (long r = total + static_cast<long>(t - used) * kBM + tid; r < a.P; r += static_cast<long>(gridDim.x - used) * kBM) a.row_tags_out[r] = 0;
     }
     return;
   }
-  const bool narrow = t >= whole;
-  const int tile = narrow ? whole + ((t - whole) >> 2) : t;
+  const int at = t < walkers ? t * a.walk : walked + (t - walkers);  // in the list, a unit counted as one
+  const bool narrow = at >= whole;
+  const int tile = narrow ? whole + ((at - whole) >> 2) : at;
+  int left = t < walkers ? a.walk : 1;  // tiles of this workgroup, the one at hand included
   const bool apart = tile >= listed;  // of a moved block
   const int place = apart ? tile - listed : tile;
   int e = 0, row0 = 0, rows = 0, seat0 = 0, n0 = 0;
@@ -272,9 +291,12 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
       } else {
         const int blocks = second ? many1 + few1 - moved1 : blocks0;
         const int g = min(over_tn(local) / kPatchRows, blocks / kPatchRows);
+        // of a patch the first a.walk column tiles of its row blocks, one row block after the other, then the next ones (a.walk divides tn)
         const int r = local - g * kPatchRows * tn, wide = min(blocks - g * kPatchRows, kPatchRows);
-        col = wide == 4 ? r >> 2 : wide == 3 ? static_cast<int>(__umulhi(static_cast<uint32_t>(r), 0x55555556u)) : wide == 2 ? r >> 1 : r;
-        block = g * kPatchRows + r - col * wide;
+        const int run = a.walk > 1 ? over_walk(r) : r;
+        const int runs = wide == 4 ? run >> 2 : wide == 3 ? static_cast<int>(__umulhi(static_cast<uint32_t>(run), 0x55555556u)) : wide == 2 ? run >> 1 : run;
+        block = g * kPatchRows + run - runs * wide;
+        col = runs * a.walk + r - run * a.walk;
       }
       const uint64_t wp = second ? two.w[1] : two.w[0];
       e = base + 2 * src + (second ? 1 : 0);
@@ -294,11 +316,11 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     two = read_two(base);
   }
   if (narrow) {
-    n0 += ((t - whole) & 3) * kUnitCols;
+    n0 += ((at - whole) & 3) * kUnitCols;
     if (n0 >= a.N) return;
   }
   const int K = a.K;
-  const int k_tiles = (K + kBK - 1) / kBK;
+  const int k_tiles = __builtin_amdgcn_readfirstlane((K + kBK - 1) / kBK);
   // A last K-step that K does not fill: before it is requested, and nothing after it is, the lanes whose chunk of 8 elements
   // lies behind K are turned to an offset past any extent, so they fill LDS with zeros.  (K is a multiple of 8.)  The K loop
   // pays one scalar comparison for it: 16 x 2048 rows 1024 -> 4096 282.8 us without it, 281.5 with it.
@@ -329,17 +351,22 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // ---- epilogue: bias + activation, bf16, 32 rows at a time through this wavefront's image -----
   // transposed accumulator: element r of tile (i, j) is output row 16 i + lane % 16, column (of the
   // wavefront's) 16 j + 4 * (lane / 16) + r, i.e. a lane holds 4 consecutive columns (8 bytes) of its row.
-  auto epilogue = [&](auto& acc, int first_row, int mine, int col_w) {
+  auto epilogue = [&](auto& acc, int first_row, int mine, int col_w, uint32_t images) {
     constexpr int MT = sizeof(acc) / sizeof(acc[0]), NT = sizeof(acc[0]) / sizeof(acc[0][0]);
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane), "+s"(images));  // (else what follows from it is kept in registers all through the K loops of a walk)
+    const int frag_row = lane & 15, frag_k = lane >> 4;
     const int row_w = row0 + first_row;
     const global_bf16 bias = a.bias != nullptr ? (global_bf16)(a.bias[e]) : (global_bf16)nullptr;
     constexpr int kOutB = OUTF32 ? 4 : 2;                 // bytes of one output element
-    constexpr int kImageRow = NT * 16 * kOutB + 16;      // padded row of this wavefront's 32-row image
-    constexpr int kImageB = 32 * kImageRow;
-    static_assert(kWaves * kImageB <= kLdsBytes, "the output images must fit the stages");
-    char* const image = smem + wave * kImageB;
     constexpr int kChunk = 16 / kOutB;                    // elements of one 16-byte store
-    constexpr int kChunksPerRow = NT * 16 / kChunk;
+    constexpr int kCols = OUTF32 ? 32 : NT * 16;          // columns of an image
+    constexpr int kChunksPerRow = kCols / kChunk;
+    constexpr int kImageRow = kCols * kOutB, kImageB = 32 * kImageRow;
+    static_assert(kWaves * kImageB <= kTileB, "the output images must fit one slot");
+    char* const image = smem + images + wave * kImageB;
+    // the chunks of an image row are swizzled like those of the stages
+    auto slot = [](int row, int chunk) { return (chunk ^ (kChunksPerRow == 4 ? (row >> 2) & 3 : (row >> 1) & 7)) * 16; };
     constexpr int kRowsPerPass = kWave / kChunksPerRow;
     // the bias of this lane's columns, all loads in one round trip
     bf16x4 bv[NT];
@@ -361,52 +388,56 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
         }
       }
   #pragma unroll
-      for (int ii = 0; ii < 2; ++ii) {
+      for (int j0 = 0; j0 < NT; j0 += kCols / 16) {
   #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          const bf16x4 b4 = bv[j];
-          float v[4];
+        for (int ii = 0; ii < 2; ++ii) {
   #pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] = apply_act<ACT>(acc[2 * i + ii][j][q] + static_cast<float>(b4[q]));
-          char* const to = image + (ii * 16 + frag_row) * kImageRow + (16 * j + 4 * frag_k) * kOutB;
-          if constexpr (OUTF32) {
-            *reinterpret_cast<f32x4*>(to) = f32x4{v[0] + 0.0f, v[1] + 0.0f, v[2] + 0.0f, v[3] + 0.0f};  // -0 -> +0, as a combine would
-          } else {
-            *reinterpret_cast<bf16x4*>(to) = bf16x4{static_cast<__bf16>(v[0]), static_cast<__bf16>(v[1]),
-                                                    static_cast<__bf16>(v[2]), static_cast<__bf16>(v[3])};
-          }
-        }
-      }
-      wave_fence();
-      const int rows_i = min(32, mine - i * 32);
-      const int c = lane % kChunksPerRow;
-      char* const out_b = OUTF32 ? reinterpret_cast<char*>(a.out_f32) : reinterpret_cast<char*>(a.out);
+          for (int j = j0; j < j0 + kCols / 16; ++j) {
+            const bf16x4 b4 = bv[j];
+            float v[4];
   #pragma unroll
-      for (int p = 0; p < 32 / kRowsPerPass; ++p) {
-        const int rl = p * kRowsPerPass + lane / kChunksPerRow;
-        long row = row_w + i * 32 + rl;
-        bool live = rl < rows_i && col_w + c * kChunk < a.N;
-        if constexpr (ROUTED) {
-          if (a.scatter) {
-            const int to = __shfl(cell, rl, kWave);
-            live = live && to >= 0;
-            row = to;
-          }
-        }
-        if (live) {
-          u32x4 v = *reinterpret_cast<const u32x4*>(image + rl * kImageRow + c * 16);
-          if constexpr (ROUTED && !OUTF32) {
-            if (a.scatter) {  // the combine this store stands for adds the row to zero: -0 becomes +0
-  #pragma unroll
-              for (int w = 0; w < 4; ++w) v[w] = plus_zero<BRT_BF16>(v[w]);
+            for (int q = 0; q < 4; ++q) v[q] = apply_act<ACT>(acc[2 * i + ii][j][q] + static_cast<float>(b4[q]));
+            const int row = ii * 16 + frag_row, at = (16 * (j - j0) + 4 * frag_k) * kOutB;  // in the image
+            char* const to = image + row * kImageRow + slot(row, at / 16) + at % 16;
+            if constexpr (OUTF32) {
+              *reinterpret_cast<f32x4*>(to) = f32x4{v[0] + 0.0f, v[1] + 0.0f, v[2] + 0.0f, v[3] + 0.0f};  // -0 -> +0, as a combine would
+            } else {
+              *reinterpret_cast<bf16x4*>(to) = bf16x4{static_cast<__bf16>(v[0]), static_cast<__bf16>(v[1]),
+                                                      static_cast<__bf16>(v[2]), static_cast<__bf16>(v[3])};
             }
           }
-          u32x4* const to = reinterpret_cast<u32x4*>(out_b + (static_cast<size_t>(row) * a.N + col_w) * kOutB + c * 16);
-          if (a.plain_out) *to = v;
-          else stream_out(v, to);
         }
+        wave_fence();
+        const int rows_i = min(32, mine - i * 32);
+        const int c = lane % kChunksPerRow, col = col_w + j0 * 16 + c * kChunk;
+        char* const out_b = OUTF32 ? reinterpret_cast<char*>(a.out_f32) : reinterpret_cast<char*>(a.out);
+  #pragma unroll
+        for (int p = 0; p < 32 / kRowsPerPass; ++p) {
+          const int rl = p * kRowsPerPass + lane / kChunksPerRow;
+          long row = row_w + i * 32 + rl;
+          bool live = rl < rows_i && col < a.N;
+          if constexpr (ROUTED) {
+            if (a.scatter) {
+              const int to = __shfl(cell, rl, kWave);
+              live = live && to >= 0;
+              row = to;
+            }
+          }
+          if (live) {
+            u32x4 v = *reinterpret_cast<const u32x4*>(image + rl * kImageRow + slot(rl, c));
+            if constexpr (ROUTED && !OUTF32) {
+              if (a.scatter) {  // the combine this store stands for adds the row to zero: -0 becomes +0
+  #pragma unroll
+                for (int w = 0; w < 4; ++w) v[w] = plus_zero<BRT_BF16>(v[w]);
+              }
+            }
+            u32x4* const to = reinterpret_cast<u32x4*>(out_b + (static_cast<size_t>(row) * a.N + col) * kOutB);
+            if (a.plain_out) *to = v;
+            else stream_out(v, to);
+          }
+        }
+        wave_fence();
       }
-      wave_fence();
     }
   };
 
@@ -534,7 +565,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
       if (mine > 0) {
         loop(std::true_type{});
         mfma_wait_states();
-        epilogue(acc, first_row, mine, n0 + tile_w * 32);
+        epilogue(acc, first_row, mine, n0 + tile_w * 32, 0);
       } else {
         loop(std::false_type{});
       }
@@ -547,24 +578,34 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
 
   // ---- global -> LDS ---------------------------------------------------------------------------
   // A load fills one row group: 8 tile rows, a whole 128-byte line of each.  Group 0 loads the
-  // activation rows, wavefront wn taking row groups wn + 4 i (i = 0..7); group 1 the weight rows,
-  // wavefront wn taking the 64 rows of its own columns, row groups 8 wn + i.  Lane l lands at slot
+  // activation rows, group 1 the weight rows, wavefront wn row groups 8 wn + i (i = 0..7).  Lane l lands at slot
   // l & 7 of row l >> 3 of the group and fetches chunk (l & 7) ^ ((row >> 1) & 7) of that row.  A row
   // that does not exist (past the expert's last row, past N) gets an offset past any extent: zeros,
   // no memory request.
   // Every wavefront keeps the eight offsets of its rows in registers (the K-step alone goes into
   // the scalar offset).  Gathered rows need that -- the cells of a row group are anywhere in x --
   // and it takes the bounds check out of the loop for the others.
-  const i32x4 res = in_scalars(wm == 0
+  // An M phase is as long as its instructions take to issue, so the eight requests are eight instructions and two writes of M0: four
+  // loads share one value, the instruction's own offset, 1 KB apart, moves them in LDS, and the registers hold the place in the
+  // buffer less that offset, in a buffer that starts kBack bytes early.  When nothing more is to be requested the extent becomes
+  // zero.  (With M0 computed and written for each load and a branch around it, against this, of the time that the kernel took with neither and
+  // 32 x 32 x 16 MFMAs: 8192 -> 2048 0.983 and 0.952, 2048 -> 8192 0.964 and 0.932, ragged loads 8192 -> 2048 1.01 and 0.97.)
+  constexpr uint32_t kBack = 3 * 1024;
+  auto start_early = [](i32x4 r) {
+    const uint64_t at = (static_cast<uint64_t>(static_cast<uint32_t>(r[1])) << 32 | static_cast<uint32_t>(r[0])) - kBack;
+    r[0] = static_cast<int>(at), r[1] = static_cast<int>(at >> 32) & 0xffff;
+    r[2] = static_cast<int>(static_cast<uint32_t>(r[2]) + kBack);
+    return r;
+  };
+  i32x4 res = in_scalars(start_early(wm == 0
       ? (gather ? make_rsrc(a.x, static_cast<size_t>(a.T) * K * 2)
                 : make_rsrc(a.x + static_cast<size_t>(row0) * K, static_cast<size_t>(a.P - row0) * K * 2))
-      : make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2));
+      : make_rsrc(w_e + static_cast<size_t>(n0) * K, static_cast<size_t>(a.N - n0) * K * 2)));
   const int cols = a.N - n0;  // weight rows that exist from n0 on
   uint32_t off[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const int group = wm == 0 ? wn + 4 * i : wn * 8 + i;
-    const int row = group * 8 + (lane >> 3);
+    const int row = (wn * 8 + i) * 8 + (lane >> 3);
     const uint32_t chunk = (lane & 7) ^ ((row >> 1) & 7);
     int at = row;
     bool there = row < (wm == 0 ? rows : cols);
@@ -574,14 +615,12 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
         there = at >= 0;
       }
     }
-    off[i] = there ? (static_cast<uint32_t>(at) * K + chunk * 8) * 2 : kOutOfRange;
+    off[i] = there ? (static_cast<uint32_t>(at) * K + chunk * 8) * 2 + kBack - (i & 3) * 1024 : kOutOfRange;
   }
   if constexpr (ROUTED) __syncthreads();  // everyone has read the cells; the loads may overwrite them
-  auto load_a = [&](int kt, uint32_t slot, int i) {
-    load_to_lds(res, off[i], kt * kRowB, lds0 + slot + (wn + 4 * i) * 1024);
-  };
-  auto load_b = [&](int kt, uint32_t slot, int i) {
-    load_to_lds(res, off[i], kt * kRowB, lds0 + kBBase + slot + (wn * 8 + i) * 1024);
+  const uint32_t lds_rows = lds0 + (wm == 0 ? 0 : kBBase) + wn * 8 * 1024;
+  auto load = [&](uint32_t from, uint32_t slot, auto i) {
+    load_to_lds<(i & 3) * 1024>(res, off[i], from, lds_rows + slot + (i & 4) * 1024);
   };
 
   // ---- fragments -------------------------------------------------------------------------------
@@ -596,88 +635,75 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   const int frag_w = kBBase + (wn * kNT * 16 + frag_row) * kRowB;
 
   f32x4 acc[kMT][kNT];
-#pragma unroll
-  for (int i = 0; i < kMT; ++i)
-#pragma unroll
-    for (int j = 0; j < kNT; ++j) acc[i][j] = f32x4{};
   bf16x8 fw[kSub][kNT], fx[kSub][kMT];
   const int mine = min(rows - first_row, half);  // rows of this wavefront
   // pairs of its row tiles that hold rows (wave-uniform)
   const int pairs = __builtin_amdgcn_readfirstlane(max((mine + 31) >> 5, 0));
 
+  // Before the request of K-step `turn` some lanes' offsets change: those of the chunks behind K, or, where a walk goes on to a last
+  // column tile of fewer than 256 columns (K is whole there), those of the weight rows that it does not have.
   auto cut_off = [&] {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) cut_chunk(off[i], wm == 0 ? wn + 4 * i : wn * 8 + i);
+    for (int i = 0; i < 8; ++i) {
+      if (part >= 0) {
+        cut_chunk(off[i], wn * 8 + i);
+      } else if (wm == 1) {
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        if ((wn * 8 + i) * 8 + (l >> 3) >= a.N % kBN) off[i] = kOutOfRange;
+      }
+    }
   };
   // prologue: K-steps 0 and 1 (both whole: K >= 128)
-  if (wm == 0) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) load_a(0, 0, i);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) load_a(1, kTileB, i);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) load_b(0, 0, i);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) load_b(1, kTileB, i);
-  }
+  using Eight = std::make_integer_sequence<int, 8>;
+  for_each([&](auto i) { load(0, 0, i); }, Eight{});
+  for_each([&](auto i) { load(kRowB, kTileB, i); }, Eight{});
   wait_loads_but_8();  // K-step 0
   block_barrier();
-  // Group 1 starts one phase late.  From here on a barrier ends group 0's M phase and group 1's C
-  // phase, the next one group 0's C phase and group 1's M phase, and so on.
-  if (wm == 1) block_barrier();
+  // The K-steps of a walk's tiles follow one another in the rings: the slots of the K-step being read and of the one being
+  // requested, where the latter starts in its rows, and what takes it from the end of a tile's K to the start of the next tile's.
+  uint32_t a_cur = 0, a_load = 2 * kTileB, b_cur = 0, from = 2 * kRowB;
+  const uint32_t turn_back = (wm == 0 ? 0 : static_cast<uint32_t>(kBN) * K * 2) - static_cast<uint32_t>(k_tiles) * kRowB;
+  const bool narrow_last = a.N % kBN != 0;
   // The K loop, for a wavefront whose first NI row tiles hold rows.  A ragged expert's last row
   // block reads no fragments and issues no MFMAs for the other row tiles, so a block of few rows
   // runs at the pace of its weight stream instead of that of 256 rows of matrix work.  The
   // wavefronts of a workgroup may run different instances: the barriers and the requests are the same in all.
   auto k_loop = [&](auto ni_tag) {
     constexpr int NI = decltype(ni_tag)::value;
-    uint32_t a_cur = 0, a_load = 2 * kTileB;  // ring slots: the K-step being read, the one being requested
+    const int turn = left == 2 && narrow_last && n0 + 2 * kBN > a.N ? k_tiles : part;
     for (int kt = 0; kt < k_tiles; ++kt) {
-      const uint32_t b_cur = (kt & 1) * kTileB;
-      const bool more = kt + 2 < k_tiles;
-      if (kt + 2 == part) cut_off();
+      if (kt + 2 == turn) cut_off();
+      if (kt + 2 == k_tiles) {
+        from += turn_back;
+        if (left == 1) res[2] = 0;
+      }
       const char* const pa = smem + a_cur + frag_x;
       const char* const pb = smem + b_cur + frag_w;
-      // ---- M phase: fragments of K-step kt into registers, requests for K-step kt + 2 ----------
+      // ---- M phase: fragments of K-step kt into registers, requests for K-step kt + 2.  Group 0's activation rows go into the slot that
+      // held K-step kt - 1: both groups have read it.  Group 1's weight rows go into the slot it is reading: group 0 read these rows a
+      // phase ago, and this wavefront's own weight fragments are in registers after the wait.
       if constexpr (NI > 0) {
 #pragma unroll
         for (int ks = 0; ks < kSub; ++ks)
 #pragma unroll
           for (int j = 0; j < kNT; ++j) fw[ks][j] = *reinterpret_cast<const bf16x8*>(pb + frag_off(ks) + j * 16 * kRowB);
       }
-      if (wm == 0) {
-        // the activation rows go into the slot that held K-step kt - 1: both groups have read it
-#pragma unroll
-        for (int ks = 0; ks < kSub; ++ks) {
-#pragma unroll
-          for (int i = 0; i < kMT; ++i) {
+      const uint32_t slot = wm == 0 ? a_load : b_cur;
+      if (wm == 1) wait_lds();
+      __builtin_amdgcn_sched_barrier(0);
+      for_each(
+          [&](auto i) {
             if constexpr (NI > 0) {
-              if (i < NI) fx[ks][i] = *reinterpret_cast<const bf16x8*>(pa + frag_off(ks) + i * 16 * kRowB);
-            }
-            if ((i & 1) && more) load_a(kt + 2, a_load, ks * 4 + (i >> 1));
-          }
-        }
-        wait_lds();
-      } else {
-        // the weight rows go into the slot this wavefront is reading: group 0 read these rows a
-        // phase ago, and this wavefront's own weight fragments are in registers after the wait
-        wait_lds();
 #pragma unroll
-        for (int ks = 0; ks < kSub; ++ks) {
-#pragma unroll
-          for (int i = 0; i < kMT; ++i) {
-            if constexpr (NI > 0) {
-              if (i < NI) fx[ks][i] = *reinterpret_cast<const bf16x8*>(pa + frag_off(ks) + i * 16 * kRowB);
+              for (int ks = 0; ks < kSub; ++ks)
+                if (i < NI) fx[ks][i] = *reinterpret_cast<const bf16x8*>(pa + frag_off(ks) + i * 16 * kRowB);
             }
-            if ((i & 1) && more) load_b(kt + 2, b_cur, ks * 4 + (i >> 1));
-          }
-        }
-        wait_lds();
-        // the weight rows of K-step kt + 1 have landed (group 0 reads them after this barrier)
-        if (more) wait_loads_but_8();
-        else wait_loads_all();
-      }
+            load(from, slot, i);
+          },
+          Eight{});
+      wait_lds();
+      if (wm == 1) wait_loads_but_8();  // the weight rows of K-step kt + 1 have landed (group 0 reads them after this barrier)
       // MFMAs [first, last) of the K-step's 8 x NI, in (ks, i, j) order
       auto multiply = [&](auto first_tag, auto last_tag) {
         constexpr int kFirst = decltype(first_tag)::value, kLast = decltype(last_tag)::value;
@@ -705,31 +731,43 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
       multiply(std::integral_constant<int, kHead>{}, std::integral_constant<int, kSub * kMT * kNT>{});
       __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_sched_barrier(0);
-      if (wm == 0) {  // the activation rows of K-step kt + 1 have landed
-        if (more) wait_loads_but_8();
-        else wait_loads_all();
-      }
-      block_barrier();
+      if (wm == 0) wait_loads_but_8();  // the activation rows of K-step kt + 1 have landed
+      // (group 1 goes from its last C phase straight into the epilogue)
+      if (wm == 0 || kt + 1 < k_tiles) block_barrier();
       a_cur = a_cur == 2 * kTileB ? 0 : a_cur + kTileB;
       a_load = a_load == 2 * kTileB ? 0 : a_load + kTileB;
+      b_cur ^= kTileB;
+      from += kRowB;
     }
   };
-  const long long clock0 = __builtin_amdgcn_s_memtime(), tick0 = __builtin_amdgcn_s_memrealtime();
-  if (pairs == 4) k_loop(std::integral_constant<int, 8>{});
-  else if (pairs == 3) k_loop(std::integral_constant<int, 6>{});
-  else if (pairs == 2) k_loop(std::integral_constant<int, 4>{});
-  else if (pairs == 1) k_loop(std::integral_constant<int, 2>{});
-  else k_loop(std::integral_constant<int, 0>{});
-  mfma_wait_states();
-  if (a.clocks != nullptr && t == 0 && tid == 0) {  // measurement aid: this wavefront's K loop
-    a.clocks[0] = __builtin_amdgcn_s_memtime() - clock0;
-    a.clocks[1] = __builtin_amdgcn_s_memrealtime() - tick0;
-    a.clocks[2] = k_tiles;
+  for (;;) {
+#pragma unroll
+    for (int i = 0; i < kMT; ++i)
+#pragma unroll
+      for (int j = 0; j < kNT; ++j) acc[i][j] = f32x4{};
+    // Group 1 runs one phase late.  From here on a barrier ends group 0's M phase and group 1's C
+    // phase, the next one group 0's C phase and group 1's M phase, and so on.
+    if (wm == 1) block_barrier();
+    const long long clock0 = __builtin_amdgcn_s_memtime(), tick0 = __builtin_amdgcn_s_memrealtime();
+    if (pairs == 4) k_loop(std::integral_constant<int, 8>{});
+    else if (pairs == 3) k_loop(std::integral_constant<int, 6>{});
+    else if (pairs == 2) k_loop(std::integral_constant<int, 4>{});
+    else if (pairs == 1) k_loop(std::integral_constant<int, 2>{});
+    else k_loop(std::integral_constant<int, 0>{});
+    mfma_wait_states();
+    if (a.clocks != nullptr && t == 0 && tid == 0) {  // measurement aid: this wavefront's K loop
+      a.clocks[0] = __builtin_amdgcn_s_memtime() - clock0;
+      a.clocks[1] = __builtin_amdgcn_s_memrealtime() - tick0;
+      a.clocks[2] = k_tiles;
+    }
+    if (left == 1) wait_loads_all();  // (of the requests of nothing: a workgroup does not end while a load into its LDS is under way)
+    // The last M phase of both groups is over since group 0's last barrier, and the slot of the last activation rows, the next one to
+    // be requested, holds the images: the two K-steps of the next tile that are under way or have landed lie in the others.
+    epilogue(acc, first_row, mine, n0 + wn * kNT * 16, a_load);
+    if (--left == 0) break;
+    n0 += kBN;
+    block_barrier();  // the images are read, their slot may be filled
   }
-  if (wm == 0) block_barrier();  // group 1's last C phase
-  block_barrier();               // no wavefront reads a stage any more: the epilogue may write over them
-
-  epilogue(acc, first_row, mine, n0 + wn * kNT * 16);
 }
 
 // The sum over experts of ceil(M_e / 256) never exceeds P / 256 + E; whole rounds of XCD patches.  What the loads leave of it is room for
@@ -750,16 +788,41 @@ long workgroups_of_list(int P, int E, int tiles_n) {
   return (entries + kRound - 1) / kRound * kRound;
 }
 
+// A list of up to `entries` tiles of which whole rounds are walked, `walk` tiles to a workgroup: the workgroups it needs at most, with
+// the units of an end that is cut and one to clear row tags.  (A list one tile short of another walked round needs more than a longer one.)
+long workgroups_that_walk(long entries, int walk) {
+  const long per = static_cast<long>(walk) * kRound, rounds = entries / per;
+  const long most = rounds == 0 ? entries : std::max(entries - rounds * (per - kRound), rounds * kRound + per - kRound - 1);
+  return std::min(entries, (most + 4 * kMostCutOfFewRows + 1 + kRound - 1) / kRound * kRound);
+}
+
+// Column tiles that a workgroup of the whole rounds walks: 2, or where their number is odd 3 or 5.  A walked tile costs neither a look
+// at the loads nor a wait for its first K-steps nor the end of a workgroup, 4 us of the 33 that a tile of K = 1024 takes (us, one tile a workgroup
+// and this many: 64 x 300 rows 768 -> 3072 + GELU 153 and 140, skewed top-2 rows of 32 experts 1024 -> 4096 + GELU 155 and 149, 16 x 2048 rows
+// 256 -> 1024 34.0 and 31.2, 8 x 4000 rows 768 -> 768 46.3 and 45.3; 128 experts of ragged loads 1024 -> 4096 389 and 361).  With 4 of them even loads of
+// many rounds gain another 1 to 2 % (512 -> 2048 85.7 and 84.5), skewed ones lose 3 to 6 (158 for the 149).  Where K is long there is
+// little to win and there are few column tiles, of which then fewer row blocks of an XCD share the weights: 16 skewed experts of 32768 rows
+// 4096 -> 1024 222 and 235, 1024 -> 1024 63.3 and 61.4, 4096 -> 2048 417 and 411, 8 x 4096 rows 8192 -> 2048 762 and 771.
+int walk_of_list(const GemmArgs& a) {
+  if (a.K % kBK != 0 || a.K > (a.tiles_n < 8 ? 1024 : 4096)) return 1;
+  for (int w : {2, 3, 5})
+    if (a.tiles_n % w == 0) return w;
+  return 1;
+}
+
 template <int ACT, bool ROUTED, bool OUTF32>
 int launch_pingpong(GemmArgs& a, hipStream_t st) {
   a.tiles_n = (a.N + kBN - 1) / kBN;
-  const long grid = workgroups_of_list(a.P, a.E, a.tiles_n);
+  long grid = workgroups_of_list(a.P, a.E, a.tiles_n);
   // The timed form wants the clocks of a whole tile, also of a list that would be cut to the last: it is told of no workgroups for units.
   // (A test of a.clocks in the kernel itself cost 32768 rows of 16 experts 1024 -> 4096 -> 1024 7 us of 577.)
   a.grid = a.clocks != nullptr ? 0 : static_cast<int>(grid);
   a.tiles_n_inverse = 0xffffffffu / static_cast<uint32_t>(a.tiles_n);
+  a.walk = a.clocks != nullptr ? 1 : walk_of_list(a);
+  a.walk_inverse = 0xffffffffu / static_cast<uint32_t>(a.walk);
   auto* fn = &grouped_gemm_pingpong_kernel<ACT, ROUTED, OUTF32>;
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(fn), kLdsBytes); rc != BRT_OK) return rc;
+  if (a.walk > 1) grid = workgroups_that_walk(grid, a.walk);
   hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(grid)), dim3(kWaves * 64), kLdsBytes, st, a);
   return check_launch("grouped_gemm_pingpong_kernel");
 }

@@ -705,6 +705,50 @@ def test_ping_pong_tiles_with_routing_and_fp32_output(T, E, K, N, k, cap, pad):
     del ws
 
 
+# whole rounds of two, three and five column tiles a workgroup: two K-steps and odd numbers of them (the rings go on where the last tile left
+# them), last column tiles of fewer columns, light and empty experts among the walked row blocks
+@pytest.mark.parametrize("loads,K,N,walk", [
+    ([5000, 3000, 300, 0, 20000, 31, 97, 2304], 128, 4096, 2),
+    ([9000, 1, 10000, 129, 161, 65], 192, 2040, 2),
+    ([2048] * 12, 320, 2000, 2),
+    ([40000, 300, 0, 46000, 100], 320, 768, 3),
+    ([80000, 40], 192, 520, 3),
+    ([50000, 200, 30000], 128, 1272, 5),
+])
+def test_walks_over_column_tiles(loads, K, N, walk):
+    """The bits of the same rows with K filled up with zeros to a width that is not walked (no multiple of 64), in the plain, fp32-output and
+    gathering forms; the library's result within the tolerance."""
+    from brainstorm_amd.jit import grouped_linear
+
+    P, E, tn = sum(loads), len(loads), -(-N // 256)
+    tiles = sum(-(-m // 256) for m in loads) * tn
+    assert _kernel_for(P, E, K, N) == _kernel_for(P, E, K + 8, N) == "ping-pong"
+    assert tn % walk == 0 and all(tn % w for w in (2, 3) if w < walk) and tiles - 116 >= 256 * walk  # (up to 116 tiles are cut)
+    run(loads, K, N, act="gelu", bias=True, slack=100)
+    g = torch.Generator().manual_seed(K + N)
+    x = torch.randn(P, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(E, N, K, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    d_loads = torch.tensor(loads, dtype=torch.int32, device="cuda")
+    order = torch.randperm(P, generator=g).cuda()
+    row_entries = (order + 1).to(torch.int32)  # row r of the layout holds cell order[r]
+    cells = torch.empty_like(x)
+    cells[order] = x
+
+    def product(pad, dtype=torch.bfloat16, **form):
+        xs, ws = (torch.nn.functional.pad(v, (0, pad)).contiguous() for v in (cells if form else x, w))
+        out = torch.full((P, N), float("nan"), dtype=dtype, device="cuda")
+        table = torch.tensor([ws[e].data_ptr() for e in range(E)], dtype=torch.int64, device="cuda")
+        grouped_linear(xs, out, table, None, d_loads, K + pad, N, **form)
+        torch.cuda.synchronize()
+        return out
+
+    want = product(8, torch.float32)
+    assert torch.equal(product(0, torch.float32).view(torch.int32), want.view(torch.int32))
+    assert torch.equal(product(0).float(), want.to(torch.bfloat16).float())
+    gathered = product(0, row_entries=row_entries, entries_per_cell=1, gather=True)
+    assert torch.equal(gathered.float(), want.to(torch.bfloat16).float())
+
+
 @pytest.mark.parametrize("T,E,K,N,k,cap,pad", [
     (16500, 4, 128, 2048, 1, 4140, False),   # overflow dropped, every expert with few rows over whole blocks
     (4500, 4, 320, 6912, 1, 1026, True),     # padded to the capacity: last blocks of two rows
