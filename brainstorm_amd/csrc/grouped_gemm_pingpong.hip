@@ -94,6 +94,7 @@ static_assert(kRound == 1 << kRoundBits);
 // is left to gain (98 blocks 2048 -> 8192, 12.25 rounds: 763 us cut, 756 not).
 constexpr int kFewRows = 128, kMostCut = 104, kMostCutOfFewRows = 116, kMostRounds = 10;
 constexpr int kUnitCols = 64;
+constexpr int kStreamed = 2 | 16;  // cache policy of a buffer store: nt sc1
 struct ListEnd {
   int moved, cut;  // row blocks of few rows put behind the list, tiles cut in all
 };
@@ -351,13 +352,15 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // ---- epilogue: bias + activation, bf16, 32 rows at a time through this wavefront's image -----
   // transposed accumulator: element r of tile (i, j) is output row 16 i + lane % 16, column (of the
   // wavefront's) 16 j + 4 * (lane / 16) + r, i.e. a lane holds 4 consecutive columns (8 bytes) of its row.
-  auto epilogue = [&](auto& acc, int first_row, int mine, int col_w, uint32_t images) {
+  // Rows and columns that are not there are left to the bounds of the buffer that is stored to, and without a bias nothing is added
+  // (a sum of products that starts at +0 is never -0).  With a branch for each row and a zero added, and so, us: 4 x 8000 rows 256 -> 1024 + GELU 31.5
+  // and 30.3, 16 x 2048 rows 1024 -> 4096 + GELU 252 and 247, 8 x 4096 rows 8192 -> 2048 746 and 736.
+  auto epilogue = [&](auto& acc, int first_row, int mine, int col_w, uint32_t images, auto with_bias) {
     constexpr int MT = sizeof(acc) / sizeof(acc[0]), NT = sizeof(acc[0]) / sizeof(acc[0][0]);
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane), "+s"(images));  // (else what follows from it is kept in registers all through the K loops of a walk)
     const int frag_row = lane & 15, frag_k = lane >> 4;
     const int row_w = row0 + first_row;
-    const global_bf16 bias = a.bias != nullptr ? (global_bf16)(a.bias[e]) : (global_bf16)nullptr;
     constexpr int kOutB = OUTF32 ? 4 : 2;                 // bytes of one output element
     constexpr int kChunk = 16 / kOutB;                    // elements of one 16-byte store
     constexpr int kCols = OUTF32 ? 32 : NT * 16;          // columns of an image
@@ -369,23 +372,30 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     auto slot = [](int row, int chunk) { return (chunk ^ (kChunksPerRow == 4 ? (row >> 2) & 3 : (row >> 1) & 7)) * 16; };
     constexpr int kRowsPerPass = kWave / kChunksPerRow;
     // the bias of this lane's columns, all loads in one round trip
+    constexpr bool kBias = decltype(with_bias)::value;
     bf16x4 bv[NT];
+    if constexpr (kBias) {
+      const global_bf16 bias = (global_bf16)(a.bias[e]);
   #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int col = col_w + j * 16 + 4 * frag_k;
-      bv[j] = bf16x4{};
-      if (bias != nullptr && col < a.N) bv[j] = *(global_bf16x4)(bias + col);
+      for (int j = 0; j < NT; ++j) {
+        const int col = col_w + j * 16 + 4 * frag_k;
+        bv[j] = bf16x4{};
+        if (col < a.N) bv[j] = *(global_bf16x4)(bias + col);
+      }
     }
+    const bool scatter = ROUTED && a.scatter != 0;
+    char* const out_b = OUTF32 ? reinterpret_cast<char*>(a.out_f32) : reinterpret_cast<char*>(a.out);
+    const uint32_t row_b = static_cast<uint32_t>(a.N) * kOutB;
+    const __amdgpu_buffer_rsrc_t to_rows = __builtin_amdgcn_make_buffer_rsrc(
+        out_b + static_cast<size_t>(row_w) * row_b, 0, static_cast<int>(max(mine, 0) * row_b), 0x00020000);
   #pragma unroll
     for (int i = 0; i < MT / 2; ++i) {
       if (i * 32 >= mine) break;  // wave-uniform
       // scattered rows: lane r of the pass holds the cell of row r (read again: LDS held operands)
       int cell = -1;
-      if constexpr (ROUTED) {
-        if (a.scatter && lane < min(32, mine - i * 32)) {
-          const int r = row_w + i * 32 + lane;
-          cell = routed_cell(a, e, r, r - row0 + seat0);
-        }
+      if (scatter && lane < min(32, mine - i * 32)) {
+        const int r = row_w + i * 32 + lane;
+        cell = routed_cell(a, e, r, r - row0 + seat0);
       }
   #pragma unroll
       for (int j0 = 0; j0 < NT; j0 += kCols / 16) {
@@ -393,10 +403,12 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
         for (int ii = 0; ii < 2; ++ii) {
   #pragma unroll
           for (int j = j0; j < j0 + kCols / 16; ++j) {
-            const bf16x4 b4 = bv[j];
             float v[4];
   #pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] = apply_act<ACT>(acc[2 * i + ii][j][q] + static_cast<float>(b4[q]));
+            for (int q = 0; q < 4; ++q) {
+              const float sum = acc[2 * i + ii][j][q];
+              v[q] = apply_act<ACT>(kBias ? sum + static_cast<float>(bv[j][q]) : sum);
+            }
             const int row = ii * 16 + frag_row, at = (16 * (j - j0) + 4 * frag_k) * kOutB;  // in the image
             char* const to = image + row * kImageRow + slot(row, at / 16) + at % 16;
             if constexpr (OUTF32) {
@@ -408,33 +420,36 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
           }
         }
         wave_fence();
-        const int rows_i = min(32, mine - i * 32);
         const int c = lane % kChunksPerRow, col = col_w + j0 * 16 + c * kChunk;
-        char* const out_b = OUTF32 ? reinterpret_cast<char*>(a.out_f32) : reinterpret_cast<char*>(a.out);
+        constexpr int kPasses = 32 / kRowsPerPass;
+        u32x4 held[kPasses];
   #pragma unroll
-        for (int p = 0; p < 32 / kRowsPerPass; ++p) {
-          const int rl = p * kRowsPerPass + lane / kChunksPerRow;
-          long row = row_w + i * 32 + rl;
-          bool live = rl < rows_i && col < a.N;
-          if constexpr (ROUTED) {
-            if (a.scatter) {
-              const int to = __shfl(cell, rl, kWave);
-              live = live && to >= 0;
-              row = to;
-            }
-          }
-          if (live) {
-            u32x4 v = *reinterpret_cast<const u32x4*>(image + rl * kImageRow + slot(rl, c));
-            if constexpr (ROUTED && !OUTF32) {
-              if (a.scatter) {  // the combine this store stands for adds the row to zero: -0 becomes +0
+        for (int p = 0; p < kPasses; ++p) {
+          const int row = p * kRowsPerPass + lane / kChunksPerRow;
+          held[p] = *reinterpret_cast<const u32x4*>(image + row * kImageRow + slot(row, c));
+        }
+        if (scatter) {
   #pragma unroll
-                for (int w = 0; w < 4; ++w) v[w] = plus_zero<BRT_BF16>(v[w]);
-              }
+          for (int p = 0; p < kPasses; ++p) {
+            const int to_row = __shfl(cell, p * kRowsPerPass + lane / kChunksPerRow, kWave);
+            if (to_row < 0 || col >= a.N) continue;
+            if constexpr (!OUTF32) {  // the combine this store stands for adds the row to zero: -0 becomes +0
+  #pragma unroll
+              for (int w = 0; w < 4; ++w) held[p][w] = plus_zero<BRT_BF16>(held[p][w]);
             }
-            u32x4* const to = reinterpret_cast<u32x4*>(out_b + (static_cast<size_t>(row) * a.N + col) * kOutB);
-            if (a.plain_out) *to = v;
-            else stream_out(v, to);
+            u32x4* const to = reinterpret_cast<u32x4*>(out_b + static_cast<size_t>(to_row) * row_b + col * kOutB);
+            if (a.plain_out) *to = held[p];
+            else stream_out(held[p], to);
           }
+        } else {
+          uint32_t at = col < a.N ? static_cast<uint32_t>(i * 32 + lane / kChunksPerRow) * row_b + col * kOutB : kOutOfRange;
+          auto store = [&](auto policy) {
+  #pragma unroll
+            for (int p = 0; p < kPasses; ++p, at += kRowsPerPass * row_b)
+              __builtin_amdgcn_raw_buffer_store_b128(held[p], to_rows, at, 0, decltype(policy)::value);
+          };
+          if (a.plain_out) store(std::integral_constant<int, 0>{});
+          else store(std::integral_constant<int, kStreamed>{});
         }
         wave_fence();
       }
@@ -565,7 +580,8 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
       if (mine > 0) {
         loop(std::true_type{});
         mfma_wait_states();
-        epilogue(acc, first_row, mine, n0 + tile_w * 32, 0);
+        if (a.bias != nullptr) epilogue(acc, first_row, mine, n0 + tile_w * 32, 0, std::true_type{});
+        else epilogue(acc, first_row, mine, n0 + tile_w * 32, 0, std::false_type{});
       } else {
         loop(std::false_type{});
       }
@@ -763,7 +779,8 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     if (left == 1) wait_loads_all();  // (of the requests of nothing: a workgroup does not end while a load into its LDS is under way)
     // The last M phase of both groups is over since group 0's last barrier, and the slot of the last activation rows, the next one to
     // be requested, holds the images: the two K-steps of the next tile that are under way or have landed lie in the others.
-    epilogue(acc, first_row, mine, n0 + wn * kNT * 16, a_load);
+    if (a.bias != nullptr) epilogue(acc, first_row, mine, n0 + wn * kNT * 16, a_load, std::true_type{});
+    else epilogue(acc, first_row, mine, n0 + wn * kNT * 16, a_load, std::false_type{});
     if (--left == 0) break;
     n0 += kBN;
     block_barrier();  // the images are read, their slot may be filled
@@ -829,8 +846,10 @@ int launch_pingpong(GemmArgs& a, hipStream_t st) {
 
 }  // namespace
 
-// Shapes the ping-pong tiles take: K of at least two K-steps of 64; every form but the weighted accumulate.
-bool pingpong_gemm_applies(const GemmArgs& a) { return a.gates == nullptr && a.K >= 2 * kBK; }
+// Shapes the ping-pong tiles take: K of at least two K-steps of 64, widths that keep the offsets inside a tile within 32 bits; every form but the
+// weighted accumulate.
+constexpr int kMostWidth = 1 << 20;
+bool pingpong_gemm_applies(const GemmArgs& a) { return a.gates == nullptr && a.K >= 2 * kBK && a.K <= kMostWidth && a.N <= kMostWidth; }
 
 template <int ACT>
 int launch_pingpong_form(GemmArgs& a, hipStream_t st) {
