@@ -29,8 +29,8 @@ struct GemmArgs {
   int tiles_n, tiles_m_max;
   int walk, groups_n;  // column tiles one workgroup walks, ceil(tiles_n / walk)
   int grid;                  // workgroups, 0 where no tile may be cut into units (ping-pong kernel)
-  uint32_t tiles_n_inverse, walk_inverse;  // (2^32 - 1) / tiles_n, / walk (ping-pong kernel)
-  int patch;           // workgroups in patch order (experts with several row blocks), see the kernel
+  uint32_t tiles_n_inverse, walk_inverse;  // (2^32 - 1) / tiles_n (ping-pong and few-rows kernel), / walk (ping-pong kernel)
+  int patch;           // workgroups in patch order, see the kernels
   // measurement aid (ping-pong kernel only): non-null, the workgroup of the first tile writes the
   // shader clocks (s_memtime) and the ticks of the constant 100 MHz counter (s_memrealtime) its
   // first wavefront spent in the K loop, and the number of K-steps, into clocks[0..2]

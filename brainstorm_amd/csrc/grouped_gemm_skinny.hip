@@ -90,6 +90,7 @@ __device__ __forceinline__ void wait_lds() {
 }
 
 constexpr int kWaves = 4;
+constexpr int kXcds = 8;
 
 template <int XR, int NT, int D, bool X32>
 struct Shape {
@@ -117,15 +118,36 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = a.K;
 
-  // ---- which tile: column tiles of a row block are consecutive, so they spread over the XCDs -----
-  const int block = blockIdx.x / a.tiles_n, n0 = (blockIdx.x - block * a.tiles_n) * H::kBN;
+  // ---- which tile: an entry of the list of tiles (experts, their row blocks, column tiles).  The workgroups go to the XCDs in
+  // turn, so in the order of the list the column tiles of a row block spread over the XCDs; in patch order every XCD takes an
+  // eighth of the list, whose rows of x it reads alone.
+  int m = lane < a.E ? a.loads[lane] : 0;
+  uint64_t wp = lane < a.E ? reinterpret_cast<uint64_t>(a.w[lane]) : 0;
+  auto row_blocks = [](int rows_of_e) { return (rows_of_e + XR - 1) / XR; };
+  int block, column, idle = 0;  // idle: behind which many workgroups without a tile this one stands
+  if (a.patch) {
+    int total = read_lane(wave_inclusive_scan(row_blocks(m)), kWave - 1);
+    for (int base = kWave; base < a.E; base += kWave)
+      total += read_lane(wave_inclusive_scan(base + lane < a.E ? row_blocks(a.loads[base + lane]) : 0), kWave - 1);
+    const int tiles = min(total, a.tiles_m_max) * a.tiles_n, share = (tiles + kXcds - 1) / kXcds;
+    const int xcd = blockIdx.x % kXcds, turn = blockIdx.x / kXcds;
+    const int before = min(xcd * share, tiles), own = min(share, tiles - before);
+    const unsigned tile = before + turn;
+    block = __umulhi(tile, a.tiles_n_inverse), column = tile - block * a.tiles_n;
+    if (column >= a.tiles_n) ++block, column -= a.tiles_n;
+    if (turn >= own) block = total, column = 0, idle = xcd * (gridDim.x / kXcds) - before + turn - own;
+  } else {
+    block = blockIdx.x / a.tiles_n, column = blockIdx.x - block * a.tiles_n;
+  }
+  const int n0 = column * H::kBN;
   int e = -1, row0 = 0, rows = 0, seat0 = 0, carry_t = 0, carry_m = 0;
   const __bf16* w_e = nullptr;
   for (int base = 0; base < a.E; base += kWave) {
-    const int el = base + lane;
-    const int m = el < a.E ? a.loads[el] : 0;
-    const uint64_t wp = el < a.E ? reinterpret_cast<uint64_t>(a.w[el]) : 0;
-    const int blocks = (m + XR - 1) / XR;
+    if (base != 0) {
+      m = base + lane < a.E ? a.loads[base + lane] : 0;
+      wp = base + lane < a.E ? reinterpret_cast<uint64_t>(a.w[base + lane]) : 0;
+    }
+    const int blocks = row_blocks(m);
     const int incl_t = wave_inclusive_scan(blocks), incl_m = wave_inclusive_scan(m);
     const int first = carry_t + incl_t - blocks;
     const unsigned long long hit = __ballot(block >= first && block < first + blocks);
@@ -147,7 +169,7 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
     // Row blocks past the last one clear the tags of the rows no path owns, XR rows each: the grid
     // holds P / XR + min(E, P) of them (rounded up), the experts use at most (total + (XR - 1) * used experts) / XR.
     if (ROUTED && a.row_tags_out != nullptr && n0 == 0) {
-      const long r = static_cast<long>(carry_m) + static_cast<long>(block - carry_t) * XR + tid;
+      const long r = static_cast<long>(carry_m) + static_cast<long>(block - carry_t + idle) * XR + tid;
       if (tid < XR && r < a.P) a.row_tags_out[r] = 0;
     }
     return;
@@ -379,15 +401,39 @@ __global__ __launch_bounds__(kWaves * kWave) void grouped_gemm_skinny_kernel(Gem
   }
 }
 
+// Estimated tiles of `block` x 64 of the result; an expert's last row block is taken as half full.
+double narrow_tiles(const GemmArgs& a, int block) {
+  const long used = std::min(a.E, a.P);
+  const double rows = static_cast<double>(a.P) / used;
+  return used * (rows > block ? rows / block + 0.5 : 1.0) * ((a.N + 63) / 64);
+}
+
+// Where the tiles are dealt in patch order.  In the order of the list every XCD's L2 draws all rows of x: eight times their bytes, beside
+// weights that come once.  Dealt by expert they come once too: 12 x 95 rows 1280 -> 320 10.9 -> 7.4 us, 8 x 97 rows 4160 -> 1040
+// 36.5 -> 27.6, 16 x 64 fp32 rows 2048 -> 512 17.0 -> 13.9.  Taken where the seven copies saved are a good part of the bytes (8 times the rows of x
+// a fifth of the weights or more), of contracting shapes of more than one row block per expert and a tile for most CUs.  Of 74
+// drawn shapes that it takes the mean is 1.18 times as fast in patch order, 3 are more than 2 % slower: weight rows 8 KB apart (8 x 115 skewed
+// rows 4096 -> 1024 32.9 and 36.2).  Not taken: few tiles, which pay 0.1 us more for finding theirs (4 x 104 rows 768 -> 768 5.9 and 6.1),
+// expanding shapes, whose output lines and weights the XCDs then write and read far apart (4 x 120 rows 2048 -> 8192 42 and 46), and
+// weights of 0.14 GB, of part-filled lines 40 MB, or more, likewise (16 x 123 rows 3008 -> 1504 54 and 57, 16 x 60 rows 2096 -> 1048 31 and 34).
+bool experts_stay_on_an_xcd(const GemmArgs& a) {
+  const long used = std::min(a.E, a.P);
+  return a.N <= a.K && a.P > 32 * used && 2.0 * used * a.N * a.K < (a.K % kBK == 0 ? 1.4e8 : 4e7) && narrow_tiles(a, 32) >= 150 &&
+         (a.x_f32 ? 16.0 : 8.0) * a.P >= 0.2 * used * a.N;
+}
+
 template <int XR, int NT, int D, int ACT, bool ROUTED, bool OUTF32, bool X32>
 int launch(GemmArgs& a, hipStream_t st) {
   using H = Shape<XR, NT, D, X32>;
   a.tiles_n = (a.N + H::kBN - 1) / H::kBN;
+  a.tiles_n_inverse = 0xffffffffu / static_cast<uint32_t>(a.tiles_n);
   // the sum over experts of ceil(M_e / XR) never exceeds P / XR + min(E, P)
   const long blocks = (static_cast<long>(a.P) + XR - 1) / XR + std::min(a.E, a.P);
+  a.tiles_m_max = static_cast<int>(blocks);
+  a.patch = experts_stay_on_an_xcd(a);
   auto* fn = &grouped_gemm_skinny_kernel<XR, NT, D, ACT, ROUTED, OUTF32, X32>;
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(fn), H::kLds); rc != BRT_OK) return rc;
-  hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks * a.tiles_n)), dim3(kWaves * kWave), H::kLds, st, a);
+  hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>((blocks * a.tiles_n + kXcds - 1) / kXcds * kXcds)), dim3(kWaves * kWave), H::kLds, st, a);
   return check_launch("grouped_gemm_skinny_kernel");
 }
 
@@ -457,12 +503,6 @@ bool skinny_gemm_applies(const GemmArgs& a) {
 }
 
 namespace {
-// Estimated tiles of `block` x 64 of the result; an expert's last row block is taken as half full.
-double narrow_tiles(const GemmArgs& a, int block) {
-  const long used = std::min(a.E, a.P);
-  const double rows = static_cast<double>(a.P) / used;
-  return used * (rows > block ? rows / block + 0.5 : 1.0) * ((a.N + 63) / 64);
-}
 bool takes_64_rows(const GemmArgs& a) { return a.P > 32l * std::min(a.E, a.P) && narrow_tiles(a, 64) >= 192; }
 }  // namespace
 

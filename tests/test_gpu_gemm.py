@@ -883,6 +883,8 @@ def _few_rows_tile(P, E, K, N):
     (1000, 20, 136, 776, 55, False, (64, 64, 3)),          # blocks of 64 rows and their remainders
     (1000, 20, 328, 776, 70, True, (64, 64, 3)),
     (1000, 20, 1096, 776, 60, True, (64, 64, 4)),
+    (2400, 70, 264, 200, 40, False, (64, 64, 3)),          # dealt by expert, more than 64 of them
+    (600, 9, 1096, 456, 70, False, (32, 64, 5)),           # dealt by expert, eighths of the list end inside an expert
     (50, 20, 1224, 1032, 60, True, (64, 64, 4)),           # loads name slots past the tag matrix
 ])
 def test_every_form_of_the_row_streaming_kernels(T, E, K, N, cap, pad, kernel):
