@@ -38,6 +38,7 @@ __all__ = [
     "split_fused_cells_to_paths",
     "fuse_split_cells_from_paths",
     "combine_with_indices_and_loads",
+    "combine_flows",
     "combine_with_src_indices",
     "gate_topk",
     "route_by_path",
@@ -613,6 +614,16 @@ def _sum_rows_by_index(in_data, index, n, shape):
         zeros = torch.zeros(shape, dtype=in_data.dtype, device=in_data.device)
         return torch.scatter_reduce(zeros, 0, expanded, in_data, "sum")
     return _lib.native().sum_rows_by_index(in_data, index, n)
+
+
+def combine_flows(datas: List[torch.Tensor], tags: List[torch.Tensor]) -> Optional[tuple]:
+    """``fuse_split_cells_from_paths`` (router.cc:348-369) and the tag-mode combine (router.cc:449-472) of its result, from the
+    flows where they are: ``(rows, tags, number of tags)``, bit for bit, or None where the general way is to be taken (other
+    types, more than 64 flows or 8192 rows, tags too far apart, a compiler, tracer or mode that looks on)."""
+    if torch.compiler.is_compiling():
+        return None
+    native = _lib.native_or_none()
+    return None if native is None else native.combine_flows(datas, tags)
 
 
 # legacy name (sample/cpp/router.ipynb:258-266) of the seat-index combine

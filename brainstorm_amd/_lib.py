@@ -111,6 +111,14 @@ SIGNATURES = {
         _c_int,
         [_c_ptr, _c_int, ctypes.c_long, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     ),
+    "brt_hip_unique_tags_of_flows": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
+    ),
+    "brt_hip_combine_flows": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
+    ),
     "brt_hip_combine_by_index_workspace_bytes": (_c_size, [_c_int, _c_int]),
     "brt_hip_combine_by_index": (
         _c_int,

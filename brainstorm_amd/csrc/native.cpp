@@ -646,44 +646,67 @@ bool seen_within(const int32_t* word, std::chrono::microseconds limit) {
   return false;
 }
 
-// Copies from the device on the current stream into pinned memory and waits for the copy (other Python
-// threads run meanwhile).  Few words are stored there by a kernel and watched for; more, or a stream that is being
-// captured (where reading back is an error), take the runtime's copy and wait.
+// Pinned memory for a few words that a kernel on the current stream stores, with a last one behind them that says that they are there
+// (other Python threads run while this one waits).  Not watched: more words than a kernel stores quickly, or a stream that
+// is being captured (where reading back is an error); these take the runtime's copy and wait.
+struct HostWords {
+  at::DataPtr host;
+  hipStream_t st;
+  size_t bytes;
+  const char* what;
+  int32_t* seen_from_device = nullptr;  // non-null: watched
+
+  HostWords(const Tensor& t, size_t n, const char* name) : bytes(n), what(name) {
+    constexpr size_t kFewBytes = 4096;
+    host = at::getHostAllocator(at::kCUDA)->allocate(bytes + 4);
+    st = c10::hip::getCurrentHIPStream(t.get_device()).stream();
+    if (bytes > kFewBytes || bytes % 4 != 0) return;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    void* address = nullptr;
+    if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
+        hipHostGetDevicePointer(&address, host.get(), 0) != hipSuccess) {
+      (void)hipGetLastError();  // what asking left behind, if anything
+      return;
+    }
+    seen_from_device = static_cast<int32_t*>(address);
+    __atomic_store_n(word(), 0, __ATOMIC_RELEASE);
+  }
+  int32_t* word() const { return static_cast<int32_t*>(host.get()) + bytes / 4; }
+
+  // Waits for the words of a watched stream; of another, copies them from the device first.
+  const void* read(const Tensor& t) {
+    hipError_t rc = hipSuccess;
+    bool seen = false;
+    if (seen_from_device != nullptr) {
+      Py_BEGIN_ALLOW_THREADS
+      seen = seen_within(word(), std::chrono::microseconds(500));
+      Py_END_ALLOW_THREADS
+    } else {
+      rc = hipMemcpyAsync(host.get(), ptr(t), bytes, hipMemcpyDeviceToHost, st);
+    }
+    if (rc == hipSuccess && !seen) {
+      Py_BEGIN_ALLOW_THREADS
+      rc = hipStreamSynchronize(st);
+      Py_END_ALLOW_THREADS
+    }
+    if (rc != hipSuccess) {
+      (void)hipGetLastError();  // reported here, not by the next launch that looks for an error
+      runtime_error(std::string(what) + ": " + hipGetErrorString(rc));
+    }
+    return host.get();
+  }
+};
+
+// Copies from the device on the current stream into pinned memory and waits for the copy.
 at::DataPtr read_back(const Tensor& t, size_t bytes, const char* what) {
-  constexpr size_t kFewBytes = 4096;
-  at::DataPtr host = at::getHostAllocator(at::kCUDA)->allocate(bytes + 4);
-  const hipStream_t st = c10::hip::getCurrentHIPStream(t.get_device()).stream();
-  void* seen_from_device = nullptr;
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  bool watch = bytes <= kFewBytes && bytes % 4 == 0;
-  if (watch && (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
-                hipHostGetDevicePointer(&seen_from_device, host.get(), 0) != hipSuccess)) {
-    (void)hipGetLastError();  // what asking left behind, if anything
-    watch = false;
-  }
-  hipError_t rc = hipSuccess;
-  if (watch) {
-    int32_t* const word = static_cast<int32_t*>(host.get()) + bytes / 4;
-    __atomic_store_n(word, 0, __ATOMIC_RELEASE);
+  HostWords words(t, bytes, what);
+  if (words.seen_from_device != nullptr) {
     ++g_calls;
-    if (brt_hip_copy_to_host(iptr(t), static_cast<int32_t*>(seen_from_device), static_cast<int>(bytes / 4), st) != BRT_OK)
+    if (brt_hip_copy_to_host(iptr(t), words.seen_from_device, static_cast<int>(bytes / 4), words.st) != BRT_OK)
       runtime_error(std::string(what) + ": " + brt_hip_last_error());
-    Py_BEGIN_ALLOW_THREADS
-    watch = seen_within(word, std::chrono::microseconds(500));
-    Py_END_ALLOW_THREADS
-  } else {
-    rc = hipMemcpyAsync(host.get(), ptr(t), bytes, hipMemcpyDeviceToHost, st);
   }
-  if (rc == hipSuccess && !watch) {
-    Py_BEGIN_ALLOW_THREADS
-    rc = hipStreamSynchronize(st);
-    Py_END_ALLOW_THREADS
-  }
-  if (rc != hipSuccess) {
-    (void)hipGetLastError();  // reported here, not by the next launch that looks for an error
-    runtime_error(std::string(what) + ": " + hipGetErrorString(rc));
-  }
-  return host;
+  words.read(t);
+  return std::move(words.host);
 }
 
 // The values of an int32 vector as a list.
@@ -837,6 +860,55 @@ PyObject* sum_rows_by_index(const Args& a) {
   return wrap(out);
 }
 
+// The rows of the flows (a list), their tags (a list of vectors) -> (the rows of every tag added up in the order of the flows, the tags
+// in ascending order, their number as an int32 vector), or None where a launch over the flows themselves does not take them
+PyObject* combine_flows(const Args& a) {
+  if (!PyList_Check(a.v[0]) || !PyList_Check(a.v[1])) return none();
+  const Py_ssize_t count = PyList_GET_SIZE(a.v[0]);
+  if (count < 1 || count > BRT_MAX_FLOWS || PyList_GET_SIZE(a.v[1]) != count) return none();
+  std::vector<Tensor> datas(count), tags(count);
+  std::vector<int32_t> rows(count);
+  int64_t n = 0;
+  for (Py_ssize_t f = 0; f < count; ++f) {
+    PyObject *const d = PyList_GET_ITEM(a.v[0], f), *const t = PyList_GET_ITEM(a.v[1], f);
+    if (!THPVariable_CheckExact(d) || !THPVariable_CheckExact(t)) return none();
+    datas[f] = THPVariable_Unpack(d), tags[f] = THPVariable_Unpack(t);
+    for (const Tensor* x : {&datas[f], &tags[f]})
+      if (!unobserved(*x) || !x->is_cuda() || x->layout() != at::kStrided || x->is_neg() || x->dim() < 1 || x->device() != datas[0].device() ||
+          x->key_set().has(c10::DispatchKey::FuncTorchBatched))
+        return none();
+    if (datas[f].scalar_type() != datas[0].scalar_type() || tags[f].scalar_type() != tags[0].scalar_type() ||
+        datas[f].sizes().slice(1) != datas[0].sizes().slice(1) || tags[f].dim() != 1 || tags[f].size(0) != datas[f].size(0))
+      return none();
+    n += datas[f].size(0);
+    if (n > BRT_FLOW_ROWS_MAX) return none();
+    rows[f] = static_cast<int32_t>(datas[f].size(0));
+  }
+  const int type = code_of(datas[0].scalar_type());
+  const bool narrow = tags[0].scalar_type() == at::kInt;
+  const int64_t cell = c10::multiply_integers(datas[0].sizes().slice(1));
+  if (n < 2 || type < 0 || (!narrow && tags[0].scalar_type() != at::kLong) || cell < 1 || cell > INT32_MAX) return none();
+  const c10::DeviceGuard guard(datas[0].device());
+  std::vector<const void*> data_of(count), tags_of(count);
+  for (Py_ssize_t f = 0; f < count; ++f) {
+    datas[f] = dense(datas[f]), tags[f] = dense(tags[f]);
+    data_of[f] = ptr(datas[f]), tags_of[f] = ptr(tags[f]);
+    if (rows[f] > 0 && (data_of[f] == nullptr || tags_of[f] == nullptr)) return none();
+  }
+  const Tensor& like = datas[0];
+  Tensor unique = empty({n}, tags[0].scalar_type(), like), number = empty({1}, at::kInt, like);
+  const Tensor lists = empty({2 * n}, at::kInt, like), found = empty({3}, at::kLong, like);
+  int32_t *const head = iptr(lists), *const next = head + n;
+  HostWords words(like, 24, "reading the number of tags");
+  check(brt_hip_unique_tags_of_flows(tags_of.data(), rows.data(), count, narrow ? 32 : 64, ptr(unique), head, next, iptr(number),
+                                     static_cast<int64_t*>(ptr(found)), words.seen_from_device, words.st));
+  const int64_t n_out = *static_cast<const int64_t*>(words.read(found));
+  if (n_out < 0) return none();
+  Tensor out = empty(rows_of(like, n_out), like.scalar_type(), like);
+  check(brt_hip_combine_flows(data_of.data(), rows.data(), count, ptr(out), head, next, cell, n_out, type, words.st));
+  return tuple(wrap(out), wrap(unique.narrow(0, 0, n_out)), wrap(number));
+}
+
 // value, like -> [value] as an int32 vector on like's device, without a wait
 PyObject* one_value(const Args& a) {
   const Tensor& like = as_it_is(a.v[1]);
@@ -872,7 +944,7 @@ PyMethodDef methods[] = {
     BRT_ENTRY(grouped_linear_f32, 16), BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5),        BRT_ENTRY(int_list, 1),
     BRT_ENTRY(ordinary, 3),         BRT_ENTRY(plain, 1),            BRT_ENTRY(of_class, 2),            BRT_ENTRY(matrix, 4),
     BRT_ENTRY(grid, 5),                BRT_ENTRY(split_rows, 4),
-    BRT_ENTRY(sum_rows_by_index, 3), BRT_ENTRY(one_value, 2),         BRT_ENTRY(unique_tags, 1),      BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
+    BRT_ENTRY(sum_rows_by_index, 3), BRT_ENTRY(combine_flows, 2), BRT_ENTRY(one_value, 2),         BRT_ENTRY(unique_tags, 1),      BRT_ENTRY(calls, 0),            {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "brt_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

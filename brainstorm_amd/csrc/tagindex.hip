@@ -15,6 +15,7 @@
 //     not depend on the order in which the atomics landed and every output row is written once.
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "common.hpp"
 #include "rows.hpp"
@@ -127,11 +128,11 @@ __device__ __forceinline__ void key_batch(const K* __restrict__ keys, int n, int
     v[j] = keys[min(base + j * kScanThreads + static_cast<int>(threadIdx.x), n - 1)];  // n >= 1
 }
 
-// The first batch, `held`, stays in registers for the inverse at the end.  The number of unique keys is
-// returned to the last thread.
+// The rank of every tag in the table, and the unique tags.  The number of unique keys is returned to the last thread; the first
+// batch of keys, `held`, is in registers.
 template <typename K>
-__device__ __forceinline__ int unique_in_lds(const K* __restrict__ keys, int n, long lo, int range, const K (&held)[kKeysInFlight],
-                                             K* __restrict__ unique, int64_t* __restrict__ inverse, int* s_table) {
+__device__ __forceinline__ int ranks_in_lds(const K* __restrict__ keys, int n, long lo, int range, const K (&held)[kKeysInFlight],
+                                            K* __restrict__ unique, int* s_table) {
   __shared__ int s_wave[kScanThreads / kWave];
   const int tid = threadIdx.x, wave = tid >> 6;
   for (int i = tid; i < range; i += kScanThreads) s_table[i] = 0;
@@ -169,6 +170,15 @@ __device__ __forceinline__ int unique_in_lds(const K* __restrict__ keys, int n, 
     rank += flag;
   }
   __syncthreads();
+  return rank;
+}
+
+// ... and the inverse, for which the first batch of keys stays in registers.
+template <typename K>
+__device__ __forceinline__ int unique_in_lds(const K* __restrict__ keys, int n, long lo, int range, const K (&held)[kKeysInFlight],
+                                             K* __restrict__ unique, int64_t* __restrict__ inverse, int* s_table) {
+  const int tid = threadIdx.x;
+  const int rank = ranks_in_lds(keys, n, lo, range, held, unique, s_table);
   for (int base = 0; base < n; base += kKeysInFlight * kScanThreads) {
     K v[kKeysInFlight];
     if (base == 0) {
@@ -204,10 +214,18 @@ __global__ __launch_bounds__(kScanThreads) void unique_small_kernel(const K* __r
 // library calls took three launches and a wait of the host before this one (gathering 2048 cells of 4 flows by
 // their tags 243 -> 166 us).
 template <typename K>
+__device__ __forceinline__ void range_of_workgroup(K& lo, K& hi) {
+  __shared__ K s_lo[kScanThreads / kWave], s_hi[kScanThreads / kWave];
+  for (int d = 1; d < kWave; d <<= 1) lo = min(lo, __shfl_xor(lo, d, kWave)), hi = max(hi, __shfl_xor(hi, d, kWave));
+  if (lane_id() == 0) s_lo[threadIdx.x >> 6] = lo, s_hi[threadIdx.x >> 6] = hi;
+  __syncthreads();
+  for (int w = 0; w < kScanThreads / kWave; ++w) lo = min(lo, s_lo[w]), hi = max(hi, s_hi[w]);
+}
+
+template <typename K>
 __global__ __launch_bounds__(kScanThreads) void unique_whole_kernel(const K* __restrict__ keys, int n, K* __restrict__ unique,
                                                                     int64_t* __restrict__ inverse, int64_t* __restrict__ found) {
   extern __shared__ int s_table[];
-  __shared__ K s_lo[kScanThreads / kWave], s_hi[kScanThreads / kWave];
   K held[kKeysInFlight];
   key_batch(keys, n, 0, held);
   K lo = held[0], hi = held[0];
@@ -221,10 +239,7 @@ __global__ __launch_bounds__(kScanThreads) void unique_whole_kernel(const K* __r
     key_batch(keys, n, base, v);
     take(v);
   }
-  for (int d = 1; d < kWave; d <<= 1) lo = min(lo, __shfl_xor(lo, d, kWave)), hi = max(hi, __shfl_xor(hi, d, kWave));
-  if (lane_id() == 0) s_lo[threadIdx.x >> 6] = lo, s_hi[threadIdx.x >> 6] = hi;
-  __syncthreads();
-  for (int w = 0; w < kScanThreads / kWave; ++w) lo = min(lo, s_lo[w]), hi = max(hi, s_hi[w]);
+  range_of_workgroup(lo, hi);
   const uint64_t span = static_cast<uint64_t>(hi) - static_cast<uint64_t>(lo);  // range - 1, whatever the signs
   const bool last = threadIdx.x == kScanThreads - 1;
   if (last) found[1] = lo, found[2] = hi;
@@ -264,8 +279,89 @@ __global__ __launch_bounds__(kScanThreads) void clear_and_link_kernel(const K* _
   }
 }
 
+// Rows that lie in several buffers, one behind the other: row p is row p - start[f] of the buffer of flow f.
+constexpr int kMaxFlows = BRT_MAX_FLOWS, kFlowRows = BRT_FLOW_ROWS_MAX;
+static_assert(kMaxFlows == kWave && kFlowRows == kKeysInFlight * kScanThreads, "a lane per flow, a thread's keys in registers");
+struct Flows {
+  const void* rows[kMaxFlows];
+  int start[kMaxFlows + 1];  // start[count] and all behind it: the number of rows
+  int count;
+};
+
+// Unique tags, the lists of the rows behind every one of them (as link_rows_kernel makes them) and their number, for the tags of
+// several flows, in one launch of one workgroup: up to kFlowRows tags, which stay in registers, and a range that the table
+// holds, which then serves as the heads of the lists.  found and its copy in host memory are {number or -1, smallest,
+// largest}; a word behind the latter tells the host that it is whole.  Bound by latency.  Concatenating tags and rows, unique,
+// reading its number back, clearing the heads, linking and a fill were eight launches, and 10 of 48 us of kernels went into copies of
+// rows: 2048 fp32 cells of 512 elements over 4 flows, two each, scattered and gathered 101 -> 74 us.
+template <typename K>
+__global__ __launch_bounds__(kScanThreads) void unique_flows_kernel(Flows flows, K* __restrict__ unique, int* __restrict__ head,
+                                                                    int* __restrict__ next, int* __restrict__ number,
+                                                                    int64_t* __restrict__ found, int* host) {
+  extern __shared__ int s_table[];
+  __shared__ const K* s_rows[kMaxFlows];
+  __shared__ int s_start[kMaxFlows];
+  __shared__ int s_count;
+  const int tid = threadIdx.x, n = flows.start[kMaxFlows];
+  if (tid < kMaxFlows) {
+    s_rows[tid] = static_cast<const K*>(flows.rows[tid]);
+    s_start[tid] = flows.start[tid];
+  }
+  __syncthreads();
+  K held[kKeysInFlight];
+#pragma unroll
+  for (int j = 0; j < kKeysInFlight; ++j) {
+    const int i = min(j * kScanThreads + tid, n - 1);
+    int f = 0;  // the last flow that starts at or before i: the one that holds it
+#pragma unroll
+    for (int step = kMaxFlows / 2; step != 0; step >>= 1) f += s_start[f + step] <= i ? step : 0;
+    held[j] = s_rows[f][i - s_start[f]];
+  }
+  K lo = held[0], hi = held[0];
+#pragma unroll
+  for (int j = 1; j < kKeysInFlight; ++j) lo = min(lo, held[j]), hi = max(hi, held[j]);
+  range_of_workgroup(lo, hi);
+  const uint64_t span = static_cast<uint64_t>(hi) - static_cast<uint64_t>(lo);
+  int count = -1;
+  if (span < kSmallRange)
+    count = ranks_in_lds<K>(nullptr, n, static_cast<long>(lo), static_cast<int>(span) + 1, held, unique, s_table);
+  if (tid == kScanThreads - 1) {
+    s_count = count;
+    const int64_t out[3] = {count, static_cast<int64_t>(lo), static_cast<int64_t>(hi)};
+    *number = count;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      found[i] = out[i];
+      if (host != nullptr) {
+        host[2 * i] = static_cast<int>(out[i]);
+        host[2 * i + 1] = static_cast<int>(out[i] >> 32);
+      }
+    }
+    if (host != nullptr) {
+      __threadfence_system();
+      __hip_atomic_store(host + 6, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+  if (span >= kSmallRange) return;
+  int rank[kKeysInFlight];
+#pragma unroll
+  for (int j = 0; j < kKeysInFlight; ++j) rank[j] = s_table[static_cast<long>(held[j]) - static_cast<long>(lo)];
+  __syncthreads();
+  count = s_count;
+  for (int r = tid; r < count; r += kScanThreads) s_table[r] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kKeysInFlight; ++j) {
+    const int p = j * kScanThreads + tid;
+    if (p < n) next[p] = __hip_atomic_exchange(&s_table[rank[j]], p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __syncthreads();
+  for (int r = tid; r < count; r += kScanThreads) head[r] = s_table[r];
+}
+
+struct NoFlows {};
 struct SumArgs {
-  const void* src;
+  const void* src;  // (FLOWS: unused)
   void* dst;
   const int* head;
   const int* next;
@@ -276,8 +372,10 @@ struct SumArgs {
 // (lane i holds the i-th row met), ranked against each other and moved to ascending order with
 // one cross-lane permute; a list longer than a wavefront is summed by repeated search instead
 // (for every next row, walk the list for the smallest row number above the last one).
-template <int BYTES, int IN_DT, int OUT_DT>
-__global__ __launch_bounds__(256) void sum_rows_by_index_kernel(SumArgs a) {
+// FLOWS: the rows lie in several buffers; a lane keeps the first row and the address of a flow, and the flow of a row is found
+// with one ballot.
+template <int BYTES, int IN_DT, int OUT_DT, bool FLOWS>
+__global__ __launch_bounds__(256) void sum_rows_by_index_kernel(SumArgs a, std::conditional_t<FLOWS, Flows, NoFlows> flows) {
   using U = typename Unit<BYTES>::type;
   constexpr int NE = BYTES / elem_bytes(IN_DT);
   constexpr int OUT_BYTES = NE * elem_bytes(OUT_DT);
@@ -287,6 +385,22 @@ __global__ __launch_bounds__(256) void sum_rows_by_index_kernel(SumArgs a) {
   if (r >= a.n_out) return;
   const U* __restrict__ src = static_cast<const U*>(a.src);
   char* __restrict__ dst = static_cast<char*>(a.dst) + static_cast<size_t>(r) * a.cpr * OUT_BYTES;
+  int flow_start = 0;
+  uint64_t flow_rows = 0;
+  if constexpr (FLOWS) {
+    flow_start = flows.start[lane];
+    flow_rows = reinterpret_cast<uint64_t>(flows.rows[lane]);
+  }
+  auto row = [&](int p) -> const U* {  // p: the same in the whole wavefront
+    if constexpr (FLOWS) {
+      const int f = __popcll(__ballot(flow_start <= p)) - 1;  // the last flow that starts at or before p
+      const uint64_t from = static_cast<uint64_t>(static_cast<uint32_t>(read_lane(static_cast<int>(flow_rows), f))) |
+                            static_cast<uint64_t>(static_cast<uint32_t>(read_lane(static_cast<int>(flow_rows >> 32), f))) << 32;
+      return reinterpret_cast<const U*>(from) + static_cast<size_t>(p - read_lane(flow_start, f)) * a.cpr;
+    } else {
+      return src + static_cast<size_t>(p) * a.cpr;
+    }
+  };
 
   int cur = __builtin_amdgcn_readfirstlane(a.head[r]);
   int count = 0, mine = INT_MAX;
@@ -317,8 +431,8 @@ __global__ __launch_bounds__(256) void sum_rows_by_index_kernel(SumArgs a) {
 #pragma unroll
         for (int u = 0; u < kAhead; ++u) {
           if (i0 + u < count) {
-            const int p = read_lane(ordered, i0 + u);
-            if (live) val[u] = src[static_cast<size_t>(p) * a.cpr + off];
+            const U* const from = row(read_lane(ordered, i0 + u));
+            if (live) val[u] = from[off];
           }
         }
 #pragma unroll
@@ -342,9 +456,10 @@ __global__ __launch_bounds__(256) void sum_rows_by_index_kernel(SumArgs a) {
         }
         if (best == INT_MAX) break;
         last = best;
+        const U* const from = row(best);
         if (live) {
           float x[NE];
-          unpack<IN_DT, BYTES>(src[static_cast<size_t>(best) * a.cpr + off], x);
+          unpack<IN_DT, BYTES>(from[off], x);
 #pragma unroll
           for (int q = 0; q < NE; ++q) acc[q] += x[q];
         }
@@ -356,14 +471,32 @@ __global__ __launch_bounds__(256) void sum_rows_by_index_kernel(SumArgs a) {
   }
 }
 
-template <int IN_DT, int OUT_DT>
-void launch_sum(int unit, const SumArgs& a, hipStream_t st) {
+template <int IN_DT, int OUT_DT, typename F = NoFlows>
+void launch_sum(int unit, const SumArgs& a, hipStream_t st, const F& flows = {}) {
   const dim3 grid((a.n_out + 3) / 4), block(256);
-  if (unit == 16) hipLaunchKernelGGL((sum_rows_by_index_kernel<16, IN_DT, OUT_DT>), grid, block, 0, st, a);
-  else if (unit == 8) hipLaunchKernelGGL((sum_rows_by_index_kernel<8, IN_DT, OUT_DT>), grid, block, 0, st, a);
-  else if (unit == 4) hipLaunchKernelGGL((sum_rows_by_index_kernel<4, IN_DT, OUT_DT>), grid, block, 0, st, a);
+  constexpr bool kFlows = std::is_same_v<F, Flows>;
+  if (unit == 16) hipLaunchKernelGGL((sum_rows_by_index_kernel<16, IN_DT, OUT_DT, kFlows>), grid, block, 0, st, a, flows);
+  else if (unit == 8) hipLaunchKernelGGL((sum_rows_by_index_kernel<8, IN_DT, OUT_DT, kFlows>), grid, block, 0, st, a, flows);
+  else if (unit == 4) hipLaunchKernelGGL((sum_rows_by_index_kernel<4, IN_DT, OUT_DT, kFlows>), grid, block, 0, st, a, flows);
   else if constexpr (IN_DT != BRT_F32)
-    hipLaunchKernelGGL((sum_rows_by_index_kernel<2, IN_DT, OUT_DT>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((sum_rows_by_index_kernel<2, IN_DT, OUT_DT, kFlows>), grid, block, 0, st, a, flows);
+}
+
+// The flows of a launch: false where a row count is negative, a flow with rows has no address, or they are too many.
+bool collect_flows(const void* const* rows, const int32_t* counts, int flow_num, Flows* out) {
+  if (rows == nullptr || counts == nullptr || flow_num < 1 || flow_num > kMaxFlows) return false;
+  long start = 0;
+  for (int f = 0; f < flow_num; ++f) {
+    if (counts[f] < 0 || (counts[f] > 0 && rows[f] == nullptr)) return false;
+    out->rows[f] = rows[f];
+    out->start[f] = static_cast<int>(start);
+    start += counts[f];
+    if (start > INT_MAX) return false;
+  }
+  for (int f = flow_num; f < kMaxFlows; ++f) out->rows[f] = nullptr;
+  for (int f = flow_num; f <= kMaxFlows; ++f) out->start[f] = static_cast<int>(start);
+  out->count = flow_num;
+  return true;
 }
 
 long scan_blocks(long range) { return (range + kScanChunk - 1) / kScanChunk; }
@@ -462,6 +595,56 @@ extern "C" int brt_hip_unique_tags_whole(const void* tags, int tag_bits, long n,
     hipLaunchKernelGGL(unique_whole_kernel<int64_t>, dim3(1), dim3(kScanThreads), lds, as_stream(stream),
                        static_cast<const int64_t*>(tags), static_cast<int>(n), static_cast<int64_t*>(unique_tags), inverse, found);
   return check_launch("unique_whole_kernel");
+}
+
+extern "C" int brt_hip_unique_tags_of_flows(const void* const* tags, const int32_t* rows, int flow_num, int tag_bits, void* unique_tags,
+                                            int32_t* head, int32_t* next, int32_t* n_unique, int64_t* found, int32_t* host,
+                                            void* stream) {
+  if (tag_bits != 32 && tag_bits != 64) return fail(BRT_E_INVALID, "tag_bits must be 32 or 64, got %d", tag_bits);
+  Flows flows;
+  if (!collect_flows(tags, rows, flow_num, &flows)) return fail(BRT_E_INVALID, "bad flows (%d of them)", flow_num);
+  const int n = flows.start[kMaxFlows];
+  if (n < 1) return fail(BRT_E_INVALID, "no tags");
+  if (n > kFlowRows) return fail(BRT_E_UNSUPPORTED, "more than %d tags", kFlowRows);
+  if (!unique_tags || !head || !next || !n_unique || !found) return fail(BRT_E_INVALID, "null argument");
+  for (int f = 0; f < flow_num; ++f)
+    if (!aligned(tags[f], tag_bits / 8)) return fail(BRT_E_INVALID, "tags are not aligned to their size");
+  const int lds = kSmallRange * static_cast<int>(sizeof(int));
+  const bool narrow = tag_bits == 32;
+  const void* fn = narrow ? reinterpret_cast<const void*>(&unique_flows_kernel<int32_t>)
+                          : reinterpret_cast<const void*>(&unique_flows_kernel<int64_t>);
+  if (const int rc = allow_dynamic_lds(fn, lds); rc != BRT_OK) return rc;
+  if (narrow)
+    hipLaunchKernelGGL(unique_flows_kernel<int32_t>, dim3(1), dim3(kScanThreads), lds, as_stream(stream), flows,
+                       static_cast<int32_t*>(unique_tags), head, next, n_unique, found, host);
+  else
+    hipLaunchKernelGGL(unique_flows_kernel<int64_t>, dim3(1), dim3(kScanThreads), lds, as_stream(stream), flows,
+                       static_cast<int64_t*>(unique_tags), head, next, n_unique, found, host);
+  return check_launch("unique_flows_kernel");
+}
+
+extern "C" int brt_hip_combine_flows(const void* const* in_data, const int32_t* rows, int flow_num, void* out_data, const int32_t* head,
+                                     const int32_t* next, int cell, int n_out, int dtype, void* stream) {
+  if (cell < 0 || n_out < 0) return fail(BRT_E_INVALID, "bad shape cell=%d n_out=%d", cell, n_out);
+  if (dtype != BRT_F32 && dtype != BRT_F16 && dtype != BRT_BF16) return fail(BRT_E_UNSUPPORTED, "dtype %d", dtype);
+  Flows flows;
+  if (!collect_flows(in_data, rows, flow_num, &flows)) return fail(BRT_E_INVALID, "bad flows (%d of them)", flow_num);
+  if (n_out == 0 || cell == 0) return BRT_OK;
+  if (!out_data || !head || !next) return fail(BRT_E_INVALID, "null argument");
+  const int es = elem_bytes(dtype);
+  const size_t row_bytes = static_cast<size_t>(cell) * es;
+  uintptr_t address = reinterpret_cast<uintptr_t>(out_data);
+  for (int f = 0; f < flow_num; ++f)
+    if (rows[f] > 0) address |= reinterpret_cast<uintptr_t>(in_data[f]);
+  int unit = 0;
+  for (int b = 16; b >= es && unit == 0; b >>= 1)
+    if (row_bytes % b == 0 && address % b == 0) unit = b;
+  if (unit == 0) return fail(BRT_E_INVALID, "rows are not aligned to their element size");
+  const SumArgs a{nullptr, out_data, head, next, n_out, static_cast<int>(row_bytes / unit)};
+  if (dtype == BRT_F32) launch_sum<BRT_F32, BRT_F32>(unit, a, as_stream(stream), flows);
+  else if (dtype == BRT_F16) launch_sum<BRT_F16, BRT_F16>(unit, a, as_stream(stream), flows);
+  else launch_sum<BRT_BF16, BRT_BF16>(unit, a, as_stream(stream), flows);
+  return check_launch("combine_flows");
 }
 
 extern "C" size_t brt_hip_combine_by_index_workspace_bytes(int P, int n_out) {

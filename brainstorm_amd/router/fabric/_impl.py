@@ -327,24 +327,33 @@ class CombineFabric(FabricBase):
                 load_stack[-1] = torch.tensor([n], dtype=torch.int32, device=data.device)
                 out_flows.append(init_grid_tensor(data, tag_stack, load_stack, extra))
                 continue
-            if self.is_tag_index:
-                fused, fused_tags, route_indices = c_router.fuse_split_cells_from_paths(
-                    datas, is_tag_fuse=True, loads=loads, tags=tags)
-                fused_loads = None
-            else:
-                (fused,) = c_router.fuse_split_cells_from_paths(datas)
-                fused_loads, route_indices, fused_tags = loads[0], tags[0], None
-            result = c_router.combine_with_indices_and_loads(
-                fused, route_indices, fused_loads, score if self.transform else None, residual,
-                max_path_padding=self.max_path_padding, ever_padded=self.ever_padded,
-                is_tag_index=self.is_tag_index, tags=fused_tags)
-            if self.is_tag_index:
+            result = None
+            if self.is_tag_index and residual is None and not self.ever_padded:
+                result = c_router.combine_flows(datas, tags)
+            if result is not None:
                 out_data, out_tag, out_load = result
             else:
-                (out_data,), out_tag, out_load = result, None, None
+                out_data, out_tag, out_load = self._combine_fused(datas, tags, loads, score, residual)
             out_flow = init_grid_tensor(out_data, tag_stack[:-1], load_stack[:-1], extra)
             out_flows.append(out_flow.pack(out_tag, out_load))
         return out_flows
+
+    def _combine_fused(self, datas, tags, loads, score, residual):
+        if self.is_tag_index:
+            fused, fused_tags, route_indices = c_router.fuse_split_cells_from_paths(
+                datas, is_tag_fuse=True, loads=loads, tags=tags)
+            fused_loads = None
+        else:
+            (fused,) = c_router.fuse_split_cells_from_paths(datas)
+            fused_loads, route_indices, fused_tags = loads[0], tags[0], None
+        result = c_router.combine_with_indices_and_loads(
+            fused, route_indices, fused_loads, score if self.transform else None, residual,
+            max_path_padding=self.max_path_padding, ever_padded=self.ever_padded,
+            is_tag_index=self.is_tag_index, tags=fused_tags)
+        if self.is_tag_index:
+            return result
+        (out_data,) = result
+        return out_data, None, None
 
 
 # ----------------------------------------------------------------------------- fused

@@ -374,7 +374,14 @@ int brt_hip_grouped_gemm_accumulate(const void* x, const void* const* weights,
  *   dtypes as brt_hip_combine: fp32, fp16, bf16, or a 16-bit input with fp32 output.
  *   out_data is written whole; it needs no zero fill.
  *
- * Both take a caller-provided workspace (4-byte aligned, size from the query functions) and
+ * brt_hip_unique_tags_of_flows and brt_hip_combine_flows are the two for rows that lie in up to BRT_MAX_FLOWS
+ *   buffers (`flow_num` host arrays of device addresses and row counts), as if these had been concatenated
+ *   (router.cc:348-369) first.  The former takes 1 to BRT_FLOW_ROWS_MAX tags in all, writes `unique_tags` (room for every
+ *   tag), the lists of the rows of every unique tag (`head` and `next`, room for every tag), their number to `n_unique` [1] and
+ *   `found` as above; with `host` (host memory that the device can write, 7 words, or null) also the 6 words of `found`
+ *   followed by a 1, which the host may watch.  The latter takes the lists and `n_out` = that number; its result has the type of the rows.
+ *
+ * unique_tags and combine_by_index take a caller-provided workspace (4-byte aligned, size from the query functions) and
  * queue 1 to 5 small launches on `stream` (small inputs are handled by a single workgroup).
  */
 size_t brt_hip_unique_tags_workspace_bytes(long lo, long hi);
@@ -384,6 +391,13 @@ int brt_hip_unique_tags(const void* tags, int tag_bits, long n, long lo, long hi
 #define BRT_UNIQUE_WHOLE_MAX 32768
 int brt_hip_unique_tags_whole(const void* tags, int tag_bits, long n, void* unique_tags,
                               int64_t* inverse, int64_t* found, void* stream);
+#define BRT_MAX_FLOWS 64
+#define BRT_FLOW_ROWS_MAX 8192
+int brt_hip_unique_tags_of_flows(const void* const* tags, const int32_t* rows, int flow_num, int tag_bits,
+                                 void* unique_tags, int32_t* head, int32_t* next, int32_t* n_unique,
+                                 int64_t* found, int32_t* host, void* stream);
+int brt_hip_combine_flows(const void* const* in_data, const int32_t* rows, int flow_num, void* out_data,
+                          const int32_t* head, const int32_t* next, int cell, int n_out, int dtype, void* stream);
 size_t brt_hip_combine_by_index_workspace_bytes(int P, int n_out);
 int brt_hip_combine_by_index(const void* in_data, void* out_data, const void* index, int index_bits,
                              int P, int cell, int n_out, void* workspace, size_t workspace_bytes,

@@ -923,6 +923,54 @@ def test_identity_fabrics_on_the_gpu(brt_mod):
     assert torch.allclose(brt.to_torch_tensor(out1), one * 7.0, rtol=1e-6, atol=1e-6)
 
 
+# flows gathered where they are: empty ones, one and the most of them, rows of every unit, views off alignment, tags on one cell (a list
+# longer than a wavefront) and on the ends of the widest range; the last four are left to the general way
+@pytest.mark.parametrize("rows,high,cell,dtype,tag_type,taken", [
+    ([700, 0, 300, 24], 900, 512, torch.float32, torch.int32, True),
+    ([1, 1], 1, 8, torch.bfloat16, torch.int64, True),
+    ([128] * 64, 5000, 3, torch.float16, torch.int32, True),
+    ([0, 0, 4096, 4095, 0, 1], 32768, 100, torch.bfloat16, torch.int64, True),
+    ([150, 90], 2, 10, torch.float32, torch.int32, True),
+    ([8192], 4000, 1, torch.float16, torch.int32, True),
+    ([4096, 4097], 4000, 8, torch.float32, torch.int32, False),
+    ([30, 30], 32769, 8, torch.float32, torch.int32, False),
+    ([10] * 65, 100, 8, torch.float32, torch.int32, False),
+    ([20, 20], 30, 8, torch.float64, torch.int32, False),
+])
+@pytest.mark.parametrize("shifted", [False, True])
+def test_flows_are_gathered_where_they_are(brt_mod, rows, high, cell, dtype, tag_type, taken, shifted):
+    from brainstorm_amd._C import router as c_router
+
+    g = torch.Generator().manual_seed(sum(rows) + cell)
+    datas, tags = [], []
+    for n in rows:
+        room = torch.randn(n * cell + 1, generator=g).to(dtype).cuda()
+        datas.append(room[1:].view(n, cell) if shifted else room[:-1].view(n, cell))
+        tags.append(torch.randint(1, high + 1, (n,), generator=g).to(tag_type).cuda())
+    long = next(t for t in tags if t.numel() > 0)
+    long[0] = 1
+    last = next(t for t in reversed(tags) if t.numel() > 0)
+    last[-1] = high
+    got = c_router.combine_flows(datas, tags)
+    assert (got is not None) == taken
+    if not taken:
+        return
+    fused, unique, inverse = c_router.fuse_split_cells_from_paths(datas, is_tag_fuse=True, tags=tags)
+    want = c_router.combine_with_indices_and_loads(fused, inverse, None, tags=unique, is_tag_index=True, ever_padded=False)
+    for a, b in zip(got, want):
+        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b)
+
+
+def test_flows_of_unequal_rows_are_refused_as_before(brt_mod):
+    from brainstorm_amd._C import router as c_router
+
+    x, tags = torch.zeros(4, 8, device="cuda"), torch.arange(4, dtype=torch.int32, device="cuda")
+    for other in (x[:, :4], x.bfloat16(), x.cpu(), x.double(), x.unsqueeze(2)):
+        assert c_router.combine_flows([x, other], [tags, tags]) is None
+    assert c_router.combine_flows([x, x], [tags, tags[:3]]) is None
+    assert c_router.combine_flows([x, x], [tags, tags.long()]) is None
+
+
 def test_placeholder_combine_gives_empty_flows_of_the_recorded_shape(brt_mod):
     _, _, _, GatherRouter = brt_mod
     dev = torch.device("cuda", torch.cuda.current_device())
