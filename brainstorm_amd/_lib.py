@@ -68,6 +68,10 @@ SIGNATURES = {
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     ),
+    "brt_hip_combine_by_tags_cleared": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    ),
     "brt_hip_topk_hot_mask": (
         _c_int,
         [_c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr],

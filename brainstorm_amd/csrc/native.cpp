@@ -384,14 +384,20 @@ PyObject* combine(const Args& a) {
   }
   const int out_type = code_of(out.scalar_type());
   if (out_type < 0 || out.numel() != T * cell) runtime_error("out_data does not match [cell_num, *cell_shape]");
-  // scatter form (identical rows; cells without a row keep the residual)
-  if (residual.defined() && !gates.defined() && !a.none(7) && cell * in.element_size() % 16 == 0 &&
-      (out_type == in_type || out_type == BRT_F32)) {
+  // scatter form (identical rows; cells without a row keep the residual, or become zero)
+  const bool scatters = !gates.defined() && !a.none(7) && cell * in.element_size() % 16 == 0 && (out_type == in_type || out_type == BRT_F32);
+  if (scatters && residual.defined()) {
     const Tensor tags = a.tensor(7);
     check(brt_hip_combine_by_tags(ptr(in), ptr(out), iptr(tags), P, cell, T, in_type, out_type, stream_of(in)));
+    return wrap(out);
+  }
+  const Tensor loads =
+      dense(given_loads.device() == in.device() ? given_loads : given_loads.to(in.options().dtype(at::kInt), /*non_blocking=*/true));
+  if (scatters && E <= 64 && reinterpret_cast<uintptr_t>(ptr(in)) % 16 == 0) {
+    const Tensor tags = a.tensor(7);
+    check(brt_hip_combine_by_tags_cleared(ptr(in), ptr(out), iptr(tags), iptr(route), iptr(loads), T, cell, E, P, mpl, in_type, out_type,
+                                          stream_of(in)));
   } else {
-    const Tensor loads =
-        dense(given_loads.device() == in.device() ? given_loads : given_loads.to(in.options().dtype(at::kInt), /*non_blocking=*/true));
     check(brt_hip_combine(ptr(in), ptr(out), ptr(gates), iptr(route), iptr(loads), T, cell, E, P, mpl, residual.defined(),
                           in_type, out_type, gates.defined() ? code_of(gates.scalar_type()) : BRT_F32, stream_of(in)));
   }

@@ -1084,14 +1084,14 @@ struct CombineRowsArgs {
 };
 
 template <int IN_DT, int OUT_DT, int LS, int UPR>
-__global__ __launch_bounds__(kBlock) void combine_rows_kernel(CombineRowsArgs a) {
+__device__ __forceinline__ void combine_rows(const CombineRowsArgs& a, int block) {
   using U = u32x4;
   constexpr int NE = 16 / elem_bytes(IN_DT);
   constexpr int OUT_BYTES = NE * elem_bytes(OUT_DT);
   constexpr int LPR = 1 << LS;
   constexpr int GROUPS = kWave >> LS;
   const int lane = threadIdx.x & (kWave - 1);
-  const long wave = static_cast<long>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const long wave = static_cast<long>(block) * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int gidx = lane >> LS, glane = lane & (LPR - 1);
   const long p0 = wave * a.rows_pw;
   const int np = static_cast<int>(max(0l, min(static_cast<long>(a.rows_pw), a.P - p0)));
@@ -1138,6 +1138,61 @@ __global__ __launch_bounds__(kBlock) void combine_rows_kernel(CombineRowsArgs a)
           }
         }
       }
+    }
+  }
+}
+
+template <int IN_DT, int OUT_DT, int LS, int UPR>
+__global__ __launch_bounds__(kBlock) void combine_rows_kernel(CombineRowsArgs a) {
+  combine_rows<IN_DT, OUT_DT, LS, UPR>(a, blockIdx.x);
+}
+
+// The scatter form into a result that starts from nothing: the first `clear_blocks` workgroups read the index words, all of a
+// wavefront's in one round trip, and write zeros to the cells that own no row, the others move the rows.  Neither part waits for the
+// other, and no cell is written by both.  Bound by memory; the gather form reads the index words of a cell before it knows which row to
+// load (in a trace, us, gather form and this one: 65536 bf16 cells of 512 elements 30.2 and 27.5, 32768 fp32 cells of 1024 58.9 and 51.5, 65536 bf16
+// of 768 with a fixed stride 42.6 and 41.0, 100352 fp16 of 96 likewise 12.2 and 11.4).
+struct ClearedArgs {
+  CombineRowsArgs r;
+  const int* idx;
+  const int* loads;
+  int E, mpl, ep_shift, clear_blocks;
+};
+constexpr int kClearLoads = 8;  // index loads of a wavefront in flight
+
+template <int IN_DT, int OUT_DT, int LS, int UPR>
+__global__ __launch_bounds__(kBlock) void combine_rows_cleared_kernel(ClearedArgs a) {
+  if (static_cast<int>(blockIdx.x) >= a.clear_blocks) {
+    combine_rows<IN_DT, OUT_DT, LS, UPR>(a.r, blockIdx.x - a.clear_blocks);
+    return;
+  }
+  constexpr int kUnits = elem_bytes(OUT_DT) / elem_bytes(IN_DT);  // 16-byte units of the result for one of a row
+  const int lane = threadIdx.x & (kWave - 1);
+  const long wave = static_cast<long>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int E = a.E, ep_shift = a.ep_shift, ep = 1 << ep_shift, rps = kWave >> ep_shift;
+  const int e = lane & (ep - 1), sub = lane >> ep_shift;
+  const unsigned long long seg = ep == kWave ? ~0ull : ((1ull << ep) - 1ull) << (sub * ep);
+  const long t0 = wave * (kClearLoads * rps);
+  const int nt = static_cast<int>(max(0l, min(static_cast<long>(kClearLoads * rps), a.r.T - t0)));
+  if (nt == 0) return;
+  const int* const idx = a.idx + t0 * E;
+  int v[kClearLoads];
+#pragma unroll
+  for (int u = 0; u < kClearLoads; ++u) v[u] = idx[min(u * rps + sub, nt - 1) * E + min(e, E - 1)];
+  const SmallTables tab = small_tables(a.loads, E, a.mpl, ep_shift, lane);
+  const int units = a.r.cpr * kUnits;
+  u32x4* const dst = static_cast<u32x4*>(a.r.dst);
+  const u32x4 zero = {};
+#pragma unroll
+  for (int u = 0; u < kClearLoads; ++u) {
+    const bool owns = e < E && v[u] >= 1 && v[u] <= tab.load_e && tab.start_e + v[u] - 1 < a.r.P;
+    // the first lane of every cell without a row (cells of this load: rps)
+    unsigned long long bare = __ballot((__ballot(owns) & seg) == 0 && e == 0 && u * rps + sub < nt);
+    while (bare != 0) {  // wave-uniform: one cell at a time, the whole wavefront on its units
+      const int first = __builtin_ctzll(bare);
+      bare &= bare - 1;
+      u32x4* const to = dst + static_cast<size_t>(t0 + u * rps + (first >> ep_shift)) * units;
+      for (int off = lane; off < units; off += kWave) store_unit<LS >= 4>(to + off, zero);
     }
   }
 }
@@ -1390,14 +1445,18 @@ extern "C" int brt_hip_combine(const void* src, void* dst, const void* gates,
   return check_launch("combine_kernel");
 }
 
-extern "C" int brt_hip_combine_by_tags(const void* src, void* dst, const int32_t* row_tags, int P,
-                                       int cell, int T, int in_dtype, int out_dtype, void* stream) {
+namespace {
+
+// indices non-null: cells without a row are cleared, else they keep what they hold
+int combine_by_tags(const void* src, void* dst, const int32_t* row_tags, const int32_t* indices, const int32_t* loads, int P, int cell, int T,
+                    int E, int max_path_load, int in_dtype, int out_dtype, void* stream) {
+  const bool clears = indices != nullptr;
   if (T < 0 || cell < 0 || P < 0) return fail(BRT_E_INVALID, "bad shape T=%d cell=%d P=%d", T, cell, P);
   if ((in_dtype != BRT_F32 && in_dtype != BRT_F16 && in_dtype != BRT_BF16) ||
       (out_dtype != in_dtype && out_dtype != BRT_F32))
     return fail(BRT_E_UNSUPPORTED, "dtype pair %d -> %d is not supported", in_dtype, out_dtype);
-  if (P == 0 || cell == 0 || T == 0) return BRT_OK;
-  if (!src || !dst || !row_tags) return fail(BRT_E_INVALID, "null argument");
+  if ((P == 0 && !clears) || cell == 0 || T == 0) return BRT_OK;
+  if (!dst || (P > 0 && (!src || !row_tags))) return fail(BRT_E_INVALID, "null argument");
   const size_t row_bytes = static_cast<size_t>(cell) * elem_bytes(in_dtype);
   if (row_bytes % 16 != 0 || !aligned(src, 16) || !aligned(dst, 16))
     return fail(BRT_E_UNSUPPORTED, "rows must be whole 16-byte units (row is %zu bytes)", row_bytes);
@@ -1412,13 +1471,24 @@ extern "C" int brt_hip_combine_by_tags(const void* src, void* dst, const int32_t
   a.rows_pw = rows;
   const long n_waves = (static_cast<long>(P) + rows - 1) / rows;
   const int waves_pb = kBlock / kWave;
-  const dim3 grid(static_cast<unsigned>((n_waves + waves_pb - 1) / waves_pb)), block(kBlock);
+  ClearedArgs c{};
+  long blocks = (n_waves + waves_pb - 1) / waves_pb;
+  if (clears) {
+    while ((1 << c.ep_shift) < E) ++c.ep_shift;
+    const long cells_pb = static_cast<long>(waves_pb) * kClearLoads * (kWave >> c.ep_shift);
+    c.idx = indices; c.loads = loads; c.E = E; c.mpl = max_path_load;
+    c.clear_blocks = static_cast<int>((T + cells_pb - 1) / cells_pb);
+    c.r = a;
+    blocks += c.clear_blocks;
+  }
+  const dim3 grid(static_cast<unsigned>(blocks)), block(kBlock);
   hipStream_t st = as_stream(stream);
 #define BRT_ROWS_LAUNCH(IN, OUT)                                                          \
   {                                                                                       \
     auto launch = [&](auto ls, auto upr) {                                                \
-      hipLaunchKernelGGL((combine_rows_kernel<IN, OUT, decltype(ls)::value, decltype(upr)::value>), \
-                         grid, block, 0, st, a);                                          \
+      constexpr int LS = decltype(ls)::value, UPR = decltype(upr)::value;                 \
+      if (clears) hipLaunchKernelGGL((combine_rows_cleared_kernel<IN, OUT, LS, UPR>), grid, block, 0, st, c); \
+      else hipLaunchKernelGGL((combine_rows_kernel<IN, OUT, LS, UPR>), grid, block, 0, st, a);  \
     };                                                                                    \
     using std::integral_constant;                                                         \
     if (a.cpr > 2 * kWave) launch(integral_constant<int, 6>{}, integral_constant<int, 4>{});        \
@@ -1436,4 +1506,21 @@ extern "C" int brt_hip_combine_by_tags(const void* src, void* dst, const int32_t
   else BRT_ROWS_LAUNCH(BRT_BF16, BRT_F32)
 #undef BRT_ROWS_LAUNCH
   return check_launch("combine_rows_kernel");
+}
+
+}  // namespace
+
+extern "C" int brt_hip_combine_by_tags(const void* src, void* dst, const int32_t* row_tags, int P,
+                                       int cell, int T, int in_dtype, int out_dtype, void* stream) {
+  return combine_by_tags(src, dst, row_tags, nullptr, nullptr, P, cell, T, 0, 0, in_dtype, out_dtype, stream);
+}
+
+extern "C" int brt_hip_combine_by_tags_cleared(const void* src, void* dst, const int32_t* row_tags, const int32_t* indices,
+                                               const int32_t* loads, int T, int cell, int E, int P, int max_path_load, int in_dtype,
+                                               int out_dtype, void* stream) {
+  if (E <= 0 || max_path_load < 0) return fail(BRT_E_INVALID, "bad shape E=%d max_path_load=%d", E, max_path_load);
+  if (E > kWave) return fail(BRT_E_UNSUPPORTED, "more than %d paths", kWave);
+  if (static_cast<long>(T) * E >= (1l << 31)) return fail(BRT_E_UNSUPPORTED, "T*E >= 2^31");
+  if (!indices || !loads) return fail(BRT_E_INVALID, "null argument");
+  return combine_by_tags(src, dst, row_tags, indices, loads, P, cell, T, E, max_path_load, in_dtype, out_dtype, stream);
 }

@@ -224,6 +224,11 @@ int brt_hip_combine(const void* src, void* dst, const void* gates, const int32_t
  */
 int brt_hip_combine_by_tags(const void* src, void* dst, const int32_t* row_tags, int P, int cell,
                             int T, int in_dtype, int out_dtype, void* stream);
+/* The same into a result that starts from nothing: cells that own no row by `indices` (the [T,E] seat indices the rows were dispatched
+ * with, up to 64 paths), `loads` and `max_path_load` (as in brt_hip_combine) become zero rows, so every element of dst is written. */
+int brt_hip_combine_by_tags_cleared(const void* src, void* dst, const int32_t* row_tags, const int32_t* indices,
+                                    const int32_t* loads, int T, int cell, int E, int P, int max_path_load, int in_dtype,
+                                    int out_dtype, void* stream);
 
 /*
  * Gate front-end (the three torch launches of TopKProtocol.make_route_decision,

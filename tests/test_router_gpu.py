@@ -923,6 +923,39 @@ def test_identity_fabrics_on_the_gpu(brt_mod):
     assert torch.allclose(brt.to_torch_tensor(out1), one * 7.0, rtol=1e-6, atol=1e-6)
 
 
+# the scatter form that clears the cells without a row, against the gather form: one to 64 paths, cells behind the last whole load, few
+# and most of them without a row, fixed strides, rows of one unit to several a lane, widened results
+@pytest.mark.parametrize("T,E,cell,dtype,out_dtype,cap,pad,stride", [
+    (1, 1, 8, torch.bfloat16, None, None, False, 0),
+    (2, 3, 8, torch.bfloat16, None, None, False, 0),
+    (1000, 8, 96, torch.float16, None, 100, True, 100),
+    (1025, 8, 96, torch.float16, torch.float32, 90, True, 128),
+    (513, 64, 512, torch.float32, None, 5, False, 0),
+    (777, 33, 1000, torch.bfloat16, torch.float32, 20, False, 0),
+    (300, 5, 2056, torch.float32, None, 1, False, 0),
+    (4099, 2, 4, torch.float32, None, 1500, False, 0),
+    (700, 65, 64, torch.float32, None, 8, False, 0),
+])
+def test_combine_without_a_residual_clears_the_cells_without_a_row(brt_mod, T, E, cell, dtype, out_dtype, cap, pad, stride):
+    from brainstorm_amd._C import router as c_router
+
+    g = torch.Generator().manual_seed(T + E)
+    mask = torch.zeros(T, E, dtype=torch.int32).scatter_(1, torch.randint(0, E, (T, 1), generator=g), 1)
+    mask[torch.rand(T, generator=g) < 0.1] = 0
+    x = torch.randn(T, cell, generator=g).to(dtype)
+    x[:, 0] = -0.0
+    x[0] = float("inf")
+    x, mask = x.cuda(), mask.cuda()
+    caps = None if cap is None else torch.tensor([cap], dtype=torch.int32, device="cuda")
+    route = c_router.generate_route(mask, caps, pad, False, single_path=True)
+    (rows,) = c_router.dispatch_with_indices_and_loads(x, route.indices, route.loads, None, False, None, stride > 0, stride, route=route)
+    assert route.row_tags is not None
+    args = (rows, route.indices, route.loads, None, None, stride > 0)
+    (got,) = c_router.combine_with_indices_and_loads(*args, out_dtype=out_dtype, route=route)
+    (want,) = c_router.combine_with_indices_and_loads(*args, out_dtype=out_dtype)
+    assert got.dtype == want.dtype and torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
 # flows gathered where they are: empty ones, one and the most of them, rows of every unit, views off alignment, tags on one cell (a list
 # longer than a wavefront) and on the ends of the widest range; the last four are left to the general way
 @pytest.mark.parametrize("rows,high,cell,dtype,tag_type,taken", [
