@@ -97,7 +97,7 @@ class Route:
     take their general forms (pre-zeroed output, index-driven combine)."""
 
     __slots__ = ("indices", "loads", "counts", "is_tag_index", "single_path", "cells", "paths",
-                 "row_tags", "row_tags_stride", "_versions")
+                 "row_tags", "row_tags_stride", "host_loads", "_versions")
 
     def __init__(self, indices, loads, counts, is_tag_index, single_path):
         self.indices, self.loads, self.counts = indices, loads, counts
@@ -106,6 +106,7 @@ class Route:
         self.cells, self.paths = indices.shape
         self.row_tags = None        # [P] int32: 1-based cell of each row of the layout, 0 = no cell
         self.row_tags_stride = 0    # max_path_load the rows were laid out with (0 = packed)
+        self.host_loads = None      # the values of loads, once a dispatch has read them
         self._versions = (indices._version, loads._version)
 
     def owns(self, route_indices: torch.Tensor, loads: torch.Tensor) -> bool:
@@ -300,6 +301,7 @@ def dispatch_with_indices_and_loads(
     route: Optional[Route] = None,
     rows: Optional[int] = None,
     host_loads: Optional[List[int]] = None,
+    likely_rows: Optional[int] = None,
 ) -> List[torch.Tensor]:
     """router.cc:131-273.  Returns ``[out]`` or ``[out, new_tags]``.  ``route`` (keyword only,
     not in the reference): the :class:`Route` the indices came from; the kernel then zero-fills
@@ -308,7 +310,10 @@ def dispatch_with_indices_and_loads(
     bound of ``sum(loads)`` known to the caller; the output then has that many rows (those past
     the loads are zero) and the loads are not read back to the host (router.cc:197-201 sizes
     the output from ``loads.sum().item()``, which stalls the stream; that is what happens without
-    ``rows``).  ``host_loads`` (likewise): the values of ``loads``, where the caller has just read them."""
+    ``rows``).  ``host_loads`` (likewise): the values of ``loads``, where the caller has just read them.
+    ``likely_rows`` (likewise): as many rows as ``sum(loads)`` will hardly exceed; while the host waits for the loads, the rows
+    are moved into room for that many already, of which the result is the first ``sum(loads)`` (all of them are moved
+    again where the room did not do)."""
     _check_on_device(in_data, "in_data")
     _check_on_device(route_indices, "route_indices")
     _check_int32(route_indices, "route_indices")
@@ -325,6 +330,15 @@ def dispatch_with_indices_and_loads(
             hidden_tags = route.single_path and is_1d_routing and not tag_generating
     _check_int32(loads, "loads")
     native = _lib.native()
+    if (likely_rows is not None and counts is not None and is_1d_routing and not max_path_padding and rows is None
+            and host_loads is None and loads.is_cuda and loads.numel() == route_indices.size(1)
+            and likely_rows * (in_data.nbytes // in_data.size(0)) <= _MOST_ROOM):
+        out, new_tags, route.host_loads = native.dispatch_and_read(
+            in_data, route_indices, loads, counts, gates, tags if tag_generating else None,
+            tag_generating or hidden_tags, likely_rows)
+        if hidden_tags:
+            route.row_tags, route.row_tags_stride = new_tags, 0
+        return [out, new_tags] if tag_generating else [out]
     dev_loads = loads if loads.is_cuda else loads.to(in_data.device, non_blocking=True)
     # rows of the dispatched buffer (router.cc:189-202); data dependent, so one
     # host read of the loads unless a fixed per-path stride was given
@@ -346,6 +360,12 @@ def dispatch_with_indices_and_loads(
     if hidden_tags:
         route.row_tags, route.row_tags_stride = new_tags, mpl
     return [out, new_tags] if tag_generating else [out]
+
+
+# Room for rows that are moved before their number is known.  What the loads leave of it stays allocated as long as the result, and
+# the 4 to 7 us that it spares (1024 fp32 cells over 16 experts: scatter, FFN 512 -> 2048 and gather 67.6 -> 60.1 us, scatter and gather alone
+# 46.3 -> 42.5; 2048 cells, two paths each, through the default routers 75.0 -> 71.1) are nothing beside rows of more bytes than these.
+_MOST_ROOM = 1 << 26
 
 
 def loads_on_host(loads: torch.Tensor) -> List[int]:

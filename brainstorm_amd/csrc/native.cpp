@@ -315,7 +315,107 @@ PyObject* route_by_path(const Args& a) {  // path_ids, paths, capacities, cap_pa
   return tuple(wrap(loads), wrap(counts), wrap(seat_rows), wrap(row_entries));
 }
 
+// ---- host reads --------------------------------------------------------------------------------------
+// Whether the word that a kernel sets behind its data is set, within the time that a program's next few launches
+// would take; behind more work than that the caller waits for the stream, which does not keep a core busy.
+bool seen_within(const int32_t* word, std::chrono::microseconds limit) {
+  const auto end = std::chrono::steady_clock::now() + limit;
+  do {
+    for (int i = 0; i < 64; ++i) {
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != 0) return true;
+      __builtin_ia32_pause();
+    }
+  } while (std::chrono::steady_clock::now() < end);
+  return false;
+}
+
+// Pinned memory for a few words that a kernel on the current stream stores, with a last one behind them that says that they are there
+// (other Python threads run while this one waits).  Not watched: more words than a kernel stores quickly, or a stream that
+// is being captured (where reading back is an error); these take the runtime's copy and wait.
+struct HostWords {
+  at::DataPtr host;
+  hipStream_t st;
+  size_t bytes;
+  const char* what;
+  int32_t* seen_from_device = nullptr;  // non-null: watched
+
+  HostWords(const Tensor& t, size_t n, const char* name) : bytes(n), what(name) {
+    constexpr size_t kFewBytes = 4096;
+    host = at::getHostAllocator(at::kCUDA)->allocate(bytes + 4);
+    st = c10::hip::getCurrentHIPStream(t.get_device()).stream();
+    if (bytes > kFewBytes || bytes % 4 != 0) return;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    void* address = nullptr;
+    if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
+        hipHostGetDevicePointer(&address, host.get(), 0) != hipSuccess) {
+      (void)hipGetLastError();  // what asking left behind, if anything
+      return;
+    }
+    seen_from_device = static_cast<int32_t*>(address);
+    __atomic_store_n(word(), 0, __ATOMIC_RELEASE);
+  }
+  int32_t* word() const { return static_cast<int32_t*>(host.get()) + bytes / 4; }
+
+  // A kernel that copies the words of a watched stream.
+  void request(const Tensor& t) {
+    if (seen_from_device == nullptr) return;
+    ++g_calls;
+    if (brt_hip_copy_to_host(iptr(t), seen_from_device, static_cast<int>(bytes / 4), st) != BRT_OK)
+      runtime_error(std::string(what) + ": " + brt_hip_last_error());
+  }
+
+  // Waits for the words of a watched stream; of another, copies them from the device first.
+  const void* read(const Tensor& t) {
+    hipError_t rc = hipSuccess;
+    bool seen = false;
+    if (seen_from_device != nullptr) {
+      Py_BEGIN_ALLOW_THREADS
+      seen = seen_within(word(), std::chrono::microseconds(500));
+      Py_END_ALLOW_THREADS
+    } else {
+      rc = hipMemcpyAsync(host.get(), ptr(t), bytes, hipMemcpyDeviceToHost, st);
+    }
+    if (rc == hipSuccess && !seen) {
+      Py_BEGIN_ALLOW_THREADS
+      rc = hipStreamSynchronize(st);
+      Py_END_ALLOW_THREADS
+    }
+    if (rc != hipSuccess) {
+      (void)hipGetLastError();  // reported here, not by the next launch that looks for an error
+      runtime_error(std::string(what) + ": " + hipGetErrorString(rc));
+    }
+    return host.get();
+  }
+};
+
+// Copies from the device on the current stream into pinned memory and waits for the copy.
+at::DataPtr read_back(const Tensor& t, size_t bytes, const char* what) {
+  HostWords words(t, bytes, what);
+  words.request(t);
+  words.read(t);
+  return std::move(words.host);
+}
+
+PyObject* list_of(const int32_t* values, int64_t n) {
+  PyObject* const list = PyList_New(n);
+  for (int64_t i = 0; i < n; ++i) PyList_SET_ITEM(list, i, PyLong_FromLong(values[i]));
+  return list;
+}
+
 // ---- rows --------------------------------------------------------------------------------------------
+void take_gates_and_tags(Tensor& gates, Tensor& old_tags, const Tensor& in, const Tensor& route) {
+  if (gates.defined()) {
+    on_device(gates, "gates");
+    if (gates.scalar_type() != in.scalar_type()) runtime_error("gates must have the dtype of in_data");  // router.cc:226
+    gates = dense(gates);
+  }
+  if (old_tags.defined()) {
+    on_device(old_tags, "tags");
+    if (old_tags.scalar_type() != route.scalar_type()) runtime_error("tags must have the dtype of route_indices");
+    old_tags = dense(old_tags);
+  }
+}
+
 // in_data, route_indices, loads (on the device), counts, gates, old_tags, tags wanted, rows of the output,
 // max_path_load, is_1d_routing, is_tag_index, outputs pre-zeroed -> (out, new_tags or None)
 PyObject* dispatch(const Args& a) {
@@ -338,22 +438,50 @@ PyObject* dispatch(const Args& a) {
     shape.erase(shape.begin());
   }
   Tensor out = clear ? zeros(shape, in.scalar_type(), in) : empty(shape, in.scalar_type(), in);
-  if (gates.defined()) {
-    if (!one_d) runtime_error("gates are only supported with 1-d routing");  // route.cu:362
-    on_device(gates, "gates");
-    if (gates.scalar_type() != in.scalar_type()) runtime_error("gates must have the dtype of in_data");  // router.cc:226
-    gates = dense(gates);
-  }
-  if (old_tags.defined()) {
-    on_device(old_tags, "tags");
-    if (old_tags.scalar_type() != route.scalar_type()) runtime_error("tags must have the dtype of route_indices");
-    old_tags = dense(old_tags);
-  }
+  if (gates.defined() && !one_d) runtime_error("gates are only supported with 1-d routing");  // route.cu:362
+  take_gates_and_tags(gates, old_tags, in, route);
   Tensor tags;
   if (want_tags) tags = clear ? zeros({total}, at::kInt, in) : empty({total}, at::kInt, in);
   check(brt_hip_dispatch(ptr(in), ptr(out), ptr(gates), iptr(route), iptr(loads), iptr(counts), iptr(old_tags), iptr(tags),
                          T, cell, E, total, mpl, one_d, tag_index, code_of(in.scalar_type()), stream_of(in)));
   return tuple(wrap(out), want_tags ? wrap(tags) : none());
+}
+
+// in_data, route_indices, loads, counts, gates, old_tags, tags wanted, rows that will do -> (out, new_tags or None, the loads as a list).
+// The rows of the output are the sum of the loads, which the host has to wait for.  Meanwhile the rows are moved into room for as many
+// as will do by what the caller knows, and the result is cut to the sum; where they did not do, they are moved again.  (1-d seat
+// routing, packed.)
+PyObject* dispatch_and_read(const Args& a) {
+  const Tensor given = a.tensor(0), route = dense(a.tensor(1)), loads = dense(a.tensor(2)), counts = a.tensor(3);
+  Tensor gates = a.tensor_or_none(4), old_tags = a.tensor_or_none(5), out, tags;
+  const bool want_tags = a.flag(6);
+  const int64_t room = a.integer(7);
+  const Tensor in = dense(given);
+  int32(loads, "loads");
+  const c10::DeviceGuard guard(in.device());
+  const int64_t T = in.size(0), E = route.size(1), cell = divided(in.numel(), T);
+  if (loads.numel() != E) runtime_error("loads must have one entry per path");
+  take_gates_and_tags(gates, old_tags, in, route);
+  auto move_rows = [&](int64_t rows) {
+    out = empty(rows_of(in, rows), in.scalar_type(), in);
+    if (want_tags) tags = empty({rows}, at::kInt, in);
+    check(brt_hip_dispatch(ptr(in), ptr(out), ptr(gates), iptr(route), iptr(loads), iptr(counts), iptr(old_tags), iptr(tags), T, cell, E, rows, 0,
+                           1, 0, code_of(in.scalar_type()), stream_of(in)));
+  };
+  HostWords words(loads, E * 4, "reading the loads");
+  words.request(loads);
+  const bool ahead = words.seen_from_device != nullptr;
+  if (ahead) move_rows(room);
+  const int32_t* const v = static_cast<const int32_t*>(words.read(loads));
+  int64_t total = 0;
+  for (int64_t e = 0; e < E; ++e) total += v[e];
+  if (!ahead || total > room) {
+    move_rows(total);
+  } else if (total < room) {
+    out.unsafeGetTensorImpl()->set_sizes_contiguous(rows_of(in, total));
+    if (want_tags) tags.unsafeGetTensorImpl()->set_sizes_contiguous({total});
+  }
+  return tuple(wrap(out), want_tags ? wrap(tags) : none(), list_of(v, E));
 }
 
 // in_data, route_indices, loads, gates, out_data, out_dtype, max_path_padding, row_tags (a single-path route whose
@@ -638,83 +766,7 @@ PyObject* cast_f32_to_bf16(const Args& a) {
   return wrap(rounded_to_bf16(given));
 }
 
-// ---- host reads --------------------------------------------------------------------------------------
-// Whether the word that a kernel sets behind its data is set, within the time that a program's next few launches
-// would take; behind more work than that the caller waits for the stream, which does not keep a core busy.
-bool seen_within(const int32_t* word, std::chrono::microseconds limit) {
-  const auto end = std::chrono::steady_clock::now() + limit;
-  do {
-    for (int i = 0; i < 64; ++i) {
-      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != 0) return true;
-      __builtin_ia32_pause();
-    }
-  } while (std::chrono::steady_clock::now() < end);
-  return false;
-}
-
-// Pinned memory for a few words that a kernel on the current stream stores, with a last one behind them that says that they are there
-// (other Python threads run while this one waits).  Not watched: more words than a kernel stores quickly, or a stream that
-// is being captured (where reading back is an error); these take the runtime's copy and wait.
-struct HostWords {
-  at::DataPtr host;
-  hipStream_t st;
-  size_t bytes;
-  const char* what;
-  int32_t* seen_from_device = nullptr;  // non-null: watched
-
-  HostWords(const Tensor& t, size_t n, const char* name) : bytes(n), what(name) {
-    constexpr size_t kFewBytes = 4096;
-    host = at::getHostAllocator(at::kCUDA)->allocate(bytes + 4);
-    st = c10::hip::getCurrentHIPStream(t.get_device()).stream();
-    if (bytes > kFewBytes || bytes % 4 != 0) return;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    void* address = nullptr;
-    if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
-        hipHostGetDevicePointer(&address, host.get(), 0) != hipSuccess) {
-      (void)hipGetLastError();  // what asking left behind, if anything
-      return;
-    }
-    seen_from_device = static_cast<int32_t*>(address);
-    __atomic_store_n(word(), 0, __ATOMIC_RELEASE);
-  }
-  int32_t* word() const { return static_cast<int32_t*>(host.get()) + bytes / 4; }
-
-  // Waits for the words of a watched stream; of another, copies them from the device first.
-  const void* read(const Tensor& t) {
-    hipError_t rc = hipSuccess;
-    bool seen = false;
-    if (seen_from_device != nullptr) {
-      Py_BEGIN_ALLOW_THREADS
-      seen = seen_within(word(), std::chrono::microseconds(500));
-      Py_END_ALLOW_THREADS
-    } else {
-      rc = hipMemcpyAsync(host.get(), ptr(t), bytes, hipMemcpyDeviceToHost, st);
-    }
-    if (rc == hipSuccess && !seen) {
-      Py_BEGIN_ALLOW_THREADS
-      rc = hipStreamSynchronize(st);
-      Py_END_ALLOW_THREADS
-    }
-    if (rc != hipSuccess) {
-      (void)hipGetLastError();  // reported here, not by the next launch that looks for an error
-      runtime_error(std::string(what) + ": " + hipGetErrorString(rc));
-    }
-    return host.get();
-  }
-};
-
-// Copies from the device on the current stream into pinned memory and waits for the copy.
-at::DataPtr read_back(const Tensor& t, size_t bytes, const char* what) {
-  HostWords words(t, bytes, what);
-  if (words.seen_from_device != nullptr) {
-    ++g_calls;
-    if (brt_hip_copy_to_host(iptr(t), words.seen_from_device, static_cast<int>(bytes / 4), words.st) != BRT_OK)
-      runtime_error(std::string(what) + ": " + brt_hip_last_error());
-  }
-  words.read(t);
-  return std::move(words.host);
-}
-
+// ---- values on the host ------------------------------------------------------------------------------
 // The values of an int32 vector as a list.
 PyObject* int_list(const Args& a) {
   const Tensor given = a.tensor(0);
@@ -732,9 +784,7 @@ PyObject* int_list(const Args& a) {
   } else if (n > 0) {
     values = iptr(t);
   }
-  PyObject* const list = PyList_New(n);
-  for (int64_t i = 0; i < n; ++i) PyList_SET_ITEM(list, i, PyLong_FromLong(values[i]));
-  return list;
+  return list_of(values, n);
 }
 
 // tags (a vector of 1 to BRT_UNIQUE_WHOLE_MAX int32 or int64 on the device) -> (unique, inverse, lo, hi), the first
@@ -945,7 +995,7 @@ PyObject* entry(PyObject*, PyObject* const* v, Py_ssize_t n) {
 PyMethodDef methods[] = {
     BRT_ENTRY(topk_hot_mask, 2),    BRT_ENTRY(gate_topk, 4),           BRT_ENTRY(throttle_hotmask, 3),
     BRT_ENTRY(generate, 5),         BRT_ENTRY(route_and_dispatch, 7),  BRT_ENTRY(route_by_path, 7),
-    BRT_ENTRY(dispatch, 12),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
+    BRT_ENTRY(dispatch, 12),  BRT_ENTRY(dispatch_and_read, 8),        BRT_ENTRY(combine, 8),             BRT_ENTRY(combine_by_row_tags, 5),
     BRT_ENTRY(top1_to_capacity, 2), BRT_ENTRY(top1_route_to_capacity, 4), BRT_ENTRY(dispatch_by_rows, 5), BRT_ENTRY(combine_by_rows, 7),     BRT_ENTRY(grouped_linear, 16),
     BRT_ENTRY(grouped_linear_f32, 16), BRT_ENTRY(cast_f32_to_bf16, 1), BRT_ENTRY(branch_key, 5),        BRT_ENTRY(int_list, 1),
     BRT_ENTRY(ordinary, 3),         BRT_ENTRY(plain, 1),            BRT_ENTRY(of_class, 2),            BRT_ENTRY(matrix, 4),

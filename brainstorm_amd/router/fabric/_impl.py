@@ -204,6 +204,9 @@ class DispatchFabric(FabricBase):
     ``path_wise_padding``, ``max_path_padding``, ``max_path_load``.
     """
 
+    #: as many rows as the route of the forward call in progress will hardly exceed, where that is known
+    _likely_rows: Optional[int] = None
+
     def __init__(self, flow_num: int, route_logic: Union[str, List[str]] = "1d",
                  transform: Union[bool, List[bool]] = False, **kwargs):
         index_format = kwargs.pop("index_format", "tag_index")
@@ -236,6 +239,8 @@ class DispatchFabric(FabricBase):
                 path_wise_padding=self.path_wise_padding, is_tag_index=as_tags,
                 single_path=getattr(hot_mask, "_brt_single_path", False))
         self.__dict__["_route"] = route  # (not through nn.Module's attribute registration)
+        per_cell = 1 if route.single_path else getattr(hot_mask, "_brt_paths_per_cell", 0)
+        self.__dict__["_likely_rows"] = route.cells * per_cell if per_cell and not self.capacity_padding else None
         route_indices, loads = route.indices, route.loads
         self.capture_flow_stats(in_flows, route_indices, loads)
         all_out_flows, score = self.dispatch(in_flows, route_indices, loads, score)
@@ -253,7 +258,7 @@ class DispatchFabric(FabricBase):
             flow_data, route_indices, loads, score if self.transforms[flow_idx] else None,
             self.is_tag_index, flow_tag, self.max_path_padding, self.max_path_load,
             self.route_logics[flow_idx] == "1d", route=self._route,
-            rows=self._static_rows(flow_data, route_indices), host_loads=host_loads)
+            rows=self._static_rows(flow_data, route_indices), host_loads=host_loads, likely_rows=self._likely_rows)
 
     def _static_rows(self, flow_data, route_indices) -> Optional[int]:
         return None  # size the output from the loads, as the reference does
@@ -263,13 +268,19 @@ class DispatchFabric(FabricBase):
         path_num = route_indices.size(1)
         # the rows are sized and split by the same loads: one read-back for both, and for all flows
         host_loads = None
-        if not self.max_path_padding and loads.dtype == torch.int32 and loads.dim() == 1:
+        reads = not self.max_path_padding and loads.dtype == torch.int32 and loads.dim() == 1
+        if reads and self._likely_rows is None:
             host_loads = c_router.loads_on_host(loads)
         for flow_idx in range(self.flow_num):
             data, tags, load_stack, extra = to_torch_tensor(in_flows[flow_idx], retrieve_attr=True)
             flow_tag = tags[-1]
             tags, load_stack = tags[:-1], load_stack[:-1]
             routed = self._dispatch_flow(flow_idx, data, flow_tag, route_indices, loads, score, host_loads)
+            if reads and host_loads is None:  # read by the dispatch, if it took them so
+                route = self._route
+                host_loads = route.host_loads if route is not None and route.owns(route_indices, loads) else None
+                if host_loads is None:
+                    host_loads = c_router.loads_on_host(loads)
             if self.is_tag_index:
                 routed_data, routed_tags = routed
                 datas, path_loads, path_tags = c_router.split_fused_cells_to_paths(

@@ -130,7 +130,9 @@ class TopKProtocol(ProtocolBase):
                 and score.dtype in (torch.float32, torch.float16, torch.bfloat16)):
             path_ids, scores = c_router.gate_topk(score, self.top_k)
             return CompactHotMask(path_ids, scores, score.shape[1])
-        return _topk_hot_mask(score, self.top_k)
+        hot_mask = _topk_hot_mask(score, self.top_k)
+        hot_mask._brt_paths_per_cell = self.top_k  # what a dispatch makes room for before it knows the loads
+        return hot_mask
 
 
 @register_protocol("switch_top1")

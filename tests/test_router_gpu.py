@@ -923,6 +923,61 @@ def test_identity_fabrics_on_the_gpu(brt_mod):
     assert torch.allclose(brt.to_torch_tensor(out1), one * 7.0, rtol=1e-6, atol=1e-6)
 
 
+@pytest.mark.parametrize("k,cap", [(1, None), (1, 7), (2, None), (2, 30)])
+@pytest.mark.parametrize("tags", [False, True])
+def test_rows_moved_before_their_number_is_known(brt_mod, k, cap, tags):
+    """Room for all, for more and for too few rows, and none: the rows, their tags and the loads are those of a dispatch that waits."""
+    from brainstorm_amd._C import router as c_router
+
+    T, E, cell = 301, 13, 40
+    g = torch.Generator().manual_seed(k)
+    mask = torch.zeros(T, E, dtype=torch.int32).scatter_(1, torch.rand(T, E, generator=g).topk(k).indices, 1).cuda()
+    x = torch.randn(T, cell, generator=g).cuda()
+    caps = None if cap is None else torch.tensor([cap], dtype=torch.int32, device="cuda")
+    old = torch.randperm(T, generator=g).to(torch.int32).cuda() + 1 if tags else None
+
+    def dispatched(likely):
+        route = c_router.generate_route(mask, caps, single_path=k == 1)
+        out = c_router.dispatch_with_indices_and_loads(x, route.indices, route.loads, None, tags, old, route=route, likely_rows=likely)
+        return out + ([route.row_tags] if k == 1 and not tags else []), route
+
+    want, route = dispatched(None)
+    total = int(route.loads.sum())
+    assert route.host_loads is None
+    for likely in (total, T * k, total + 1, total - 1, 0):
+        got, route = dispatched(likely)
+        assert route.host_loads == route.loads.tolist()
+        assert len(got) == len(want)
+        for a, b in zip(got, want):
+            assert a.shape == b.shape and a.stride() == b.stride() and a.storage_offset() == 0 and torch.equal(a, b)
+
+
+def test_a_mask_that_a_hook_fills_up_is_dispatched_whole(brt_mod):
+    brt, _, ScatterRouter, GatherRouter = brt_mod
+    x, score = torch.randn(64, 24).cuda(), torch.randn(64, 5).cuda()
+    for fabric in ({}, {"fabric_type": "fused_dispatch"}):
+        scatter = ScatterRouter(protocol_type="topk", protocol_kwargs={"top_k": 2}, **fabric).cuda()
+        scatter.protocol.register_forward_hook(lambda module, args, mask: mask.fill_(1))
+        flows = scatter(brt.Annotator([0])(x), score)
+        rows = [brt.to_torch_tensor(f) for f in flows] if isinstance(flows, list) else list(brt.to_torch_tensor(flows).split(64))
+        assert len(rows) == 5 and all(torch.equal(r, x) for r in rows)
+
+
+def test_loads_that_a_fabric_is_handed_are_read_themselves(brt_mod):
+    """dispatch() with another route than that of the last forward call: its loads, not those that call has read."""
+    brt, c_router, ScatterRouter, _ = brt_mod
+    x, score = torch.randn(64, 24).cuda(), torch.randn(64, 4).cuda()
+    scatter = ScatterRouter(protocol_type="topk").cuda()
+    cells = brt.Annotator([0])(x)
+    scatter(cells, score)
+    mask = torch.zeros(64, 4, dtype=torch.int32, device="cuda")
+    mask[:, 2] = 1
+    indices, loads = c_router.generate_indices_and_loads(mask)
+    (flows,), _ = scatter.fabric.dispatch([cells], indices, loads, score)
+    assert [brt.to_torch_tensor(f).shape[0] for f in flows] == [0, 0, 64, 0]
+    assert torch.equal(brt.to_torch_tensor(flows[2]), x)
+
+
 # the scatter form that clears the cells without a row, against the gather form: one to 64 paths, cells behind the last whole load, few
 # and most of them without a row, fixed strides, rows of one unit to several a lane, widened results
 @pytest.mark.parametrize("T,E,cell,dtype,out_dtype,cap,pad,stride", [
