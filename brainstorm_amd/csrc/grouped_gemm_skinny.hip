@@ -469,15 +469,21 @@ int launch_act(GemmArgs& a, int act, hipStream_t st) {
 //     1024 -> 2560, 160 tiles, 21.5 -> 20.9; not 16 x 40 rows 3840 -> 1920, 236 MB).
 //   - More: up to 96 tiles (8 x 120 rows 768 -> 3072 19.0 -> 15.6, 3072 -> 768 46.4 -> 21.0, 16 x 100 rows
 //     768 -> 1536 18.6 -> 15.1; 112 tiles, 14 x 120 rows 1024 -> 2048: 22.3 there, 23.3 here; 144 tiles, 16 x 120
-//     rows 1024 -> 2304: 22.7 and 30.5) of up to 32 experts (32 x 120 rows 2048 -> 512 35.1 -> 29.5; with more of
-//     them every XCD reads most of x and of the weights: 64 x 120 rows 2048 -> 256 35.7 there, 43.1 here),
+//     rows 1024 -> 2304: 22.7 and 30.5) of up to 32 experts (32 x 120 rows 2048 -> 512 35.1 -> 25.3),
 //     and up to 160 with fewer experts than XCDs, some of which the 160-row kernel leaves idle (4 x 120 rows
 //     2048 -> 8192 69.3 -> 41.9).
+//     With 24 experts or more, up to 400 rows each, the contracting shapes that are dealt by expert, up to 100 tiles and 70 MB of
+//     weights or 150 and 40: their rows and weights come to an L2 once, where the 160-row kernel's few tiles leave CUs idle and each walks
+//     all of K (64 x 120 rows 2048 -> 256 37.1 -> 25.7, 1024 -> 256 22.0 -> 13.6, 48 x 204 rows 512 -> 128 17.7 -> 6.8, 24 x 216 rows
+//     1920 -> 640 38.8 -> 36.5).  Of 110 drawn shapes that this takes from that kernel the mean is 1.79 times as fast, one is slower
+//     (32 x 352 rows 1536 -> 384 32.5 and 34.3).  Not with fewer experts (16 x 280 rows 1280 -> 1280 30.5 and 40.5), more tiles
+//     (128 x 224 rows 256 -> 256 15.3 and 17.4) or more weights (128 x 181 rows 896 -> 224, 51 MB, 27.9 and 34.4).
 bool few_rows_by_weight(const GemmArgs& a) {
   const long used = std::min(a.E, a.P);
   const long tiles = std::max<long>((a.P + 159) / 160, used) * ((a.N + 255) / 256);
   const double weight_bytes = 2.0 * used * a.N * a.K;
   if (a.P > 64 * used) {
+    if (used >= 24 && a.P <= 400 * used && tiles <= 150 && weight_bytes <= (tiles <= 100 ? 7e7 : 4e7) && experts_stay_on_an_xcd(a)) return true;
     if (tiles <= 96) return used <= 32;
     return a.P <= 128 * used && tiles <= 160 && used < 8 && weight_bytes < 1.5e8;
   }

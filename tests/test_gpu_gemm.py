@@ -604,6 +604,20 @@ def test_few_rows_where_wide_tiles_fill_part_of_a_round(loads, K, N, kernel):
     run(loads, K, N, act="gelu", bias=True)
 
 
+# contracting shapes of several row blocks, dealt by expert: the ends of the rule, part-filled K-steps and columns, experts without rows
+@pytest.mark.parametrize("loads,K,N,kernel", [
+    ([120] * 32 + [0, 1, 300], 512, 512, "few rows"),
+    ([400] * 34, 1024, 256, "few rows"),
+    ([401] * 34, 1024, 256, "160 rows"),
+    ([200] * 23, 1024, 1024, "160 rows"),
+    ([90] * 69 + [0], 296, 200, "few rows"),
+    ([65, 64, 66, 0, 900] * 20, 136, 136, "few rows"),
+])
+def test_few_rows_of_contracting_shapes_dealt_by_expert(loads, K, N, kernel):
+    assert _kernel_for(sum(loads), len(loads), K, N) == kernel
+    run(loads, K, N, act="gelu", bias=True)
+
+
 # K = 64 n + 8, 56 and others: the part-filled K-step is the third and later ones, in the list and in units of 64, 128 and 256 rows whose
 # rings of four to eight K-steps it ends inside, at the end of and behind
 @pytest.mark.parametrize("loads,K,N", [
