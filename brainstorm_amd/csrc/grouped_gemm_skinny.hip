@@ -414,12 +414,29 @@ double narrow_tiles(const GemmArgs& a, int block) {
 // a fifth of the weights or more), of contracting shapes of more than one row block per expert and a tile for most CUs.  Of 74
 // drawn shapes that it takes the mean is 1.18 times as fast in patch order, 3 are more than 2 % slower: weight rows 8 KB apart (8 x 115 skewed
 // rows 4096 -> 1024 32.9 and 36.2).  Not taken: few tiles, which pay 0.1 us more for finding theirs (4 x 104 rows 768 -> 768 5.9 and 6.1),
-// expanding shapes, whose output lines and weights the XCDs then write and read far apart (4 x 120 rows 2048 -> 8192 42 and 46), and
+// large expanding shapes, whose output lines and weights the XCDs then write and read far apart (4 x 120 rows 2048 -> 8192 42 and 46), and
 // weights of 0.14 GB, of part-filled lines 40 MB, or more, likewise (16 x 123 rows 3008 -> 1504 54 and 57, 16 x 60 rows 2096 -> 1048 31 and 34).
 bool experts_stay_on_an_xcd(const GemmArgs& a) {
   const long used = std::min(a.E, a.P);
   return a.N <= a.K && a.P > 32 * used && 2.0 * used * a.N * a.K < (a.K % kBK == 0 ? 1.4e8 : 4e7) && narrow_tiles(a, 32) >= 150 &&
          (a.x_f32 ? 16.0 : 8.0) * a.P >= 0.2 * used * a.N;
+}
+
+// Tiles of the 160-row kernel, 256 columns wide.
+long wide_tiles(const GemmArgs& a) {
+  return std::max<long>((a.P + 159) / 160, std::min(a.E, a.P)) * ((a.N + 255) / 256);
+}
+
+// Expanding shapes of 65 to 400 rows per expert that are taken because they are dealt in patch order too: with few and small tiles the 160-row
+// kernel is as slow as its busiest CU, and up to 40 MB of weights stay near (us, 160-row kernel and this one: 32 x 163 rows
+// 256 -> 1024 31 and 14, 64 x 94 rows 128 -> 256 15 and 5.6, 12 x 233 rows 576 -> 2304 41 and 23, 24 x 322 rows 192 -> 768 12.4 and 12.2).  Of 80 other
+// drawn shapes the mean is 1.52 times as fast, three are slower (24 x 174 skewed rows 576 -> 1152 19.3 and 21.1).
+// Only where the rows are whole lines; not with fewer experts (8 x 343 rows 960 -> 1920 26.1 and 26.5), more weights (24 x 124 rows 512 -> 2048, 50 MB, 18.7 and 23.1) or
+// more tiles (128 x 120 rows 128 -> 512, 256 of them, 13.3 and 17.4).
+bool expanding_and_dealt(const GemmArgs& a) {
+  const long used = std::min(a.E, a.P), tiles = wide_tiles(a);
+  return a.N > a.K && a.K % kBK == 0 && used >= 12 && a.P > 64 * used && a.P <= 400 * used && tiles <= 170 && (tiles > 96 || used > 32) &&
+         2.0 * used * a.N * a.K <= 4e7;
 }
 
 template <int XR, int NT, int D, int ACT, bool ROUTED, bool OUTF32, bool X32>
@@ -430,7 +447,7 @@ int launch(GemmArgs& a, hipStream_t st) {
   // the sum over experts of ceil(M_e / XR) never exceeds P / XR + min(E, P)
   const long blocks = (static_cast<long>(a.P) + XR - 1) / XR + std::min(a.E, a.P);
   a.tiles_m_max = static_cast<int>(blocks);
-  a.patch = experts_stay_on_an_xcd(a);
+  a.patch = experts_stay_on_an_xcd(a) || expanding_and_dealt(a);
   auto* fn = &grouped_gemm_skinny_kernel<XR, NT, D, ACT, ROUTED, OUTF32, X32>;
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(fn), H::kLds); rc != BRT_OK) return rc;
   hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>((blocks * a.tiles_n + kXcds - 1) / kXcds * kXcds)), dim3(kWaves * kWave), H::kLds, st, a);
@@ -480,9 +497,10 @@ int launch_act(GemmArgs& a, int act, hipStream_t st) {
 //     (128 x 224 rows 256 -> 256 15.3 and 17.4) or more weights (128 x 181 rows 896 -> 224, 51 MB, 27.9 and 34.4).
 bool few_rows_by_weight(const GemmArgs& a) {
   const long used = std::min(a.E, a.P);
-  const long tiles = std::max<long>((a.P + 159) / 160, used) * ((a.N + 255) / 256);
+  const long tiles = wide_tiles(a);
   const double weight_bytes = 2.0 * used * a.N * a.K;
   if (a.P > 64 * used) {
+    if (expanding_and_dealt(a)) return true;
     if (used >= 24 && a.P <= 400 * used && tiles <= 150 && weight_bytes <= (tiles <= 100 ? 7e7 : 4e7) && experts_stay_on_an_xcd(a)) return true;
     if (tiles <= 96) return used <= 32;
     return a.P <= 128 * used && tiles <= 160 && used < 8 && weight_bytes < 1.5e8;

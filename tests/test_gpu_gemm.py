@@ -604,7 +604,7 @@ def test_few_rows_where_wide_tiles_fill_part_of_a_round(loads, K, N, kernel):
     run(loads, K, N, act="gelu", bias=True)
 
 
-# contracting shapes of several row blocks, dealt by expert: the ends of the rule, part-filled K-steps and columns, experts without rows
+# shapes of several row blocks, contracting and expanding, dealt by expert: the ends of the rules, part-filled K-steps and columns, experts without rows
 @pytest.mark.parametrize("loads,K,N,kernel", [
     ([120] * 32 + [0, 1, 300], 512, 512, "few rows"),
     ([400] * 34, 1024, 256, "few rows"),
@@ -612,8 +612,12 @@ def test_few_rows_where_wide_tiles_fill_part_of_a_round(loads, K, N, kernel):
     ([200] * 23, 1024, 1024, "160 rows"),
     ([90] * 69 + [0], 296, 200, "few rows"),
     ([65, 64, 66, 0, 900] * 20, 136, 136, "few rows"),
+    ([120] * 33 + [0, 300], 128, 520, "few rows"),
+    ([300] * 12, 384, 1536, "few rows"),
+    ([300] * 11, 384, 1536, "160 rows"),
+    ([1, 0, 700, 64, 65] * 13, 128, 264, "few rows"),
 ])
-def test_few_rows_of_contracting_shapes_dealt_by_expert(loads, K, N, kernel):
+def test_few_rows_of_shapes_dealt_by_expert(loads, K, N, kernel):
     assert _kernel_for(sum(loads), len(loads), K, N) == kernel
     run(loads, K, N, act="gelu", bias=True)
 
