@@ -16,7 +16,7 @@ from brainstorm_amd import _lib
 from brainstorm_amd._C import router as c_router
 from brainstorm_amd.router.protocol._impl import CompactHotMask
 from brainstorm_amd.runtime.deferred import lazy_tensor
-from brainstorm_amd.router.utils import make_kwargs
+from brainstorm_amd.router.utils import make_kwargs, paths_per_cell
 from brainstorm_amd.runtime import Registry
 from brainstorm_amd.runtime.deferred import DeferredState
 from brainstorm_amd.runtime.grid_tensor import GridTensor, init_grid_tensor, to_torch_tensor
@@ -233,13 +233,15 @@ class DispatchFabric(FabricBase):
         caps = runtime_capacities if runtime_capacities is not None else self.supported_capacities
         in_flows = [in_flow] if self.flow_num == 1 else in_flow
         as_tags = self._defers(in_flows, runtime_capacities, hot_mask)
+        per_cell = paths_per_cell(hot_mask)
         if route is None or as_tags:
             route = c_router.generate_route(
                 hot_mask, supported_capacities=caps, capacity_padding=self.capacity_padding,
                 path_wise_padding=self.path_wise_padding, is_tag_index=as_tags,
-                single_path=getattr(hot_mask, "_brt_single_path", False))
+                single_path=per_cell == 1)
         self.__dict__["_route"] = route  # (not through nn.Module's attribute registration)
-        per_cell = 1 if route.single_path else getattr(hot_mask, "_brt_paths_per_cell", 0)
+        if route.single_path:
+            per_cell = 1
         self.__dict__["_likely_rows"] = route.cells * per_cell if per_cell and not self.capacity_padding else None
         route_indices, loads = route.indices, route.loads
         self.capture_flow_stats(in_flows, route_indices, loads)
@@ -422,7 +424,7 @@ class FusedDispatchFabric(DispatchFabric):
         return self._host_caps_list
 
     def _defers(self, in_flows, runtime_capacities, hot_mask) -> bool:
-        if not (self.defer_dispatch and getattr(hot_mask, "_brt_single_path", False)):
+        if not (self.defer_dispatch and paths_per_cell(hot_mask) == 1):
             return False
         if runtime_capacities is not None or self.max_path_padding or any(self.transforms):
             return False
@@ -528,7 +530,7 @@ class FusedDispatchFabric(DispatchFabric):
         return (out if self.flow_num == 1 else [out]), score
 
     def _in_one_step(self, in_flows, runtime_capacities, hot_mask) -> bool:
-        if not (self.static_rows and getattr(hot_mask, "_brt_single_path", False)):
+        if not (self.static_rows and paths_per_cell(hot_mask) == 1):
             return False
         if self.defer_dispatch and self._defers(in_flows, runtime_capacities, hot_mask):
             return False

@@ -12,7 +12,7 @@ import torch
 import torch.nn as nn
 
 from brainstorm_amd._C import router as c_router
-from brainstorm_amd.router.utils import make_kwargs
+from brainstorm_amd.router.utils import make_kwargs, mark_paths
 from brainstorm_amd.runtime import Registry
 
 
@@ -23,8 +23,9 @@ class ProtocolBase(nn.Module):
         super().__init__()
         self.debug = os.environ.get("BRT_DEBUG", "False").lower() in ("true", "1")
 
-    #: True when the protocol never routes a cell to more than one path; the hot mask is
-    #: then marked so that the fabrics can use the tag-driven combine
+    #: Set by a protocol of a program's own that never routes a cell to more than one path: the hot mask that its forward
+    #: returns is then marked, so that the fabrics can use the tag-driven combine.  (The protocols below mark the masks they
+    #: make where they make them: a subclass that decides otherwise does not inherit their promise.)
     single_path = False
 
     def forward(self, score: torch.Tensor, *args, **kwargs):
@@ -32,8 +33,7 @@ class ProtocolBase(nn.Module):
         if self.debug:
             self.check_decision(decisions, score)
         if self.single_path:
-            hot_mask = decisions[0] if isinstance(decisions, (tuple, list)) else decisions
-            hot_mask._brt_single_path = True
+            mark_paths(decisions[0] if isinstance(decisions, (tuple, list)) else decisions, 1)
         return decisions
 
     def make_route_decision(self, score, **kwargs):
@@ -89,8 +89,7 @@ class CompactHotMask:
         if self._dense is None:
             self._dense = torch.zeros(tuple(self.shape), dtype=torch.int32, device=self.device).scatter_(
                 1, self.path_ids.long(), 1)
-            if getattr(self, "_brt_single_path", False):
-                self._dense._brt_single_path = True
+            mark_paths(self._dense, self.path_ids.shape[1])
         return self._dense
 
 
@@ -120,7 +119,6 @@ class TopKProtocol(ProtocolBase):
     def __init__(self, top_k=1):
         super().__init__()
         self.top_k = top_k
-        self.single_path = top_k == 1
         #: set by a ScatterRouter whose fabric takes the compact route: the decision is handed
         #: over as path ids (one kernel, k words per cell) instead of the [cells, paths] mask
         self.compact = False
@@ -131,7 +129,7 @@ class TopKProtocol(ProtocolBase):
             path_ids, scores = c_router.gate_topk(score, self.top_k)
             return CompactHotMask(path_ids, scores, score.shape[1])
         hot_mask = _topk_hot_mask(score, self.top_k)
-        hot_mask._brt_paths_per_cell = self.top_k  # what a dispatch makes room for before it knows the loads
+        mark_paths(hot_mask, self.top_k)
         return hot_mask
 
 
@@ -146,12 +144,15 @@ class SwitchTop1Protocol(ProtocolBase):
 
     def __init__(self, one_hot: bool = False, **kwargs):
         super().__init__(**kwargs)
-        self.single_path = bool(one_hot)
+        self.one_hot = bool(one_hot)
 
     def make_route_decision(self, score):
         mask = score.reshape(-1, score.shape[-1]).to(torch.int32, non_blocking=True)
-        # never the caller's own tensor object: the single-path mark is set on what is returned
-        return mask.view_as(mask) if mask is score else mask
+        # never the caller's own tensor object: the mark is set on what is returned
+        mask = mask.view_as(mask) if mask is score else mask
+        if self.one_hot:
+            mark_paths(mask, 1)
+        return mask
 
     def update(self, supported_capacities):
         self.supported_capacities = supported_capacities
@@ -296,9 +297,8 @@ def throttle_to_capacity(hot_mask, prefix, capacity, by_score=False, score=None)
 
 @register_protocol("swin_moe")
 class SwinMoEProtocol(ProtocolBase):
-    """protocol/swin_moe.py:69-144 (the maintained ``make_route_decision``)."""
-
-    single_path = True  # only the first of the top-k choices is routed (swin_moe.py:138-144)
+    """protocol/swin_moe.py:69-144 (the maintained ``make_route_decision``).  Only the first of the top-k choices is routed
+    (swin_moe.py:138-144)."""
 
     def __init__(self, top_k=2, capacity_factor=0, gate_noise=0.0, group=None, is_postscore=True,
                  batch_prioritized_routing=False, normalize_gate=True, is_gshard_loss=True,
@@ -331,12 +331,14 @@ class SwinMoEProtocol(ProtocolBase):
             made = (c_router.top1_to_capacity(score, cap) if padding is None
                     else c_router.top1_route_to_capacity(score, cap, *padding))
             if made is not None:
+                mark_paths(made[0], 1)
                 return (*made[:2], score, loss, *made[2:])
         mask = _topk_hot_mask(score, 1)  # the first of the top-k choices (swin_moe.py:101-107)
         runtime_capacities = torch.full((paths,), cap, dtype=torch.int32, device=score.device)
         prefix = torch.zeros((paths,), dtype=torch.int32, device=score.device)
         hot_mask, _ = throttle_to_capacity(
             mask, prefix, runtime_capacities, self.batch_prioritized_routing, score)
+        mark_paths(hot_mask, 1)
         decision = (hot_mask, runtime_capacities, score, loss)
         return decision if padding is None else (*decision, None)
 

@@ -5,7 +5,7 @@ from typing import Any, Dict, List, Optional
 import numpy as np
 import torch
 
-__all__ = ["pad_to_max", "make_kwargs", "empty_flows", "assert_compatibility"]
+__all__ = ["pad_to_max", "make_kwargs", "empty_flows", "assert_compatibility", "mark_paths", "paths_per_cell"]
 
 
 def pad_to_max(tensors: List[torch.Tensor], pad_value=0) -> List[torch.Tensor]:
@@ -40,3 +40,19 @@ def assert_compatibility(instance, k, expected_v, given_v) -> None:
     assert expected_v == given_v, (
         f"compatibility check failed for {type(instance).__name__}, caused by keyword "
         f"argument {k}: expected {expected_v}, given {given_v}")
+
+
+def mark_paths(hot_mask: torch.Tensor, most: int) -> None:
+    """Notes on a hot mask that, as it stands, no row of it has more than ``most`` nonzeros.  The note is worth nothing once the
+    mask is edited in place (by a forward hook, or between protocol and fabric), so it goes with the mask's version counter; a
+    tensor that has none is not marked."""
+    if hot_mask.is_inference():
+        return
+    hot_mask._brt_paths_per_cell, hot_mask._brt_single_path = most, most == 1
+    hot_mask._brt_marked_at = hot_mask._version
+
+
+def paths_per_cell(hot_mask) -> int:
+    """The paths that a row of the mask has at most, by a mark that still holds; 0 where that is not known."""
+    marked_at = getattr(hot_mask, "_brt_marked_at", None)
+    return hot_mask._brt_paths_per_cell if marked_at is not None and marked_at == hot_mask._version else 0

@@ -963,6 +963,27 @@ def test_a_mask_that_a_hook_fills_up_is_dispatched_whole(brt_mod):
         assert len(rows) == 5 and all(torch.equal(r, x) for r in rows)
 
 
+@pytest.mark.parametrize("form", [None, {}, {"static_rows": True}, {"defer_dispatch": True}])
+@pytest.mark.parametrize("with_residual", [False, True])
+def test_a_mask_that_a_hook_adds_paths_to_is_summed(brt_mod, form, with_residual):
+    """A top-1 decision whose mask a hook edits in place: every path that it names is added up, in every fabric form."""
+    brt, c_router, ScatterRouter, GatherRouter = brt_mod
+    T, E, d = 70, 5, 24
+    x, score = torch.randn(T, d).cuda(), torch.randn(T, E).cuda()
+    fabric = {} if form is None else {"fabric_type": "fused_dispatch", "fabric_kwargs": form}
+    scatter = ScatterRouter(protocol_type="topk", protocol_kwargs={"top_k": 1}, **fabric).cuda()
+    gather = GatherRouter(**({} if form is None else {"fabric_type": "fused_combine"})).cuda()
+    scatter.protocol.register_forward_hook(lambda module, args, mask: (mask[:, 1:4].fill_(1), None)[1])
+    mask = torch.zeros(T, E, dtype=torch.int32, device="cuda").scatter_(1, score.argmax(1, keepdim=True), 1)
+    mask[:, 1:4] = 1
+    indices, loads = c_router.generate_indices_and_loads(mask)
+    (rows,) = c_router.dispatch_with_indices_and_loads(x, indices, loads)
+    residual = torch.randn(T, d).cuda() if with_residual and form is not None else None
+    (want,) = c_router.combine_with_indices_and_loads(rows, indices, loads, None, None if residual is None else residual.clone())
+    out = gather(scatter(brt.Annotator([0])(x), score), residual)
+    assert torch.equal(brt.to_torch_tensor(out), want)
+
+
 def test_loads_that_a_fabric_is_handed_are_read_themselves(brt_mod):
     """dispatch() with another route than that of the last forward call: its loads, not those that call has read."""
     brt, c_router, ScatterRouter, _ = brt_mod
