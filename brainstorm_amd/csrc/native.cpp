@@ -331,13 +331,16 @@ bool seen_within(const int32_t* word, std::chrono::microseconds limit) {
 
 // Pinned memory for a few words that a kernel on the current stream stores, with a last one behind them that says that they are there
 // (other Python threads run while this one waits).  Not watched: more words than a kernel stores quickly, or a stream that
-// is being captured (where reading back is an error); these take the runtime's copy and wait.
+// is being captured (where reading back is an error); these take the runtime's copy and wait.  The memory goes back to its
+// allocator, which knows nothing of the stream, only when nothing that is queued stores to it any more, also where an
+// exception ends the use between request and read.
 struct HostWords {
   at::DataPtr host;
   hipStream_t st;
   size_t bytes;
   const char* what;
   int32_t* seen_from_device = nullptr;  // non-null: watched
+  bool queued = false;                  // something that stores here may be
 
   HostWords(const Tensor& t, size_t n, const char* name) : bytes(n), what(name) {
     constexpr size_t kFewBytes = 4096;
@@ -354,12 +357,25 @@ struct HostWords {
     seen_from_device = static_cast<int32_t*>(address);
     __atomic_store_n(word(), 0, __ATOMIC_RELEASE);
   }
+  HostWords(const HostWords&) = delete;
+  ~HostWords() {
+    if (!queued) return;
+    hipError_t rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = hipStreamSynchronize(st);
+    Py_END_ALLOW_THREADS
+    if (rc != hipSuccess) {
+      (void)hipGetLastError();
+      (void)host.release_context();  // kept for ever: what became of the stores is not known
+    }
+  }
   int32_t* word() const { return static_cast<int32_t*>(host.get()) + bytes / 4; }
 
   // A kernel that copies the words of a watched stream.
   void request(const Tensor& t) {
     if (seen_from_device == nullptr) return;
     ++g_calls;
+    queued = true;
     if (brt_hip_copy_to_host(iptr(t), seen_from_device, static_cast<int>(bytes / 4), st) != BRT_OK)
       runtime_error(std::string(what) + ": " + brt_hip_last_error());
   }
@@ -373,6 +389,7 @@ struct HostWords {
       seen = seen_within(word(), std::chrono::microseconds(500));
       Py_END_ALLOW_THREADS
     } else {
+      queued = true;
       rc = hipMemcpyAsync(host.get(), ptr(t), bytes, hipMemcpyDeviceToHost, st);
     }
     if (rc == hipSuccess && !seen) {
@@ -384,6 +401,7 @@ struct HostWords {
       (void)hipGetLastError();  // reported here, not by the next launch that looks for an error
       runtime_error(std::string(what) + ": " + hipGetErrorString(rc));
     }
+    queued = false;
     return host.get();
   }
 };
@@ -449,8 +467,8 @@ PyObject* dispatch(const Args& a) {
 
 // in_data, route_indices, loads, counts, gates, old_tags, tags wanted, rows that will do -> (out, new_tags or None, the loads as a list).
 // The rows of the output are the sum of the loads, which the host has to wait for.  Meanwhile the rows are moved into room for as many
-// as will do by what the caller knows, and the result is cut to the sum; where they did not do, they are moved again.  (1-d seat
-// routing, packed.)
+// as will do by what the caller knows, and the result is cut to the sum; where they did not do, they are moved again, and where the
+// device has no memory for the room, they are moved once the sum is known.  (1-d seat routing, packed.)
 PyObject* dispatch_and_read(const Args& a) {
   const Tensor given = a.tensor(0), route = dense(a.tensor(1)), loads = dense(a.tensor(2)), counts = a.tensor(3);
   Tensor gates = a.tensor_or_none(4), old_tags = a.tensor_or_none(5), out, tags;
@@ -462,20 +480,31 @@ PyObject* dispatch_and_read(const Args& a) {
   const int64_t T = in.size(0), E = route.size(1), cell = divided(in.numel(), T);
   if (loads.numel() != E) runtime_error("loads must have one entry per path");
   take_gates_and_tags(gates, old_tags, in, route);
-  auto move_rows = [&](int64_t rows) {
+  auto make_room = [&](int64_t rows) {
+    out = tags = Tensor();
     out = empty(rows_of(in, rows), in.scalar_type(), in);
     if (want_tags) tags = empty({rows}, at::kInt, in);
+  };
+  auto move_rows = [&](int64_t rows) {
     check(brt_hip_dispatch(ptr(in), ptr(out), ptr(gates), iptr(route), iptr(loads), iptr(counts), iptr(old_tags), iptr(tags), T, cell, E, rows, 0,
                            1, 0, code_of(in.scalar_type()), stream_of(in)));
   };
   HostWords words(loads, E * 4, "reading the loads");
   words.request(loads);
-  const bool ahead = words.seen_from_device != nullptr;
+  bool ahead = words.seen_from_device != nullptr;
+  if (ahead) {
+    try {
+      make_room(room);
+    } catch (const c10::OutOfMemoryError&) {
+      ahead = false;
+    }
+  }
   if (ahead) move_rows(room);
   const int32_t* const v = static_cast<const int32_t*>(words.read(loads));
   int64_t total = 0;
   for (int64_t e = 0; e < E; ++e) total += v[e];
   if (!ahead || total > room) {
+    make_room(total);
     move_rows(total);
   } else if (total < room) {
     out.unsafeGetTensorImpl()->set_sizes_contiguous(rows_of(in, total));
@@ -956,6 +985,7 @@ PyObject* combine_flows(const Args& a) {
   const Tensor lists = empty({2 * n}, at::kInt, like), found = empty({3}, at::kLong, like);
   int32_t *const head = iptr(lists), *const next = head + n;
   HostWords words(like, 24, "reading the number of tags");
+  words.queued = true;
   check(brt_hip_unique_tags_of_flows(tags_of.data(), rows.data(), count, narrow ? 32 : 64, ptr(unique), head, next, iptr(number),
                                      static_cast<int64_t*>(ptr(found)), words.seen_from_device, words.st));
   const int64_t n_out = *static_cast<const int64_t*>(words.read(found));

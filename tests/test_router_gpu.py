@@ -952,6 +952,50 @@ def test_rows_moved_before_their_number_is_known(brt_mod, k, cap, tags):
             assert a.shape == b.shape and a.stride() == b.stride() and a.storage_offset() == 0 and torch.equal(a, b)
 
 
+def test_rows_are_moved_later_where_there_is_no_room_for_them(brt_mod):
+    """A card that holds the rows there are, but not those there could be: they are moved when the loads are known."""
+    from brainstorm_amd._C import router as c_router
+
+    T, E, cell, cap = 15000, 4, 1024, 8
+    x = torch.randn(T, cell, device="cuda")
+    mask = torch.zeros(T, E, dtype=torch.int32, device="cuda")
+    mask[:, 1] = 1
+    route = c_router.generate_route(mask, torch.tensor([cap], dtype=torch.int32, device="cuda"), single_path=True)
+    (want,) = c_router.dispatch_with_indices_and_loads(x, route.indices, route.loads, route=route)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    limit = torch.cuda.memory_reserved() + (64 << 20)
+    torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(0).total_memory)
+    taken = []
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            while True:
+                taken.append(torch.empty(16 << 20, dtype=torch.uint8, device="cuda"))
+        taken.pop()  # less than 48 MB in one piece; the rows of all cells are 61 MB
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            torch.empty(T, cell, device="cuda")
+        (got,) = c_router.dispatch_with_indices_and_loads(x, route.indices, route.loads, route=route, likely_rows=T)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert got.shape[0] == cap and torch.equal(got, want)
+    assert route.host_loads == route.loads.tolist() and torch.equal(route.row_tags.cpu(), torch.arange(1, cap + 1, dtype=torch.int32))
+
+
+def test_a_failed_dispatch_leaves_nothing_queued_that_stores_to_host_memory(brt_mod):
+    """The words that the loads are read through go back to their allocator when the exception leaves the call."""
+    from brainstorm_amd import _lib
+    from brainstorm_amd._C import router as c_router
+
+    mask = torch.eye(4, dtype=torch.int32, device="cuda")
+    route = c_router.generate_route(mask, single_path=True)
+    x = torch.zeros(4, 8, dtype=torch.float64, device="cuda")  # no type of the kernels
+    torch.cuda.synchronize()
+    torch.cuda._sleep(20_000_000)
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        _lib.native().dispatch_and_read(x, route.indices, route.loads, route.counts, None, None, False, 4)
+    assert torch.cuda.current_stream().query()
+
+
 def test_a_mask_that_a_hook_fills_up_is_dispatched_whole(brt_mod):
     brt, _, ScatterRouter, GatherRouter = brt_mod
     x, score = torch.randn(64, 24).cuda(), torch.randn(64, 5).cuda()
