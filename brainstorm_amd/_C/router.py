@@ -362,8 +362,8 @@ def dispatch_with_indices_and_loads(
     return [out, new_tags] if tag_generating else [out]
 
 
-# Room for rows that are moved before their number is known.  What the loads leave of it stays allocated as long as the result, and
-# the 4 to 7 us that it spares (1024 fp32 cells over 16 experts: scatter, FFN 512 -> 2048 and gather 67.6 -> 60.1 us, scatter and gather alone
+# Room for rows that are moved before their number is known.  What the loads leave of it stays allocated as long as the
+# result (whose storage ends with its rows), and the 4 to 7 us that it spares (1024 fp32 cells over 16 experts: scatter, FFN 512 -> 2048 and gather 67.6 -> 60.1 us, scatter and gather alone
 # 46.3 -> 42.5; 2048 cells, two paths each, through the default routers 75.0 -> 71.1) are nothing beside rows of more bytes than these.
 _MOST_ROOM = 1 << 26
 

@@ -506,9 +506,13 @@ PyObject* dispatch_and_read(const Args& a) {
   if (!ahead || total > room) {
     make_room(total);
     move_rows(total);
-  } else if (total < room) {
-    out.unsafeGetTensorImpl()->set_sizes_contiguous(rows_of(in, total));
-    if (want_tags) tags.unsafeGetTensorImpl()->set_sizes_contiguous({total});
+  } else if (total < room) {  // the storage ends with the rows too: it is saved and compared whole
+    auto cut = [](const Tensor& t, at::IntArrayRef shape) {
+      t.unsafeGetTensorImpl()->set_sizes_contiguous(shape);
+      t.storage().unsafeGetStorageImpl()->set_nbytes(t.nbytes());
+    };
+    cut(out, rows_of(in, total));
+    if (want_tags) cut(tags, {total});
   }
   return tuple(wrap(out), want_tags ? wrap(tags) : none(), list_of(v, E));
 }

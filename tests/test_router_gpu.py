@@ -950,6 +950,7 @@ def test_rows_moved_before_their_number_is_known(brt_mod, k, cap, tags):
         assert len(got) == len(want)
         for a, b in zip(got, want):
             assert a.shape == b.shape and a.stride() == b.stride() and a.storage_offset() == 0 and torch.equal(a, b)
+            assert a.untyped_storage().nbytes() == b.untyped_storage().nbytes()
 
 
 def test_rows_are_moved_later_where_there_is_no_room_for_them(brt_mod):
