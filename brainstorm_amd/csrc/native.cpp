@@ -554,7 +554,11 @@ PyObject* combine(const Args& a) {
   }
   const Tensor loads =
       dense(given_loads.device() == in.device() ? given_loads : given_loads.to(in.options().dtype(at::kInt), /*non_blocking=*/true));
-  if (scatters && E <= 64 && reinterpret_cast<uintptr_t>(ptr(in)) % 16 == 0) {
+  // Results that fill the last-level cache are written better in order (us, bf16 cells over 8 paths of which all, nine and five of ten have a
+  // row, scatter and gather form: 16384 of 8192 elements 109, 105 and 69, and 104, 97 and 63; of 6000, 197 MB, 85, 81 and 53, and
+  // 83, 78 and 46; 131072 of 512, 134 MB, 46, 44 and 35, and 56, 43 and 33; 16384 of 2048, 67 MB, 23, 21 and 19, and 24, 23 and 19).
+  constexpr int64_t kMostScattered = 5ll << 25;
+  if (scatters && E <= 64 && reinterpret_cast<uintptr_t>(ptr(in)) % 16 == 0 && out.numel() * out.element_size() < kMostScattered) {
     const Tensor tags = a.tensor(7);
     check(brt_hip_combine_by_tags_cleared(ptr(in), ptr(out), iptr(tags), iptr(route), iptr(loads), T, cell, E, P, mpl, in_type, out_type,
                                           stream_of(in)));

@@ -1056,6 +1056,11 @@ def test_loads_that_a_fabric_is_handed_are_read_themselves(brt_mod):
     (300, 5, 2056, torch.float32, None, 1, False, 0),
     (4099, 2, 4, torch.float32, None, 1500, False, 0),
     (700, 65, 64, torch.float32, None, 8, False, 0),
+    (9, 3, 20000, torch.float32, None, 1, False, 0),
+    (2500, 3, 2056, torch.bfloat16, torch.float32, 4, False, 0),
+    (70001, 1, 16, torch.bfloat16, None, 30000, False, 0),
+    (20000, 4, 24, torch.float16, torch.float32, 900, False, 0),
+    (12290, 64, 72, torch.bfloat16, None, 100, False, 0),
 ])
 def test_combine_without_a_residual_clears_the_cells_without_a_row(brt_mod, T, E, cell, dtype, out_dtype, cap, pad, stride):
     from brainstorm_amd._C import router as c_router
@@ -1075,6 +1080,38 @@ def test_combine_without_a_residual_clears_the_cells_without_a_row(brt_mod, T, E
     (got,) = c_router.combine_with_indices_and_loads(*args, out_dtype=out_dtype, route=route)
     (want,) = c_router.combine_with_indices_and_loads(*args, out_dtype=out_dtype)
     assert got.dtype == want.dtype and torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
+@pytest.mark.parametrize("T,E,cell", [(16384, 2, 2048), (2048, 1, 16)])
+def test_clearing_cells_is_spread_over_the_card(brt_mod, T, E, cell):
+    """Cells that hardly ever own a row: clearing them takes what the gather form takes for them (2.9 and 16 times that when
+    a wavefront cleared all the cells it had looked at, one by one)."""
+    from brainstorm_amd._C import router as c_router
+
+    mask = torch.zeros(T, E, dtype=torch.int32, device="cuda")
+    mask[::100, E - 1] = 1
+    x = torch.randn(T, cell, device="cuda")
+    route = c_router.generate_route(mask, single_path=True)
+    (rows,) = c_router.dispatch_with_indices_and_loads(x, route.indices, route.loads, route=route)
+
+    def us(form):
+        graph, best = torch.cuda.CUDAGraph(), float("inf")
+        c_router.combine_with_indices_and_loads(rows, route.indices, route.loads, route=form)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                c_router.combine_with_indices_and_loads(rows, route.indices, route.loads, route=form)
+        for _ in range(10):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            graph.replay()
+            end.record()
+            end.synchronize()
+            best = min(best, begin.elapsed_time(end) * 50)
+        return best
+
+    scatter, gather = us(route), us(None)
+    assert scatter < 1.7 * gather, (scatter, gather)
 
 
 # flows gathered where they are: empty ones, one and the most of them, rows of every unit, views off alignment, tags on one cell (a list
