@@ -499,8 +499,11 @@ def fuse_split_cells_from_paths(
     is_tag_fuse: bool = False,
     loads: Optional[List[torch.Tensor]] = None,
     tags: Optional[List[torch.Tensor]] = None,
+    *,
+    tag_range: Optional[Tuple[int, int]] = None,
 ) -> List[torch.Tensor]:
-    """router.cc:348-369."""
+    """router.cc:348-369.  ``tag_range`` (keyword only, not in the reference): the smallest and the largest tag, where the
+    caller has just read them."""
     out_data = torch.cat(in_data, 0)
     if is_load_fuse:
         if loads is None:
@@ -510,7 +513,7 @@ def fuse_split_cells_from_paths(
         if tags is None:
             raise RuntimeError("is_tag_fuse needs tags")
         out_tags = torch.cat(tags, 0)
-        new_tags, global_seat_indices = _unique_tags(out_tags)
+        new_tags, global_seat_indices = _unique_tags(out_tags, tag_range)
         return [out_data, new_tags, global_seat_indices]
     return [out_data]
 
@@ -518,7 +521,7 @@ def fuse_split_cells_from_paths(
 _UNIQUE_WHOLE_MAX = 1 << 15  # BRT_UNIQUE_WHOLE_MAX
 
 
-def _unique_tags(tags: torch.Tensor):
+def _unique_tags(tags: torch.Tensor, tag_range: Optional[Tuple[int, int]] = None):
     """``torch.unique(tags, sorted=True, return_inverse=True)`` (router.cc:362-366) without the
     sort: tags are cell numbers, so a presence table over ``[min, max]`` and one prefix sum give
     the same two tensors.  Tag sets that are sparse in their range (or not a 1-d int32 / int64
@@ -528,7 +531,9 @@ def _unique_tags(tags: torch.Tensor):
         return torch.unique(tags, sorted=True, return_inverse=True)
     with _device_guard(tags.device):
         tags = tags.contiguous()
-        if n <= _UNIQUE_WHOLE_MAX:  # one launch that finds the range itself, one read-back
+        if tag_range is not None:
+            lo, hi = tag_range
+        elif n <= _UNIQUE_WHOLE_MAX:  # one launch that finds the range itself, one read-back
             unique, inverse, lo, hi = _lib.native().unique_tags(tags)
             if unique is not None:
                 return unique, inverse
@@ -636,14 +641,20 @@ def _sum_rows_by_index(in_data, index, n, shape):
     return _lib.native().sum_rows_by_index(in_data, index, n)
 
 
-def combine_flows(datas: List[torch.Tensor], tags: List[torch.Tensor]) -> Optional[tuple]:
+def combine_flows(datas: List[torch.Tensor], tags: List[torch.Tensor], tag_range: Optional[list] = None) -> Optional[tuple]:
     """``fuse_split_cells_from_paths`` (router.cc:348-369) and the tag-mode combine (router.cc:449-472) of its result, from the
     flows where they are: ``(rows, tags, number of tags)``, bit for bit, or None where the general way is to be taken (other
-    types, more than 64 flows or 8192 rows, tags too far apart, a compiler, tracer or mode that looks on)."""
+    types, more than 64 flows or 8192 rows, tags too far apart, a compiler, tracer or mode that looks on).  Tags too far apart
+    have been read: the smallest and the largest are appended to ``tag_range``."""
     if torch.compiler.is_compiling():
         return None
     native = _lib.native_or_none()
-    return None if native is None else native.combine_flows(datas, tags)
+    made = None if native is None else native.combine_flows(datas, tags)
+    if made is None or len(made) == 3:
+        return made
+    if tag_range is not None:
+        tag_range.extend(made)
+    return None
 
 
 # legacy name (sample/cpp/router.ipynb:258-266) of the seat-index combine

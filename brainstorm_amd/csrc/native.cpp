@@ -954,7 +954,8 @@ PyObject* sum_rows_by_index(const Args& a) {
 }
 
 // The rows of the flows (a list), their tags (a list of vectors) -> (the rows of every tag added up in the order of the flows, the tags
-// in ascending order, their number as an int32 vector), or None where a launch over the flows themselves does not take them
+// in ascending order, their number as an int32 vector), (smallest tag, largest tag) where these are too far apart for the launch over the
+// flows themselves, or None where it does not take the flows
 PyObject* combine_flows(const Args& a) {
   if (!PyList_Check(a.v[0]) || !PyList_Check(a.v[1])) return none();
   const Py_ssize_t count = PyList_GET_SIZE(a.v[0]);
@@ -996,8 +997,9 @@ PyObject* combine_flows(const Args& a) {
   words.queued = true;
   check(brt_hip_unique_tags_of_flows(tags_of.data(), rows.data(), count, narrow ? 32 : 64, ptr(unique), head, next, iptr(number),
                                      static_cast<int64_t*>(ptr(found)), words.seen_from_device, words.st));
-  const int64_t n_out = *static_cast<const int64_t*>(words.read(found));
-  if (n_out < 0) return none();
+  const int64_t* const read = static_cast<const int64_t*>(words.read(found));
+  const int64_t n_out = read[0];
+  if (n_out < 0) return tuple(PyLong_FromLongLong(read[1]), PyLong_FromLongLong(read[2]));
   Tensor out = empty(rows_of(like, n_out), like.scalar_type(), like);
   check(brt_hip_combine_flows(data_of.data(), rows.data(), count, ptr(out), head, next, cell, n_out, type, words.st));
   return tuple(wrap(out), wrap(unique.narrow(0, 0, n_out)), wrap(number));

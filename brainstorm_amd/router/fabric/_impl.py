@@ -340,21 +340,21 @@ class CombineFabric(FabricBase):
                 load_stack[-1] = torch.tensor([n], dtype=torch.int32, device=data.device)
                 out_flows.append(init_grid_tensor(data, tag_stack, load_stack, extra))
                 continue
-            result = None
+            result, tag_range = None, []
             if self.is_tag_index and residual is None and not self.ever_padded:
-                result = c_router.combine_flows(datas, tags)
+                result = c_router.combine_flows(datas, tags, tag_range)
             if result is not None:
                 out_data, out_tag, out_load = result
             else:
-                out_data, out_tag, out_load = self._combine_fused(datas, tags, loads, score, residual)
+                out_data, out_tag, out_load = self._combine_fused(datas, tags, loads, score, residual, tag_range or None)
             out_flow = init_grid_tensor(out_data, tag_stack[:-1], load_stack[:-1], extra)
             out_flows.append(out_flow.pack(out_tag, out_load))
         return out_flows
 
-    def _combine_fused(self, datas, tags, loads, score, residual):
+    def _combine_fused(self, datas, tags, loads, score, residual, tag_range):
         if self.is_tag_index:
             fused, fused_tags, route_indices = c_router.fuse_split_cells_from_paths(
-                datas, is_tag_fuse=True, loads=loads, tags=tags)
+                datas, is_tag_fuse=True, loads=loads, tags=tags, tag_range=tag_range)
             fused_loads = None
         else:
             (fused,) = c_router.fuse_split_cells_from_paths(datas)

@@ -1152,6 +1152,36 @@ def test_flows_are_gathered_where_they_are(brt_mod, rows, high, cell, dtype, tag
         assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("high", [32769, 100000, 3000000])
+def test_the_range_of_sparse_tags_is_read_once(brt_mod, monkeypatch, high):
+    """Tags too far apart for the launch over the flows: the general way is handed the range that this launch has found."""
+    brt, c_router, _, GatherRouter = brt_mod
+    from brainstorm_amd import _lib
+    from brainstorm_amd.runtime.grid_tensor import init_grid_tensor
+
+    g = torch.Generator().manual_seed(high)
+    datas, tags = [], []
+    for n in (300, 0, 41):
+        datas.append(torch.randn(n, 24, generator=g).cuda())
+        tags.append(torch.randint(2, high, (n,), generator=g, dtype=torch.int32).cuda())
+    tags[0][7], tags[2][3] = 1, high
+    fused, unique, inverse = c_router.fuse_split_cells_from_paths(datas, is_tag_fuse=True, tags=tags)
+    want = c_router.combine_with_indices_and_loads(fused, inverse, None, tags=unique, is_tag_index=True, ever_padded=False)
+
+    class WithoutASecondLook:
+        unique_tags = property(lambda self: pytest.fail("the range is looked for again"))
+
+        def __getattr__(self, name):
+            return getattr(native, name)
+
+    native = _lib.native()
+    monkeypatch.setattr(_lib, "native", WithoutASecondLook)
+    loads = [torch.tensor([d.shape[0]], dtype=torch.int32, device="cuda") for d in datas]
+    flows = [init_grid_tensor(d, [None, t], [None, n], None) for d, t, n in zip(datas, tags, loads)]
+    out = GatherRouter().cuda()(flows)
+    assert torch.equal(brt.to_torch_tensor(out), want[0]) and torch.equal(out.tag, want[1])
+
+
 def test_flows_of_unequal_rows_are_refused_as_before(brt_mod):
     from brainstorm_amd._C import router as c_router
 
