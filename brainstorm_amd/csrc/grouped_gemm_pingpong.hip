@@ -604,9 +604,11 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
   // An M phase is as long as its instructions take to issue, so the eight requests are eight instructions and two writes of M0: four
   // loads share one value, the instruction's own offset, 1 KB apart, moves them in LDS, and the registers hold the place in the
   // buffer less that offset, in a buffer that starts kBack bytes early.  When nothing more is to be requested the extent becomes
-  // zero.  (With M0 computed and written for each load and a branch around it, against this, of the time that the kernel took with neither and
+  // kBack, which no offset is below, and the scalar offset 0: whether a request is in range must not hang on a scalar offset that is more
+  // than the extent (by the documents a raw buffer's bound is the extent less the scalar offset).  (With M0 computed and written for each load and a branch around it, against this, of the time that the kernel took with neither and
   // 32 x 32 x 16 MFMAs: 8192 -> 2048 0.983 and 0.952, 2048 -> 8192 0.964 and 0.932, ragged loads 8192 -> 2048 1.01 and 0.97.)
   constexpr uint32_t kBack = 3 * 1024;
+  static_assert(kBack >= kRowB, "the scalar offsets of the two last, empty K-steps are 0 and kRowB");
   auto start_early = [](i32x4 r) {
     const uint64_t at = (static_cast<uint64_t>(static_cast<uint32_t>(r[1])) << 32 | static_cast<uint32_t>(r[0])) - kBack;
     r[0] = static_cast<int>(at), r[1] = static_cast<int>(at >> 32) & 0xffff;
@@ -691,8 +693,8 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     for (int kt = 0; kt < k_tiles; ++kt) {
       if (kt + 2 == turn) cut_off();
       if (kt + 2 == k_tiles) {
-        from += turn_back;
-        if (left == 1) res[2] = 0;
+        from = left == 1 ? 0 : from + turn_back;
+        if (left == 1) res[2] = kBack;
       }
       const char* const pa = smem + a_cur + frag_x;
       const char* const pb = smem + b_cur + frag_w;
