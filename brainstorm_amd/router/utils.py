@@ -46,13 +46,16 @@ def mark_paths(hot_mask: torch.Tensor, most: int) -> None:
     """Notes on a hot mask that, as it stands, no row of it has more than ``most`` nonzeros.  The note is worth nothing once the
     mask is edited in place (by a forward hook, or between protocol and fabric), so it goes with the mask's version counter; a
     tensor that has none is not marked."""
-    if hot_mask.is_inference():
+    try:
+        version = hot_mask._version
+    except RuntimeError:  # an inference tensor
         return
-    hot_mask._brt_paths_per_cell, hot_mask._brt_single_path = most, most == 1
-    hot_mask._brt_marked_at = hot_mask._version
+    hot_mask._brt_paths_per_cell = most, version
+    if most == 1:
+        hot_mask._brt_single_path = True
 
 
 def paths_per_cell(hot_mask) -> int:
     """The paths that a row of the mask has at most, by a mark that still holds; 0 where that is not known."""
-    marked_at = getattr(hot_mask, "_brt_marked_at", None)
-    return hot_mask._brt_paths_per_cell if marked_at is not None and marked_at == hot_mask._version else 0
+    most, version = getattr(hot_mask, "_brt_paths_per_cell", (0, None))
+    return most if most and version == hot_mask._version else 0
