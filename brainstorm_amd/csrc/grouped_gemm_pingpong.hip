@@ -757,6 +757,7 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
       b_cur ^= kTileB;
       from += kRowB;
     }
+    if constexpr (NI > 0) mfma_wait_states();  // in here: where the instances meet, accumulators might be moved
   };
   for (;;) {
 #pragma unroll
@@ -772,7 +773,6 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
     else if (pairs == 2) k_loop(std::integral_constant<int, 4>{});
     else if (pairs == 1) k_loop(std::integral_constant<int, 2>{});
     else k_loop(std::integral_constant<int, 0>{});
-    mfma_wait_states();
     if (a.clocks != nullptr && t == 0 && tid == 0) {  // measurement aid: this wavefront's K loop
       a.clocks[0] = __builtin_amdgcn_s_memtime() - clock0;
       a.clocks[1] = __builtin_amdgcn_s_memrealtime() - tick0;
