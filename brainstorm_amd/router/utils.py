@@ -1,5 +1,6 @@
 """Small helpers shared by routers, protocols and fabrics
 (reference: python/brt/router/utils.py)."""
+import weakref
 from typing import Any, Dict, List, Optional
 
 import numpy as np
@@ -42,6 +43,19 @@ def assert_compatibility(instance, k, expected_v, given_v) -> None:
         f"argument {k}: expected {expected_v}, given {given_v}")
 
 
+class _PathMark:
+    """The paths that a row of one mask has at most.  It holds for that tensor object as it stood: not for a copy, whose
+    version counter starts anew and may agree with that of another state (a pickled mark comes back as an empty set)."""
+
+    __slots__ = ("most", "version", "mask")
+
+    def __init__(self, most: int, version: int, mask: torch.Tensor):
+        self.most, self.version, self.mask = most, version, weakref.ref(mask)
+
+    def __reduce__(self):
+        return set, ()
+
+
 def mark_paths(hot_mask: torch.Tensor, most: int) -> None:
     """Notes on a hot mask that, as it stands, no row of it has more than ``most`` nonzeros.  The note is worth nothing once the
     mask is edited in place (by a forward hook, or between protocol and fabric), so it goes with the mask's version counter; a
@@ -50,12 +64,14 @@ def mark_paths(hot_mask: torch.Tensor, most: int) -> None:
         version = hot_mask._version
     except RuntimeError:  # an inference tensor
         return
-    hot_mask._brt_paths_per_cell = most, version
+    hot_mask._brt_paths_per_cell = _PathMark(most, version, hot_mask)
     if most == 1:
         hot_mask._brt_single_path = True
 
 
 def paths_per_cell(hot_mask) -> int:
     """The paths that a row of the mask has at most, by a mark that still holds; 0 where that is not known."""
-    most, version = getattr(hot_mask, "_brt_paths_per_cell", (0, None))
-    return most if most and version == hot_mask._version else 0
+    mark = getattr(hot_mask, "_brt_paths_per_cell", None)
+    if type(mark) is not _PathMark or mark.mask() is not hot_mask or mark.version != hot_mask._version:
+        return 0
+    return mark.most

@@ -1,4 +1,7 @@
 """What a hot mask's mark promises holds for the mask as the fabric receives it (no GPU needed)."""
+import copy
+import io
+
 import pytest
 import torch
 
@@ -88,3 +91,32 @@ def test_masks_without_a_version_counter_are_not_marked():
     with torch.inference_mode():
         mask = make_protocol("topk", {"top_k": 1})(torch.randn(5, 3))
     assert paths_per_cell(mask) == 0 and int(mask.sum()) == 5
+
+
+def _saved_and_loaded(mask):
+    file = io.BytesIO()
+    torch.save(mask, file)
+    file.seek(0)
+    return torch.load(file, weights_only=True)
+
+
+@pytest.mark.parametrize("copied", [copy.copy, copy.deepcopy, _saved_and_loaded])
+@pytest.mark.parametrize("edits", range(4))
+def test_copies_do_not_inherit_the_mark(monkeypatch, copied, edits):
+    """The version counter of a copy starts anew: what it says of the copy says nothing about what was done to the mask."""
+    mask = make_protocol("topk", {"top_k": 1})(torch.randn(5, 3))
+    for _ in range(edits):
+        mask.fill_(1)
+    other = copied(mask)
+    assert torch.equal(other, mask) and paths_per_cell(other) == 0
+    assert not _single_path_of(monkeypatch, other)
+    assert paths_per_cell(mask) == (0 if edits else 1)
+
+
+@pytest.mark.parametrize("fullgraph", [False, True])
+def test_a_compiled_decision_is_marked(fullgraph):
+    protocol = make_protocol("topk", {"top_k": 1})
+    mask = torch.compile(protocol, backend="eager", fullgraph=fullgraph)(torch.randn(6, 4))
+    assert paths_per_cell(mask) == 1
+    mask[0] = 1
+    assert paths_per_cell(mask) == 0
