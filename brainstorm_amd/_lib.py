@@ -172,6 +172,7 @@ SIGNATURES = {
     "brt_hip_probe_mfma_rate": (_c_int, [_c_int, _c_int, _c_ptr, _c_ptr]),
     "brt_hip_grouped_gemm_kernel": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int]),
     "brt_hip_grouped_gemm_tiles_cut": (_c_int, [_c_ptr, _c_int, _c_int, _c_int, _c_int]),
+    "brt_hip_grouped_gemm_walk": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_ptr]),
     "brt_hip_grouped_gemm_timed": (
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],

@@ -829,19 +829,24 @@ int walk_of_list(const GemmArgs& a) {
   return 1;
 }
 
-template <int ACT, bool ROUTED, bool OUTF32>
-int launch_pingpong(GemmArgs& a, hipStream_t st) {
+// Fills in how the list of tiles is laid out and walked; the workgroups to launch.
+long plan_list(GemmArgs& a) {
   a.tiles_n = (a.N + kBN - 1) / kBN;
-  long grid = workgroups_of_list(a.P, a.E, a.tiles_n);
+  const long grid = workgroups_of_list(a.P, a.E, a.tiles_n);
   // The timed form wants the clocks of a whole tile, also of a list that would be cut to the last: it is told of no workgroups for units.
   // (A test of a.clocks in the kernel itself cost 32768 rows of 16 experts 1024 -> 4096 -> 1024 7 us of 577.)
   a.grid = a.clocks != nullptr ? 0 : static_cast<int>(grid);
   a.tiles_n_inverse = 0xffffffffu / static_cast<uint32_t>(a.tiles_n);
   a.walk = a.clocks != nullptr ? 1 : walk_of_list(a);
   a.walk_inverse = 0xffffffffu / static_cast<uint32_t>(a.walk);
+  return a.walk > 1 ? workgroups_that_walk(grid, a.walk) : grid;
+}
+
+template <int ACT, bool ROUTED, bool OUTF32>
+int launch_pingpong(GemmArgs& a, hipStream_t st) {
+  const long grid = plan_list(a);
   auto* fn = &grouped_gemm_pingpong_kernel<ACT, ROUTED, OUTF32>;
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(fn), kLdsBytes); rc != BRT_OK) return rc;
-  if (a.walk > 1) grid = workgroups_that_walk(grid, a.walk);
   hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(grid)), dim3(kWaves * 64), kLdsBytes, st, a);
   return check_launch("grouped_gemm_pingpong_kernel");
 }
@@ -892,4 +897,13 @@ extern "C" int brt_hip_grouped_gemm_tiles_cut(const int32_t* loads, int E, int P
   }
   if (blocks * a.tiles_n > 0x7fffffffll) return fail(BRT_E_INVALID, "%ld row blocks of %d tiles", blocks, a.tiles_n);
   return end_of_list(a, static_cast<int>(blocks * a.tiles_n), few, [&](int n) { return n / a.tiles_n; }).cut;
+}
+
+extern "C" int brt_hip_grouped_gemm_walk(int E, int P, int K, int N, int* workgroups) {
+  using namespace brt;
+  if (!workgroups || E <= 0 || P <= 0 || K <= 0 || N <= 0) return fail(BRT_E_INVALID, "bad arguments E=%d P=%d K=%d N=%d", E, P, K, N);
+  GemmArgs a{};
+  a.E = E; a.P = P; a.K = K; a.N = N;
+  *workgroups = static_cast<int>(plan_list(a));
+  return a.walk;
 }

@@ -525,6 +525,11 @@ int brt_hip_grouped_gemm_kernel(int E, int P, int K, int N, int accumulates);
  * [E] in host memory; row_tags: a routed form that writes row tags.
  */
 int brt_hip_grouped_gemm_tiles_cut(const int32_t* loads, int E, int P, int N, int row_tags);
+/*
+ * ... and how many column tiles of a row block one of its workgroups walks in the whole rounds of the list (1: none walks),
+ * with the workgroups it is launched with.
+ */
+int brt_hip_grouped_gemm_walk(int E, int P, int K, int N, int* workgroups);
 
 /*
  * Measurement aid (no counterpart in the reference; bench.py reports what it reads beside the
