@@ -810,22 +810,21 @@ int grouped_gemm_impl(const void* x, const void* const* weights, const void* con
   // (grouped_gemm_pingpong.hip), whose 256 x 256 tile moves a third fewer operand bytes per flop,
   // when its tiles fill a round over the CUs to three quarters or more.  The tile count is an estimate: the
   // loads are on the device; an expert's last row block is taken as half full.  Measured in one
-  // process against the 160-row kernel: 8 experts x 4096 rows 2048 -> 8192 -> 2048 1165 / 993 ->
-  // 962 / 793 us, the ragged task-MoE shape 1585 / 1374 -> 1355 / 1211 us, the top-2 shape's
-  // expanding GEMM (1232 tiles) 212 -> 166 us, 8 x 1824 rows 4096 -> 1024 (256 tiles) 146 -> 99 us; with one to two rounds, whose
-  // end is cut into units, 8 x 1000 rows 4096 -> 2048 148 -> 115 us, 64 x 400 rows 3072 -> 768 172 -> 145, 4 x 8000 rows 256 -> 1024 58 -> 34
-  // (60 shapes of 1.0 to 2.0 rounds: 1.29 times as fast in the mean).  Between 1.25 and 1.5 rounds the end is too long to be
+  // process against the 160-row kernel, us there and here: 8 experts x 4096 rows 2048 -> 8192 1055 and 811, 8192 -> 2048 998 and
+  // 744, 32 x 1024 rows 1024 -> 4096 360 and 236, 8 x 1824 rows 4096 -> 1024 (256 tiles) 147 and 90; with one to two rounds, whose
+  // end is cut into units, 8 x 1000 rows 4096 -> 2048 147 and 94, 64 x 400 rows 3072 -> 768 178 and 145, 4 x 8000 rows 256 -> 1024 44 and 27.
+  // Between 1.25 and 1.5 rounds the end is too long to be
   // cut and too short to fill the second round, and where the 160-row kernel is through in two rounds of its own
-  // the two are level on average (60 x 270 rows 4096 -> 1024 170 us there, 188 here; 12 x 1092 rows
-  // 5888 -> 1472 216 and 257; 64 x 337 rows 2816 -> 704 156 and 128): those stay there, and those of up to 1.6 rounds for which two
-  // narrow workgroups of it fit a CU (4 x 8070 rows 1280 -> 640 62 and 68).  Below three quarters of a round the 160-row
-  // tiles spread better (4 x 4060 rows 1792 -> 448, half a round, 37.9 us there, 46.9 here).
-  // Widths that are no multiple of a K-step of 64 are under the same rule: 8 x 1024 rows 1592 -> 6368 278 us there, 187 here,
-  // 6368 -> 1592 218 and 176, 4 x 3000 rows 4384 -> 1096 155 and 120, 64 x 400 rows 360 -> 1440 105 and 63, 12 x 700 rows 7200 -> 1800
-  // 279 and 276, 4 x 4000 rows 264 -> 528 (three column tiles for 528 columns) 22.5 and 22.8.
-  // Even loads a little over one 256-row block are the weak spot: with 257 to 320 rows the two are level in the mean, as long as the
-  // end of the list is cut (16 x 296 rows 4032 -> 2312 138 us there, 134 here), and those win by up to a quarter where the last blocks fill
-  // half a round or a whole one (16 x 266 rows 3416 -> 2976 151 and 186); of the same averages ragged loads are 0.9 and skewed ones 0.77 of
+  // it is the faster or the slower one by a tenth to a fifth (60 x 270 rows 4096 -> 1024 177 us there, 195 here; 12 x 1092 rows
+  // 5888 -> 1472 211 and 234; 64 x 337 rows 2816 -> 704 154 and 126): those stay there, and those of up to 1.6 rounds for which two
+  // narrow workgroups of it fit a CU (4 x 8070 rows 1280 -> 640 64 and 66).  Below three quarters of a round the 160-row
+  // tiles spread better (4 x 4060 rows 1792 -> 448, half a round, 39.4 us there, 43.3 here).
+  // Widths that are no multiple of a K-step of 64 are under the same rule: 8 x 1024 rows 1592 -> 6368 250 us there, 152 here,
+  // 6368 -> 1592 205 and 156, 4 x 3000 rows 4384 -> 1096 143 and 99, 64 x 400 rows 360 -> 1440 81 and 48, 12 x 700 rows 7200 -> 1800
+  // 273 and 268, 4 x 4000 rows 264 -> 528 (three column tiles for 528 columns) 18.8 and 16.4.
+  // Even loads a little over one 256-row block are the weak spot: those win here whose end of the
+  // list is cut (16 x 296 rows 4032 -> 2312 131 us there, 124 here), and those lose up to a quarter where the last blocks fill
+  // half a round or a whole one (16 x 266 rows 3416 -> 2976 150 and 185); ragged loads of the same average take 0.71 and skewed ones 0.67 of
   // their time here, and the host does not know which it has.
   // The rule is the same for gathered, scattered and fp32-output rows: a gathering 1024 -> 4096 GEMM with GELU over 32768
   // rows of 16 experts takes 437 us on the 160-row kernel and 336 us here; fp32 output, 420 drawn shapes of one to two rounds, 0.81 of that

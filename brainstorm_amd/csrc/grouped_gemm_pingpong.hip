@@ -85,13 +85,14 @@ constexpr int kXcds = 8, kCusPerXcd = 32, kPatchRows = 4;
 constexpr int kRoundBits = 8, kRound = kXcds * kCusPerXcd;  // tiles of a whole round
 static_assert(kRound == 1 << kRoundBits);
 // The end of the list that is cut into units (see the kernel).  It takes the CUs one round of units up to 64 tiles and two up to 128,
-// against a round in which the tiles leave most CUs idle.  A unit of 256 rows takes 0.4 to 0.5 of a tile's time (4 x 1024 rows
-// 4096 -> 1024, 256 units: 40 us against 102 us for the 64 tiles they are made of), one of up to 128 rows half of what its block
-// takes as a tile (38 us and 73).  Of lists of one to two rounds (us, not cut and cut): 65 tiles 0.79 to 0.96 of the time, 80 tiles 0.93
-// to 0.95 (4 x 1704 rows 1504 -> 3008 80 and 75), 92 to 104 tiles 0.96 to 1.02, 108 and more 1.00 to 1.08 (8 x 785 skewed rows
-// 3592 -> 3272 191 and 205, 64 x 393 rows 2288 -> 736 127 and 135); where all of them are blocks of few rows 105 tiles 0.83 to 0.92
-// (60 x 265 rows 4152 -> 592) and 116 0.89, 128 of 128 rows 1.07 (32 x 640 rows 6024 -> 928 311 and 333).  In a list of more than ten rounds the CUs are no longer in step, and nothing
-// is left to gain (98 blocks 2048 -> 8192, 12.25 rounds: 763 us cut, 756 not).
+// against a round in which the tiles leave most CUs idle.  A unit of 256 rows takes 0.4 of a tile's time (4 x 1024 rows
+// 4096 -> 1024, 256 units: 38 us against 90 us for the 64 tiles they are made of), one of up to 128 rows half of what its block
+// takes as a tile.  Of lists of one to two and a half rounds (50 drawn ones; us, not cut and cut): up to 60 tiles 0.71 to 0.90 of the time (one 1.02),
+// 61 to 76 tiles 0.80 to 1.01, 77 to 91 tiles 0.87 to 1.02 (4 x 1704 rows 1504 -> 3008 74 and 73), 92 to 104 tiles 0.95 to 1.05, 108 and more,
+// which are left whole, 0.91 to 1.13 if they were cut (24 x 934 rows 3696 -> 984 198 and 221, 64 x 393 rows 2288 -> 736 125 and 135);
+// where all of them are blocks of few rows 104 tiles 0.81 and 0.87 (60 x 265 rows 4152 -> 592 202 and 163), 128 of 128 rows 1.05
+// (32 x 640 rows 6024 -> 928 307 and 322).  In a list of more than ten rounds the CUs are no longer in step, and nothing
+// is left to gain (98 blocks 2048 -> 8192, 12.25 rounds: level).
 constexpr int kFewRows = 128, kMostCut = 104, kMostCutOfFewRows = 116, kMostRounds = 10;
 constexpr int kUnitCols = 64;
 constexpr int kStreamed = 2 | 16;  // cache policy of a buffer store: nt sc1
@@ -791,8 +792,8 @@ __global__ __launch_bounds__(kWaves * 64) void grouped_gemm_pingpong_kernel(Gemm
 
 // The sum over experts of ceil(M_e / 256) never exceeds P / 256 + E; whole rounds of XCD patches.  What the loads leave of it is room for
 // units, and of experts with a little over whole blocks each nothing is left, so there are as many workgroups as the end of a list of
-// even loads needs (us, without them and with them: 60 x 274 rows 7608 -> 608 378 and 328, 16 x 296 rows 4032 -> 2312 151 and 134, 32 x 294
-// rows 7448 -> 1096 347 and 279).  Room for the longest end of any list costs others more than it gives: 64 x 400 rows 768 -> 3072
+// even loads needs (us, without them and with them: 60 x 274 rows 7608 -> 608 373 and 326, 16 x 296 rows 4032 -> 2312 139 and 120, 32 x 294
+// rows 7448 -> 1096 344 and 276).  Room for the longest end of any list costs others more than it gives: 64 x 400 rows 768 -> 3072
 // 141 -> 147 us, 16 x 2048 rows 4096 -> 1024 213 -> 218.
 long workgroups_of_list(int P, int E, int tiles_n) {
   const long used = std::min(E, P), rows = used > 0 ? (P + used - 1) / used : 0, over = rows % kBM;

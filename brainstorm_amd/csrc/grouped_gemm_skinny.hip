@@ -432,7 +432,9 @@ long wide_tiles(const GemmArgs& a) {
 // 256 -> 1024 31 and 14, 64 x 94 rows 128 -> 256 15 and 5.6, 12 x 233 rows 576 -> 2304 41 and 23, 24 x 322 rows 192 -> 768 12.4 and 12.2).  Of 80 other
 // drawn shapes the mean is 1.52 times as fast, three are slower (24 x 174 skewed rows 576 -> 1152 19.3 and 21.1).
 // Only where the rows are whole lines; not with fewer experts (8 x 343 rows 960 -> 1920 26.1 and 26.5), more weights (24 x 124 rows 512 -> 2048, 50 MB, 18.7 and 23.1) or
-// more tiles (128 x 120 rows 128 -> 512, 256 of them, 13.3 and 17.4).
+// more tiles (128 x 120 rows 128 -> 512, 256 of them, 13.3 and 17.4).  Up to 96 tiles of up to 32 experts are this kernel's in any case (below)
+// and stay in the order of the list.  (Dealt as well, 60 drawn ones take 0.95 of the
+// time in the mean, from 0.60 -- 21 x 225 rows 384 -> 576 13.3 and 7.9 -- to 1.02.)
 bool expanding_and_dealt(const GemmArgs& a) {
   const long used = std::min(a.E, a.P), tiles = wide_tiles(a);
   return a.N > a.K && a.K % kBK == 0 && used >= 12 && a.P > 64 * used && a.P <= 400 * used && tiles <= 170 && (tiles > 96 || used > 32) &&
