@@ -233,15 +233,15 @@ class DispatchFabric(FabricBase):
         caps = runtime_capacities if runtime_capacities is not None else self.supported_capacities
         in_flows = [in_flow] if self.flow_num == 1 else in_flow
         as_tags = self._defers(in_flows, runtime_capacities, hot_mask)
-        per_cell = paths_per_cell(hot_mask)
         if route is None or as_tags:
+            per_cell = paths_per_cell(hot_mask)
             route = c_router.generate_route(
                 hot_mask, supported_capacities=caps, capacity_padding=self.capacity_padding,
                 path_wise_padding=self.path_wise_padding, is_tag_index=as_tags,
                 single_path=per_cell == 1)
+        else:
+            per_cell = 1 if route.single_path else paths_per_cell(hot_mask)
         self.__dict__["_route"] = route  # (not through nn.Module's attribute registration)
-        if route.single_path:
-            per_cell = 1
         self.__dict__["_likely_rows"] = route.cells * per_cell if per_cell and not self.capacity_padding else None
         route_indices, loads = route.indices, route.loads
         self.capture_flow_stats(in_flows, route_indices, loads)

@@ -43,14 +43,12 @@ def assert_compatibility(instance, k, expected_v, given_v) -> None:
         f"argument {k}: expected {expected_v}, given {given_v}")
 
 
-class _PathMark:
-    """The paths that a row of one mask has at most.  It holds for that tensor object as it stood: not for a copy, whose
-    version counter starts anew and may agree with that of another state (a pickled mark comes back as an empty set)."""
+class _PathMark(tuple):
+    """(the paths that a row of one mask has at most, the mask's version counter, a weak reference to it).  It holds for that
+    tensor object as it stood: not for a copy, whose version counter starts anew and may agree with that of another state (a
+    pickled mark comes back as an empty set)."""
 
-    __slots__ = ("most", "version", "mask")
-
-    def __init__(self, most: int, version: int, mask: torch.Tensor):
-        self.most, self.version, self.mask = most, version, weakref.ref(mask)
+    __slots__ = ()
 
     def __reduce__(self):
         return set, ()
@@ -61,10 +59,9 @@ def mark_paths(hot_mask: torch.Tensor, most: int) -> None:
     mask is edited in place (by a forward hook, or between protocol and fabric), so it goes with the mask's version counter; a
     tensor that has none is not marked."""
     try:
-        version = hot_mask._version
+        hot_mask._brt_paths_per_cell = _PathMark((most, hot_mask._version, weakref.ref(hot_mask)))
     except RuntimeError:  # an inference tensor
         return
-    hot_mask._brt_paths_per_cell = _PathMark(most, version, hot_mask)
     if most == 1:
         hot_mask._brt_single_path = True
 
@@ -72,6 +69,6 @@ def mark_paths(hot_mask: torch.Tensor, most: int) -> None:
 def paths_per_cell(hot_mask) -> int:
     """The paths that a row of the mask has at most, by a mark that still holds; 0 where that is not known."""
     mark = getattr(hot_mask, "_brt_paths_per_cell", None)
-    if type(mark) is not _PathMark or mark.mask() is not hot_mask or mark.version != hot_mask._version:
+    if type(mark) is not _PathMark or mark[1] != hot_mask._version or mark[2]() is not hot_mask:
         return 0
-    return mark.most
+    return mark[0]
