@@ -184,8 +184,8 @@ def summarize_counters(pairs, counters, commit):
     print("Averages per launch; SQ, TCP and TCC counters are summed over the chip (SQ wave-cycle counters "
           "advance once per 4 clocks), GRBM_GUI_ACTIVE over the 8 XCDs. "
           "`mfma busy` = SQ_VALU_MFMA_BUSY_CYCLES / (1024 SIMDs x GRBM_GUI_ACTIVE / 8): the share of the "
-          "kernel's duration in which a SIMD's matrix pipe is busy (the counter advances by 32 per "
-          "`v_mfma_f32_32x32x16_bf16`); `flop` = SQ_INSTS_VALU_MFMA_MOPS_BF16 x 512 (every row tile of a "
+          "kernel's duration in which a SIMD's matrix pipe is busy (the counter advances by 16 per "
+          "`v_mfma_f32_16x16x32_bf16`, by 32 per `v_mfma_f32_32x32x16_bf16`); `flop` = SQ_INSTS_VALU_MFMA_MOPS_BF16 x 512 (every row tile of a "
           "row block is multiplied, filled or not).\n")
     seen = {}
     for pair in pairs:

@@ -24,8 +24,8 @@
 //     rows one phase earlier), once its own weight fragments are in registers.  Every request has
 //     three to four phases to land, and each wavefront issues its 8 loads of a K-step in its M
 //     phase, between fragment reads.  A K-step is 2 x 1024 clocks of MFMA per SIMD and measures
-//     about 2150, at the 1.5 to 1.7 GHz that the part sustains with them: it is the package's power that sets the time of a K-step
-//     (1.35 to 1.45 us; with fewer clocks the clock rate falls), so what counts is its energy.  That of the 16 x 16 x 32 instruction is
+//     2150 to 2270, at the 1.5 to 1.8 GHz that the part sustains with them: it is the package's power that sets the time of a K-step
+//     (1.3 to 1.45 us; with fewer clocks the clock rate falls), so what counts is its energy.  That of the 16 x 16 x 32 instruction is
 //     lower than that of v_mfma_f32_32x32x16_bf16, which reads and writes every accumulator twice as often; both sum the products of
 //     an output element to the same bits.  us, 32 x 32 x 16 and this: 8 x 4096 rows 2048 -> 8192 + GELU 906 and 876, 8192 -> 2048 776 and
 //     752, 16 x 2048 rows 1024 -> 4096 + GELU 271 and 262, 4096 -> 1024 210 and 204, 64 x 400 rows 768 -> 3072 + GELU 161 and 155.
