@@ -142,6 +142,8 @@ class SwitchTop1Protocol(ProtocolBase):
     mask comes from the caller, so nothing is assumed by default: a row with several ones is
     routed to all of them and summed, as in the reference."""
 
+    one_hot = False  # (of a protocol that was saved before it had the attribute)
+
     def __init__(self, one_hot: bool = False, **kwargs):
         super().__init__(**kwargs)
         self.one_hot = bool(one_hot)

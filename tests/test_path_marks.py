@@ -120,3 +120,15 @@ def test_a_compiled_decision_is_marked(fullgraph):
     assert paths_per_cell(mask) == 1
     mask[0] = 1
     assert paths_per_cell(mask) == 0
+
+
+@pytest.mark.parametrize("one_hot", [False, True])
+def test_protocols_saved_before_they_made_their_marks_run(one_hot):
+    """A protocol object whose attributes are those of an earlier version: `single_path` where there is `one_hot` now."""
+    protocol = make_protocol("switch_top1", {"one_hot": one_hot})
+    del protocol.__dict__["one_hot"]
+    protocol.single_path = one_hot
+    assert paths_per_cell(protocol(torch.eye(4, dtype=torch.int32))) == (1 if one_hot else 0)
+    protocol = make_protocol("topk", {"top_k": 1})
+    protocol.single_path = True
+    assert paths_per_cell(protocol(torch.randn(5, 3))) == 1
